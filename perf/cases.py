@@ -42,28 +42,28 @@ LLAMA = {
 def listed():
     return [
         # an utterance of a small deployment through the encoder
-        {"name": "encode base, 1 window", "kind": "encode", "model": "whisper-base", "windows": 1},
+        {"name": "encode base 1 window", "kind": "encode", "model": "whisper-base", "windows": 1},
         # the served model: one utterance, and several that arrive together
-        {"name": "encode large, 1 window", "kind": "encode", "model": "whisper-large-v3", "windows": 1},
-        {"name": "encode large, 6 windows", "kind": "encode", "model": "whisper-large-v3", "windows": 6},
+        {"name": "encode large 1 window", "kind": "encode", "model": "whisper-large-v3", "windows": 1},
+        {"name": "encode large 6 windows", "kind": "encode", "model": "whisper-large-v3", "windows": 6},
         # one greedy token for eight live utterances
-        {"name": "transcript token, 8 streams", "kind": "step", "model": "whisper-large-v3", "streams": 8, "context": 60},
+        {"name": "transcript token 8 streams", "kind": "step", "model": "whisper-large-v3", "streams": 8, "context": 60},
         # a chunk of an intent prompt behind a cached prefix, and a long prompt as one pass
         {"name": "prompt chunk of 320", "kind": "prompt", "model": "llama3-8b", "seqs": 1, "tokens": 320, "past": 192},
         {"name": "prompt of 2048", "kind": "prompt", "model": "llama3-8b", "seqs": 1, "tokens": 2048, "past": 0},
         # one token for eight live replies
-        {"name": "token, 8 replies", "kind": "token", "model": "llama3-8b", "seqs": 8, "context": 600},
+        {"name": "token 8 replies", "kind": "token", "model": "llama3-8b", "seqs": 8, "context": 600},
         # sliding-window attention: a prompt, and a token for eight sequences
-        {"name": "window attention, prompt", "kind": "window", "seqs": 1, "tokens": 2048, "past": 0, "heads": 16, "groups": 4,
+        {"name": "window attention prompt", "kind": "window", "seqs": 1, "tokens": 2048, "past": 0, "heads": 16, "groups": 4,
          "dim": 128, "rot": 64, "window": 1024, "softcap": 0.0, "keep_first": 0, "gate": False, "sink": True, "bias": False},
-        {"name": "window attention, token", "kind": "window", "seqs": 8, "tokens": 1, "past": 2047, "heads": 16, "groups": 4,
+        {"name": "window attention token", "kind": "window", "seqs": 8, "tokens": 1, "past": 2047, "heads": 16, "groups": 4,
          "dim": 128, "rot": 64, "window": 1024, "softcap": 0.0, "keep_first": 0, "gate": False, "sink": True, "bias": False},
         # routed experts of a prompt
-        {"name": "experts, prompt", "kind": "experts", "tokens": 2048, "width": 2048, "ff": 1408, "experts": 16, "top": 4, "act": "swiglu"},
+        {"name": "experts prompt", "kind": "experts", "tokens": 2048, "width": 2048, "ff": 1408, "experts": 16, "top": 4, "act": "swiglu"},
         # the gated delta rule of a prompt, decays per key channel
-        {"name": "delta rule, prompt", "kind": "delta", "seqs": 1, "tokens": 2048, "past": False, "heads": 16, "groups": 4, "dim": 128, "channel": True},
+        {"name": "delta rule prompt", "kind": "delta", "seqs": 1, "tokens": 2048, "past": False, "heads": 16, "groups": 4, "dim": 128, "channel": True},
         # latent attention of a prompt
-        {"name": "latent attention, prompt", "kind": "latent", "seqs": 1, "tokens": 2048, "past": 0, "heads": 16, "window": 0, "gate": True},
+        {"name": "latent attention prompt", "kind": "latent", "seqs": 1, "tokens": 2048, "past": 0, "heads": 16, "window": 0, "gate": True},
     ]
 
 
