@@ -1,0 +1,175 @@
+// Shared parts of the two split-K tiled GEMMs (gemm_sk.hip, gemm_pipe.hip): launch
+// parameters, the in-launch reduction of a tile's K chunks, and the epilogues.
+#pragma once
+#include "common.h"
+
+#define SK_BK 64
+
+enum { SK_BF16 = 0, SK_SWIGLU = 1, SK_RESID = 2 };
+
+struct GemmSkParams {
+  const void* x; long long ldx;   // [M, K] bf16 rows
+  const void* w;                  // [N, K] bf16 row-major (SwiGLU: gate rows [0, N/2), up [N/2, N))
+  int M, N, K, S;                 // S: K chunks per output tile
+  int epi, act;                   // act (SK_BF16): 0 none, 1 GELU (erf) after the bias
+  const float* bias;              // [N] f32 or null (SK_BF16, SK_RESID)
+  void* y; long long ldy;         // bf16 output (SK_RESID: the residual, updated in place)
+  float* ws;                      // S > 1: [tiles][S][BM * BN] f32 partials
+  int* counters;                  // S > 1: [tiles] ints, zero on entry (left zero)
+  int layout;
+};
+
+// s_waitcnt vmcnt(N) with expcnt / lgkmcnt at their maxima (gfx9 encoding:
+// vmcnt[3:0] in bits 3:0, vmcnt[5:4] in bits 15:14)
+template <int N>
+__device__ __forceinline__ void sk_wait_vm() {
+  static_assert(N >= 0 && N < 64, "vmcnt range");
+  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
+}
+
+// GELU through erfc's rational form (Abramowitz and Stegun 7.1.26, |error| <= 1.5e-7):
+// (v + |v|) / 2 - |v| erfc(|v| / sqrt 2) / 2 has no cancellation in the negative tail, where
+// 1 + erf(z) keeps an absolute error of half an ulp of one, and a third of erff's
+// instructions - with one wave per SIMD nothing hides an epilogue's arithmetic.
+__device__ __forceinline__ float sk_gelu(float v) {
+  const float a = fabsf(v), c = fminf(a, 1e4f);        // erfc is 0 there; no inf * 0
+  const float t = __builtin_amdgcn_rcpf(1.f + 0.23164188f * c);   // 0.3275911 / sqrt 2
+  const float q = t * (0.254829592f + t * (-0.284496736f + t * (1.421413741f + t * (-1.453152027f + t * 1.061405429f))));
+  const float e = __builtin_amdgcn_exp2f(c * c * -0.72134752044448170f);   // exp(-c^2 / 2)
+  return (0.5f * v + 0.5f * a) - 0.5f * c * (q * e);
+}
+
+__device__ __forceinline__ float sk_swiglu(float g, float u) {   // silu(g) u
+  return g * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(g * -1.4426950408889634f)) * u;
+}
+
+// Publish this chunk's partial; the tile's last arriver gets the sum of all S in
+// `acc` and returns true, the others return false.
+template <int NW, int FN, int FM>
+__device__ __forceinline__ bool sk_reduce(const GemmSkParams& p, float4v (&acc)[FN][FM], int tile, int s,
+                                          int wave, int lane, int* flag) {
+  const int S = p.S;
+  constexpr int PER_WAVE = FN * FM * 256;      // floats per wave partial (16 B per lane per fragment)
+  float* mine = p.ws + (((size_t)tile * S + s) * NW + wave) * PER_WAVE;
+#pragma unroll
+  for (int i = 0; i < FN; ++i)
+#pragma unroll
+    for (int j = 0; j < FM; ++j)
+      *reinterpret_cast<float4v*>(mine + ((i * FM + j) * 64 + lane) * 4) = acc[i][j];
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    const int t = __hip_atomic_fetch_add(p.counters + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const int last = t == S - 1;
+    if (last) __hip_atomic_store(p.counters + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    *flag = last;
+  }
+  __syncthreads();
+  if (!*flag) return false;
+  if (threadIdx.x == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  // fixed chunk order 0..S-1, every partial (this workgroup's own included)
+  // read back from the workspace: the sum does not depend on who arrived
+  // last, and needs no second accumulator array (the 256 x 256 tile has no
+  // registers for one). Loads go in groups of up to 16 fragments.
+  constexpr int GI = FM >= 16 ? 1 : (16 / FM < FN ? 16 / FM : FN);
+  static_assert(FN % GI == 0, "fragment groups");
+  for (int c = 0; c < S; ++c) {
+    const float* theirs = p.ws + (((size_t)tile * S + c) * NW + wave) * PER_WAVE;
+#pragma unroll
+    for (int i0 = 0; i0 < FN; i0 += GI) {
+      float4v v[GI][FM];
+#pragma unroll
+      for (int i = 0; i < GI; ++i)
+#pragma unroll
+        for (int j = 0; j < FM; ++j)
+          v[i][j] = *reinterpret_cast<const float4v*>(theirs + (((i0 + i) * FM + j) * 64 + lane) * 4);
+#pragma unroll
+      for (int i = 0; i < GI; ++i)
+#pragma unroll
+        for (int j = 0; j < FM; ++j) acc[i0 + i][j] = c == 0 ? v[i][j] : acc[i0 + i][j] + v[i][j];
+    }
+  }
+  return true;
+}
+
+// acc[i][j] = C[n = nw + 16 i + 4 fq + r][m = mw + 16 j + fr] of one wave; fw: its first
+// SwiGLU output feature.
+template <int EPI, int FN, int FM>
+__device__ __forceinline__ void sk_epilogue(const GemmSkParams& p, float4v (&acc)[FN][FM], int nw, int fw,
+                                            int mw, int fr, int fq) {
+  const int M = p.M;
+  bf16_t* Y = reinterpret_cast<bf16_t*>(p.y);
+  if constexpr (EPI == SK_SWIGLU) {
+#pragma unroll
+    for (int j = 0; j < FM; ++j) {
+      const int m = mw + 16 * j + fr;
+      if (m >= M) continue;
+#pragma unroll
+      for (int i = 0; i < FN / 2; ++i) {
+        const int f = fw + 16 * i + 4 * fq;
+        float o[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          o[r] = sk_swiglu(acc[i][j][r], acc[i + FN / 2][j][r]);
+        }
+        *reinterpret_cast<uint2*>(Y + (size_t)m * p.ldy + f) =
+            make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
+      }
+      __builtin_amdgcn_sched_barrier(0);   // a row block's accumulators at a time
+    }
+  } else if constexpr (EPI == SK_RESID) {
+    float4 bv[FN];
+#pragma unroll
+    for (int i = 0; i < FN; ++i) {
+      const int n = nw + 16 * i + 4 * fq;
+      bv[i] = p.bias ? *reinterpret_cast<const float4*>(p.bias + n) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+#pragma unroll
+    for (int j = 0; j < FM; ++j) {
+      const int m = mw + 16 * j + fr;
+      if (m >= M) continue;
+#pragma unroll
+      for (int i = 0; i < FN; ++i) {
+        const int n = nw + 16 * i + 4 * fq;
+        uint2* yp = reinterpret_cast<uint2*>(Y + (size_t)m * p.ldy + n);
+        const uint2 rv = *yp;
+        const float o0 = bf2f(rv.x & 0xffff) + (acc[i][j][0] + bv[i].x);
+        const float o1 = bf2f(rv.x >> 16) + (acc[i][j][1] + bv[i].y);
+        const float o2 = bf2f(rv.y & 0xffff) + (acc[i][j][2] + bv[i].z);
+        const float o3 = bf2f(rv.y >> 16) + (acc[i][j][3] + bv[i].w);
+        *yp = make_uint2(pack_bf16x2(o0, o1), pack_bf16x2(o2, o3));
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  } else {
+    float4 bv[FN];
+#pragma unroll
+    for (int i = 0; i < FN; ++i) {
+      const int n = nw + 16 * i + 4 * fq;
+      bv[i] = p.bias ? *reinterpret_cast<const float4*>(p.bias + n) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+#pragma unroll
+    for (int j = 0; j < FM; ++j) {
+      const int m = mw + 16 * j + fr;
+      if (m >= M) continue;
+#pragma unroll
+      for (int i = 0; i < FN; ++i) {
+        const int n = nw + 16 * i + 4 * fq;
+        float o[4] = {acc[i][j][0] + bv[i].x, acc[i][j][1] + bv[i].y, acc[i][j][2] + bv[i].z,
+                      acc[i][j][3] + bv[i].w};
+        if (p.act == 1) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) o[r] = sk_gelu(o[r]);
+        }
+        *reinterpret_cast<uint2*>(Y + (size_t)m * p.ldy + n) =
+            make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+}
+

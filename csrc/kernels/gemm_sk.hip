@@ -2,6 +2,10 @@
 // Y[M, N] = X[M, K] W[N, K]^T for the projections of a prompt pass (Llama
 // prefill: M = a few hundred to a few thousand rows) and the Whisper encoder.
 //
+// This file holds the general form (any feature count that is a multiple of 64, any row
+// alignment that 16-byte loads take) and the entry point; gemm_pipe.hip has the pipelined
+// form that serves everything else.
+//
 // Why split-K inside the launch: at M ~ 300 a projection has few output tiles
 // (qkv 6144 x 4096: 240 tiles of 128 x 64; o / down 4096 wide: 160), far fewer
 // than the 256 CUs x 2-3 resident workgroups, and a whole tile's K loop is one
@@ -25,31 +29,7 @@
 //   SK_RESID  y = bf16(y + (acc + bias)): the row-parallel projections (o,
 //             down, encoder o / fc2) add straight into the residual stream, one
 //             rounding.
-#include "common.h"
-
-#define SK_BK 64
-
-enum { SK_BF16 = 0, SK_SWIGLU = 1, SK_RESID = 2 };
-
-struct GemmSkParams {
-  const void* x; long long ldx;   // [M, K] bf16 rows
-  const void* w;                  // [N, K] bf16 row-major (SwiGLU: gate rows [0, N/2), up [N/2, N))
-  int M, N, K, S;                 // S: K chunks per output tile
-  int epi, act;                   // act (SK_BF16): 0 none, 1 GELU (erf) after the bias
-  const float* bias;              // [N] f32 or null (SK_BF16, SK_RESID)
-  void* y; long long ldy;         // bf16 output (SK_RESID: the residual, updated in place)
-  float* ws;                      // S > 1: [tiles][S][BM * BN] f32 partials
-  int* counters;                  // S > 1: [tiles] ints, zero on entry (left zero)
-  int layout;
-};
-
-// s_waitcnt vmcnt(N) with expcnt / lgkmcnt at their maxima (gfx9 encoding:
-// vmcnt[3:0] in bits 3:0, vmcnt[5:4] in bits 15:14)
-template <int N>
-__device__ __forceinline__ void sk_wait_vm() {
-  static_assert(N >= 0 && N < 64, "vmcnt range");
-  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
-}
+#include "gemm_sk.h"
 
 template <int WN, int WM, int FN, int FM, int NBUF, int EPI>
 __global__ __launch_bounds__(64 * WN * WM) void gemm_sk_kernel(GemmSkParams p) {
@@ -188,126 +168,8 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_sk_kernel(GemmSkParams p) {
     compute(t % NBUF);
   }
 
-  // ---- split-K: publish this chunk's partial, the tile's last arriver sums them
-  if (S > 1) {
-    constexpr int PER_WAVE = FN * FM * 256;      // floats per wave partial (16 B per lane per fragment)
-    float* mine = p.ws + (((size_t)tile * S + s) * NW + wave) * PER_WAVE;
-#pragma unroll
-    for (int i = 0; i < FN; ++i)
-#pragma unroll
-      for (int j = 0; j < FM; ++j)
-        *reinterpret_cast<float4v*>(mine + ((i * FM + j) * 64 + lane) * 4) = acc[i][j];
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    int* flag = reinterpret_cast<int*>(lds);     // the one LDS array (guide §5 item 4a)
-    if (threadIdx.x == 0) {
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      const int t = __hip_atomic_fetch_add(p.counters + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      const int last = t == S - 1;
-      if (last) __hip_atomic_store(p.counters + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      *flag = last;
-    }
-    __syncthreads();
-    if (!*flag) return;
-    if (threadIdx.x == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    // fixed chunk order 0..S-1, every partial (this workgroup's own included)
-    // read back from the workspace: the sum does not depend on who arrived
-    // last, and needs no second accumulator array (the 256 x 256 tile has no
-    // registers for one). Loads go in groups of up to 16 fragments.
-    constexpr int GI = FM >= 16 ? 1 : (16 / FM < FN ? 16 / FM : FN);
-    static_assert(FN % GI == 0, "fragment groups");
-    for (int c = 0; c < S; ++c) {
-      const float* theirs = p.ws + (((size_t)tile * S + c) * NW + wave) * PER_WAVE;
-#pragma unroll
-      for (int i0 = 0; i0 < FN; i0 += GI) {
-        float4v v[GI][FM];
-#pragma unroll
-        for (int i = 0; i < GI; ++i)
-#pragma unroll
-          for (int j = 0; j < FM; ++j)
-            v[i][j] = *reinterpret_cast<const float4v*>(theirs + (((i0 + i) * FM + j) * 64 + lane) * 4);
-#pragma unroll
-        for (int i = 0; i < GI; ++i)
-#pragma unroll
-          for (int j = 0; j < FM; ++j) acc[i0 + i][j] = c == 0 ? v[i][j] : acc[i0 + i][j] + v[i][j];
-      }
-    }
-  }
-
-  // ---- epilogue: acc[i][j] = C[n = n0 + TN wn + 16 i + 4 fq + r][m = m0 + TM wm + 16 j + fr]
-  bf16_t* Y = reinterpret_cast<bf16_t*>(p.y);
-  if constexpr (EPI == SK_SWIGLU) {
-#pragma unroll
-    for (int j = 0; j < FM; ++j) {
-      const int m = m0 + wm * TM + 16 * j + fr;
-      if (m >= M) continue;
-#pragma unroll
-      for (int i = 0; i < FN / 2; ++i) {
-        const int f = (n0 >> 1) + wn * (TN / 2) + 16 * i + 4 * fq;
-        float o[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float g = bf2f(f2bf(acc[i][j][r])), u = bf2f(f2bf(acc[i + FN / 2][j][r]));
-          o[r] = g / (1.f + __expf(-g)) * u;
-        }
-        *reinterpret_cast<uint2*>(Y + (size_t)m * p.ldy + f) =
-            make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
-      }
-    }
-  } else if constexpr (EPI == SK_RESID) {
-    float4 bv[FN];
-#pragma unroll
-    for (int i = 0; i < FN; ++i) {
-      const int n = n0 + wn * TN + 16 * i + 4 * fq;
-      bv[i] = p.bias ? *reinterpret_cast<const float4*>(p.bias + n) : make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-#pragma unroll
-    for (int j = 0; j < FM; ++j) {
-      const int m = m0 + wm * TM + 16 * j + fr;
-      if (m >= M) continue;
-#pragma unroll
-      for (int i = 0; i < FN; ++i) {
-        const int n = n0 + wn * TN + 16 * i + 4 * fq;
-        uint2* yp = reinterpret_cast<uint2*>(Y + (size_t)m * p.ldy + n);
-        const uint2 rv = *yp;
-        const float o0 = bf2f(rv.x & 0xffff) + (acc[i][j][0] + bv[i].x);
-        const float o1 = bf2f(rv.x >> 16) + (acc[i][j][1] + bv[i].y);
-        const float o2 = bf2f(rv.y & 0xffff) + (acc[i][j][2] + bv[i].z);
-        const float o3 = bf2f(rv.y >> 16) + (acc[i][j][3] + bv[i].w);
-        *yp = make_uint2(pack_bf16x2(o0, o1), pack_bf16x2(o2, o3));
-      }
-    }
-  } else {
-    float4 bv[FN];
-#pragma unroll
-    for (int i = 0; i < FN; ++i) {
-      const int n = n0 + wn * TN + 16 * i + 4 * fq;
-      bv[i] = p.bias ? *reinterpret_cast<const float4*>(p.bias + n) : make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-#pragma unroll
-    for (int j = 0; j < FM; ++j) {
-      const int m = m0 + wm * TM + 16 * j + fr;
-      if (m >= M) continue;
-#pragma unroll
-      for (int i = 0; i < FN; ++i) {
-        const int n = n0 + wn * TN + 16 * i + 4 * fq;
-        float o[4] = {acc[i][j][0] + bv[i].x, acc[i][j][1] + bv[i].y, acc[i][j][2] + bv[i].z,
-                      acc[i][j][3] + bv[i].w};
-        if (p.act == 1) {
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const float v = bf2f(f2bf(o[r]));
-            o[r] = 0.5f * v * (1.f + erff(v * 0.70710678118654752f));
-          }
-        }
-        *reinterpret_cast<uint2*>(Y + (size_t)m * p.ldy + n) =
-            make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
-      }
-    }
-  }
+  if (S > 1 && !sk_reduce<NW, FN, FM>(p, acc, tile, s, wave, lane, reinterpret_cast<int*>(lds))) return;
+  sk_epilogue<EPI, FN, FM>(p, acc, n0 + wn * TN, (n0 >> 1) + wn * (TN / 2), m0 + wm * TM, fr, fq);
 }
 
 template <int WN, int WM, int FN, int FM, int NBUF>
@@ -335,21 +197,11 @@ static int sk_launch(const GemmSkParams& p, hipStream_t st) {
   return (int)hipGetLastError();
 }
 
-// layout -> (features BN x rows BM, waves, stages):
-//   0: 128 x 128, 2 x 2 waves of 64 x 64, 2 stages (64 KB LDS)
-//   1: 128 x  64, 2 x 2 waves of 64 x 32, 2 stages (48 KB)
-//   2: 256 x  64, 4 x 1 waves of 64 x 64, 2 stages (80 KB)
-//   3: 256 x 128, 4 x 2 waves of 64 x 64, 2 stages (96 KB)
-//   4: 128 x  64, 3 stages (72 KB)
-//   5: 128 x 128, 3 stages (96 KB)
-//   6: 256 x 256, 2 x 4 waves of 128 x 64, 2 stages (128 KB)
-//   7:  64 x  64, 2 x 2 waves of 32 x 32, 2 stages (32 KB)
-//   8: 256 x  64, 3 stages (120 KB)
-//   9: 256 x 128, 3 stages (144 KB): two 48 KB stages in flight per CU
-//  10: 128 x 128, 4 stages (128 KB)
-//  11: 128 x  64, 4 stages (96 KB)
-// (short-K shapes - the Whisper encoder's K = 1280, 20 stages - are bound by
-// the bytes one CU keeps in flight: a deeper ring is the lever there)
+int gemm_pipe(const GemmSkParams& p, int layout, hipStream_t st);   // gemm_pipe.hip
+
+// layout: 1: 128 x 64 (2 x 2 waves of 64 x 32), 7: 64 x 64 (2 x 2 waves of 32 x 32), two
+// stages each - the general forms, for feature counts that are no multiple of 128 and rows
+// that are not 16-byte aligned; 12 on: the pipelined tiles of gemm_pipe.hip
 extern "C" int loqa_gemm_sk(const GemmSkParams* p, hipStream_t st) {
   if (!p || p->M <= 0 || p->S < 1 || p->epi < 0 || p->epi > 2 || !p->x || !p->w || !p->y)
     return (int)hipErrorInvalidValue;
@@ -357,29 +209,8 @@ extern "C" int loqa_gemm_sk(const GemmSkParams* p, hipStream_t st) {
   if (p->ldx % 8 || p->ldy % 4) return (int)hipErrorInvalidValue;
   if ((p->epi == SK_SWIGLU && p->bias) || (p->epi != SK_BF16 && p->act)) return (int)hipErrorInvalidValue;
   switch (p->layout) {
-    case 0: return sk_launch<2, 2, 4, 4, 2>(*p, st);
     case 1: return sk_launch<2, 2, 4, 2, 2>(*p, st);
-    case 2: return sk_launch<4, 1, 4, 4, 2>(*p, st);
-    case 3: return sk_launch<4, 2, 4, 4, 2>(*p, st);
-    case 4: return sk_launch<2, 2, 4, 2, 3>(*p, st);
-    case 5: return sk_launch<2, 2, 4, 4, 3>(*p, st);
-    case 6: return sk_launch<2, 4, 8, 4, 2>(*p, st);
     case 7: return sk_launch<2, 2, 2, 2, 2>(*p, st);
-    case 8: return sk_launch<4, 1, 4, 4, 3>(*p, st);
-    case 9: return sk_launch<4, 2, 4, 4, 3>(*p, st);
-    case 10: return sk_launch<2, 2, 4, 4, 4>(*p, st);
-    case 11: return sk_launch<2, 2, 4, 2, 4>(*p, st);
-    default: return (int)hipErrorInvalidValue;
+    default: return gemm_pipe(*p, p->layout - 12, st);
   }
-}
-
-// tile geometry of a layout (features, rows) for the host-side planner
-extern "C" int loqa_gemm_sk_dims(int layout, int* bn, int* bm) {
-  static const int dims[12][2] = {{128, 128}, {128, 64}, {256, 64}, {256, 128}, {128, 64},
-                                  {128, 128}, {256, 256}, {64, 64}, {256, 64}, {256, 128},
-                                  {128, 128}, {128, 64}};
-  if (layout < 0 || layout > 11) return (int)hipErrorInvalidValue;
-  *bn = dims[layout][0];
-  *bm = dims[layout][1];
-  return 0;
 }

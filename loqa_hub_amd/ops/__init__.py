@@ -1625,57 +1625,40 @@ def gemm_tile(x: torch.Tensor, w: torch.Tensor, *, bias: torch.Tensor | None = N
 
 
 # ---------------------------------------------------------------------------
-# Split-K tiled GEMM with an in-launch reduction (csrc/kernels/gemm_sk.hip)
+# Split-K tiled GEMM with an in-launch reduction (csrc/kernels/gemm_sk.hip, gemm_pipe.hip)
 _SK_EPI = {"bf16": 0, "swiglu": 1, "resid": 2}
-# layout -> (features, rows, resident workgroups per CU (LDS), per-CU efficiency)
-# efficiency: relative MFMA rate of the wave tile (LDS bytes per MFMA: 64 x 64
-# = 1.0; 64 x 32 tiles read 1.5x the LDS per MFMA; 128 x 64 0.75x)
-SK_LAYOUTS = {0: (128, 128, 2, 1.0), 1: (128, 64, 3, 0.85), 2: (256, 64, 2, 1.0),
-              3: (256, 128, 1, 1.0), 4: (128, 64, 2, 0.9), 5: (128, 128, 1, 1.05),
-              6: (256, 256, 1, 1.15), 7: (64, 64, 4, 0.6), 8: (256, 64, 1, 1.05),
-              9: (256, 128, 1, 1.1), 10: (128, 128, 1, 1.1), 11: (128, 64, 1, 0.95)}
+# layout -> (features, rows, us a K step of 64 takes a compute unit, us around a tile's K
+# loop): 1 and 7 are the general form, 12 on the pipelined tiles, one workgroup per CU. The
+# times are fitted to 77 measured shapes (80 to 3000 rows, N 1280 to 28672, K 1280 to 14336,
+# cold weights, 1 to 8 K chunks): the plan they give is within 1 % of the fastest layout on
+# average, within 13 % at worst.
+SK_LAYOUTS = {1: (128, 64, 0.60, 4.0), 7: (64, 64, 0.55, 4.0),
+              12: (256, 256, 1.20, 10.3), 13: (256, 192, 1.075, 5.5), 14: (192, 256, 1.073, 5.5),
+              15: (256, 128, 0.908, 4.0), 16: (128, 256, 0.784, 6.6), 17: (128, 192, 0.667, 4.6),
+              18: (192, 192, 0.854, 4.6), 19: (128, 64, 0.309, 4.3), 20: (128, 128, 0.498, 3.6)}
+SK_PIPE = 12              # the first pipelined layout
 SK_CUS = 256
 _SK_WS: dict = {}
 
 
-# measured picks (scripts/exp/gemm_sk_bench.py --grid, cold weights, one
-# MI355X; profiles/r4_gemm_sk_grid.txt): (N, K) -> [(max M, layout, chunks)]
-SK_TABLE = {
-    (6144, 4096): [(400, 4, 1), (900, 5, 1), (1 << 30, 0, 1)],        # Llama-3-8B qkv
-    (4096, 4096): [(900, 4, 1), (1 << 30, 1, 1)],                     # o
-    (28672, 4096): [(400, 4, 1), (1 << 30, 0, 1)],                    # gate|up
-    (4096, 14336): [(400, 8, 3), (900, 0, 3), (1 << 30, 0, 1)],       # down
-    (3840, 1280): [(1 << 30, 0, 1)],                                  # Whisper-large-v3 enc qkv
-    (1280, 1280): [(2000, 4, 1), (4000, 5, 1), (1 << 30, 3, 1)],      # enc o
-    (5120, 1280): [(1 << 30, 0, 1)],                                  # enc fc1
-    (1280, 5120): [(2000, 4, 1), (4000, 5, 1), (1 << 30, 0, 1)],      # enc fc2
-}
-
-
-def gemm_sk_plan(M: int, N: int, K: int, epi: str = "bf16",
-                 layouts=(0, 1, 2, 3, 4, 5)) -> tuple[int, int]:
-    """(layout, K chunks) for a shape: the measured table for the served
-    shapes, else an analytic plan - the fewest
-    MFMA-cycle rounds over the resident workgroup slots, counting padded rows
-    and wave-tile efficiency, with at most 3 K chunks (each chunk's partial
-    costs a write and a serial read in the reduction: 16 chunks measured up
-    to 7x slower than 1)."""
-    for m_max, lay, s in SK_TABLE.get((N, K), ()):
-        if M <= m_max and N % SK_LAYOUTS[lay][0] == 0:
-            return lay, s
+def gemm_sk_plan(M: int, N: int, K: int, epi: str = "bf16", pipe: bool = True) -> tuple[int, int]:
+    """(layout, K chunks) for a shape: the fewest microseconds by SK_LAYOUTS, counting whole
+    rounds of tiles over the compute units. K chunks fill the chip where the tiles do not;
+    each costs a write and a serial read of the tile's f32 partial (6 us, and 37 us a MB per
+    chunk, fitted with the rest), so they pay for few rows and long K only. ``pipe`` False:
+    the general layouts only (operands the pipelined tiles do not take)."""
     KT = K // 64
     best, best_t = (7, 1), float("inf")
-    for lay in layouts:
-        bn, bm, occ, eff = SK_LAYOUTS[lay]
-        if N % bn:
+    for lay, (bn, bm, step, around) in SK_LAYOUTS.items():
+        if N % bn or (lay >= SK_PIPE) != (pipe and N % 128 == 0):
             continue
         tiles = -(-M // bm) * (N // bn)
-        for s in (1, 2, 3):
-            if s > KT or (s > 1 and KT // s < 8) or (epi == "swiglu" and s > 1):
+        for s in (1, 2, 3, 4, 6, 8):
+            if s > 1 and KT // s < 8:
                 continue
-            grid = tiles * s
-            rounds = -(-grid // (SK_CUS * occ))
-            t = rounds * occ * bm * bn * (KT / s) / eff + (s - 1) * bm * bn * 64.0
+            t = -(-tiles * s // SK_CUS) * (-(-KT // s) * step + around)
+            if s > 1:
+                t += 6.3 + s * bn * bm * 4 / 27e3
             if t < best_t:
                 best, best_t = (lay, s), t
     return best
@@ -1751,8 +1734,13 @@ def gemm_sk(x: torch.Tensor, w: torch.Tensor, *, epi: str = "bf16", bias: torch.
         raise TypeError("gemm_sk needs bf16 operands")
     if x.stride(1) != 1 or not w.is_contiguous():
         raise ValueError("gemm_sk needs K-contiguous operands")
+    y = residual if epi == "resid" else out
     if layout is None or splits is None:
-        pl, ps = gemm_sk_plan(M, N, K, epi)
+        # the pipelined tiles move whole 16-byte pieces of the rows at 32-bit offsets
+        pipe = x.stride(0) >= K and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 \
+            and N * K < 1 << 31 and x.stride(0) < 1 << 21 \
+            and (y is None or (y.stride(0) % 8 == 0 and y.data_ptr() % 16 == 0))
+        pl, ps = gemm_sk_plan(M, N, K, epi, pipe)
         layout = pl if layout is None else layout
         splits = ps if splits is None else splits
     bn, bm = SK_LAYOUTS[layout][:2]
@@ -1851,87 +1839,9 @@ def gemm_ws(x: torch.Tensor, w: torch.Tensor, *, epi: str = "bf16", bias: torch.
 
 
 # ---------------------------------------------------------------------------
-# Projection dispatch for prompt passes (prefill, Whisper encoder): the
-# hand-written GEMM measured fastest per (N, K) and row count
-# (scripts/exp/gemm_sk_bench.py --grid, cold weights; profiles/r4_gemm_proj_grid.txt):
-# ("sk", layout, K chunks) = gemm_sk, ("ws", depth[, K chunks]) = gemm_ws.
-PROJ_TABLE = {
-    # the chunked prompt passes (LOQA_CHUNK_PREFILL) also run 64-256 rows:
-    # more K chunks fill the CUs there (profiles/r4_gemm_small_m.txt; a 32 /
-    # 128-row pass 4.81 / 6.33 vs 6.70 / 7.21 ms, headline neutral:
-    # profiles/r4_ab_proj_small_m.txt)
-    (6144, 4096): [(64, ("sk", 4, 4)), (128, ("sk", 4, 2)), (400, ("sk", 4, 1)),
-                   (900, ("sk", 5, 1)), (1 << 30, ("sk", 0, 1))],                         # Llama qkv
-    (4096, 4096): [(128, ("sk", 4, 4)), (256, ("sk", 4, 2)), (900, ("sk", 4, 1)),
-                   (1 << 30, ("sk", 0, 1))],                                               # o
-    (28672, 4096): [(256, ("ws", 1)), (384, ("ws", 0)), (900, ("ws", 0)),
-                    (1 << 30, ("sk", 6, 1))],                                              # gate|up
-    # 400-1000 rows (whole-prompt passes of two or three prompts, nothing
-    # decoding): down on the weight-streaming GEMM with K chunks, gate|up on it
-    # unsplit (600 rows: 94 vs 118 us, 160 vs 196 us; profiles/r4_ws_splitk.txt).
-    # At 300-400 rows, the chunked passes beside the Whisper decoder, the split-K
-    # weight-streaming down too: round 4's 3 pairs read neutral (19.03 vs 19.07),
-    # round 5's 5 interleaved pairs all favour it - mixed pass 13.0 -> 12.4 ms,
-    # +1.2% utt/s (profiles/r5_ab_down_ws.txt)
-    (4096, 14336): [(64, ("sk", 4, 8)), (128, ("sk", 5, 8)), (256, ("sk", 5, 4)),
-                    (400, ("ws", 0, 4)), (700, ("ws", 0, 4)), (1000, ("ws", 0, 2)),
-                    (1 << 30, ("sk", 6, 3))],                                              # down
-    # encoder qkv / fc1: gemm_ws is ~8% faster alone (24.2 / 25.8 vs 26.2 / 28.2
-    # us) but its long-lived 512-thread workgroups cost the concurrent decoders
-    # more than that (encoder on ws: 18.82 / 19.02 vs 19.15 / 18.99 utt/s)
-    (3840, 1280): [(2000, ("sk", 1, 1)), (1 << 30, ("sk", 6, 1))],                        # enc qkv
-    (1280, 1280): [(2000, ("sk", 4, 1)), (1 << 30, ("sk", 5, 1))],                        # enc o
-    (5120, 1280): [(2000, ("sk", 0, 1)), (1 << 30, ("sk", 6, 1))],                        # enc fc1
-    (1280, 5120): [(2000, ("sk", 4, 1)), (1 << 30, ("sk", 5, 1))],                        # enc fc2
-    # Llama-3-70B TP=8 shards, prompt passes of ~320 rows (grid search,
-    # profiles/r5_tp70_shard_grid.jsonl): the planner's (4, 2) / (5, 1) picks
-    # were 38.1 / 85.3 us, these 27.2 / 69.7 us (hipBLASLt 28.1 / 69.8); o and
-    # down shards keep the planner's (5, 1) (15.2 / 37.6 us)
-    # deeper LDS rings (layouts 9 / 11, profiles/r5_sk_grid_deep.jsonl): 25.6 /
-    # 62.9 us vs 26.9 / 68.9 (a TP rank runs no decoder beside its prompt pass)
-    (1280, 8192): [(512, ("sk", 11, 4))],                                                  # qkv/8
-    (7168, 8192): [(512, ("sk", 9, 3))],                                                   # gate|up/8
-}
-# the 8B prompt-pass projections at ~300 rows on the 4-stage rings (qkv 32.7 ->
-# 30.3, o 32.0 -> 30.2, down 76.3 -> 73.4 us alone; one workgroup per CU
-# instead of two beside the decoders): LOQA_SK_DEEP
-SK_DEEP = os.environ.get("LOQA_SK_DEEP", "0") == "1"
-# experiment override of the <= 400-row (chunked prompt pass) pick of a shape:
-# "NxK:sk,layout,chunks;NxK:ws,depth,chunks"
-for _ov in filter(None, os.environ.get("LOQA_PROJ_OVERRIDE", "").split(";")):
-    try:
-        _shape, _pick = _ov.split(":")
-        _n, _k = map(int, _shape.split("x"))
-        _kind, *_args = _pick.split(",")
-        if _kind not in ("sk", "ws"):
-            raise ValueError(_kind)
-        PROJ_TABLE[(_n, _k)] = [(400, (_kind, *map(int, _args)))] + [
-            e for e in PROJ_TABLE.get((_n, _k), []) if e[0] > 400]
-    except ValueError:
-        import warnings
-        warnings.warn(f"LOQA_PROJ_OVERRIDE: ignoring malformed entry {_ov!r}")
-if SK_DEEP:
-    PROJ_TABLE[(6144, 4096)].insert(2, (400, ("sk", 11, 1)))
-    PROJ_TABLE[(4096, 4096)].insert(2, (400, ("sk", 11, 1)))
-    PROJ_TABLE[(4096, 14336)][3] = (400, ("sk", 9, 4))
-
-
+# Projections of prompt passes (prefill, Whisper encoder)
 def proj(x: torch.Tensor, w: torch.Tensor, *, epi: str = "bf16", bias: torch.Tensor | None = None,
          act: str | None = None, residual: torch.Tensor | None = None) -> torch.Tensor:
-    """A prompt-pass projection on the fastest hand-written GEMM for its shape
-    (``PROJ_TABLE``; shapes outside it: the gemm_sk planner). Epilogues as
-    :func:`gemm_sk`."""
-    M = x.shape[0]
-    N, K = w.shape
-    choice = None
-    for m_max, c in PROJ_TABLE.get((N, K), ()):
-        if M <= m_max:
-            choice = c
-            break
-    if choice is not None and choice[0] == "ws" and N % 128 == 0:
-        return gemm_ws(x, w, epi=epi, bias=bias, act=act, residual=residual, depth=choice[1],
-                       splits=choice[2] if len(choice) > 2 else 1)
-    if choice is not None and choice[0] == "sk" and N % SK_LAYOUTS[choice[1]][0] == 0:
-        return gemm_sk(x, w, epi=epi, bias=bias, act=act, residual=residual, layout=choice[1],
-                       splits=choice[2])
+    """A prompt-pass projection: :func:`gemm_sk` with the layout and K chunks its plan gives
+    for the shape."""
     return gemm_sk(x, w, epi=epi, bias=bias, act=act, residual=residual)

@@ -1,0 +1,78 @@
+"""The pipelined tiles behind ops.gemm_sk (csrc/kernels/gemm_pipe.hip): which operands they
+take, the edges of tiles and rings, and GELU at the ends of its range."""
+import pytest
+import torch
+
+from loqa_hub_amd import ops
+
+
+def _close(a, b, k):
+    # a bf16 result of an f32 sum of k products: half an ulp (2^-9) of the value, and the sum's
+    # own rounding, at most k 2^-24 of the magnitudes added (bounded by 4 sigma of the sum)
+    tol = 2.0 ** -8 * b.abs() + (k * 2.0 ** -22 + 2.0 ** -9) * b.std()
+    assert torch.all((a.double() - b).abs() <= tol), ((a.double() - b).abs() - tol).max().item()
+
+
+def test_plan_takes_the_general_layouts_where_the_tiles_do_not_fit():
+    for M, N, K in ((1, 64, 64), (300, 192, 256), (5000, 4160, 512)):
+        assert N % 128 and ops.gemm_sk_plan(M, N, K)[0] == 7
+    for M in (1, 64, 65, 320, 2048, 9000):
+        for N, K in ((1280, 5120), (6144, 4096), (128, 64), (28672, 4096)):
+            assert ops.gemm_sk_plan(M, N, K, pipe=False)[0] in (1, 7)
+            lay, s = ops.gemm_sk_plan(M, N, K)
+            assert lay >= ops.SK_PIPE and N % ops.SK_LAYOUTS[lay][0] == 0
+            assert s == 1 or K // 64 // s >= 8
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", [k for k in sorted(ops.SK_LAYOUTS) if k >= ops.SK_PIPE])
+@pytest.mark.parametrize("stages", [1, 2, 3, 7])
+def test_short_k_and_ragged_rows(layout, stages):
+    """Fewer K steps than the rings hold, rows around the tile's edge, rows wider than K, and
+    an output that is a column block of a wider matrix."""
+    bn, bm = ops.SK_LAYOUTS[layout][:2]
+    K = 64 * stages
+    g = torch.Generator().manual_seed(layout)
+    for M in (1, bm - 1, bm, bm + 1):
+        x = torch.randn(M, K + 24, generator=g).bfloat16().cuda()[:, 8:8 + K]
+        w = torch.randn(2 * bn, K, generator=g).bfloat16().cuda()
+        ref = x.double() @ w.double().t()
+        wide = torch.full((M, 2 * bn + 64), 7.0, dtype=torch.bfloat16, device="cuda")
+        y = ops.gemm_sk(x, w, layout=layout, splits=1, out=wide[:, 32:32 + 2 * bn])
+        _close(y, ref, K)
+        assert (wide[:, :32] == 7).all() and (wide[:, 32 + 2 * bn:] == 7).all()
+        res = torch.randn(M, 2 * bn, generator=g).bfloat16().cuda()
+        want = res.double() + ref
+        _close(ops.gemm_sk(x, w, epi="resid", residual=res, layout=layout, splits=stages), want, K)
+        h = ref[:, :bn]
+        _close(ops.gemm_sk(x, w, epi="swiglu", layout=layout, splits=1), h * torch.sigmoid(h) * ref[:, bn:], K)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("epi", ["bf16", "resid", "swiglu"])
+def test_rows_that_are_not_16_byte_aligned(epi):
+    """Output rows 8 bytes apart from alignment take the general form: same result."""
+    g = torch.Generator().manual_seed(3)
+    x, w = torch.randn(150, 256, generator=g).bfloat16().cuda(), torch.randn(256, 256, generator=g).bfloat16().cuda()
+    n = 128 if epi == "swiglu" else 256
+    want = ops.gemm_sk(x, w, epi=epi, residual=torch.zeros(150, 256, dtype=torch.bfloat16, device="cuda") if epi == "resid" else None)
+    wide = torch.zeros(150, n + 4, dtype=torch.bfloat16, device="cuda")
+    y = ops.gemm_sk(x, w, epi=epi, residual=wide[:, :n] if epi == "resid" else None, out=None if epi == "resid" else wide[:, :n])
+    _close(y, want.double(), 256)
+
+
+@pytest.mark.gpu
+def test_gelu_over_its_whole_range():
+    """gelu(b) for biases from the far negative tail to the largest finite value, and the
+    infinities and NaN as 0.5 v (1 + erf(v / sqrt 2)) gives them."""
+    b = torch.cat([torch.linspace(-8, 8, 1021), torch.tensor([3e38, 1e20, -1e20])]).cuda()
+    x, w = torch.zeros(3, 64, dtype=torch.bfloat16, device="cuda"), torch.zeros(1024, 64, dtype=torch.bfloat16, device="cuda")
+    y = ops.gemm_sk(x, w, bias=b, act="gelu")[1].double()
+    v = b.double()
+    want = 0.5 * v * torch.special.erfc(-v / 2 ** 0.5)
+    # the rational form's 1.5e-7 times |v| / 2, and bf16's half ulp
+    assert torch.all((y - want).abs() <= 2.0 ** -8 * want.abs() + 1e-7 * v.abs().clamp(max=16))
+    edge = torch.full((128,), float("inf"), device="cuda")
+    edge[1], edge[2] = -float("inf"), float("nan")
+    got = ops.gemm_sk(x, w[:128], bias=edge, act="gelu")[0]
+    assert got[0] == float("inf") and got[1].isnan() and got[2].isnan()
