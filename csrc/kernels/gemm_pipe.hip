@@ -28,100 +28,9 @@
 // 12 tile edges pass its L2 per K step instead of 33 (8192^3: 1290 -> 1365 TFLOP/s against
 // groups of 8).
 #include "gemm_sk.h"
+#include "gemm_pipe.h"
 
 #define GP_GROUP 4
-
-// In place, on the accumulation registers: left to the register allocator, the builtin's
-// result and addend part ways and every MFMA is followed by register moves. Nothing but
-// other MFMAs, FN FM issues away, touches the accumulators inside the loop.
-__device__ __forceinline__ void gp_mfma(float4v& c, const bf16x8& a, const bf16x8& b) {
-  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
-}
-
-// 16 bytes per lane of [base, base + bytes) at off + soff, straight into LDS (lane l at
-// dst + 16 l); out of range reads as zero.
-__device__ __forceinline__ void gp_load_lds(const bf16_t* base, unsigned bytes, unsigned char* dst, unsigned off,
-                                            unsigned soff) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(base), 0, bytes, 0x00020000),
-      (__attribute__((address_space(3))) void*)dst, 16, off, soff, 0, 0);
-}
-
-// workgroups per CU by LDS
-template <int FN, int FM, int NA, int NB> constexpr int gp_per_cu() {
-  return 160 * 1024 / ((NA * FN + NB * FM) * 32 * 128);
-}
-
-// Epilogue of one wave through its own part of LDS. The accumulators of an MFMA tile hold
-// four neighbouring features of one row per lane, so storing them directly makes every
-// 8-byte piece of an instruction a line of its own (9000 x 3840 x 1280: 26 of 96 us went
-// into the stores, 38 with the residual's loads). Instead the finished bf16 pieces go to
-// LDS and leave as whole rows, 16 bytes a lane; the residual comes in the same way.
-template <int EPI, int FN, int FM>
-__device__ __forceinline__ void gp_epilogue(const GemmSkParams& p, float4v (&acc)[FN][FM], unsigned char* my, int nw,
-                                            int fw, int mw, int lane) {
-  constexpr int ON = EPI == SK_SWIGLU ? 8 * FN : 16 * FN;   // output features of the wave
-  constexpr int LD = ON * 2 + 16;                           // bytes of a row in LDS
-  constexpr int CPR = ON / 8;                               // 16-byte chunks of a row
-  constexpr int CH = 16 * FM * CPR / 64;                    // chunks per lane
-  static_assert(CH * 64 == 16 * FM * CPR, "chunks must split evenly over the lanes");
-  typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-  const int fr = lane & 15, fq = lane >> 4;
-  bf16_t* Y = reinterpret_cast<bf16_t*>(p.y) + (EPI == SK_SWIGLU ? fw : nw);
-  const int rows = p.M - mw;                                // rows of the wave's tile that exist
-  if constexpr (EPI == SK_RESID) {
-    u32x4 v[CH];
-#pragma unroll
-    for (int k = 0; k < CH; ++k) {
-      const int id = lane + 64 * k, r = min(id / CPR, rows - 1), c = id % CPR;
-      if (rows > 0) v[k] = *reinterpret_cast<const u32x4*>(Y + (size_t)(mw + r) * p.ldy + c * 8);
-    }
-#pragma unroll
-    for (int k = 0; k < CH; ++k) {
-      const int id = lane + 64 * k;
-      *reinterpret_cast<u32x4*>(my + (id / CPR) * LD + (id % CPR) * 16) = v[k];
-    }
-  }
-  float4 bv[FN];
-  if constexpr (EPI != SK_SWIGLU)
-#pragma unroll
-    for (int i = 0; i < FN; ++i)
-      bv[i] = p.bias ? *reinterpret_cast<const float4*>(p.bias + nw + 16 * i + 4 * fq) : make_float4(0.f, 0.f, 0.f, 0.f);
-  __builtin_amdgcn_wave_barrier();
-#pragma unroll
-  for (int j = 0; j < FM; ++j) {
-    unsigned char* row = my + (16 * j + fr) * LD + fq * 8;
-#pragma unroll
-    for (int i = 0; i < (EPI == SK_SWIGLU ? FN / 2 : FN); ++i) {
-      uint2* at = reinterpret_cast<uint2*>(row + i * 32);
-      float o[4];
-      if constexpr (EPI == SK_SWIGLU) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) o[r] = sk_swiglu(acc[i][j][r], acc[i + FN / 2][j][r]);
-      } else {
-        o[0] = acc[i][j][0] + bv[i].x; o[1] = acc[i][j][1] + bv[i].y;
-        o[2] = acc[i][j][2] + bv[i].z; o[3] = acc[i][j][3] + bv[i].w;
-        if constexpr (EPI == SK_RESID) {
-          const uint2 rv = *at;
-          o[0] += bf2f(rv.x & 0xffff); o[1] += bf2f(rv.x >> 16);
-          o[2] += bf2f(rv.y & 0xffff); o[3] += bf2f(rv.y >> 16);
-        } else if (p.act == 1) {
-#pragma unroll
-          for (int r = 0; r < 4; ++r) o[r] = sk_gelu(o[r]);
-        }
-      }
-      *at = make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
-    }
-    __builtin_amdgcn_sched_barrier(0);   // a row block's accumulators at a time
-  }
-  __builtin_amdgcn_wave_barrier();
-#pragma unroll
-  for (int k = 0; k < CH; ++k) {
-    const int id = lane + 64 * k, r = id / CPR, c = id % CPR;
-    const u32x4 v = *reinterpret_cast<const u32x4*>(my + r * LD + c * 16);
-    if (r < rows) *reinterpret_cast<u32x4*>(Y + (size_t)(mw + r) * p.ldy + c * 8) = v;
-  }
-}
 
 template <int FN, int FM, int NA, int NB, int EPI>
 __global__ __launch_bounds__(256, (gp_per_cu<FN, FM, NA, NB>())) void gemm_pipe_kernel(GemmSkParams p) {
@@ -131,7 +40,7 @@ __global__ __launch_bounds__(256, (gp_per_cu<FN, FM, NA, NB>())) void gemm_pipe_
   constexpr int IA = BN / 8 / NW, IB = BM / 8 / NW;   // 1 KB direct-to-LDS loads per wave and stage
   static_assert(IA * 8 * NW == BN && IB * 8 * NW == BM, "rows must split evenly over the waves");
   constexpr int XRING = NA * BN * 128;                // where the ring of X stages starts
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[XRING + NB * BM * 128];
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[gp_lds_bytes<FN, FM, NA, NB>()];
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -186,87 +95,36 @@ __global__ __launch_bounds__(256, (gp_per_cu<FN, FM, NA, NB>())) void gemm_pipe_
                 on ? t * (SK_BK * 2) : 0);
   };
 
-  const int fr = lane & 15, fq = lane >> 4;
-  // a fragment's place: rows 16 i apart keep the swizzle, the other K half is 64 bytes away
-  const int swz = 16 * (fq ^ ((fr >> 1) & 7));
-  const int abase = (wn * TN + fr) * 128 + swz, bbase = XRING + (wm * TM + fr) * 128 + swz;
   float4v acc[FN][FM];
-#pragma unroll
-  for (int i = 0; i < FN; ++i)
-#pragma unroll
-    for (int j = 0; j < FM; ++j) {
-      acc[i][j] = float4v{0.f, 0.f, 0.f, 0.f};
-      asm volatile("" : "+a"(acc[i][j]));
-    }
-  bf16x8 af[2][FN], bfr[2][FM];
-  // read q (0 .. FN + FM - 1) of a K half into its register set
-  auto read = [&](int q, int sa, int sb, int half) {
-    if (q < FM)
-      bfr[half][q] = *reinterpret_cast<const bf16x8*>(lds + sb * (BM * 128) + ((bbase ^ (64 * half)) + q * 2048));
-    else
-      af[half][q - FM] = *reinterpret_cast<const bf16x8*>(lds + sa * (BN * 128) + ((abase ^ (64 * half)) + (q - FM) * 2048));
-  };
-  constexpr int MF = FN * FM, R = FN + FM;
-  constexpr int SPAN = MF * 7 / 8;                 // reads are spread over this many MFMAs
-  // loads issued behind those of stage t + 1 when it is waited for in the middle of stage t
-  constexpr int BEHIND_W = (NA - 2) * (IA + IB), BEHIND_X = (NB - 1) * IA + (NB - 2) * IB;
-  constexpr int BEHIND = BEHIND_W < BEHIND_X ? BEHIND_W : BEHIND_X;
-
-#pragma unroll
-  for (int q = 0; q < NB || q < NA - 1; ++q) {
-#pragma unroll
-    for (int i = 0; i < IA; ++i)
-      if (q < NA - 1) load_w(i, q, q);
-#pragma unroll
-    for (int i = 0; i < IB; ++i)
-      if (q < NB) load_x(i, q, q);
-  }
-  sk_wait_vm<(NA - 2) * IA + (NB - 1) * IB>();     // stage 0 is here
-  __builtin_amdgcn_s_barrier();
-#pragma unroll
-  for (int q = 0; q < R; ++q) read(q, 0, 0, 0);
-  int sa = 0, sb = 0;                              // ring slots of stage t
-  for (int t = 0; t < nt; ++t) {
-    const int sp = sa == 0 ? NA - 1 : sa - 1;      // freed in the middle of stage t - 1
-#pragma unroll
-    for (int x = 0; x < MF; ++x) {
-      gp_mfma(acc[x / FM][x % FM], af[0][x / FM], bfr[0][x % FM]);
-#pragma unroll
-      for (int q = x * R / SPAN; q < (x + 1) * R / SPAN && q < R; ++q) read(q, sa, sb, 1);
-#pragma unroll
-      for (int q = x * IA / MF; q < (x + 1) * IA / MF; ++q) load_w(q, sp, t + NA - 1);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // this wave has read all of stage t,
-    sk_wait_vm<BEHIND>();                                // and its part of t + 1 has landed
-    __builtin_amdgcn_s_barrier();
-    const int na = sa + 1 == NA ? 0 : sa + 1, nb2 = sb + 1 == NB ? 0 : sb + 1;
-#pragma unroll
-    for (int x = 0; x < MF; ++x) {
-      gp_mfma(acc[x / FM][x % FM], af[1][x / FM], bfr[1][x % FM]);
-#pragma unroll
-      for (int q = x * R / SPAN; q < (x + 1) * R / SPAN && q < R; ++q) read(q, na, nb2, 0);
-#pragma unroll
-      for (int q = x * IB / MF; q < (x + 1) * IB / MF; ++q) load_x(q, sb, t + NB);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    sa = na;
-    sb = nb2;
-  }
-  // no load into LDS outlives the loop; the last MFMAs' results are 16 cycles away from
-  // being readable, and only this wait tells the compiler's moves so
-  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n s_nop 15\n s_nop 15" ::: "memory");
-#pragma unroll
-  for (int i = 0; i < FN; ++i)
-#pragma unroll
-    for (int j = 0; j < FM; ++j) asm volatile("" : "+a"(acc[i][j]));
+  gp_loop<FN, FM, NA, NB>(acc, lds, nt, wn, wm, lane, load_w, load_x);
 
   if (S > 1 && !sk_reduce<NW, FN, FM>(p, acc, tile, s, wave, lane, reinterpret_cast<int*>(lds))) return;
   // every wave has read its last fragments, every load has landed: the rings are free
   constexpr int WAVE_LDS = TM * (TN * 2 + 16);
   static_assert(WAVE_LDS * NW <= XRING + NB * BM * 128, "the epilogue's rows must fit the rings");
   __syncthreads();
-  gp_epilogue<EPI, FN, FM>(p, acc, lds + wave * WAVE_LDS, n0 + wn * TN, (n0 >> 1) + wn * (TN / 2), m0 + wm * TM, lane);
+  unsigned char* my = lds + wave * WAVE_LDS;
+  const int mw = m0 + wm * TM, nw = n0 + wn * TN, fq = lane >> 4;
+  bf16_t* Y = reinterpret_cast<bf16_t*>(p.y) + (size_t)mw * p.ldy;
+  if constexpr (EPI == SK_SWIGLU) {
+    gp_store<FN / 2, FM, false>(my, Y + (n0 >> 1) + wn * (TN / 2), p.ldy, M - mw, TN / 2, lane, [&](int i, int j, float* o) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[r] = sk_swiglu(acc[i][j][r], acc[i + FN / 2][j][r]);
+    });
+  } else {
+    float4v bv[FN];
+#pragma unroll
+    for (int i = 0; i < FN; ++i)
+      bv[i] = p.bias ? *reinterpret_cast<const float4v*>(p.bias + nw + 16 * i + 4 * fq) : float4v{0.f, 0.f, 0.f, 0.f};
+    const bool gelu = EPI == SK_BF16 && p.act == 1;
+    gp_store<FN, FM, EPI == SK_RESID>(my, Y + nw, p.ldy, M - mw, TN, lane, [&](int i, int j, float* o) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        o[r] += acc[i][j][r] + bv[i][r];
+        if (gelu) o[r] = sk_gelu(o[r]);
+      }
+    });
+  }
 }
 
 template <int FN, int FM, int NA, int NB>

@@ -88,7 +88,7 @@ SEQMIX_SOURCES = ("norm_dyt.hip", "attn_latent.hip", "attn_latent_prefill.hip", 
                   "moe.hip", "seq_rows.hip", "norm_scalar.hip", "attn_sigmoid.hip",
                   "norm_rms1p.hip", "attn_window.hip", "mamba2.hip", "matrix_memory.hip",
                   "delta_rule.hip", "norm_layer.hip", "linear_chunks.hip",
-                  "delta_chunks.hip")
+                  "delta_chunks.hip", "moe_pipe.hip")
 
 # hipcc may not form packed-f32 VALU instructions from scalar float code
 NO_PACKED_F32 = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
@@ -104,7 +104,7 @@ def build(force: bool = False, debug: bool = False, only=None, quiet: bool = Fal
     ksrc = [p for p in allk if os.path.basename(p) not in SEQMIX_SOURCES]
     allh = sorted(glob.glob(os.path.join(CSRC, "kernels", "*.h")))
     khdr = [p for p in allh if os.path.basename(p) != "seqmix.h"]
-    shdr = [p for p in allh if os.path.basename(p) in ("common.h", "seqmix.h")]
+    shdr = [p for p in allh if os.path.basename(p) in ("common.h", "seqmix.h", "gemm_pipe.h")]
     rsrc = sorted(glob.glob(os.path.join(CSRC, "runtime", "*.cpp")))
     rhdr = sorted(glob.glob(os.path.join(CSRC, "runtime", "*.h")))
     rflags = [*opt, "-std=c++17", "-D__HIP_PLATFORM_AMD__"]
