@@ -1,13 +1,19 @@
-// Whisper audio front-end on the GPU (SURVEY §2.4 K2 log_mel, K3 conv1d stem).
+// Whisper audio front-end on the GPU (log_mel, im2col of the conv1d stem).
 //
-// log_mel: the STFT is a GEMM. Each 256-thread workgroup owns 32 frames of one
-// utterance: the reflect-padded, Hann-windowed frames are staged in LDS, then
-// the four waves run exact-f32 MFMA (v_mfma_f32_32x32x2_f32, guide §3 "FP32-input
-// MFMA" - log-mel needs f32 dynamic range, bf16 would not do) against the
-// cos/sin DFT basis, square-sum to the power spectrum in LDS, and project onto
-// the mel filterbank with a second f32 MFMA. log10 + per-utterance max are fused
-// into the epilogue; a tiny second kernel applies whisper's max-8 clamp and
-// (x + 4) / 4 scaling and emits bf16.
+// log_mel: the STFT is a GEMM. A workgroup owns 16 frames of one utterance: their samples
+// come to LDS once, are windowed and folded (y[n] + y[400 - n] for the cosines, y[n] -
+// y[400 - n] for the sines: the basis rows n and 400 - n are equal up to the sine's sign,
+// so half the K range does), eight waves run exact-f32 MFMA (v_mfma_f32_16x16x4_f32;
+// log-mel needs f32 dynamic range) against the DFT basis, two bin tiles a wave, and square
+// into LDS. A mel band is a handful of neighbouring bins, so the filterbank is a short sum
+// per band over the bins where its row is not zero. log10 and the
+// workgroup's maximum are fused into the epilogue, which writes time-major rows; a second
+// kernel takes the utterance's maximum and applies whisper's max-8
+// clamp and (x + 4) / 4 scaling and emits bf16, time-major (the conv stem's rows, padded
+// with zero columns) or mel-major.
+// One 30 s window, 80 / 128 mels: 69 / 92 us before (32 frames a workgroup, 94 of them, the
+// whole K range, filterbank as a GEMM whose operand loads formed one chain), @@ us now; what
+// is left is the chain of basis loads of one workgroup per CU.
 //
 // im2col: k=3, pad=1 conv1d input unfolding so the conv becomes a plain GEMM
 // (hipBLASLt) followed by the fused bias+GELU(+pos) epilogue (elementwise.hip).
@@ -17,172 +23,172 @@
 #define NFFT 400
 #define HOP 160
 #define NBINS 201
-#define BIN_TILES 7         // 7 x 32 = 224 >= 201 bins
 #define BASIS_LD 224
-#define FRAMES_PER_WG 32
-// LDS row strides are odd (in dwords): the MFMA A operands are read one frame
-// (power row) per lane, 32 lanes per ds_read_b32 group with banks (a/4) % 32,
-// so an even stride put 2 (400) or 8 (204) rows on each bank - 16- / 4-way
-// conflicts (SQ_LDS_BANK_CONFLICT ~9.6 extra cycles per cycle)
-#define FRAME_LD 401        // 400 taps + 1
-#define POW_LD 203          // 202 used (K padded to even) + 1
+#define FPW 16              // frames of a workgroup
+#define SPAN ((FPW - 1) * HOP + NFFT)
+#define FOLD_LD 208         // 201 taps, padded with zeros to whole k-steps (of 4)
+#define POW_LD 209          // 13 tiles of 16 bins + 1
 
-typedef float f16v __attribute__((ext_vector_type(16)));
+typedef float f4v __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ f16v mfma_f32(float a, float b, const f16v& c) {
-  return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
-}
-
-__device__ __forceinline__ void atomic_max_float(float* addr, float v) {
-  if (v >= 0.f)
-    atomicMax(reinterpret_cast<int*>(addr), __float_as_int(v));
-  else
-    atomicMin(reinterpret_cast<unsigned int*>(addr), __float_as_uint(v));
-}
-
-// audio: [B, n_samples] f32;  window: [400];  cosb/sinb: [400, 224];
-// filt: [n_mels, 201];  out: [B, n_mels, n_frames] f32 (log10 mel);  gmax: [B]
-//
-// 8 waves: wave w < 7 owns DFT bin tile w (32 bins) for the workgroup's 32
-// frames, then waves 0..3 own one 32-mel tile each. Every MFMA chain is split
-// into two independent accumulator pairs (even / odd k-steps) and the DFT basis
-// for 16 k-steps is loaded before its MFMAs, so a wave is neither one
-// dependent MFMA chain nor one global load per k-step (the 4-wave form, two bin
-// tiles per wave, measured ~370 us per 30-s utterance).
+// audio: [B, n_samples] f32;  window: [400];  cosb/sinb: [400, 224];  filt: [n_mels, 201];
+// range: [n_mels, 2] first and past-the-last bin of each band;
+// out: [B, n_frames, n_mels] f32 (log10 mel);  gmax: [B, gridDim.x] maximum of each workgroup
 __global__ __launch_bounds__(512) void logmel_kernel(
     const float* __restrict__ audio, int n_samples, const float* __restrict__ window,
     const float* __restrict__ cosb, const float* __restrict__ sinb,
-    const float* __restrict__ filt, int n_mels, float* __restrict__ out, int n_frames,
-    float* __restrict__ gmax) {
-  __shared__ float frames[FRAMES_PER_WG][FRAME_LD];
-  __shared__ float power[FRAMES_PER_WG][POW_LD];
-  const int b = blockIdx.y;
-  const int f0 = blockIdx.x * FRAMES_PER_WG;
+    const float* __restrict__ filt, const int* __restrict__ range, int n_mels, float* __restrict__ out,
+    int n_frames, float* __restrict__ gmax) {
+  __shared__ float raw[SPAN];
+  __shared__ float even[FPW][FOLD_LD + 1], odd[FPW][FOLD_LD + 1];   // odd row strides: a lane per frame
+  __shared__ float power[FPW][POW_LD];
+  __shared__ float top[8];
+  const int b = blockIdx.y, f0 = blockIdx.x * FPW;
   const float* x = audio + (size_t)b * n_samples;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int hi = lane >> 5, lo = lane & 31;
+  const int fr = lane & 15, kq = lane >> 4;
 
-  // 1. reflect-padded (center=True) windowed frames -> LDS
-  for (int i = threadIdx.x; i < FRAMES_PER_WG * NFFT; i += blockDim.x) {
-    const int f = i / NFFT, n = i - f * NFFT;
-    int idx = (f0 + f) * HOP + n - NFFT / 2;
+  // wave w < 7 has the bins 32 w .. 32 w + 31 (201 of 224 exist); 52 k-steps of 4 taps (the last
+  // ones meet zeros) in four blocks of 13, whose basis values are loaded one block ahead, the
+  // first before the samples: the basis comes from far away when other work ran in between
+  const int bin = wave * 32 + fr;
+  const float* cb = cosb + (size_t)kq * BASIS_LD + bin;
+  const float* sb = sinb + (size_t)kq * BASIS_LD + bin;
+  float c[2][13][2], n[2][13][2];
+  auto load = [&](int blk) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < 13; ++u)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        c[blk & 1][u][t] = cb[(size_t)(52 * blk + 4 * u) * BASIS_LD + 16 * t];
+        n[blk & 1][u][t] = sb[(size_t)(52 * blk + 4 * u) * BASIS_LD + 16 * t];
+      }
+  };
+  if (wave < 7) load(0);
+
+  // the samples of all frames, reflected at the ends (center = True)
+  for (int i = threadIdx.x; i < SPAN; i += 512) {
+    int idx = f0 * HOP + i - NFFT / 2;
     if (idx < 0) idx = -idx;
-    if (idx >= n_samples) idx = 2 * (n_samples - 1) - idx;
-    frames[f][n] = (f0 + f < n_frames) ? x[idx] * window[n] : 0.f;
+    if (idx >= n_samples) idx = max(2 * (n_samples - 1) - idx, 0);   // frames past the end: any sample
+    raw[i] = x[idx];
   }
-  for (int i = threadIdx.x; i < FRAMES_PER_WG * POW_LD; i += blockDim.x)
-    (&power[0][0])[i] = 0.f;
   __syncthreads();
-
-  // 2. power spectrum: wave w handles bin tile w
-  if (wave < BIN_TILES) {
-    f16v re0, im0, re1, im1;
-#pragma unroll
-    for (int j = 0; j < 16; ++j) { re0[j] = 0.f; im0[j] = 0.f; re1[j] = 0.f; im1[j] = 0.f; }
-    const int bin = wave * 32 + lo;
-    const float* cb = cosb + hi * BASIS_LD + bin;
-    const float* sb = sinb + hi * BASIS_LD + bin;
-    // NFFT = 400 = 12 x 32 + 16: blocks of 16 k-steps (32 taps) then a tail of 8
-    int k = 0;
-    for (; k + 32 <= NFFT; k += 32) {
-      float bc[16], bs[16];
-#pragma unroll
-      for (int u = 0; u < 16; ++u) {
-        bc[u] = cb[(size_t)(k + 2 * u) * BASIS_LD];
-        bs[u] = sb[(size_t)(k + 2 * u) * BASIS_LD];
-      }
-#pragma unroll
-      for (int u = 0; u < 16; u += 2) {
-        const float a0 = frames[lo][k + 2 * u + hi], a1 = frames[lo][k + 2 * u + 2 + hi];
-        re0 = mfma_f32(a0, bc[u], re0);
-        im0 = mfma_f32(a0, bs[u], im0);
-        re1 = mfma_f32(a1, bc[u + 1], re1);
-        im1 = mfma_f32(a1, bs[u + 1], im1);
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < (NFFT % 32) / 2; ++u) {
-      const float a = frames[lo][k + 2 * u + hi];
-      re0 = mfma_f32(a, cb[(size_t)(k + 2 * u) * BASIS_LD], re0);
-      im0 = mfma_f32(a, sb[(size_t)(k + 2 * u) * BASIS_LD], im0);
-    }
-    // C layout: col = lane&31 (bin), row = (j&3) + 8*(j>>2) + 4*hi (frame)
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      const int fr = (j & 3) + 8 * (j >> 2) + 4 * hi;
-      const float r = re0[j] + re1[j], im = im0[j] + im1[j];
-      if (bin < NBINS) power[fr][bin] = r * r + im * im;
-    }
+  for (int i = threadIdx.x; i < FPW * FOLD_LD; i += 512) {
+    const int f = i / FOLD_LD, n = i - f * FOLD_LD;
+    const float lo = n <= NFFT / 2 ? raw[f * HOP + n] * window[n] : 0.f;
+    const bool two = n > 0 && n < NFFT / 2;
+    const float hi = two ? raw[f * HOP + NFFT - n] * window[NFFT - n] : 0.f;
+    even[f][n] = lo + hi;
+    odd[f][n] = two ? lo - hi : 0.f;
   }
   __syncthreads();
 
-  // 3. mel projection: wave w -> mel tile w (32 mels), K = 202 (power col 201 = 0)
-  float wmax = -FLT_MAX;
-  if (wave * 32 < n_mels) {
-    f16v acc0, acc1;
+  // power spectrum
+  if (wave < 7) {
+    f4v re[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}}, im[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-    for (int j = 0; j < 16; ++j) { acc0[j] = 0.f; acc1[j] = 0.f; }
-    const int mel = wave * 32 + lo;
-    const bool mv = mel < n_mels;
-    const float* fr_ = filt + (size_t)(mv ? mel : 0) * NBINS;
-#pragma unroll 2
-    for (int k = 0; k < NBINS + 1; k += 4) {    // 202 = 50 x 4 + 2
-      const float f0v = (mv && k + hi < NBINS) ? fr_[k + hi] : 0.f;
-      const float f1v = (mv && k + 2 + hi < NBINS && k + 2 < NBINS + 1) ? fr_[k + 2 + hi] : 0.f;
-      acc0 = mfma_f32(power[lo][k + hi], f0v, acc0);
-      if (k + 2 < NBINS + 1) acc1 = mfma_f32(power[lo][k + 2 + hi], f1v, acc1);
-    }
-    if (mv) {
-      float* orow = out + ((size_t)b * n_mels + mel) * n_frames;
+    for (int blk = 0; blk < 4; ++blk) {
+      if (blk < 3) load(blk + 1);
 #pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        const int fr = f0 + (j & 3) + 8 * (j >> 2) + 4 * hi;
-        if (fr < n_frames) {
-          const float lv = log10f(fmaxf(acc0[j] + acc1[j], 1e-10f));
-          orow[fr] = lv;
-          wmax = fmaxf(wmax, lv);
+      for (int u = 0; u < 13; ++u) {
+        const int k = 52 * blk + 4 * u + kq;
+        const float e = even[fr][k], o = odd[fr][k];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          re[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(e, c[blk & 1][u][t], re[t], 0, 0, 0);
+          im[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(o, n[blk & 1][u][t], im[t], 0, 0, 0);
         }
+      }
+    }
+    // column = lane & 15 (bin), row = 4 (lane / 16) + r (frame)
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (bin + 16 * t < NBINS) power[4 * kq + r][bin + 16 * t] = re[t][r] * re[t][r] + im[t][r] * im[t][r];
+  }
+  __syncthreads();
+
+  // a thread per band and four frames
+  float wmax = -FLT_MAX;
+  const int mel = threadIdx.x & 127, fg = threadIdx.x >> 7;
+  if (mel < n_mels) {
+    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+    const int hi = range[2 * mel + 1];
+    for (int j = range[2 * mel]; j < hi; ++j) {
+      const float w = filt[(size_t)mel * NBINS + j];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[r] += power[4 * fg + r][j] * w;
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int f = f0 + 4 * fg + r;
+      if (f < n_frames) {
+        const float lv = log10f(fmaxf(acc[r], 1e-10f));
+        out[((size_t)b * n_frames + f) * n_mels + mel] = lv;
+        wmax = fmaxf(wmax, lv);
       }
     }
   }
   wmax = wave_max(wmax);
-  if (lane == 0 && wmax > -FLT_MAX) atomic_max_float(gmax + b, wmax);
+  if (lane == 0) top[wave] = wmax;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int w = 1; w < 8; ++w) wmax = fmaxf(wmax, top[w]);
+    gmax[(size_t)b * gridDim.x + blockIdx.x] = wmax;
+  }
 }
 
-__global__ void fill_kernel(float* p, int n, float v) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = v;
-}
-
-// out_bf16[b, m, t] = (max(x, gmax[b] - 8) + 4) / 4
-__global__ void logmel_finalize_kernel(const float* __restrict__ x, const float* __restrict__ gmax,
-                                       bf16_t* __restrict__ y, long long per_b, long long total) {
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < total;
-       i += (long long)gridDim.x * blockDim.x) {
-    const int b = (int)(i / per_b);
-    const float v = fmaxf(x[i], gmax[b] - 8.f);
+// x [B, frames, M] f32 -> (max(x, top - 8) + 4) / 4 in bf16, top the maximum of the utterance's
+// `groups` entries of gmax: rows [B, frames, cols] with zeros in the columns from M on, or
+// (cols = 0) mel-major [B, M, frames]. One utterance per blockIdx.y.
+__global__ __launch_bounds__(256) void logmel_finalize_kernel(const float* __restrict__ x,
+                                                              const float* __restrict__ gmax, int groups,
+                                                              bf16_t* __restrict__ y, int frames, int M, int cols) {
+  __shared__ float top[4];
+  const int b = blockIdx.y;
+  float mx = -FLT_MAX;
+  for (int g = threadIdx.x; g < groups; g += 256) mx = fmaxf(mx, gmax[(size_t)b * groups + g]);
+  mx = wave_max(mx);
+  if ((threadIdx.x & 63) == 0) top[threadIdx.x >> 6] = mx;
+  __syncthreads();
+  const float lo = fmaxf(fmaxf(top[0], top[1]), fmaxf(top[2], top[3])) - 8.f;
+  const int width = cols ? cols : M;
+  const long long total = (long long)frames * width;
+  x += (size_t)b * frames * M;
+  y += (size_t)b * total;
+  for (long long i = blockIdx.x * 256LL + threadIdx.x; i < total; i += gridDim.x * 256LL) {
+    int t, m;
+    if (cols) {
+      t = (int)(i / cols);
+      m = (int)(i - (long long)t * cols);
+    } else {
+      m = (int)(i / frames);
+      t = (int)(i - (long long)m * frames);
+    }
+    const float v = m < M ? fmaxf(x[(size_t)t * M + m], lo) : -4.f;
     y[i] = f2bf((v + 4.f) * 0.25f);
   }
 }
 
 extern "C" int loqa_log_mel(const float* audio, int B, int n_samples, const float* window,
-                            const float* cosb, const float* sinb, const float* filt, int n_mels,
-                            float* work, float* gmax, void* out_bf16, int n_frames,
+                            const float* cosb, const float* sinb, const float* filt, const int* range, int n_mels,
+                            float* work, float* gmax, void* out_bf16, int n_frames, int cols,
                             hipStream_t s) {
   if (B <= 0) return 0;
-  if (n_frames <= 0 || n_mels <= 0 || n_mels > 128 || n_samples <= NFFT / 2)
+  if (n_frames <= 0 || n_mels <= 0 || n_mels > 128 || n_samples <= NFFT / 2 || (cols && cols < n_mels))
     return (int)hipErrorInvalidValue;
-  hipLaunchKernelGGL(fill_kernel, dim3((B + 255) / 256), dim3(256), 0, s, gmax, B, -FLT_MAX);
-  dim3 grid((n_frames + FRAMES_PER_WG - 1) / FRAMES_PER_WG, B);
+  dim3 grid((n_frames + FPW - 1) / FPW, B);
   hipLaunchKernelGGL(logmel_kernel, grid, dim3(512), 0, s, audio, n_samples, window, cosb, sinb,
-                     filt, n_mels, work, n_frames, gmax);
+                     filt, range, n_mels, work, n_frames, gmax);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return (int)e;
-  const long long per_b = (long long)n_mels * n_frames, total = per_b * B;
-  long long blocks = (total + 255) / 256;
+  long long blocks = ((long long)n_frames * (cols ? cols : n_mels) + 1023) / 1024;
   if (blocks > 8192) blocks = 8192;
-  hipLaunchKernelGGL(logmel_finalize_kernel, dim3((unsigned)blocks), dim3(256), 0, s, work, gmax,
-                     (bf16_t*)out_bf16, per_b, total);
+  hipLaunchKernelGGL(logmel_finalize_kernel, dim3((unsigned)blocks, B), dim3(256), 0, s, work, gmax, (int)grid.x,
+                     (bf16_t*)out_bf16, n_frames, n_mels, cols);
   return (int)hipGetLastError();
 }
 

@@ -103,7 +103,11 @@ class WhisperWeights:
                          if device.type == "cuda" and d % 128 == 0 and ENC_O_SPLITS else None)
         # conv stem weights in the implicit-im2col order (k = tap * Cin + c)
         # and f32 biases for the tiled GEMM's epilogue
-        self.conv1_wt = ops.conv_k3_weight(self.conv1_w, cfg.n_mels)
+        # (input channels padded with zeros to the GEMM's K step of 64)
+        self.mel_cols = -(-cfg.n_mels // 64) * 64
+        c1 = self.conv1_w.reshape(d, cfg.n_mels, 3)
+        self.conv1_wt = ops.conv_k3_weight(
+            torch.nn.functional.pad(c1, (0, 0, 0, self.mel_cols - cfg.n_mels)).reshape(d, -1), self.mel_cols)
         self.conv2_wt = ops.conv_k3_weight(self.conv2_w, d)
         self.conv1_bf, self.conv2_bf = self.conv1_b.float(), self.conv2_b.float()
         self.enc_fc1_bf = [L["fc1_b"].float() for L in self.enc]
@@ -197,18 +201,18 @@ class WhisperModel:
         cfg, w = self.cfg, self.w
         B = audio.shape[0]
         d, M = cfg.d_model, cfg.n_mels
-        mel = ops.log_mel(audio, self.mel)  # [B, M, 3000] bf16
-        frames = mel.shape[-1]
-        tile = ENC_TILE and audio.is_cuda and d % 128 == 0 and M % 64 == 0
+        frames = audio.shape[1] // 160
+        tile = ENC_TILE and audio.is_cuda and d % 128 == 0
         if tile:
             # conv1d stem on the tiled MFMA GEMM: the loader gathers the k = 3
             # taps from time-major rows (no column matrix), bias + GELU (+ the
             # sinusoidal positions for conv2) in the epilogue
-            mel_t = mel.transpose(1, 2).contiguous().view(B * frames, M)
+            mel_t = ops.log_mel_rows(audio, self.mel, w.mel_cols)     # [B * 3000, M, padded] bf16
             x1 = ops.gemm_tile(mel_t, w.conv1_wt, bias=w.conv1_bf, act="gelu", conv=(B, 1), layout=0)
             x = ops.gemm_tile(x1, w.conv2_wt, bias=w.conv2_bf, act="gelu", pos=w.pos_enc,
                               conv=(B, 2), layout=0)
         else:
+            mel = ops.log_mel(audio, self.mel)  # [B, M, 3000] bf16
             cols = ops.im2col_k3(mel, (M * frames, frames, 1), B, M, frames, 1)
             x1 = ops.linear(cols, w.conv1_w)                      # [B*3000, d]
             ops.gelu_bias_(x1, w.conv1_b)

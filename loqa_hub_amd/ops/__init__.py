@@ -331,21 +331,36 @@ def pcm16_to_f32_padded(pcm: torch.Tensor, offsets: torch.Tensor, ld: int,
     return out, sumsq[:S]
 
 
-def log_mel(audio: torch.Tensor, consts: "ref.MelConstants") -> torch.Tensor:
-    """audio [B, n_samples] f32 (padded to 30 s) -> whisper log-mel [B, n_mels, frames] bf16."""
-    if not _gpu(audio):
-        return ref.log_mel(audio, consts).to(torch.bfloat16)
+def _log_mel(audio: torch.Tensor, consts: "ref.MelConstants", cols: int) -> torch.Tensor:
     assert audio.dtype == torch.float32 and audio.is_contiguous() and audio.dim() == 2
     B, n = audio.shape
     frames = n // 160
     c = consts.to(audio.device)
-    work = torch.empty(B, c.n_mels, frames, dtype=torch.float32, device=audio.device)
-    gmax = torch.empty(B, dtype=torch.float32, device=audio.device)
-    out = torch.empty(B, c.n_mels, frames, dtype=torch.bfloat16, device=audio.device)
+    work = torch.empty(B, frames, c.n_mels, dtype=torch.float32, device=audio.device)
+    gmax = torch.empty(B, -(-frames // 16), dtype=torch.float32, device=audio.device)   # a maximum per workgroup
+    shape = (B, frames, cols) if cols else (B, c.n_mels, frames)
+    out = torch.empty(shape, dtype=torch.bfloat16, device=audio.device)
     check(kernels().loqa_log_mel(ptr(audio), B, n, ptr(c.window), ptr(c.cos_basis),
-                                 ptr(c.sin_basis), ptr(c.filters), c.n_mels, ptr(work), ptr(gmax),
-                                 ptr(out), frames, stream_ptr(audio)), "log_mel")
+                                 ptr(c.sin_basis), ptr(c.filters), ptr(c.ranges), c.n_mels, ptr(work), ptr(gmax),
+                                 ptr(out), frames, cols, stream_ptr(audio)), "log_mel")
     return out
+
+
+def log_mel(audio: torch.Tensor, consts: "ref.MelConstants") -> torch.Tensor:
+    """audio [B, n_samples] f32 (padded to 30 s) -> whisper log-mel [B, n_mels, frames] bf16."""
+    if not _gpu(audio):
+        return ref.log_mel(audio, consts).to(torch.bfloat16)
+    return _log_mel(audio, consts, 0)
+
+
+def log_mel_rows(audio: torch.Tensor, consts: "ref.MelConstants", cols: int) -> torch.Tensor:
+    """The same as time-major rows [B * frames, cols], zeros in the columns past n_mels (the
+    conv stem's input, channels padded to what its GEMM takes)."""
+    assert cols >= consts.n_mels
+    if not _gpu(audio):
+        m = ref.log_mel(audio, consts).to(torch.bfloat16).transpose(1, 2)
+        return torch.nn.functional.pad(m, (0, cols - m.shape[2])).reshape(-1, cols)
+    return _log_mel(audio, consts, cols).view(-1, cols)
 
 
 def im2col_k3(x: torch.Tensor, strides: tuple[int, int, int], B: int, C: int, L: int,

@@ -104,8 +104,8 @@ _KERNEL_SIGS = {
                        c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,
                        c_int, c_float, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_int,
                        c_void_p],
-    "loqa_log_mel": [c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int,
-                     c_void_p, c_void_p, c_void_p, c_int, c_void_p],
+    "loqa_log_mel": [c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int,
+                     c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p],
     "loqa_im2col_k3": [c_void_p, c_ll, c_ll, c_ll, c_int, c_int, c_int, c_int, c_void_p,
                        c_void_p],
     "loqa_skinny_gemm": [c_void_p, c_ll, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int,

@@ -237,6 +237,14 @@ class MelConstants:
     cos_basis: torch.Tensor   # [400, 224]
     sin_basis: torch.Tensor   # [400, 224]
     filters: torch.Tensor     # [n_mels, 201]
+    ranges: torch.Tensor | None = None   # [n_mels, 2] int32: first and past-the-last bin of a band
+
+    def __post_init__(self):
+        if self.ranges is None:
+            on = self.filters.cpu() != 0
+            lo = torch.where(on.any(1), on.int().argmax(1), 0)
+            hi = torch.where(on.any(1), on.shape[1] - on.flip(1).int().argmax(1), 0)
+            self.ranges = torch.stack([lo, hi], 1).to(torch.int32).contiguous().to(self.filters.device)
 
     @staticmethod
     def create(n_mels: int = 80) -> "MelConstants":
@@ -260,7 +268,8 @@ class MelConstants:
         key = str(device)
         if key not in cache:
             cache[key] = MelConstants(self.n_mels, self.window.to(device), self.cos_basis.to(device),
-                                      self.sin_basis.to(device), self.filters.to(device))
+                                      self.sin_basis.to(device), self.filters.to(device),
+                                      self.ranges.to(device))
         return cache[key]
 
 
