@@ -1,11 +1,10 @@
-// Flash attention forward for CDNA4 (SURVEY §2.4 K5, K7, K8, K12, K13).
+// Flash attention forward for CDNA4.
 //
 // One kernel family covers every attention in the hub:
-//   * PREFILL mode  - 128 query rows of ONE head per workgroup (Whisper encoder,
+//   * PREFILL mode  - a block of query rows of ONE head per workgroup (Whisper encoder,
 //                     Llama prompt prefill, VITS text encoder). Causal or not.
-//                     Served by attn_prefill2_kernel below (8 waves, key range
-//                     split between two wave groups); LOQA_ATTN_V1=1 selects
-//                     the original 4-wave attn_fwd_kernel.
+//                     attn_pipe_kernel below; rows off 16 bytes and cache blocks of
+//                     other sizes than 8, 16, 32, .. take attn_fwd_kernel (4 waves).
 //   * GROUPED mode  - all query heads of ONE kv head x a few query tokens per
 //                     workgroup (decode / jump-forward extend, GQA), with
 //                     split-K over the context and a separate combine kernel.
@@ -18,15 +17,14 @@
 //                    The query lands on the MFMA lane, so the softmax row
 //                    max/sum is in-register + one lane^32 exchange.
 //   O^T += V^T * P^T : the S^T accumulator, exp2'ed and packed to bf16, IS the B
-//                    operand (guide §3 "accumulator tile as next operand"); the
+//                    operand (the accumulator tile as next operand); the
 //                    V^T fragment comes from ds_read_b64_tr_b16 transposed reads
-//                    of the row-major V tile (guide T10). O^T also has the
+//                    of the row-major V tile. O^T also has the
 //                    query on the lane, so the online-softmax rescale is a
 //                    per-lane scalar multiply.
 // LDS rows are padded (K: +16 B, V: +64 B) so that both the b128 row reads and
-// the tr_b16 reads are bank-conflict free (guide §2, G4).
-#include "common.h"
-#include <cstdlib>
+// the tr_b16 reads are bank-conflict free (attn_fwd_kernel).
+#include "flash_pipe.h"
 
 #define ATT_THREADS 256
 #define ATT_WAVES 4
@@ -313,46 +311,43 @@ __global__ __launch_bounds__(ATT_THREADS, QR == 2 ? 2 : 1) void attn_fwd_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// PREFILL / ENCODER attention, split-KV inside the workgroup.
+// PREFILL / ENCODER attention on the pipelined tile loop (flash_pipe.h).
 //
-// The 4-wave prefill kernel above gives one workgroup 128-256 query rows of one
-// head, so a Whisper encoder pass at batch 1 (1500 frames x 20 heads) is 120
-// workgroups on a 256-CU chip with ONE wave per SIMD: the softmax VALU, the
-// K/V staging and the MFMAs of that wave serialize (measured 107 us per layer,
-// ~110 TFLOP/s). Here a workgroup is 8 waves over 128 query rows: waves 0-3
-// take the first half of the key tiles, waves 4-7 the second half (same query
-// rows, same lane layout), so every CU holds two waves per SIMD whose MFMA and
-// VALU phases overlap, and the grid doubles. Each half streams its K/V tiles
-// through registers into its own double-buffered LDS ring (guide T14: issue the
-// global loads of tile i+1 before computing tile i, write them to LDS after) -
-// one barrier per tile, no drain. The halves merge their (m, l, O) through LDS
-// at the end. Softmax work per score: max on raw scores, one fma + exp2 (scale
-// folded), masking only on the tail / causal-diagonal tiles (wave-uniform test).
-template <int D>
-struct AttnSmem2 {
-  bf16_t k[2][2][KV_TILE][D + 8];   // [half][stage]
-  bf16_t v[2][2][KV_TILE][D + 32];
-};
-
-template <int D, bool PAGED>
-__global__ __launch_bounds__(512, 1) void attn_prefill2_kernel(AttnParams p) {
-  __shared__ __attribute__((aligned(16))) AttnSmem2<D> sm;
-  constexpr int NS = D / 16, NDT = D / 32, CH = D / 8;
-  constexpr int NC = KV_TILE * CH / 256;      // 16-byte chunks per thread per operand
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int half = wave >> 2, w4 = wave & 3;
-  const int th = threadIdx.x & 255;
-  const int h = lane >> 5;
+// A workgroup is QW KS waves: QW blocks of 32 query rows of one head, the key tiles split
+// into KS runs with a ring of their own; the runs' (m, l, O) meet in LDS at the end.
+// One 30 s window has 1500 rows: 128 rows a workgroup are 240 workgroups at 20 heads, but 96
+// at 8, where 64 rows and four runs fill the chip (launch_attn() has the rule).
+// us a pass before (8 waves in step, K / V through registers, padded rows) and now: 1500 rows x 8
+// heads of 64: 23.4, 15.6; x 20 heads: 24, 22.8; 6 x 1500 x 20: 133, 100; 128 columns causal from a
+// paged cache: 2048 x 32 heads: 91, 60; 4 x that: 294, 198; 320 x 32 heads: 19, 19. What is left
+// above the VALU's and MFMAs' time: the loads' share of LDS and L2 (a third at 128 columns with
+// two runs), the barrier and the maxima, each of which all waves of a workgroup meet together.
+// PAGES: 0 contiguous rows, 1 cache blocks of 64 rows or more, 2 of 8, 16 or 32.
+template <int D, int PAGES, int QW, int KS>
+__global__ __launch_bounds__(64 * QW * KS, D == 64 && QW * KS == 4 ? 3 : 2) void attn_pipe_kernel(AttnParams p) {
+  constexpr bool PAGED = PAGES > 0;
+  using L = FlashLds<D, D>;
+  constexpr int NS = D / 16, NDT = D / 32, NTH = 64 * QW;
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int run = wave / QW, wq = wave % QW, th = threadIdx.x - run * NTH, h = lane >> 5;
   int bx, by, bz;
   {
-    const int gx = gridDim.x, gy = gridDim.y;
-    const int n = gx * gy * gridDim.z;
-    const int lin = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z);
-    const int logical = xcd_remap(lin, n);
-    bx = logical % gx;
-    by = (logical / gx) % gy;
-    bz = logical / (gx * gy);
+    const int gx = gridDim.x, gy = gridDim.y, heads = gy * gridDim.z, n = gx * heads;
+    const int logical = xcd_remap(blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z), n);
+    int hd = logical / gx;
+    bx = logical - hd * gx;
+    if (p.causal) {
+      // row blocks with the most keys first, over all heads of an XCD where these are whole
+      if (heads % 8 == 0) {
+        const int hp = heads / 8, xcd = logical / (hp * gx), at = logical - xcd * hp * gx;
+        bx = at / hp;
+        hd = xcd * hp + at - bx * hp;
+      }
+      bx = gx - 1 - bx;
+    }
+    by = hd % gy;
+    bz = hd / gy;
   }
   const int b = bz;
   const int q0 = p.cu_q[b];
@@ -365,19 +360,17 @@ __global__ __launch_bounds__(512, 1) void attn_prefill2_kernel(AttnParams p) {
     klen = p.ctx_lens ? p.ctx_lens[b] : p.cu_k[b + 1] - k0;
   }
   const int head = by, kvh = head / (p.Hq / p.Hkv);
-  const int row_lo = bx * 128;
+  const int row_lo = bx * (32 * QW);
   if (row_lo >= qlen) return;                               // whole workgroup: uniform
-  const int row_hi = min(qlen - 1, row_lo + 127);
-  const int qi = row_lo + w4 * 32 + (lane & 31);
+  const int row_hi = min(qlen - 1, row_lo + 32 * QW - 1);
+  const int qi = row_lo + wq * 32 + (lane & 31);
   const bool row_valid = qi < qlen;
-  const int qpos_lo = klen - qlen + row_lo + w4 * 32;       // wave's first / last query position
-  const int qpos_hi = qpos_lo + 31;
+  const int qpos_lo = klen - qlen + row_lo + wq * 32;       // wave's first query position
   int kend = klen;
   if (p.causal) kend = min(kend, klen - qlen + row_hi + 1);
-  const int ntiles = kend > 0 ? (kend + KV_TILE - 1) / KV_TILE : 0;
-  const int n0 = (ntiles + 1) >> 1;
-  const int my_t0 = half ? n0 : 0;
-  const int my_n = half ? ntiles - n0 : n0;
+  const int ntiles = kend > 0 ? (kend + FL_KEYS - 1) / FL_KEYS : 0;
+  const int per = (ntiles + KS - 1) / KS;                   // tiles of a run; the last may have fewer
+  const int first = run * per;
 
   bf16x8 qf[NS];
   {
@@ -393,192 +386,73 @@ __global__ __launch_bounds__(512, 1) void attn_prefill2_kernel(AttnParams p) {
   for (int i = 0; i < NDT; ++i)
 #pragma unroll
     for (int j = 0; j < 16; ++j) acc[i][j] = 0.f;
-  float m_run = -1e30f, l_run = 0.f;
-  const float sl2 = p.scale_log2;
+  float m = -1e30f, l = 0.f;
 
+  const FlFetch<D, NTH, false, false> kf(th, D, PAGED ? D : p.kv_stride);
+  const FlFetch<D, NTH, true, false> vf(th, D, PAGED ? D : p.kv_stride);
+  // Where a fetch stands: tiles come in order, one call each; past the last tile it stays there.
+  // Rows past kend read the last key again (finite scores, masked to -inf, so P = 0).
+  const int kt0 = max(min(first, ntiles - 1), 0) * FL_KEYS;
   const int* btab = PAGED ? p.block_tables + (size_t)b * p.max_blocks : nullptr;
-  // Loads are unconditional (rows past kend re-read the last key - finite
-  // values whose scores are masked to -inf, so P = 0 exactly; a half past its
-  // last tile re-reads a valid tile): a load under a branch makes hipcc fall
-  // back to vmcnt(0) at the first MFMA, serialising the prefetch.
-#define ATT2_ROW_OFF(KT, i, key_, cc_)                                                \
-    const int c = th + (i) * 256;                                                     \
-    const int kr = c / CH, cc_ = (c - kr * CH) * 8;                                   \
-    const int key_ = min((KT) + kr, kend - 1);                                        \
-    size_t off;                                                                       \
-    if (PAGED) {                                                                      \
-      const int bi = key_ / p.blk, bo = key_ - bi * p.blk;                            \
-      off = (((size_t)btab[bi] * p.Hkv + kvh) * p.blk + bo) * D + cc_;                \
-    } else {                                                                          \
-      off = (size_t)(k0 + key_) * p.kv_stride + (size_t)kvh * D + cc_;                \
-    }
-#define ATT2_LOAD1(SRC, KT, R)                                                        \
-  _Pragma("clang loop unroll(full)") for (int i = 0; i < NC; ++i) {                   \
-    ATT2_ROW_OFF(KT, i, key, cc)                                                      \
-    R[i] = *reinterpret_cast<const u32x4*>(SRC + off);                                \
-  }
-#define ATT2_STORE1(DST, R)                                                           \
-  _Pragma("clang loop unroll(full)") for (int i = 0; i < NC; ++i) {                   \
-    const int c = th + i * 256;                                                       \
-    const int kr = c / CH, cc = (c - kr * CH) * 8;                                    \
-    *reinterpret_cast<u32x4*>(&DST[kr][cc]) = R[i];                                   \
-  }
-  // S^T = K Q^T for the tile in K stage KST (two 32-key halves; the query is
-  // this lane's column)
-#define ATT2_QK(KST, ST)                                                              \
-  {                                                                                   \
-    const bf16_t(*ks_)[D + 8] = sm.k[half][KST];                                      \
-    _Pragma("unroll") for (int t = 0; t < 2; ++t) {                                   \
-      _Pragma("unroll") for (int j = 0; j < 16; ++j) ST[t][j] = 0.f;                  \
-      _Pragma("unroll") for (int s = 0; s < NS; ++s) {                                \
-        const bf16x8 a = *reinterpret_cast<const bf16x8*>(&ks_[32 * t + (lane & 31)][16 * s + 8 * h]); \
-        ST[t] = mfma32(a, qf[s], ST[t]);                                              \
-      }                                                                               \
-    }                                                                                 \
-  }
-
-  // online softmax of the scores ST of the tile at key KT, then O^T += V^T P^T
-  // with V from V stage VST
-  auto softmax_pv = [&](float16v (&st)[2], int vst, int kt) __attribute__((always_inline)) {
-    // masking only where a key can be invalid for this wave (wave-uniform test)
-    if (kt + KV_TILE > kend || (p.causal && kt + KV_TILE - 1 > qpos_lo)) {
-      const int lim = (p.causal ? min(kend, klen - qlen + qi + 1) : kend) - kt - 4 * h;
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int j = 0; j < 16; ++j)
-          if (32 * t + (j & 3) + 8 * (j >> 2) >= lim) st[t][j] = -INFINITY;
-    }
-    float mx = st[0][0];
-#pragma unroll
-    for (int j = 1; j < 16; ++j) mx = fmaxf(mx, st[0][j]);
-#pragma unroll
-    for (int j = 0; j < 16; ++j) mx = fmaxf(mx, st[1][j]);
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    const float m_new = fmaxf(m_run, mx * sl2);
-    const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-    bf16x8 pf[2][2];
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int s2 = 0; s2 < 2; ++s2)
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-          pf[t][s2][j] = (__bf16)__builtin_amdgcn_exp2f(fmaf(st[t][8 * s2 + j], sl2, -m_new));
-    // row sums on the matrix core (ones . P^T: every output row is the sum
-    // over the tile's 64 keys of the bf16 P that also feeds O), which has
-    // slack here, instead of 32 VALU adds + a cross-lane exchange
-    {
-      bf16x8 ones;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) ones[j] = (__bf16)1.0f;
-      float16v ls = {};
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2) ls = mfma32(ones, pf[t][s2], ls);
-      l_run = l_run * alpha + ls[0];
-    }
-    m_run = m_new;
-#pragma unroll
-    for (int i = 0; i < NDT; ++i)
-#pragma unroll
-      for (int j = 0; j < 16; ++j) acc[i][j] *= alpha;
-    const bf16_t(*vt_s)[D + 32] = sm.v[half][vst];
-    const int g = lane >> 4, li = lane & 15;
-#pragma unroll
-    for (int dt = 0; dt < NDT; ++dt) {
-      const int c0 = 32 * dt + 16 * (g & 1) + 4 * (li & 3);
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2) {
-          const int kb = 32 * t + 16 * s2 + 4 * h + (li >> 2);
-          const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-              (__attribute__((address_space(3))) v4s*)(&vt_s[kb][c0]));
-          const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-              (__attribute__((address_space(3))) v4s*)(&vt_s[kb + 8][c0]));
-          short8 a8;
-          a8[0] = lo[0]; a8[1] = lo[1]; a8[2] = lo[2]; a8[3] = lo[3];
-          a8[4] = hi[0]; a8[5] = hi[1]; a8[6] = hi[2]; a8[7] = hi[3];
-          acc[dt] = mfma32(*reinterpret_cast<bf16x8*>(&a8), pf[t][s2], acc[dt]);
-        }
-    }
+  const unsigned page_bytes = (unsigned)(p.Hkv * p.blk) * (D * 2);
+  struct At {
+    const bf16_t* row;               // contiguous: the tile's first row
+    int kt;
+    FlPages pages;
   };
-#define ATT2_BARRIER()                                                                \
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                                  \
-  __builtin_amdgcn_s_barrier();                                                       \
-  asm volatile("" ::: "memory");
-
-  // two K/V stages; tile i+1 is loaded to registers while tile i is computed
-  if (ntiles > 0) {
-    const int kt0 = min(my_t0, ntiles - 1) * KV_TILE;
-    u32x4 kreg[NC], vreg[NC];   // native vectors: HIP's uint4 struct copies stay in scratch
-    ATT2_LOAD1(p.k, kt0, kreg)
-    ATT2_LOAD1(p.v, kt0, vreg)
-    ATT2_STORE1(sm.k[half][0], kreg)
-    ATT2_STORE1(sm.v[half][0], vreg)
-  }
-  for (int it = 0; it < n0; ++it) {
-    const int stage = it & 1;
-    const int kt = (my_t0 + it) * KV_TILE;
-    const int ktn = min(my_t0 + it + 1, ntiles - 1) * KV_TILE;   // next tile (clamped)
-    u32x4 kreg[NC], vreg[NC];
-    ATT2_LOAD1(p.k, ktn, kreg)                       // lands during this tile's math
-    ATT2_LOAD1(p.v, ktn, vreg)
-    ATT2_BARRIER()                                   // stage `stage` written by every wave
-    if (it < my_n && !(p.causal && kt > qpos_hi)) {
-      float16v st[2];
-      ATT2_QK(stage, st)
-      softmax_pv(st, stage, kt);
+  auto start = [&](const bf16_t* src) __attribute__((always_inline)) {
+    return At{src + (PAGED ? (size_t)kvh * p.blk * D : (size_t)(k0 + kt0) * p.kv_stride + (size_t)kvh * D), kt0,
+              FlPages(btab, PAGED ? 31 - __clz(p.blk) : 0, kend)};
+  };
+  auto fetch = [&](const auto& f, At& a, unsigned stage) __attribute__((always_inline)) {
+    const int last = kend - 1 - a.kt;
+    if constexpr (!PAGED) {
+      f.strided(stage, a.row, last);
+      if (last >= FL_KEYS) a.row += FL_KEYS * p.kv_stride;
+    } else {
+      a.pages.hold(a.kt, lane);
+      auto at = [&](int r) __attribute__((always_inline)) {
+        const int key = a.kt + r;
+        const unsigned long long off = (unsigned long long)(unsigned)a.pages.page(key) * page_bytes;
+        return (const bf16_t*)((const char*)a.row + off + (unsigned)(key & (p.blk - 1)) * (D * 2));
+      };
+      if constexpr (PAGES == 1)
+        f.strided(stage, at(0), last);
+      else
+        f.paged(stage, last, at);
     }
-    // that stage was last read before this tile's barrier; past a half's last
-    // tile the write is never read
-    ATT2_STORE1(sm.k[half][stage ^ 1], kreg)
-    ATT2_STORE1(sm.v[half][stage ^ 1], vreg)
-  }
-#undef ATT2_ROW_OFF
-#undef ATT2_LOAD1
-#undef ATT2_STORE1
-#undef ATT2_QK
-#undef ATT2_BARRIER
+    if (last >= FL_KEYS) a.kt += FL_KEYS;
+  };
+  At ka = start(p.k), va = start(p.v);
+  const unsigned ring = fl_lds_at(lds) + run * L::RING;
+  fl_loop<D, D>(
+      qf, acc, m, l, ring, per, p.scale_log2, lane,
+      [&](float16v(&st)[2], int i) __attribute__((always_inline)) {
+        // masking only where a key can be invalid for this wave (wave-uniform test)
+        const int kt = (first + i) * FL_KEYS;
+        if (kt + FL_KEYS > kend || (p.causal && kt + FL_KEYS - 1 > qpos_lo)) {
+          const int lim = (p.causal ? min(kend, klen - qlen + qi + 1) : kend) - kt - 4 * h;
+#pragma unroll
+          for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int j = 0; j < 16; ++j)
+              if (32 * t + (j & 3) + 8 * (j >> 2) >= lim) st[t][j] = -INFINITY;
+        }
+      },
+      [&](int, unsigned stage) __attribute__((always_inline)) { fetch(kf, ka, stage); },
+      [&](int, unsigned stage) __attribute__((always_inline)) { fetch(vf, va, stage); });
 
-  // ---- merge the two halves: waves 4-7 hand (m, l, O) to waves 0-3 through LDS
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();                        // every wave done with the K/V rings
-  asm volatile("" ::: "memory");
-  float* xo = reinterpret_cast<float*>(&sm);           // [4 waves][NDT * 16][64 lanes]
-  float* xml = xo + 4 * NDT * 16 * 64;                 // [4 waves][2][64 lanes]
-  if (half) {
-#pragma unroll
-    for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-      for (int j = 0; j < 16; ++j) xo[(w4 * NDT * 16 + dt * 16 + j) * 64 + lane] = acc[dt][j];
-    xml[(w4 * 2) * 64 + lane] = m_run;
-    xml[(w4 * 2 + 1) * 64 + lane] = l_run;
-  }
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-  if (half || !row_valid) return;
-  const float m1 = xml[(w4 * 2) * 64 + lane], l1 = xml[(w4 * 2 + 1) * 64 + lane];
-  const float m = fmaxf(m_run, m1);
-  const float a0 = exp2f(m_run - m), a1 = exp2f(m1 - m);
-  const float l = l_run * a0 + l1 * a1;
+  fl_sync();                                                // every wave is done with the rings
+  fl_merge<NDT, QW, KS>(acc, m, l, reinterpret_cast<float*>(lds), run, wq, lane);
+  if (run) return;
   const float inv = l > 0.f ? 1.f / l : 0.f;
-  const float s0 = a0 * inv, s1 = a1 * inv;
-  bf16_t* orow = p.o + (size_t)(q0 + qi) * p.o_stride + (size_t)head * D;
 #pragma unroll
-  for (int dt = 0; dt < NDT; ++dt)
+  for (int d = 0; d < NDT; ++d)
 #pragma unroll
-    for (int g4 = 0; g4 < 4; ++g4) {
-      const int d0 = 32 * dt + 8 * g4 + 4 * h;
-      float o[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        o[r] = acc[dt][4 * g4 + r] * s0 + xo[(w4 * NDT * 16 + dt * 16 + 4 * g4 + r) * 64 + lane] * s1;
-      *reinterpret_cast<uint2*>(orow + d0) = make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
-    }
+    for (int j = 0; j < 16; ++j) acc[d][j] *= inv;
+  fl_store<NDT>(acc, lds + fl_merge_bytes(NDT, QW, KS) + wq * fl_store_bytes(NDT),
+                p.o + (size_t)(q0 + row_lo + wq * 32) * p.o_stride + (size_t)head * D, p.o_stride,
+                qlen - row_lo - wq * 32, D, lane);
 }
 
 // Combine split-K partials: one workgroup of D threads per (token, head).
@@ -600,17 +474,44 @@ __global__ void attn_combine_kernel(const float* __restrict__ part_o,
   o[(size_t)tok * o_stride + (size_t)head * D + d] = f2bf(l > 0.f ? acc / l : 0.f);
 }
 
+template <int D, int PAGES, int QW, int KS>
+static int launch_pipe(const AttnParams& p, int B, int max_q, hipStream_t s) {
+  constexpr int ring = KS * FlashLds<D, D>::RING, end = fl_merge_bytes(D / 32, QW, KS) + QW * fl_store_bytes(D / 32);
+  constexpr int bytes = ring > end ? ring : end;
+  static_assert(bytes <= 160 * 1024, "LDS of a CU");
+  const dim3 grid((max_q + 32 * QW - 1) / (32 * QW), p.Hq, B);
+  hipLaunchKernelGGL((attn_pipe_kernel<D, PAGES, QW, KS>), grid, dim3(64 * QW * KS), bytes, s, p);
+  return (int)hipGetLastError();
+}
+
+// 64 rows and all runs that LDS holds while these workgroups are one round of the 256 CUs; then
+// 128 rows and two runs; with more work, 128 rows and one run in four waves, two or three
+// workgroups a CU, which are out of step with each other. us a pass (64-row form, 128 / two,
+// 128 / one): 1500 x 8 heads of 64: 15.6, 20, 25; x 20 heads: 26, 22.7, 27; 6 x 1500 x 20 heads:
+// 133, 124, 106; 128 columns, paged: 320 rows behind 1000 x 32 heads: 31, 32, 40; 2048 x 32 heads
+// causal: 101, 60, 70; 4 x that: 349, 238, 200
+template <int D, int PAGES>
+static int launch_rows(const AttnParams& p, int B, int max_q, hipStream_t s) {
+  const long n64 = (long)((max_q + 63) / 64) * p.Hq * B, n128 = (long)((max_q + 127) / 128) * p.Hq * B;
+  if (n64 <= 256) return launch_pipe<D, PAGES, 2, D == 64 ? 4 : 2>(p, B, max_q, s);
+  if (n128 <= (D == 64 ? 256 : 512)) return launch_pipe<D, PAGES, 4, 2>(p, B, max_q, s);
+  return launch_pipe<D, PAGES, 4, 1>(p, B, max_q, s);
+}
+
 template <int D, bool PAGED, bool GROUPED>
 static int launch_attn(const AttnParams& p, int B, int max_q, hipStream_t s) {
   dim3 grid;
+  if (!GROUPED) {
+    // The direct-to-LDS loads and whole-row stores take 16-byte aligned rows, a tile's rows within
+    // 32-bit offsets, and cache blocks in which eight (four) rows of one load lie together.
+    const bool rows16 = (((size_t)p.q | (size_t)p.k | (size_t)p.v | (size_t)p.o) & 15) == 0 &&
+                        ((p.q_stride | p.kv_stride | p.o_stride) & 7) == 0 && p.kv_stride < (1 << 24);
+    const bool blocks = p.blk >= 8 && (p.blk & (p.blk - 1)) == 0 && (long)p.Hkv * p.blk < (1 << 22);
+    if (rows16 && !PAGED) return launch_rows<D, 0>(p, B, max_q, s);
+    if (rows16 && blocks) return p.blk >= FL_KEYS ? launch_rows<D, 1>(p, B, max_q, s) : launch_rows<D, 2>(p, B, max_q, s);
+  }
   // QR = 2 (64 query rows per wave) where it pays: D = 64 prefill / encoder
   constexpr int QR = (!GROUPED && D == 64) ? 2 : 1;
-  static const bool v1 = getenv("LOQA_ATTN_V1") != nullptr;
-  if (!GROUPED && !v1) {
-    grid = dim3((max_q + 127) / 128, p.Hq, B);
-    hipLaunchKernelGGL((attn_prefill2_kernel<D, PAGED>), grid, dim3(512), 0, s, p);
-    return (int)hipGetLastError();
-  }
   if (GROUPED)
     grid = dim3(p.num_splits, p.Hkv, B);
   else

@@ -1,0 +1,366 @@
+// Device parts of the software-pipelined flash attention (attention.hip, attn_window.hip,
+// attn_latent_prefill.hip): a wave's 32 query rows over a run of 64-key tiles.
+//
+// S^T = K Q^T (v_mfma_f32_32x32x16_bf16: the query lands on the MFMA lane, so row maxima and
+// sums are in-register plus one exchange with lane ^ 32) and O^T += V^T P^T with the exp2'ed
+// S^T as the B operand as it stands, V^T by transposed LDS reads of the row-major V tile.
+//
+// What bounds a tile of a wave: at 64 / 64 head columns the VALU (32 exp2 of 8 cycles, fma,
+// maximum, conversion, rescaling: ~700 cycles) as much as the MFMAs (640), at 128 / 128 the
+// MFMAs (1024). Done one after the other they add up, and two waves of a SIMD that share a barrier
+// per tile stay in step instead of filling each other's gaps. So the scores of tile i + 1 are
+// computed between the exponentials of tile i (first half of the keys), its first P V product
+// between those of the second half, and the second P V product covers the row maxima of
+// i + 1. O is rescaled in a branch, when a row of the wave has a new maximum.
+// (Rescaling only when a maximum passes the reference point by a factor of 256 made the 64
+// column form 6 % faster, but the largest weights then no longer lie just below a power of two,
+// where bf16's rounding is finest: 4 to 10 % more error.)
+// K and V come straight to LDS (16 bytes a lane), two stages each, K one tile ahead of V; a
+// lane fetches the chunk that its LDS place holds after an XOR of chunk and row, so rows need
+// no padding and both kinds of LDS reads are free of bank conflicts. Taken back: a third stage
+// (nothing: the loads cost LDS and L2 time, not waiting), spreading the loads between the MFMAs,
+// eight fragments in flight, the barrier between the last MFMAs of a tile (5 % slower).
+#pragma once
+#include "common.h"
+
+#define FL_KEYS 64                     // keys of a tile
+
+typedef short fl_v4s __attribute__((ext_vector_type(4)));
+typedef float fl_f2 __attribute__((ext_vector_type(2)));
+typedef __bf16 fl_b2 __attribute__((ext_vector_type(2)));
+typedef unsigned fl_u4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ float16v fl_mfma(const bf16x8& a, const bf16x8& b, const float16v& c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+
+template <int V> struct Fl { static constexpr int value = V; };
+
+template <int DK, int DV> struct FlashLds {
+  static constexpr int K = FL_KEYS * DK * 2, V = FL_KEYS * DV * 2;   // bytes of a stage
+  static constexpr int RING = 2 * (K + V);                           // K stages, then V stages
+};
+
+// Chunk (16 bytes) c of row r lies at place c ^ swz(r). K: 16 rows of one chunk are read at
+// once, V: four rows of four chunks; a 256-byte row covers the 64 banks, a 128-byte row half.
+template <int D> __device__ __forceinline__ int fl_kswz(int r) { return D % 128 == 0 ? r & 15 : (r >> 1) & 7; }
+template <int D> __device__ __forceinline__ int fl_vswz(int r) { return D % 128 == 0 ? (r & 3) << 2 : (r & 2) << 1; }
+
+// LDS by its byte address, which leaves the base and the constant part of an access to one
+// register and the instruction's offset.
+#define FL_LDS __attribute__((address_space(3)))
+__device__ __forceinline__ unsigned fl_lds_at(unsigned char* p) { return (unsigned)(size_t)(FL_LDS unsigned char*)p; }
+template <typename T> __device__ __forceinline__ FL_LDS T* fl_lds(unsigned at) { return (FL_LDS T*)(size_t)at; }
+
+// 16 bytes per lane straight to LDS (lane l at dst + 16 l, dst wave-uniform). As the builtin, each
+// load made the compiler wait for all of them before the next transposed LDS read, of whose
+// address it knows nothing; the waits are fl_sync()'s. No register is written.
+__device__ __forceinline__ void fl_load_lds(const bf16_t* base, unsigned off, unsigned dst) {   // base wave-uniform
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(off), "s"(base) : "memory", "m0");
+}
+
+// The fetch of one tile of K (ISV = false) or V rows into a stage by the NTH threads (whole
+// waves) of a group, th the thread. Rows past `last` read row `last`; PAD: only cols of the D
+// columns exist (the others' places in LDS are left as they are).
+template <int D, int NTH, bool ISV, bool PAD> struct FlFetch {
+  static constexpr int CH = D / 8, N = FL_KEYS * CH / NTH;
+  static constexpr int RG = 64 % CH == 0 ? 64 / CH : 1;     // rows of one instruction of a wave, if whole
+  static_assert(N * NTH == FL_KEYS * CH, "whole chunks per thread");
+  int th, cols;
+  unsigned st;                         // stride of the rows in bytes (64 st < 2^32)
+  __device__ __forceinline__ int row(int i) const { return NTH % CH == 0 ? th / CH + i * (NTH / CH) : (th + i * NTH) / CH; }
+  __device__ __forceinline__ int chunk(int i) const {
+    const int r = row(i);
+    return ((th + i * NTH) - r * CH) ^ (ISV ? fl_vswz<D>(r) : fl_kswz<D>(r));
+  }
+  __device__ __forceinline__ FlFetch(int th_, int cols_, long long stride) : th(th_), cols(cols_), st((unsigned)stride * 2) {}
+  __device__ __forceinline__ unsigned dst(unsigned stage) const { return __builtin_amdgcn_readfirstlane(stage + (th & ~63) * 16); }
+  // rows at the stride, from the tile's first (wave-uniform)
+  __device__ __forceinline__ void strided(unsigned stage, const bf16_t* base, int last) const {
+    const unsigned d = dst(stage);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      unsigned off = (unsigned)row(i) * st + chunk(i) * 16;
+      if (last < FL_KEYS - 1) off -= (unsigned)max(row(i) - last, 0) * st;
+      if (!PAD || chunk(i) * 8 < cols) fl_load_lds(base, off, d + i * NTH * 16);
+    }
+  }
+  // rows in pages of a multiple of RG: at(r), called with wave-uniform multiples of RG, the first of RG rows
+  template <typename At> __device__ __forceinline__ void paged(unsigned stage, int last, At&& at) const {
+    static_assert(64 % CH == 0, "whole rows per instruction");
+    const unsigned d = dst(stage);
+    const int w0 = __builtin_amdgcn_readfirstlane(th & ~63) / CH, in = (th & 63) / CH;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int r = min(w0 + i * (NTH / CH), last & ~(RG - 1));
+      const bf16_t* base = at(r);
+      unsigned off = (unsigned)in * st + chunk(i) * 16;
+      if (last < FL_KEYS - 1) off -= (unsigned)max(in - (last - r), 0) * st;
+      if (!PAD || chunk(i) * 8 < cols) fl_load_lds(base, off, d + i * NTH * 16);
+    }
+  }
+};
+
+// A sequence's block table for pages of 1 << sh rows, 64 entries at a time (one a lane).
+struct FlPages {
+  const int* tab;
+  int sh, last, base, held;            // last: the last page of use
+  __device__ __forceinline__ FlPages(const int* t, int sh_, int keys)
+      : tab(t), sh(sh_), last(max(keys - 1, 0) >> sh_), base(-64), held(0) {}
+  // the table's part for keys kt .. kt + 63 (at most 64 pages)
+  __device__ __forceinline__ void hold(int kt, int lane) {
+    if (min((kt + FL_KEYS - 1) >> sh, last) >= base + 64) {
+      base = __builtin_amdgcn_readfirstlane(kt >> sh);
+      held = tab[min(base + lane, last)];
+    }
+  }
+  __device__ __forceinline__ int page(int key) const { return __builtin_amdgcn_readlane(held, (key >> sh) - base); }
+};
+
+// every load of this wave has landed, its LDS reads are done, and so for the other waves
+__device__ __forceinline__ void fl_sync() {
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+__device__ __forceinline__ float fl_max32(float x) {   // over lane and lane ^ 32
+  typedef unsigned u2 __attribute__((ext_vector_type(2)));
+  const u2 r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+__device__ __forceinline__ float fl_both32(float x) {  // lane + lane ^ 32
+  typedef unsigned u2 __attribute__((ext_vector_type(2)));
+  const u2 r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// The tiles 0 .. n - 1 of a group of waves that share a ring (n the same for every wave that
+// meets the barriers): acc and l get sum P V and sum P relative to exp2(m), scores in units
+// of sl2 (> 0). prep(st, i) masks (or transforms) the scores of tile i: register 16 t + j of
+// lane (column, h) is key 32 t + (j & 3) + 8 (j >> 2) + 4 h; a wave whose rows see nothing of a
+// tile masks all of it (it would wait for the others anyway, and one path through the loop
+// leaves the registers where they are). load_k / load_v(i, stage) start the fetch of tile i;
+// they are called for i = 0, 1, 2, .. up to n (K) and n - 1 (V); for i = n they must fetch
+// something that exists (or nothing).
+// Before the call m = -1e30, l = 0, acc = 0; ring must not be in use. After it the waves
+// are not synchronised.
+template <int DK, int DV, typename Prep, typename LoadK, typename LoadV>
+__device__ __forceinline__ void fl_loop(const bf16x8 (&qf)[DK / 16], float16v (&acc)[DV / 32], float& m, float& l,
+                                        unsigned ring, int n, float sl2, int lane, Prep&& prep,
+                                        LoadK&& load_k, LoadV&& load_v) {
+  using L = FlashLds<DK, DV>;
+  // The sums of a tile's (rounded) P: as one more output column block where the VALU is what
+  // is short, as dot products with ones where the MFMAs are.
+  constexpr bool ROW = DV <= 64;
+  constexpr int NS = DK / 16, NDT = DV / 32, NQ = 2 * NS, NW = NDT + ROW, NP = 2 * NW;
+  const int h = lane >> 5, li = lane & 15;
+  // K fragment (t, s): row 32 t + (lane & 31), chunk 2 s + h; the XOR keeps the chunk's part
+  // above its 3 or 4 bits, so that part and t are constants added to a lane's base
+  constexpr int KM = DK % 128 == 0 ? 8 : 4;            // fragments of a swizzled run
+  unsigned kb[KM];
+#pragma unroll
+  for (int s = 0; s < KM; ++s) kb[s] = ring + (lane & 31) * (DK * 2) + ((2 * s + h) ^ fl_kswz<DK>(lane & 31)) * 16;
+  // V fragment (t, s2, dt): rows 32 t + 16 s2 + 4 h + (li >> 2), + 8, columns 32 dt + 16 (lane / 16 & 1) + 4 (li & 3)
+  unsigned vb[NDT];
+#pragma unroll
+  for (int d = 0; d < NDT; ++d)
+    vb[d] = ring + 2 * L::K + (4 * h + (li >> 2)) * (DV * 2) +
+            ((4 * d + 2 * ((lane >> 4) & 1) + ((li & 3) >> 1)) ^ fl_vswz<DV>(li >> 2)) * 16 + (li & 1) * 8;
+  constexpr int KR = 4, VR = 4;                        // fragments in flight + 1
+  const float16v zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  bf16x8 ones;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) ones[j] = (__bf16)1.0f;
+  const fl_b2 one2 = {(__bf16)1.0f, (__bf16)1.0f};
+
+  // Q is here before the first load whose wait the compiler does not know
+  bf16x8 qr[NS];
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    qr[s] = qf[s];
+    asm volatile("" : "+v"(qr[s]));
+  }
+  // cur: scores of tile i (SM: softmax and P V of it), nxt: of tile i + 1 (QK: compute them);
+  // V of i lies in stage S, K of i + 1 in stage 1 - S
+  auto body = [&](auto qk, auto sm, auto slot, float16v(&cur)[2], float16v(&nxt)[2], int i) __attribute__((always_inline)) {
+    constexpr bool QK = decltype(qk)::value != 0, SM = decltype(sm)::value != 0;
+    constexpr int S = decltype(slot)::value;
+    bf16x8 kf[KR], vf[VR];
+    fl_u4 pf[2][2];
+    auto kread = [&](int u, int stage) __attribute__((always_inline)) {
+      const int t = u & 1, s = u >> 1;
+      kf[u % KR] = *fl_lds<bf16x8>(kb[s % KM] + (stage * L::K + 32 * t * DK * 2 + s / KM * KM * 32));
+    };
+    auto vread = [&](int v) __attribute__((always_inline)) {      // v = (2 t + s2) NDT + dt
+      const int ts = v / NDT, d = v % NDT;
+      const unsigned a = vb[d] + (S * L::V + 16 * ts * DV * 2);
+      const fl_v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(fl_lds<fl_v4s>(a));
+      const fl_v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(fl_lds<fl_v4s>(a + 8 * DV * 2));
+      short8 a8;
+      a8[0] = lo[0]; a8[1] = lo[1]; a8[2] = lo[2]; a8[3] = lo[3];
+      a8[4] = hi[0]; a8[5] = hi[1]; a8[6] = hi[2]; a8[7] = hi[3];
+      vf[v % VR] = *reinterpret_cast<bf16x8*>(&a8);
+    };
+    // the exponentials of slice w of N: pairs of scores of key half t
+    auto exps = [&](int t, int w, int N) __attribute__((always_inline)) {
+#pragma unroll
+      for (int q = w * 8 / N; q < (w + 1) * 8 / N; ++q) {
+        fl_f2 e;
+        e[0] = __builtin_amdgcn_exp2f(fmaf(cur[t][2 * q], sl2, -m));
+        e[1] = __builtin_amdgcn_exp2f(fmaf(cur[t][2 * q + 1], sl2, -m));
+        const fl_b2 b = __builtin_convertvector(e, fl_b2);
+        pf[t][q >> 2][q & 3] = __builtin_bit_cast(unsigned, b);
+        if constexpr (!ROW) l = __builtin_amdgcn_fdot2_f32_bf16(b, one2, l, false);
+      }
+    };
+    float16v ls;
+    auto pv = [&](int t, int w) __attribute__((always_inline)) {  // MFMA w of half t; reads three ahead
+      const int s2 = w / NW, d = w % NW - ROW, v = (2 * t + s2) * NDT + d;
+      const bf16x8 p8 = __builtin_bit_cast(bf16x8, pf[t][s2]);
+      if (d < 0)
+        ls = fl_mfma(ones, p8, t + s2 == 0 ? zero : ls);
+      else {
+        acc[d] = fl_mfma(vf[v % VR], p8, acc[d]);
+        if (v + VR - 1 < 4 * NDT) vread(v + VR - 1);
+      }
+    };
+    // tile i's V and i + 1's K are here, the K of i and the V of i - 1 have been read
+    fl_sync();
+    if constexpr (QK) {
+#pragma unroll
+      for (int u = 0; u < KR - 1; ++u) kread(u, 1 - S);
+      load_k(i + 2, ring + S * L::K);
+      load_v(i + 1, ring + 2 * L::K + (1 - S) * L::V);
+    }
+#pragma unroll
+    for (int u = 0; u < NQ; ++u) {
+      if constexpr (QK) {
+        const int t = u & 1, s = u >> 1;
+        nxt[t] = fl_mfma(kf[u % KR], qr[s], s == 0 ? zero : nxt[t]);
+        if (u + KR - 1 < NQ) kread(u + KR - 1, 1 - S);
+      }
+      if constexpr (SM) {
+        exps(0, u, NQ);
+        if (u >= NQ - (VR - 1)) vread(u - (NQ - (VR - 1)));
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // what is used in a later block stays computed in this one
+    if constexpr (SM) asm volatile("" : "+v"(pf[0][0]), "+v"(pf[0][1]));
+    if constexpr (QK) prep(nxt, i + 1);
+    if constexpr (SM) {
+#pragma unroll
+      for (int w = 0; w < NP; ++w) {
+        pv(0, w);
+        exps(1, w, NP);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    float mx[2] = {-INFINITY, -INFINITY};
+#pragma unroll
+    for (int w = 0; w < NP; ++w) {
+      if constexpr (SM) pv(1, w);
+      if constexpr (QK) {
+#pragma unroll
+        for (int q = w * 16 / NP; q < (w + 1) * 16 / NP; ++q)
+          mx[q & 1] = fmaxf(fmaxf(mx[q & 1], nxt[q >> 3][2 * (q & 7)]), nxt[q >> 3][2 * (q & 7) + 1]);
+      }
+      if constexpr (SM) __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (SM && ROW) l += ls[0];
+    if constexpr (QK) {
+      const float top = fl_max32(fmaxf(mx[0], mx[1])) * sl2;
+      if (__any(top > m)) {
+        const float m_new = fmaxf(m, top), alpha = __builtin_amdgcn_exp2f(m - m_new);
+        m = m_new;
+        l *= alpha;
+#pragma unroll
+        for (int d = 0; d < NDT; ++d) {
+#pragma unroll
+          for (int j = 0; j < 16; ++j) acc[d][j] *= alpha;
+          asm volatile("" : "+v"(acc[d]));              // one value, so that no path copies it
+        }
+      }
+    }
+  };
+
+  if (n <= 0) return;
+  float16v sa[2], sb[2];
+  load_k(0, ring);
+  body(Fl<1>{}, Fl<0>{}, Fl<1>{}, sb, sa, -1);         // scores of tile 0; fetches K 1 and V 0
+  int i = 0;
+  for (; i + 2 < n; i += 2) {
+    body(Fl<1>{}, Fl<1>{}, Fl<0>{}, sa, sb, i);
+    body(Fl<1>{}, Fl<1>{}, Fl<1>{}, sb, sa, i + 1);
+  }
+  if (i + 1 < n) {
+    body(Fl<1>{}, Fl<1>{}, Fl<0>{}, sa, sb, i);
+    sa[0] = sb[0];
+    sa[1] = sb[1];
+#pragma unroll
+    for (int d = 0; d < NDT; ++d) vb[d] += L::V;        // the last tile's V lies in the other stage
+  }
+  body(Fl<0>{}, Fl<1>{}, Fl<0>{}, sa, sb, n - 1);
+  if constexpr (!ROW) l = fl_both32(l);                 // a lane has summed its half of the keys
+}
+
+// ---- the end of a pass. The KS runs of a query block meet in LDS: run 0 leaves with the
+// joint (m, l, acc) of its QW waves. Called by all waves, the rings no longer in use.
+__host__ __device__ constexpr int fl_merge_bytes(int NDT, int QW, int KS) { return (KS - 1) * QW * (NDT * 16 + 2) * 256; }
+
+template <int NDT, int QW, int KS>
+__device__ __forceinline__ void fl_merge(float16v (&acc)[NDT], float& m, float& l, float* x, int run, int wq, int lane) {
+  if constexpr (KS > 1) {
+    constexpr int PER = (NDT * 16 + 2) * 64;
+    if (run) {
+      float* my = x + ((run - 1) * QW + wq) * PER + lane;
+#pragma unroll
+      for (int d = 0; d < NDT; ++d)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) my[(d * 16 + j) * 64] = acc[d][j];
+      my[NDT * 16 * 64] = m;
+      my[(NDT * 16 + 1) * 64] = l;
+    }
+    fl_sync();
+    if (run) return;
+#pragma unroll
+    for (int r = 1; r < KS; ++r) {
+      const float* o = x + ((r - 1) * QW + wq) * PER + lane;
+      const float m1 = o[NDT * 16 * 64], l1 = o[(NDT * 16 + 1) * 64];
+      const float top = fmaxf(m, m1), a0 = exp2f(m - top), a1 = exp2f(m1 - top);
+      m = top;
+      l = l * a0 + l1 * a1;
+#pragma unroll
+      for (int d = 0; d < NDT; ++d)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) acc[d][j] = acc[d][j] * a0 + o[(d * 16 + j) * 64] * a1;
+    }
+  }
+}
+
+// A wave's 32 rows as bf16 to y (rows ld apart, `rows` of them exist, `cols` <= 32 NDT columns,
+// a multiple of 8), turned through LDS: a lane's accumulators are 4 columns of its row, and 8-byte
+// pieces of 32 rows in one store make every piece a line of its own.
+__host__ __device__ constexpr int fl_store_bytes(int NDT) { return 32 * (NDT * 64 + 16); }
+
+template <int NDT>
+__device__ __forceinline__ void fl_store(const float16v (&acc)[NDT], unsigned char* my, bf16_t* y, long long ld, int rows,
+                                         int cols, int lane) {
+  constexpr int LD = NDT * 64 + 16, CPR = NDT * 4;
+  const int h = lane >> 5;
+#pragma unroll
+  for (int d = 0; d < NDT; ++d)
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      *reinterpret_cast<uint2*>(my + (lane & 31) * LD + (32 * d + 8 * g + 4 * h) * 2) =
+          make_uint2(pack_bf16x2(acc[d][4 * g], acc[d][4 * g + 1]), pack_bf16x2(acc[d][4 * g + 2], acc[d][4 * g + 3]));
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll
+  for (int k = 0; k < 32 * CPR / 64; ++k) {
+    const int id = lane + 64 * k, r = id / CPR, c = id % CPR;
+    const fl_u4 v = *reinterpret_cast<const fl_u4*>(my + r * LD + c * 16);
+    if (r < rows && c * 8 < cols) *reinterpret_cast<fl_u4*>(y + (size_t)r * ld + c * 8) = v;
+  }
+}

@@ -104,7 +104,7 @@ def build(force: bool = False, debug: bool = False, only=None, quiet: bool = Fal
     ksrc = [p for p in allk if os.path.basename(p) not in SEQMIX_SOURCES]
     allh = sorted(glob.glob(os.path.join(CSRC, "kernels", "*.h")))
     khdr = [p for p in allh if os.path.basename(p) != "seqmix.h"]
-    shdr = [p for p in allh if os.path.basename(p) in ("common.h", "seqmix.h", "gemm_pipe.h")]
+    shdr = [p for p in allh if os.path.basename(p) in ("common.h", "seqmix.h", "gemm_pipe.h", "flash_pipe.h")]
     rsrc = sorted(glob.glob(os.path.join(CSRC, "runtime", "*.cpp")))
     rhdr = sorted(glob.glob(os.path.join(CSRC, "runtime", "*.h")))
     rflags = [*opt, "-std=c++17", "-D__HIP_PLATFORM_AMD__"]

@@ -1,7 +1,6 @@
-"""Prefill / encoder attention (attn_prefill2_kernel): device time per call on the Whisper-large-v3
+"""Prefill / encoder attention (attn_pipe_kernel): device time per call on the Whisper-large-v3
 encoder (1500 frames, 20 heads, D 64) and Llama-3-8B prompt (GQA 32/8, D 128,
-causal) shapes, plus max error vs the fp32 reference. LOQA_ATTN_V1=1 selects
-the 4-wave kernel."""
+causal) shapes, plus max error vs the fp32 reference."""
 import json
 import os
 import sys
@@ -42,4 +41,4 @@ for name, (B, T, H, Hkv, D, causal) in cases.items():
     fl = 4 * B * T * T * D * H * (0.5 if causal else 1.0)
     res[name] = {"us": round(us, 1), "TF": round(fl / us / 1e6), "max_err": round(err, 4)}
     print(name, res[name], flush=True)
-print(json.dumps({"v1": bool(os.environ.get("LOQA_ATTN_V1")), **res}))
+print(json.dumps(res))

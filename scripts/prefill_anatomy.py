@@ -1,7 +1,7 @@
 """Per-pass anatomy of the LLM prompt prefill from a rocprofv3 kernel trace.
 
 A Llama prefill pass is recognised by its causal flash-attention kernels
-(``attn_prefill2_kernel<128, true>``, one per layer; the Whisper encoder's
+(``attn_pipe_kernel<128, ..>``, one per layer; the Whisper encoder's
 are non-causal D = 64). For each pass: GPU span (first to last kernel of the
 pass on its queue, so time other engines' kernels interleave is included),
 summed kernel time of the pass's own queue inside the span, the idle gaps on
@@ -16,7 +16,7 @@ import sys
 
 
 # kernels only the Llama prefill launches (its hipBLASLt GEMMs are shared names)
-LLM_PREFILL = ("attn_prefill2_kernel<128, true>", "rope_kv_append", "rmsnorm", "silu_mul",
+LLM_PREFILL = ("attn_pipe_kernel<128", "rope_kv_append", "rmsnorm", "silu_mul",
                "gemm_prefill2_kernel", "slab_rope_append")
 
 
@@ -31,7 +31,7 @@ def main(path, layers=32):
             rows.append((int(r["Start_Timestamp"]), int(r["End_Timestamp"]), (r["Queue_Id"], r["Stream_Id"]),
                          r["Kernel_Name"]))
     rows.sort()
-    attn = [i for i, r in enumerate(rows) if "attn_prefill2_kernel<128, true>" in r[3]]
+    attn = [i for i, r in enumerate(rows) if "attn_pipe_kernel<128" in r[3]]
     if not attn:
         print("no LLM prefill passes in the trace")
         return

@@ -1,0 +1,90 @@
+"""The pipelined attention kernel (csrc/kernels/flash_pipe.h, attention.hip) at the edges of its
+tiles, key runs and pages, against float64.
+
+Bound: the weights are rounded to bf16 (relative 2^-9) in the numerator and in their sum, the
+result once more; scores and sums are f32. |error| <= 3 * 2^-9 * sum(p |v|) / sum(p) + f32 noise."""
+import math
+
+import pytest
+import torch
+
+from loqa_hub_amd import ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _check(qlens, klens, Hq, Hkv, D, causal, page=0, q_pad=0, shift=0, seed=0, spread=1.0):
+    g = torch.Generator().manual_seed(seed)
+    B, Tq, Tk = len(qlens), sum(qlens), sum(klens)
+    q = (spread * torch.randn(Tq, Hq * D + q_pad, generator=g)).bfloat16().to(DEV)
+    k = torch.randn(Tk, Hkv, D, generator=g).bfloat16().to(DEV)
+    v = torch.randn(Tk, Hkv, D, generator=g).bfloat16().to(DEV)
+    cu = lambda x: torch.tensor([0] + x).cumsum(0).int().to(DEV)
+    kw = dict(n_heads=Hq, n_kv=Hkv, head_dim=D, causal=causal, max_q=max(qlens))
+    cq, ck = cu(qlens), cu(klens)
+    if page:
+        per = [-(-x // page) for x in klens]
+        ids = torch.randperm(sum(per) + 3, generator=g).int()
+        bt = torch.zeros(B, max(per), dtype=torch.int32)
+        kc = torch.full((sum(per) + 3, Hkv, page, D), float("nan"), dtype=torch.bfloat16, device=DEV)
+        vc = kc.clone()
+        at = 0
+        for b, n in enumerate(klens):
+            for x in range(per[b]):
+                bt[b, x] = ids[at]
+                m = min(page, n - x * page)
+                rows = slice(int(ck[b]) + x * page, int(ck[b]) + x * page + m)
+                kc[ids[at], :, :m], vc[ids[at], :, :m] = k[rows].transpose(0, 1), v[rows].transpose(0, 1)
+                at += 1
+        ctx = torch.tensor(klens, dtype=torch.int32, device=DEV)
+        o = ops.attention(q, kc, vc, cq, ctx_lens=ctx, block_tables=bt.to(DEV), max_k=max(klens), **kw)
+    else:
+        o = torch.empty(Tq, Hq * D + shift, dtype=torch.bfloat16, device=DEV)[:, shift:]
+        ops.attention(q, k.view(Tk, -1), v.view(Tk, -1), cq, cu_k=ck, out=o, **kw)
+    for b, (n, m) in enumerate(zip(qlens, klens)):
+        qs = q[int(cq[b]):int(cq[b]) + n, :Hq * D].double().view(n, Hq, D).transpose(0, 1)
+        ks = k[int(ck[b]):int(ck[b]) + m].double().repeat_interleave(Hq // Hkv, 1).permute(1, 2, 0).contiguous()
+        vs = v[int(ck[b]):int(ck[b]) + m].double().repeat_interleave(Hq // Hkv, 1).transpose(0, 1).contiguous()
+        s = torch.bmm(qs, ks) / math.sqrt(D)
+        if causal:
+            away = torch.arange(m, device=DEV)[None] - (torch.arange(n, device=DEV)[:, None] + m - n)
+            s.masked_fill_(away > 0, -math.inf)
+        p = s.softmax(-1)
+        want, size = torch.bmm(p, vs), torch.bmm(p, vs.abs())
+        got = o[int(cq[b]):int(cq[b]) + n].double().view(n, Hq, D).transpose(0, 1)
+        assert ((got - want).abs() <= 3 * 2.0 ** -9 * size + 1e-5).all(), (b, n, m)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("causal", [False, True])
+def test_tiles_and_runs(D, causal):
+    # row blocks of 32, one to five key tiles (every way they split into runs), and their edges
+    lens = [1, 2, 31, 32, 33, 63, 64, 65, 127, 128, 129, 191, 192, 193, 256, 257, 319]
+    _check(lens, lens, 4, 2, D, causal)
+    _check([1, 5, 40, 64, 3], [64, 197, 129, 321, 1500], 2, 1, D, causal, seed=1)
+    _check([70], [70], 4, 2, D, causal, q_pad=8, seed=2)
+
+
+@pytest.mark.parametrize("D,B,H,n", [(64, 1, 20, 1500), (64, 3, 20, 1500), (128, 1, 32, 520), (128, 5, 32, 520)])
+def test_every_block_height(D, B, H, n):
+    # the grids that take 128 rows with two runs, and 128 rows with one
+    _check([n] * B, [n] * B, H, H // 4, D, D == 128, seed=3)
+
+
+@pytest.mark.parametrize("page", [1, 8, 16, 24, 32, 64, 128, 1024])
+@pytest.mark.parametrize("D", [64, 128])
+def test_pages(D, page):
+    # unused rows of a page hold NaN; more than 64 pages a sequence where they are small
+    _check([1, 7, 65, 130], [700, 7, 1100, 193], 4, 2, D, True, page=page, seed=4)
+
+
+def test_peaked_and_flat():
+    for spread in (0.0, 1e-3, 30.0):
+        _check([100], [300], 2, 2, 64, False, seed=5, spread=spread)
+        _check([100], [300], 2, 2, 128, True, seed=6, spread=spread)
+
+
+def test_rows_off_16_bytes_take_the_other_kernel():
+    _check([50, 9], [50, 200], 2, 2, 64, True, q_pad=4, seed=7)
+    _check([50, 9], [50, 200], 2, 2, 128, False, shift=4, seed=8)
