@@ -45,8 +45,9 @@
 // contexts the windows are also dealt out to several workgroups per row, whose
 // partial triples a small combine launch merges.
 //
-// window_attn_mfma_kernel (bf16, D up to 256 and Dv up to 512 in multiples of 8,
-// padded with zeros in LDS to the next built size; prompt portions): a
+// window_attn_pipe_kernel (attn_window_pipe.hip; bf16, D up to 128 and Dv up to 512 in
+// multiples of 8, 16-byte rows, pages of 8, 16, 32, .. keys; prompt portions), and
+// window_attn_mfma_kernel (D up to 256, any page size, rows of 4-byte alignment): a
 // workgroup per (64, 128 or 256 query rows of one sequence, query head, up to 128
 // of its value columns: wider values are shared out, every part forming the scores
 // again); each wave owns 32 rows. The block-table entries of the key range go to LDS once.
@@ -57,18 +58,6 @@
 // between the kept first tokens and the rows' windows are skipped, and a tile
 // that every row of a wave sees whole takes a path without per-score tests.
 #include "seqmix.h"
-
-struct WinAttnParams {
-  const void* q; const void* kc; const void* vc; int blk; long cache_rows;
-  const int* cu_q; const int* ctx; const int* bt; int max_blocks; const int* pos;
-  const void* gate; long gate_ld; float scale, cap; int window, keep_first;
-  int B, T, H, G, D, Dv; void* o;
-  int ns; float* part;               // key splits over workgroups and their partial results
-  const float* sink;                 // [H] or null: exp(sink[h]) joins head h's softmax denominator
-  const float* slopes;               // [H] or null: slopes[h] * (i - j) comes off head h's score
-  long o_ld;                         // row stride of o (head h at column h * Dv)
-  int vparts;                        // matrix-core form: workgroups that share a head's value columns
-};
 
 // K / V pages (and the block table) are read through pointers in the global
 // address space: a load through a generic pointer counts against the LDS
@@ -589,9 +578,9 @@ __device__ __forceinline__ float tanh_fast(float z) {
   return 1.f - 2.f * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(2.885390081777927f * z));
 }
 
-// DK, DV: the sizes in LDS and registers. PAD: the model's key size p.D <= DK or the
-// workgroup's value columns (<= DV) are fewer (multiples of 8); the rest is zero.
-template <int DK, int DV, int WM_WAVES, bool PAD>
+// DK, DV: the sizes in LDS and registers; the model's key size p.D <= DK and the
+// workgroup's value columns (<= DV) may be fewer (multiples of 8), the rest is zero.
+template <int DK, int DV, int WM_WAVES>
 __global__ __launch_bounds__(64 * WM_WAVES) void window_attn_mfma_kernel(WinAttnParams p) {
   __shared__ __attribute__((aligned(16))) WinMfmaSmem<DK, DV> sm;
   __shared__ int pages[WM_MAXPG];
@@ -601,7 +590,7 @@ __global__ __launch_bounds__(64 * WM_WAVES) void window_attn_mfma_kernel(WinAttn
   const int head = (int)blockIdx.y / p.vparts, b = blockIdx.z;
   const int v0 = ((int)blockIdx.y % p.vparts) * DV;    // this workgroup's value columns
   const int g = head / (p.H / p.G);
-  const int D = PAD ? p.D : DK, Dv = PAD ? min(DV, p.Dv - v0) : DV;
+  const int D = p.D, Dv = min(DV, p.Dv - v0);
   const int q0 = p.cu_q[b], qlen = p.cu_q[b + 1] - q0;
   // long row blocks (the most keys) start first
   const int nblk = (int)gridDim.x;
@@ -630,7 +619,7 @@ __global__ __launch_bounds__(64 * WM_WAVES) void window_attn_mfma_kernel(WinAttn
                          (size_t)head * D;
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-      uint4 v = valid && (!PAD || 16 * s + 8 * h < D)
+      uint4 v = valid && 16 * s + 8 * h < D
                     ? *reinterpret_cast<const uint4*>(qrow + 16 * s + 8 * h) : make_uint4(0, 0, 0, 0);
       qf[s] = *reinterpret_cast<bf16x8*>(&v);
     }
@@ -672,14 +661,14 @@ __global__ __launch_bounds__(64 * WM_WAVES) void window_attn_mfma_kernel(WinAttn
 #pragma unroll
     for (int j = 0; j < NKC; ++j) {
       const int c = threadIdx.x + WM_THREADS * j, kr = c / CHK, cc = (c - kr * CHK) * 8;
-      pk[j] = kt + kr < kend && (!PAD || cc < D)
+      pk[j] = kt + kr < kend && cc < D
                   ? *reinterpret_cast<const WA_GLOBAL wa_u32x4*>(kbase + page_row(kt + kr) * kst + cc)
                   : wa_u32x4{0, 0, 0, 0};
     }
 #pragma unroll
     for (int j = 0; j < NVC; ++j) {
       const int c = threadIdx.x + WM_THREADS * j, kr = c / CHV, cc = (c - kr * CHV) * 8;
-      pv[j] = kt + kr < kend && (!PAD || cc < Dv)
+      pv[j] = kt + kr < kend && cc < Dv
                   ? *reinterpret_cast<const WA_GLOBAL wa_u32x4*>(vbase + page_row(kt + kr) * vst + cc)
                   : wa_u32x4{0, 0, 0, 0};
     }
@@ -816,7 +805,7 @@ __global__ __launch_bounds__(64 * WM_WAVES) void window_attn_mfma_kernel(WinAttn
 #pragma unroll
     for (int g8 = 0; g8 < 4; ++g8) {
       const int d0 = 32 * dt + 8 * g8 + 4 * h;
-      if (PAD && d0 >= Dv) continue;
+      if (d0 >= Dv) continue;
       float o4[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) o4[i] = acc[dt][4 * g8 + i] * inv;
@@ -838,32 +827,18 @@ int window_attention_mfma(const WinAttnParams& p0, int max_q, hipStream_t st) {
   if (max_q <= 0) return 0;
   WinAttnParams p = p0;
   p.vparts = (p.Dv + 127) / 128;
-  // the widest row block the longest feed fills: the tiles' staging (gather
-  // through the page table, LDS stores, barriers) is paid once per block and
-  // tile, and measured times fall with the block width even when the grid
-  // shrinks below the number of compute units
-  const int waves = max_q > 128 ? 8 : (max_q > 64 ? 4 : 2);
+  const int rc = window_attention_pipe(p, max_q, st);
+  if (rc >= 0) return rc;
+  // other sizes and places: the next built size, in two block widths (the tiles' staging is
+  // paid once per block and tile)
+  const int waves = max_q > 128 ? 8 : 2;
   const dim3 grid((max_q + waves * 32 - 1) / (waves * 32), p.H * p.vparts, p.B);
-#define GO(A, C)                                                                              \
-  if (p.D == A && (p.Dv == C || (C == 128 && p.Dv % C == 0))) {                                                              \
-    if (waves == 8)                                                                           \
-      hipLaunchKernelGGL((window_attn_mfma_kernel<A, C, 8, false>), grid, dim3(512), 0, st, p); \
-    else if (waves == 4)                                                                      \
-      hipLaunchKernelGGL((window_attn_mfma_kernel<A, C, 4, false>), grid, dim3(256), 0, st, p); \
-    else                                                                                      \
-      hipLaunchKernelGGL((window_attn_mfma_kernel<A, C, 2, false>), grid, dim3(128), 0, st, p); \
-    return (int)hipGetLastError();                                                            \
-  }
-  GO(64, 64) GO(128, 64) GO(64, 128) GO(128, 128)
-#undef GO
-  // other sizes: the next built size, in two block widths
-  const dim3 grid_p = waves == 8 ? grid : dim3((max_q + 63) / 64, p.H * p.vparts, p.B);
 #define GO(A, C)                                                                              \
   if (p.D <= A && (p.Dv <= C || C == 128)) {                                                              \
     if (waves == 8)                                                                           \
-      hipLaunchKernelGGL((window_attn_mfma_kernel<A, C, 8, true>), grid_p, dim3(512), 0, st, p); \
+      hipLaunchKernelGGL((window_attn_mfma_kernel<A, C, 8>), grid, dim3(512), 0, st, p);      \
     else                                                                                      \
-      hipLaunchKernelGGL((window_attn_mfma_kernel<A, C, 2, true>), grid_p, dim3(128), 0, st, p); \
+      hipLaunchKernelGGL((window_attn_mfma_kernel<A, C, 2>), grid, dim3(128), 0, st, p);      \
     return (int)hipGetLastError();                                                            \
   }
   GO(64, 64) GO(64, 128) GO(128, 64) GO(128, 128) GO(256, 64) GO(256, 128)

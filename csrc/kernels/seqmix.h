@@ -2,7 +2,7 @@
 // (norm_dyt.hip, attn_latent.hip, lightning.hip, moe.hip, seq_rows.hip,
 // attn_sigmoid.hip, norm_scalar.hip, norm_rms1p.hip, attn_window.hip, mamba2.hip,
 // matrix_memory.hip, delta_rule.hip, norm_layer.hip, linear_chunks.hip,
-// delta_chunks.hip).
+// delta_chunks.hip, moe_pipe.hip, attn_window_pipe.hip).
 //
 // Activations are bfloat16 or float32, chosen at run time by a dtype code
 // (0: bf16, 1: f32); every kernel is a template over the storage type and does
@@ -141,3 +141,18 @@ __device__ __forceinline__ int seq_chunks_before(const int* __restrict__ cu_q, i
 }
 
 static inline int ceil_div(long a, long b) { return (int)((a + b - 1) / b); }
+
+// windowed attention (attn_window.hip, attn_window_pipe.hip)
+struct WinAttnParams {
+  const void* q; const void* kc; const void* vc; int blk; long cache_rows;
+  const int* cu_q; const int* ctx; const int* bt; int max_blocks; const int* pos;
+  const void* gate; long gate_ld; float scale, cap; int window, keep_first;
+  int B, T, H, G, D, Dv; void* o;
+  int ns; float* part;               // key splits over workgroups and their partial results
+  const float* sink;                 // [H] or null: exp(sink[h]) joins head h's softmax denominator
+  const float* slopes;               // [H] or null: slopes[h] * (i - j) comes off head h's score
+  long o_ld;                         // row stride of o (head h at column h * Dv)
+  int vparts;                        // matrix-core form: workgroups that share a head's value columns
+};
+// Prompt portions on the pipelined tile loop; -1 where it does not take the sizes or places.
+int window_attention_pipe(const WinAttnParams& p, int max_q, hipStream_t st);

@@ -1,0 +1,101 @@
+"""Prompt portions of the windowed paged attention (csrc/kernels/attn_window_pipe.hip) at the edges
+of row blocks, key runs, windows, kept tokens, pages and head sizes, against float64.
+
+Bound: weights rounded to bf16 in numerator and sum (relative 2^-9 each), the gate through a
+1-ulp reciprocal, the result rounded once: |error| <= 4 * 2^-9 * sum(p |v|) / den + f32 noise
+(a soft cap moves scores by up to 2^-20 of the cap)."""
+import math
+
+import pytest
+import torch
+
+from loqa_hub_amd.ops import seqmix
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _check(feeds, pasts, H, G, D, Dv, window, keep=0, cap=0.0, slopes=False, sink=False, gate=False, blk=16, scale=None,
+           out_pad=0, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    B, T, lens = len(feeds), sum(feeds), [f + p for f, p in zip(feeds, pasts)]
+    per = [-(-n // blk) for n in lens]
+    scale = D ** -0.5 if scale is None else scale
+    q = torch.randn(T, H * D, generator=g).bfloat16().to(DEV)
+    kc = torch.full((sum(per) + 2, blk, G * D), float("nan"), dtype=torch.bfloat16)
+    vc = torch.full((sum(per) + 2, blk, G * Dv), float("nan"), dtype=torch.bfloat16)
+    ids = torch.randperm(sum(per) + 2, generator=g).int()
+    bt = torch.zeros(B, max(per), dtype=torch.int32)
+    ks, vs, at = [], [], 0
+    for b, n in enumerate(lens):
+        k, v = torch.randn(n, G * D, generator=g).bfloat16(), torch.randn(n, G * Dv, generator=g).bfloat16()
+        bt[b, :per[b]] = ids[at:at + per[b]]
+        at += per[b]
+        rows = (bt[b, :per[b]].long()[:, None] * blk + torch.arange(blk)).reshape(-1)[:n]
+        kc.view(-1, G * D)[rows], vc.view(-1, G * Dv)[rows] = k, v
+        ks.append(k.to(DEV).double().view(n, G, D))
+        vs.append(v.to(DEV).double().view(n, G, Dv))
+    cu = torch.tensor([0] + feeds).cumsum(0).int().to(DEV)
+    pos = torch.cat([torch.arange(p, p + f) for f, p in zip(feeds, pasts)]).int().to(DEV)
+    sk = torch.randn(H, generator=g).to(DEV) if sink else None
+    sl = (torch.rand(H, generator=g) * 0.02).to(DEV) if slopes else None
+    gt = torch.randn(T, H * Dv, generator=g).bfloat16().to(DEV) if gate else None
+    o = torch.empty(T, H * Dv + out_pad, dtype=torch.bfloat16, device=DEV)[:, :H * Dv]
+    seqmix.window_attention(q, kc.to(DEV), vc.to(DEV), cu, torch.tensor(lens, dtype=torch.int32, device=DEV), bt.to(DEV), pos,
+                            scale, cap, window, keep, gt, H, G, D, Dv, max_q=max(feeds), max_ctx=max(lens), matrix_cores=True,
+                            sink=sk, slopes=sl, out=o)
+    for b, (f, n) in enumerate(zip(feeds, lens)):
+        rows = slice(int(cu[b]), int(cu[b]) + f)
+        k = ks[b].repeat_interleave(H // G, 1).permute(1, 2, 0).contiguous()
+        v = vs[b].repeat_interleave(H // G, 1).transpose(0, 1).contiguous()
+        s = torch.bmm(q[rows].double().view(f, H, D).transpose(0, 1), k) * scale
+        if cap:
+            s = cap * torch.tanh(s / cap)
+        away = pos[rows, None] - torch.arange(n, device=DEV)[None]
+        if sl is not None:
+            s = s - sl.double()[:, None, None] * away
+        seen = away >= 0
+        if window:
+            seen &= (away < window) | (torch.arange(n, device=DEV)[None] < keep)
+        s = s.masked_fill(~seen, -math.inf)
+        top = s.amax(-1, keepdim=True)
+        if sk is not None:
+            top = torch.maximum(top, sk.double()[:, None, None])
+        p = (s - top).exp()
+        p = p / (p.sum(-1, keepdim=True) + ((sk.double()[:, None, None] - top).exp() if sk is not None else 0.0))
+        want, size = torch.bmm(p, v), torch.bmm(p, v.abs())
+        if gt is not None:
+            w = torch.sigmoid(gt[rows].double()).view(f, H, Dv).transpose(0, 1)
+            want, size = want * w, size * w
+        got = o[rows].double().view(f, H, Dv).transpose(0, 1)
+        assert ((got - want).abs() <= 4 * 2.0 ** -9 * size + 1e-5).all(), (b, f, n)
+
+
+@pytest.mark.parametrize("window,keep", [(0, 0), (1, 0), (64, 0), (100, 5), (100, 70), (300, 300), (65, 64)])
+@pytest.mark.parametrize("D,Dv", [(64, 64), (64, 128), (128, 64), (128, 128), (96, 72), (40, 256)])
+def test_windows(D, Dv, window, keep):
+    _check([1, 33, 64, 130, 257], [300, 0, 513, 31, 64], 4, 2, D, Dv, window, keep, sink=True, gate=True, seed=window)
+
+
+@pytest.mark.parametrize("blk", [1, 8, 16, 24, 64, 256])
+def test_pages(blk):
+    _check([70, 3, 200], [700, 90, 5], 4, 2, 128, 128, 128, 3, blk=blk, seed=blk)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("B,T,H", [(1, 300, 4), (2, 520, 40), (3, 900, 40)])
+def test_every_block_height(D, B, T, H):
+    _check([T] * B, [7] * B, H, 4, D, D, 200, 4, seed=T)
+
+
+@pytest.mark.parametrize("D,Dv", [(64, 64), (128, 128), (72, 48), (128, 40)])
+def test_transformed_scores(D, Dv):
+    _check([90, 40], [100, 0], 4, 2, D, Dv, 0, cap=20.0, seed=1)
+    _check([90, 40], [100, 0], 4, 2, D, Dv, 77, 2, slopes=True, sink=True, seed=2)
+    _check([90, 40], [100, 0], 4, 2, D, Dv, 77, 2, cap=5.0, slopes=True, gate=True, seed=3)
+    _check([50], [10], 4, 2, D, Dv, 0, scale=-0.1, seed=4)
+
+
+def test_other_places_take_the_other_kernel():
+    _check([60], [40], 4, 2, 64, 64, 0, out_pad=4, seed=5)
+    _check([60, 300], [40, 0], 4, 2, 192, 64, 100, 3, seed=6)
