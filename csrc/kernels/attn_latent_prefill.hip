@@ -3,29 +3,24 @@
 // For passes with many query rows the folded form (attn_latent.hip) would pay
 // R + Dr multiply-adds per score and R per value entry; here the keys and
 // values are first materialised per head from the gathered latent rows (two
-// vendor GEMMs: k_un = W_uk c, v = W_uv c), and a flash kernel in the manner of
-// attention.hip's attn_fwd_kernel runs over [key, head, DK] / [key, head, DV]:
-//   S^T = K Q^T (v_mfma_f32_32x32x16_bf16, the query on the MFMA lane so the
-//   online softmax is in-register), O^T += V^T P^T with the exp2'ed S^T as the
-//   B operand and V^T read from LDS with transposed reads.
-// Differences from the Llama kernel: DK != DV (rotary part only in the keys),
-// zero-padded head sizes (DK, DV are the next instantiated sizes), the causal
-// bound comes from each row's absolute position (with a sliding window the keys
-// before it are neither gathered nor visited), a learned per-head sink joins the
-// softmax denominator at the end, and the output gate sigmoid(gate) is applied
-// in the epilogue, which writes unpadded heads into rows of any stride.
+// vendor GEMMs: k_un = W_uk c, v = W_uv c), and the pipelined tile loop of the other prompt
+// attentions (flash_pipe.h) runs over [key, head, DK] / [key, head, DV].
+// What is its own: DK != DV (rotary part only in the keys), zero-padded head sizes (DK, DV are
+// the next instantiated sizes), the causal bound from each row's absolute position (with a
+// sliding window the keys before it are neither gathered nor visited), a learned per-head sink
+// in the softmax denominator, and the output gate sigmoid(gate), applied before the unpadded
+// heads go to rows of any stride.
+// 2048 rows of 16 heads, 192 / 128: 99.5 us before (128 rows in four waves, tiles through
+// registers, scores, exponentials and products one after the other), 55 now; 4 x that: 365, 120;
+// 256 / 128: 111, 75. A single prompt is one round of the CUs, as long as its last rows (32
+// tiles, 16.5 on average); smaller blocks with one wave a SIMD were no faster.
 //
 // Helpers: latent_gather_kernel copies the last cu_k[b + 1] - cu_k[b] latent rows
 // of each sequence from its pages into contiguous [sum L, R] / [sum L, Dr] buffers; latent_kfill_kernel
 // writes the shared rotary key part into every head's key row;
 // rope_pairs_kernel rotates the queries' rotary part in place.
+#include "flash_pipe.h"
 #include "seqmix.h"
-
-#define LP_THREADS 256
-#define LP_WAVES 4
-#define LP_TILE 64
-
-typedef short lp_v4s __attribute__((ext_vector_type(4)));
 
 struct LatPrefillParams {
   const bf16_t* q; long q_st;       // [T, H, DK]
@@ -37,45 +32,59 @@ struct LatPrefillParams {
   const float* sink; float scale_log2;
   int H, Dv, window;
   const bf16_t* gate; long gate_ld; // [T, H * Dv] or null
-  int runs;                         // output and gate rows can be accessed in runs of four
+  int runs, rows16;                 // gate rows can be read in runs of four, output rows written in runs of eight
 };
 
-template <int DK, int DV>
-struct LatPrefillSmem {
-  bf16_t k[LP_TILE][DK + 8];
-  bf16_t v[LP_TILE][DV + 32];
-};
-
-template <int DK, int DV>
-__global__ __launch_bounds__(LP_THREADS) void latent_prefill_kernel(LatPrefillParams p) {
-  __shared__ __attribute__((aligned(16))) LatPrefillSmem<DK, DV> sm;
-  constexpr int NS = DK / 16, NDT = DV / 32;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, h = lane >> 5;
-  const int head = blockIdx.y, b = blockIdx.z;
+// QW blocks of 32 query rows, the keys in KS runs. At 192 / 128 a run's ring is 80 KB of LDS and a
+// tile's working set with two waves a SIMD all of the registers; the 256-column keys take one wave.
+template <int DK, int DV, int QW, int KS>
+__global__ __launch_bounds__(64 * QW * KS, DK > 192 ? 1 : 2) void latent_prefill_kernel(LatPrefillParams p) {
+  using L = FlashLds<DK, DV>;
+  constexpr int NS = DK / 16, NDT = DV / 32, NTH = 64 * QW;
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int run = wave / QW, wq = wave % QW, th = threadIdx.x - run * NTH, h = lane >> 5;
+  int bx, head, b;
+  {
+    // row blocks with the most keys first, over all heads of an XCD where these are whole
+    const int gx = gridDim.x, gy = gridDim.y, heads = gy * gridDim.z;
+    const int at = xcd_remap(blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z), gx * heads);
+    int hd = at / gx;
+    bx = at - hd * gx;
+    if (heads % 8 == 0) {
+      const int hp = heads / 8, xcd = at / (hp * gx), in = at - xcd * hp * gx;
+      bx = in / hp;
+      hd = xcd * hp + in - bx * hp;
+    }
+    bx = gx - 1 - bx;
+    b = hd / gy;
+    head = hd - b * gy;
+  }
   const int q0 = p.cu_q[b], qlen = p.cu_q[b + 1] - q0;
-  const int row_lo = blockIdx.x * (LP_WAVES * 32);
-  if (row_lo >= qlen) return;
-  const int row_hi = min(qlen - 1, row_lo + LP_WAVES * 32 - 1);
+  const int row_lo = bx * (32 * QW);
+  if (row_lo >= qlen) return;                             // whole workgroup: uniform
+  const int row_hi = min(qlen - 1, row_lo + 32 * QW - 1);
   const int k0 = p.cu_k[b], klen = p.cu_k[b + 1] - k0;
   const int koff = p.ctx[b] - klen;                       // position of the buffer's first key
-  const int qi = row_lo + wave * 32 + (lane & 31);
+  const int qi = row_lo + wq * 32 + (lane & 31);
   const bool valid = qi < qlen;
   // positions relative to the buffer's first key
-  const int qpos = p.pos[q0 + (valid ? qi : row_hi)] - koff;
+  const int qpos = p.pos[q0 + min(qi, row_hi)] - koff;
   const int kend = min(klen, p.pos[q0 + row_hi] - koff + 1);   // positions grow along a sequence
-  const int first = p.window > 0 ? max(0, p.pos[q0 + row_lo] - koff - p.window + 1) : 0;
-  const int kt0 = first / LP_TILE * LP_TILE;
+  const int kt0 = p.window > 0 ? max(0, p.pos[q0 + row_lo] - koff - p.window + 1) / FL_KEYS * FL_KEYS : 0;
+  const int ntiles = kend > kt0 ? (kend - kt0 + FL_KEYS - 1) / FL_KEYS : 0;
   // what this wave's rows see at all
-  const int wpos_lo = p.pos[q0 + min(row_lo + wave * 32, row_hi)] - koff;
-  const int wpos_hi = p.pos[q0 + min(row_lo + wave * 32 + 31, row_hi)] - koff;
+  const int wpos_lo = __builtin_amdgcn_readfirstlane(p.pos[q0 + min(row_lo + wq * 32, row_hi)]) - koff;
+  const int wpos_hi = __builtin_amdgcn_readfirstlane(p.pos[q0 + min(row_lo + wq * 32 + 31, row_hi)]) - koff;
+  const int per = (ntiles + KS - 1) / KS, first = run * per;
 
   bf16x8 qf[NS];
   {
-    const bf16_t* qrow = p.q + (size_t)(q0 + (valid ? qi : row_hi)) * p.q_st + (size_t)head * DK;
+    const bf16_t* qrow = p.q + (size_t)(q0 + min(qi, row_hi)) * p.q_st + (size_t)head * DK;
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-      uint4 v = valid ? *reinterpret_cast<const uint4*>(qrow + 16 * s + 8 * h) : make_uint4(0, 0, 0, 0);
-      qf[s] = *reinterpret_cast<bf16x8*>(&v);
+      const uint4 v = valid ? *reinterpret_cast<const uint4*>(qrow + 16 * s + 8 * h) : make_uint4(0, 0, 0, 0);
+      qf[s] = *reinterpret_cast<const bf16x8*>(&v);
     }
   }
   float16v acc[NDT];
@@ -83,173 +92,98 @@ __global__ __launch_bounds__(LP_THREADS) void latent_prefill_kernel(LatPrefillPa
   for (int i = 0; i < NDT; ++i)
 #pragma unroll
     for (int j = 0; j < 16; ++j) acc[i][j] = 0.f;
-  float m_run = -1e30f, l_run = 0.f;
-  constexpr int CHK = DK / 8, CHV = DV / 8;
-  const size_t kst = (size_t)p.H * DK, vst = (size_t)p.H * DV;
-  const bf16_t* kbase = p.k + (size_t)k0 * kst + (size_t)head * DK;
-  const bf16_t* vbase = p.v + (size_t)k0 * vst + (size_t)head * DV;
-
-  // K / V tiles go through registers: the next tile's 16-byte chunks are
-  // requested before this tile's math and stored to LDS after it
-  constexpr int NKC = LP_TILE * CHK / LP_THREADS, NVC = LP_TILE * CHV / LP_THREADS;
-  uint4 pk[NKC], pv[NVC];
-  auto fetch = [&](int kt) {
-#pragma unroll
-    for (int j = 0; j < NKC; ++j) {
-      const int c = threadIdx.x + LP_THREADS * j, kr = c / CHK, cc = (c - kr * CHK) * 8;
-      pk[j] = kt + kr < kend ? *reinterpret_cast<const uint4*>(kbase + (size_t)(kt + kr) * kst + cc)
-                             : make_uint4(0, 0, 0, 0);
-    }
-#pragma unroll
-    for (int j = 0; j < NVC; ++j) {
-      const int c = threadIdx.x + LP_THREADS * j, kr = c / CHV, cc = (c - kr * CHV) * 8;
-      pv[j] = kt + kr < kend ? *reinterpret_cast<const uint4*>(vbase + (size_t)(kt + kr) * vst + cc)
-                             : make_uint4(0, 0, 0, 0);
+  float m = -1e30f, l = 0.f;
+  // where a fetch stands: tiles come in order; past the last one it stays there
+  const FlFetch<DK, NTH, false, false> kf(th, DK, (long long)p.H * DK);
+  const FlFetch<DV, NTH, true, false> vf(th, DV, (long long)p.H * DV);
+  struct At {
+    const bf16_t* row;
+    int kt;
+  };
+  const int at0 = kt0 + max(min(first, ntiles - 1), 0) * FL_KEYS;
+  At ka{p.k + ((size_t)(k0 + at0) * p.H + head) * DK, at0}, va{p.v + ((size_t)(k0 + at0) * p.H + head) * DV, at0};
+  auto fetch = [&](const auto& f, At& a, int cols, unsigned stage) __attribute__((always_inline)) {
+    const int last = kend - 1 - a.kt;
+    f.strided(stage, a.row, last);
+    if (last >= FL_KEYS) {
+      a.row += (size_t)FL_KEYS * p.H * cols;
+      a.kt += FL_KEYS;
     }
   };
-  fetch(kt0);
-  for (int kt = kt0; kt < kend; kt += LP_TILE) {
-    __syncthreads();
+  const bool neg = !(p.scale_log2 > 0.f);                 // the loop's maxima are of growing scores
+  fl_loop<DK, DV>(
+      qf, acc, m, l, fl_lds_at(lds) + run * L::RING, per, neg ? 1.f : p.scale_log2, lane,
+      [&](float16v(&st)[2], int i) __attribute__((always_inline)) {
+        const int kt = kt0 + (first + i) * FL_KEYS;       // tiles past the last lie behind kend
+        if (neg) {
 #pragma unroll
-    for (int j = 0; j < NKC; ++j) {
-      const int c = threadIdx.x + LP_THREADS * j, kr = c / CHK, cc = (c - kr * CHK) * 8;
-      *reinterpret_cast<uint4*>(&sm.k[kr][cc]) = pk[j];
-    }
+          for (int t = 0; t < 2; ++t)
 #pragma unroll
-    for (int j = 0; j < NVC; ++j) {
-      const int c = threadIdx.x + LP_THREADS * j, kr = c / CHV, cc = (c - kr * CHV) * 8;
-      *reinterpret_cast<uint4*>(&sm.v[kr][cc]) = pv[j];
-    }
-    __syncthreads();
-    if (kt + LP_TILE < kend) fetch(kt + LP_TILE);
-    // a wave whose rows see nothing of this tile only keeps the barriers
-    // (a scalar branch: matrix instructions ignore the lane mask)
-    if (__builtin_amdgcn_readfirstlane(
-            kt > wpos_hi || (p.window > 0 && kt + LP_TILE <= wpos_lo - p.window + 1)))
-      continue;
-
-    float16v st[2];
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-#pragma unroll
-      for (int j = 0; j < 16; ++j) st[t][j] = 0.f;
-#pragma unroll
-      for (int s = 0; s < NS; ++s) {
-        const bf16x8 a = *reinterpret_cast<const bf16x8*>(&sm.k[32 * t + (lane & 31)][16 * s + 8 * h]);
-        st[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, qf[s], st[t], 0, 0, 0);
-      }
-    }
-    bf16x8 pf[2][2];
-    {
-      float mx = -INFINITY;
-      // a tile that every row of this wave sees whole needs no per-score tests
-      const bool whole = kt + LP_TILE - 1 <= wpos_lo && kt + LP_TILE <= kend &&
-                         (p.window <= 0 || wpos_hi - kt < p.window);
-      if (__builtin_amdgcn_readfirstlane(whole)) {
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-          for (int j = 0; j < 16; ++j) {
-            st[t][j] *= p.scale_log2;
-            mx = fmaxf(mx, st[t][j]);
-          }
-      } else {
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-          for (int j = 0; j < 16; ++j) {
-            const int key = kt + 32 * t + (j & 3) + 8 * (j >> 2) + 4 * h;
-            float sv = st[t][j] * p.scale_log2;
-            if (key >= kend || key > qpos || (p.window > 0 && qpos - key >= p.window)) sv = -INFINITY;
-            st[t][j] = sv;
-            mx = fmaxf(mx, sv);
-          }
-      }
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-      const float m_new = fmaxf(m_run, mx);
-      // the hardware's exp2: the arguments are <= 0, and what falls below the
-      // normal range may flush to zero
-      const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-      float ls = 0.f;
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2)
-#pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            const float e = __builtin_amdgcn_exp2f(st[t][8 * s2 + j] - m_new);
-            ls += e;
-            pf[t][s2][j] = (__bf16)e;
-          }
-      ls += __shfl_xor(ls, 32, 64);
-      l_run = l_run * alpha + ls;
-      m_run = m_new;
-#pragma unroll
-      for (int i = 0; i < NDT; ++i)
-#pragma unroll
-        for (int j = 0; j < 16; ++j) acc[i][j] *= alpha;
-    }
-    const int g = lane >> 4, li = lane & 15;
-#pragma unroll
-    for (int dt = 0; dt < NDT; ++dt) {
-      const int c0 = 32 * dt + 16 * (g & 1) + 4 * (li & 3);
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2) {
-          const int kb = 32 * t + 16 * s2 + 4 * h + (li >> 2);
-          const lp_v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-              (__attribute__((address_space(3))) lp_v4s*)(&sm.v[kb][c0]));
-          const lp_v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-              (__attribute__((address_space(3))) lp_v4s*)(&sm.v[kb + 8][c0]));
-          short8 a8;
-          a8[0] = lo[0]; a8[1] = lo[1]; a8[2] = lo[2]; a8[3] = lo[3];
-          a8[4] = hi[0]; a8[5] = hi[1]; a8[6] = hi[2]; a8[7] = hi[3];
-          acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<bf16x8*>(&a8),
-                                                            pf[t][s2], acc[dt], 0, 0, 0);
+            for (int j = 0; j < 16; ++j) st[t][j] *= p.scale_log2;
         }
-    }
-  }
-  if (!valid) return;
+        // a tile that every row of this wave sees whole needs no per-score tests
+        const bool whole = kt + FL_KEYS - 1 <= wpos_lo && kt + FL_KEYS <= kend && (p.window <= 0 || wpos_hi - kt < p.window);
+        if (!whole) {
+          const int lim = min(kend, qpos + 1) - kt - 4 * h;
+          const int lo = p.window > 0 ? qpos - p.window + 1 - kt - 4 * h : -FL_KEYS;
+#pragma unroll
+          for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int j = 0; j < 16; ++j) {
+              const int c = 32 * t + (j & 3) + 8 * (j >> 2);
+              if (c >= lim || c < lo) st[t][j] = -INFINITY;
+            }
+        }
+      },
+      [&](int, unsigned stage) __attribute__((always_inline)) { fetch(kf, ka, DK, stage); },
+      [&](int, unsigned stage) __attribute__((always_inline)) { fetch(vf, va, DV, stage); });
+
+  fl_sync();                                              // every wave is done with the rings
+  fl_merge<NDT, QW, KS>(acc, m, l, reinterpret_cast<float*>(lds), run, wq, lane);
+  if (run) return;
   // the sink joins the denominator only (log2 domain, like the scores)
-  float f = 1.f, den = l_run;
+  float f = 1.f, den = l;
   if (p.sink) {
     const float sk = p.sink[head] * 1.4426950408889634f;
-    const float M = fmaxf(m_run, sk);
-    f = exp2f(m_run - M);
-    den = l_run * f + exp2f(sk - M);
+    const float M = fmaxf(m, sk);
+    f = exp2f(m - M);
+    den = l * f + exp2f(sk - M);
   }
   const float inv = den > 0.f ? f / den : 0.f;
-  bf16_t* orow = p.o + (size_t)(q0 + qi) * p.o_ld + (size_t)head * p.Dv;
-  const bf16_t* grow = p.gate ? p.gate + (size_t)(q0 + qi) * p.gate_ld + (size_t)head * p.Dv : nullptr;
+  const bf16_t* grow = p.gate ? p.gate + (size_t)(q0 + min(qi, row_hi)) * p.gate_ld + (size_t)head * p.Dv : nullptr;
 #pragma unroll
-  for (int dt = 0; dt < NDT; ++dt)
+  for (int d = 0; d < NDT; ++d)
 #pragma unroll
     for (int g4 = 0; g4 < 4; ++g4) {
-      const int d0 = 32 * dt + 8 * g4 + 4 * h;
-      if (d0 >= p.Dv) continue;
-      float o4[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) o4[i] = acc[dt][4 * g4 + i] * inv;
-      if (p.runs) {
-        if (grow) {
-          float gv[4];
+      const int d0 = 32 * d + 8 * g4 + 4 * h;
+      float gv[4] = {0.f, 0.f, 0.f, 0.f};
+      if (grow && d0 < p.Dv) {
+        if (p.runs) {
           ld_run<bf16_t, 4>(grow + d0, gv);
+        } else {
 #pragma unroll
-          for (int i = 0; i < 4; ++i) o4[i] *= sigmoid_fast(gv[i]);
+          for (int i = 0; i < 4; ++i)
+            if (d0 + i < p.Dv) gv[i] = bf2f(grow[d0 + i]);
         }
-        st_run<bf16_t, 4>(orow + d0, o4);
-      } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (d0 + i < p.Dv)
-            orow[d0 + i] = f2bf(grow ? o4[i] * sigmoid_fast(bf2f(grow[d0 + i])) : o4[i]);
       }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[d][4 * g4 + i] *= grow ? inv * sigmoid_fast(gv[i]) : inv;
     }
+  if (p.rows16) {
+    fl_store<NDT>(acc, lds + fl_merge_bytes(NDT, QW, KS) + wq * fl_store_bytes(NDT),
+                  p.o + (size_t)(q0 + row_lo + wq * 32) * p.o_ld + (size_t)head * p.Dv, p.o_ld, qlen - row_lo - wq * 32, p.Dv, lane);
+  } else if (valid) {
+    bf16_t* orow = p.o + (size_t)(q0 + qi) * p.o_ld + (size_t)head * p.Dv;
+#pragma unroll
+    for (int d = 0; d < NDT; ++d)
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        const int e = 32 * d + 8 * (j >> 2) + 4 * h + (j & 3);
+        if (e < p.Dv) orow[e] = f2bf(acc[d][j]);
+      }
+  }
 }
 
-// The last latent rows of every sequence (as many as its share of cu_k), gathered
-// from its pages in position order.
 __global__ __launch_bounds__(256) void latent_gather_kernel(
     const bf16_t* __restrict__ cache, int blk, const int* __restrict__ bt, int max_blocks,
     const int* __restrict__ cu_k, const int* __restrict__ ctx, int R, int Dr,
@@ -338,15 +272,32 @@ extern "C" int loqa_latent_prefill(const void* q, long q_st, const void* k, cons
   p.pos = (const int*)pos; p.ctx = (const int*)ctx; p.Dv = Dv; p.window = window;
   p.sink = (const float*)sink; p.scale_log2 = scale * 1.4426950408889634f; p.H = H;
   p.gate = (const bf16_t*)gate; p.gate_ld = gate_ld;
-  p.runs = Dv % 4 == 0 && o_ld % 4 == 0 && ((size_t)o & 7) == 0 &&
-           (!gate || (gate_ld % 4 == 0 && ((size_t)gate & 7) == 0));
-  const dim3 grid((max_q + LP_WAVES * 32 - 1) / (LP_WAVES * 32), H, B);
+  p.runs = Dv % 4 == 0 && (!gate || (gate_ld % 4 == 0 && ((size_t)gate & 7) == 0));
+  p.rows16 = Dv % 8 == 0 && o_ld % 8 == 0 && ((size_t)o & 15) == 0;
+  // the direct-to-LDS loads take 16-byte rows, a tile's rows within 32-bit offsets
+  if ((((size_t)k | (size_t)v) & 15) || (long)H * DK >= (1L << 24)) return (int)hipErrorInvalidValue;
+  // 128 rows and two runs (one round of the CUs, 160 KB of LDS at 192 columns), or one run, whose
+  // workgroups share a CU
+  const long n64 = (long)((max_q + 63) / 64) * H * B, n128 = (long)((max_q + 127) / 128) * H * B;
+#define RUN(A, C, QW, KS)                                                                     \
+  do {                                                                                        \
+    constexpr int ring = KS * FlashLds<A, C>::RING;                                           \
+    constexpr int end = fl_merge_bytes(C / 32, QW, KS) + QW * fl_store_bytes(C / 32);         \
+    constexpr int bytes = ring > end ? ring : end;                                            \
+    static_assert(bytes <= 160 * 1024, "LDS of a CU");                                        \
+    const dim3 grid((max_q + 32 * QW - 1) / (32 * QW), H, B);                                 \
+    hipLaunchKernelGGL((latent_prefill_kernel<A, C, QW, KS>), grid, dim3(64 * QW * KS), bytes, st, p); \
+    return (int)hipGetLastError();                                                            \
+  } while (0)
 #define GO(A, C)                                                                              \
   if (DK == A && DV == C) {                                                                   \
-    hipLaunchKernelGGL((latent_prefill_kernel<A, C>), grid, dim3(LP_THREADS), 0, st, p);      \
-    return (int)hipGetLastError();                                                            \
+    constexpr int K2 = A > 192 ? 1 : 2;                                                       \
+    if (n64 <= 256) RUN(A, C, 2, K2);                                                         \
+    else if (n128 <= 512) RUN(A, C, 4, K2);                                                   \
+    else RUN(A, C, 4, 1);                                                                     \
   }
   GO(64, 64) GO(128, 64) GO(192, 64) GO(256, 64) GO(64, 128) GO(128, 128) GO(192, 128) GO(256, 128)
 #undef GO
+#undef RUN
   return (int)hipErrorInvalidValue;
 }

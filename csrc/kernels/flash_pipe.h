@@ -1,4 +1,4 @@
-// Device parts of the software-pipelined flash attention (attention.hip, attn_window.hip,
+// Device parts of the software-pipelined flash attention (attention.hip, attn_window_pipe.hip,
 // attn_latent_prefill.hip): a wave's 32 query rows over a run of 64-key tiles.
 //
 // S^T = K Q^T (v_mfma_f32_32x32x16_bf16: the query lands on the MFMA lane, so row maxima and

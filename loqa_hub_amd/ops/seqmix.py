@@ -331,6 +331,9 @@ def latent_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu_q: torc
     if out is None:
         out = torch.empty(T, H * Dv, dtype=q.dtype, device=q.device)
     assert out.shape == (T, H * Dv) and out.stride(1) == 1 and out.dtype == q.dtype
+    # the kernel's loads take 16-byte rows (tensors that torch made start on them)
+    k = k if k.data_ptr() % 16 == 0 else k.clone()
+    v = v if v.data_ptr() % 16 == 0 else v.clone()
     check(kernels().loqa_latent_prefill(
         ptr(q), q.stride(0), ptr(k), ptr(v), ptr(out), out.stride(0), ptr(cu_q), ptr(cu_k),
         ptr(ctx_lens), ptr(positions), ptr(sink), float(scale), int(window), ptr(gate),

@@ -1,0 +1,64 @@
+"""The prompt pass of the latent attention (csrc/kernels/attn_latent_prefill.hip) at the edges of row
+blocks, key runs and windows, for every built head size, against float64.
+
+Bound: weights rounded to bf16 in numerator and sum, the gate through a 1-ulp reciprocal, the
+result rounded once: |error| <= 4 * 2^-9 * sum(p |v|) / den + f32 noise."""
+import math
+
+import pytest
+import torch
+
+from loqa_hub_amd.ops import seqmix
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _check(feeds, pasts, H, DK, DV, Dv, window=0, sink=False, gate=False, scale=None, shift=0, gate_shift=0, kv_shift=0, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    lens = [f + p for f, p in zip(feeds, pasts)]
+    kept = [min(n, f + window - 1) if window else n for f, n in zip(feeds, lens)]
+    T, L, scale = sum(feeds), sum(kept), DK ** -0.5 if scale is None else scale
+    rnd = lambda *s: torch.randn(*s, generator=g).bfloat16().to(DEV)
+    at = lambda t: torch.cat([torch.zeros(kv_shift, dtype=t.dtype, device=DEV), t.reshape(-1)])[kv_shift:].view(t.shape)
+    q, k, v = rnd(T, H, DK), at(rnd(L, H, DK)), at(rnd(L, H, DV))
+    cu = lambda x: torch.tensor([0] + x).cumsum(0).int().to(DEV)
+    cq, ck = cu(feeds), cu(kept)
+    pos = torch.cat([torch.arange(p, p + f) for f, p in zip(feeds, pasts)]).int().to(DEV)
+    ctx = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    sk = torch.randn(H, generator=g).to(DEV) if sink else None
+    gt = rnd(T, H * Dv + gate_shift)[:, gate_shift:] if gate else None
+    o = torch.empty(T, H * Dv + shift, dtype=torch.bfloat16, device=DEV)[:, shift:]
+    seqmix.latent_prefill(q, k, v, cq, ck, ctx, pos, sk, scale, max(feeds), Dv, window, gt, out=o)
+    for b, (f, n, m) in enumerate(zip(feeds, lens, kept)):
+        rows, keys = slice(int(cq[b]), int(cq[b]) + f), slice(int(ck[b]), int(ck[b]) + m)
+        s = torch.bmm(q[rows].double().transpose(0, 1), k[keys].double().permute(1, 2, 0).contiguous()) * scale
+        away = pos[rows, None] - torch.arange(n - m, n, device=DEV)[None]
+        seen = (away >= 0) & (away < window) if window else away >= 0
+        s = s.masked_fill(~seen, -math.inf)
+        top = s.amax(-1, keepdim=True)
+        if sk is not None:
+            top = torch.maximum(top, sk.double()[:, None, None])
+        p = (s - top).exp()
+        p = p / (p.sum(-1, keepdim=True) + ((sk.double()[:, None, None] - top).exp() if sk is not None else 0.0))
+        vs = v[keys, :, :Dv].double().transpose(0, 1).contiguous()
+        want, size = torch.bmm(p, vs), torch.bmm(p, vs.abs())
+        if gt is not None:
+            w = torch.sigmoid(gt[rows].double()).view(f, H, Dv).transpose(0, 1)
+            want, size = want * w, size * w
+        got = o[rows].double().view(f, H, Dv).transpose(0, 1)
+        assert ((got - want).abs() <= 4 * 2.0 ** -9 * size + 1e-5).all(), (b, f, n)
+
+
+@pytest.mark.parametrize("DK", seqmix.PREFILL_DK)
+@pytest.mark.parametrize("DV", seqmix.PREFILL_DV)
+def test_sizes_and_edges(DK, DV):
+    _check([1, 33, 64, 129, 200], [300, 0, 191, 31, 64], 2, DK, DV, DV, sink=True, gate=True, seed=DK)
+    _check([70, 5], [250, 700], 2, DK, DV, DV - 12, window=65, seed=DV)
+    _check([90], [0], 2, DK, DV, DV - 3, gate=True, scale=-0.05, seed=1)
+    _check([40, 30], [100, 0], 2, DK, DV, DV, gate=True, shift=3, gate_shift=1, kv_shift=1, seed=2)
+
+
+@pytest.mark.parametrize("B,T,H", [(1, 700, 8), (2, 700, 24), (4, 900, 24)])
+def test_every_block_height(B, T, H):
+    _check([T] * B, [7] * B, H, 192, 128, 128, 300, sink=True, seed=B)
