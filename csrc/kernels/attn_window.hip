@@ -26,7 +26,10 @@
 // rotation; no norm at all; values blended with another layer's value rows of the same tokens;
 // side columns of a parallel layer (seqmix.h).
 //
-// window_attn_keys_kernel (any dtype, any head size up to 512; decode steps,
+// window_attn_token_kernel (attn_window_token.hip; bf16, heads up to 128 in multiples of 8, up
+// to 16 heads a group; decode steps and short feeds), and
+//
+// window_attn_keys_kernel (any dtype, any head size up to 512; the other decode steps,
 // short feeds and the exact f32 mode): a workgroup per (token, key/value head)
 // serves REP query heads of the group at once, so K and V are read once per
 // group. The visible keys go in 64-key windows aligned to multiples of 64
@@ -101,20 +104,6 @@ __device__ __forceinline__ float wa_group_sum(float v, int gs) {
   if (gs >= 32) v += __shfl_xor(v, 16, 64);
   if (gs >= 64) v += __shfl_xor(v, 32, 64);
   return v;
-}
-
-// The sequence of flat row t: the number of feed starts cu_q[1 .. B - 1] at or
-// before t. Every lane tests one start, so a batch of up to 64 sequences costs
-// one round trip instead of a chain of dependent loads (all lanes must be active).
-__device__ __forceinline__ int wa_seq_of_row(const int* __restrict__ cu_q, int B, int t) {
-  const int lane = threadIdx.x & 63;
-  int b = 0;
-  for (int base = 1; base < B; base += 64) {
-    const int i = base + lane;
-    const bool at_or_before = i < B && cu_q[i] <= t;
-    b += __popcll(__ballot(at_or_before));
-  }
-  return b;
 }
 
 // ------------------------------------------------------------------ q / k rows
@@ -917,6 +906,15 @@ extern "C" int loqa_window_attention(const void* q, int dt, const void* kc, cons
                        ((size_t)o & 7) == 0;
   if (mfma && dt == 0 && D % 8 == 0 && D <= 256 && Dv % 8 == 0 && Dv <= 512 && runs_ok)
     return window_attention_mfma(p, max_q, st);
+  if (ns > 1 && part) { p.ns = ns; p.part = (float*)part; }
+  if (dt == 0) {
+    const int rc = window_attention_token(p, st);
+    if (rc > 0) return rc;
+    if (rc == 0) {
+      if (p.ns > 1) hipLaunchKernelGGL(window_attn_combine_kernel<bf16_t>, dim3(T, H), dim3(128), 0, st, p);
+      return (int)hipGetLastError();
+    }
+  }
   const int rep = H / G;
   // value layout: whole rows in 16-byte runs when Dv / (elements per run) is a
   // power of two up to 64, else a column per lane (2 or 8 columns)
@@ -925,7 +923,6 @@ extern "C" int loqa_window_attention(const void* q, int dt, const void* kc, cons
   const int nv = rows ? 0 : (Dv <= 128 ? 2 : 8);
   int R = rep >= 8 ? 8 : (rep >= 4 ? 4 : (rep >= 2 ? 2 : 1));
   if (nv == 8 && R > 4) R = 4;
-  if (ns > 1 && part) { p.ns = ns; p.part = (float*)part; }
   // few workgroups (decode steps): 16 waves share a row's keys, else 4
   auto lds_of = [&](int nw) {
     const size_t a = (size_t)(R * D + nw * (R + 1) * 64) * 4;

@@ -1,0 +1,229 @@
+// Token steps of the windowed paged attention (attn_window.hip), bf16, head sizes up to 128: few
+// query rows against many keys, bound by the reads of K and V and, at the sizes of a step, by
+// the chain from the block table over the keys and their maximum to the values and the merge.
+//
+// A workgroup of 16 waves serves one token and key head (ns: or a share of its keys). A wave
+// takes 32 keys at a time: K rows go from the pages straight to the A operands of the score
+// MFMAs (16 x 16 x 32; the group's query heads, up to 16, are the columns), V rows straight to
+// its part of LDS meanwhile, whence transposed reads make them the A operands of the second
+// product, whose B operand the exponentials of the scores are as they lie. All of a wave's loads
+// are in flight together, maxima of 16 heads cost two exchanges, and 512 keys of a row are read
+// at once, so that windows of some 1000 keys need neither key splits nor a second launch.
+// The weights stay what 32 bits hold: each goes as a sum of three bf16 (24 bits).
+// 8 tokens, 16 heads (4 key heads) of 128, window 1024: 20.6 + 3.9 us before (a key on one lane
+// at a time, 12 cross-lane steps a head and 64 keys, five key splits and their merge), 12.4 now,
+// two rounds of loads; up to 500 keys 17 before, 6.5 now; 64 tokens behind 2000: 168, 100.
+#include "flash_pipe.h"
+#include "seqmix.h"
+
+#define WT_KEYS 32
+
+__device__ __forceinline__ float wt_max16(float x) {   // over lanes 16 apart: all keys of a head
+  typedef unsigned u2 __attribute__((ext_vector_type(2)));
+  const u2 r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fl_max32(fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])));
+}
+__device__ __forceinline__ float wt_sum16(float x) {
+  typedef unsigned u2 __attribute__((ext_vector_type(2)));
+  const u2 r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fl_both32(__uint_as_float(r[0]) + __uint_as_float(r[1]));
+}
+
+// place of chunk c of V row r: a half wave reads 8 rows of two chunks
+template <int DV> __device__ __forceinline__ int wt_swz(int r) { return DV == 128 ? 2 * (r & 7) : 2 * ((r >> 1) & 3); }
+
+template <int DK, int DV, int WT_WAVES>
+__global__ __launch_bounds__(64 * WT_WAVES, 4) void window_attn_token_kernel(WinAttnParams p) {
+  constexpr int NS = DK / 32, NDT = DV / 16, CH = DV / 8, NV = WT_KEYS * CH / 64;
+  constexpr int VB = WT_KEYS * DV * 2;                       // bytes of a wave's V tile
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c = lane & 15, q4 = lane >> 4;                   // head column, key quarter
+  const int t = blockIdx.x, g = blockIdx.y, sp = blockIdx.z;
+  if (t >= p.cu_q[p.B]) return;
+  const int b = wa_seq_of_row(p.cu_q, p.B, t);
+  const int rep = p.H / p.G, D = p.D, Dv = p.Dv;
+  const int pq = p.pos[t];
+  const int hi = min(pq, p.ctx[b] - 1);
+  const int lo = p.window > 0 ? max(0, pq - p.window + 1) : 0;
+  // tiles of 32 keys: the kept first tokens before the window, then from its first key on
+  const int kept = p.window > 0 ? min(p.keep_first, min(lo, hi + 1)) : 0;
+  const int n1 = kept > 0 ? (kept + WT_KEYS - 1) / WT_KEYS : 0;
+  const int nt = n1 + max(hi - lo + WT_KEYS, 0) / WT_KEYS;
+  const int* bt = p.bt + (size_t)b * p.max_blocks;
+  const bf16_t* kc = (const bf16_t*)p.kc + (size_t)g * D;
+  const bf16_t* vc = (const bf16_t*)p.vc + (size_t)g * Dv;
+  const size_t kst = (size_t)p.G * D, vst = (size_t)p.G * Dv;
+
+  bf16x8 qf[NS];
+  {
+    const bf16_t* qr = (const bf16_t*)p.q + ((size_t)t * p.H + g * rep + min(c, rep - 1)) * D;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      const int e = 32 * s + 8 * q4;
+      const uint4 v = c < rep && e < D ? *reinterpret_cast<const uint4*>(qr + e) : make_uint4(0, 0, 0, 0);
+      qf[s] = *reinterpret_cast<const bf16x8*>(&v);
+    }
+  }
+  const float slope = p.slopes ? p.slopes[g * rep + min(c, rep - 1)] : 0.f;
+  float4v acc[NDT];
+#pragma unroll
+  for (int d = 0; d < NDT; ++d) acc[d] = float4v{0.f, 0.f, 0.f, 0.f};
+  float m = -1e30f, l = 0.f;                                 // base 2
+  constexpr float LOG2E = 1.4426950408889634f;
+  const unsigned my = fl_lds_at(lds) + wave * VB;
+  for (int wk = sp * WT_WAVES + wave; wk < nt; wk += p.ns * WT_WAVES) {
+    const int k0 = wk < n1 ? wk * WT_KEYS : lo + (wk - n1) * WT_KEYS, end = wk < n1 ? kept : hi + 1;
+    // lane r names the cache row of key k0 + r % 32 (past the last key: that one's)
+    const int jc = min(k0 + (lane & 31), end - 1), pi = jc / p.blk;
+    const int row = (int)min(max((long)bt[pi] * p.blk + (jc - pi * p.blk), 0L), p.cache_rows - 1);
+    uint4 kr[2][NS];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const bf16_t* r = kc + (size_t)__shfl(row, 16 * u + c) * kst;
+#pragma unroll
+      for (int s = 0; s < NS; ++s) {
+        const int e = 32 * s + 8 * q4;
+        kr[u][s] = e < D ? *reinterpret_cast<const uint4*>(r + e) : make_uint4(0, 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int id = lane + 64 * i, r = id / CH, ch = (id % CH) ^ wt_swz<DV>(r);
+      const bf16_t* src = vc + (size_t)__shfl(row, r) * vst + ch * 8;
+      if (ch * 8 < Dv) fl_load_lds(src, __builtin_amdgcn_readfirstlane(my + i * 1024));
+    }
+    float4v st[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      st[u] = float4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < NS; ++s)
+        st[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<bf16x8*>(&kr[u][s]), qf[s], st[u], 0, 0, 0);
+    }
+    // score (u, r) of lane (c, q4): head c, key k0 + 16 u + 4 q4 + r
+    float mx = -INFINITY;
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int j = k0 + 16 * u + 4 * q4 + r;
+        float sv = st[u][r] * p.scale;
+        if (p.cap > 0.f) sv = p.cap * tanhf(sv / p.cap);
+        sv = (sv - slope * (float)(pq - j)) * LOG2E;
+        if (j >= end) sv = -INFINITY;
+        st[u][r] = sv;
+        mx = fmaxf(mx, sv);
+      }
+    const float mn = fmaxf(m, wt_max16(mx));
+    const float alpha = __builtin_amdgcn_exp2f(m - mn);
+    m = mn;
+    l *= alpha;
+    bf16x8 pw[3];
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float e = __builtin_amdgcn_exp2f(st[u][r] - mn);
+        l += e;
+        const __bf16 h0 = (__bf16)e;
+        const float e1 = e - (float)h0;
+        const __bf16 h1 = (__bf16)e1;
+        pw[0][4 * u + r] = h0;
+        pw[1][4 * u + r] = h1;
+        pw[2][4 * u + r] = (__bf16)(e1 - (float)h1);
+      }
+#pragma unroll
+    for (int d = 0; d < NDT; ++d) acc[d] *= alpha;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");         // this wave's V tile is here
+#pragma unroll
+    for (int d = 0; d < NDT; ++d) {
+      bf16x8 a;
+      short8 a8;
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const int r = 16 * u + 4 * q4 + (c >> 2), ch = (2 * d + ((c & 3) >> 1)) ^ wt_swz<DV>(r);
+        const fl_v4s v = __builtin_amdgcn_ds_read_tr16_b64_v4i16(fl_lds<fl_v4s>(my + r * (DV * 2) + ch * 16 + (c & 1) * 8));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) a8[4 * u + i] = v[i];
+      }
+      a = *reinterpret_cast<bf16x8*>(&a8);
+#pragma unroll
+      for (int w = 0; w < 3; ++w) acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, pw[w], acc[d], 0, 0, 0);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // read, before the next tile's loads
+  }
+  l = wt_sum16(l);
+
+  // the waves' partials, in wave order: acc (d, r) of lane (c, q4) is column 16 d + 4 q4 + r of head c
+  __syncthreads();
+  float* mm = reinterpret_cast<float*>(lds);                 // [waves][16]
+  float* ll = mm + WT_WAVES * 16;
+  float* aa = ll + WT_WAVES * 16;                            // [waves][rep][DV]
+  if (q4 == 0) {
+    mm[wave * 16 + c] = m;
+    ll[wave * 16 + c] = l;
+  }
+  if (c < rep)
+#pragma unroll
+    for (int d = 0; d < NDT; ++d)
+      *reinterpret_cast<float4v*>(aa + ((size_t)wave * rep + c) * DV + 16 * d + 4 * q4) = acc[d];
+  __syncthreads();
+  for (int idx = threadIdx.x; idx < rep * Dv; idx += 64 * WT_WAVES) {
+    const int r = idx / Dv, e = idx - r * Dv, h = g * rep + r;
+    const bool snk = p.sink && p.ns == 1;                    // with key splits the combine launch adds it
+    const float sk = snk ? p.sink[h] * LOG2E : -1e30f;
+    float M = sk;
+#pragma unroll
+    for (int w = 0; w < WT_WAVES; ++w) M = fmaxf(M, mm[w * 16 + r]);
+    float num = 0.f, den = snk ? __builtin_amdgcn_exp2f(sk - M) : 0.f;
+#pragma unroll
+    for (int w = 0; w < WT_WAVES; ++w) {
+      const float f = __builtin_amdgcn_exp2f(mm[w * 16 + r] - M);
+      num += f * aa[((size_t)w * rep + r) * DV + e];
+      den += f * ll[w * 16 + r];
+    }
+    if (p.ns > 1) {                                          // the combine launch (natural units) finishes the row
+      float* pr = p.part + (((size_t)t * p.H + h) * p.ns + sp) * (Dv + 2);
+      if (e == 0) {
+        pr[0] = M / LOG2E;
+        pr[1] = den;
+      }
+      pr[2 + e] = num;
+      continue;
+    }
+    float out = den > 0.f ? num / den : 0.f;
+    if (p.gate) out *= sigmoid_f(bf2f(((const bf16_t*)p.gate)[(size_t)t * p.gate_ld + (size_t)h * Dv + e]));
+    ((bf16_t*)p.o)[(size_t)t * p.o_ld + (size_t)h * Dv + e] = f2bf(out);
+  }
+}
+
+// -1: not these sizes or places. The caller launches the combine for p.ns > 1.
+int window_attention_token(const WinAttnParams& p, hipStream_t st) {
+  const int rep = p.H / p.G;
+  if (p.D > 128 || p.Dv > 128 || p.D % 8 || p.Dv % 8 || rep > 16 || p.cache_rows > 0x7fffffffL ||
+      (((size_t)p.q | (size_t)p.kc | (size_t)p.vc) & 15))
+    return -1;
+  const dim3 grid(p.T, p.G, p.ns);
+  // Enough rows to fill the chip: four waves, whose workgroups share a CU and wait in turn (us,
+  // 16 and 4 waves: 32 tokens of 4 key heads, 1024 keys: 21, 24; 80 tokens, 512 keys: 24, 21; 240
+  // tokens of 16 key heads of 64, 1000 keys: 130, 94).
+  const bool many = (long)p.T * p.G >= 256;
+#define RUN(A, C, W)                                                                                    \
+  do {                                                                                                  \
+    const int ring = W * WT_KEYS * C * 2, end = W * (32 + rep * C) * 4;                                 \
+    hipLaunchKernelGGL((window_attn_token_kernel<A, C, W>), grid, dim3(64 * W), ring > end ? ring : end, st, p); \
+    return (int)hipGetLastError();                                                                      \
+  } while (0)
+#define GO(A, C)                                                                                        \
+  do {                                                                                                  \
+    if (many) RUN(A, C, 4);                                                                             \
+    RUN(A, C, 16);                                                                                      \
+  } while (0)
+  if (p.D <= 64) {
+    if (p.Dv <= 64) GO(64, 64); else GO(64, 128);
+  }
+  if (p.Dv <= 64) GO(128, 64); else GO(128, 128);
+#undef RUN
+#undef GO
+}

@@ -58,6 +58,9 @@ template <typename T> __device__ __forceinline__ FL_LDS T* fl_lds(unsigned at) {
 __device__ __forceinline__ void fl_load_lds(const bf16_t* base, unsigned off, unsigned dst) {   // base wave-uniform
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(off), "s"(base) : "memory", "m0");
 }
+__device__ __forceinline__ void fl_load_lds(const bf16_t* at, unsigned dst) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(dst), "v"(at) : "memory", "m0");
+}
 
 // The fetch of one tile of K (ISV = false) or V rows into a stage by the NTH threads (whole
 // waves) of a group, th the thread. Rows past `last` read row `last`; PAD: only cols of the D

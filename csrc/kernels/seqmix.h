@@ -2,7 +2,8 @@
 // (norm_dyt.hip, attn_latent.hip, lightning.hip, moe.hip, seq_rows.hip,
 // attn_sigmoid.hip, norm_scalar.hip, norm_rms1p.hip, attn_window.hip, mamba2.hip,
 // matrix_memory.hip, delta_rule.hip, norm_layer.hip, linear_chunks.hip,
-// delta_chunks.hip, moe_pipe.hip, attn_window_pipe.hip).
+// delta_chunks.hip, moe_pipe.hip, attn_window_pipe.hip,
+// attn_window_token.hip).
 //
 // Activations are bfloat16 or float32, chosen at run time by a dtype code
 // (0: bf16, 1: f32); every kernel is a template over the storage type and does
@@ -156,3 +157,19 @@ struct WinAttnParams {
 };
 // Prompt portions on the pipelined tile loop; -1 where it does not take the sizes or places.
 int window_attention_pipe(const WinAttnParams& p, int max_q, hipStream_t st);
+// Token steps on the matrix cores (attn_window_token.hip), likewise.
+int window_attention_token(const WinAttnParams& p, hipStream_t st);
+
+// The sequence of flat row t: the number of feed starts cu_q[1 .. B - 1] at or
+// before t. Every lane tests one start, so a batch of up to 64 sequences costs
+// one round trip instead of a chain of dependent loads (all lanes must be active).
+__device__ __forceinline__ int wa_seq_of_row(const int* __restrict__ cu_q, int B, int t) {
+  const int lane = threadIdx.x & 63;
+  int b = 0;
+  for (int base = 1; base < B; base += 64) {
+    const int i = base + lane;
+    const bool at_or_before = i < B && cu_q[i] <= t;
+    b += __popcll(__ballot(at_or_before));
+  }
+  return b;
+}

@@ -923,8 +923,10 @@ def window_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
         # 64-key windows a row can have, four (one per wave) to a workgroup
         keys = max(int(max_ctx), 1) if window <= 0 else min(max(int(max_ctx), 1),
                                                            window + 64 + keep_first)
+        # (a workgroup of the matrix-core token form reads 512 keys at once)
+        once = 1152 if q.dtype == torch.bfloat16 and D <= 128 and Dv <= 128 and D % 8 == Dv % 8 == 0 and H // G <= 16 else 256
         key_splits = 1 if mfma or T * G >= 256 else \
-            max(1, min(16, -(-keys // 256), 512 // max(1, T * G)))
+            max(1, min(16, -(-keys // once), 512 // max(1, T * G)))
     if key_splits > 1 and not mfma:
         part = torch.empty(T * H * key_splits * (Dv + 2), dtype=torch.float32, device=q.device)
     else:
