@@ -298,6 +298,89 @@ __global__ __launch_bounds__(256) void qk_prep_append_kernel(QkPrepParams<T> p, 
   side_relu2<T>(side, t);
 }
 
+// The same for prompts, bf16, heads of 64 or 128: eight entries a lane, so that a wave takes eight
+// or four heads at once. With two a lane the arithmetic of a head (root, division, six steps of
+// the sum) is that of 64 lanes for 128 entries, and 2048 tokens of 16 + 4 heads of 128 took 15.7 us,
+// the VALU's time; now 9.5. Norms per head only.
+template <int D>
+__global__ __launch_bounds__(256) void qk_prep_append_runs_kernel(QkPrepParams<bf16_t> p, SideCols side) {
+  constexpr int L = D / 8, HW = 64 / L;                  // lanes of a head, heads of a wave
+  const int t = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int H = p.H, G = p.G, Dv = p.Dv, e0 = 8 * (lane % L);
+  const int pos = p.pos[t];
+  const long slot = p.kvslots[t];
+  const bool store = slot >= 0 && slot < p.cache_rows;
+  const bf16_t* ur = p.u + (size_t)t * p.ldu;
+  const float temp = p.coef == 0.f ? 1.f : 1.f + p.coef * logf((float)((pos + 1) / p.every) + 1.f);
+  float cs[8];
+  if (p.dims) {
+    const float* csr = p.cs + (size_t)min(max(pos, 0), p.max_pos - 1) * p.dims;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const bool in = e0 + 2 * i < p.dims;
+      const float2 v = in ? *reinterpret_cast<const float2*>(csr + e0 + 2 * i) : make_float2(1.f, 0.f);
+      cs[2 * i] = v.x;
+      cs[2 * i + 1] = v.y;
+    }
+  }
+  for (int job = wave * HW + lane / L; job - lane / L < H + G; job += 4 * HW) {
+    const bool in = job < H + G, isq = job < H;
+    uint4 raw = make_uint4(0, 0, 0, 0);
+    if (in) raw = *reinterpret_cast<const uint4*>(ur + (size_t)job * D + e0);
+    if (in && !isq && p.v_off < 0 && store)              // the values are the keys as projected
+      *reinterpret_cast<uint4*>(p.vc + (size_t)slot * G * Dv + (size_t)(job - H) * Dv + e0) = raw;
+    float a[8];
+    unpack8(raw, a);
+    if (p.norm == QKN_HEAD_W) {
+      float ss = 0.f;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) ss += a[i] * a[i];
+      const float inv = 1.f / sqrtf(wa_group_sum(ss, L) / (float)D + p.eps);
+      const float* wn = (isq ? p.qn : p.kn) + e0;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) a[i] *= inv * wn[i];
+    }
+    if (p.dims) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float c = cs[2 * i], s = cs[2 * i + 1];
+        const float x = a[2 * i] * c - a[2 * i + 1] * s, y = a[2 * i + 1] * c + a[2 * i] * s;
+        a[2 * i] = x;
+        a[2 * i + 1] = y;
+      }
+    }
+    float inv = isq ? temp : 1.f;
+    if (p.norm == QKN_HEAD) {
+      float ss = 0.f;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) ss += a[i] * a[i];
+      inv /= sqrtf(wa_group_sum(ss, L) / (float)D + p.eps);
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) a[i] *= inv;
+    if (in && (isq || store))
+      *reinterpret_cast<uint4*>((isq ? p.q + (size_t)t * H * D + (size_t)job * D
+                                     : p.kc + (size_t)slot * G * D + (size_t)(job - H) * D) + e0) = pack8(a);
+  }
+  if (p.v_off >= 0 && store) {
+    bf16_t* vr = p.vc + (size_t)slot * G * Dv;
+    const bf16_t* vs = ur + p.v_off;
+    const bf16_t* fr = p.vf ? p.vf + (size_t)t * p.vf_ld : nullptr;
+    for (int c = 4 * threadIdx.x; c < G * Dv; c += 4 * 256) {
+      float v[4];
+      ld_run<bf16_t, 4>(vs + c, v);
+      if (fr) {                                          // (1 - lam) v + lam v_first
+        float f[4];
+        ld_run<bf16_t, 4>(fr + c, f);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = (1.f - p.lam) * v[i] + p.lam * f[i];
+      }
+      st_run<bf16_t, 4>(vr + c, v);
+    }
+  }
+  side_relu2<bf16_t>(side, t);
+}
+
 // ------------------------------------------------------------ few rows, many keys
 template <typename T, int REP, int NV, int NW>
 __global__ __launch_bounds__(64 * NW) void window_attn_keys_kernel(WinAttnParams p) {
@@ -876,6 +959,19 @@ extern "C" int loqa_qk_prep_append(const void* u, int dt, long ldu, int H, int G
     else if (D <= 128) GO(TT, 1, true); else if (D <= 256) GO(TT, 2, true);                    \
     else GO(TT, 4, true);                                                                      \
   } while (0)
+  // prompts of heads that split into 16-byte runs (steps of few tokens are bound by their loads'
+  // latency, where a head per wave has more of them in flight)
+  if (dt == 0 && T >= 256 && (D == 64 || D == 128) && norm != QKN_WHOLE && ldu % 8 == 0 && (v_off < 0 || vruns) &&
+      (v_off >= 0 || Dv % 8 == 0) && aligned(u, 16) && aligned(q, 16) && aligned(kc, 16) && aligned(vc, 16) && aligned(cs, 8)) {
+    const QkPrepParams<bf16_t> p{(const bf16_t*)u, ldu, H, G, D, Dv, v_off, (const float*)cs, max_pos, dims, eps, coef, every,
+                                 (const int*)pos, (bf16_t*)kc, (bf16_t*)vc, (long)blk * nblocks, (const int*)kvslots, (bf16_t*)q,
+                                 (const float*)qn, (const float*)kn, norm, (const bf16_t*)vf, vf_ld, lam, vruns};
+    if (D == 64)
+      hipLaunchKernelGGL(qk_prep_append_runs_kernel<64>, dim3(T), dim3(256), 0, st, p, side);
+    else
+      hipLaunchKernelGGL(qk_prep_append_runs_kernel<128>, dim3(T), dim3(256), 0, st, p, side);
+    return (int)hipGetLastError();
+  }
   if (dt == 0) BY_D(bf16_t); else BY_D(float);
 #undef BY_D
 #undef GO
