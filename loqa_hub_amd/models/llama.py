@@ -417,9 +417,8 @@ class LlamaModel:
 
     def _forward_prefill_hw(self, meta: StepMeta, k_cache, v_cache, attn_ws, x, h
                             ) -> torch.Tensor:
-        """Prompt pass on the hand-written GEMMs (``ops.proj``: per shape the
-        measured faster of the split-K tiled GEMM, whose K chunks are summed
-        in-launch, and the row-resident weight-streaming GEMM; tensor parallel:
+        """Prompt pass on the hand-written GEMMs (``ops.proj``: pipelined tiles
+        planned per shape, whose K chunks are summed in-launch; tensor parallel:
         the same GEMMs on the rank's shards, the row-parallel o / down partials
         summed by the custom all-reduce - no hipBLASLt on any rank): per layer qkv
         (bf16) -> RoPE + KV append -> flash attention -> o added straight into
