@@ -13,8 +13,7 @@
 // with zero columns) or mel-major.
 // One 30 s window, 80 / 128 mels: 69 / 92 us before (32 frames a workgroup, 94 of them, the
 // whole K range, the filterbank as a GEMM whose operand loads formed one chain, an atomic per
-// wave), 20 / 23 us now; what
-// is left is the chain of basis loads of one workgroup per CU.
+// wave), 20 / 24 us now; what is left is the chain of basis loads of one workgroup per CU.
 //
 // im2col: k=3, pad=1 conv1d input unfolding so the conv becomes a plain GEMM
 // (hipBLASLt) followed by the fused bias+GELU(+pos) epilogue (elementwise.hip).
