@@ -88,3 +88,29 @@ def test_peaked_and_flat():
 def test_rows_off_16_bytes_take_the_other_kernel():
     _check([50, 9], [50, 200], 2, 2, 64, True, q_pad=4, seed=7)
     _check([50, 9], [50, 200], 2, 2, 128, False, shift=4, seed=8)
+
+
+def _us(call, n=20):
+    for _ in range(3):
+        call()
+    at = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+    at[0].record()
+    for _ in range(n):
+        call()
+    at[1].record()
+    torch.cuda.synchronize()
+    return at[0].elapsed_time(at[1]) * 1e3 / n
+
+
+@pytest.mark.parametrize("D,H,G", [(64, 20, 20), (128, 32, 8)])
+def test_other_places_cost_no_multiple(D, H, G):
+    # blocks that are no power of two find a row per chunk (1.2 to 1.9 times the time of the
+    # others, 4 to 5.5 times on a kernel without key runs)
+    def call(page):
+        per = -(-1000 // page)
+        kc = torch.randn(per, G, page, D, device=DEV).bfloat16()
+        q, bt = torch.randn(40, H * D, device=DEV).bfloat16(), torch.randperm(per, device=DEV).int()[None].contiguous()
+        cu, ctx = torch.tensor([0, 40], dtype=torch.int32, device=DEV), torch.tensor([1000], dtype=torch.int32, device=DEV)
+        return lambda: ops.attention(q, kc, kc, cu, n_heads=H, n_kv=G, head_dim=D, causal=True, max_q=40, ctx_lens=ctx,
+                                     block_tables=bt, max_k=1000)
+    assert _us(call(12)) < 3 * _us(call(16))
