@@ -692,12 +692,17 @@ static int launch_pipe(const AttnParams& p, int B, int max_q, hipStream_t s) {
 // workgroups a CU, which are out of step with each other. us a pass (64-row form, 128 / two,
 // 128 / one): 1500 x 8 heads of 64: 15.6, 20, 25; x 20 heads: 26, 22.7, 27; 6 x 1500 x 20 heads:
 // 133, 124, 106; 128 columns, paged: 320 rows behind 1000 x 32 heads: 31, 32, 40; 2048 x 32 heads
-// causal: 101, 60, 70; 4 x that: 349, 238, 200
+// causal: 101, 60, 70; 4 x that: 349, 238, 200.
+// Long causal prompts of 64-column heads stay with two runs longer: half of the work is gone and
+// the last rows' chain of tiles is what the pass lasts (128 / two, 128 / one): 1400 x 32 heads 24,
+// 29; 2048 x 20 heads 40, 50; 4096 x 12 heads 68, 94, x 20 heads 116, 121; but 4 x 700 x 16 heads
+// 18.0, 17.0, 3000 x 20 heads 76, 62, 4096 x 32 heads 121, 102.
 template <int D, int PAGES>
 static int launch_rows(const AttnParams& p, int B, int max_q, hipStream_t s) {
   const long n64 = (long)((max_q + 63) / 64) * p.Hq * B, n128 = (long)((max_q + 127) / 128) * p.Hq * B;
+  const long two = D == 128 ? 512 : !p.causal || max_q < 1024 ? 256 : max_q < 4096 ? 384 : 640;
   if (n64 <= 256) return launch_pipe<D, PAGES, 2, D == 64 ? 4 : 2>(p, B, max_q, s);
-  if (n128 <= (D == 64 ? 256 : 512)) return launch_pipe<D, PAGES, 4, 2>(p, B, max_q, s);
+  if (n128 <= two) return launch_pipe<D, PAGES, 4, 2>(p, B, max_q, s);
   return launch_pipe<D, PAGES, 4, 1>(p, B, max_q, s);
 }
 
