@@ -54,9 +54,15 @@ template <typename T> __device__ __forceinline__ FL_LDS T* fl_lds(unsigned at) {
 
 // 16 bytes per lane straight to LDS (lane l at dst + 16 l, dst wave-uniform). As the builtin, each
 // load made the compiler wait for all of them before the next transposed LDS read, of whose
-// address it knows nothing; the waits are fl_sync()'s. No register is written.
+// address it knows nothing; the waits are fl_sync()'s. No vector register is written.
+// A vector memory instruction may read a scalar register 5 wait states after a vector instruction
+// (v_readlane: page numbers, spilled scalars) wrote it at the earliest, and the compiler does not
+// look into the asm. The scalar unit has no such limit: the base goes through a scalar copy, which
+// is also the wait state that m0 asks for.
 __device__ __forceinline__ void fl_load_lds(const bf16_t* base, unsigned off, unsigned dst) {   // base wave-uniform
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(off), "s"(base) : "memory", "m0");
+  unsigned long long at;
+  asm volatile("s_mov_b32 m0, %1\n\ts_mov_b64 %0, %3\n\tglobal_load_lds_dwordx4 %2, %0"
+               : "=&s"(at) : "s"(dst), "v"(off), "s"(base) : "memory", "m0");
 }
 __device__ __forceinline__ void fl_load_lds(const bf16_t* at, unsigned dst) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(dst), "v"(at) : "memory", "m0");
