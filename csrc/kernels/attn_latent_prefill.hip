@@ -37,6 +37,10 @@ struct LatPrefillParams {
 
 // QW blocks of 32 query rows, the keys in KS runs. At 192 / 128 a run's ring is 80 KB of LDS and a
 // tile's working set with two waves a SIMD all of the registers; the 256-column keys take one wave.
+// The bound of two stands also where LDS holds one (64 rows in two runs): from 257 registers on the
+// compiler keeps MFMA results in the accumulation registers and moves them for every rescaling.
+// us with 256 registers (10 spilled at 192 / 128) and with 320 (none): 300 rows x 16 heads 13.8, 14.7;
+// 2048 x 8 heads 37.2, 41.8, at 128 / 128 30.6, 36.9.
 template <int DK, int DV, int QW, int KS>
 __global__ __launch_bounds__(64 * QW * KS, DK > 192 ? 1 : 2) void latent_prefill_kernel(LatPrefillParams p) {
   using L = FlashLds<DK, DV>;
@@ -276,8 +280,9 @@ extern "C" int loqa_latent_prefill(const void* q, long q_st, const void* k, cons
   p.rows16 = Dv % 8 == 0 && o_ld % 8 == 0 && ((size_t)o & 15) == 0;
   // the direct-to-LDS loads take 16-byte rows, a tile's rows within 32-bit offsets
   if ((((size_t)k | (size_t)v) & 15) || (long)H * DK >= (1L << 24)) return (int)hipErrorInvalidValue;
-  // 128 rows and two runs (one round of the CUs, 160 KB of LDS at 192 columns), or one run, whose
-  // workgroups share a CU
+  // 64 rows and two runs (keys of 256 columns: one) while these workgroups are one round of the
+  // CUs, then 128 rows and two runs (160 KB of LDS at 192 columns), or one run, whose workgroups
+  // share a CU
   const long n64 = (long)((max_q + 63) / 64) * H * B, n128 = (long)((max_q + 127) / 128) * H * B;
 #define RUN(A, C, QW, KS)                                                                     \
   do {                                                                                        \
