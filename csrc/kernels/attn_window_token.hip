@@ -9,7 +9,8 @@
 // product, whose B operand the exponentials of the scores are as they lie. All of a wave's loads
 // are in flight together, maxima of 16 heads cost two exchanges, and 512 keys of a row are read
 // at once, so that windows of some 1000 keys need neither key splits nor a second launch.
-// The weights stay what 32 bits hold: each goes as a sum of three bf16 (24 bits).
+// The weights stay what 32 bits hold: each goes as a sum of three bf16 (24 bits), none of them
+// negative or zero, so that an infinite value stays one.
 // 8 tokens, 16 heads (4 key heads) of 128, window 1024: 20.6 + 3.9 us before (a key on one lane
 // at a time, 12 cross-lane steps a head and 64 keys, five key splits and their merge), 12.4 now,
 // two rounds of loads; up to 500 keys 17 before, 6.5 now; 64 tokens behind 2000: 168, 100.
@@ -124,14 +125,16 @@ __global__ __launch_bounds__(64 * WT_WAVES, 4) void window_attn_token_kernel(Win
     for (int u = 0; u < 2; ++u)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const float e = __builtin_amdgcn_exp2f(st[u][r] - mn);
+        // the weight's leading, middle and last 8 bits, cut off toward zero (exact); a part that
+        // is zero would make 0 x inf of an infinite value: it is 2^-126, nothing beside weights up to 1
+        float e = __builtin_amdgcn_exp2f(st[u][r] - mn);
         l += e;
-        const __bf16 h0 = (__bf16)e;
-        const float e1 = e - (float)h0;
-        const __bf16 h1 = (__bf16)e1;
-        pw[0][4 * u + r] = h0;
-        pw[1][4 * u + r] = h1;
-        pw[2][4 * u + r] = (__bf16)(e1 - (float)h1);
+#pragma unroll
+        for (int w = 0; w < 3; ++w) {
+          const float h = __uint_as_float(__float_as_uint(e) & 0xffff0000u);
+          pw[w][4 * u + r] = (__bf16)fmaxf(h, 1.17549435e-38f);
+          e -= h;
+        }
       }
 #pragma unroll
     for (int d = 0; d < NDT; ++d) acc[d] *= alpha;

@@ -94,3 +94,24 @@ def test_many_rows(rows):
     # from 256 rows x key heads on: four waves a workgroup
     _check([rows, 5, rows], [77, 600, 0], 8, 4, 128, 128, 300, 2, slopes=True, seed=rows)
     _check([rows, 5, rows], [77, 600, 0], 8, 4, 64, 128, cap=15.0, gate=True, seed=rows)
+
+
+@pytest.mark.parametrize("value", [math.inf, -math.inf, math.nan])
+def test_values_that_are_not_finite(value):
+    # keys 0 .. 99, one of them with such values: the result where it is seen, nothing else of it
+    kc, vc = torch.randn(7, 16, 64, device=DEV).bfloat16(), torch.randn(7, 16, 64, device=DEV).bfloat16()
+    bt, cu = torch.arange(7, dtype=torch.int32, device=DEV)[None].contiguous(), torch.tensor([0, 1], dtype=torch.int32, device=DEV)
+    ctx, pos = torch.tensor([100], dtype=torch.int32, device=DEV), torch.tensor([99], dtype=torch.int32, device=DEV)
+    q = torch.randn(1, 128, device=DEV).bfloat16()
+    for key in (0, 31, 60, 99):
+        v = vc.clone()
+        v.view(-1, 64)[key, 5] = value
+        for window in (0, 40):
+            o = seqmix.window_attention(q, kc, v, cu, ctx, bt, pos, 0.125, 0.0, window, 0, None, 2, 1, 64, 64, max_q=1, max_ctx=100)
+            hit = o.view(2, 64)[:, 5].float().cpu()
+            if window and key < 60:
+                assert hit.isfinite().all()
+            else:
+                assert torch.equal(hit, torch.full((2,), value)) or math.isnan(value) and hit.isnan().all(), (key, hit)
+            o.view(2, 64)[:, 5] = 0
+            assert o.isfinite().all()
