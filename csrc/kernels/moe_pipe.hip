@@ -125,6 +125,7 @@ bool moe_pipe(const void* A, long rows, const void* W, const void* plan, int P, 
   if (K % GP_BK || N % 8 || rows * K * 2 >= 0xfffffff0l || (long)N * (gated ? 2 : 1) * K * 2 >= 0xfffffff0l ||
       ((size_t)A | (size_t)W | (size_t)out) & 15)
     return false;
+  if (E <= 0) return true;                                // identity experts only: nothing to multiply
   // the tile whose rounds over the compute units take least, with an expert's last tile half
   // empty on average
   const int used = E < P ? E : P;

@@ -55,3 +55,14 @@ def test_plan_is_a_permutation_by_expert(P, E):
     assert off.tolist() == [0] + torch.bincount(e, minlength=E + 1).cumsum(0).tolist()
     assert torch.equal(perm.sort().values, torch.arange(P)) and torch.equal(pos[perm], torch.arange(P, dtype=torch.int32))
     assert torch.equal(e[perm], e.sort().values)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [3, 200])
+@pytest.mark.parametrize("gated", [True, False])
+def test_identity_experts_only(T, gated):
+    h, wt = torch.randn(T, 64).bfloat16(), torch.rand(T, 2)
+    up, down = torch.empty(0, 128 if gated else 64, 64).bfloat16(), torch.empty(0, 64, 64).bfloat16()
+    got = seqmix.moe_experts(h.cuda(), torch.randint(0, 3, (T, 2), dtype=torch.int32).cuda(), wt.cuda(), up.cuda(), down.cuda(), gated)
+    # two f32 products of 24 x 8 bits and their sum
+    assert torch.allclose(got.cpu(), h.float() * wt.sum(1, keepdim=True), rtol=2.0 ** -21, atol=0)
