@@ -43,6 +43,7 @@ __global__ __launch_bounds__(512) void logmel_kernel(
   __shared__ float even[FPW][FOLD_LD + 1], odd[FPW][FOLD_LD + 1];   // odd row strides: a lane per frame
   __shared__ float power[FPW][POW_LD];
   __shared__ float top[8];
+  __shared__ int lost[FPW];            // the frame has bins that are not finite
   const int b = blockIdx.y, f0 = blockIdx.x * FPW;
   const float* x = audio + (size_t)b * n_samples;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -66,6 +67,7 @@ __global__ __launch_bounds__(512) void logmel_kernel(
   };
   if (wave < 7) load(0);
 
+  if (threadIdx.x < FPW) lost[threadIdx.x] = 0;
   // the samples of all frames, reflected at the ends (center = True)
   for (int i = threadIdx.x; i < SPAN; i += 512) {
     int idx = f0 * HOP + i - NFFT / 2;
@@ -106,11 +108,16 @@ __global__ __launch_bounds__(512) void logmel_kernel(
     for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        if (bin + 16 * t < NBINS) power[4 * kq + r][bin + 16 * t] = re[t][r] * re[t][r] + im[t][r] * im[t][r];
+        if (bin + 16 * t < NBINS) {
+          const float e = re[t][r] * re[t][r] + im[t][r] * im[t][r];
+          power[4 * kq + r][bin + 16 * t] = e;
+          if (!(e < INFINITY)) lost[4 * kq + r] = 1;
+        }
   }
   __syncthreads();
 
-  // a thread per band and four frames
+  // a thread per band and four frames; a frame with samples that are not finite, or whose power is
+  // not, counts as silent: the maximum below is of the others, which keep their values
   float wmax = -FLT_MAX;
   const int mel = threadIdx.x & 127, fg = threadIdx.x >> 7;
   if (mel < n_mels) {
@@ -125,7 +132,7 @@ __global__ __launch_bounds__(512) void logmel_kernel(
     for (int r = 0; r < 4; ++r) {
       const int f = f0 + 4 * fg + r;
       if (f < n_frames) {
-        const float lv = log10f(fmaxf(acc[r], 1e-10f));
+        const float lv = log10f(lost[4 * fg + r] ? 1e-10f : fmaxf(acc[r], 1e-10f));
         out[((size_t)b * n_frames + f) * n_mels + mel] = lv;
         wmax = fmaxf(wmax, lv);
       }

@@ -50,3 +50,18 @@ def test_encoder_of_80_bands_on_the_tiled_path(monkeypatch):
     b = model.encode(audio).float()
     # the two paths round the residual stream at other places: a few bf16 ulps after three layers
     assert (a - b).norm() <= 0.01 * b.norm()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")])
+def test_samples_that_are_not_finite_cost_their_frames_only(value):
+    c = ref.MelConstants.create(80)
+    x = torch.from_numpy(0.1 * np.random.RandomState(3).randn(2, 16000)).float()
+    bad = x.clone()
+    bad[0, 8000] = value
+    st = torch.stft(x.double(), 400, 160, window=c.window.double(), return_complex=True, center=True, pad_mode="reflect")
+    lg = (c.filters.double() @ st[..., :100].abs().square()).clamp(min=1e-10).log10()
+    lg[0, :, 49:52] = -10                                 # 160 t - 200 <= 8000 < 160 t + 200: silence
+    want = (torch.maximum(lg, lg.amax((1, 2), keepdim=True) - 8) + 4) / 4
+    got = ops.log_mel(bad.cuda(), c).cpu()
+    assert (got.double() - want).abs().max() <= 2.0 ** -8 * want.abs().clamp(min=1).max() + 1e-3
