@@ -863,6 +863,16 @@ def window_mfma_sizes(D: int, Dv: int) -> bool:
     return D % 8 == 0 and 0 < D <= 256 and Dv % 8 == 0 and 0 < Dv <= 512
 
 
+def window_token_takes(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, H: int, G: int,
+                       D: int, Dv: int) -> bool:
+    """Whether token steps run in the matrix-core form (``csrc/kernels/attn_window_token.hip``, whose
+    rule this is): bf16, heads up to 128 in multiples of 8, up to 16 query heads a key head, rows
+    that start on 16 bytes."""
+    return (q.dtype == torch.bfloat16 and D <= 128 and Dv <= 128 and D % 8 == 0 and Dv % 8 == 0
+            and H // G <= 16 and k_cache.shape[0] * k_cache.shape[1] < 1 << 31
+            and (q.data_ptr() | k_cache.data_ptr() | v_cache.data_ptr()) % 16 == 0)
+
+
 def window_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
                      cu_q: torch.Tensor, ctx_lens: torch.Tensor, block_tables: torch.Tensor,
                      positions: torch.Tensor, scale: float, softcap: float, window: int,
@@ -920,13 +930,14 @@ def window_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
         and (gate is None or (gs % 4 == 0 and gate.data_ptr() % 8 == 0))
     part = None
     if key_splits is None:
-        # 64-key windows a row can have, four (one per wave) to a workgroup
-        keys = max(int(max_ctx), 1) if window <= 0 else min(max(int(max_ctx), 1),
-                                                           window + 64 + keep_first)
-        # (a workgroup of the matrix-core token form reads 512 keys at once)
-        once = 1152 if q.dtype == torch.bfloat16 and D <= 128 and Dv <= 128 and D % 8 == Dv % 8 == 0 and H // G <= 16 else 256
-        key_splits = 1 if mfma or T * G >= 256 else \
-            max(1, min(16, -(-keys // once), 512 // max(1, T * G)))
+        key_splits = 1
+        if not mfma and T * G < 256:
+            # 64-key windows a row can have, four (one per wave) to a workgroup; the matrix-core token
+            # form reads 512 keys a round, and up to 1152 two or three rounds cost less than splits and
+            # their merge
+            keys = max(int(max_ctx), 1) if window <= 0 else min(max(int(max_ctx), 1), window + 64 + keep_first)
+            once = 1152 if window_token_takes(q, k_cache, v_cache, H, G, D, Dv) else 256
+            key_splits = max(1, min(16, -(-keys // once), 512 // max(1, T * G)))
     if key_splits > 1 and not mfma:
         part = torch.empty(T * H * key_splits * (Dv + 2), dtype=torch.float32, device=q.device)
     else:

@@ -115,3 +115,29 @@ def test_values_that_are_not_finite(value):
                 assert torch.equal(hit, torch.full((2,), value)) or math.isnan(value) and hit.isnan().all(), (key, hit)
             o.view(2, 64)[:, 5] = 0
             assert o.isfinite().all()
+
+
+def test_key_splits_of_the_other_form():
+    # caches that do not start on 16 bytes take the other kernel, whose workgroups read 256 keys a
+    # round: as many splits as before (with the splits of this form twice the time)
+    T, G, n = 8, 4, 3000
+    per = -(-n // 16)
+    flat = torch.randn(T * per * 16 * G * 128 + 4, device=DEV).bfloat16()
+    kc = flat[4:].view(T * per, 16, G * 128)
+    bt = torch.randperm(T * per, device=DEV).int().view(T, per).contiguous()
+    q, cu = torch.randn(T, 16 * 128, device=DEV).bfloat16(), torch.arange(T + 1, dtype=torch.int32, device=DEV)
+    ctx, pos = torch.full((T,), n, dtype=torch.int32, device=DEV), torch.full((T,), n - 1, dtype=torch.int32, device=DEV)
+
+    def us(splits):
+        call = lambda: seqmix.window_attention(q, kc, kc, cu, ctx, bt, pos, 0.1, 0.0, 0, 0, None, 16, G, 128, 128, max_q=1, max_ctx=n,
+                                               key_splits=splits)
+        for _ in range(3):
+            call()
+        at = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        at[0].record()
+        for _ in range(20):
+            call()
+        at[1].record()
+        torch.cuda.synchronize()
+        return at[0].elapsed_time(at[1])
+    assert us(None) < 1.4 * us(12)
