@@ -16,6 +16,7 @@ from __future__ import annotations
 
 import copy
 import ctypes
+import functools
 import math
 import os
 
@@ -1661,7 +1662,15 @@ def gemm_sk_plan(M: int, N: int, K: int, epi: str = "bf16", pipe: bool = True) -
     rounds of tiles over the compute units. K chunks fill the chip where the tiles do not;
     each costs a write and a serial read of the tile's f32 partial (6 us, and 37 us a MB per
     chunk, fitted with the rest), so they pay for few rows and long K only. ``pipe`` False:
-    the general layouts only (operands the pipelined tiles do not take)."""
+    the general layouts only (operands the pipelined tiles do not take). The epilogue
+    ``epi`` is not in the model."""
+    return _sk_plan(M, N, K, pipe)
+
+
+# a function of plain values that an eager pass asks for every projection: 10 to 19 us on the host
+# each time, 0.1 for a shape that was asked before
+@functools.lru_cache(maxsize=4096)
+def _sk_plan(M: int, N: int, K: int, pipe: bool) -> tuple[int, int]:
     KT = K // 64
     best, best_t = (7, 1), float("inf")
     for lay, (bn, bm, step, around) in SK_LAYOUTS.items():
@@ -1755,7 +1764,7 @@ def gemm_sk(x: torch.Tensor, w: torch.Tensor, *, epi: str = "bf16", bias: torch.
         pipe = x.stride(0) >= K and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 \
             and N * K < 1 << 31 and x.stride(0) < 1 << 21 \
             and (y is None or (y.stride(0) % 8 == 0 and y.data_ptr() % 16 == 0))
-        pl, ps = gemm_sk_plan(M, N, K, epi, pipe)
+        pl, ps = _sk_plan(M, N, K, pipe)
         layout = pl if layout is None else layout
         splits = ps if splits is None else splits
     bn, bm = SK_LAYOUTS[layout][:2]

@@ -24,6 +24,15 @@ def test_plan_takes_the_general_layouts_where_the_tiles_do_not_fit():
             assert s == 1 or K // 64 // s >= 8
 
 
+def test_plan_of_a_shape_is_made_once():
+    M, N, K = 333, 6144, 4096
+    plan = ops.gemm_sk_plan(M, N, K)
+    made = ops._sk_plan.cache_info().misses
+    assert [ops.gemm_sk_plan(M, N, K, epi) for epi in ("bf16", "resid", "swiglu")] == [plan] * 3
+    assert ops._sk_plan.cache_info().misses == made
+    assert ops.gemm_sk_plan(M, N, K, pipe=False) != plan and ops._sk_plan.__wrapped__(M, N, K, True) == plan
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("layout", [k for k in sorted(ops.SK_LAYOUTS) if k >= ops.SK_PIPE])
 @pytest.mark.parametrize("stages", [1, 2, 3, 7])
