@@ -1653,28 +1653,33 @@ SK_LAYOUTS = {1: (128, 64, 0.60, 4.0), 7: (64, 64, 0.55, 4.0),
               15: (256, 128, 0.908, 4.0), 16: (128, 256, 0.784, 6.6), 17: (128, 192, 0.667, 4.6),
               18: (192, 192, 0.854, 4.6), 19: (128, 64, 0.309, 4.3), 20: (128, 128, 0.498, 3.6)}
 SK_PIPE = 12              # the first pipelined layout
+# numbers of layouts that are gone (other stage counts and wave splits of the general form, 256
+# features x 64 rows) -> the pipelined tile of that size, or the next smaller one
+SK_RENAMED = {0: 20, 2: 19, 3: 15, 4: 19, 5: 20, 6: 12, 8: 19, 9: 15, 10: 20, 11: 19}
 SK_CUS = 256
 _SK_WS: dict = {}
 
 
-def gemm_sk_plan(M: int, N: int, K: int, epi: str = "bf16", pipe: bool = True) -> tuple[int, int]:
+def gemm_sk_plan(M: int, N: int, K: int, epi: str = "bf16", layouts=None, *,
+                 pipe: bool = True) -> tuple[int, int]:
     """(layout, K chunks) for a shape: the fewest microseconds by SK_LAYOUTS, counting whole
     rounds of tiles over the compute units. K chunks fill the chip where the tiles do not;
     each costs a write and a serial read of the tile's f32 partial (6 us, and 37 us a MB per
     chunk, fitted with the rest), so they pay for few rows and long K only. ``pipe`` False:
-    the general layouts only (operands the pipelined tiles do not take). The epilogue
-    ``epi`` is not in the model."""
-    return _sk_plan(M, N, K, pipe)
+    the general layouts only (operands the pipelined tiles do not take). ``layouts``: among
+    these only (numbers of SK_LAYOUTS or SK_RENAMED). The epilogue ``epi`` is not in the model."""
+    return _sk_plan(M, N, K, pipe, None if layouts is None else tuple(layouts))
 
 
 # a function of plain values that an eager pass asks for every projection: 10 to 19 us on the host
 # each time, 0.1 for a shape that was asked before
 @functools.lru_cache(maxsize=4096)
-def _sk_plan(M: int, N: int, K: int, pipe: bool) -> tuple[int, int]:
+def _sk_plan(M: int, N: int, K: int, pipe: bool, layouts: tuple | None = None) -> tuple[int, int]:
     KT = K // 64
+    only = SK_LAYOUTS if layouts is None else {SK_RENAMED.get(x, x) for x in layouts}
     best, best_t = (7, 1), float("inf")
     for lay, (bn, bm, step, around) in SK_LAYOUTS.items():
-        if N % bn or (lay >= SK_PIPE) != (pipe and N % 128 == 0):
+        if N % bn or (lay >= SK_PIPE) != (pipe and N % 128 == 0) or lay not in only:
             continue
         tiles = -(-M // bm) * (N // bn)
         for s in (1, 2, 3, 4, 6, 8):
@@ -1741,7 +1746,8 @@ def gemm_sk(x: torch.Tensor, w: torch.Tensor, *, epi: str = "bf16", bias: torch.
     x [M, K] bf16 (row stride may exceed K), w [N, K] bf16 row-major.
     ``epi``: "bf16" -> [M, N] (+ f32 ``bias``, ``act`` "gelu"); "swiglu" -> silu(gate) * up
     [M, N / 2] (gate rows [0, N/2), up rows [N/2, N)); "resid" -> ``residual``
-    [M, N] += X W^T (+ ``bias``) in place (one bf16 rounding), returned."""
+    [M, N] += X W^T (+ ``bias``) in place (one bf16 rounding), returned. ``layout``: a number of
+    SK_LAYOUTS or SK_RENAMED (None: the plan's)."""
     N, K = w.shape
     M = x.shape[0]
     assert x.shape[1] == K, (x.shape, w.shape)
@@ -1759,7 +1765,7 @@ def gemm_sk(x: torch.Tensor, w: torch.Tensor, *, epi: str = "bf16", bias: torch.
     if x.stride(1) != 1 or not w.is_contiguous():
         raise ValueError("gemm_sk needs K-contiguous operands")
     y = residual if epi == "resid" else out
-    if layout is None or splits is None:
+    if layout is None or splits is None or layout in SK_RENAMED:
         # the pipelined tiles move whole 16-byte pieces of the rows at 32-bit offsets
         pipe = x.stride(0) >= K and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 \
             and N * K < 1 << 31 and x.stride(0) < 1 << 21 \
@@ -1767,6 +1773,8 @@ def gemm_sk(x: torch.Tensor, w: torch.Tensor, *, epi: str = "bf16", bias: torch.
         pl, ps = _sk_plan(M, N, K, pipe)
         layout = pl if layout is None else layout
         splits = ps if splits is None else splits
+        if layout in SK_RENAMED:
+            layout = SK_RENAMED[layout] if pipe else 1
     bn, bm = SK_LAYOUTS[layout][:2]
     if N % bn or K % 64:
         raise ValueError(f"gemm_sk layout {layout}: N {N} / K {K} not tileable")

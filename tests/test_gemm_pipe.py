@@ -33,6 +33,27 @@ def test_plan_of_a_shape_is_made_once():
     assert ops.gemm_sk_plan(M, N, K, pipe=False) != plan and ops._sk_plan.__wrapped__(M, N, K, True) == plan
 
 
+def test_plan_among_some_layouts():
+    for layouts in ((0, 1, 2, 3, 4, 5), [12], (6,), (20, 7)):
+        lay, _ = ops.gemm_sk_plan(300, 6144, 4096, "bf16", layouts)
+        assert lay in {ops.SK_RENAMED.get(x, x) for x in layouts}
+    assert ops.gemm_sk_plan(300, 6144, 4096, layouts=(0, 4), pipe=False)[0] in (1, 7)
+    assert set(ops.SK_RENAMED) | set(ops.SK_LAYOUTS) == set(range(21))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", sorted(ops.SK_RENAMED))
+@pytest.mark.parametrize("off", [0, 4])
+def test_layout_numbers_that_are_gone(layout, off):
+    """They still name a tile; output rows that are not 16-byte aligned take the general one."""
+    g = torch.Generator().manual_seed(layout)
+    x, w = torch.randn(150, 1024, generator=g).bfloat16().cuda(), (torch.randn(512, 1024, generator=g) / 32).bfloat16().cuda()
+    for splits in (None, 1, 2):
+        y = torch.zeros(150, 512 + off, dtype=torch.bfloat16, device="cuda")[:, :512]
+        ops.gemm_sk(x, w, layout=layout, splits=splits, out=y)
+        _close(y, x.double() @ w.double().t(), 1024)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("layout", [k for k in sorted(ops.SK_LAYOUTS) if k >= ops.SK_PIPE])
 @pytest.mark.parametrize("stages", [1, 2, 3, 7])
