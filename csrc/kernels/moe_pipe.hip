@@ -19,12 +19,16 @@
 
 #define MP_GROUP 4
 
+// In full 32 bits: the hardware's exp2 and reciprocal (sigmoid_fast) are off by up to |a| ulp, which
+// makes the whole call's error against 64 bits larger in the fifth digit (512 tokens: 0.00234913,
+// 0.00234917), for 2 to 3 % less time (16 experts of 2048 x 1408, 4 a token; 64 tokens 61.0, 59.8 us;
+// 512: 87.8, 85.7; 2048: 189, 183).
 template <int MODE> __device__ __forceinline__ float moe_act(float a, float u, float limit) {
-  if constexpr (MODE == 1) return a * sigmoid_fast(a) * u;
+  if constexpr (MODE == 1) return silu_f(a) * u;
   else if constexpr (MODE == 2) { const float r = fmaxf(a, 0.f); return r * r; }
   else if constexpr (MODE == 3) {
     const float g = fminf(a, limit);
-    return g * sigmoid_fast(1.702f * g) * (fminf(fmaxf(u, -limit), limit) + 1.f);
+    return g * sigmoid_f(1.702f * g) * (fminf(fmaxf(u, -limit), limit) + 1.f);
   } else return a;
 }
 

@@ -66,3 +66,24 @@ def test_identity_experts_only(T, gated):
     got = seqmix.moe_experts(h.cuda(), torch.randint(0, 3, (T, 2), dtype=torch.int32).cuda(), wt.cuda(), up.cuda(), down.cuda(), gated)
     # two f32 products of 24 x 8 bits and their sum
     assert torch.allclose(got.cpu(), h.float() * wt.sum(1, keepdim=True), rtol=2.0 ** -21, atol=0)
+
+
+@pytest.mark.gpu
+def test_activation_keeps_32_bits():
+    # gate sums of two columns, up products of one, an identity behind them: the output is the
+    # activation itself, rounded to bfloat16
+    T, F = 4096, 64
+    a = -20 - 60 * torch.rand(T, F, generator=torch.Generator().manual_seed(0), dtype=torch.float64)
+    hi = a.bfloat16()
+    lo = (a - hi.double()).bfloat16()
+    h = torch.cat([hi, lo, torch.ones(T, 1).bfloat16(), torch.zeros(T, F - 1).bfloat16()], 1)
+    up, down = torch.zeros(1, 2 * F, 3 * F), torch.zeros(1, 3 * F, F)
+    up[0, :F, :F] = up[0, :F, F:2 * F] = down[0, :F] = torch.eye(F)
+    up[0, F:, 2 * F] = 1
+    got = seqmix.moe_experts(h.cuda(), torch.zeros(T, 1, dtype=torch.int32).cuda(), torch.ones(T, 1).cuda(), up.bfloat16().cuda(),
+                             down.bfloat16().cuda(), True).cpu()[:, :F]
+    s = hi.double() + lo.double()
+    want = (s * torch.sigmoid(s)).bfloat16().float()
+    # an error of 2 ulp (exponential, sum and quotient: 2^-22) moves 2^-22 / 2^-8 of the values over
+    # a rounding boundary at the most; sigmoid_fast's some 2e-4 of them
+    assert (got != want).float().mean() <= 2.0 ** -14
