@@ -1644,15 +1644,18 @@ def gemm_tile(x: torch.Tensor, w: torch.Tensor, *, bias: torch.Tensor | None = N
 # Split-K tiled GEMM with an in-launch reduction (csrc/kernels/gemm_sk.hip, gemm_pipe.hip)
 _SK_EPI = {"bf16": 0, "swiglu": 1, "resid": 2}
 # layout -> (features, rows, us a K step of 64 takes a compute unit, us around a tile's K
-# loop): 1 and 7 are the general form, 12 on the pipelined tiles, one workgroup per CU. The
-# times are fitted to 77 measured shapes (80 to 3000 rows, N 1280 to 28672, K 1280 to 14336,
-# cold weights, 1 to 8 K chunks): the plan they give is within 1 % of the fastest layout on
-# average, within 13 % at worst.
+# loop): 1 and 7 are the general form, 12 on the pipelined tiles, one workgroup per CU. Times
+# fitted to measured ones without an epilogue of weight: they are there to rank, and 0.60 to 1.35
+# of what a whole call takes (0.67 on average with GELU). Over 60 shapes (80 to 9000 rows, N 512
+# to 28672, K 512 to 14336, cold weights, every layout and K split: profiles/gemm_plan_grid.txt)
+# the plan is the fastest in 54, 0.6 % behind the fastest on average and 16 % at worst (9000 x
+# 2048 x 512 with GELU: 46.8 us, 40.3).
 SK_LAYOUTS = {1: (128, 64, 0.60, 4.0), 7: (64, 64, 0.55, 4.0),
               12: (256, 256, 1.20, 10.3), 13: (256, 192, 1.075, 5.5), 14: (192, 256, 1.073, 5.5),
               15: (256, 128, 0.908, 4.0), 16: (128, 256, 0.784, 6.6), 17: (128, 192, 0.667, 4.6),
               18: (192, 192, 0.854, 4.6), 19: (128, 64, 0.309, 4.3), 20: (128, 128, 0.498, 3.6)}
 SK_PIPE = 12              # the first pipelined layout
+SK_WHOLE = 12             # the layout that the plan does not split along K
 # numbers of layouts that are gone (other stage counts and wave splits of the general form, 256
 # features x 64 rows) -> the pipelined tile of that size, or the next smaller one
 SK_RENAMED = {0: 20, 2: 19, 3: 15, 4: 19, 5: 20, 6: 12, 8: 19, 9: 15, 10: 20, 11: 19}
@@ -1665,7 +1668,10 @@ def gemm_sk_plan(M: int, N: int, K: int, epi: str = "bf16", layouts=None, *,
     """(layout, K chunks) for a shape: the fewest microseconds by SK_LAYOUTS, counting whole
     rounds of tiles over the compute units. K chunks fill the chip where the tiles do not;
     each costs a write and a serial read of the tile's f32 partial (6 us, and 37 us a MB per
-    chunk, fitted with the rest), so they pay for few rows and long K only. ``pipe`` False:
+    chunk, fitted with the rest), so they pay for few rows and long K only, and never on 256 x 256
+    tiles: these fill the chip with MFMAs, where a K step takes longer than the fit has it (4096 x
+    14336: 1280 rows in three chunks 160 us, the 256 x 192 tiles in two 135; 2048 rows in two 205,
+    the 128 x 256 tiles whole 182; the fastest in none of the 60 shapes). ``pipe`` False:
     the general layouts only (operands the pipelined tiles do not take). ``layouts``: among
     these only (numbers of SK_LAYOUTS or SK_RENAMED). The epilogue ``epi`` is not in the model."""
     return _sk_plan(M, N, K, pipe, None if layouts is None else tuple(layouts))
@@ -1683,7 +1689,7 @@ def _sk_plan(M: int, N: int, K: int, pipe: bool, layouts: tuple | None = None) -
             continue
         tiles = -(-M // bm) * (N // bn)
         for s in (1, 2, 3, 4, 6, 8):
-            if s > 1 and KT // s < 8:
+            if s > 1 and (KT // s < 8 or lay == SK_WHOLE):
                 continue
             t = -(-tiles * s // SK_CUS) * (-(-KT // s) * step + around)
             if s > 1:

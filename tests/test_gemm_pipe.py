@@ -41,6 +41,15 @@ def test_plan_among_some_layouts():
     assert set(ops.SK_RENAMED) | set(ops.SK_LAYOUTS) == set(range(21))
 
 
+def test_largest_tiles_are_not_split():
+    # 1280 x 4096 x 14336: 160 us in three chunks of 256 x 256 tiles, 135 in two of 256 x 192
+    for M in (1, 80, 640, 1000, 1280, 2048, 3000, 9000):
+        for N, K in ((512, 2048), (1280, 5120), (4096, 4096), (4096, 14336), (7168, 8192), (8192, 28672)):
+            lay, s = ops.gemm_sk_plan(M, N, K)
+            assert lay != ops.SK_WHOLE or s == 1, (M, N, K)
+    assert ops.gemm_sk_plan(1280, 4096, 14336) == (13, 2) and ops.gemm_sk_plan(2048, 4096, 14336) == (16, 1)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("layout", sorted(ops.SK_RENAMED))
 @pytest.mark.parametrize("off", [0, 4])
