@@ -9,7 +9,8 @@
 // the next instantiated sizes), the causal bound from each row's absolute position (with a
 // sliding window the keys before it are neither gathered nor visited), a learned per-head sink
 // in the softmax denominator, and the output gate sigmoid(gate), applied before the unpadded
-// heads go to rows of any stride.
+// heads go to rows of any stride. Numerator and denominator are of the same rounded weights
+// (flash_pipe.h has the errors).
 // 2048 rows of 16 heads, 192 / 128: 99.5 us before (128 rows in four waves, tiles through
 // registers, scores, exponentials and products one after the other), 55 now; 4 x that: 365, 120;
 // 256 / 128: 111, 75. A single prompt is one round of the CUs, as long as its last rows (32

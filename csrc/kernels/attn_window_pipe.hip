@@ -4,7 +4,8 @@
 // A workgroup is QW KS waves: QW blocks of 32 query rows of one head (and up to 128 of its value
 // columns), the key tiles that these rows see split into KS runs. Tiles that lie wholly between
 // the kept first tokens and the rows' windows are skipped; a tile that every row of a wave sees
-// whole takes no per-score tests. Head sizes between the built ones are padded in LDS.
+// whole takes no per-score tests. Head sizes between the built ones are padded in LDS. Numerator
+// and denominator are of the same rounded weights (flash_pipe.h has the errors).
 // What bounds it at 128 columns: MFMAs, LDS and L2 about alike (flash_pipe.h). 2048 rows of 16
 // heads (4 key heads) of 128, window 1024: 92 us before (256 rows a workgroup, half of the CUs;
 // tiles through registers; maximum, exponentials and products one after the other), 35 now; without a window 128, 50; 64 rows behind 2000: 99, 29.
@@ -187,6 +188,11 @@ static int launch(const WinAttnParams& p, int max_q, hipStream_t st) {
 
 // 64 query rows and two key runs while these workgroups are one round of the 256 CUs, then 128
 // rows and two runs, then 128 rows and one run in four waves, two workgroups a CU.
+// Transformed scores (GEN) have the middle form only, as each form is four more kernels to build;
+// it is the faster one against the kernel before it at every size measured (cap 20, 4 key heads,
+// window 1024; us before, now: 32 rows x 16 heads of 64: 11.9, 10.1; 100 rows x 8 of 128: 17.0,
+// 12.4; 320 behind 1000 x 16 of 128: 102, 51; 2048 x 32 of 128: 115, 93; 4096: 222, 184). The rule
+// of the other scores would give 100 rows 11.6, 320 behind 1000 46.8, 4096 x 32 169.
 template <int DK, int DV>
 static int launch_rows(const WinAttnParams& p, int max_q, hipStream_t st) {
   if (p.cap > 0.f || p.slopes || !(p.scale > 0.f)) return launch<DK, DV, 4, 2, true>(p, max_q, st);

@@ -1,5 +1,5 @@
 // Device parts of the software-pipelined tile GEMM (gemm_pipe.hip; the experts' grouped
-// GEMM in moe.hip): direct-to-LDS loads, the K loop of a tile, and the way of a wave's
+// GEMM in moe_pipe.hip): direct-to-LDS loads, the K loop of a tile, and the way of a wave's
 // results through LDS.
 #pragma once
 #include "common.h"

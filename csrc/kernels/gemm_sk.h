@@ -30,7 +30,10 @@ __device__ __forceinline__ void sk_wait_vm() {
 // GELU through erfc's rational form (Abramowitz and Stegun 7.1.26, |error| <= 1.5e-7):
 // (v + |v|) / 2 - |v| erfc(|v| / sqrt 2) / 2 has no cancellation in the negative tail, where
 // 1 + erf(z) keeps an absolute error of half an ulp of one, and a third of erff's
-// instructions - with one wave per SIMD nothing hides an epilogue's arithmetic.
+// instructions - with one wave per SIMD nothing hides an epilogue's arithmetic. Its argument is the
+// f32 sum, where it was rounded to bf16 before erff: largest relative error of the bf16 result over
+// the values from -6 on, before and now: -6 to -5 1.04, 0.0072; -4 to -3 0.033, 0.0041 (rounding the
+// result alone: 0.0039); -2 to -1 0.0097, 0.0039; above 0 0.0079, 0.0039.
 __device__ __forceinline__ float sk_gelu(float v) {
   const float a = fabsf(v), c = fminf(a, 1e4f);        // erfc is 0 there; no inf * 0
   const float t = __builtin_amdgcn_rcpf(1.f + 0.23164188f * c);   // 0.3275911 / sqrt 2

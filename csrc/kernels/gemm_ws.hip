@@ -1,6 +1,8 @@
 // Row-resident weight-streaming MFMA GEMM for prompt passes:
 // Y[M, N] = X[M, K] W[N, K]^T with M up to a few hundred rows (one prefill pass
-// of the intent decoder: ~300 - 1200 prompt tokens).
+// of the intent decoder: ~300 - 1200 prompt tokens). The models' projections run on gemm_pipe.hip,
+// which is faster for their shapes; this one is an op of its own (ops.gemm_ws) and what the
+// benchmarks compare with.
 //
 // At M ~ 300 a projection is bounded by streaming its weights (gate|up: 235 MB,
 // ~45 us at HBM speed) about as much as by its MFMA work, and a square output

@@ -170,7 +170,7 @@ def main() -> int:
         out["prefill"] = {"rows": T, "rank_pass_ms_local": round(pf_ms, 3),
                           "allreduces": n_ar, "allreduce_bytes": nbytes,
                           "projected_pass_ms": [round(pf_ms + ar[0], 2), round(pf_ms + ar[1], 2)],
-                          "gemms": "ops.proj (gemm_sk / gemm_ws), no hipBLASLt"}
+                          "gemms": "ops.proj (gemm_sk), no hipBLASLt"}
     print(json.dumps(out), flush=True)
     return 0
 
