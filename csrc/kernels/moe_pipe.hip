@@ -12,8 +12,8 @@
 // Bound by the way L2 -> LDS and by the last round of tiles, as in gemm_pipe.hip; with few
 // tokens by the stream of cold weights, which the smallest tile's four stages keep in
 // flight. Against the form without LDS for the weights it replaces (whole moe_experts call,
-// 16 experts of 2048 x 1408, 4 a token): 1 token 83 -> 28 us, 64: 127 -> 62, 512: 262 -> 92,
-// 2048: 543 -> 188, 4000: 881 -> 307.
+// 16 experts of 2048 x 1408, 4 a token): 1 token 83 -> 26 us, 64: 114 -> 61, 512: 263 -> 89,
+// 2048: 537 -> 190, 4000: 894 -> 312.
 #include "seqmix.h"
 #include "gemm_pipe.h"
 
