@@ -93,13 +93,16 @@ def test_rows_off_16_bytes_take_the_other_kernel():
 def _us(call, n=20):
     for _ in range(3):
         call()
-    at = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
-    at[0].record()
-    for _ in range(n):
-        call()
-    at[1].record()
-    torch.cuda.synchronize()
-    return at[0].elapsed_time(at[1]) * 1e3 / n
+    us = []
+    for _ in range(8):                # the fastest of eight: clocks that have yet to rise do not count
+        at = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        at[0].record()
+        for _ in range(n):
+            call()
+        at[1].record()
+        torch.cuda.synchronize()
+        us.append(at[0].elapsed_time(at[1]) * 1e3 / n)
+    return min(us)
 
 
 @pytest.mark.parametrize("D,H,G", [(64, 20, 20), (128, 32, 8)])

@@ -133,11 +133,14 @@ def test_key_splits_of_the_other_form():
                                                key_splits=splits)
         for _ in range(3):
             call()
-        at = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
-        at[0].record()
-        for _ in range(20):
-            call()
-        at[1].record()
-        torch.cuda.synchronize()
-        return at[0].elapsed_time(at[1])
+        got = []
+        for _ in range(8):            # the fastest of eight: clocks that have yet to rise do not count
+            at = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+            at[0].record()
+            for _ in range(20):
+                call()
+            at[1].record()
+            torch.cuda.synchronize()
+            got.append(at[0].elapsed_time(at[1]))
+        return min(got)
     assert us(None) < 1.4 * us(12)
