@@ -379,7 +379,8 @@ __global__ __launch_bounds__(64 * QW * KS, D == 64 && QW * KS == 4 ? 3 : 2) void
       [&](int, unsigned stage) __attribute__((always_inline)) { fetch(vf, va, stage); });
 
   fl_sync();                                                // every wave is done with the rings
-  fl_merge<NDT, QW, KS>(acc, m, l, reinterpret_cast<float*>(lds), run, wq, lane);
+  fl_merge<NDT, QW, KS>(acc, m, l, reinterpret_cast<float*>(lds), run, wq, lane,
+                         KS == 4 && ntiles <= 1);   // (with two runs it would save less and cost long prompts up to 2 %)
   if (run) return;
   const float inv = l > 0.f ? 1.f / l : 0.f;
 #pragma unroll

@@ -96,6 +96,7 @@ def _us(call, n=20):
     us = []
     for _ in range(8):                # the fastest of eight: clocks that have yet to rise do not count
         at = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        torch.cuda._sleep(500000)     # the host is ahead
         at[0].record()
         for _ in range(n):
             call()
@@ -130,3 +131,12 @@ def test_long_causal_prompts():
                                      causal=True, max_q=n, cu_k=cu)
     # fewer heads take no longer (0.96 of 32 heads' time; 1.22 on one run)
     assert _us(call(20)) < 1.1 * _us(call(32))
+
+
+def test_one_tile_has_nothing_to_merge():
+    def call(n, H=32):
+        q, cu = torch.randn(n, 3 * H * 64, device=DEV).bfloat16(), torch.tensor([0, n], dtype=torch.int32, device=DEV)
+        return lambda: ops.attention(q[:, :H * 64], q[:, H * 64:2 * H * 64], q[:, 2 * H * 64:], cu, n_heads=H, n_kv=H, head_dim=64,
+                                     causal=True, max_q=n, cu_k=cu)
+    # 0.88 of the time of two tiles; 1.00 with the merge of runs that have none
+    assert _us(call(64)) < 0.95 * _us(call(100))
