@@ -283,7 +283,8 @@ extern "C" int loqa_latent_prefill(const void* q, long q_st, const void* k, cons
   if ((((size_t)k | (size_t)v) & 15) || (long)H * DK >= (1L << 24)) return (int)hipErrorInvalidValue;
   // 64 rows and two runs (keys of 256 columns: one) while these workgroups are one round of the
   // CUs, then 128 rows and two runs (160 KB of LDS at 192 columns), or one run, whose workgroups
-  // share a CU
+  // share a CU: with feeds of up to 128 rows from a second round on (us with two runs and with one,
+  // 9 feeds x 32 heads: 20 rows, 192 / 128 columns: 18, 9.8; 128 rows behind 300: 41.5, 31)
   const long n64 = (long)((max_q + 63) / 64) * H * B, n128 = (long)((max_q + 127) / 128) * H * B;
 #define RUN(A, C, QW, KS)                                                                     \
   do {                                                                                        \
@@ -299,7 +300,7 @@ extern "C" int loqa_latent_prefill(const void* q, long q_st, const void* k, cons
   if (DK == A && DV == C) {                                                                   \
     constexpr int K2 = A > 192 ? 1 : 2;                                                       \
     if (n64 <= 256) RUN(A, C, 2, K2);                                                         \
-    else if (n128 <= 512) RUN(A, C, 4, K2);                                                   \
+    else if (n128 <= (max_q <= 128 ? 256 : 512)) RUN(A, C, 4, K2);                                                   \
     else RUN(A, C, 4, 1);                                                                     \
   }
   GO(64, 64) GO(128, 64) GO(192, 64) GO(256, 64) GO(64, 128) GO(128, 128) GO(192, 128) GO(256, 128)

@@ -187,18 +187,20 @@ static int launch(const WinAttnParams& p, int max_q, hipStream_t st) {
 }
 
 // 64 query rows and two key runs while these workgroups are one round of the 256 CUs, then 128
-// rows and two runs, then 128 rows and one run in four waves, two workgroups a CU.
-// Transformed scores (GEN) have the middle form only, as each form is four more kernels to build;
-// it is the faster one against the kernel before it at every size measured (cap 20, 4 key heads,
-// window 1024; us before, now: 32 rows x 16 heads of 64: 11.9, 10.1; 100 rows x 8 of 128: 17.0,
-// 12.4; 320 behind 1000 x 16 of 128: 102, 51; 2048 x 32 of 128: 115, 93; 4096: 222, 184). The rule
-// of the other scores would give 100 rows 11.6, 320 behind 1000 46.8, 4096 x 32 169.
+// rows and two runs, then 128 rows and one run in four waves, two or three workgroups a CU. Feeds
+// of up to 128 rows, whose chain of tiles is short, take the last form from a second round on (us
+// with two runs and with one, 9 feeds x 32 heads: 20 rows, 64 columns: 14.3, 7.6; 128 rows behind
+// 300, 128 columns: 39, 29). Transformed scores (GEN) go without the first form, which would
+// be four more kernels to build (100 rows x 8 heads of 128: 12.4, with it 11.6; 320 behind 1000
+// x 16: 51, 47).
 template <int DK, int DV>
 static int launch_rows(const WinAttnParams& p, int max_q, hipStream_t st) {
-  if (p.cap > 0.f || p.slopes || !(p.scale > 0.f)) return launch<DK, DV, 4, 2, true>(p, max_q, st);
   const long hd = (long)p.H * p.vparts * p.B, n64 = (max_q + 63) / 64 * hd, n128 = (max_q + 127) / 128 * hd;
+  const bool one = n128 > (max_q <= 128 ? 256 : 512);
+  if (p.cap > 0.f || p.slopes || !(p.scale > 0.f))
+    return one ? launch<DK, DV, 4, 1, true>(p, max_q, st) : launch<DK, DV, 4, 2, true>(p, max_q, st);
   if (n64 <= 256) return launch<DK, DV, 2, 2, false>(p, max_q, st);
-  if (n128 <= 512) return launch<DK, DV, 4, 2, false>(p, max_q, st);
+  if (!one) return launch<DK, DV, 4, 2, false>(p, max_q, st);
   return launch<DK, DV, 4, 1, false>(p, max_q, st);
 }
 
