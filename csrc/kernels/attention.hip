@@ -694,6 +694,9 @@ static int launch_pipe(const AttnParams& p, int B, int max_q, hipStream_t s) {
 // 128 / one): 1500 x 8 heads of 64: 15.6, 20, 25; x 20 heads: 26, 22.7, 27; 6 x 1500 x 20 heads:
 // 133, 124, 106; 128 columns, paged: 320 rows behind 1000 x 32 heads: 31, 32, 40; 2048 x 32 heads
 // causal: 101, 60, 70; 4 x that: 349, 238, 200.
+// Short prompts of 128-column heads leave two runs at a second round: their chain of tiles is
+// short (128 / two, 128 / one; 9 prompts x 32 heads: 40 rows 14.7, 7.7; 128 behind 300 31.4, 22.6;
+// behind 1500 72.7, 63.6).
 // Long causal prompts of 64-column heads stay with two runs longer: half of the work is gone and
 // the last rows' chain of tiles is what the pass lasts (128 / two, 128 / one): 1400 x 32 heads 24,
 // 29; 2048 x 20 heads 40, 50; 4096 x 12 heads 68, 94, x 20 heads 116, 121; but 4 x 700 x 16 heads
@@ -701,7 +704,7 @@ static int launch_pipe(const AttnParams& p, int B, int max_q, hipStream_t s) {
 template <int D, int PAGES>
 static int launch_rows(const AttnParams& p, int B, int max_q, hipStream_t s) {
   const long n64 = (long)((max_q + 63) / 64) * p.Hq * B, n128 = (long)((max_q + 127) / 128) * p.Hq * B;
-  const long two = D == 128 ? 512 : !p.causal || max_q < 1024 ? 256 : max_q < 4096 ? 384 : 640;
+  const long two = D == 128 ? (max_q <= 128 ? 256 : 512) : !p.causal || max_q < 1024 ? 256 : max_q < 4096 ? 384 : 640;
   if (n64 <= 256) return launch_pipe<D, PAGES, 2, D == 64 ? 4 : 2>(p, B, max_q, s);
   if (n128 <= two) return launch_pipe<D, PAGES, 4, 2>(p, B, max_q, s);
   return launch_pipe<D, PAGES, 4, 1>(p, B, max_q, s);

@@ -140,3 +140,17 @@ def test_one_tile_has_nothing_to_merge():
                                      causal=True, max_q=n, cu_k=cu)
     # 0.88 of the time of two tiles; 1.00 with the merge of runs that have none
     assert _us(call(64)) < 0.95 * _us(call(100))
+
+
+def test_many_short_prompts():
+    # 128-column heads: more prompts than CUs do not take a second round (a ninth prompt: 1.0 of the
+    # time; 1.8 with two key runs)
+    _check([20, 1, 64, 33, 40, 40, 40, 40, 40], [20, 90, 64, 33, 40, 400, 40, 40, 41], 32, 8, 128, True, page=16, seed=11)
+
+    def call(B, n=40, H=32, G=8, D=128):
+        q, kc = torch.randn(B * n, H * D, device=DEV).bfloat16(), torch.randn(3 * B, G, 16, D, device=DEV).bfloat16()
+        cu, ctx = torch.arange(0, B * n + 1, n, dtype=torch.int32, device=DEV), torch.full((B,), n, dtype=torch.int32, device=DEV)
+        bt = torch.arange(3 * B, dtype=torch.int32, device=DEV).view(B, 3)
+        return lambda: ops.attention(q, kc, kc, cu, n_heads=H, n_kv=G, head_dim=D, causal=True, max_q=n, ctx_lens=ctx, block_tables=bt,
+                                     max_k=n)
+    assert _us(call(9)) < 1.4 * _us(call(8))
