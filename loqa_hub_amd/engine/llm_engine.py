@@ -392,7 +392,7 @@ class LLMEngine:
         graph = torch.cuda.CUDAGraph()
         k = ops._lib.kernels()
         # thread-local capture: the other GPU worker thread keeps running
-        with torch.cuda.graph(graph, capture_error_mode="thread_local"):
+        with ops.graph_capture(graph, capture_error_mode="thread_local"):
             st = ops._lib.stream_ptr(d32)
             src_off = dev["src"].data_ptr() // 4 - d32.data_ptr() // 4
             ops._lib.check(k.loqa_step_fetch(

@@ -440,7 +440,7 @@ class STTEngine:
         k = ops._lib.kernels()
         lib = ops._lib
         # thread-local capture: the other GPU worker thread keeps running
-        with torch.cuda.graph(graph, capture_error_mode="thread_local"):
+        with ops.graph_capture(graph, capture_error_mode="thread_local"):
             st = lib.stream_ptr(d32)
             src_off = dev["src"].data_ptr() // 4 - d32.data_ptr() // 4
             lib.check(k.loqa_step_fetch(
@@ -497,7 +497,7 @@ class STTEngine:
             self.model.encode(audio)
         torch.cuda.current_stream(self.device).wait_stream(s)
         graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(graph, pool=self._enc_graph_pool, capture_error_mode="thread_local"):
+        with ops.graph_capture(graph, pool=self._enc_graph_pool, capture_error_mode="thread_local"):
             out = self.model.encode(audio)
         g = {"graph": graph, "audio": audio, "out": out}
         self._enc_graphs[B] = g

@@ -358,7 +358,7 @@ class VitsGraphRunner:
         g = torch.cuda.CUDAGraph()
         # the placed TTS stream (never a new pool stream: utils/streams.py);
         # thread-local capture: the decoder threads keep launching meanwhile
-        with torch.cuda.graph(g, pool=self.pool, stream=st, capture_error_mode="thread_local"):
+        with ops.graph_capture(g, pool=self.pool, stream=st, capture_error_mode="thread_local"):
             out = fn()
         self.stats["captures"] += 1
         return g, out

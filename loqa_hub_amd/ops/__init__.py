@@ -14,6 +14,9 @@ elementwise/normalisation/attention/audio op around them is ours.
 """
 from __future__ import annotations
 
+import threading
+import gc
+import contextlib
 import copy
 import ctypes
 import functools
@@ -530,7 +533,7 @@ class contended_tuning:
                              rowsq_tiles=128)
         self._stream.synchronize()
         self._g = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(self._g, stream=self._stream):
+        with graph_capture(self._g, stream=self._stream):
             for i in range(12):
                 skinny_fused(self._x, self._ws[i % 3], "silu", self._scr, splits=1, rt=2, wr=4,
                              norm=True, rowsq_tiles=128)
@@ -652,7 +655,7 @@ def graph_time(fn, reps: int = 8, trials: int = 3) -> float:
             fn()
     torch.cuda.current_stream().wait_stream(s)
     g = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(g, capture_error_mode="thread_local"):
+    with graph_capture(g, capture_error_mode="thread_local"):
         for _ in range(reps):
             fn()
     g.replay()
@@ -1638,6 +1641,32 @@ def gemm_tile(x: torch.Tensor, w: torch.Tensor, *, bias: torch.Tensor | None = N
     p.layout = lay
     check(kernels().loqa_gemm_tile(ctypes.byref(p), stream_ptr(x)), "gemm_tile")
     return y
+
+
+# ---------------------------------------------------------------------------
+# Graph capture
+_CAPTURES = [0, False]     # captures that run now, whether the collector was on before them
+_CAPTURES_LOCK = threading.Lock()
+
+
+@contextlib.contextmanager
+def graph_capture(graph: "torch.cuda.CUDAGraph", **kw):
+    """``torch.cuda.graph`` during which no cyclic garbage is collected: a dropped engine's graphs
+    and streams are destroyed through HIP calls that a capturing thread may not make, and an
+    error in a destructor aborts the process."""
+    with _CAPTURES_LOCK:
+        if _CAPTURES[0] == 0:
+            _CAPTURES[1] = gc.isenabled()
+            gc.disable()
+        _CAPTURES[0] += 1
+    try:
+        with torch.cuda.graph(graph, **kw):
+            yield
+    finally:
+        with _CAPTURES_LOCK:
+            _CAPTURES[0] -= 1
+            if _CAPTURES[0] == 0 and _CAPTURES[1]:
+                gc.enable()
 
 
 # ---------------------------------------------------------------------------
