@@ -24,8 +24,8 @@
 //
 // delta_pass_kernel (a workgroup per sequence, head and 16 value columns) walks the
 // chunks in order with the state in MFMA accumulators: W S and (P q) S, u = U - W S,
-// S <- P(16) S + K^T u, o = (P q) S + B u. The four waves split the key channels and
-// add up W S through LDS. With v_mfma_f32_16x16x4_f32 lane 16 g + m holds of an
+// S <- P(16) S + K^T u, o = (P q) S + B u. Four waves split the key channels and
+// add up W S through LDS, two more form the outputs behind them. With v_mfma_f32_16x16x4_f32 lane 16 g + m holds of an
 // accumulator the rows 4 g + r (register r) of column m, and of a B operand row g of
 // a step; taking the rows 4 g + r as step r's k indices makes an accumulator's
 // registers the B operands of the next product as they are, and the A operand's four
@@ -44,8 +44,10 @@ struct DcParams {
   float* ws; float* o; int B;
 };
 
-// Workspace of one (chunk, head), DP the padded key size: W [16][DP], P q [16][DP],
-// (P(16, j) k_j) as [DP][16], P(16) [DP], U as [Dv][16], B [16][16].
+// Workspace of one (chunk, head), DP the padded key size: W and P q in the order of the MFMA
+// operand (per 16 channels a kilobyte: channels 4 g .. of token m at 16 g + m), (P(16, j) k_j)
+// as [DP][16], P(16) [DP], U as [Dv][16], B [16][16]. The pass reads all of it, so every load
+// there is a whole kilobyte: as rows of DP, W and P q came in 64-byte pieces.
 __host__ __device__ __forceinline__ size_t dc_stride(int DP, int Dv) {
   return (size_t)49 * DP + 16 * Dv + 256;
 }
@@ -127,7 +129,8 @@ __global__ __launch_bounds__(256) void delta_local_kernel(DcParams p) {
   }
   // a = P(i) k_i, c = P(i) q_i now
 #pragma unroll
-  for (int m = 0; m < NT; ++m) st_run<float, 4>(ws + 16 * DP + i * DP + 64 * m + 4 * q, c[m]);
+  for (int m = 0; m < NT; ++m)
+    st_run<float, 4>(ws + 16 * DP + (4 * m + q / 4) * 256 + (16 * (q % 4) + i) * 4, c[m]);
   // P(16, j) k_j and P(16), a thread per channel
   for (int d = tid; d < DP; d += 256) {
     float r = 1.f, kk[DC_C];
@@ -161,127 +164,212 @@ __global__ __launch_bounds__(256) void delta_local_kernel(DcParams p) {
     }
     if (key) {
 #pragma unroll
-      for (int t = 0; t < DC_C; ++t) ws[t * DP + col] = x[t];
+      for (int t = 0; t < DC_C; ++t) ks[t][col] = x[t];      // a column is its thread's own
     } else {
 #pragma unroll
       for (int t = 0; t < DC_C; t += 4)
         st_run<float, 4>(ws + 49 * DP + (size_t)(col - DP) * DC_C + t, x + t);
     }
   }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < NT; ++j) {
+    const int at = tid + 256 * j, l = at & 63;
+    float w[4];
+    ld_run<float, 4>(&ks[l & 15][16 * (at >> 6) + 4 * (l >> 4)], w);
+    st_run<float, 4>(ws + at * 4, w);
+  }
 }
 
-// (2 workgroups per CU at least: the accumulators stay in ordinary registers, which
-// the next products read as operands)
+// Every wave of the workgroup is here and its LDS writes are visible; global loads stay in
+// flight. Called from both roles of delta_pass_kernel, the same number of times by each.
+__device__ __forceinline__ void dc_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// The chunks of a sequence are a serial chain: X = W S, u = U - X, S <- P S + K^T u, with X
+// added up over the waves in between. Nothing but that may stand in its way: waves 0 - 3 run
+// the chain, with (P q) S while X travels through LDS, and leave their parts of X
+// and of (P q) S there; waves 4 and 5 take every other chunk, add up, form the outputs and
+// store them (DC_RING: what chunk c leaves is read before the barrier of chunk c + 2). Loads
+// are buffer loads, a chunk's block as the buffer: its address is a scalar and a lane's offset
+// stays. As four waves that did it all, with addresses per lane, a chunk took 1950 cycles, 800
+// of them MFMAs; now 1350 (2048 tokens, 16 heads of 128 x 128: 119 -> 79 us).
+#define DC_RING 3
+
 template <int NT>
-__global__ __launch_bounds__(256, 2) void delta_pass_kernel(DcParams p) {
-  constexpr int DP = 64 * NT, NS = NT <= 2 ? 4 : 2;
-  __shared__ float4v xs[2][4][64], ys[2][4][64];
+__global__ __launch_bounds__(384, 2) void delta_pass_kernel(DcParams p) {
+  constexpr int DP = 64 * NT;
+  __shared__ float4v xs[DC_RING][4][64], ys[DC_RING][4][64];
   const int b = blockIdx.x, h = blockIdx.y, e0 = blockIdx.z * 16;
-  const int q0 = p.cu_q[b], len = p.cu_q[b + 1] - q0;
+  const int q0 = __builtin_amdgcn_readfirstlane(p.cu_q[b]);
+  const int len = __builtin_amdgcn_readfirstlane(p.cu_q[b + 1]) - q0;
   if (len <= 0) return;
-  const int before = seq_chunks_before<DC_C>(p.cu_q, b);
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, m = lane & 15, g = lane >> 4;
+  const int before = __builtin_amdgcn_readfirstlane(seq_chunks_before<DC_C>(p.cu_q, b));
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, m = lane & 15, g = lane >> 4;
   const int D = p.D, Dv = p.Dv, nc = (len + DC_C - 1) / DC_C;
   const bool col = e0 + m < Dv;
   const int ec = min(e0 + m, Dv - 1);
-  // state [slots, H, Dv, D]: the wave's tile t holds the channels 16 (NT wave + t) ..
-  float* Sg = p.state + (((size_t)p.slots[b] * p.H + h) * Dv + ec) * D;
-  const bool fresh = p.pos[q0] == 0;
-  float4v S[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int d = 16 * (NT * wave + t) + 4 * g + r;
-      S[t][r] = !fresh && d < D ? Sg[d] : 0.f;
-    }
   const size_t st = dc_stride(DP, Dv), step = st * p.H;
   const float* ws = p.ws + ((size_t)before * p.H + h) * st;
-  struct Set { float4v W[NT], Q[NT], K[NT], G[NT], U; float B; };
-  auto fetch = [&](Set& f, int c) {
-    const float* w = ws + (size_t)c * step;
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      const int d0 = 16 * (NT * wave + t);
-      f.W[t] = *reinterpret_cast<const float4v*>(w + m * DP + d0 + 4 * g);
-      f.Q[t] = *reinterpret_cast<const float4v*>(w + 16 * DP + m * DP + d0 + 4 * g);
-      f.K[t] = *reinterpret_cast<const float4v*>(w + 32 * DP + (d0 + m) * DC_C + 4 * g);
-      f.G[t] = *reinterpret_cast<const float4v*>(w + 48 * DP + d0 + 4 * g);
-    }
-    f.U = *reinterpret_cast<const float4v*>(w + 49 * DP + (size_t)ec * DC_C + 4 * g);
-    f.B = w[49 * DP + 16 * Dv + m * DC_C + 4 * g + wave];
-  };
-  // the outputs of chunk c: wave w takes the tokens 4 g + w
-  auto outputs = [&](int c, int par) {
-    const float* y = reinterpret_cast<const float*>(&ys[par][0][lane]) + wave;
-    const float s = (y[0] + y[256]) + (y[512] + y[768]);
-    const int t = c * DC_C + 4 * g + wave;
-    if (col && t < len) p.o[(size_t)(q0 + t) * p.H * Dv + (size_t)h * Dv + e0 + m] = s;
-  };
   const float4v zero = {0.f, 0.f, 0.f, 0.f};
-  auto chunk = [&](Set& f, int c, int par) {
-    float4v X = zero, Y = zero;
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        X = __builtin_amdgcn_mfma_f32_16x16x4f32(f.W[t][r], S[t][r], X, 0, 0, 0);
-    xs[par][wave][lane] = X;
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        Y = __builtin_amdgcn_mfma_f32_16x16x4f32(f.Q[t][r], S[t][r], Y, 0, 0, 0);
-    __syncthreads();
-    const float4v u = f.U - ((xs[par][0][lane] + xs[par][1][lane]) +
-                             (xs[par][2][lane] + xs[par][3][lane]));
-#pragma unroll
-    for (int t = 0; t < NT; ++t) S[t] *= f.G[t];
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-#pragma unroll
-      for (int t = 0; t < NT; ++t)
-        S[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.K[t][r], u[r], S[t], 0, 0, 0);
-    const float uw = wave < 2 ? (wave == 0 ? u[0] : u[1]) : (wave == 2 ? u[2] : u[3]);
-    ys[par][wave][lane] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.B, uw, Y, 0, 0, 0);
-    // every wave wrote chunk c - 1's part before this chunk's barrier
-    if (c > 0) outputs(c - 1, par ^ 1);
-    fetch(f, min(c + NS, nc - 1));       // unconditional: the waits count loads
+  // 16 bytes a lane of a chunk's block: part (floats) and block are scalars, at (bytes) the lane's
+  auto load = [&](const float* block, int part, unsigned at) {
+    typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+    const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(block), 0, (int)(st * 4), 0x00020000), at, part * 4, 0);
+    return __builtin_bit_cast(float4v, v);
   };
-  // NS chunks' inputs in flight: a chunk takes less time than a trip to memory
-  Set f0, f1, f2, f3;
-  fetch(f0, 0);
-  fetch(f1, min(1, nc - 1));
-  int c = 0;
-  if constexpr (NS == 4) {
-    fetch(f2, min(2, nc - 1));
-    fetch(f3, min(3, nc - 1));
-    for (; c + 3 < nc; c += 4) {
-      chunk(f0, c, 0);
-      chunk(f1, c + 1, 1);
-      chunk(f2, c + 2, 0);
-      chunk(f3, c + 3, 1);
-    }
-    if (c < nc) chunk(f0, c, 0);
-    if (c + 1 < nc) chunk(f1, c + 1, 1);
-    if (c + 2 < nc) chunk(f2, c + 2, 0);
-  } else {
-    for (; c + 1 < nc; c += 2) {
-      chunk(f0, c, 0);
-      chunk(f1, c + 1, 1);
-    }
-    if (c < nc) chunk(f0, c, 0);
-  }
-  __syncthreads();
-  outputs(nc - 1, (nc - 1) & 1);
-  if (col)
+  const unsigned l16 = lane * 16, g16 = g * 16, k16 = (m * DC_C + 4 * g) * 4, u16 = (ec * DC_C + 4 * g) * 4;
+  auto sum = [&](const float4v (&v)[4][64]) { return (v[0][lane] + v[1][lane]) + (v[2][lane] + v[3][lane]); };
+  int slot = 0;
+  auto next = [](int at) { return at + 1 == DC_RING ? 0 : at + 1; };
+  if (wave < 4) {
+    // state [slots, H, Dv, D]: the wave's tile t holds the channels 16 (NT wave + t) ..
+    float* Sg = p.state + (((size_t)p.slots[b] * p.H + h) * Dv + ec) * D;
+    const bool fresh = p.pos[q0] == 0;
+    float4v S[NT];
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int d = 16 * (NT * wave + t) + 4 * g + r;
-        if (d < D) Sg[d] = S[t][r];
+        S[t][r] = !fresh && d < D ? Sg[d] : 0.f;
       }
+    struct Set { float4v W[NT], Q[NT], K[NT], G[NT], U; };
+    const float* block = ws;                // of the next chunk to fetch, then again the last one's:
+    int more = nc - 1;                      // loads in flight are counted, so none is left out
+    auto advance = [&]() {
+      block += more > 0 ? step : 0;
+      --more;
+    };
+    // A set's loads one by one: W and P q, two per tile, then K and P, then U. As a burst behind
+    // the MFMAs they queued up before the cache and took 20 us of a pass of 2048 tokens.
+    auto fetch = [&](Set& f, int k) {
+      const int t = (k % (2 * NT)) / 2, d0 = 16 * (NT * wave + t);
+      if (k == 4 * NT) f.U = load(block, 49 * DP, u16);
+      else if (k < 2 * NT && k % 2 == 0) f.W[t] = load(block, 16 * d0, l16);
+      else if (k < 2 * NT) f.Q[t] = load(block, 16 * DP + 16 * d0, l16);
+      else if (k % 2 == 0) f.K[t] = load(block, 32 * DP + 16 * d0, k16);
+      else f.G[t] = load(block, 48 * DP + d0, g16);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto fetch_all = [&](Set& f) {
+#pragma unroll
+      for (int k = 0; k <= 4 * NT; ++k) fetch(f, k);
+      advance();
+    };
+    // one chunk from f, and the loads of a later one into its set n
+    auto chunk = [&](Set& f, Set& n) {
+      float4v X = zero, Y = zero;
+#pragma unroll
+      for (int k = 0; k < 4 * NT; ++k) {
+        X = __builtin_amdgcn_mfma_f32_16x16x4f32(f.W[k / 4][k % 4], S[k / 4][k % 4], X, 0, 0, 0);
+        if (k % 2 == 1) fetch(n, k / 2);
+      }
+      xs[slot][wave][lane] = X;
+#pragma unroll
+      for (int k = 0; k < 4 * NT; ++k)
+        Y = __builtin_amdgcn_mfma_f32_16x16x4f32(f.Q[k / 4][k % 4], S[k / 4][k % 4], Y, 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      dc_barrier();
+      float4v x[4];
+#pragma unroll
+      for (int w = 0; w < 4; ++w) x[w] = xs[slot][w][lane];
+      fetch(n, 4 * NT);
+      const float4v u = f.U - ((x[0] + x[1]) + (x[2] + x[3]));
+#pragma unroll
+      for (int t = 0; t < NT; ++t) S[t] *= f.G[t];
+#pragma unroll
+      for (int k = 0; k < 4 * NT; ++k) {
+        S[k % NT] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.K[k % NT][k / NT], u[k / NT], S[k % NT], 0, 0, 0);
+        if (k % 2 == 1) fetch(n, 2 * NT + k / 2);
+      }
+      advance();
+      ys[slot][wave][lane] = Y;
+      slot = next(slot);
+    };
+    // the inputs of NS - 1 chunks in flight: a chunk takes less time than a trip to memory
+    constexpr int NS = NT <= 2 ? 4 : 2;
+    Set f0, f1, f2, f3;
+    fetch_all(f0);
+    int c = 0;
+    if constexpr (NS == 4) {
+      fetch_all(f1);
+      fetch_all(f2);
+      for (; c + 3 < nc; c += 4) {
+        chunk(f0, f3);
+        chunk(f1, f0);
+        chunk(f2, f1);
+        chunk(f3, f2);
+      }
+      if (c < nc) chunk(f0, f3);
+      if (c + 1 < nc) chunk(f1, f0);
+      if (c + 2 < nc) chunk(f2, f1);
+    } else {
+      for (; c + 1 < nc; c += 2) {
+        chunk(f0, f1);
+        chunk(f1, f0);
+      }
+      if (c < nc) chunk(f0, f1);
+    }
+    dc_barrier();
+    if (col)
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int d = 16 * (NT * wave + t) + 4 * g + r;
+          if (d < D) Sg[d] = S[t][r];
+        }
+  } else {
+    const int ldo = p.H * Dv, turn = wave - 4;
+    unsigned ro[4];                           // of a lane's entries in a chunk's rows; past every buffer if its column is none
+#pragma unroll
+    for (int r = 0; r < 4; ++r) ro[r] = col ? ((4u * g + r) * ldo + m) * 4 : 0xfffffff0u;
+    struct Set { float4v U, B; };
+    auto fetch = [&](Set& f, int c) {
+      const float* block = ws + (size_t)min(c, nc - 1) * step;
+      f.U = load(block, 49 * DP, u16);
+      f.B = load(block, 49 * DP + 16 * Dv, k16);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    int passed = 0;                           // barriers behind this wave, nc + 1 in the end
+    auto pass = [&](int upto) {
+      for (upto = min(upto, nc + 1); passed < upto; ++passed) dc_barrier();
+    };
+    auto chunk = [&](Set& f, int c) {
+      pass(c + 2);                            // chunk c has left its parts
+      slot = min(c, nc - 1) % DC_RING;        // (past the last chunk: that one again, unstored)
+      const float4v u = f.U - sum(xs[slot]);
+      float4v Y = sum(ys[slot]);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) Y = __builtin_amdgcn_mfma_f32_16x16x4f32(f.B[r], u[r], Y, 0, 0, 0);
+      // rows past the feed's end are past the buffer's, and are not stored
+      const int rows = min(len - c * DC_C, DC_C);
+      const auto out = __builtin_amdgcn_make_buffer_rsrc(
+          p.o + (size_t)(q0 + min(c, nc - 1) * DC_C) * ldo + (size_t)h * Dv + e0, 0, rows > 0 ? ((rows - 1) * ldo + min(16, Dv - e0)) * 4 : 0,
+          0x00020000);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(Y[r]), out, ro[r], 0, 0);
+      fetch(f, c + 8);
+    };
+    Set f0, f1, f2, f3;
+    fetch(f0, turn);
+    fetch(f1, turn + 2);
+    fetch(f2, turn + 4);
+    fetch(f3, turn + 6);
+    for (int c = turn; c < nc; c += 8) {
+      chunk(f0, c);
+      chunk(f1, c + 2);
+      chunk(f2, c + 4);
+      chunk(f3, c + 6);
+    }
+    pass(nc + 1);
+  }
 }
 
 extern "C" long loqa_delta_chunks_ws(int H, int D, int Dv, int B, int T) {
@@ -307,7 +395,7 @@ extern "C" int loqa_delta_chunks(const void* act, long ld, int H, int D, int Dv,
       hipLaunchKernelGGL((delta_local_kernel<NT, true>), gl, dim3(256), 0, st, p);               \
     else                                                                                         \
       hipLaunchKernelGGL((delta_local_kernel<NT, false>), gl, dim3(256), 0, st, p);              \
-    hipLaunchKernelGGL(delta_pass_kernel<NT>, gp, dim3(256), 0, st, p);                          \
+    hipLaunchKernelGGL(delta_pass_kernel<NT>, gp, dim3(384), 0, st, p);                          \
   } while (0)
   if (D <= 64) GO(1); else if (D <= 128) GO(2); else GO(4);
 #undef GO
