@@ -30,6 +30,17 @@ __device__ __forceinline__ void gp_load_lds(const bf16_t* base, unsigned bytes, 
       (__attribute__((address_space(3))) void*)dst, 16, off, soff, 0, 0);
 }
 
+// Worker `id` of `n` waves touches its share of [base, base + bytes), kilobyte by kilobyte, so
+// that the lines are in the Infinity Cache when a later launch asks for them: loads into a
+// kilobyte of LDS that nobody reads, as many in flight as the counter allows.
+__device__ __forceinline__ void gp_touch(const void* base, long long bytes, unsigned char* dst, int id, int n, int lane) {
+  const int pieces = (int)(bytes >> 10);
+  for (int k = id; k < pieces; k += n) {
+    gp_load_lds(reinterpret_cast<const bf16_t*>(base), (unsigned)bytes, dst, lane * 16, (unsigned)k << 10);
+    gp_wait_vm<60>();
+  }
+}
+
 // workgroups per CU by LDS
 template <int FN, int FM, int NA, int NB> constexpr int gp_per_cu() {
   return 160 * 1024 / ((NA * FN + NB * FM) * 32 * 128);

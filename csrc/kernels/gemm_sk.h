@@ -17,6 +17,8 @@ struct GemmSkParams {
   float* ws;                      // S > 1: [tiles][S][BM * BN] f32 partials
   int* counters;                  // S > 1: [tiles] ints, zero on entry (left zero)
   int layout;
+  int ahead_wgs;                  // workgroups behind the tiles' that only touch what follows (pipelined tiles)
+  const void* ahead[2]; long long ahead_bytes[2];   // weights of later launches, null or empty: none
 };
 
 // s_waitcnt vmcnt(N) with expcnt / lgkmcnt at their maxima (gfx9 encoding:

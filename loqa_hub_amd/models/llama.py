@@ -437,12 +437,12 @@ class LlamaModel:
                 # TP: the previous down partials (all-reduced) join the residual here
                 h = (ops.rmsnorm(residual, L["attn_norm"], cfg.norm_eps) if dn is None else
                      ops.rmsnorm(dn, L["attn_norm"], cfg.norm_eps, residual=residual))
-            qkv = ops.proj(h, L["wqkv"])
+            qkv = ops.proj(h, L["wqkv"], ahead=(L["wo"],))
             ops.rope_kv_append(qkv, meta.positions, w.cos_sin, k_cache[li], v_cache[li], meta.slots,
                                H, Hkv, D)
             attn = self._prompt_attention(meta, qkv, k_cache[li], v_cache[li], attn_ws)
             if tp.world == 1:
-                ops.proj(attn, L["wo"], epi="resid", residual=residual)
+                ops.proj(attn, L["wo"], epi="resid", residual=residual, ahead=(L["w_gate_up"],))
                 hn = ops.rmsnorm(residual, L["mlp_norm"], cfg.norm_eps)
             else:
                 # row-parallel o: this rank's partial on the hand-written GEMM,
@@ -451,9 +451,10 @@ class LlamaModel:
                 o = ops.proj(attn, L["wo"])
                 tp.all_reduce_(o)
                 hn = ops.rmsnorm(o, L["mlp_norm"], cfg.norm_eps, residual=residual)
-            a = ops.proj(hn, L["w_gate_up"], epi="swiglu")
+            a = ops.proj(hn, L["w_gate_up"], epi="swiglu", ahead=(L["w_down"],))
             if tp.world == 1:
-                ops.proj(a, L["w_down"], epi="resid", residual=residual)
+                nxt = w.layers[li + 1]["wqkv"] if li + 1 < len(w.layers) else None
+                ops.proj(a, L["w_down"], epi="resid", residual=residual, ahead=(nxt,) if nxt is not None else ())
             else:
                 dn = ops.proj(a, L["w_down"])
                 tp.all_reduce_(dn)

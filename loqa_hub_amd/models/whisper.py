@@ -266,14 +266,16 @@ class WhisperModel:
         d, H, D = cfg.d_model, cfg.n_heads, cfg.head_dim
         residual = x.contiguous()
         for i, L in enumerate(w.enc):
+            nxt = w.enc[i + 1] if i + 1 < len(w.enc) else None
             h = ops.layernorm(residual, L["ln1_w"], L["ln1_b"], 1e-5)
-            qkv = ops.proj(h, L["wqkv"], bias=w.enc_qkv_bf[i])
+            qkv = ops.proj(h, L["wqkv"], bias=w.enc_qkv_bf[i], ahead=(L["fc1"],))
             a = ops.attention(qkv, qkv[:, d:], qkv[:, 2 * d:], cu, n_heads=H, n_kv=H, head_dim=D,
                               causal=False, max_q=T, cu_k=cu)
             ops.proj(a, L["wo"], epi="resid", residual=residual, bias=w.enc_o_bf[i])
             h = ops.layernorm(residual, L["ln2_w"], L["ln2_b"], 1e-5)
-            m = ops.proj(h, L["fc1"], bias=w.enc_fc1_bf[i], act="gelu")
-            ops.proj(m, L["fc2"], epi="resid", residual=residual, bias=w.enc_fc2_bf[i])
+            m = ops.proj(h, L["fc1"], bias=w.enc_fc1_bf[i], act="gelu", ahead=(L["fc2"],))
+            ops.proj(m, L["fc2"], epi="resid", residual=residual, bias=w.enc_fc2_bf[i],
+                     ahead=(nxt["wqkv"], nxt["wo"]) if nxt else ())
         return ops.layernorm(residual, w.enc_ln_w, w.enc_ln_b, 1e-5)
 
     def cross_kv(self, enc: torch.Tensor) -> list[torch.Tensor]:

@@ -1754,6 +1754,36 @@ def _sk_workspace(dev: torch.device, stream: int, floats: int, tiles: int):
     return ws
 
 
+# What a launch touches for later ones (:func:`_ahead`): by how many workgroups (under 8 the launch
+# gets a tail, above 32 they take the L2 from the tiles), how much one of them brings in and how
+# much the memory moves beside the launch's own weights, both per microsecond of SK_LAYOUTS' time.
+# The last is the rule that matters: 320 rows x 28672 x 4096, bound by its 235 MB, took 78 us and
+# with the next 117 MB 95. Weights under 4 MB arrive within a microsecond (Whisper base: no gain).
+AHEAD_WGS = (8, 32)
+AHEAD_WG_BYTES_PER_US = 100_000
+AHEAD_BYTES_PER_US = 3_000_000
+AHEAD_MIN_BYTES = 4 << 20
+
+
+def _ahead(p, ahead: tuple, tiles: int) -> None:
+    """Workgroups behind the ``tiles`` of a launch, on compute units that have none, touch those of
+    the weights ``ahead`` that fit into the time that the launch takes. A layer's weights are cold
+    when their launch starts: 1500 x 1280 x 5120 in 128 x 64 tiles took 0.42 us a K step from HBM and
+    0.30 from the Infinity Cache, 1500 x 5120 x 1280 20.4 and 16.4 us before its epilogue, while the
+    240 tiles of either leave 16 compute units and most of the memory's bandwidth idle."""
+    wgs = min(SK_CUS - tiles, AHEAD_WGS[1])
+    if wgs < AHEAD_WGS[0] or max(w.numel() for w in ahead) * 2 < AHEAD_MIN_BYTES:
+        return
+    step, around = SK_LAYOUTS[p.layout][2:]
+    us = p.K // 64 / p.S * step + around
+    left = int(min(us * wgs * AHEAD_WG_BYTES_PER_US, us * AHEAD_BYTES_PER_US - 2.0 * p.N * p.K))
+    for i, w in enumerate(ahead[:2]):
+        n = w.numel() * w.element_size()
+        if n <= min(left, 0x7fffffff) and w.is_contiguous():
+            p.ahead_wgs, p.ahead[i], p.ahead_bytes[i] = wgs, w.data_ptr(), n
+            left -= n
+
+
 def _sk_ref(x: torch.Tensor, w: torch.Tensor, epi: str, bias, residual, act: str | None = None):
     y = x.float() @ w.float().t()
     if epi == "swiglu":
@@ -1774,7 +1804,7 @@ def _sk_ref(x: torch.Tensor, w: torch.Tensor, epi: str, bias, residual, act: str
 def gemm_sk(x: torch.Tensor, w: torch.Tensor, *, epi: str = "bf16", bias: torch.Tensor | None = None,
             act: str | None = None, residual: torch.Tensor | None = None,
             out: torch.Tensor | None = None, layout: int | None = None,
-            splits: int | None = None) -> torch.Tensor:
+            splits: int | None = None, ahead: tuple = ()) -> torch.Tensor:
     """Y = X W^T on the split-K tiled GEMM (``csrc/kernels/gemm_sk.hip``); the
     S K-chunks of a tile are summed in-launch by the tile's last workgroup.
 
@@ -1782,7 +1812,8 @@ def gemm_sk(x: torch.Tensor, w: torch.Tensor, *, epi: str = "bf16", bias: torch.
     ``epi``: "bf16" -> [M, N] (+ f32 ``bias``, ``act`` "gelu"); "swiglu" -> silu(gate) * up
     [M, N / 2] (gate rows [0, N/2), up rows [N/2, N)); "resid" -> ``residual``
     [M, N] += X W^T (+ ``bias``) in place (one bf16 rounding), returned. ``layout``: a number of
-    SK_LAYOUTS or SK_RENAMED (None: the plan's)."""
+    SK_LAYOUTS or SK_RENAMED (None: the plan's). ``ahead``: up to two weights that later launches
+    will read, touched meanwhile by workgroups on compute units that have no tile (:func:`_ahead`)."""
     N, K = w.shape
     M = x.shape[0]
     assert x.shape[1] == K, (x.shape, w.shape)
@@ -1835,6 +1866,8 @@ def gemm_sk(x: torch.Tensor, w: torch.Tensor, *, epi: str = "bf16", bias: torch.
         ws, cnt = _sk_workspace(x.device, st, tiles * splits * bm * bn, tiles)
         p.ws, p.counters = ptr(ws), ptr(cnt)
     p.layout = layout
+    if ahead and layout >= SK_PIPE:
+        _ahead(p, ahead, -(-M // bm) * (N // bn) * splits)
     check(kernels().loqa_gemm_sk(ctypes.byref(p), st), "gemm_sk")
     return y
 
@@ -1908,7 +1941,8 @@ def gemm_ws(x: torch.Tensor, w: torch.Tensor, *, epi: str = "bf16", bias: torch.
 # ---------------------------------------------------------------------------
 # Projections of prompt passes (prefill, Whisper encoder)
 def proj(x: torch.Tensor, w: torch.Tensor, *, epi: str = "bf16", bias: torch.Tensor | None = None,
-         act: str | None = None, residual: torch.Tensor | None = None) -> torch.Tensor:
+         act: str | None = None, residual: torch.Tensor | None = None,
+         ahead: tuple = ()) -> torch.Tensor:
     """A prompt-pass projection: :func:`gemm_sk` with the layout and K chunks its plan gives
     for the shape."""
-    return gemm_sk(x, w, epi=epi, bias=bias, act=act, residual=residual)
+    return gemm_sk(x, w, epi=epi, bias=bias, act=act, residual=residual, ahead=ahead)

@@ -1,0 +1,48 @@
+"""Weights touched ahead by a projection's launch (ops._ahead, gemm_pipe.hip): when, and that the
+product does not notice."""
+import pytest
+import torch
+
+from loqa_hub_amd import ops
+from loqa_hub_amd.ops import _lib
+
+
+def _params(N, K, layout=15, S=1):
+    p = _lib.GemmSkParams()
+    p.N, p.K, p.S, p.layout = N, K, S, layout
+    return p
+
+
+def test_what_is_touched():
+    big, small = torch.empty(5120, 1280, dtype=torch.bfloat16), torch.empty(512, 2048, dtype=torch.bfloat16)
+
+    def touched(p, ahead, tiles):
+        ops._ahead(p, ahead, tiles)
+        return p.ahead_wgs, [int(n) for n in p.ahead_bytes]
+    assert touched(_params(5120, 1280), (big,), 240) == (16, [big.numel() * 2, 0])
+    assert touched(_params(5120, 1280), (big, small), 240) == (16, [big.numel() * 2, small.numel() * 2])
+    assert touched(_params(5120, 1280), (big,), 249) == (0, [0, 0])         # no compute units left
+    assert touched(_params(5120, 1280), (big,), 720) == (0, [0, 0])         # several rounds of tiles
+    assert touched(_params(512, 512), (small,), 96) == (0, [0, 0])          # small weights come by themselves
+    assert touched(_params(28672, 4096, 13), (torch.empty(1, dtype=torch.bfloat16).expand(4096, 14336),), 224) == (0, [0, 0])
+    assert touched(_params(5120, 1280), (big.t(),), 240) == (0, [0, 0])     # not one run of memory
+    # a launch that its own weights keep the memory busy for
+    assert touched(_params(28672, 4096, 13), (torch.empty(4096, 4096, dtype=torch.bfloat16),), 224) == (0, [0, 0])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", [k for k in sorted(ops.SK_LAYOUTS) if k >= ops.SK_PIPE])
+def test_product_is_the_same(layout):
+    g = torch.Generator().manual_seed(layout)
+    x = torch.randn(300, 1024, generator=g).bfloat16().cuda()
+    w = (torch.randn(768, 1024, generator=g) / 32).bfloat16().cuda()
+    later = torch.randn(2_200_001, generator=g).bfloat16().cuda()[:2_200_000 + layout % 2]   # off whole kilobytes
+    for splits in (1, 2) if layout != ops.SK_WHOLE else (1,):
+        for kw in ({}, {"epi": "swiglu"}, {"act": "gelu"}):
+            if kw.get("epi") == "swiglu" and 768 % (2 * ops.SK_LAYOUTS[layout][0]):
+                continue
+            want = ops.gemm_sk(x, w, layout=layout, splits=splits, **kw)
+            keep = later.clone()
+            for ahead in ((later,), (later, w), (w[:8], later[:2_100_000])):
+                assert torch.equal(ops.gemm_sk(x, w, layout=layout, splits=splits, ahead=ahead, **kw), want)
+            assert torch.equal(later, keep)
