@@ -31,9 +31,12 @@ __device__ __forceinline__ bf16_t f2bf(float f) {
   return *reinterpret_cast<bf16_t*>(&b);
 }
 
-// Pack two floats into one dword of two bf16 (lo in the low half).
+// Pack two floats into one dword of two bf16 (lo in the low half): one v_cvt_pk_bf16_f32, where
+// two single conversions took four instructions.
 __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
-  return (uint32_t)f2bf(lo) | ((uint32_t)f2bf(hi) << 16);
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{lo, hi}), bf16x2));
 }
 
 __device__ __forceinline__ void unpack8(const uint4& v, float* f) {

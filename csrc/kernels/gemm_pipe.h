@@ -4,6 +4,8 @@
 #pragma once
 #include "common.h"
 
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+
 #define GP_BK 64                       // K entries of a stage: 128-byte LDS rows
 
 // s_waitcnt vmcnt(N), the other counters at their maxima (vmcnt[3:0] in bits 3:0,
@@ -138,25 +140,23 @@ __device__ __forceinline__ void gp_loop(float4v (&acc)[FN][FM], const unsigned c
 // four neighbouring features of one row per lane, so storing them directly makes every
 // 8-byte piece of an instruction a line of its own (9000 x 3840 x 1280: 26 of 96 us went
 // into the stores, 38 with a residual's loads). Instead the finished bf16 pieces go to LDS
-// and leave as whole rows, 16 bytes a lane; with ADD the old rows come in the same way
-// and value(i, j, o) finds them in o. FO: 16-wide feature blocks of the output; rows, cols:
+// and leave as whole rows, 16 bytes a lane; with ADD the old rows are there already
+// (GpRows) and value(i, j, o) finds them in o. FO: 16-wide feature blocks of the output; rows, cols:
 // what of the wave's 16 FM x 16 FO corner exists (cols a multiple of 8).
-template <int FO, int FM, bool ADD, typename Value>
-__device__ __forceinline__ void gp_store(unsigned char* my, bf16_t* y, long ldy, int rows, int cols, int lane,
-                                         Value&& value) {
-  constexpr int LD = FO * 32 + 16;                          // bytes of a row in LDS
-  constexpr int CPR = FO * 2;                               // 16-byte chunks of a row
-  constexpr int CH = 16 * FM * CPR / 64;                    // chunks per lane
+template <int FO, int FM> struct GpRows {                  // a wave's corner as 16-byte chunks of rows
+  static constexpr int LD = FO * 32 + 16;                   // bytes of a row in LDS
+  static constexpr int CPR = FO * 2;                        // chunks of a row
+  static constexpr int CH = 16 * FM * CPR / 64;             // chunks per lane
   static_assert(CH * 64 == 16 * FM * CPR, "chunks must split evenly over the lanes");
-  typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-  const int fr = lane & 15, fq = lane >> 4;
-  if constexpr (ADD) {
-    u32x4 v[CH];
+  u32x4 v[CH];
+  __device__ __forceinline__ void load(const bf16_t* y, long ldy, int rows, int cols, int lane) {
 #pragma unroll
     for (int k = 0; k < CH; ++k) {
       const int id = lane + 64 * k, r = min(id / CPR, rows - 1), c = id % CPR;
       if (rows > 0 && c * 8 < cols) v[k] = *reinterpret_cast<const u32x4*>(y + (size_t)r * ldy + c * 8);
     }
+  }
+  __device__ __forceinline__ void to_lds(unsigned char* my, int lane) const {
 #pragma unroll
     for (int k = 0; k < CH; ++k) {
       const int id = lane + 64 * k;
@@ -164,6 +164,14 @@ __device__ __forceinline__ void gp_store(unsigned char* my, bf16_t* y, long ldy,
     }
     __builtin_amdgcn_wave_barrier();
   }
+};
+
+template <int FO, int FM, bool ADD, typename Value>
+__device__ __forceinline__ void gp_store(unsigned char* my, bf16_t* y, long ldy, int rows, int cols, int lane,
+                                         Value&& value) {
+  using R = GpRows<FO, FM>;
+  constexpr int LD = R::LD, CPR = R::CPR, CH = R::CH;
+  const int fr = lane & 15, fq = lane >> 4;
 #pragma unroll
   for (int j = 0; j < FM; ++j) {
     unsigned char* row = my + (16 * j + fr) * LD + fq * 8;

@@ -1,0 +1,5 @@
+// The pipelined tile GEMM (gemm_pipe.hip) with workgroups behind the tiles' that touch the weights
+// of later launches.
+#include "gemm_pipe_tile.h"
+
+int gemm_pipe_ahead(const GemmSkParams& p, int layout, hipStream_t st) { return gp_layout<true>(p, layout, st); }

@@ -5,7 +5,7 @@
 
 #define SK_BK 64
 
-enum { SK_BF16 = 0, SK_SWIGLU = 1, SK_RESID = 2 };
+enum { SK_BF16 = 0, SK_SWIGLU = 1, SK_RESID = 2, SK_GELU = 3 };   // (SK_GELU: the pipelined tiles' SK_BF16 with act 1)
 
 struct GemmSkParams {
   const void* x; long long ldx;   // [M, K] bf16 rows
@@ -29,19 +29,29 @@ __device__ __forceinline__ void sk_wait_vm() {
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
 }
 
-// GELU through erfc's rational form (Abramowitz and Stegun 7.1.26, |error| <= 1.5e-7):
-// (v + |v|) / 2 - |v| erfc(|v| / sqrt 2) / 2 has no cancellation in the negative tail, where
-// 1 + erf(z) keeps an absolute error of half an ulp of one, and a third of erff's
-// instructions - with one wave per SIMD nothing hides an epilogue's arithmetic. Its argument is the
-// f32 sum, where it was rounded to bf16 before erff: largest relative error of the bf16 result over
-// the values from -6 on, before and now: -6 to -5 1.04, 0.0072; -4 to -3 0.033, 0.0041 (rounding the
-// result alone: 0.0039); -2 to -1 0.0097, 0.0039; above 0 0.0079, 0.0039.
-__device__ __forceinline__ float sk_gelu(float v) {
-  const float a = fabsf(v), c = fminf(a, 1e4f);        // erfc is 0 there; no inf * 0
-  const float t = __builtin_amdgcn_rcpf(1.f + 0.23164188f * c);   // 0.3275911 / sqrt 2
-  const float q = t * (0.254829592f + t * (-0.284496736f + t * (1.421413741f + t * (-1.453152027f + t * 1.061405429f))));
-  const float e = __builtin_amdgcn_exp2f(c * c * -0.72134752044448170f);   // exp(-c^2 / 2)
-  return (0.5f * v + 0.5f * a) - 0.5f * c * (q * e);
+// GELU as (v + |v|) / 2 - |v| Phi(-|v|), no cancellation in the negative tail, with log2 Phi(-a) as
+// a polynomial of degree 10 fitted on [0, 6.5] (largest error 6.3e-7; it falls without end beyond):
+// one transcendental instruction, and a quarter less issue time than the rational form of erfc
+// (Abramowitz and Stegun 7.1.26) with its reciprocal - with one wave per SIMD nothing hides an
+// epilogue's arithmetic. Its argument is the f32 sum. Largest relative error of the bf16 result, erfc's
+// form and this one: -7 to -6 0.0102, 0.0039; -6 to -5 0.0074, 0.0039; -5 to -4 0.0054, 0.0039; -4 to
+// -3 0.0042, 0.0039; from -3 on 0.0039 both (rounding the result alone: 0.0039).
+// Four values at a time, so that four chains of the polynomial run side by side on one set of
+// constants.
+__device__ __forceinline__ void sk_gelu4(float* v) {
+  constexpr float C[] = {3.011999468e-07f, -4.531088052e-06f, 3.564885992e-05f, -1.246613683e-04f, -3.609243722e-04f,
+                         7.453413680e-03f, -5.284556746e-02f, -4.590584338e-01f, -1.151129246f, -9.999993443e-01f};
+  float e[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) e[r] = -8.442756716e-09f;
+#pragma unroll
+  for (int k = 0; k < 10; ++k)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) e[r] = e[r] * fabsf(v[r]) + C[k];
+  // |v| once more, held below infinity on the positive side only: -inf is inf * 0, as with erf
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    v[r] = fmaxf(v[r], 0.f) - fmaxf(-v[r], fminf(v[r], 1e30f)) * __builtin_amdgcn_exp2f(e[r]);
 }
 
 __device__ __forceinline__ float sk_swiglu(float g, float u) {   // silu(g) u
@@ -166,10 +176,7 @@ __device__ __forceinline__ void sk_epilogue(const GemmSkParams& p, float4v (&acc
         const int n = nw + 16 * i + 4 * fq;
         float o[4] = {acc[i][j][0] + bv[i].x, acc[i][j][1] + bv[i].y, acc[i][j][2] + bv[i].z,
                       acc[i][j][3] + bv[i].w};
-        if (p.act == 1) {
-#pragma unroll
-          for (int r = 0; r < 4; ++r) o[r] = sk_gelu(o[r]);
-        }
+        if (p.act == 1) sk_gelu4(o);
         *reinterpret_cast<uint2*>(Y + (size_t)m * p.ldy + n) =
             make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
       }
