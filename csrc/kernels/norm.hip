@@ -1,10 +1,11 @@
 // Fused normalisation kernels (SURVEY §2.4 K4 layernorm, K10 rmsnorm).
 //
-// One 256-thread workgroup per row; the row stays in registers between the
-// statistics pass and the scale pass, so HBM traffic is exactly
+// The row stays in registers between the statistics pass and the scale pass, so HBM traffic is
+// exactly
 //   read x (+ read residual, write residual) + write y.
-// Rows are loaded as 16-byte vectors (8 bf16 per lane, guide G13). Supports
-// d % 8 == 0 and d <= 256 * 8 * MAXV.
+// Rows are loaded as 16-byte vectors (8 bf16 per lane, guide G13). A row is a wave's
+// (norm_rows_kernel) or, where it is long and there are few, a 256-thread workgroup's (up to d =
+// 256 * 8 * MAXV). d % 8 == 0.
 #include "common.h"
 
 #define NORM_THREADS 256
@@ -141,10 +142,126 @@ __global__ __launch_bounds__(NORM_THREADS) void layernorm_kernel(
 
 // row_idx (int64, may be null) selects the source rows; it is not combined with
 // residual (the wrapper rejects that).
+// The sum over a wave, in every lane; exchanges in the VALU as far as they go, where a shuffle
+// takes a trip through LDS.
+template <int CTRL> __device__ __forceinline__ float dpp_add(float v) {
+  return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
+}
+__device__ __forceinline__ float row_sum(float v) {
+  v = dpp_add<0xB1>(v);     // lane ^ 1
+  v = dpp_add<0x4E>(v);     // lane ^ 2
+  v = dpp_add<0x141>(v);    // the other half of 8
+  v = dpp_add<0x140>(v);    // the other half of 16
+  v += __shfl_xor(v, 16, 64);
+  return v + __shfl_xor(v, 32, 64);
+}
+
+// Layer norm (LN) or rms norm, a wave per row, VEC 16-byte pieces of it a lane (d <= 512 VEC), no
+// barrier. With a workgroup per row two barriers and LDS sums a row stood between its loads and
+// its stores, and 96 of 256 threads had nothing at 1280 columns; us a layer norm, before and now:
+// 96 x 1280 3.2, 2.7; 1500 x 512 5.1, 2.5; 1500 x 1280 6.1, 3.9; 9000 x 1280 23.2, 11.5 (46 MB).
+// Pieces past the row's end are loaded from its last one and not used: a load behind a condition,
+// with zeros as the alternative, becomes one through a generic pointer.
+template <int VEC, bool LN>
+__global__ __launch_bounds__(NORM_THREADS) void norm_rows_kernel(
+    const bf16_t* __restrict__ x, bf16_t* __restrict__ residual, const bf16_t* __restrict__ w,
+    const bf16_t* __restrict__ b, bf16_t* __restrict__ y, int rows, int d, float eps,
+    const int64_t* __restrict__ row_idx) {
+  const int lane = threadIdx.x & 63, nvec = d >> 3;
+  const int row = blockIdx.x * (NORM_THREADS / 64) + (threadIdx.x >> 6);
+  if (row >= rows) return;
+  const int src = row_idx ? (int)row_idx[row] : row;
+  const uint4* xr = reinterpret_cast<const uint4*>(x + (size_t)src * d);
+  uint4* rr = residual ? reinterpret_cast<uint4*>(residual + (size_t)row * d) : nullptr;
+  uint4 xv[VEC], wv[VEC], bv[VEC];
+#pragma unroll
+  for (int i = 0; i < VEC; ++i) xv[i] = xr[min(lane + 64 * i, nvec - 1)];
+#pragma unroll
+  for (int i = 0; i < VEC; ++i) {
+    wv[i] = reinterpret_cast<const uint4*>(w)[min(lane + 64 * i, nvec - 1)];
+    if (LN) bv[i] = reinterpret_cast<const uint4*>(b)[min(lane + 64 * i, nvec - 1)];
+  }
+  if (rr) {
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) {
+      float f[8], r[8];
+      unpack8(xv[i], f);
+      unpack8(rr[min(lane + 64 * i, nvec - 1)], r);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) f[j] += r[j];
+      xv[i] = pack8(f);
+    }
+#pragma unroll
+    for (int i = 0; i < VEC; ++i)
+      if (lane + 64 * i < nvec) rr[lane + 64 * i] = xv[i];
+  }
+  float mean = 0.f, q = 0.f;
+  if (LN) {
+#pragma unroll
+    for (int i = 0; i < VEC; ++i)
+      if (lane + 64 * i < nvec) {
+        float f[8];
+        unpack8(xv[i], f);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) mean += f[j];
+      }
+    mean = row_sum(mean) / (float)d;
+  }
+#pragma unroll
+  for (int i = 0; i < VEC; ++i)
+    if (lane + 64 * i < nvec) {
+      float f[8];
+      unpack8(xv[i], f);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float t = LN ? f[j] - mean : f[j];
+        q += t * t;
+      }
+    }
+  const float inv = rsqrtf(row_sum(q) / (float)d + eps);
+  uint4* yr = reinterpret_cast<uint4*>(y + (size_t)row * d);
+#pragma unroll
+  for (int i = 0; i < VEC; ++i)
+    if (lane + 64 * i < nvec) {
+      float f[8], wf[8], bf[8];
+      unpack8(xv[i], f);
+      unpack8(wv[i], wf);
+      if (LN) unpack8(bv[i], bf);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) f[j] = LN ? (f[j] - mean) * inv * wf[j] + bf[j] : f[j] * inv * wf[j];
+      yr[lane + 64 * i] = pack8(f);
+    }
+}
+
+// A wave per row, or a workgroup? The wave's chain of pieces is longer, the workgroup has two
+// barriers (workgroup, wave, us; rms norm but where said): 8 rows x 2048 2.6, 2.6, x 4096 2.9, 3.3;
+// 320 x 3072 3.3, 3.1, x 4096 3.3, 3.6; layer norm 1500 x 4096 9.6, 7.9; 2048 x 4096 8.4, 8.0. A
+// residual's rows come and go on the same chain: 96 x 512 2.7, 2.2, x 1280 2.8, 3.0; 1500 x 2048 6.5,
+// 6.6; 2048 x 1280 6.1, 5.8, x 4096 16.3, 15.4.
+static bool wave_per_row(int rows, int d, bool residual) {
+  if (d <= 0 || d > 4096) return false;
+  return residual ? d <= 1024 || rows >= 2048 : d <= 3072 || rows >= 1024;
+}
+
+template <bool LN>
+static int norm_rows(const void* x, void* residual, const void* w, const void* b, void* y, int rows, int d, float eps,
+                     const int64_t* row_idx, hipStream_t s) {
+#define GO(VEC)                                                                                                     \
+  case VEC:                                                                                                         \
+    hipLaunchKernelGGL((norm_rows_kernel<VEC, LN>), dim3((rows + NORM_THREADS / 64 - 1) / (NORM_THREADS / 64)),     \
+                       dim3(NORM_THREADS), 0, s, (const bf16_t*)x, (bf16_t*)residual, (const bf16_t*)w,             \
+                       (const bf16_t*)b, (bf16_t*)y, rows, d, eps, row_idx);                                        \
+    break
+  switch ((d + 511) / 512) { GO(1); GO(2); GO(3); GO(4); GO(5); GO(6); GO(7); GO(8); }
+#undef GO
+  return (int)hipGetLastError();
+}
+
 extern "C" int loqa_rmsnorm(const void* x, void* residual, const void* w, void* y,
                             int rows, int d, float eps, const int64_t* row_idx, hipStream_t s) {
   if (d % 8 != 0 || d > NORM_THREADS * 8 * MAXV || rows <= 0) return (int)hipErrorInvalidValue;
   if (row_idx && residual) return (int)hipErrorInvalidValue;
+  if (wave_per_row(rows, d, residual)) return norm_rows<false>(x, residual, w, nullptr, y, rows, d, eps, row_idx, s);
   hipLaunchKernelGGL(rmsnorm_kernel, dim3(rows), dim3(NORM_THREADS), 0, s,
                      (const bf16_t*)x, (bf16_t*)residual, (const bf16_t*)w, (bf16_t*)y, d, eps,
                      row_idx);
@@ -156,6 +273,7 @@ extern "C" int loqa_layernorm(const void* x, void* residual, const void* w, cons
                               hipStream_t s) {
   if (d % 8 != 0 || d > NORM_THREADS * 8 * MAXV || rows <= 0) return (int)hipErrorInvalidValue;
   if (row_idx && residual) return (int)hipErrorInvalidValue;
+  if (wave_per_row(rows, d, residual)) return norm_rows<true>(x, residual, w, b, y, rows, d, eps, row_idx, s);
   hipLaunchKernelGGL(layernorm_kernel, dim3(rows), dim3(NORM_THREADS), 0, s,
                      (const bf16_t*)x, (bf16_t*)residual, (const bf16_t*)w, (const bf16_t*)b,
                      (bf16_t*)y, d, eps, row_idx);
