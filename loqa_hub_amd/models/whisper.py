@@ -208,9 +208,8 @@ class WhisperModel:
             # taps from time-major rows (no column matrix), bias + GELU (+ the
             # sinusoidal positions for conv2) in the epilogue
             mel_t = ops.log_mel_rows(audio, self.mel, w.mel_cols)     # [B * 3000, M, padded] bf16
-            x1 = ops.gemm_tile(mel_t, w.conv1_wt, bias=w.conv1_bf, act="gelu", conv=(B, 1), layout=0)
-            x = ops.gemm_tile(x1, w.conv2_wt, bias=w.conv2_bf, act="gelu", pos=w.pos_enc,
-                              conv=(B, 2), layout=0)
+            x1 = ops.conv_k3_gelu(mel_t, w.conv1_wt, w.conv1_bf, B, 1)
+            x = ops.conv_k3_gelu(x1, w.conv2_wt, w.conv2_bf, B, 2, pos=w.pos_enc)
         else:
             mel = ops.log_mel(audio, self.mel)  # [B, M, 3000] bf16
             cols = ops.im2col_k3(mel, (M * frames, frames, 1), B, M, frames, 1)

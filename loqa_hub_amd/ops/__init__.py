@@ -1939,6 +1939,42 @@ def gemm_ws(x: torch.Tensor, w: torch.Tensor, *, epi: str = "bf16", bias: torch.
 
 
 # ---------------------------------------------------------------------------
+# Conv stem of the Whisper encoder (csrc/kernels/conv_pipe.hip)
+CONV_LAYOUTS = (15, 19, 20)
+
+
+def conv_k3_gelu(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor, B: int, stride: int,
+                 pos: torch.Tensor | None = None) -> torch.Tensor:
+    """GELU(conv1d(x)) (+ ``pos`` rows m % len(pos)), k = 3, padding 1: x time-major [B * T_in, Cin]
+    bf16, w a :func:`conv_k3_weight` [N, 3 * Cin], f32 ``bias`` -> [B * T_out, N] bf16. On the
+    pipelined tiles; feature or channel counts they do not take go to :func:`gemm_tile`."""
+    N, cin = w.shape[0], x.shape[1]
+    if not _gpu(x) or N % 128 or cin % 64 or x.stride(1) != 1 or x.stride(0) % 8 or x.stride(0) >= 1 << 21 or x.data_ptr() % 16:
+        return gemm_tile(x, w, bias=bias, act="gelu", pos=pos, conv=(B, stride), layout=0)
+    if x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or not w.is_contiguous() or w.data_ptr() % 16:
+        raise TypeError("conv_k3_gelu needs contiguous bf16 weights and bf16 rows")
+    assert w.shape[1] == 3 * cin and x.shape[0] % B == 0
+    assert bias.dtype == torch.float32 and bias.is_contiguous() and bias.numel() == N
+    p = _lib.ConvPipeParams()
+    p.tin = x.shape[0] // B
+    p.tout = (p.tin - 1) // stride + 1
+    p.x, p.ldx, p.w, p.bias = ptr(x), x.stride(0), ptr(w), ptr(bias)
+    p.M, p.N, p.cin, p.stride = B * p.tout, N, cin, stride
+    if pos is not None:
+        assert pos.dtype == torch.bfloat16 and pos.is_contiguous() and pos.shape[1] == N and pos.data_ptr() % 16 == 0
+        p.pos, p.pos_rows = ptr(pos), pos.shape[0]
+    y = torch.empty(p.M, N, dtype=torch.bfloat16, device=x.device)
+    p.y, p.ldy = ptr(y), N
+
+    def us(layout):      # whole tiles by SK_LAYOUTS, as the projections' plan
+        bn, bm, step, around = SK_LAYOUTS[layout]
+        return -(-(-(-p.M // bm) * (N // bn)) // SK_CUS) * (3 * cin // 64 * step + around) if N % bn == 0 else float("inf")
+    p.layout = min(CONV_LAYOUTS, key=us)
+    check(kernels().loqa_conv_pipe(ctypes.byref(p), stream_ptr(x)), "conv_pipe")
+    return y
+
+
+# ---------------------------------------------------------------------------
 # Projections of prompt passes (prefill, Whisper encoder)
 def proj(x: torch.Tensor, w: torch.Tensor, *, epi: str = "bf16", bias: torch.Tensor | None = None,
          act: str | None = None, residual: torch.Tensor | None = None,

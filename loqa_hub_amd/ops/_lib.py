@@ -77,6 +77,16 @@ class GemmSkParams(ctypes.Structure):
     ]
 
 
+class ConvPipeParams(ctypes.Structure):
+    """Mirror of ``ConvPipeParams`` in csrc/kernels/conv_pipe.hip."""
+    _fields_ = [
+        ("x", c_void_p), ("ldx", c_ll), ("w", c_void_p),
+        ("M", c_int), ("N", c_int), ("cin", c_int), ("tin", c_int), ("tout", c_int), ("stride", c_int),
+        ("bias", c_void_p), ("pos", c_void_p), ("pos_rows", c_int),
+        ("y", c_void_p), ("ldy", c_ll), ("layout", c_int),
+    ]
+
+
 class GemmWsParams(ctypes.Structure):
     """Mirror of ``GemmWsParams`` in csrc/kernels/gemm_ws.hip."""
     _fields_ = [
@@ -115,6 +125,7 @@ _KERNEL_SIGS = {
     "loqa_skinny_fused": [c_void_p, c_void_p],
     "loqa_gemm_tile": [c_void_p, c_void_p],
     "loqa_gemm_sk": [c_void_p, c_void_p],
+    "loqa_conv_pipe": [c_void_p, c_void_p],
     "loqa_gemm_ws": [c_void_p, c_int, c_void_p],
     "loqa_attn_decode": [c_void_p, c_ll, c_void_p, c_void_p, c_ll, c_void_p, c_void_p, c_ll,
                          c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,

@@ -1,0 +1,33 @@
+"""The encoder's conv stem on the pipelined tiles (csrc/kernels/conv_pipe.hip): windows that end
+inside tiles, both strides, odd and even lengths, rows wider than the channels."""
+import pytest
+import torch
+
+from loqa_hub_amd import ops
+
+
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+@pytest.mark.parametrize("B,tin,cin,N,stride", [(1, 300, 128, 128, 1), (3, 97, 64, 256, 2), (5, 33, 128, 384, 1), (2, 1, 64, 128, 1),
+                                                (70, 2, 64, 128, 2), (2, 3000, 128, 256, 1), (4, 1500, 512, 512, 2)])
+def test_conv(device, B, tin, cin, N, stride):
+    g = torch.Generator().manual_seed(tin + N)
+    tout = (tin - 1) // stride + 1
+    x = torch.randn(B * tin, cin + 16, generator=g).bfloat16()[:, 8:8 + cin]
+    w = (torch.randn(N, cin, 3, generator=g) * (3 * cin) ** -0.5).bfloat16()
+    bias, pos = torch.randn(N, generator=g) * 0.1, torch.randn(tout, N, generator=g).bfloat16()
+    wt = ops.conv_k3_weight(w.reshape(N, -1), cin).to(device)
+    v = torch.nn.functional.conv1d(x.double().view(B, tin, cin).transpose(1, 2), w.double(), bias.double(), stride, 1)
+    a = v.transpose(1, 2).reshape(B * tout, N)
+    v = torch.nn.functional.gelu(a)
+    wide = torch.zeros(B * tin, cin + 16, dtype=torch.bfloat16)
+    wide[:, 8:8 + cin] = x
+    for xd in (wide.to(device)[:, 8:8 + cin], x.contiguous().to(device)):
+        for p in (None, pos):
+            want = v if p is None else v + p.double().repeat(B, 1)
+            y = ops.conv_k3_gelu(xd, wt, bias.to(device), B, stride, pos=None if p is None else p.to(device)).double().cpu()
+            # bf16 has 8 significant bits: half an ulp is at most 2^-8 of the value. That of the result
+            # and, in the plain form, of GELU's
+            # argument (times GELU's largest slope, 1.13) and of its value before the positions; f32
+            # sums of 3 cin products
+            tol = 2.0 ** -8 * (want.abs() + v.abs() + 1.13 * a.abs()) * 1.01 + 1e-5
+            assert torch.all((y - want).abs() <= tol), (y - want).abs().max()
