@@ -2,10 +2,9 @@
 //
 // For passes with many query rows the folded form (attn_latent.hip) would pay
 // R + Dr multiply-adds per score and R per value entry; here the keys and
-// values are first materialised per head from the gathered latent rows (two
-// vendor GEMMs: k_un = W_uk c, v = W_uv c), and the pipelined tile loop of the other prompt
+// values are first materialised per head from the latent rows (latent_kv.hip), and the pipelined tile loop of the other prompt
 // attentions (flash_pipe.h) runs over [key, head, DK] / [key, head, DV].
-// What is its own: DK != DV (rotary part only in the keys), zero-padded head sizes (DK, DV are
+// Queries may come unrotated: a row's entries are turned as they are loaded. What is its own: DK != DV (rotary part only in the keys), zero-padded head sizes (DK, DV are
 // the next instantiated sizes), the causal bound from each row's absolute position (with a
 // sliding window the keys before it are neither gathered nor visited), a learned per-head sink
 // in the softmax denominator, and the output gate sigmoid(gate), applied before the unpadded
@@ -33,6 +32,7 @@ struct LatPrefillParams {
   const float* sink; float scale_log2;
   int H, Dv, window;
   const bf16_t* gate; long gate_ld; // [T, H * Dv] or null
+  const float* cs; int max_pos, rot0, rot_dims;   // queries to be rotated: tables, first entry and width (null: done)
   int runs, rows16;                 // gate rows can be read in runs of four, output rows written in runs of eight
 };
 
@@ -88,7 +88,22 @@ __global__ __launch_bounds__(64 * QW * KS, DK > 192 ? 1 : 2) void latent_prefill
     const bf16_t* qrow = p.q + (size_t)(q0 + min(qi, row_hi)) * p.q_st + (size_t)head * DK;
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-      const uint4 v = valid ? *reinterpret_cast<const uint4*>(qrow + 16 * s + 8 * h) : make_uint4(0, 0, 0, 0);
+      uint4 v = valid ? *reinterpret_cast<const uint4*>(qrow + 16 * s + 8 * h) : make_uint4(0, 0, 0, 0);
+      const int e = 16 * s + 8 * h - p.rot0;
+      if (p.cs && e >= 0 && e < p.rot_dims) {
+        const float* c = p.cs + (size_t)min(max(p.pos[q0 + min(qi, row_hi)], 0), p.max_pos - 1) * p.rot_dims + e;
+        float t[8], f[8];
+        ld_run<float, 4>(c, t);
+        ld_run<float, 4>(c + 4, t + 4);
+        unpack8(v, f);
+#pragma unroll
+        for (int i = 0; i < 8; i += 2) {
+          const float a = f[i], z = f[i + 1];
+          f[i] = a * t[i] - z * t[i + 1];
+          f[i + 1] = z * t[i] + a * t[i + 1];
+        }
+        v = pack8(f);
+      }
       qf[s] = *reinterpret_cast<const bf16x8*>(&v);
     }
   }
@@ -268,8 +283,11 @@ extern "C" int loqa_latent_prefill(const void* q, long q_st, const void* k, cons
                                    long o_ld, const void* cu_q, const void* cu_k, const void* ctx,
                                    const void* pos, const void* sink, float scale, int window,
                                    const void* gate, long gate_ld, int B, int H, int max_q, int DK,
-                                   int DV, int Dv, hipStream_t st) {
+                                   int DV, int Dv, const void* cs, int max_pos, int rot0, int rot_dims,
+                                   hipStream_t st) {
   if (B <= 0 || H <= 0 || max_q <= 0) return 0;
+  if (cs && (max_pos <= 0 || rot0 < 0 || rot0 % 8 || rot_dims <= 0 || rot_dims % 8 || rot0 + rot_dims > DK || ((size_t)cs & 15)))
+    return (int)hipErrorInvalidValue;
   if (Dv <= 0 || Dv > DV || o_ld < (long)H * Dv || !ctx) return (int)hipErrorInvalidValue;
   LatPrefillParams p;
   p.q = (const bf16_t*)q; p.q_st = q_st; p.k = (const bf16_t*)k; p.v = (const bf16_t*)v;
@@ -277,6 +295,7 @@ extern "C" int loqa_latent_prefill(const void* q, long q_st, const void* k, cons
   p.pos = (const int*)pos; p.ctx = (const int*)ctx; p.Dv = Dv; p.window = window;
   p.sink = (const float*)sink; p.scale_log2 = scale * 1.4426950408889634f; p.H = H;
   p.gate = (const bf16_t*)gate; p.gate_ld = gate_ld;
+  p.cs = (const float*)cs; p.max_pos = max_pos; p.rot0 = rot0; p.rot_dims = rot_dims;
   p.runs = Dv % 4 == 0 && (!gate || (gate_ld % 4 == 0 && ((size_t)gate & 7) == 0));
   p.rows16 = Dv % 8 == 0 && o_ld % 8 == 0 && ((size_t)o & 15) == 0;
   // the direct-to-LDS loads take 16-byte rows, a tile's rows within 32-bit offsets

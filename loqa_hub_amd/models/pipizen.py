@@ -59,8 +59,9 @@ def latent_prompt_layout(L: dict, m, dtype, device) -> None:
         out[:, :per] = w.view(H, per, -1)
         return out.view(H * to, -1).contiguous()
     L["wq"], L["qw"] = pad_rows(L["wq"], D + Dr, DKp), DKp
-    L["wuk_p"] = pad_rows(L["wuk"].reshape(H * D, R), D, DKp)
-    L["wuv_p"] = pad_rows(L["wuv_t"].transpose(1, 2).reshape(H * Dv, R), Dv, DVp)
+    # keys and values of all heads as one product (seqmix.latent_keys_values)
+    L["wkv_p"] = torch.cat([pad_rows(L["wuk"].reshape(H * D, R), D, DKp),
+                            pad_rows(L["wuv_t"].transpose(1, 2).reshape(H * Dv, R), Dv, DVp)])
     L["prompt_sizes"] = (DKp, DVp)
 
 
@@ -82,14 +83,11 @@ def latent_heads(L: dict, m, q: torch.Tensor, pages: torch.Tensor, meta, prompt_
         DKp, DVp = L["prompt_sizes"]
         cu_k, total_k = meta.window_k[window] if window > 0 else (meta.cu_k, meta.total_k)
         reach = min(meta.max_ctx, meta.max_q + window - 1) if window > 0 else meta.max_ctx
-        cl, kr = seqmix.latent_gather(pages, meta.block_tables, cu_k, meta.ctx_lens, total_k,
-                                      reach, R)
-        k = ops.linear(cl, L["wuk_p"]).view(-1, H, DKp)
-        seqmix.latent_kfill_(k, kr, D)
-        v = ops.linear(cl, L["wuv_p"]).view(-1, H, DVp)
-        seqmix.rope_pairs_(q, D, m.rot.dims, meta.positions, L["cos_sin"])
+        k, v = seqmix.latent_keys_values(pages, meta.block_tables, cu_k, meta.ctx_lens, total_k, reach,
+                                         L["wkv_p"], H, DKp, DVp, D)
         return seqmix.latent_prefill(q, k, v, meta.cu_q, cu_k, meta.ctx_lens, meta.positions,
-                                     L["sink"], m.scale, meta.max_q, Dv, window, gate, out)
+                                     L["sink"], m.scale, meta.max_q, Dv, window, gate, out,
+                                     (D, m.rot.dims, L["cos_sin"]))
     qa = torch.bmm(q[:, :, :D].transpose(0, 1), L["wuk"])            # [H, T, R]
     lat = seqmix.latent_attention(qa, q[:, :, D:D + Dr], pages, meta.cu_q, meta.ctx_lens,
                                   meta.block_tables, meta.positions, L["cos_sin"], L["sink"],

@@ -288,6 +288,42 @@ def latent_kfill_(k: torch.Tensor, kr: torch.Tensor, D: int) -> None:
           "latent_kfill")
 
 
+KV_LAYOUTS = {13: (256, 192, 1.075, 5.5), 20: (128, 128, 0.498, 3.6), 19: (128, 64, 0.309, 4.3)}   # as ops.SK_LAYOUTS
+
+
+def latent_keys_values(cache: torch.Tensor, block_tables: torch.Tensor, cu_k: torch.Tensor,
+                       ctx_lens: torch.Tensor, total_k: int, max_ctx: int, wkv: torch.Tensor, H: int,
+                       DK: int, DV: int, D: int) -> tuple[torch.Tensor, torch.Tensor]:
+    """Keys [total_k, H, DK] and values [total_k, H, DV] (bf16, GPU) of the rows that
+    :func:`latent_gather` would bring: ``wkv`` [H DK + H DV, R] times the latents, the rotary part at
+    the entries from ``D`` on of every head's key. One launch off the pages (``latent_kv.hip``);
+    sizes, alignments and caches that it does not take: gather, products and fill."""
+    R = wkv.shape[1]
+    Dr = cache.shape[2] - R
+    assert wkv.shape[0] == H * (DK + DV) and cache.is_contiguous() and D + Dr <= DK
+    fits = [n for n, (bn, _, _, _) in KV_LAYOUTS.items() if H * DK % bn == 0 and H * DV % bn == 0]
+    if not fits or R % 64 or Dr > 64 or Dr % 16 or D % 16 or cache.numel() >= 1 << 30 or cache.data_ptr() % 16 or \
+            wkv.data_ptr() % 16 or not wkv.is_contiguous() or not total_k:
+        cl, kr = latent_gather(cache, block_tables, cu_k, ctx_lens, total_k, max_ctx, R)
+        k = torch.nn.functional.linear(cl, wkv[:H * DK]).view(-1, H, DK)
+        latent_kfill_(k, kr, D)
+        return k, torch.nn.functional.linear(cl, wkv[H * DK:]).view(-1, H, DV)
+    assert cache.is_cuda and cache.dtype == wkv.dtype == torch.bfloat16
+    _i32c(block_tables, "block_tables"); _i32c(cu_k, "cu_k"); _i32c(ctx_lens, "ctx_lens")
+    B = block_tables.shape[0]
+    assert cu_k.numel() == B + 1 and ctx_lens.numel() == B
+    k = torch.empty(total_k, H, DK, dtype=cache.dtype, device=cache.device)
+    v = torch.empty(total_k, H, DV, dtype=cache.dtype, device=cache.device)
+
+    def us(layout):
+        bn, bm, step, around = KV_LAYOUTS[layout]
+        return -(-(-(-total_k // bm) * (H * (DK + DV) // bn)) // 256) * (R // 64 * step + around)
+    check(kernels().loqa_latent_kv(ptr(cache), cache.numel() * 2, cache.shape[1], cache.shape[2], ptr(block_tables),
+                                   block_tables.shape[1], ptr(cu_k), ptr(ctx_lens), B, total_k, ptr(wkv), R, H, DK,
+                                   DV, D, ptr(k), ptr(v), min(fits, key=us), stream_ptr(cache)), "latent_kv")
+    return k, v
+
+
 def rope_pairs_(x: torch.Tensor, off: int, dims: int, positions: torch.Tensor,
                 cos_sin: torch.Tensor) -> None:
     """Rotate in place the interleaved pairs x[t, h, off : off + dims] (bf16)."""
@@ -303,10 +339,11 @@ def rope_pairs_(x: torch.Tensor, off: int, dims: int, positions: torch.Tensor,
 def latent_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu_q: torch.Tensor,
                    cu_k: torch.Tensor, ctx_lens: torch.Tensor, positions: torch.Tensor,
                    sink: torch.Tensor | None, scale: float, max_q: int, Dv: int, window: int = 0,
-                   gate: torch.Tensor | None = None, out: torch.Tensor | None = None
-                   ) -> torch.Tensor:
+                   gate: torch.Tensor | None = None, out: torch.Tensor | None = None,
+                   rot: tuple | None = None) -> torch.Tensor:
     """Causal flash attention of a prompt pass on the matrix cores: q [T, H, DK]
-    (rotated), k [L, H, DK], v [L, H, DV] per-head keys / values of the gathered
+    (rotated, or with ``rot`` = (first entry, width, cos_sin) to be rotated as
+    :func:`rope_pairs_` does it, in the launch), k [L, H, DK], v [L, H, DV] per-head keys / values of the gathered
     contexts (``cu_k``: the last keys of each sequence's ``ctx_lens``), a query at
     absolute position p sees the keys up to p of its sequence, with ``window`` > 0
     only p - window + 1 .. p; ``sink`` [H] joins the softmax denominator; ``gate``
@@ -331,13 +368,24 @@ def latent_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu_q: torc
     if out is None:
         out = torch.empty(T, H * Dv, dtype=q.dtype, device=q.device)
     assert out.shape == (T, H * Dv) and out.stride(1) == 1 and out.dtype == q.dtype
+    cs, turn = None, (0, 0, 0)
+    if rot is not None and rot[1]:
+        off, dims, cs = rot
+        _f32c(cs, "cos_sin")
+        assert cs.shape[1] * 2 == dims and off + dims <= DK and positions.numel() >= T
+        if off % 8 or dims % 8 or cs.data_ptr() % 16:       # the launch turns runs of eight entries
+            q = q.clone()
+            rope_pairs_(q, off, dims, positions, cs)
+            cs = None
+        else:
+            turn = (cs.shape[0], off, dims)
     # the kernel's loads take 16-byte rows (tensors that torch made start on them)
     k = k if k.data_ptr() % 16 == 0 else k.clone()
     v = v if v.data_ptr() % 16 == 0 else v.clone()
     check(kernels().loqa_latent_prefill(
         ptr(q), q.stride(0), ptr(k), ptr(v), ptr(out), out.stride(0), ptr(cu_q), ptr(cu_k),
         ptr(ctx_lens), ptr(positions), ptr(sink), float(scale), int(window), ptr(gate),
-        gate.stride(0) if gate is not None else 0, B, H, int(max_q), DK, DV, Dv, stream_ptr(q)),
+        gate.stride(0) if gate is not None else 0, B, H, int(max_q), DK, DV, Dv, ptr(cs), *turn, stream_ptr(q)),
         "latent_prefill")
     return out
 
