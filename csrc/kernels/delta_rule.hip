@@ -56,7 +56,25 @@ __device__ __forceinline__ int dr_seq_of_row(const int* __restrict__ cu_q, int B
   return b;
 }
 
-__device__ __forceinline__ float dr_softplus(float z) { return z > 20.f ? z : log1pf(expf(z)); }
+// e^x to two ulp on the hardware's 2^x: the product with log2 e as a rounded value and its
+// remainder (log2 e = 1.44269502 + 1.92596e-8). Infinities and NaN as expf has them.
+__device__ __forceinline__ float dr_exp(float x) {
+  const float t = x * 1.44269502f;
+  const float e = __builtin_amdgcn_exp2f(t);
+  const float r = fmaf(x, 1.44269502f, -t) + x * 1.92596303e-8f;
+  return fabsf(t) < 200.f ? fmaf(e, r * 0.693147181f, e) : e;
+}
+// log(1 + e^z) = max(z, 0) + log(1 + e^-|z|), the latter of u = 1 + e^-|z| as it was rounded and of
+// what the rounding lost, over u. With expf and log1pf and a division for the head a decay took 126
+// instructions, 14 of the 31 us of 2048 tokens with 16 x 128 of them; 23 us now. Error of the decays
+// against 64 bits, before and now (root mean square): pre-activations -2 to 2, a to 1: 3.12e-8,
+// 3.13e-8; 2 to 20: 1.86e-7, 1.85e-7; -10 to -2: 1.82e-8 both.
+__device__ __forceinline__ float dr_softplus(float z) {
+  const float e = dr_exp(-fabsf(z)), u = 1.f + e;
+  return fmaxf(z, 0.f) + fmaf(__builtin_amdgcn_logf(u), 0.693147181f, (e - (u - 1.f)) * __builtin_amdgcn_rcpf(u));
+}
+// e^(a softplus(z)): a token's decay (expf: its last half ulp counts in a decay next to one)
+__device__ __forceinline__ float dr_decay(float a, float z) { return expf(a * dr_softplus(z)); }
 
 template <int CTRL> __device__ __forceinline__ float dr_dpp(float v) {
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
@@ -87,8 +105,9 @@ __device__ __forceinline__ void dr_gates(const TU* ub, const float* gz, int H, i
                                          const float* a_neg, const float* dt_bias, float* tok,
                                          float* g) {
   if constexpr (CHAN) {
+    const int shift = (D & (D - 1)) ? -1 : __ffs(D) - 1;
     for (int i = blockIdx.y * 64 + threadIdx.x; i < H * D; i += 64 * gridDim.y)
-      g[i] = expf(a_neg[i / D] * dr_softplus(gz[i] + dt_bias[i]));
+      g[i] = dr_decay(a_neg[shift >= 0 ? i >> shift : i / D], gz[i] + dt_bias[i]);
     if (blockIdx.y == 0)
       for (int h = threadIdx.x; h < H; h += 64) {
         tok[2 * h] = 1.f;
@@ -96,7 +115,7 @@ __device__ __forceinline__ void dr_gates(const TU* ub, const float* gz, int H, i
       }
   } else if (blockIdx.y == 0) {
     for (int h = threadIdx.x; h < H; h += 64) {
-      tok[2 * h] = expf(a_neg[h] * dr_softplus(gz[H + h] + dt_bias[h]));
+      tok[2 * h] = dr_decay(a_neg[h], gz[H + h] + dt_bias[h]);
       tok[2 * h + 1] = sigmoid_f(gz[h]);
     }
   }
