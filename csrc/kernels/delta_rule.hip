@@ -56,22 +56,24 @@ __device__ __forceinline__ int dr_seq_of_row(const int* __restrict__ cu_q, int B
   return b;
 }
 
-// e^x to two ulp on the hardware's 2^x: the product with log2 e as a rounded value and its
-// remainder (log2 e = 1.44269502 + 1.92596e-8). Infinities and NaN as expf has them.
-__device__ __forceinline__ float dr_exp(float x) {
-  const float t = x * 1.44269502f;
-  const float e = __builtin_amdgcn_exp2f(t);
-  const float r = fmaf(x, 1.44269502f, -t) + x * 1.92596303e-8f;
-  return fabsf(t) < 200.f ? fmaf(e, r * 0.693147181f, e) : e;
-}
-// log(1 + e^z) = max(z, 0) + log(1 + e^-|z|), the latter of u = 1 + e^-|z| as it was rounded and of
-// what the rounding lost, over u. With expf and log1pf and a division for the head a decay took 126
-// instructions, 14 of the 31 us of 2048 tokens with 16 x 128 of them; 23 us now. Error of the decays
-// against 64 bits, before and now (root mean square): pre-activations -2 to 2, a to 1: 3.12e-8,
-// 3.13e-8; 2 to 20: 1.86e-7, 1.85e-7; -10 to -2: 1.82e-8 both.
+// log(1 + e^z) = max(z, 0) + log(1 + e), e = e^-|z|, the latter as 2 atanh(s) of s = e / (2 + e) at
+// most 1/3: atanh(s) = s + s^3 Q(s^2), Q fitted at Chebyshev points (3.8e-10 of the value), and what
+// s lost in rounding added last. With log1pf, and a division for the head, a decay took 126
+// instructions: 14 of the 31 us of 2048 tokens with 16 x 128 of them; 24 us now. The decays' error
+// against 64 bits, root mean square, before and now: pre-activations -10 to -2, -a to 1, 1.82e-8
+// both, -a 1 to 16 2.33e-8 both; -2 to 2 3.12e-8, 3.09e-8 and 3.37e-7, 3.27e-7; 2 to 20, -a to 1,
+// 1.86e-7, 1.85e-7 (softplus by itself: the same below 0, 3.1e-8 and 3.3e-8 from 0 to 1, 2.6e-8 and
+// 2.5e-8 from 1 to 2). The hardware's logarithm of 1 + e is 1 us less, but lost a tenth more there.
 __device__ __forceinline__ float dr_softplus(float z) {
-  const float e = dr_exp(-fabsf(z)), u = 1.f + e;
-  return fmaxf(z, 0.f) + fmaf(__builtin_amdgcn_logf(u), 0.693147181f, (e - (u - 1.f)) * __builtin_amdgcn_rcpf(u));
+#pragma clang fp contract(off)  // s0 has to be the rounded product wherever it stands
+  const float e = expf(-fabsf(z)), d = 2.f + e, r = __builtin_amdgcn_rcpf(d);
+  const float s0 = e * r, rest = fmaf(-s0, e - (d - 2.f), fmaf(-s0, d, e)) * r, s = s0 + rest;
+  const float t = s * s, s2 = s + s;
+  float q = fmaf(t, 0.116184026f, 0.108519383f);
+  q = fmaf(t, q, 0.142962679f);
+  q = fmaf(t, q, 0.199998513f);
+  q = fmaf(t, q, 0.333333343f);
+  return fmaxf(z, 0.f) + (s2 + fmaf(s2 * t, q, 2.f * (s0 - s + rest)));
 }
 // e^(a softplus(z)): a token's decay (expf: its last half ulp counts in a decay next to one)
 __device__ __forceinline__ float dr_decay(float a, float z) { return expf(a * dr_softplus(z)); }
