@@ -152,7 +152,8 @@ __global__ void rope_kv_append_kernel(bf16_t* __restrict__ qkv, int stride,
 // Same operation, every load of the row issued before any store: the loop form
 // above reads, rotates and writes one 4-element group per trip, and its
 // in-place q stores keep the compiler from hoisting the next trip's loads, so
-// a thread pays one memory round trip per group (5 at Llama-3-8B's 40 heads).
+// a thread pays one memory round trip per group (5 at 40 heads of 128). For widths that are
+// no power of two, and rows off 16 bytes.
 // Here each thread holds up to RK groups (and its V piece) in registers.
 template <int RK>
 __global__ __launch_bounds__(128) void rope_kv_append_batched_kernel(
@@ -237,11 +238,90 @@ __global__ __launch_bounds__(128) void rope_kv_append_batched_kernel(
   }
 }
 
+// Widths of 16 times a power of two: a thread keeps its eight columns (and the eight half a head
+// further) for all the heads it takes, so a row's rotation is loaded once a thread, in 16-byte pieces
+// like the heads; V counts as heads without a rotation. All loads stand before the first store; past
+// the last head they read V's last one again, which nothing stores into.
+// Bound by memory from 2000 rows on (24 KB a row at 32 + 2 x 8 heads of 128: 50 MB at 2048 rows, part
+// of it still in the caches), by a launch and one trip to memory below. us, the kernel below and this
+// one, 1 / 320 / 2048 / 4096 rows: 32 + 2 x 8 of 128 5.2, 4.1 / 6.5, 4.0 / 12.2, 8.2 / 21.4, 16.3; 20 +
+// 2 x 20 of 64 without rotation 3.5, 3.1 / 4.3, 3.2 / 6.6, 4.8 / 11.3, 9.3; 32 + 2 x 32 of 128 (one
+// group a trip before) 5.8, 3.8 / 7.9, 5.4 / 17.5, 16.1 / 32.6, 30.9.
+template <int RK>
+__global__ __launch_bounds__(128) void rope_kv_append_runs_kernel(
+    bf16_t* __restrict__ qkv, int stride, const int* __restrict__ positions,
+    const float2* __restrict__ cs, bf16_t* __restrict__ kc, bf16_t* __restrict__ vc,
+    const int* __restrict__ slots, int Hq, int Hkv, int D, int blk, int shift) {
+  const int t = blockIdx.x, half = D >> 1, nh = Hq + 2 * Hkv;
+  const int c = (threadIdx.x & ((1 << shift) - 1)) * 8, h0 = threadIdx.x >> shift, step = 128 >> shift;
+  bf16_t* row = qkv + (size_t)t * stride;
+  uint4 lo[RK], hi[RK];
+#pragma unroll
+  for (int k = 0; k < RK; ++k) {
+    const bf16_t* base = row + min(h0 + k * step, nh - 1) * D + c;
+    lo[k] = *reinterpret_cast<const uint4*>(base);
+    hi[k] = *reinterpret_cast<const uint4*>(base + half);
+  }
+  float4 e[4];
+  if (cs) {
+    const float4* csr = reinterpret_cast<const float4*>(cs + (size_t)positions[t] * half + c);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) e[j] = csr[j];
+  }
+  const int slot = slots ? slots[t] : -1, page = slot / blk, o = slot - page * blk;
+#pragma unroll
+  for (int k = 0; k < RK; ++k) {
+    const int h = h0 + k * step;
+    if (cs && h < Hq + Hkv) {
+      float a[8], b[8], ra[8], rb[8];
+      unpack8(lo[k], a);
+      unpack8(hi[k], b);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float x = j & 1 ? e[j >> 1].z : e[j >> 1].x, y = j & 1 ? e[j >> 1].w : e[j >> 1].y;
+        ra[j] = a[j] * x - b[j] * y;
+        rb[j] = b[j] * x + a[j] * y;
+      }
+      lo[k] = pack8(ra);
+      hi[k] = pack8(rb);
+    }
+    bf16_t* dst = row + h * D;
+    bool put = h < Hq && cs;
+    if (h >= Hq) {
+      const int g = h < Hq + Hkv ? h - Hq : h - Hq - Hkv;
+      dst = (h < Hq + Hkv ? kc : vc) + (((size_t)page * Hkv + g) * blk + o) * D;
+      put = slot >= 0 && h < nh;
+    }
+    if (put) {
+      *reinterpret_cast<uint4*>(dst + c) = lo[k];
+      *reinterpret_cast<uint4*>(dst + c + half) = hi[k];
+    }
+  }
+}
+
 extern "C" int loqa_rope_kv_append(void* qkv, int stride, const int* positions, const void* cs,
                                    void* kc, void* vc, const int* slots, int T, int Hq, int Hkv,
                                    int D, int blk, hipStream_t s) {
   if (T <= 0) return 0;
   if (D % 8 != 0 || stride < (Hq + 2 * Hkv) * D || (cs && !positions)) return (int)hipErrorInvalidValue;
+  // In 16-byte pieces wherever rows, caches and rotation lie so and a thread's heads fit its registers:
+  // faster at every size measured (1 to 4096 rows, widths 32, 64 and 128).
+  const int pv = D / 16, rk = (Hq + 2 * Hkv) * pv / 128 + ((Hq + 2 * Hkv) * pv % 128 != 0);
+  const bool runs = D % 16 == 0 && pv <= 128 && (pv & (pv - 1)) == 0 && Hkv > 0 && rk <= 6 && stride % 8 == 0 &&
+                    (((size_t)qkv | (size_t)kc | (size_t)vc | (size_t)cs) & 15) == 0;
+#define RUNS(RK)                                                                                \
+  hipLaunchKernelGGL(rope_kv_append_runs_kernel<RK>, dim3(T), dim3(128), 0, s, (bf16_t*)qkv, stride, \
+                     positions, (const float2*)cs, (bf16_t*)kc, (bf16_t*)vc, slots, Hq, Hkv, D, blk, \
+                     __builtin_ctz(pv))
+  if (runs) {
+    if (rk == 1) RUNS(1);
+    else if (rk == 2) RUNS(2);
+    else if (rk == 3) RUNS(3);
+    else if (rk == 4) RUNS(4);
+    else RUNS(6);
+    return (int)hipGetLastError();
+  }
+#undef RUNS
   if ((Hq + Hkv) * (D / 8) <= 8 * 128 && Hkv * (D / 8) <= 128) {
     hipLaunchKernelGGL(rope_kv_append_batched_kernel<8>, dim3(T), dim3(128), 0, s, (bf16_t*)qkv,
                        stride, positions, (const float2*)cs, (bf16_t*)kc, (bf16_t*)vc, slots, Hq,
