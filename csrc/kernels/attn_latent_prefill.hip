@@ -2,20 +2,21 @@
 //
 // For passes with many query rows the folded form (attn_latent.hip) would pay
 // R + Dr multiply-adds per score and R per value entry; here the keys and
-// values are first materialised per head from the latent rows (latent_kv.hip), and the pipelined tile loop of the other prompt
-// attentions (flash_pipe.h) runs over [key, head, DK] / [key, head, DV].
-// Queries may come unrotated: a row's entries are turned as they are loaded. What is its own: DK != DV (rotary part only in the keys), zero-padded head sizes (DK, DV are
-// the next instantiated sizes), the causal bound from each row's absolute position (with a
-// sliding window the keys before it are neither gathered nor visited), a learned per-head sink
-// in the softmax denominator, and the output gate sigmoid(gate), applied before the unpadded
-// heads go to rows of any stride. Numerator and denominator are of the same rounded weights
-// (flash_pipe.h has the errors).
+// values are first materialised per head from the latent rows (latent_kv.hip), and the pipelined
+// tile loop of the other prompt attentions (flash_pipe.h) runs over [key, head, DK] / [key, head, DV].
+// Queries may come unrotated: a row's entries are turned as they are loaded. What is its own: DK != DV
+// (rotary part only in the keys), zero-padded head sizes (DK, DV are the next instantiated sizes), the
+// causal bound from each row's absolute position (with a sliding window the keys before it are neither
+// gathered nor visited), a learned per-head sink in the softmax denominator, and the output gate
+// sigmoid(gate), applied before the unpadded heads go to rows of any stride. Numerator and denominator
+// are of the same rounded weights (flash_pipe.h has the errors).
 // 2048 rows of 16 heads, 192 / 128: 99.5 us before (128 rows in four waves, tiles through
 // registers, scores, exponentials and products one after the other), 55 now; 4 x that: 365, 120;
 // 256 / 128: 111, 75. A single prompt is one round of the CUs, as long as its last rows (32
 // tiles, 16.5 on average); smaller blocks with one wave a SIMD were no faster.
 //
-// Helpers: latent_gather_kernel copies the last cu_k[b + 1] - cu_k[b] latent rows
+// Helpers, for the sizes and alignments that latent_kv.hip does not take and queries that come turned:
+// latent_gather_kernel copies the last cu_k[b + 1] - cu_k[b] latent rows
 // of each sequence from its pages into contiguous [sum L, R] / [sum L, Dr] buffers; latent_kfill_kernel
 // writes the shared rotary key part into every head's key row;
 // rope_pairs_kernel rotates the queries' rotary part in place.

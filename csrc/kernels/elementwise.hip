@@ -585,7 +585,7 @@ extern "C" int loqa_step_publish(const int* out, int n, void* res, int stride, i
 }
 
 // ---------------------------------------------------------------------------
-// Counter-based random init (seeded random-init weights, SURVEY §5.4): element
+// Counter-based random init (seeded random-init weights): element
 // (r, c) of a [rows, cols] block at (row0, col0) of a conceptual [*, ld] tensor
 // gets scale * (u0 + u1 + u2 + u3 - 2) with u_k = fmix32(4 * idx + k + s) / 2^32
 // (Irwin-Hall(4): mean 0, variance 1/3 - the caller folds sqrt(3) into scale),

@@ -1,4 +1,4 @@
-// Fused normalisation kernels (SURVEY §2.4 K4 layernorm, K10 rmsnorm).
+// Fused normalisation kernels (layer norm, rms norm).
 //
 // The row stays in registers between the statistics pass and the scale pass, so HBM traffic is
 // exactly

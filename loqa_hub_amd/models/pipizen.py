@@ -77,9 +77,9 @@ def latent_heads(L: dict, m, q: torch.Tensor, pages: torch.Tensor, meta, prompt_
     T = q.shape[0]
     q = q.view(T, H, L["qw"])
     if "prompt_sizes" in L and meta.max_q >= prompt_min_q and meta.cu_k is not None:
-        # prompt pass: per-head keys / values from the gathered latents (the
-        # whole contexts, or what the rows' windows reach), then flash attention
-        # on the matrix cores
+        # prompt pass: per-head keys / values from the latents on their pages (the
+        # whole contexts, or what the rows' windows reach) in one product, then flash
+        # attention on the matrix cores, which turns the queries as it loads them
         DKp, DVp = L["prompt_sizes"]
         cu_k, total_k = meta.window_k[window] if window > 0 else (meta.cu_k, meta.total_k)
         reach = min(meta.max_ctx, meta.max_q + window - 1) if window > 0 else meta.max_ctx

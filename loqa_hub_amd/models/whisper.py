@@ -204,8 +204,8 @@ class WhisperModel:
         frames = audio.shape[1] // 160
         tile = ENC_TILE and audio.is_cuda and d % 128 == 0
         if tile:
-            # conv1d stem on the tiled MFMA GEMM: the loader gathers the k = 3
-            # taps from time-major rows (no column matrix), bias + GELU (+ the
+            # conv1d stem on the pipelined tiles: an output row's k = 3 taps lie one behind
+            # the other in the time-major rows (no column matrix), bias + GELU (+ the
             # sinusoidal positions for conv2) in the epilogue
             mel_t = ops.log_mel_rows(audio, self.mel, w.mel_cols)     # [B * 3000, M, padded] bf16
             x1 = ops.conv_k3_gelu(mel_t, w.conv1_wt, w.conv1_bf, B, 1)

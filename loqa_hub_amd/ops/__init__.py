@@ -1678,7 +1678,8 @@ _SK_EPI = {"bf16": 0, "swiglu": 1, "resid": 2}
 # of what a whole call takes (0.67 on average with GELU). Over 60 shapes (80 to 9000 rows, N 512
 # to 28672, K 512 to 14336, cold weights, every layout and K split: profiles/gemm_plan_grid.txt)
 # the plan is the fastest in 54, 0.6 % behind the fastest on average and 16 % at worst (9000 x
-# 2048 x 512 with GELU: 46.8 us, 40.3).
+# 2048 x 512 with GELU: 46.8 us, 40.3). Measured before the epilogues took their present form
+# (calls with GELU 8 to 10 % faster: 1500 and 9000 x 5120 x 1280).
 SK_LAYOUTS = {1: (128, 64, 0.60, 4.0), 7: (64, 64, 0.55, 4.0),
               12: (256, 256, 1.20, 10.3), 13: (256, 192, 1.075, 5.5), 14: (192, 256, 1.073, 5.5),
               15: (256, 128, 0.908, 4.0), 16: (128, 256, 0.784, 6.6), 17: (128, 192, 0.667, 4.6),
