@@ -101,6 +101,19 @@ def test_rows_that_are_not_16_byte_aligned(epi):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("lo,hi,more", [(-13.1, -9, 0.006), (-9, -7, 0.001), (-7, -5, 0.0002), (-5, -0.001, 0.00002), (0.001, 9, 0.000002)])
+def test_gelu_relative_error(lo, hi, more):
+    """Relative to the value, down to the smallest ones that bf16 holds: its half ulp (2^-9 of the next power
+    of two, 2^-8 of the value at most) and ``more``, the largest relative error of the f32 value with a margin of a
+    fifth or more (measured 0.0048, 0.00065, 0.00016, 0.00001 and 0.0000003)."""
+    b = torch.linspace(lo, hi, 4096).cuda()
+    x, w = torch.zeros(1, 64, dtype=torch.bfloat16, device="cuda"), torch.zeros(4096, 64, dtype=torch.bfloat16, device="cuda")
+    y, v = ops.gemm_sk(x, w, bias=b, act="gelu")[0].double(), b.double()
+    want = 0.5 * v * torch.special.erfc(-v / 2 ** 0.5)
+    assert torch.all((y - want).abs() <= (2.0 ** -8 + more * 1.01) * want.abs())
+
+
+@pytest.mark.gpu
 def test_gelu_over_its_whole_range():
     """gelu(b) for biases from the far negative tail to the largest finite value, and the
     infinities and NaN as 0.5 v (1 + erf(v / sqrt 2)) gives them."""
@@ -109,7 +122,7 @@ def test_gelu_over_its_whole_range():
     y = ops.gemm_sk(x, w, bias=b, act="gelu")[1].double()
     v = b.double()
     want = 0.5 * v * torch.special.erfc(-v / 2 ** 0.5)
-    # the rational form's 1.5e-7 times |v| / 2, and bf16's half ulp
+    # bf16's half ulp; f32 rounding, and values below bf16's normal ones (relative errors: above)
     assert torch.all((y - want).abs() <= 2.0 ** -8 * want.abs() + 1e-7 * v.abs().clamp(max=16))
     edge = torch.full((128,), float("inf"), device="cuda")
     edge[1], edge[2] = -float("inf"), float("nan")
