@@ -33,3 +33,26 @@ def test_norms(rows, d):
         y = f(x, residual=s)
         assert torch.equal(s, (x.float() + r.float()).bfloat16())
         check(y, s, ln)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ln", [False, True])
+@pytest.mark.parametrize("d", [2048, 3072, 4096])
+def test_small_entries_behind_a_large_one(ln, d):
+    """Squares of 1 behind one of 2^24 in a lane's chain round away one by one; a piece's own sum does not. eps
+    leaves a ten-thousandth of the mean square, so that what the sum lost shows in bf16."""
+    x = torch.ones(2048, d)
+    x[:, 7:512:8] = 4096
+    if ln:
+        x.view(2048, -1, 2, 8)[:, :, 1] *= -1      # a mean of 0
+    v = x.double()
+    v = v - v.mean(-1, keepdim=True) if ln else v
+    ms = v.square().mean(-1, keepdim=True)
+    eps = -float(ms[0]) * (1 - 1e-4)
+    w, b = torch.ones(d).bfloat16().cuda(), torch.zeros(d).bfloat16().cuda()
+    xd = x.bfloat16().cuda()
+    y = (ops.layernorm(xd, w, b, eps) if ln else ops.rmsnorm(xd, w, eps)).double().cpu()
+    want = v / (ms + torch.tensor(eps, dtype=torch.float32).double()).sqrt()
+    # bf16's half ulp, and of the mean square 6 half ulps of f32 (7 squares of 1 rounded to even in a lane,
+    # the lanes' sums, the quotient; one chain: 23, 39 and 55), ten thousand times, halved by the root
+    assert torch.all((y - want).abs() <= (2.0 ** -8 + 6 * 2.0 ** -24 * 0.5e4) * want.abs())
