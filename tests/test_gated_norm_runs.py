@@ -24,3 +24,21 @@ def test_groups(per, T, groups, dt):
             y = seqmix.gated_rmsnorm(o, w, gate, 1e-6, dt, groups=groups, **kw).double()
             # half an ulp of bf16 results, a few 2^-24 of f32 ones
             assert torch.all((y - want).abs() <= (2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -20) * want.abs() + 1e-6)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("per", [64, 128, 256, 512])
+def test_small_entries_behind_a_large_one(per):
+    """Squares of 1 behind one of 2^24 round away one by one in a chain. eps leaves a ten-thousandth of the mean
+    square, so that what the sum lost shows."""
+    T = 4096
+    x = torch.ones(T, per)
+    x[:, ::8] = 4096
+    ms = x.double().square().mean(-1, keepdim=True)
+    eps = -float(ms[0]) * (1 - 1e-4)
+    o, w, z = x.cuda(), torch.ones(per).cuda(), torch.zeros(T, per).cuda()
+    y = seqmix.gated_rmsnorm(o, w, z, eps, torch.float32).double().cpu()
+    want = 0.5 * x.double() / (ms + torch.tensor(eps, dtype=torch.float32).double()).sqrt()
+    # of the mean square 4 half ulps of f32 (a square of 1 a lane, the lanes' sums; a chain of eight: 7),
+    # ten thousand times, halved by the root
+    assert torch.all((y - want).abs() <= 4 * 2.0 ** -24 * 0.5e4 * want.abs())
