@@ -1773,7 +1773,7 @@ def _ahead(p, ahead: tuple, tiles: int) -> None:
     0.30 from the Infinity Cache, 1500 x 5120 x 1280 20.4 and 16.4 us before its epilogue, while the
     240 tiles of either leave 16 compute units and most of the memory's bandwidth idle."""
     wgs = min(SK_CUS - tiles, AHEAD_WGS[1])
-    if wgs < AHEAD_WGS[0] or max(w.numel() for w in ahead) * 2 < AHEAD_MIN_BYTES:
+    if wgs < AHEAD_WGS[0] or max(w.numel() * w.element_size() for w in ahead) < AHEAD_MIN_BYTES:
         return
     step, around = SK_LAYOUTS[p.layout][2:]
     us = p.K // 64 / p.S * step + around
@@ -1820,6 +1820,9 @@ def gemm_sk(x: torch.Tensor, w: torch.Tensor, *, epi: str = "bf16", bias: torch.
     assert x.shape[1] == K, (x.shape, w.shape)
     if epi == "resid":
         assert residual is not None and residual.shape == (M, N)
+    for a in ahead:
+        if not isinstance(a, torch.Tensor) or a.device != x.device:
+            raise ValueError("ahead takes tensors on the device of the rows")
     if not _gpu(x):
         y = _sk_ref(x, w, epi, bias, residual, act)
         dst = residual if epi == "resid" else out

@@ -30,6 +30,19 @@ def test_what_is_touched():
     assert touched(_params(28672, 4096, 13), (torch.empty(4096, 4096, dtype=torch.bfloat16),), 224) == (0, [0, 0])
 
 
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+def test_only_tensors_of_the_same_device(device):
+    """What is touched goes to the launch as an address: tensors elsewhere are refused before it."""
+    x, w = torch.zeros(300, 1024, dtype=torch.bfloat16, device=device), torch.zeros(256, 1024, dtype=torch.bfloat16, device=device)
+    here = torch.zeros(2_200_000, dtype=torch.bfloat16, device=device)
+    others = [here.to("meta"), here.data_ptr(), None] + ([here.cpu()] if device == "cuda" else [])
+    for call in (ops.proj, ops.gemm_sk):
+        call(x, w, ahead=(here,))
+        for bad in others:
+            with pytest.raises(ValueError):
+                call(x, w, ahead=(here, bad))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("layout", [k for k in sorted(ops.SK_LAYOUTS) if k >= ops.SK_PIPE])
 def test_product_is_the_same(layout):
