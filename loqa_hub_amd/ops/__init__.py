@@ -1951,21 +1951,25 @@ def conv_k3_gelu(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor, B: int, s
                  pos: torch.Tensor | None = None) -> torch.Tensor:
     """GELU(conv1d(x)) (+ ``pos`` rows m % len(pos)), k = 3, padding 1: x time-major [B * T_in, Cin]
     bf16, w a :func:`conv_k3_weight` [N, 3 * Cin], f32 ``bias`` -> [B * T_out, N] bf16. On the
-    pipelined tiles; feature or channel counts they do not take go to :func:`gemm_tile`."""
-    N, cin = w.shape[0], x.shape[1]
-    if not _gpu(x) or N % 128 or cin % 64 or x.stride(1) != 1 or x.stride(0) % 8 or x.stride(0) >= 1 << 21 or x.data_ptr() % 16:
+    pipelined tiles; sizes, strides and alignments they do not take go to :func:`gemm_tile`."""
+    N, cin, tin = w.shape[0], x.shape[1], x.shape[0] // B
+    tout = (tin - 1) // stride + 1
+    # what the launch asks for: whole tiles of features and K steps, 16-byte pieces, and 32-bit offsets within
+    # the input rows that a tile of 128 (the largest of CONV_LAYOUTS) reaches, over several windows' ends too
+    if not _gpu(x) or N % 128 or cin % 64 or x.stride(1) != 1 or x.stride(0) % 8 or not cin <= x.stride(0) < 1 << 21 \
+            or tout < 1 or (128 * stride + 2 * (128 // tout + 2)) * x.stride(0) * 2 >= 0x7fffffff \
+            or x.data_ptr() % 16 or w.data_ptr() % 16 or (pos is not None and pos.data_ptr() % 16):
         return gemm_tile(x, w, bias=bias, act="gelu", pos=pos, conv=(B, stride), layout=0)
-    if x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or not w.is_contiguous() or w.data_ptr() % 16:
+    if x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or not w.is_contiguous():
         raise TypeError("conv_k3_gelu needs contiguous bf16 weights and bf16 rows")
     assert w.shape[1] == 3 * cin and x.shape[0] % B == 0
     assert bias.dtype == torch.float32 and bias.is_contiguous() and bias.numel() == N
     p = _lib.ConvPipeParams()
-    p.tin = x.shape[0] // B
-    p.tout = (p.tin - 1) // stride + 1
+    p.tin, p.tout = tin, tout
     p.x, p.ldx, p.w, p.bias = ptr(x), x.stride(0), ptr(w), ptr(bias)
     p.M, p.N, p.cin, p.stride = B * p.tout, N, cin, stride
     if pos is not None:
-        assert pos.dtype == torch.bfloat16 and pos.is_contiguous() and pos.shape[1] == N and pos.data_ptr() % 16 == 0
+        assert pos.dtype == torch.bfloat16 and pos.is_contiguous() and pos.shape[1] == N
         p.pos, p.pos_rows = ptr(pos), pos.shape[0]
     y = torch.empty(p.M, N, dtype=torch.bfloat16, device=x.device)
     p.y, p.ldy = ptr(y), N

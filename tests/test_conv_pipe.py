@@ -31,3 +31,33 @@ def test_conv(device, B, tin, cin, N, stride):
             # sums of 3 cin products
             tol = 2.0 ** -8 * (want.abs() + v.abs() + 1.13 * a.abs()) * 1.01 + 1e-5
             assert torch.all((y - want).abs() <= tol), (y - want).abs().max()
+
+
+@pytest.mark.parametrize("case", ["fits", "features", "channels", "rows 8 bytes off", "weights 8 bytes off", "positions 8 bytes off",
+                                  "row stride", "rows far apart", "short windows far apart"])
+def test_which_kernel(case, monkeypatch):
+    """Everything that the pipelined launch refuses goes to gemm_tile, nothing else does."""
+    monkeypatch.setattr(ops, "_gpu", lambda x: True)
+    monkeypatch.setattr(ops, "gemm_tile", lambda *a, **k: "gemm_tile")
+    monkeypatch.setattr(ops, "stream_ptr", lambda x: 0)
+    asked = []
+    monkeypatch.setattr(ops, "check", lambda *a: None)
+    monkeypatch.setattr(ops, "kernels", lambda: type("K", (), {"loqa_conv_pipe": lambda self, p, s: asked.append(p)})())
+    N, cin, tin, ld, dev = 128, 64, 40, 64, "cpu"
+    if case == "features":
+        N = 192
+    if case == "channels":
+        cin = ld = 96
+    if case == "row stride":
+        ld = 68
+    if case == "rows far apart":
+        ld, dev = 1 << 21, "meta"
+    if case == "short windows far apart":
+        ld, tin, dev = (1 << 21) - 8, 1, "meta"
+
+    def make(rows, cols, off=0):
+        return torch.zeros(rows * cols + 16, dtype=torch.bfloat16, device=dev)[off:off + rows * cols].view(rows, cols)
+    x = make(2 * tin, ld, 4 if case.startswith("rows 8") else 0)[:, :cin]
+    w, pos = make(N, 3 * cin, 4 if case.startswith("weights") else 0), make(tin, N, 4 if case.startswith("positions") else 0)
+    y = ops.conv_k3_gelu(x, w, torch.zeros(N), 2, 2 if tin == 1 or ld > 1 << 20 else 1, pos=pos)
+    assert (y == "gemm_tile") if case != "fits" else (len(asked) == 1 and y.shape == (80, N))
