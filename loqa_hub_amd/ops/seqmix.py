@@ -302,8 +302,8 @@ def latent_keys_values(cache: torch.Tensor, block_tables: torch.Tensor, cu_k: to
     Dr = cache.shape[2] - R
     assert wkv.shape[0] == H * (DK + DV) and cache.is_contiguous() and D + Dr <= DK
     fits = [n for n, (bn, _, _, _) in KV_LAYOUTS.items() if H * DK % bn == 0 and H * DV % bn == 0]
-    if not fits or R % 64 or Dr > 64 or Dr % 16 or D % 16 or cache.numel() >= 1 << 30 or cache.data_ptr() % 16 or \
-            wkv.data_ptr() % 16 or not wkv.is_contiguous() or not total_k:
+    if not fits or R % 64 or Dr > 64 or Dr % 16 or D % 16 or DK % 16 or wkv.shape[0] >= 1 << 20 or cache.numel() >= 1 << 30 or \
+            cache.data_ptr() % 16 or wkv.data_ptr() % 16 or not wkv.is_contiguous() or not total_k:
         cl, kr = latent_gather(cache, block_tables, cu_k, ctx_lens, total_k, max_ctx, R)
         k = torch.nn.functional.linear(cl, wkv[:H * DK]).view(-1, H, DK)
         latent_kfill_(k, kr, D)

@@ -47,6 +47,39 @@ def test_keys_values(layout, H, DK, DV, D, R, Dr, lens, monkeypatch):
         assert torch.all((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5)
 
 
+@pytest.mark.parametrize("case", ["fits", "rank", "rotary part", "tiles", "head width", "all heads' rows", "cache size", "no rows"])
+def test_which_form(case, monkeypatch):
+    """Everything that the launch refuses is gathered and multiplied, nothing else is."""
+    H, DK, DV, D, R, Dr, blocks, total, dev = 4, 192, 128, 128, 512, 64, 8, 5, "cpu"
+    if case == "rank":
+        R = 520
+    elif case == "rotary part":
+        Dr, D = 80, 112
+    elif case == "tiles":
+        H, DK, DV, D = 1, 192, 32, 128
+    elif case == "head width":
+        H, DK, D, Dr = 16, 136, 64, 64
+    elif case == "all heads' rows":
+        H, DK, DV, D, R, Dr, dev = 8192, 64, 64, 32, 64, 16, "meta"
+    elif case == "cache size":
+        blocks, dev = 1 << 18, "meta"
+    elif case == "no rows":
+        total = 0
+    cache = torch.zeros(blocks, 16, R + Dr, dtype=torch.bfloat16, device=dev)
+    w = torch.zeros(H * (DK + DV), R, dtype=torch.bfloat16, device=dev)
+
+    class Gathered(Exception):
+        pass
+
+    def gather(*a):
+        raise Gathered
+    monkeypatch.setattr(seqmix, "latent_gather", gather)
+    i32 = torch.zeros(2, dtype=torch.int32)
+    # (past the rule the launch wants GPU tensors)
+    with pytest.raises(AssertionError if case == "fits" else Gathered):
+        seqmix.latent_keys_values(cache, i32[None, :1], i32, i32[:1], total, 5, w, H, DK, DV, D)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("off,dims", [(128, 64), (128, 32), (64, 40), (130, 12)])
 def test_queries_turned_in_the_launch(off, dims):
