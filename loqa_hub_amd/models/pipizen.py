@@ -59,9 +59,12 @@ def latent_prompt_layout(L: dict, m, dtype, device) -> None:
         out[:, :per] = w.view(H, per, -1)
         return out.view(H * to, -1).contiguous()
     L["wq"], L["qw"] = pad_rows(L["wq"], D + Dr, DKp), DKp
-    # keys and values of all heads as one product (seqmix.latent_keys_values)
-    L["wkv_p"] = torch.cat([pad_rows(L["wuk"].reshape(H * D, R), D, DKp),
-                            pad_rows(L["wuv_t"].transpose(1, 2).reshape(H * Dv, R), Dv, DVp)])
+    # keys and values of all heads as one product (seqmix.latent_keys_values), written once
+    wkv = torch.empty(H * (DKp + DVp), R, dtype=dt, device=dev)
+    k, v = wkv[:H * DKp].view(H, DKp, R), wkv[H * DKp:].view(H, DVp, R)
+    k[:, :D], v[:, :Dv] = L["wuk"], L["wuv_t"].transpose(1, 2)
+    k[:, D:], v[:, Dv:] = 0, 0
+    L["wkv_p"] = wkv
     L["prompt_sizes"] = (DKp, DVp)
 
 
