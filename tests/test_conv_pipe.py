@@ -6,10 +6,15 @@ import torch
 from loqa_hub_amd import ops
 
 
-@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+@pytest.mark.parametrize("device,layout", [("cpu", None)] + [pytest.param("cuda", n, marks=pytest.mark.gpu) for n in (None, *ops.CONV_LAYOUTS)])
 @pytest.mark.parametrize("B,tin,cin,N,stride", [(1, 300, 128, 128, 1), (3, 97, 64, 256, 2), (5, 33, 128, 384, 1), (2, 1, 64, 128, 1),
-                                                (70, 2, 64, 128, 2), (2, 3000, 128, 256, 1), (4, 1500, 512, 512, 2)])
-def test_conv(device, B, tin, cin, N, stride):
+                                                (70, 2, 64, 128, 2), (2, 3000, 128, 256, 1), (4, 1500, 512, 512, 2), (7, 190, 64, 512, 1),
+                                                (130, 2, 64, 256, 2)])
+def test_conv(device, layout, B, tin, cin, N, stride, monkeypatch):
+    if layout is not None:
+        if N % ops.SK_LAYOUTS[layout][0]:
+            pytest.skip("no whole tiles")
+        monkeypatch.setattr(ops, "CONV_LAYOUTS", (layout,))
     g = torch.Generator().manual_seed(tin + N)
     tout = (tin - 1) // stride + 1
     x = torch.randn(B * tin, cin + 16, generator=g).bfloat16()[:, 8:8 + cin]

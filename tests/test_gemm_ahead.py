@@ -45,17 +45,29 @@ def test_only_tensors_of_the_same_device(device):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("layout", [k for k in sorted(ops.SK_LAYOUTS) if k >= ops.SK_PIPE])
-def test_product_is_the_same(layout):
+def test_product_is_the_same(layout, monkeypatch):
     g = torch.Generator().manual_seed(layout)
     x = torch.randn(300, 1024, generator=g).bfloat16().cuda()
     w = (torch.randn(768, 1024, generator=g) / 32).bfloat16().cuda()
+    bias, old = torch.randn(768, generator=g).cuda(), torch.randn(300, 768, generator=g).bfloat16().cuda()
     later = torch.randn(2_200_001, generator=g).bfloat16().cuda()[:2_200_000 + layout % 2]   # off whole kilobytes
+    seen, rule = [], ops._ahead
+
+    def counted(p, *a):
+        rule(p, *a)
+        seen.append((p.ahead_wgs, sum(n > 0 for n in p.ahead_bytes)))
+    monkeypatch.setattr(ops, "_ahead", counted)
     for splits in (1, 2) if layout != ops.SK_WHOLE else (1,):
-        for kw in ({}, {"epi": "swiglu"}, {"act": "gelu"}):
-            if kw.get("epi") == "swiglu" and 768 % (2 * ops.SK_LAYOUTS[layout][0]):
-                continue
-            want = ops.gemm_sk(x, w, layout=layout, splits=splits, **kw)
+        for kw in ({}, {"bias": bias}, {"act": "gelu"}, {"act": "gelu", "bias": bias}, {"epi": "swiglu"}, {"epi": "resid"},
+                   {"epi": "resid", "bias": bias}):
+            def call(**more):
+                if kw.get("epi") == "resid":         # added to in place
+                    more["residual"] = old.clone()
+                return ops.gemm_sk(x, w, layout=layout, splits=splits, **kw, **more)
+            want = call()
             keep = later.clone()
             for ahead in ((later,), (later, w), (w[:8], later[:2_100_000])):
-                assert torch.equal(ops.gemm_sk(x, w, layout=layout, splits=splits, ahead=ahead, **kw), want)
+                seen.clear()
+                assert torch.equal(call(ahead=ahead), want)
+                assert len(seen) == 1 and seen[0][0] >= ops.AHEAD_WGS[0] and seen[0][1] == len(ahead)
             assert torch.equal(later, keep)
