@@ -1755,12 +1755,24 @@ def _sk_workspace(dev: torch.device, stream: int, floats: int, tiles: int):
     return ws
 
 
-# What a launch touches for later ones (:func:`_ahead`): by how many workgroups (under 8 the launch
-# gets a tail, above 32 they take the L2 from the tiles), how much one of them brings in and how
-# much the memory moves beside the launch's own weights, both per microsecond of SK_LAYOUTS' time.
-# The last is the rule that matters: 320 rows x 28672 x 4096, bound by its 235 MB, took 78 us and
-# with the next 117 MB 95. Weights under 4 MB arrive within a microsecond (Whisper base: no gain).
-AHEAD_WGS = (8, 32)
+# What a launch touches for later ones (:func:`_ahead`): by how many workgroups, how much one of them
+# brings in and how much the memory moves beside the launch's own weights, both per microsecond of
+# SK_LAYOUTS' time. Measured as pairs of a launch and the one that reads the touched weights, 13 pairs of the
+# models' projections at 100 to 1500 rows, every constant moved to both sides (profiles/ahead_rule.txt; us
+# a pair without touching, with this rule, with the constant moved):
+# * under 16 workgroups the touching outlasts the tiles (they bring about 48 KB/us each): 6144 then 4096 x
+#   4096 at 700 rows 83.5, 78.0, 111.7 by 8; 3840 then 5120 x 1280 at 1500 rows 49.6, 45.8, 58.7. 64 instead of 32 are the
+#   same within 1 %.
+# * 100 KB/us each: with 50, 1280 x 5120 behind 5120 x 1280 at 700 rows (16 workgroups) is left out, 50.1, 45.6, 50.1; with
+#   200 nothing changes.
+# * 3 MB/us: with 6, launches bound by their own weights are held up: 6144 then 4096 x 4096 at 100 rows 55.1, 54.5,
+#   60.3; 28672 x 4096 then 4096 x 14336 at 320 rows 152.2, 152.4, 169.6; with 1.5 seven pairs of 1280 to
+#   4096 columns lose their gain (35.3, 32.6, 35.2). It costs one pair, 2048 x 8192 then 3072 x 2048 at 100 rows: 42.2,
+#   42.1, 38.0 with 6.
+# * weights under 4 MB: 512 x 2048 behind 2048 x 512 would gain 4 us a pair (25.2, 25.2, 20.4 at 320 rows) where they
+#   come from HBM, as in that measurement; an encoder with so small ones is 38 MB in all and
+#   finds them in the Infinity Cache from one pass to the next (Whisper base: no gain in a pass).
+AHEAD_WGS = (16, 32)
 AHEAD_WG_BYTES_PER_US = 100_000
 AHEAD_BYTES_PER_US = 3_000_000
 AHEAD_MIN_BYTES = 4 << 20

@@ -288,7 +288,12 @@ def latent_kfill_(k: torch.Tensor, kr: torch.Tensor, D: int) -> None:
           "latent_kfill")
 
 
-KV_LAYOUTS = {13: (256, 192, 1.075, 5.5), 20: (128, 128, 0.498, 3.6), 19: (128, 64, 0.309, 4.3)}   # as ops.SK_LAYOUTS
+# Tiles of latent_kv.hip (features, rows, us a K step, us around it), the times those of ops.SK_LAYOUTS. Its own are
+# longer (cold pages, rotary parts: 0.53 to 1.32 of the measured time, 0.87 on average; the 128 x 128 tile has a
+# stage less each), but they rank the tiles: over 120 shapes (64 to 7500 rows, 8 to 32 heads, rank 256 to 1024,
+# profiles/latent_kv_plan.txt) the choice is the fastest in 113, 0.2 % behind the fastest on average, 7.4 % at worst
+# (1000 rows, 16 heads of 192 / 128, rank 1024: 24.9 us, 23.2).
+KV_LAYOUTS = {13: (256, 192, 1.075, 5.5), 20: (128, 128, 0.498, 3.6), 19: (128, 64, 0.309, 4.3)}
 
 
 def latent_keys_values(cache: torch.Tensor, block_tables: torch.Tensor, cu_k: torch.Tensor,

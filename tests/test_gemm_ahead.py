@@ -22,6 +22,7 @@ def test_what_is_touched():
     assert touched(_params(5120, 1280), (big,), 240) == (16, [big.numel() * 2, 0])
     assert touched(_params(5120, 1280), (big, small), 240) == (16, [big.numel() * 2, small.numel() * 2])
     assert touched(_params(5120, 1280), (big,), 249) == (0, [0, 0])         # no compute units left
+    assert touched(_params(5120, 1280), (big,), 244) == (0, [0, 0])         # too few: they would outlast the tiles
     assert touched(_params(5120, 1280), (big,), 720) == (0, [0, 0])         # several rounds of tiles
     assert touched(_params(512, 512), (small,), 96) == (0, [0, 0])          # small weights come by themselves
     assert touched(_params(28672, 4096, 13), (torch.empty(1, dtype=torch.bfloat16).expand(4096, 14336),), 224) == (0, [0, 0])
