@@ -239,13 +239,15 @@ __global__ __launch_bounds__(NORM_THREADS) void norm_rows_kernel(
 }
 
 // A wave per row, or a workgroup? The wave's chain of pieces is longer, the workgroup has two
-// barriers (workgroup, wave, us; rms norm but where said): 8 rows x 2048 2.6, 2.6, x 4096 2.9, 3.3;
-// 320 x 3072 3.3, 3.1, x 4096 3.3, 3.6; layer norm 1500 x 4096 9.6, 7.9; 2048 x 4096 8.4, 8.0. A
-// residual's rows come and go on the same chain: 96 x 512 2.7, 2.2, x 1280 2.8, 3.0; 1500 x 2048 6.5,
-// 6.6; 2048 x 1280 6.1, 5.8, x 4096 16.3, 15.4.
-static bool wave_per_row(int rows, int d, bool residual) {
+// barriers. Times with waves over times with workgroups, both builds' calls in turn, 1 to 9000 rows:
+// up to 3072 columns 0.44 to 1.00 (rms norm) and 0.27 to 1.00 (layer norm). Beyond, one row more than fills the
+// compute units with waves costs a round: 4096 columns at 1100 / 1300 / 1600 / 1800 / 2048 / 4096 rows 1.08, 1.05, 1.02,
+// 0.97, 0.94, 0.87 (rms norm), 1.08, 0.86, 0.84, 0.86, 0.87, 0.82 (layer norm). A residual's rows come and go on
+// the same chain: up to 1024 columns 0.49 to 0.97; 1280 and more from 2048 rows on 0.76 to 1.02 (worst: 2048 x
+// 2048, 9000 x 4096), layer norm 0.62 to 0.99.
+static bool wave_per_row(int rows, int d, bool residual, bool ln) {
   if (d <= 0 || d > 4096) return false;
-  return residual ? d <= 1024 || rows >= 2048 : d <= 3072 || rows >= 1024;
+  return residual ? d <= 1024 || rows >= 2048 : d <= 3072 || rows >= (ln ? 1300 : 1800);
 }
 
 template <bool LN>
@@ -268,7 +270,7 @@ extern "C" int loqa_rmsnorm(const void* x, void* residual, const void* w, void* 
                             int rows, int d, float eps, const int64_t* row_idx, hipStream_t s) {
   if (d % 8 != 0 || d > NORM_THREADS * 8 * MAXV || rows <= 0) return (int)hipErrorInvalidValue;
   if (row_idx && residual) return (int)hipErrorInvalidValue;
-  if (wave_per_row(rows, d, residual)) return norm_rows<false>(x, residual, w, nullptr, y, rows, d, eps, row_idx, s);
+  if (wave_per_row(rows, d, residual, false)) return norm_rows<false>(x, residual, w, nullptr, y, rows, d, eps, row_idx, s);
   hipLaunchKernelGGL(rmsnorm_kernel, dim3(rows), dim3(NORM_THREADS), 0, s,
                      (const bf16_t*)x, (bf16_t*)residual, (const bf16_t*)w, (bf16_t*)y, d, eps,
                      row_idx);
@@ -280,7 +282,7 @@ extern "C" int loqa_layernorm(const void* x, void* residual, const void* w, cons
                               hipStream_t s) {
   if (d % 8 != 0 || d > NORM_THREADS * 8 * MAXV || rows <= 0) return (int)hipErrorInvalidValue;
   if (row_idx && residual) return (int)hipErrorInvalidValue;
-  if (wave_per_row(rows, d, residual)) return norm_rows<true>(x, residual, w, b, y, rows, d, eps, row_idx, s);
+  if (wave_per_row(rows, d, residual, true)) return norm_rows<true>(x, residual, w, b, y, rows, d, eps, row_idx, s);
   hipLaunchKernelGGL(layernorm_kernel, dim3(rows), dim3(NORM_THREADS), 0, s,
                      (const bf16_t*)x, (bf16_t*)residual, (const bf16_t*)w, (const bf16_t*)b,
                      (bf16_t*)y, d, eps, row_idx);
