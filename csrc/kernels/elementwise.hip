@@ -154,8 +154,9 @@ __global__ void rope_kv_append_kernel(bf16_t* __restrict__ qkv, int stride,
 // Same operation, every load of the row issued before any store: the loop form
 // above reads, rotates and writes one 4-element group per trip, and its
 // in-place q stores keep the compiler from hoisting the next trip's loads, so
-// a thread pays one memory round trip per group (5 at 40 heads of 128). For widths that are
-// no power of two, and rows off 16 bytes.
+// a thread pays one memory round trip per group (5 at 40 heads of 128). For what the kernel below does not
+// take (widths that are not 16 times a power of two, rows, caches or rotation off 16 bytes, more than six heads
+// a thread, no KV heads), as far as the groups fit; the loop form takes the rest.
 // Here each thread holds up to RK groups (and its V piece) in registers.
 template <int RK>
 __global__ __launch_bounds__(128) void rope_kv_append_batched_kernel(

@@ -1,9 +1,11 @@
 // LDS-tiled MFMA GEMM for large-M projections: Y[M, N] = X[M, K] W[N, K]^T.
 //
-// Where it runs: the conv stem (k = 3 conv1d as an implicit im2col over the time-major input rows) at
-// sizes that the pipelined tiles (conv_pipe.hip) do not take, and projections through ops.gemm_tile;
-// the models' projections run on gemm_pipe.hip. Both operands are K-contiguous row-major tensors
-// (nn.Linear weights as loaded, no shuffled copy).
+// Where it runs: the cross-attention K|V of all decoder layers in one launch per group of utterances,
+// the conv stem (k = 3 conv1d as an implicit im2col over the time-major input rows) at sizes, strides
+// and alignments that the pipelined tiles (conv_pipe.hip) do not take, fc2 as f32 slabs in the encoder
+// without the split-K form, and projections through ops.gemm_tile; the encoder's and the prompts' other
+// projections run on gemm_pipe.hip. Both operands are K-contiguous row-major tensors (nn.Linear
+// weights as loaded, no shuffled copy).
 //
 // Structure (guide §5 "Canonical CDNA GEMM", T1/T2/T4):
 //   * workgroup = WN x WM waves, each wave a (16 FN) x (16 FM) output block (FN x FM
