@@ -1,8 +1,8 @@
 #!/usr/bin/env python3
 """Headline benchmark: multi-command utterances through the on-GPU voice pipeline.
 
-BASELINE.json metric: "ms per added command (multi-cmd utterance) + utterances/sec
-at 1/2/4/8 MI355X"; config 4: 64 concurrent audio streams, Whisper-large-v3 +
+Metric: "ms per added command (multi-cmd utterance) + utterances/sec at 1/2/4/8
+MI355X"; workload: 64 concurrent audio streams, Whisper-large-v3 +
 Llama-3-8B intent, DP=8 (8 streams per GPU -> weak scaling: per-GPU work fixed).
 
 One step = every rank processes B utterances end to end (--mode batch: the
@@ -14,11 +14,11 @@ draw each rank's utterances locally from the shared seed) -> fused PCM convert/R
   -> NATS publishes (embedded broker) -> per-utterance records all_gathered.
 
 Prints ONE JSON line (rank 0). ``value`` = utterances/s over all GPUs;
-ms-per-added-command (both BASELINE.md definitions) is reported alongside.
+ms-per-added-command (both of its definitions) is reported alongside.
 Random-init weights, synthetic speech-like audio (no network / checkpoints).
 
-Modes: ``hub`` (default, the headline - BASELINE config 4 is "64 concurrent
-gRPC audio streams"): the SERVED path, the reference's hot path
+Modes: ``hub`` (default, the headline: 64 concurrent gRPC audio streams on eight
+GPUs): the SERVED path, the reference's hot path
 (``audio_service.go:926-1043``) - a ``HubServer`` per GPU (per rank under
 torchrun) with B simulated relays, each a closed loop of gRPC ``StreamAudio``
 calls (wake-word chunk, 100 ms PCM16 chunks, end of speech), per-relay-group
@@ -202,7 +202,7 @@ def hub_summary(srv, recs: list, args, events_before: int = 0) -> tuple[float | 
 
 def run_hub_dp(args) -> int:
     """``--mode hub`` over ``--gpus N`` (or with ``--tts``): the served hub as
-    deployed for BASELINE config 4 - one front-end process (gRPC relays,
+    deployed for 64 audio streams - one front-end process (gRPC relays,
     per-group arbitration, voice events in SQLite) and one worker process per
     GPU, each with the full composition (``server.build_dp_processor``). B
     relays per GPU, each a closed loop of StreamAudio calls. The front end

@@ -54,7 +54,7 @@ extern thread_local int g_loqa_launch_prio;
 
 // 16-byte load; SC1: a buffer load with the sc1 policy (reads what another
 // workgroup stored write-through in this launch, without an L2-invalidating
-// acquire fence - guide §6 Guideline 16)
+// acquire fence)
 template <int SC1>
 __device__ __forceinline__ uint4 ld16(const bf16_t* base, size_t elem, long long nbytes) {
   if constexpr (SC1) {

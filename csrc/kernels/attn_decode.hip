@@ -1,4 +1,4 @@
-// Decode / jump-forward attention over the paged KV cache (SURVEY §2.4 K12).
+// Decode / jump-forward attention over the paged KV cache.
 //
 // Decode attention is a pure KV-streaming problem: a few query rows per kv
 // head (GQA group x jump-forward tokens <= 32 -> ONE 32-row MFMA tile), so K
@@ -10,7 +10,7 @@
 //   S^T = K Q^T    : K rows go straight from HBM into the MFMA A fragments
 //                    (16 B per lane per k-slice, no LDS); Q^T is register-resident.
 //   O^T += V^T P^T : V goes through the wave's private LDS tile and is read with
-//                    ds_read_b64_tr_b16 (guide T10); P^T is the exp2'ed S^T
+//                    ds_read_b64_tr_b16; P^T is the exp2'ed S^T
 //                    accumulator repacked to bf16 in registers.
 //   merge          : the 4 waves' (m, l, O^T) are merged through LDS by wave 0.
 //   split combine  : a sequence that fits one split is normalised and written
@@ -18,8 +18,7 @@
 //                    (sc1 write-through stores), takes a ticket on the
 //                    (sequence, kv head) counter, and the last arriving split
 //                    merges all partials (sc1 loads, fixed split order) and
-//                    writes the bf16 output - no second launch (guide §5
-//                    "In-launch split-K reduction", §6 Guideline 16).
+//                    writes the bf16 output - no second launch.
 // Paged block-table entries are wave-uniform per 32-key tile (tiles are
 // 32-aligned, blk is a power of two >= 16), so they are scalar loads and the
 // K/V addresses need no per-lane dependent lookup.

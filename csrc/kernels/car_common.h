@@ -213,7 +213,7 @@ __device__ __forceinline__ void car_st_b32(float* base, unsigned bytes, size_t o
 // car_resid_kernel, and of the residual all-reduce prologue items of the next
 // fused GEMM (gemm_skinny.hip, PRO_CAR). SC1: the local results (residual
 // slice, statistics tiles) are stored write-through, for consumers in the
-// SAME launch that read them with sc1 loads (guide §6 Guideline 16).
+// SAME launch that read them with sc1 loads.
 template <int LEAN, int SC1>
 __device__ __forceinline__ void car_resid_block(const CarPeers& peers, long long in_off, long long res_off,
                                                 long long st_off, bf16_t* __restrict__ residual,

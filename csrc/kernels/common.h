@@ -4,7 +4,7 @@
 //   * bf16 tensors are passed as raw uint16 storage (`bf16_t`), converted with
 //     bit shifts on load and round-to-nearest-even (v_cvt_pk_bf16_f32) on store.
 //   * Memory-bound kernels move data in 16-byte vectors (8 x bf16 per lane):
-//     hipcc does not vectorise scalar bf16 loads (guide G13).
+//     hipcc does not vectorise scalar bf16 loads.
 //   * Wave size is 64, hard-coded; block sizes are multiples of 64.
 //   * Every launcher is `extern "C"`, takes the HIP stream explicitly and returns
 //     the hipError_t of the launch so the Python side can fail loudly.
@@ -82,8 +82,7 @@ __device__ __forceinline__ float block_sum(float v, float* scratch) {
   return t;
 }
 
-// XCD-aware bijective remap of a linear workgroup id (guide §5 "XCD swizzle must
-// be bijective"): consecutive logical tiles land on the same XCD / L2.
+// XCD-aware bijective remap of a linear workgroup id: consecutive logical tiles land on the same XCD / L2.
 __device__ __forceinline__ int xcd_remap(int orig, int nwg) {
   const int nxcd = 8;
   if (nwg <= nxcd) return orig;

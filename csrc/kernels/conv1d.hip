@@ -1,6 +1,6 @@
 // Implicit-GEMM 1-D convolution on MFMA for the VITS / HiFi-GAN stack
-// (K20 wavenet_gated_conv, K21 conv_transpose1d_upsample via
-// polyphase, K22 mrf_resblock convs, K23 tanh_out_pcm16).
+// (gated WaveNet convs, transposed-conv upsampling via polyphase, the residual blocks' convs,
+// the tanh output as PCM16).
 //
 // Activations are channels-last bf16 [B][T][C] (a row per time step, so a
 // 16-channel k-slice of one time step is one 16-byte load). The convolution is

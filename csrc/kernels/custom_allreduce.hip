@@ -1,4 +1,4 @@
-// One-shot all-reduce over IPC-mapped peer buffers (SURVEY §2.5 D4, K17).
+// One-shot all-reduce over IPC-mapped peer buffers.
 //
 // Tensor-parallel decode all-reduces are latency-bound (B x 8192 bf16 = 16-256 KB
 // per call, 2 per layer): a ring pays 2(world-1) link hops and drives 1-2 of
@@ -154,7 +154,7 @@ __global__ __launch_bounds__(256) void car_resid_kernel(CarPeers peers, long lon
                            blockIdx.x, gridDim.x);
 }
 
-// Vocab-parallel masked argmax combine (SURVEY D5): every rank publishes one
+// Vocab-parallel masked argmax combine: every rank publishes one
 // 64-bit record per row - [63:49] epoch, [48:17] order-preserving bits of the
 // row's best local logit, [16:0] 2^17-1 - global token id (larger = smaller id,
 // so ties go to the lowest id) - and every rank takes the max over ranks. The

@@ -7,7 +7,7 @@
 //       output in place.
 //   K14 SwiGLU gate: silu(gate) * up.
 //   K15 grammar-masked argmax over the vocabulary (jump-forward JSON decoding).
-// All bf16 traffic is 8-16 bytes per lane (guide G13).
+// All bf16 traffic is 8-16 bytes per lane.
 #include "common.h"
 #include <float.h>
 

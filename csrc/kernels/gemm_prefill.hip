@@ -1,6 +1,5 @@
 // Prefill-shaped GEMM (M ~ 64 - a few thousand token rows): Y = X W^T for the
-// Llama prompt projections and the Whisper encoder (SURVEY §2.4 N2 / N4;
-// PERF.md "Round 3").
+// Llama prompt projections and the Whisper encoder.
 //
 // At M ~ 318 hipBLASLt's tiles cover too few CUs for the N = 4096 projections
 // (o, down) and its large-N tiles re-read weights. Here the weights are
@@ -9,8 +8,8 @@
 // on chip (v_mfma_f32_16x16x32_bf16, A = weights, B = rows). Output: bf16 Y,
 // f32 split-K slabs [S, M, N] that the consumer (slab_rmsnorm /
 // slab_layernorm / slab_rope_append) sums in a fixed order, or SwiGLU.
-// (The round-2 version of this kernel - 4 waves along N, 128-deep chunks, two
-// barriers per chunk - is superseded by layout 3 below: faster on every shape.)
+// (An earlier form - 4 waves along N, 128-deep chunks, two barriers per chunk - was
+// slower than layout 3 below on every shape.)
 #include "common.h"
 
 typedef unsigned u32x4p __attribute__((ext_vector_type(4)));

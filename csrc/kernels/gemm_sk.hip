@@ -11,8 +11,7 @@
 // than the 256 CUs x 2-3 resident workgroups, and a whole tile's K loop is one
 // workgroup's serial latency. Splitting each tile's K range over S workgroups
 // fills the machine; the S partial accumulators are summed by the LAST
-// workgroup of the tile to finish (agent-scope release / ticket / acquire,
-// guide §5 "In-launch split-K reduction"), which then runs the epilogue - no
+// workgroup of the tile to finish (agent-scope release / ticket / acquire), which then runs the epilogue - no
 // f32 slabs for a later kernel to re-read and no extra launch. The sum is in
 // fixed chunk order over the published partials (the reducer's own included),
 // so the result is bitwise identical whoever arrives last.

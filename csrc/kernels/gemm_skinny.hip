@@ -1,6 +1,5 @@
-// Decode-shaped GEMM: out^T[N, M] = W[N, K] * x^T[K, M] for M <= 128 tokens
-// (SURVEY §2.4 "GEMM/GEMV for skinny M"; guide §5 table row "GEMV / M <= 16 decode
-// weights": operand streamed once, straight to VGPRs, deep prefetch).
+// Decode-shaped GEMM: out^T[N, M] = W[N, K] * x^T[K, M] for M <= 128 tokens:
+// weights streamed once, straight to VGPRs, with deep prefetch.
 //
 // Weight-streaming bound: every weight byte is read exactly once per decode
 // step, so the kernel is shaped for HBM bandwidth, not MFMA rate:
@@ -43,7 +42,7 @@ __device__ __forceinline__ bf16x8 ldx(const bf16_t* p) {
 
 // Source of the activation fragments: plain loads, or (XS = 1) sc1 buffer
 // loads - x was stored write-through by a prologue item of the SAME launch
-// (guide §6 Guideline 16: every handed-off byte read with sc1, no acquire)
+// (every handed-off byte read with sc1, no acquire)
 struct XSrc {
   const bf16_t* x0;                 // x base (offsets are taken from it)
   __amdgpu_buffer_rsrc_t r;
@@ -423,8 +422,7 @@ __device__ __forceinline__ void stream_k_xl(WFrag<RT, U>& f0, WFrag<RT, U>& f1, 
 //   gate|up : prologue rmsnorm(mlp_norm)  | epilogue silu(gate) * up -> bf16
 //   down    : epilogue residual add + per-tile row sum of squares
 // Split-K (S > 1) partials are reduced inside the launch by the last arriving
-// workgroup of each 32-row tile (guide §5 "in-launch split-K reduction":
-// write-through sc1 slab stores -> vmcnt(0) -> barrier -> relaxed agent ticket;
+// workgroup of each 32-row tile (write-through sc1 slab stores -> vmcnt(0) -> barrier -> relaxed agent ticket;
 // the reducer takes an agent acquire and sums the S slabs in fixed order, so
 // results are bitwise identical to the launch-boundary reduce). The RMSNorm
 // scale of a row is rebuilt in every consumer workgroup from the producer's
@@ -731,7 +729,7 @@ __device__ __forceinline__ void skinny_fused_tile(const FusedArgs& a, float* sme
   if ((WR == 1 || XL) && a.S > 1) {
     // publish this split's partial (tile-contiguous slab, sc1 write-through),
     // take a ticket; the last arriver reduces with sc1 loads (no acquire fence:
-    // every handed-off byte is stored and loaded sc1, guide §6 Guideline 16).
+    // every handed-off byte is stored and loaded sc1).
     // WR == 1: wave 0 holds the workgroup's tile; XL (WR == 4): every wave
     // publishes and tickets its own tile.
     const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(

@@ -7,7 +7,7 @@
 // projections run on gemm_pipe.hip. Both operands are K-contiguous row-major tensors (nn.Linear
 // weights as loaded, no shuffled copy).
 //
-// Structure (guide §5 "Canonical CDNA GEMM", T1/T2/T4):
+// Structure:
 //   * workgroup = WN x WM waves, each wave a (16 FN) x (16 FM) output block (FN x FM
 //     v_mfma_f32_16x16x32_bf16 tiles, W fragments as the A operand so a lane
 //     holds 4 consecutive output features of one row: 8-byte bf16 stores);

@@ -14,7 +14,7 @@
 // (rows); a wave computes 64 features x BM / 4 rows with 16x16x32 bf16 MFMAs.
 //
 // The two operands have different latencies, so they are staged at different
-// depths (guide §5 "Pipelining across barriers"): weight K-stages (16 KB, from
+// depths: weight K-stages (16 KB, from
 // HBM) NBW deep, activation K-stages (BM x 128 B, from L2) NBX deep, all by
 // global_load_lds with the bank swizzle on the source address, issued
 // activation-first so ONE counted vmcnt per step (the newest weight stage may

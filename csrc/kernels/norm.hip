@@ -3,7 +3,7 @@
 // The row stays in registers between the statistics pass and the scale pass, so HBM traffic is
 // exactly
 //   read x (+ read residual, write residual) + write y.
-// Rows are loaded as 16-byte vectors (8 bf16 per lane, guide G13). A row is a wave's
+// Rows are loaded as 16-byte vectors (8 bf16 per lane). A row is a wave's
 // (norm_rows_kernel) or, where it is long and there are few, a 256-thread workgroup's (up to d =
 // 256 * 8 * MAXV). d % 8 == 0.
 #include "common.h"

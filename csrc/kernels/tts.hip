@@ -1,5 +1,5 @@
-// VITS text-side kernels (SURVEY §2.4 N6):
-//   relpos_attention : K19 - text-encoder self-attention with windowed relative
+// VITS text-side kernels:
+//   relpos_attention : text-encoder self-attention with windowed relative
 //                      position embeddings (VITS attentions.MultiHeadAttention,
 //                      window 4, shared key/value relative tables), masked;
 //   expand_sample    : length regulation fused with prior sampling -

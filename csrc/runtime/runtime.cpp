@@ -4,13 +4,12 @@
 //                  appended into as they arrive on the gRPC stream, then moved
 //                  to HBM with hipMemcpyAsync on the consuming stream (or, opt-in,
 //                  a dedicated H2D stream); a HIP
-//                  event per transfer gates slot reuse (SURVEY §2.4 "Host<->device
-//                  data path"). Replaces the reference's per-sample Go
+//                  event per transfer gates slot reuse. Replaces the reference's per-sample Go
 //                  conversion loop + WAV/HTTP round trip (audio_service.go:1048,
 //                  stt_client.go:365).
 //  * BlockPool   - paged KV-cache block allocator with per-sequence block tables,
 //                  reference counts and a prefix cache so prompts that share the
-//                  parser template prefix share KV blocks (SURVEY §7.2 step 4).
+//                  parser template prefix share KV blocks.
 //                  The cache is looked up by a chained hash but every hit is
 //                  verified against the block's stored token prefix, so a hash
 //                  collision can never hand out another prompt's KV.
@@ -178,7 +177,7 @@ void loqa_stager_destroy(void* h) {
   delete s;
 }
 
-// Stream-in mode (SURVEY §2.4 "Host<->device data path"): every slot gets a
+// Stream-in mode: every slot gets a
 // device mirror, and loqa_stager_flush copies the samples appended since the
 // last flush with hipMemcpyAsync on `stream` - a placed side stream owned by
 // the caller (utils/streams.py "h2d"), so the transfer runs while the relay is

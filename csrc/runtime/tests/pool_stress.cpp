@@ -1,5 +1,5 @@
 // Host-side stress test of the paged-KV BlockPool (runtime.cpp), built with
-// -fsanitize=address,undefined or -fsanitize=thread (SURVEY §5.2: sanitizers on
+// -fsanitize=address,undefined or -fsanitize=thread (sanitizers on
 // host code). Several threads run random sequence lifecycles (add with prefix
 // reuse, append, publish prefix, free) against one pool; invariants checked at
 // the end: every block is either free, cached, or owned, and freeing every

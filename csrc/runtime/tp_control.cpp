@@ -1,4 +1,4 @@
-// Lock-step control ring for tensor-parallel serving (SURVEY §2.5 D4).
+// Lock-step control ring for tensor-parallel serving.
 //
 // A TP group runs one LLM engine per rank; every rank must launch the same
 // decode steps, in the same order, with the same batch - the only input that

@@ -120,8 +120,8 @@ def build(force: bool = False, debug: bool = False, only=None, quiet: bool = Fal
 
 
 def build_sanitized(kind: str = "address,undefined", out_dir: str | None = None) -> str:
-    """Host-only sanitizer build of the C++ runtime + its stress test
-    (GPU sanitizers are not available on the target pool).
+    """Host-only sanitizer build of the C++ runtime + its stress test (the GPU's own
+    sanitizers are not available).
     ``kind``: "address,undefined" or "thread". Returns the executable path."""
     out_dir = out_dir or os.path.join(HERE, "build", "sanitize")
     os.makedirs(out_dir, exist_ok=True)

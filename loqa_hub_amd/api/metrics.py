@@ -1,6 +1,6 @@
 """``/api/metrics``: Prometheus text exposition of the hub's counters (audio
 service arbitration, GPU engines, skills, NATS). The reference exposes no
-metrics endpoint (SURVEY §5.5); this is additive."""
+metrics endpoint; this is additive."""
 from __future__ import annotations
 
 from aiohttp import web

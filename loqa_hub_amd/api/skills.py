@@ -9,7 +9,7 @@ POST   /api/skills/{id}/{enable|disable|reload}
 
 Errors use the reference's JSON shape ``{"error": true, "message": ...}``
 (:372-385); ids are validated with ``validate_skill_id`` (:35-90). The reference
-never routes this handler (SURVEY C11); the hub server here does. Deliberate
+never routes this handler; the hub server here does. Deliberate
 fix: PUT actually applies the config (reference :320-353 mutates a copy and
 persists nothing).
 """

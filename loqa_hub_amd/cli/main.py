@@ -1,6 +1,6 @@
 """Hub entry point (``cmd/main.go:29-54``): logging, configuration, server.
 
-    python -m loqa_hub_amd.cli.main            # env-configured (SURVEY §5.6)
+    python -m loqa_hub_amd.cli.main            # env-configured
 
 Backends follow ``HUB_*``: with a visible GPU and ``HUB_LLM_BACKEND=gpu``
 (default) the on-device pipeline serves STT + intent parsing on ``cuda:0``;

@@ -2,7 +2,7 @@
 
 Same variable names and defaults as the reference (``internal/config/config.go``:
 Load :113-174, validate :177-211; helpers :214-255 silently fall back to the
-default on a parse error). Differences, all additive (SURVEY §3.7 #8, #9, §5.6):
+default on a parse error). Differences, all additive:
 
 * ONE config object: ``OLLAMA_URL``/``OLLAMA_MODEL``, ``NATS_URL``, ``DB_PATH``
   and ``LOG_*`` are read here instead of ad hoc in each component;
@@ -187,7 +187,7 @@ class OllamaConfig:
 
 @dataclass
 class GPUConfig:
-    """On-device pipeline (SURVEY §5.6 'New')."""
+    """On-device pipeline."""
     num_gpus: int = 0                 # 0 = all visible
     dp: int = 0                       # 0 = num_gpus
     tp: int = 1

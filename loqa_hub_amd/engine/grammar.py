@@ -17,7 +17,7 @@ Every decision point maps to one row of a packed uint32 mask table resident on
 the GPU, consumed by the fused masked-argmax kernel (K15). The number of command
 objects is fixed by the compound-utterance splitter, so the output always
 parses and has the intended command count - with random-init weights this is
-what makes the multi-command benchmark meaningful (SURVEY §7.4 item 1).
+what makes the multi-command benchmark meaningful.
 """
 from __future__ import annotations
 

@@ -1,7 +1,7 @@
 """Continuous-batching, grammar-constrained LLM engine (one per GPU).
 
 Replaces the up-to-five Ollama HTTP calls per utterance of the reference
-(SURVEY §3.2 observation 2) with ONE constrained multi-command decode whose
+with ONE constrained multi-command decode whose
 result is shared by the classifier, the bridge, the fallback parser and the
 command queue.
 
@@ -163,7 +163,7 @@ class LLMEngine:
         # tokens, each chunk in ONE pass together with every live sequence's
         # next feed (a mixed step: the live sequences advance during the prompt
         # pass instead of stalling for it); with nothing decoding the whole
-        # prompt is one pass (_mixed_step). Measured (docs/PERF.md "Round 4"):
+        # prompt is one pass (_mixed_step). Measured (docs/PERF.md):
         # 256 -> 19.49-19.64 vs 18.58-19.30 utt/s (4 interleaved pairs); chunk
         # sweep 192 / 256 / 320 / 384 / 512 -> 320 best; 128 loses (a pass is
         # expensive at any row count, so more passes cost more)
@@ -207,10 +207,10 @@ class LLMEngine:
         self._cells_lock = threading.Lock()
         # prompt placement (continuous-batching scheduler): prompt passes run on
         # the decode stream, serialised with the decode steps; while sequences
-        # decode they are the chunked mixed steps above. Removed in round 4
+        # decode they are the chunked mixed steps above. Removed
         # after measuring (docs/PERF.md): a prefill worker stream overlapped
         # with the decode steps (its GEMMs slowed every concurrent step,
-        # 17.9-18.0 vs 18.3-18.5 utt/s), round 3's rider variant (one
+        # 17.9-18.0 vs 18.3-18.5 utt/s), an earlier rider variant (one
         # jump-forward slice per live sequence on a hipBLASLt pass: the drain
         # cost what the riders saved) and coalescing holds.
         self.stats = {"prefill_tokens": 0, "decode_steps": 0, "decode_tokens": 0,
@@ -889,7 +889,7 @@ class LLMEngine:
                 if self.tp_ctl is not None:
                     # lock-step TP: the ranks' scheduler states may now differ
                     # (this rank reset, the others did not), so the group
-                    # cannot continue - stop it and report (SURVEY §5.3)
+                    # cannot continue - stop it and report
                     self._tp_fail(e)
                     break
 

@@ -1,4 +1,4 @@
-"""Pinned relay-PCM staging (SURVEY §2.4 "Host<->device data path").
+"""Pinned relay-PCM staging.
 
 Relay audio arrives on the gRPC stream as PCM16-LE chunks. On the GPU path
 every chunk is appended, as raw bytes, into a pinned (``hipHostMalloc``) slot
@@ -15,7 +15,7 @@ arrives. Two ways to HBM:
 * whole-utterance: one ``hipMemcpyAsync`` at end of speech on the encoder's
   own stream (ordered before the log-mel kernel that reads it).
 
-Utterances longer than one slot (30 s) CHAIN slots (SURVEY §5.7: the
+Utterances longer than one slot (30 s) CHAIN slots (the
 reference accumulates relay audio unboundedly, ``audio_service.go:965,1002``):
 a full slot is followed by another; with every slot busy the rest is kept on
 the host and copied at upload - nothing is dropped below ``MAX_SAMPLES``

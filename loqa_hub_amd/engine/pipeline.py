@@ -359,7 +359,7 @@ class VoicePipeline:
 
 
 def added_command_stats(jobs: list[PipelineJob]) -> dict:
-    """Both BASELINE.md definitions of 'ms per added command':
+    """Both definitions of 'ms per added command':
     * reference-equivalent: queue item durations for index >= 1
       (command_queue.go:119-121: execution + NATS publish);
     * end-to-end marginal: slope of (utterance completion latency) vs

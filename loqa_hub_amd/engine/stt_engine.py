@@ -4,8 +4,8 @@ multipart POST, JSON decode) with: pinned PCM16 -> H2D -> fused convert+RMS
 kernel -> log-mel -> encoder -> greedy decoder, batched across utterances.
 
 Random-init weights cannot produce a real transcript, so benchmark/synthetic
-requests carry their known transcript and the decoder is *teacher-forced* to it
-(SURVEY §7.4 item 1): every step still runs the full decoder forward and the
+requests carry their known transcript and the decoder is *teacher-forced* to it:
+every step still runs the full decoder forward and the
 argmax over the 51 866-entry vocabulary, so cost is that of a real greedy decode
 of the same length; only the fed-back token is the reference one.
 """
@@ -38,7 +38,7 @@ N_SAMPLES = 480000  # 30 s @ 16 kHz
 PCM_STAGER = True
 # relay PCM copied to HBM chunk by chunk while the relay speaks (pcm_staging.py)
 PCM_STREAM_IN = os.environ.get("LOQA_PCM_STREAM_IN", "1") != "0"
-# long-form audio (SURVEY §5.7): an utterance longer than 30 s is split into
+# long-form audio: an utterance longer than 30 s is split into
 # 30 s windows, encoded as extra encoder rows of the same batch (one
 # cross-attention slot each) and decoded window after window, each window's
 # decode prompted with the previous window's text (<|startofprev|>, at most

@@ -133,7 +133,7 @@ class LongUtterance:
 
 def make_long_utterance(seed: int, n_commands: int = 3, seconds: float = 45.0,
                         relay_id: str = "relay-long", sr: int = 16000) -> LongUtterance:
-    """A long-form utterance (SURVEY §5.7): the wake word and the first
+    """A long-form utterance: the wake word and the first
     commands, a long pause (low-level noise), then the LAST command after the
     30 s mark, padded to ``seconds``. Each word's samples are known, so every
     word is assigned to the 30 s window it starts in (``window_texts``)."""

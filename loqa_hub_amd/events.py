@@ -1,7 +1,7 @@
 """Voice-event domain object (``internal/events/voice_event.go``).
 
 Every utterance that reaches the pipeline produces one event; unlike the
-reference (where only ``POST /api/voice-events`` writes them, SURVEY §1.3) the
+reference (where only ``POST /api/voice-events`` writes them) the
 audio path records them too. JSON field names/shape match the Go struct tags
 (``voice_event.go:30-53``) so API clients see the same documents.
 """

@@ -6,7 +6,7 @@ Two interchangeable backends behind one ``LLMBackend`` interface:
                      the default, one decode per utterance, JSON valid by construction;
 * ``OllamaBackend``- ``POST {url}/api/generate`` with ``stream:false``
                      (command_parser.go:223-266), the reference's path, kept for
-                     BASELINE config 1 (CPU Ollama, no GPU) and as a fallback.
+                     hosts without a GPU (Ollama on the CPU) and as a fallback.
 
 ``CommandParser`` keeps the reference's observable behaviour: compound detection,
 multi-command prompt with fallback to a single-command parse on any error

@@ -9,7 +9,7 @@ response strings. In the reference this path only runs under tests; here the
 audio pipeline drives it after every multi-command parse.
 
 ``CommandQueueItem.duration`` of items with index >= 1 is the
-"ms per added command (reference-equivalent)" of BASELINE.md.
+"ms per added command (reference-equivalent)" of the benchmark.
 """
 from __future__ import annotations
 

@@ -1,14 +1,13 @@
 """OpenAI-compatible STT REST client (``internal/llm/stt_client.go``).
 
-The reference path for BASELINE config 1 (external STT service); the MI355X
+The reference's path with an external STT service; the MI355X
 path is the on-GPU Whisper engine (engine/stt_engine.py). Kept behaviour:
 ``/health`` check at construction (:89-105), ``POST /v1/audio/transcriptions``
 multipart with ``file=audio.wav`` (32-bit IEEE-float mono WAV, :365-398),
 ``model=tiny``, ``language``, ``temperature=0.0``, ``response_format=json``
 (:136-149), ``{"text": ...}`` response, then wake-word post-processing
 (:401-513, shared with the GPU path via ``transcriber.py``). The WAV body is
-built with one vectorised ``tobytes`` instead of a per-sample append
-(SURVEY §3.7 #10).
+built with one vectorised ``tobytes`` instead of a per-sample append.
 """
 from __future__ import annotations
 

@@ -1,7 +1,7 @@
 """Hub event bus on NATS - subjects and JSON payloads byte-compatible with the
 reference (``internal/messaging/nats_service.go``: event types :38-65, subjects
 :68-73, publish/subscribe :118-236). The URL comes from the single config
-object (env ``NATS_URL``), fixing the reference's config bypass (SURVEY §3.7 #8).
+object (env ``NATS_URL``), fixing the reference's config bypass.
 """
 from __future__ import annotations
 

@@ -1,6 +1,6 @@
 """Model configurations for the on-GPU STT -> intent -> TTS pipeline.
 
-Dimensions are public model-card facts (SURVEY §2.4 N1-N6). Weights are always
+Dimensions are public model-card facts. Weights are always
 seeded random-init (no network, no checkpoints); ``loqa_hub_amd.engine.weights``
 can also map safetensors files when they exist locally.
 """

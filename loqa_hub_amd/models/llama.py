@@ -12,7 +12,7 @@ Layout is MI355X-first rather than HF-module-first:
   structure lives only in the attention metadata;
 * tensor parallel: QKV/gate-up column-sharded by head / ffn slice, O/down
   row-sharded with one all-reduce each, vocab-parallel lm_head with a
-  (max, argmax) combine (SURVEY §2.5 D4/D5).
+  (max, argmax) combine.
 """
 from __future__ import annotations
 
@@ -324,7 +324,7 @@ class LlamaWeights:
 
 # prompt passes on the hand-written GEMMs (ops.proj: split-K tiled / weight-
 # streaming MFMA kernels with fused SwiGLU / residual epilogues); 0: hipBLASLt
-# (measured: 19.23 / 19.30 vs 19.15 / 18.99 utt/s, docs/PERF.md "Round 4")
+# (measured: 19.23 / 19.30 vs 19.15 / 18.99 utt/s, docs/PERF.md)
 PREFILL_HW = os.environ.get("LOQA_PREFILL_HW", "1") != "0"
 
 
@@ -427,7 +427,7 @@ class LlamaModel:
         RMSNorm. No hipBLASLt call, no f32 slab written or re-read. (o / down
         as prefill-GEMM f32 slabs summed by the next norm is 9% faster alone,
         7.73 vs 8.46 ms per 318-token pass, but ~1% slower beside the
-        decoders: docs/PERF.md "Round 4".)"""
+        decoders: docs/PERF.md.)"""
         cfg, w, tp = self.cfg, self.w, self.w.tp
         H, Hkv, D = w.h, w.hkv, cfg.head_dim
         residual = x.contiguous()

@@ -1,9 +1,9 @@
-"""Checkpoint I/O (SURVEY §5.4 "New"): safetensors mmap -> pinned host ->
+"""Checkpoint I/O: safetensors mmap -> pinned host ->
 device, in the Hugging Face tensor naming of the public Whisper and Llama
-checkpoints, plus the data-parallel weight broadcast (SURVEY §2.5 D2).
+checkpoints, plus the data-parallel weight broadcast.
 
 The reference has no model weights at all (inference lives in external
-services); BASELINE runs use seeded random init, which every rank reproduces
+services); benchmark runs use seeded random init, which every rank reproduces
 locally without communication. Real checkpoints go through here:
 
 * ``load_llama`` / ``load_whisper``: read a safetensors file (or a directory

@@ -1231,7 +1231,7 @@ def skinny_fused(x: torch.Tensor, wp, mode: str, scratch: FusedScratch, *,
     split_keys, num_splits, workspace, max_k, scale, out) follows the GEMM and
     its output is returned (mode "act": attention over contiguous K / V rows,
     keys k, v, kv_start). Two launches: the one-launch hand-off was measured
-    slower in every configuration and removed (docs/PERF.md, round 5).
+    slower in every configuration and removed (docs/PERF.md).
 
     ``prologue``: the short step that produces x runs INSIDE this launch
     (gemm_skinny.hip PRO; the weight stream starts at once, the tiles read x
@@ -1378,7 +1378,7 @@ def _prologue_standalone(pro: dict, x, scratch) -> None:
 # prologues (models/llama.py _decode_fused_tp_prologue; grid cap:
 # CustomAllReduce.prologue_wgs). Off by default: 328 instead of 567 launches
 # per config-5 rank step, bitwise the same logits, but 7.86 vs 6.87 ms per
-# step (profiles/r6_config5_prologue_ab.txt, docs/PERF.md round 6)
+# step (profiles/r6_config5_prologue_ab.txt, docs/PERF.md)
 TP_PROLOGUE = os.environ.get("LOQA_TP_PROLOGUE", "0") == "1"
 
 

@@ -1,4 +1,4 @@
-"""Custom all-reduce over IPC-mapped peer buffers (SURVEY D4/D5, K17/K18).
+"""Custom all-reduce over IPC-mapped peer buffers.
 
 ``CustomAllReduce(group)`` exports each rank's uncached staging region with
 ``hipIpcGetMemHandle``, exchanges the handles over the (CPU) process group,
@@ -216,7 +216,7 @@ class CustomAllReduce:
     def self_test(self, d: int | None = None) -> dict:
         """Run every collective of this group once on seeded random data and
         check it against the host (gloo) reduction of the same data; raise on
-        any mismatch, on every rank together (SURVEY §5.3: a TP group that
+        any mismatch, on every rank together (a TP group that
         cannot reduce correctly - a broken IPC mapping, a link, a protocol
         bug - must never start serving).
 

@@ -1,4 +1,4 @@
-"""Data-parallel utterance router across the GPUs of one node (SURVEY §2.5 D1-D3).
+"""Data-parallel utterance router across the GPUs of one node.
 
 The hub front end (rank 0) owns every relay stream; arbitration winners are
 dealt to GPU workers least-loaded-first. In the synchronous batch form used by

@@ -1,4 +1,4 @@
-"""Data-parallel serving over the GPUs of one node (SURVEY §2.5 D1/D3, §5.3).
+"""Data-parallel serving over the GPUs of one node.
 
 The hub front-end (gRPC relays, arbitration, HTTP, NATS) stays on the CPU in
 one process; every GPU gets ONE worker process (spawned, pinned to
@@ -11,7 +11,7 @@ GPU. The reference serialises every relay behind one global arbitration
 window and one HTTP STT/Ollama service (``audio_service.go:89,435``); it has no
 multi-GPU anything.
 
-Failure handling (reference: none beyond service retries, SURVEY §5.3):
+Failure handling (reference: none beyond service retries):
 
 * crash  - a worker process that exits is detected by the monitor;
 * hang   - every worker heartbeats (its own thread) with the age of its last

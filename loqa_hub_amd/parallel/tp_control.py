@@ -1,4 +1,4 @@
-"""Lock-step scheduling of a tensor-parallel LLM engine group (SURVEY §2.5 D4).
+"""Lock-step scheduling of a tensor-parallel LLM engine group.
 
 Every rank of a TP group runs the same ``LLMEngine`` scheduler loop; each
 decode step issues the same collectives on every rank, so every rank must take

@@ -1,4 +1,4 @@
-"""Tensor-parallel emulation in ONE process (VERDICT r3 #4: bitwise TP checks).
+"""Tensor-parallel emulation in ONE process (bitwise TP checks).
 
 ``TPEmulation(cfg, device, world)`` holds the ``world`` Megatron shards of the
 model (the same counter-based init as a real TP rank builds) with one KV cache

@@ -1,5 +1,5 @@
-"""Tensor-parallel serving of the intent decoder (Llama-3-70B
-at TP=8 on one 8-GPU node).
+"""Tensor-parallel serving of the intent decoder (Llama-3-70B at TP=8 on
+one 8-GPU node).
 
 One process per GPU (``torchrun --nproc-per-node N``). Rank 0 is the hub: it
 owns the gRPC / HTTP / NATS front end, the Whisper STT and VITS TTS engines and
@@ -93,8 +93,8 @@ def run_follower(eng) -> dict:
 
 
 class TPFailover:
-    """Degradation of a failed tensor-parallel group ("TP=8 ...
-    fall back to the 8B DP path and flag it in metrics"; the reference's own
+    """Degradation of a failed tensor-parallel group: fall
+    back to the 8B data-parallel path and flag it in the metrics (the reference's own
     discipline is to fall back to a working path and tell the user -
     ``audio_service.go:641-664`` bridge -> parser, ``:261-287`` service retry).
 

@@ -7,7 +7,7 @@ for the response type (:190-229), and starts execution in the background
 update is emitted per update strategy (:296-346), and the device reliability
 tracker is updated.
 
-Deliberate fix (SURVEY §3.7 #6): the reference's ``classifyCommand`` is a stub
+Deliberate fix: the reference's ``classifyCommand`` is a stub
 returning a hard-coded bedroom-lights classification, so every ack reads
 "Turning off the bedroom lights now". Here the classification comes from the
 real parse (``CommandClassifier``) and the ack / plan / status texts are

@@ -8,8 +8,8 @@ when enabled. Serves HTTP (``/health`` -> ``ok\\n`` (:137-142),
 ``/api/voice-events[/…]``, ``/api/skills[/…]``, ``/api/streaming/*``,
 ``/api/metrics``) and gRPC ``audio.AudioService/StreamAudio`` on
 ``cfg.server.grpc_port`` (:98-125). Deliberate differences from the reference:
-the skills and streaming APIs are routed (the reference leaves them unrouted,
-SURVEY C11), and every service reads the one config object.
+the skills and streaming APIs are routed (the reference leaves them
+unrouted), and every service reads the one config object.
 
 GPU engines are built lazily by ``build_gpu_processor`` so a CPU-only hub
 (config 1) never imports the HIP path.
@@ -133,7 +133,7 @@ def build_gpu_processor(cfg: Config, nats, device: str = "cuda:0", tts=None, *, 
                              max_buffer_time=sc.max_buffer_time,
                              max_tokens_per_phrase=sc.max_tokens_per_phrase)
     if llm.tp.world > 1 and g.tp_fallback_model != "none":
-        # a failed TP group degrades to a single-GPU engine (SURVEY §5.3)
+        # a failed TP group degrades to a single-GPU engine
         from .parallel.tp_serving import TPFailover
         proc.tp_failover = TPFailover(proc, g.tp_fallback_config(), device, seed=g.seed,
                                       max_seqs=g.max_batch, max_seq_len=g.max_seq_len,

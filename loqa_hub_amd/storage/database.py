@@ -3,7 +3,7 @@ mode 0750, pragmas (WAL, synchronous=NORMAL, cache_size=10000, temp_store=memory
 mmap 256 MiB, foreign_keys, busy_timeout 5 s), schema + migrations at open,
 ``vacuum`` / ``checkpoint(TRUNCATE)`` / ``stats``; plus the privacy retention
 sweep (``LOQA_DATA_RETENTION`` / ``LOQA_AUTO_CLEANUP``) that the reference only
-validates (SURVEY §1.3).
+validates.
 
 One connection guarded by a lock (sqlite3 objects are not thread-safe); the
 async API wraps calls with ``asyncio.to_thread`` where used from the loop.

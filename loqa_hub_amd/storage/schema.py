@@ -3,8 +3,8 @@
 Column set, defaults, CHECK constraints and indexes are those of the
 reference's ``internal/storage/schema.sql:4-46`` (so a database file written by
 either implementation is readable by the other). The reference's
-``migrations/001_remove_audio_hash.sql`` is never embedded or executed there
-(SURVEY §3.7 #7); here migrations are versioned through ``PRAGMA user_version``
+``migrations/001_remove_audio_hash.sql`` is never embedded or executed there;
+here migrations are versioned through ``PRAGMA user_version``
 and applied idempotently - 001 (drop ``audio_hash``) only runs when an old
 table still has that column.
 """

@@ -5,7 +5,7 @@ Builds parser + progressive TTS pipeline + interrupt handler + metrics from
 streaming self-test when enabled (failing hard only if fallback is disabled),
 supports live ``update_configuration`` (:129-164) and ``get_health_status``.
 
-Deliberate fix (SURVEY §3.7 #5): ``process_streaming_command`` registers the
+Deliberate fix: ``process_streaming_command`` registers the
 session *before* starting work; the reference looks the session up first and
 therefore always fails with "no context found" (:167-196).
 """

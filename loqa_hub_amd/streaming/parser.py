@@ -13,8 +13,8 @@ Token sources (``StreamingBackend``):
 
 ``PhraseBuffer`` flushes on the reference's boundary suffixes, at 50 tokens or
 after 2 s since the last flush (:112-124, :295-336), but tests the suffix on a
-bounded tail instead of re-joining the whole buffer per token (SURVEY §3.7 #10:
-O(1) per token instead of O(n)).
+bounded tail instead of re-joining the whole buffer per token (O(1)
+per token instead of O(n)).
 
 Disabled mode answers through the non-streaming ``CommandParser`` as a single
 token/phrase (:422-454); an empty transcription yields "I didn't hear anything.".

@@ -1,4 +1,4 @@
-"""Progressive speech of a live constrained decode (SURVEY §7.4 #5).
+"""Progressive speech of a live constrained decode.
 
 The reference streams Ollama tokens through a ``PhraseBuffer`` into the
 progressive TTS pipeline (``internal/llm/streaming_command_parser.go:162-292``

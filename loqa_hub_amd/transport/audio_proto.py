@@ -3,9 +3,9 @@
 The reference imports ``github.com/loqalabs/loqa-proto/go/audio`` (``go.mod:6``);
 the .proto is not in the reference tree and ``grpc_tools`` is not installed, so
 the descriptors are constructed with ``descriptor_pb2`` from the field usage in
-``audio_service.go:694-699,733-734,765-769,864-870,953-1008`` (SURVEY §2.3 C37).
+``audio_service.go:694-699,733-734,765-769,864-870,953-1008``.
 
-ASSUMPTION (documented, SURVEY §7.2 step 2): field numbers follow declaration
+ASSUMPTION (documented): field numbers follow declaration
 order; override with ``LOQA_PROTO_FIELDS`` (JSON ``{"AudioChunk": {"relay_id": 1,
 ...}}``) if a real relay uses different numbers.
 

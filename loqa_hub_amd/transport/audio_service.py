@@ -7,7 +7,7 @@ Behavioural spec: ``internal/grpc/audio_service.go`` - ``StreamAudio`` (:926-104
 ``sendCancellationResponse`` (:855-877), ``isRelayActive`` (:880-913),
 ``cleanupRelay`` (:916-923), success/error responses (:693-815).
 
-Redesign (SURVEY §3.7 defects #1-#4):
+Redesign:
 * the arbitration state is owned by the asyncio event loop (single-threaded
   actor) - no mutexes, so no ABBA lock-order hazard and no unlocked reads;
 * windows are keyed by ``ARBITRATION_SCOPE``: ``global`` (reference behaviour:
@@ -413,7 +413,7 @@ class AudioService:
                     relay_id = chunk.relay_id
                 # per-chunk line at DEBUG (the reference logs it at info through
                 # zap, ~1 us; a Python JSON record costs ~30 us, 5-6k chunks/s at
-                # 64 relays: docs/PERF.md "Round 5", front end); the wake word and
+                # 64 relays: docs/PERF.md, front end); the wake word and
                 # end of speech keep their info lines
                 if hublog.debug_enabled():
                     hublog.log_audio_processing_debug(relay_id, "received",

@@ -16,8 +16,8 @@ Two interchangeable implementations:
   (``streaming/progressive.py``: the reply field's phrases are synthesised and
   published on ``audio.<relay>`` while the decode runs), else as one file after
   it.
-* ``ServiceVoiceProcessor`` - the reference's external-service path
-  an STT client (``stt_client.py``), a ``CommandParser``
+* ``ServiceVoiceProcessor`` - the reference's external-service path: an
+  STT client (``stt_client.py``), a ``CommandParser``
   over any ``LLMBackend`` (Ollama), optional bridge, optional TTS client.
 """
 from __future__ import annotations

@@ -1,4 +1,4 @@
-"""Fault injection (SURVEY §5.3 "New": env ``FAULT_INJECT``).
+"""Fault injection (env ``FAULT_INJECT``).
 
 The reference has no chaos tooling; its recovery paths (STT failure -> error
 reply ``audio_service.go:764-815``, TTS graceful degrade ``:182-195``,

@@ -1,7 +1,7 @@
 """JSON encoding byte-compatible with Go's ``encoding/json.Marshal``.
 
 The hub's NATS payloads and HTTP bodies must stay byte-identical to the
-reference's (SURVEY §5.8) so existing relays/skills/devices keep working:
+reference's so existing relays/skills/devices keep working:
 compact separators, map keys sorted, HTML-significant characters escaped
 (``<`` ``>`` ``&`` -> ``\\u003c`` ...), U+2028/2029 escaped, floats in Go's
 shortest 'f'/'e' form (``1`` not ``1.0``), ``[]byte`` as base64.

@@ -6,8 +6,8 @@ decoder streams share decides how the GPU interleaves them (measured: 11 vs 19
 utt/s, docs/PERF.md "the 1.8x cliff"). Every serving stream is therefore the
 PyTorch pool stream at a FIXED index, with both pools created first thing.
 
-Round 4 removed the placement experiments that lost (CU-masked streams,
-dedicated spacer streams, pool skews, per-engine priorities; docs/PERF.md).
+The placement experiments that lost are gone (CU-masked streams, dedicated
+spacer streams, pool skews, per-engine priorities; docs/PERF.md).
 """
 from __future__ import annotations
 
@@ -59,13 +59,13 @@ def aligned_pool_stream(device: torch.device, priority: int, slot: int):
 # Explicit placement: every serving stream is the pool stream of a FIXED index
 # (its hardware queue follows from the index), whatever else drew pool streams
 # before. Defaults = the placement measured best (docs/PERF.md, "Stream
-# placement, round 3"; profiles/r3_stream_placement.txt): the LLM decoder on
+# placement"; profiles/r3_stream_placement.txt): the LLM decoder on
 # normal-priority slot 2, the Whisper decoder on high-priority slot 30, the
 # encoder worker on normal-priority slot 28, the prefill worker on slot 3
 # (pools created first thing by init_pools, so slot -> queue is fixed); VITS
 # (progressive reply speech) on normal-priority slot 29.
-# Round 3 found the old
-# implicit placement had depended on the STT upload drawing one pool stream per
+# The implicit placement
+# before had depended on the STT upload drawing one pool stream per
 # batch: removing that draw moved the LLM decoder to slot 0 and halved the
 # throughput (19.1 -> 9.8 utt/s). LOQA_SLOT_<ROLE> overrides (search).
 # The PCM stream-in copies (engine/pcm_staging.py) take the old prefill

@@ -1,4 +1,4 @@
-"""Per-stage tracing (SURVEY §5.1 "New").
+"""Per-stage tracing.
 
 The reference's only timing is ad-hoc ``time.Since`` logging
 (``stt_client.go:185,341``, ``openai_tts_client.go:206``,

@@ -1,5 +1,5 @@
 #!/usr/bin/env python3
-"""The other BASELINE.json configs on ONE MI355X (bench.py measures config 4).
+"""The other workloads on ONE MI355X (bench.py measures the 64 audio streams).
 
   --config 2  Whisper-base + TinyLlama-1.1B, single utterance at a time (one
               closed-loop stream): per-utterance latency, STT / LLM split and

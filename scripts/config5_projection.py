@@ -1,4 +1,4 @@
-"""BASELINE config 5 (Llama-3-70B intent decoder at TP=8) projected from ONE
+"""The Llama-3-70B intent decoder at TP=8 projected from ONE
 MI355X: time one TP rank's decode step at its real shard shapes.
 
 The rank-0 shard of Llama-3-70B (qkv 8192 -> 1280, o 1024 -> 8192, gate|up

@@ -1,5 +1,5 @@
-"""Served-hub FRONT END under BASELINE config-4 load, without GPUs (VERDICT
-r4 #7): the real front end (``HubServer``: grpc.aio AudioService with
+"""Served-hub FRONT END under the load of 64 audio streams, without GPUs:
+the real front end (``HubServer``: grpc.aio AudioService with
 per-group arbitration windows, the DP router, the shared-memory PCM ring,
 SQLite voice events) over N stub worker processes (``parallel/stub_worker.py``:
 fixed-latency fake GPU), driven by R concurrent relays from separate client

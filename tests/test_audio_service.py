@@ -1,6 +1,6 @@
 """gRPC audio service (C12/C37): PCM conversion, multi-relay wake-word arbitration
 (reference ``collision_detection_test.go`` / ``audio_service_test.go``), scoped
-windows (SURVEY §3.7 #3), and a real grpc.aio round trip."""
+windows, and a real grpc.aio round trip."""
 import asyncio
 
 import numpy as np

@@ -1,5 +1,5 @@
 """Per-step token budget and admission limits of the continuous-batching
-schedulers (ADVICE r1: 17+ sequences in a forced-literal run, or 33+ STT
+schedulers (17+ sequences in a forced-literal run, or 33+ STT
 arrivals feeding their SOT prompt, used to exceed the fused GEMMs' row limit
 and fail every in-flight request)."""
 import json

@@ -1,4 +1,4 @@
-"""Data-parallel serving (SURVEY D1/D3, §5.3): one worker process per device
+"""Data-parallel serving: one worker process per device
 behind the least-loaded router, crash / hang detection and re-routing, and
 FAULT_INJECT-driven failures. Workers run on the CPU here (spawned processes,
 same code path as one process per GPU)."""
@@ -120,7 +120,7 @@ def pcm16_factory(spec, device):
 
 
 def test_dp_pcm_shared_memory_ring(monkeypatch):
-    """VERDICT r4 #7: PCM reaches the workers through their shared-memory
+    """PCM reaches the workers through their shared-memory
     rings (only the slot index crosses the queue), byte-exact; slots are
     recycled when results come back (more utterances than slots); an
     utterance longer than a slot falls back to inline bytes."""
@@ -152,7 +152,7 @@ def test_dp_pcm_shared_memory_ring(monkeypatch):
 
 
 def test_dp_pcm_rings_fall_back_when_shm_is_short(monkeypatch):
-    """a POSIX segment is sparse, so a tmpfs limit surfaces as
+    """A POSIX segment is sparse, so a tmpfs limit surfaces as
     SIGBUS on first touch. The rings are reserved up front: too little free
     /dev/shm, or a failed reservation, means inline PCM (no rings, no leak)."""
     import collections
@@ -186,7 +186,7 @@ def test_dp_pcm_rings_fall_back_when_shm_is_short(monkeypatch):
 
 
 def test_pcm_stager_stream_in_failure_degrades(monkeypatch):
-    """when the device mirrors of stream-in cannot be allocated
+    """When the device mirrors of stream-in cannot be allocated
     (HBM nearly full), the stager logs and stays in whole-utterance mode
     instead of raising from its constructor (which failed every relay)."""
     from loqa_hub_amd.engine import pcm_staging

@@ -139,7 +139,7 @@ def test_native_block_pool_matches():
 
 def test_native_prefix_cache_survives_hash_collisions():
     """Every prefix hash forced to collide: hits must still be decided by the
-    stored tokens (ADVICE r1: a collision must never reuse another prompt's KV)."""
+    stored tokens (a collision must never reuse another prompt's KV)."""
     from loqa_hub_amd.engine.kv_cache import NativeBlockPool
     from loqa_hub_amd.ops import _lib
     try:
@@ -246,7 +246,7 @@ def test_bench_cpu_smoke_dp2_gloo():
 
 
 def test_bench_cpu_smoke_dp4_gloo():
-    """Four ranks (the driver runs 1/2/4/8): one NATS broker process for the
+    """Four ranks: one NATS broker process for the
     node, every rank publishes to it, records are all-gathered to rank 0."""
     out = _run([sys.executable, "-m", "torch.distributed.run", "--nnodes=1", "--nproc-per-node",
                 "4", "--master-addr", "127.0.0.1", "--master-port", "29563", "bench.py",
@@ -258,7 +258,7 @@ def test_bench_cpu_smoke_dp4_gloo():
 
 
 def test_bench_cpu_smoke_dp8_gloo():
-    """Eight ranks - the width the driver launches on an 8-GPU node
+    """Eight ranks - the width of an 8-GPU node
     (torchrun --nproc-per-node 8): per-rank served hubs (the default hub mode,
     gRPC relays), one NATS broker, records gathered to rank 0."""
     out = _run([sys.executable, "-m", "torch.distributed.run", "--nnodes=1", "--nproc-per-node",
@@ -272,7 +272,7 @@ def test_bench_cpu_smoke_dp8_gloo():
 
 def test_bench_rank_without_device_fails_fast(monkeypatch):
     """A GPU run whose rank has no device of its own exits 2 with a message
-    before any collective (VERDICT r5 #7)."""
+    before any collective."""
     import importlib.util
     spec = importlib.util.spec_from_file_location("bench_mod", os.path.join(ROOT, "bench.py"))
     bench = importlib.util.module_from_spec(spec)
@@ -660,7 +660,7 @@ def test_llm_compact_weights_match_default_cpu():
 
 
 def test_llm_compact_weights_scheduler_cpu():
-    """compact weights keep no row-major prompt-pass copies, so the
+    """Compact weights keep no row-major prompt-pass copies, so the
     continuous-batching scheduler must not send their prompts (> 64 tokens,
     the default inline limit) into a mixed pass (model.forward -> KeyError);
     they go through the fused chunked prefill and produce the same outputs

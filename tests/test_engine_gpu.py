@@ -519,7 +519,7 @@ def _rel_max(a: torch.Tensor, b: torch.Tensor) -> float:
 
 
 def test_llama3_8b_fused_graph_decode_vs_fp32_gpu():
-    """VERDICT r4 #8: Llama-3-8B shapes (4 layers + the full 128k lm_head)
+    """Llama-3-8B shapes (4 layers + the full 128k lm_head)
     through the fused, graph-replayed decode step, teacher-forced for 32
     steps after a 24-token prompt (fed 8 tokens per fused step), against an
     fp32 torch forward on the same weights (ops.reference.llama_forward_ref):
@@ -570,7 +570,7 @@ def test_llama3_8b_fused_graph_decode_vs_fp32_gpu():
 
 
 def test_whisper_large_v3_fused_graph_decode_vs_fp32_gpu():
-    """VERDICT r4 #8: Whisper-large-v3 decoder shapes (2 layers, d 1280, 20
+    """Whisper-large-v3 decoder shapes (2 layers, d 1280, 20
     heads, 51866 vocab) through the fused, graph-replayed decode step with
     cross-attention over 1500 encoder rows, teacher-forced (the 4-token SOT
     prompt, then 16 one-token steps), against an fp32 torch decoder on the

@@ -1,4 +1,4 @@
-"""FAULT_INJECT recovery paths (SURVEY §5.3) on the live on-device pipeline
+"""FAULT_INJECT recovery paths on the live on-device pipeline
 (tiny models on the CPU): STT failure -> error reply, LLM timeout -> parse-failed
 reply without commands, NATS down -> queue failure (rollback path), TTS failure
 -> text-only reply (graceful degrade)."""

@@ -1,4 +1,4 @@
-"""The served DP hub's front end under load (VERDICT r4 #7): real gRPC relays
+"""The served DP hub's front end under load: real gRPC relays
 into HubServer -> AudioService (per-group windows) -> DP router -> stub worker
 processes (fixed-latency fake GPU, PCM through the shared-memory ring).
 The full-size run (64 relays, 8 workers) is scripts/frontend_bench.py

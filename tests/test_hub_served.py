@@ -1,5 +1,4 @@
-"""The served hub on the on-device pipeline, end to end (SURVEY §3.2 hot path,
-VERDICT r2 #2-#4), on the CPU engines (the same code runs on the MI355X in
+"""The served hub on the on-device pipeline, end to end, on the CPU engines (the same code runs on the MI355X in
 ``tests/test_engine_gpu.py::test_hub_server_gpu_served``):
 
 relay gRPC stream -> arbitration -> Whisper STT -> ONE constrained decode ->
@@ -161,7 +160,7 @@ def test_hub_served_cpu(tmp_path, streaming):
 
 @pytest.mark.parametrize("streaming", [True, False])
 def test_hub_served_dp_cpu(tmp_path, streaming):
-    """The served DP hub (BASELINE config 4's serving path) does what the
+    """The served DP hub (one worker process per GPU) does what the
     1-GPU hub does: two spawned workers, each building the real per-GPU
     composition (``dp_serving._build_worker_processor``) on the CPU engines."""
     relays = ("kitchen-relay", "bedroom-relay")
@@ -171,7 +170,7 @@ def test_hub_served_dp_cpu(tmp_path, streaming):
 
 
 def test_hub_served_dp8_cpu(tmp_path):
-    """The served DP hub at the driver's 8-rank width: eight
+    """The served DP hub at the width of an 8-GPU node: eight
     spawned workers, each the real per-GPU composition on the CPU engines
     (tiny models), eight relays in their own groups - every worker is up,
     every relay is answered and every utterance is a voice event."""

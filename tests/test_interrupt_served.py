@@ -1,6 +1,6 @@
 """A new wake-word winner on a relay interrupts the reply that relay is still
-receiving (``streaming_interrupt_handler.go:69-119``, composed into the hub:
-VERDICT r3 next-round #6). The progressive reply is a streaming session of the
+receiving (``streaming_interrupt_handler.go:69-119``, composed into the hub).
+The progressive reply is a streaming session of the
 composed ``StreamingComponents``: registered with the interrupt handler while
 it is spoken, recorded (first token / first phrase / completion or interrupt)
 in the streaming metrics when it ends."""

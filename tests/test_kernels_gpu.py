@@ -1,5 +1,5 @@
 """Numerics of every HIP kernel against the plain-PyTorch fp32 reference of the
-same op (ops/reference.py). Shapes follow SURVEY §2.4."""
+same op (ops/reference.py). Shapes are the served models'."""
 import math
 
 import numpy as np

@@ -1,4 +1,4 @@
-"""Checkpoint I/O (SURVEY §5.4): safetensors round trips in the Hugging Face
+"""Checkpoint I/O: safetensors round trips in the Hugging Face
 naming for Llama and Whisper (same tensors, same model outputs), and the
 data-parallel weight broadcast (D2) over gloo with 2 ranks."""
 import os

@@ -1,4 +1,4 @@
-"""Long-form audio (SURVEY §5.7, VERDICT r4 #5): an utterance longer than
+"""Long-form audio: an utterance longer than
 Whisper's 30 s window is split into 30 s windows (extra encoder rows of one
 batch), decoded window after window with the previous window's text as the
 prompt, and the texts joined - the reference transcribes the whole
@@ -58,7 +58,7 @@ def test_stt_long_form_free_decoding_cpu():
 
 
 def test_stt_windows_capped_by_max_batch_and_hol_bypass_cpu():
-    """an utterance needing more 30 s windows than the engine has
+    """An utterance needing more 30 s windows than the engine has
     cross-attention slots is truncated (like one past LOQA_STT_MAX_WINDOWS),
     not rejected; and a short utterance may pass a long-form one that waits
     for free slots (bounded, so the long one is never starved)."""

@@ -1,4 +1,4 @@
-"""Host-code sanitizers (SURVEY §5.2): the C++ runtime's paged-KV block pool
+"""Host-code sanitizers: the C++ runtime's paged-KV block pool
 under AddressSanitizer + UBSan and ThreadSanitizer, driven by a multi-threaded
 random-lifecycle stress test (csrc/runtime/tests/pool_stress.cpp)."""
 import shutil

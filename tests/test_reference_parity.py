@@ -1,5 +1,5 @@
 """Behaviour cases of the reference's own suites that the other files do not
-re-express (SURVEY §4.2, §4.4):
+re-express:
 
 * arbitration across consecutive utterances and window clearance
   (``collision_detection_test.go:322-459,517-582``);

@@ -184,7 +184,7 @@ def test_gpu_voice_processor_batches_on_cpu(tmp_path):
 
 
 def test_deferred_logging_keeps_failures_and_call_time_args(monkeypatch, capsys):
-    """with the async log handler, WARNING+ lines are written
+    """With the async log handler, WARNING+ lines are written
     before the call returns (a process killed right after keeps them), and a
     deferred INFO line renders its args as they were at the call."""
     import logging as _logging

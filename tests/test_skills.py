@@ -254,7 +254,7 @@ SLOW_PROCESS_SKILL = textwrap.dedent('''\
 
 def test_process_skill_recovers_after_timeout(skills_root, tmp_path):
     """A timed-out call must not leave its late reply for the next call
-    (ADVICE r1: every later call would read the previous reply)."""
+    (every later call would read the previous reply)."""
     from loqa_hub_amd.skills.loader import ProcessSkill
 
     d = skills_root / "slow"

@@ -1,4 +1,4 @@
-"""Tensor parallelism (SURVEY D4/D5) on the CPU over gloo: a TP=2 group built
+"""Tensor parallelism on the CPU over gloo: a TP=2 group built
 from shards of one model computes the same logits and the same constrained
 decode as the single-process model (column-parallel QKV / gate|up / vocab,
 row-parallel O / down with all-reduce, vocab-parallel masked argmax)."""
@@ -230,7 +230,7 @@ def _failover_worker(rank, world, port, out_dir):
 
 
 def test_tp_follower_death_fails_over(tmp_path):
-    """a follower that dies mid-decode stops the
+    """A follower that dies mid-decode stops the
     TP group - the leader's in-flight requests fail loudly instead of hanging
     or decoding garbage - and serving continues on the single-rank fallback
     engine, flagged ``tp_degraded``."""
@@ -317,7 +317,7 @@ def _idle_death_worker(rank, world, port, out_dir):
 
 
 def test_tp_idle_follower_death_detected_and_fails_closed(tmp_path):
-    """a follower that dies while the leader idles is caught by the
+    """A follower that dies while the leader idles is caught by the
     heartbeat check inside the scheduler's try (the scheduler thread does not
     die with the CollectiveError): the group is marked failed, later
     submissions fail fast, and a failover that would have to invent random

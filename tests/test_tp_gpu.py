@@ -1,6 +1,6 @@
-"""Tensor-parallel serving on the GPU (BASELINE config 5's layout).
+"""Tensor-parallel serving on the GPU.
 
-The round-end box has one MI355X, so the TP ranks share cuda:0 (as in
+With one MI355X the TP ranks share cuda:0 (as in
 test_custom_allreduce_gpu.py): every collective is the real custom IPC kernel
 (row-parallel residual all-reduce, vocab-parallel argmax combine), the decode
 steps are captured HIP graphs replayed in lock step, and the scheduler of every
@@ -251,7 +251,7 @@ def _failover_worker(rank, world, port, out_dir):
 def test_tp_follower_hang_fails_over(tmp_path):
     """A TP follower that stops mid-decode: the leader fails its in-flight
     requests (no garbage tokens, no endless spin), stops the group and serves
-    on the fallback engine with ``tp_degraded`` set (SURVEY §5.3)."""
+    on the fallback engine with ``tp_degraded`` set."""
     import signal
     ctx = mp.get_context("spawn")
     port = _port()
@@ -353,7 +353,7 @@ def test_tp_decode_bitwise_equals_emulation(tmp_path, world, pro):
     """TP=W over the real IPC collectives (W processes sharing cuda:0) vs the
     single-process TP emulation of the same W shards (parallel/tp_emulation.py):
     every logit shard of every decode step and every combined greedy token is
-    BITWISE equal (replaces round 3's 2% / 90% tolerances). ``pro``: the step
+    BITWISE equal. ``pro``: the step
     with the all-reduces as prologue items of the consuming GEMMs, the ranks'
     grids capped so they are resident together (CustomAllReduce.prologue_wgs)."""
     ctx = mp.get_context("spawn")
