@@ -1674,12 +1674,11 @@ def graph_capture(graph: "torch.cuda.CUDAGraph", **kw):
 _SK_EPI = {"bf16": 0, "swiglu": 1, "resid": 2}
 # layout -> (features, rows, us a K step of 64 takes a compute unit, us around a tile's K
 # loop): 1 and 7 are the general form, 12 on the pipelined tiles, one workgroup per CU. Times
-# fitted to measured ones without an epilogue of weight: they are there to rank, and 0.60 to 1.35
-# of what a whole call takes (0.67 on average with GELU). Over 60 shapes (80 to 9000 rows, N 512
+# fitted to measured ones without an epilogue of weight: they are there to rank, and 0.69 to 1.26
+# of what a whole unsplit call takes (0.73 on average with GELU). Over 60 shapes (80 to 9000 rows, N 512
 # to 28672, K 512 to 14336, cold weights, every layout and K split: profiles/gemm_plan_grid.txt)
-# the plan is the fastest in 54, 0.6 % behind the fastest on average and 16 % at worst (9000 x
-# 2048 x 512 with GELU: 46.8 us, 40.3). Measured before the epilogues took their present form
-# (calls with GELU 8 to 10 % faster: 1500 and 9000 x 5120 x 1280).
+# the plan is the fastest in 49, 0.5 % behind the fastest on average and 7.6 % at worst (80 x 4096 x
+# 4096 in four K chunks: 19.9 us, 18.5 in three).
 SK_LAYOUTS = {1: (128, 64, 0.60, 4.0), 7: (64, 64, 0.55, 4.0),
               12: (256, 256, 1.20, 10.3), 13: (256, 192, 1.075, 5.5), 14: (192, 256, 1.073, 5.5),
               15: (256, 128, 0.908, 4.0), 16: (128, 256, 0.784, 6.6), 17: (128, 192, 0.667, 4.6),
