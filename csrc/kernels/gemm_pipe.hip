@@ -32,8 +32,8 @@
 // question) bring the weights of later launches into the Infinity Cache.
 #include "gemm_pipe_tile.h"
 
-int gemm_pipe_ahead(const GemmSkParams& p, int layout, hipStream_t st);   // gemm_pipe_ahead.hip
+int gemm_pipe_ahead(const GemmSkCall& p, int layout, hipStream_t st);   // gemm_pipe_ahead.hip
 
-int gemm_pipe(const GemmSkParams& p, int layout, hipStream_t st) {
+int gemm_pipe(const GemmSkCall& p, int layout, hipStream_t st) {
   return p.ahead_wgs ? gemm_pipe_ahead(p, layout, st) : gp_layout<false>(p, layout, st);
 }

@@ -1,14 +1,17 @@
 // The kernel behind gemm_pipe.hip, for its two translation units (one with workgroups that touch
 // later weights, one without: they compile side by side).
 #pragma once
+#include <type_traits>
 #include "gemm_sk.h"
 #include "gemm_pipe.h"
 
 
 #define GP_GROUP 4
 
+template <bool AHEAD> using GpArgs = std::conditional_t<AHEAD, GemmSkCall, GemmSkParams>;
+
 template <int FN, int FM, int NA, int NB, int EPI, bool AHEAD>
-__global__ __launch_bounds__(256, (gp_per_cu<FN, FM, NA, NB>())) void gemm_pipe_kernel(GemmSkParams p) {
+__global__ __launch_bounds__(256, (gp_per_cu<FN, FM, NA, NB>())) void gemm_pipe_kernel(GpArgs<AHEAD> p) {
   constexpr int NW = 4;
   constexpr int TN = 16 * FN, TM = 16 * FM;
   constexpr int BN = 2 * TN, BM = 2 * TM;
@@ -22,13 +25,16 @@ __global__ __launch_bounds__(256, (gp_per_cu<FN, FM, NA, NB>())) void gemm_pipe_
   const int wn = wave & 1, wm = wave >> 1;
   const int M = p.M, N = p.N, S = p.S;
   const int mblocks = (M + BM - 1) / BM, nblocks = N / BN;
-  const int tiles = AHEAD ? gridDim.x - p.ahead_wgs : gridDim.x;
-  if (AHEAD && (int)blockIdx.x >= tiles) {
-    const int at = (blockIdx.x - tiles) * NW + wave, n = p.ahead_wgs * NW;
-    gp_touch(p.ahead[0], p.ahead_bytes[0], lds + wave * 1024, at, n, lane);
-    gp_touch(p.ahead[1], p.ahead_bytes[1], lds + wave * 1024, at, n, lane);
-    gp_wait_vm<0>();
-    return;
+  int tiles = gridDim.x;
+  if constexpr (AHEAD) {
+    tiles -= p.ahead_wgs;
+    if ((int)blockIdx.x >= tiles) {
+      const int at = (blockIdx.x - tiles) * NW + wave, n = p.ahead_wgs * NW;
+      gp_touch(p.ahead[0], p.ahead_bytes[0], lds + wave * 1024, at, n, lane);
+      gp_touch(p.ahead[1], p.ahead_bytes[1], lds + wave * 1024, at, n, lane);
+      gp_wait_vm<0>();
+      return;
+    }
   }
   const int id = xcd_remap(blockIdx.x, tiles);
   const int s = id % S, tile = id / S;
@@ -124,7 +130,7 @@ __global__ __launch_bounds__(256, (gp_per_cu<FN, FM, NA, NB>())) void gemm_pipe_
 }
 
 template <int FN, int FM, int NA, int NB, bool AHEAD>
-static int gp_launch(const GemmSkParams& p, hipStream_t st) {
+static int gp_launch(const GemmSkCall& p, hipStream_t st) {
   constexpr int BN = 32 * FN, BM = 32 * FM;
   if (p.N % BN || p.K % SK_BK || p.S > p.K / SK_BK) return (int)hipErrorInvalidValue;
   // 32-bit buffer offsets: a tile's rows of X, and all of W (SwiGLU: its other half)
@@ -137,7 +143,7 @@ static int gp_launch(const GemmSkParams& p, hipStream_t st) {
       return (int)hipErrorInvalidValue;
   const long long grid = (long long)((p.M + BM - 1) / BM) * (p.N / BN) * p.S + p.ahead_wgs;
   if (grid > 0x7fffffff) return (int)hipErrorInvalidValue;
-#define GO(EPI) hipLaunchKernelGGL((gemm_pipe_kernel<FN, FM, NA, NB, EPI, AHEAD>), dim3(grid), dim3(256), 0, st, p)
+#define GO(EPI) hipLaunchKernelGGL((gemm_pipe_kernel<FN, FM, NA, NB, EPI, AHEAD>), dim3(grid), dim3(256), 0, st, static_cast<const GpArgs<AHEAD>&>(p))
   switch (p.epi) {
     case SK_SWIGLU: GO(SK_SWIGLU); break;
     case SK_RESID: GO(SK_RESID); break;
@@ -150,7 +156,7 @@ static int gp_launch(const GemmSkParams& p, hipStream_t st) {
 
 // (features x rows), stages of W and X; the smaller tiles spend the LDS on deeper rings, as
 // what they wait for is the first touch of cold weights
-template <bool AHEAD> static int gp_layout(const GemmSkParams& p, int layout, hipStream_t st) {
+template <bool AHEAD> static int gp_layout(const GemmSkCall& p, int layout, hipStream_t st) {
   switch (layout) {
     case 0: return gp_launch<8, 8, 3, 2, AHEAD>(p, st);   // 256 x 256
     case 1: return gp_launch<8, 6, 3, 2, AHEAD>(p, st);   // 256 x 192

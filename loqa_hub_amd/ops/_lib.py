@@ -66,7 +66,7 @@ class GemmTileParams(ctypes.Structure):
 
 
 class GemmSkParams(ctypes.Structure):
-    """Mirror of ``GemmSkParams`` in csrc/kernels/gemm_sk.hip."""
+    """Mirror of ``GemmSkCall`` in csrc/kernels/gemm_sk.h."""
     _fields_ = [
         ("x", c_void_p), ("ldx", c_ll), ("w", c_void_p),
         ("M", c_int), ("N", c_int), ("K", c_int), ("S", c_int),
