@@ -32,8 +32,12 @@
 // question) bring the weights of later launches into the Infinity Cache.
 #include "gemm_pipe_tile.h"
 
-int gemm_pipe_ahead(const GemmSkCall& p, int layout, hipStream_t st);   // gemm_pipe_ahead.hip
+// gemm_pipe_ahead.hip, gemm_pipe_split.hip, gemm_pipe_split_ahead.hip
+int gemm_pipe_ahead(const GemmSkCall& p, int layout, hipStream_t st);
+int gemm_pipe_split(const GemmSkCall& p, int layout, hipStream_t st);
+int gemm_pipe_split_ahead(const GemmSkCall& p, int layout, hipStream_t st);
 
 int gemm_pipe(const GemmSkCall& p, int layout, hipStream_t st) {
-  return p.ahead_wgs ? gemm_pipe_ahead(p, layout, st) : gp_layout<false>(p, layout, st);
+  if (p.S > 1) return p.ahead_wgs ? gemm_pipe_split_ahead(p, layout, st) : gemm_pipe_split(p, layout, st);
+  return p.ahead_wgs ? gemm_pipe_ahead(p, layout, st) : gp_layout<false, false>(p, layout, st);
 }

@@ -2,4 +2,4 @@
 // of later launches.
 #include "gemm_pipe_tile.h"
 
-int gemm_pipe_ahead(const GemmSkCall& p, int layout, hipStream_t st) { return gp_layout<true>(p, layout, st); }
+int gemm_pipe_ahead(const GemmSkCall& p, int layout, hipStream_t st) { return gp_layout<true, false>(p, layout, st); }

@@ -1,0 +1,57 @@
+"""K chunks of the pipelined tiles (csrc/kernels/gemm_pipe_tile.h): every workgroup of a tile sums up
+its share of it, the last to arrive those that others gave up."""
+import pytest
+import torch
+
+from loqa_hub_amd import ops
+
+
+def _close(a, b, k):
+    # as in test_gemm_pipe.py: half a bf16 ulp of the value, and the f32 sum's own rounding
+    tol = 2.0 ** -8 * b.abs() + (k * 2.0 ** -22 + 2.0 ** -9) * b.std()
+    assert torch.all((a.double() - b).abs() <= tol), ((a.double() - b).abs() - tol).max().item()
+
+
+def _words_are_zero():
+    torch.cuda.synchronize()
+    assert all(int(cnt.abs().sum()) == 0 for _, cnt in ops._SK_WS.values())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", [k for k in sorted(ops.SK_LAYOUTS) if k >= ops.SK_PIPE])
+@pytest.mark.parametrize("splits", [2, 3, 4, 5, 8, 9, 14])
+def test_shares_of_a_tile(layout, splits):
+    """More chunks than units of 16 x 16 in a share divide evenly, more than SK_SHARE, ragged rows, every epilogue."""
+    bn, bm = ops.SK_LAYOUTS[layout][:2]
+    K, N, M = 64 * 14, 2 * bn, bm + 21
+    g = torch.Generator().manual_seed(layout)
+    x = torch.randn(M, K, generator=g).bfloat16().cuda()
+    w = (torch.randn(N, K, generator=g) / 16).bfloat16().cuda()
+    b = torch.randn(N, generator=g).cuda()
+    ref = x.double() @ w.double().t()
+    first = ops.gemm_sk(x, w, bias=b, layout=layout, splits=splits)
+    _close(first, ref + b.double(), K)
+    assert torch.equal(ops.gemm_sk(x, w, bias=b, layout=layout, splits=splits), first)
+    z = ref + b.double()
+    _close(ops.gemm_sk(x, w, bias=b, act="gelu", layout=layout, splits=splits), 0.5 * z * torch.erfc(-z * 0.5 ** 0.5), K)
+    res = torch.randn(M, N, generator=g).bfloat16().cuda()
+    want = res.double() + z
+    _close(ops.gemm_sk(x, w, epi="resid", bias=b, residual=res, layout=layout, splits=splits), want, K)
+    h = ref[:, :bn]
+    _close(ops.gemm_sk(x, w, epi="swiglu", layout=layout, splits=splits), h * torch.sigmoid(h) * ref[:, bn:], K)
+    _words_are_zero()
+
+
+@pytest.mark.gpu
+def test_a_chunk_that_starts_a_round_later():
+    """300 workgroups of one a compute unit: chunks of one tile in different rounds, longer apart than a workgroup
+    waits, so that shares are given up."""
+    g = torch.Generator().manual_seed(1)
+    K = 64 * 180
+    x = torch.randn(2500, K, generator=g).bfloat16().cuda()
+    w = (torch.randn(2560, K, generator=g) / 64).bfloat16().cuda()
+    first = ops.gemm_sk(x, w, layout=12, splits=3)
+    _close(first, x.double() @ w.double().t(), K)
+    for _ in range(3):
+        assert torch.equal(ops.gemm_sk(x, w, layout=12, splits=3), first)
+    _words_are_zero()
