@@ -373,7 +373,7 @@ __device__ __forceinline__ void attn_decode_body(const AttnDecArgs& A, const int
       }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    int* cnt = counters + (size_t)b * Hkv + kvh;
+    int* cnt = counters + ((size_t)b * Hkv + kvh) * TICKET;
     if (lane == 0) {
       const int t = __hip_atomic_fetch_add(cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       if (t == nsplit - 1) __hip_atomic_store(cnt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

@@ -46,7 +46,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void attn_decode_kernel(AttnDecArgs a
 
 // q: [Tq, >=Hq*D] bf16; K/V paged caches [nb, Hkv, blk, D] (block_tables) or
 // contiguous rows (kv_stride, kv_start); out [Tq, Hq*D] bf16.
-// Requires G * max_q <= 32 and split_keys % 32 == 0; counters: >= B * Hkv zeroed ints
+// Requires G * max_q <= 32 and split_keys % 32 == 0; counters: >= B * Hkv zeroed tickets
 // (left zeroed); paged blk a power of two >= 16.
 extern "C" int loqa_attn_decode(const void* q, long long q_stride, const void* kc, const void* vc,
                                 long long kv_stride, const int* kv_start, void* o,

@@ -22,6 +22,10 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 #define WAVE 64
 
+// ints from one arrival ticket to the next: a cache line each, as the atomics of a launch's workgroups on
+// one line queue up behind each other (256 of them 5 us)
+#define TICKET 32
+
 __device__ __forceinline__ float bf2f(bf16_t h) {
   return __uint_as_float(((uint32_t)h) << 16);
 }

@@ -25,7 +25,6 @@ template <bool AHEAD> using GpArgs = std::conditional_t<AHEAD, GemmSkCall, GemmS
 #define SK_KEEP 4
 #define SK_SHARE 8
 #define SK_POLLS 48
-#define SK_WORD 32                    // ints from one tile's word to the next
 #define SK_SC1 16                     // buffer cache policy: device scope
 
 template <int NW, int FN, int FM>
@@ -158,7 +157,7 @@ __device__ __forceinline__ void sk_finish(const GemmSkParams& p, float4v (&acc)[
     }
     __builtin_amdgcn_sched_barrier(0);
   }
-  int* word = p.counters + tile * SK_WORD;
+  int* word = p.counters + tile * TICKET;
   const unsigned mine = sk_shares(word, S, s, reinterpret_cast<int*>(lds + BYTES - 16), [&]() {
     for (int u = u0; u < u1; ++u)
 #pragma unroll

@@ -15,7 +15,7 @@ struct GemmSkParams {
   const float* bias;              // [N] f32 or null (SK_BF16, SK_RESID)
   void* y; long long ldy;         // bf16 output (SK_RESID: the residual, updated in place)
   float* ws;                      // S > 1: [tiles][S][BM * BN] f32 partials
-  int* counters;                  // S > 1: [tiles] ints, zero on entry (left zero)
+  int* counters;                  // S > 1: [tiles] tickets, zero on entry (left zero)
   int layout;
   int ahead_wgs;                  // workgroups behind the tiles' that only touch what follows (pipelined tiles)
 };
@@ -86,9 +86,9 @@ __device__ __forceinline__ bool sk_reduce(const GemmSkParams& p, float4v (&acc)[
   if (threadIdx.x == 0) {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    const int t = __hip_atomic_fetch_add(p.counters + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const int t = __hip_atomic_fetch_add(p.counters + tile * TICKET, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const int last = t == S - 1;
-    if (last) __hip_atomic_store(p.counters + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (last) __hip_atomic_store(p.counters + tile * TICKET, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     *flag = last;
   }
   __syncthreads();

@@ -748,19 +748,19 @@ __device__ __forceinline__ void skinny_fused_tile(const FusedArgs& a, float* sme
     if constexpr (WR > 1) {
       int t = 0;
       if (lane == 0) {
-        t = __hip_atomic_fetch_add(&a.counters[tile], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        t = __hip_atomic_fetch_add(&a.counters[tile * TICKET], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (t == a.S - 1)
-          __hip_atomic_store(&a.counters[tile], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          __hip_atomic_store(&a.counters[tile * TICKET], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
       t = __shfl(t, 0, 64);
       if (t != a.S - 1) return;
     } else {
       __syncthreads();
       if (threadIdx.x == 0) {
-        const int t = __hip_atomic_fetch_add(&a.counters[tile], 1, __ATOMIC_RELAXED,
+        const int t = __hip_atomic_fetch_add(&a.counters[tile * TICKET], 1, __ATOMIC_RELAXED,
                                              __HIP_MEMORY_SCOPE_AGENT);
         if (t == a.S - 1)
-          __hip_atomic_store(&a.counters[tile], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          __hip_atomic_store(&a.counters[tile * TICKET], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         sred[0] = (float)t;
       }
       __syncthreads();
@@ -1269,7 +1269,7 @@ static int fused_prologue(const FusedParams* p, FusedArgs& a, hipStream_t st) {
 // (act 0 identity, 1 GELU-erf). norm: 1 RMSNorm / 2 LayerNorm of x (the bf16
 // residual) with the norm weight folded into Wp; the row statistics come from
 // rowstat_tiles partial sums. part: S * Mpad * N f32 scratch (S > 1,
-// tile-contiguous slabs); counters: >= N/(16*rt) zeroed ints. Row statistics of
+// tile-contiguous slabs); counters: >= N/(16*rt) zeroed tickets. Row statistics of
 // the residual epilogue are written per (16*rt)-row tile.
 extern "C" int loqa_skinny_fused(const FusedParams* p, hipStream_t st) {
   const int Mpad = p->Mpad, N = p->N, K = p->K, S = p->S;

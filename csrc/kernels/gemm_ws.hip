@@ -50,7 +50,7 @@ struct GemmWsParams {
   int bm;                         // rows per workgroup (multiple of 64, <= 64 * FM of the launch)
   int S;                          // K chunks (>= 1)
   float* ws;                      // S > 1: [tiles][S][bm * 128] f32 partials
-  int* counters;                  // S > 1: [tiles] ints, zero on entry (left zero)
+  int* counters;                  // S > 1: [tiles] tickets, zero on entry (left zero)
 };
 
 template <int N>
@@ -227,9 +227,9 @@ __global__ __launch_bounds__(512) void gemm_ws_kernel(GemmWsParams p) {
     if (threadIdx.x == 0) {
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      const int t = __hip_atomic_fetch_add(p.counters + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const int t = __hip_atomic_fetch_add(p.counters + tile * TICKET, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       const int last = t == S - 1;
-      if (last) __hip_atomic_store(p.counters + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (last) __hip_atomic_store(p.counters + tile * TICKET, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       *flag = last;
     }
     __syncthreads();

@@ -157,6 +157,11 @@ def rope_kv_append(qkv: torch.Tensor, positions: torch.Tensor | None, cos_sin: t
 
 
 # ----------------------------------------------------------------- attention
+def _tickets(n: int, device) -> torch.Tensor:
+    """``n`` zeroed arrival tickets, a cache line apart (TICKET of csrc/kernels/common.h)."""
+    return torch.zeros(n, 32, dtype=torch.int32, device=device)[:, 0]
+
+
 class AttnWorkspace:
     """Split-K partial buffers for grouped decode attention (allocated once per
     engine so the decode step stays graph-capturable)."""
@@ -169,7 +174,7 @@ class AttnWorkspace:
                                    device=device)
         # split-arrival tickets of the decode kernel's in-launch combine, one per
         # (sequence, kv head); the last arriving split resets its counter
-        self.counters = torch.zeros(max_tokens * n_heads, dtype=torch.int32, device=device)
+        self.counters = _tickets(max_tokens * n_heads, device)
 
 
 # decode attention (attn_decode.hip): splits of at least this many keys run on
@@ -1067,7 +1072,7 @@ class FusedScratch:
     def __init__(self, device, max_tiles: int = 8192, max_rows: int = 128):
         # max_rows = the largest Mpad (128): the 70B gate|up at Mpad 128 has
         # 3584 row tiles x 128 rows of statistics
-        self.counters = torch.zeros(max_tiles, dtype=torch.int32, device=device)
+        self.counters = _tickets(max_tiles, device)
         self.rowsq = torch.zeros(max_tiles * max_rows, dtype=torch.float32, device=device)
         self.rowsum = torch.zeros(max_tiles * max_rows, dtype=torch.float32, device=device)
         self.stat_tiles = 0   # partial tiles written by the last residual epilogue
@@ -1690,7 +1695,6 @@ SK_WHOLE = 12             # the layout that the plan does not split along K
 SK_RENAMED = {0: 20, 2: 19, 3: 15, 4: 19, 5: 20, 6: 12, 8: 19, 9: 15, 10: 20, 11: 19}
 SK_CUS = 256
 SK_FEW = 96
-SK_WORD = 32              # the pipelined tiles' arrival words are a cache line apart (gemm_pipe_tile.h)
 _SK_WS: dict = {}
 
 
@@ -1744,7 +1748,7 @@ def _sk_workspace(dev: torch.device, stream: int, floats: int, tiles: int):
     and two graphs replayed on different streams would race on it."""
     if dev.type == "cuda" and torch.cuda.is_current_stream_capturing():
         ws = (torch.empty(floats, dtype=torch.float32, device=dev),
-              torch.zeros(tiles, dtype=torch.int32, device=dev))
+              _tickets(tiles, dev))
         _SK_WS_GRAPHS.append(ws)
         return ws
     key = (dev, stream)
@@ -1753,7 +1757,7 @@ def _sk_workspace(dev: torch.device, stream: int, floats: int, tiles: int):
         f = max(floats, 0 if ws is None else ws[0].numel())
         t = max(tiles, 0 if ws is None else ws[1].numel())
         ws = (torch.empty(f, dtype=torch.float32, device=dev),
-              torch.zeros(t, dtype=torch.int32, device=dev))
+              _tickets(t, dev))
         _SK_WS[key] = ws
     return ws
 
@@ -1882,7 +1886,7 @@ def gemm_sk(x: torch.Tensor, w: torch.Tensor, *, epi: str = "bf16", bias: torch.
     st = stream_ptr(x)
     if splits > 1:
         tiles = -(-M // bm) * (N // bn)
-        ws, cnt = _sk_workspace(x.device, st, tiles * splits * bm * bn, tiles * (SK_WORD if layout >= SK_PIPE else 1))
+        ws, cnt = _sk_workspace(x.device, st, tiles * splits * bm * bn, tiles)
         p.ws, p.counters = ptr(ws), ptr(cnt)
     p.layout = layout
     if ahead and layout >= SK_PIPE:
