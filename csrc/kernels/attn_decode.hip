@@ -22,6 +22,10 @@
 // Paged block-table entries are wave-uniform per 32-key tile (tiles are
 // 32-aligned, blk is a power of two >= 16), so they are scalar loads and the
 // K/V addresses need no per-lane dependent lookup.
+//
+// Up to 16 query rows per kv head run on attn_stream.hip; this form serves 17 to 32 rows, operands off 16
+// bytes, the 8-wave and prefetching variants where they are asked for, and the attention inside the
+// fused launches of gemm_skinny.hip.
 #include "attn_decode.h"
 
 thread_local int g_loqa_launch_prio = 0;
@@ -48,6 +52,8 @@ __global__ __launch_bounds__(NW * 64, OCC) void attn_decode_kernel(AttnDecArgs a
 // contiguous rows (kv_stride, kv_start); out [Tq, Hq*D] bf16.
 // Requires G * max_q <= 32 and split_keys % 32 == 0; counters: >= B * Hkv zeroed tickets
 // (left zeroed); paged blk a power of two >= 16.
+bool attn_stream(AttnDecArgs a, int B, int max_q, int D, hipStream_t st, int* err);   // attn_stream.hip
+
 extern "C" int loqa_attn_decode(const void* q, long long q_stride, const void* kc, const void* vc,
                                 long long kv_stride, const int* kv_start, void* o,
                                 long long o_stride, const int* cu_q, const int* ctx_lens,
@@ -68,6 +74,8 @@ extern "C" int loqa_attn_decode(const void* q, long long q_stride, const void* k
                       split_keys, num_splits, part_o, part_ml, total_q, counters, (bf16_t*)o,
                       o_stride, 0, 0, g_loqa_launch_prio, 0};
   if (waves != 4 && waves != 8) return (int)hipErrorInvalidValue;
+  int err = 0;
+  if (waves == 4 && !pf && attn_stream(a, B, max_q, D, s, &err)) return err;
   if (waves == 8) {   // 512 threads: 2 waves per SIMD, 256 registers each (no PF at D = 128)
     if (D == 128)
       hipLaunchKernelGGL((attn_decode_kernel<128, 0, 8, 1>), grid, dim3(512), 0, s, a);

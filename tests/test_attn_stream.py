@@ -1,0 +1,113 @@
+"""Decode attention streamed through LDS (csrc/kernels/attn_stream.hip): tiles of 32 keys and their
+remainders, pages of every size, groups of heads up to 16 rows, splits taken together."""
+import math
+
+import pytest
+import torch
+
+from loqa_hub_amd import ops
+
+
+def _reference(q, ks, vs, qlens, H, G, D, causal):
+    """64 bits; ks, vs per sequence [keys, Hkv, D]."""
+    out, at = [], 0
+    for k, v, n in zip(ks, vs, qlens):
+        x = q[at:at + n].double().view(n, H, D)
+        s = torch.einsum("thd,lhd->htl", x, k.double().repeat_interleave(G, 1)) * D ** -0.5
+        if causal:
+            seen = torch.arange(k.shape[0], device=q.device)[None] <= torch.arange(k.shape[0] - n, k.shape[0], device=q.device)[:, None]
+            s = s.masked_fill(~seen[None], -math.inf)
+        out.append(torch.einsum("htl,lhd->thd", torch.softmax(s, -1), v.double().repeat_interleave(G, 1)).flatten(1))
+        at += n
+    return torch.cat(out)
+
+
+def _close(a, b):
+    # weights rounded to bf16 (2^-9 of each) and a bf16 result: 2^-8 of the values that the weights average
+    assert (a.double() - b).abs().max() <= 2.0 ** -7 * b.abs().max(), ((a.double() - b).abs().max(), b.abs().max())
+    assert (a.double() - b).norm() <= 4e-3 * b.norm()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,G,blk", [(64, 1, 16), (64, 4, 32), (64, 16, 64), (128, 1, 128), (128, 4, 16), (128, 3, 16), (128, 8, 64)])
+@pytest.mark.parametrize("keys", [1, 31, 33, 129, 300, 1030])
+def test_paged(D, G, blk, keys):
+    Hkv, g = 2, torch.Generator().manual_seed(keys + D)
+    H = Hkv * G
+    most = 16 // G
+    lens, qlens = [keys, max(1, keys - 17), min(keys, 5)], [1, min(most, max(1, keys - 17)), 1]
+    need = [-(-n // blk) for n in lens]
+    order = torch.randperm(sum(need) + 2, generator=g)
+    kc, vc = (torch.randn(sum(need) + 2, Hkv, blk, D, generator=g).bfloat16().cuda() for _ in range(2))
+    bt, at = torch.zeros(3, max(need), dtype=torch.int32), 0
+    for b, n in enumerate(need):
+        bt[b, :n] = order[at:at + n]
+        at += n
+    def rows(c):
+        return [c[bt[b, :need[b]].long().cuda()].transpose(1, 2).reshape(-1, Hkv, D)[:lens[b]] for b in range(3)]
+    q = torch.randn(sum(qlens), H * D, generator=g).bfloat16().cuda()
+    cu = torch.tensor([0, qlens[0], qlens[0] + qlens[1], sum(qlens)], dtype=torch.int32).cuda()
+    ref = _reference(q, rows(kc), rows(vc), qlens, H, G, D, True)
+    kw = dict(n_heads=H, n_kv=Hkv, head_dim=D, causal=True, max_q=max(qlens), ctx_lens=torch.tensor(lens, dtype=torch.int32).cuda(),
+              block_tables=bt.cuda(), grouped=True)
+    for split in (32, 128, 256):
+        ns = -(-max(lens) // split)
+        ws = ops.AttnWorkspace("cuda", 64, H, D, ns + 1)
+        for more in (0, 1):                       # as many splits as there are keys for, and one more
+            y = ops.attention(q, kc, vc, cu, split_keys=split, num_splits=ns + more, workspace=ws, **kw)
+            _close(y, ref)
+            assert torch.equal(y, ops.attention(q, kc, vc, cu, split_keys=split, num_splits=ns + more, workspace=ws, **kw))
+        assert int(ws.counters.abs().sum()) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("B,T", [(1, 1500), (3, 50), (40, 333)])
+def test_rows_in_place(D, B, T):
+    """Key and value columns of one matrix, utterances in another order than their rows, lengths of their own; the general
+    kernel (8 waves; queries off 16 bytes) beside it."""
+    H, g = 4, torch.Generator().manual_seed(B)
+    kv = torch.randn(B * T, 2 * H * D, generator=g).bfloat16().cuda()
+    who = torch.randperm(B, generator=g)
+    lens = [T - 3 * i % T for i in range(B)]
+    q = torch.randn(B, H * D + 4, generator=g).bfloat16().cuda()
+    rows = [kv[b * T:b * T + n].view(n, 2, H, D) for b, n in zip(who.tolist(), lens)]
+    cu = torch.arange(B + 1, dtype=torch.int32).cuda()
+    starts, ctx = (who * T).int().cuda(), torch.tensor(lens, dtype=torch.int32).cuda()
+    ws = ops.AttnWorkspace("cuda", 64, H, D, 8)
+
+    def run(x):
+        return ops.attention(x, kv, kv[:, H * D:], cu, n_heads=H, n_kv=H, head_dim=D, causal=False, max_q=1, cu_k=starts, ctx_lens=ctx,
+                             grouped=True, split_keys=256, num_splits=-(-T // 256), workspace=ws)
+    x = q[:, :H * D].contiguous()
+    ref = _reference(x, [r[:, 0] for r in rows], [r[:, 1] for r in rows], [1] * B, H, 1, D, False)
+    _close(run(x), ref)
+    _close(run(q[:, :H * D]), ref)                # rows 8 bytes off: the general kernel
+    assert int(ws.counters.abs().sum()) == 0
+
+
+@pytest.mark.gpu
+def test_replays_of_a_captured_call():
+    """The grid is made for the longest context, later contexts are shorter and longer."""
+    D, H, Hkv, blk = 128, 8, 2, 16
+    g = torch.Generator().manual_seed(2)
+    kc, vc = (torch.randn(40, Hkv, blk, D, generator=g).bfloat16().cuda() for _ in range(2))
+    bt = torch.randperm(40, generator=g)[None].int().cuda()
+    q, ctx = torch.randn(1, H * D, generator=g).bfloat16().cuda(), torch.tensor([640], dtype=torch.int32).cuda()
+    cu, ws = torch.tensor([0, 1], dtype=torch.int32).cuda(), ops.AttnWorkspace("cuda", 16, H, D, 5)
+
+    def run():
+        return ops.attention(q, kc, vc, cu, n_heads=H, n_kv=Hkv, head_dim=D, causal=True, max_q=1, ctx_lens=ctx, block_tables=bt,
+                             grouped=True, split_keys=128, num_splits=5, workspace=ws)
+    run()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = run()
+    for n in (640, 1, 129, 600, 32):
+        ctx.fill_(n)
+        graph.replay()
+        torch.cuda.synchronize()
+        rows = [c[bt[0].long()].transpose(1, 2).reshape(-1, Hkv, D)[:n] for c in (kc, vc)]
+        _close(y, _reference(q, [rows[0]], [rows[1]], [1], H, H // Hkv, D, True))
+        assert torch.equal(y, run())
