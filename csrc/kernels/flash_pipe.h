@@ -77,35 +77,54 @@ template <int D, int NTH, bool ISV, bool PAD> struct FlFetch {
   static_assert(N * NTH == FL_KEYS * CH, "whole chunks per thread");
   int th, cols;
   unsigned st;                         // stride of the rows in bytes (64 st < 2^32)
-  __device__ __forceinline__ int row(int i) const { return NTH % CH == 0 ? th / CH + i * (NTH / CH) : (th + i * NTH) / CH; }
-  __device__ __forceinline__ int chunk(int i) const {
-    const int r = row(i);
-    return ((th + i * NTH) - r * CH) ^ (ISV ? fl_vswz<D>(r) : fl_kswz<D>(r));
+  __device__ __forceinline__ int row(int i, int t) const { return NTH % CH == 0 ? t / CH + i * (NTH / CH) : (t + i * NTH) / CH; }
+  __device__ __forceinline__ int chunk(int i, int t) const {
+    const int r = row(i, t);
+    return ((t + i * NTH) - r * CH) ^ (ISV ? fl_vswz<D>(r) : fl_kswz<D>(r));
+  }
+  // th once more, for what the last tile alone computes and no register should hold before
+  __device__ __forceinline__ int late() const {
+    int t = th;
+    asm volatile("" : "+v"(t));
+    return t;
   }
   __device__ __forceinline__ FlFetch(int th_, int cols_, long long stride) : th(th_), cols(cols_), st((unsigned)stride * 2) {}
   __device__ __forceinline__ unsigned dst(unsigned stage) const { return __builtin_amdgcn_readfirstlane(stage + (th & ~63) * 16); }
+  // A whole tile has its own branch: the rows' clamp, as selects in every tile, was 20 to 40 vector instructions
+  // of a tile's 180, a multiplication of four times the length per load among them.
   // rows at the stride, from the tile's first (wave-uniform)
   __device__ __forceinline__ void strided(unsigned stage, const bf16_t* base, int last) const {
     const unsigned d = dst(stage);
+    if (last >= FL_KEYS - 1) {
 #pragma unroll
-    for (int i = 0; i < N; ++i) {
-      unsigned off = (unsigned)row(i) * st + chunk(i) * 16;
-      if (last < FL_KEYS - 1) off -= (unsigned)max(row(i) - last, 0) * st;
-      if (!PAD || chunk(i) * 8 < cols) fl_load_lds(base, off, d + i * NTH * 16);
+      for (int i = 0; i < N; ++i)
+        if (!PAD || chunk(i, th) * 8 < cols) fl_load_lds(base, (unsigned)row(i, th) * st + chunk(i, th) * 16, d + i * NTH * 16);
+    } else {
+      const int t = late();
+#pragma unroll
+      for (int i = 0; i < N; ++i)
+        if (!PAD || chunk(i, t) * 8 < cols) fl_load_lds(base, (unsigned)min(row(i, t), last) * st + chunk(i, t) * 16, d + i * NTH * 16);
     }
   }
   // rows in pages of a multiple of RG: at(r), called with wave-uniform multiples of RG, the first of RG rows
   template <typename At> __device__ __forceinline__ void paged(unsigned stage, int last, At&& at) const {
     static_assert(64 % CH == 0, "whole rows per instruction");
     const unsigned d = dst(stage);
-    const int w0 = __builtin_amdgcn_readfirstlane(th & ~63) / CH, in = (th & 63) / CH;
+    const int w0 = __builtin_amdgcn_readfirstlane(th & ~63) / CH;
+    if (last >= FL_KEYS - 1) {
 #pragma unroll
-    for (int i = 0; i < N; ++i) {
-      const int r = min(w0 + i * (NTH / CH), last & ~(RG - 1));
-      const bf16_t* base = at(r);
-      unsigned off = (unsigned)in * st + chunk(i) * 16;
-      if (last < FL_KEYS - 1) off -= (unsigned)max(in - (last - r), 0) * st;
-      if (!PAD || chunk(i) * 8 < cols) fl_load_lds(base, off, d + i * NTH * 16);
+      for (int i = 0; i < N; ++i) {
+        const bf16_t* base = at(w0 + i * (NTH / CH));
+        if (!PAD || chunk(i, th) * 8 < cols) fl_load_lds(base, (unsigned)((th & 63) / CH) * st + chunk(i, th) * 16, d + i * NTH * 16);
+      }
+    } else {
+      const int t = late(), in = (t & 63) / CH;
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        const int r = min(w0 + i * (NTH / CH), last & ~(RG - 1));
+        const bf16_t* base = at(r);
+        if (!PAD || chunk(i, t) * 8 < cols) fl_load_lds(base, (unsigned)min(in, last - r) * st + chunk(i, t) * 16, d + i * NTH * 16);
+      }
     }
   }
 };
