@@ -39,6 +39,23 @@ def test_rows_against_float64(n_mels, samples):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("B,samples", [(1, 16 * 160 * 256), (1, 16 * 160 * 256 + 160), (7, 48 * 2560 + 800), (300, 400)])
+def test_workgroups_that_take_several_groups_of_frames(B, samples):
+    c = ref.MelConstants.create(80)
+    x = torch.from_numpy(0.1 * np.random.RandomState(samples).randn(B, samples)).float()
+    x *= torch.logspace(0, -2, B)[:, None]                # utterances of different maxima
+    frames = samples // 160
+    st = torch.stft(x.double(), 400, 160, window=c.window.double(), return_complex=True, center=True, pad_mode="reflect")
+    lg = (c.filters.double() @ st[..., :frames].abs().square()).clamp(min=1e-10).log10()
+    want = ((torch.maximum(lg, lg.amax((1, 2), keepdim=True) - 8) + 4) / 4).transpose(1, 2)
+    for cols in (192, 83):                                # four columns a lane, and rows that are not aligned
+        rows = ops.log_mel_rows(x.cuda(), c, cols).cpu().view(B, frames, cols)
+        # the bound of the test above
+        assert (rows[..., :80].double() - want).abs().max() <= 2.0 ** -8 * want.abs().clamp(min=1).max() + 1e-3
+        assert (rows[..., 80:] == 0).all()
+
+
+@pytest.mark.gpu
 def test_encoder_of_80_bands_on_the_tiled_path(monkeypatch):
     from loqa_hub_amd.models import whisper as wm
     from loqa_hub_amd.models.configs import whisper_config
