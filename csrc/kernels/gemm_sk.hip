@@ -214,3 +214,11 @@ extern "C" int loqa_gemm_sk(const GemmSkCall* p, hipStream_t st) {
     default: return gemm_pipe(*p, p->layout - 12, st);
   }
 }
+
+// The capture that `st` records into (unique in the process), for workspaces that its launches share.
+extern "C" int loqa_capture_id(hipStream_t st, unsigned long long* id) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  const hipError_t e = hipStreamGetCaptureInfo(st, &status, id);
+  if (e != hipSuccess) return (int)e;
+  return status == hipStreamCaptureStatusActive ? 0 : (int)hipErrorInvalidValue;
+}

@@ -1736,20 +1736,28 @@ def _sk_plan(M: int, N: int, K: int, pipe: bool, layouts: tuple | None = None) -
     return best
 
 
-_SK_WS_GRAPHS: list = []   # workspaces owned by captured graphs (never reused)
+_SK_WS_GRAPHS: list = []   # workspaces of captured graphs: they live as long as the process
+_SK_WS_CAPTURE: dict = {}  # (device, stream) -> (id of its newest capture, workspace)
 
 
 def _sk_workspace(dev: torch.device, stream: int, floats: int, tiles: int):
     """Split-K partials + arrival counters (zero on entry; each tile's reducer
     re-zeroes its own). Eager launches share one growing workspace per stream
-    (stream order serialises them). A launch being CAPTURED gets a workspace of
-    its own that lives as long as the process: a shared one could be regrown
-    by a later capture, freeing memory an earlier graph still replays into,
-    and two graphs replayed on different streams would race on it."""
+    (stream order serialises them). So do the launches that one capture records on
+    one stream: the graph then clears the tickets once, not before each launch
+    (2.5 us each: 32 of them are 2 % of a pass of Whisper's large encoder). No
+    two captures share one: it could be regrown by a later capture, freeing memory
+    an earlier graph still replays into, and two graphs replayed on different
+    streams would race on it."""
     if dev.type == "cuda" and torch.cuda.is_current_stream_capturing():
-        ws = (torch.empty(floats, dtype=torch.float32, device=dev),
-              _tickets(tiles, dev))
-        _SK_WS_GRAPHS.append(ws)
+        cid = ctypes.c_uint64()
+        check(kernels().loqa_capture_id(stream, ctypes.byref(cid)), "capture_id")
+        held, ws = _SK_WS_CAPTURE.get((dev, stream), (None, None))
+        if held != cid.value or ws[0].numel() < floats or ws[1].numel() < tiles:
+            ws = (torch.empty(floats, dtype=torch.float32, device=dev),
+                  _tickets(tiles, dev))
+            _SK_WS_GRAPHS.append(ws)
+            _SK_WS_CAPTURE[(dev, stream)] = (cid.value, ws)
         return ws
     key = (dev, stream)
     ws = _SK_WS.get(key)

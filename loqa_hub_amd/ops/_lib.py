@@ -125,6 +125,7 @@ _KERNEL_SIGS = {
     "loqa_skinny_fused": [c_void_p, c_void_p],
     "loqa_gemm_tile": [c_void_p, c_void_p],
     "loqa_gemm_sk": [c_void_p, c_void_p],
+    "loqa_capture_id": [c_void_p, c_void_p],
     "loqa_conv_pipe": [c_void_p, c_void_p],
     "loqa_gemm_ws": [c_void_p, c_int, c_void_p],
     "loqa_attn_decode": [c_void_p, c_ll, c_void_p, c_void_p, c_ll, c_void_p, c_void_p, c_ll,

@@ -55,3 +55,35 @@ def test_a_chunk_that_starts_a_round_later():
     for _ in range(3):
         assert torch.equal(ops.gemm_sk(x, w, layout=12, splits=3), first)
     _words_are_zero()
+
+
+@pytest.mark.gpu
+def test_launches_of_a_capture_share_a_workspace():
+    """Two graphs, each with a launch that outgrows the first one's partials: their own memory, and every
+    replay, on two streams at once, equal to the eager result."""
+    g = torch.Generator().manual_seed(2)
+    K = 64 * 24
+    x = torch.randn(300, K, generator=g).bfloat16().cuda()
+    ws = [(torch.randn(n, K, generator=g) / 16).bfloat16().cuda() for n in (256, 1024, 256)]
+    run = lambda: [ops.gemm_sk(x, w, layout=15, splits=3) for w in ws]      # noqa: E731
+    want = run()
+    graphs, outs = [], []
+    for _ in range(2):
+        n = len(ops._SK_WS_GRAPHS)
+        graphs.append(torch.cuda.CUDAGraph())
+        with torch.cuda.graph(graphs[-1]):
+            outs.append(run())
+        assert len(ops._SK_WS_GRAPHS) == n + 2                              # the first launch's, and the larger one's
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    for _ in range(5):
+        for out in outs:
+            for y in out:
+                y.fill_(7)
+        torch.cuda.synchronize()
+        for s, gr in zip(streams, graphs):
+            with torch.cuda.stream(s):
+                gr.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(y, z) for out in outs for y, z in zip(out, want))
+        assert all(torch.equal(y, z) for y, z in zip(run(), want))
+    assert all(int(cnt.abs().sum()) == 0 for _, cnt in ops._SK_WS_GRAPHS)
