@@ -1682,8 +1682,8 @@ _SK_EPI = {"bf16": 0, "swiglu": 1, "resid": 2}
 # fitted to measured ones without an epilogue of weight: they are there to rank, and 0.69 to 1.26
 # of what a whole unsplit call takes (0.73 on average with GELU). Over 60 shapes (80 to 9000 rows, N 512
 # to 28672, K 512 to 14336, cold weights, every layout and K split: profiles/gemm_plan_grid.txt)
-# the plan is the fastest in 49, 0.6 % behind the fastest on average and 7.3 % at worst (320 x 1280 x
-# 8192 in five chunks of 128 x 64: 20.4 us, 19.0 in eight of 128 x 128).
+# the plan is the fastest in 50, 0.7 % behind the fastest on average and 8.3 % at worst (1500 x 1280 x
+# 5120 whole on 128 x 64: 29.9 us, 27.6 in three chunks of 128 x 192).
 SK_LAYOUTS = {1: (128, 64, 0.60, 4.0), 7: (64, 64, 0.55, 4.0),
               12: (256, 256, 1.20, 10.3), 13: (256, 192, 1.075, 5.5), 14: (192, 256, 1.073, 5.5),
               15: (256, 128, 0.908, 4.0), 16: (128, 256, 0.784, 6.6), 17: (128, 192, 0.667, 4.6),
@@ -1695,6 +1695,7 @@ SK_WHOLE = 12             # the layout that the plan does not split along K
 SK_RENAMED = {0: 20, 2: 19, 3: 15, 4: 19, 5: 20, 6: 12, 8: 19, 9: 15, 10: 20, 11: 19}
 SK_CUS = 256
 SK_FEW = 96
+SK_WORTH = 1.03
 _SK_WS: dict = {}
 
 
@@ -1705,7 +1706,9 @@ def gemm_sk_plan(M: int, N: int, K: int, epi: str = "bf16", layouts=None, *,
     a K step takes 0.8 of its time (1500 x 512 x 2048 on 96 of them 11.0 us, in two chunks on 192 11.6).
     K chunks fill the chip where the tiles do not; each tile then pays for the trip of its f32 partials
     through memory, 2 us and 40 us a MB, and 4 us a MB for each chunk that is read back (fitted with the
-    rest; 320 x 4096 x 4096 in four chunks of 128 x 192 22.2 us, whole 27.3 in 128 x 64), and never on 256 x 256
+    rest; 320 x 4096 x 4096 in four chunks of 128 x 192 22.2 us, whole 27.3 in 128 x 64). They have to be faster by SK_WORTH:
+    their partials and the weights that a launch touches for the next one (:func:`_ahead`) hold each other up (1500 x
+    1280 x 5120 in two chunks 28.3 us and whole 29.9 alone, but an encoder pass with 32 of them 4118 us and 4058). Never on 256 x 256
     tiles: these fill the chip with MFMAs, where a K step takes longer than the fit has it (4096 x
     14336: 1280 rows in three chunks 160 us, the 256 x 192 tiles in two 135; 2048 rows in two 205,
     the 128 x 256 tiles whole 182; the fastest in none of the 60 shapes). ``pipe`` False:
@@ -1730,7 +1733,7 @@ def _sk_plan(M: int, N: int, K: int, pipe: bool, layouts: tuple | None = None) -
                 continue
             t = -(-tiles * s // SK_CUS) * (-(-KT // s) * step * (0.8 if tiles * s <= SK_FEW else 1.0) + around)
             if s > 1:
-                t += 2.0 + bn * bm * 4e-6 * (40 + 4 * s)
+                t = SK_WORTH * (t + 2.0 + bn * bm * 4e-6 * (40 + 4 * s))
             if t < best_t:
                 best, best_t = (lay, s), t
     return best
