@@ -316,8 +316,16 @@ static int gp_launch(const GemmSkCall& p, hipStream_t st) {
       return (int)hipErrorInvalidValue;
   const long long grid = (long long)((p.M + BM - 1) / BM) * (p.N / BN) * p.S + p.ahead_wgs;
   if (grid > 0x7fffffff) return (int)hipErrorInvalidValue;
+  // GELU costs a wave 20 vector instructions a value, 10 us at 256 x 256, with the matrix cores idle: from
+  // more tiles on than compute units, two stages of W and X instead of three fit two workgroups of 128
+  // x 192 on one, whose products run beside the other's epilogue (9000 x 2048 x 512 39.7 -> 33.0 us, 12000 x
+  // 3072 x 768 79.4 -> 70.5, 9000 x 5120 x 1280 129.3 -> 126.7, always against the best of the other tiles;
+  // without GELU 15 to 30 % slower than those)
+  if constexpr (FN == 4 && FM == 6 && NA == 3 && !AHEAD && !SPLIT)
+    if (p.act == 1 && grid > 256) return gp_launch<FN, FM, 2, 2, AHEAD, SPLIT>(p, st);
 #define GO(EPI) hipLaunchKernelGGL((gemm_pipe_kernel<FN, FM, NA, NB, EPI, AHEAD, SPLIT>), dim3(grid), dim3(256), 0, st, static_cast<const GpArgs<AHEAD>&>(p))
-  switch (p.epi) {
+  if constexpr (FN == 4 && FM == 6 && NA == 2) GO(SK_GELU);
+  else switch (p.epi) {
     case SK_SWIGLU: GO(SK_SWIGLU); break;
     case SK_RESID: GO(SK_RESID); break;
     default:

@@ -1696,6 +1696,8 @@ SK_RENAMED = {0: 20, 2: 19, 3: 15, 4: 19, 5: 20, 6: 12, 8: 19, 9: 15, 10: 20, 11
 SK_CUS = 256
 SK_FEW = 96
 SK_WORTH = 1.03
+SK_GELU = 1.3e-4
+SK_PAIRED = 17            # two workgroups a compute unit, with GELU
 _SK_WS: dict = {}
 
 
@@ -1713,14 +1715,19 @@ def gemm_sk_plan(M: int, N: int, K: int, epi: str = "bf16", layouts=None, *,
     14336: 1280 rows in three chunks 160 us, the 256 x 192 tiles in two 135; 2048 rows in two 205,
     the 128 x 256 tiles whole 182; the fastest in none of the 60 shapes). ``pipe`` False:
     the general layouts only (operands the pipelined tiles do not take). ``layouts``: among
-    these only (numbers of SK_LAYOUTS or SK_RENAMED). The epilogue ``epi`` is not in the model."""
-    return _sk_plan(M, N, K, pipe, None if layouts is None else tuple(layouts))
+    these only (numbers of SK_LAYOUTS or SK_RENAMED). Of the epilogues ``epi`` only "gelu" is in the
+    model: SK_GELU us for a value of a tile, as nothing runs beside its arithmetic, except
+    where the 128 x 192 tiles are more than the compute units and two share one
+    (csrc/kernels/gemm_pipe_tile.h); then a round of pairs, and 0.68 of one for up to half of it. Over 60
+    shapes of the encoders' widths (100 to 24000 rows, N = 4 K, K 384 to 1280) the plan takes 0.4 % longer than the
+    fastest tile on average, 1.8 to 9 % in nine; without GELU in the model and pairs it was 4.3 %, up to 42."""
+    return _sk_plan(M, N, K, pipe, None if layouts is None else tuple(layouts), epi == "gelu")
 
 
 # a function of plain values that an eager pass asks for every projection: 10 to 19 us on the host
 # each time, 0.1 for a shape that was asked before
 @functools.lru_cache(maxsize=4096)
-def _sk_plan(M: int, N: int, K: int, pipe: bool, layouts: tuple | None = None) -> tuple[int, int]:
+def _sk_plan(M: int, N: int, K: int, pipe: bool, layouts: tuple | None = None, gelu: bool = False) -> tuple[int, int]:
     KT = K // 64
     only = SK_LAYOUTS if layouts is None else {SK_RENAMED.get(x, x) for x in layouts}
     best, best_t = (7, 1), float("inf")
@@ -1731,7 +1738,11 @@ def _sk_plan(M: int, N: int, K: int, pipe: bool, layouts: tuple | None = None) -
         for s in (1, 2, 3, 4, 5, 6, 8):
             if s > 1 and (KT // s < 8 or lay == SK_WHOLE):
                 continue
-            t = -(-tiles * s // SK_CUS) * (-(-KT // s) * step * (0.8 if tiles * s <= SK_FEW else 1.0) + around)
+            end = around + (SK_GELU * bn * bm / s if gelu and lay >= SK_PIPE else 0.0)
+            t = -(-tiles * s // SK_CUS) * (-(-KT // s) * step * (0.8 if tiles * s <= SK_FEW else 1.0) + end)
+            if gelu and lay == SK_PAIRED and s == 1 and tiles > SK_CUS:
+                full, rest = divmod(tiles, 2 * SK_CUS)
+                t = 2.4 + (9.0 + 1.12 * KT) * (full + (0.0 if not rest else 0.68 if rest <= SK_CUS else 1.0))
             if s > 1:
                 t = SK_WORTH * (t + 2.0 + bn * bm * 4e-6 * (40 + 4 * s))
             if t < best_t:
@@ -1870,7 +1881,7 @@ def gemm_sk(x: torch.Tensor, w: torch.Tensor, *, epi: str = "bf16", bias: torch.
         pipe = x.stride(0) >= K and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 \
             and N * K < 1 << 31 and x.stride(0) < 1 << 21 \
             and (y is None or (y.stride(0) % 8 == 0 and y.data_ptr() % 16 == 0))
-        pl, ps = _sk_plan(M, N, K, pipe)
+        pl, ps = _sk_plan(M, N, K, pipe, None, act == "gelu")
         layout = pl if layout is None else layout
         splits = ps if splits is None else splits
         if layout in SK_RENAMED:

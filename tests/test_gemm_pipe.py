@@ -128,3 +128,29 @@ def test_gelu_over_its_whole_range():
     edge[1], edge[2] = -float("inf"), float("nan")
     got = ops.gemm_sk(x, w[:128], bias=edge, act="gelu")[0]
     assert got[0] == float("inf") and got[1].isnan() and got[2].isnan()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(192 * 16 + 1, 2048, 128), (192 * 32 - 191, 2048, 64), (6000, 1280, 1280)])
+def test_two_gelu_workgroups_on_a_compute_unit(M, N, K):
+    """More 128 x 192 tiles than compute units: ragged rows, one and two K steps (fewer than stages), several rounds."""
+    assert ops.SK_LAYOUTS[ops.SK_PAIRED][:2] == (128, 192) and -(-M // 192) * (N // 128) > ops.SK_CUS
+    g = torch.Generator().manual_seed(M)
+    x = torch.randn(M, K, generator=g).bfloat16().cuda()
+    w = (torch.randn(N, K, generator=g) * K ** -0.5).bfloat16().cuda()
+    b = torch.randn(N, generator=g).cuda()
+    y = ops.gemm_sk(x, w, bias=b, act="gelu", layout=ops.SK_PAIRED, splits=1)
+    z = x.double() @ w.double().t() + b.double()
+    want = 0.5 * z * torch.erfc(-z * 0.5 ** 0.5)
+    # half a bf16 ulp of the value, and the f32 sum's own rounding
+    assert torch.all((y.double() - want).abs() <= 2.0 ** -8 * want.abs() + (K * 2.0 ** -22 + 2.0 ** -9) * want.std())
+    # every tile size sums a value's K steps in the same order
+    assert torch.equal(y, ops.gemm_sk(x, w, bias=b, act="gelu", layout=20, splits=1))
+
+
+def test_the_plan_with_gelu():
+    for M, N, K in ((9000, 2048, 512), (12000, 3072, 768), (24000, 5120, 1280)):
+        assert ops.gemm_sk_plan(M, N, K, "gelu") == (ops.SK_PAIRED, 1)
+    for M, N, K in ((100, 2048, 512), (1500, 2048, 512), (6000, 5120, 1280)):
+        assert ops.gemm_sk_plan(M, N, K, "gelu") == ops.gemm_sk_plan(M, N, K) and ops.gemm_sk_plan(M, N, K)[0] != ops.SK_PAIRED
+    assert ops.gemm_sk_plan(9000, 1088, 512, "gelu")[0] in (1, 7)
