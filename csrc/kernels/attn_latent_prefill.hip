@@ -14,6 +14,7 @@
 // registers, scores, exponentials and products one after the other), 55 now; 4 x that: 365, 120;
 // 256 / 128: 111, 75. A single prompt is one round of the CUs, as long as its last rows (32
 // tiles, 16.5 on average); smaller blocks with one wave a SIMD were no faster.
+// Few rows behind many keys: parts of a block's keys in workgroups of their own, joined in the launch (fl_join).
 //
 // Helpers, for the sizes and alignments that latent_kv.hip does not take and queries that come turned:
 // latent_gather_kernel copies the last cu_k[b + 1] - cu_k[b] latent rows
@@ -34,6 +35,7 @@ struct LatPrefillParams {
   int H, Dv, window;
   const bf16_t* gate; long gate_ld; // [T, H * Dv] or null
   const float* cs; int max_pos, rot0, rot_dims;   // queries to be rotated: tables, first entry and width (null: done)
+  int parts, cap; float* part; int* words;        // parts of a block's keys at most, of `cap` tiles at least (fl_join)
   int runs, rows16;                 // gate rows can be read in runs of four, output rows written in runs of eight
 };
 
@@ -50,7 +52,7 @@ __global__ __launch_bounds__(64 * QW * KS, DK > 192 ? 1 : 2) void latent_prefill
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int run = wave / QW, wq = wave % QW, th = threadIdx.x - run * NTH, h = lane >> 5;
-  int bx, head, b;
+  int bx, head, b, share = 0;
   {
     // row blocks with the most keys first, over all heads of an XCD where these are whole
     const int gx = gridDim.x, gy = gridDim.y, heads = gy * gridDim.z;
@@ -62,7 +64,13 @@ __global__ __launch_bounds__(64 * QW * KS, DK > 192 ? 1 : 2) void latent_prefill
       bx = in / hp;
       hd = xcd * hp + in - bx * hp;
     }
-    bx = gx - 1 - bx;
+    if (p.parts > 1) {
+      const int block = bx / p.parts;
+      share = bx - block * p.parts;
+      bx = gx / p.parts - 1 - block;
+    } else {
+      bx = gx - 1 - bx;
+    }
     b = hd / gy;
     head = hd - b * gy;
   }
@@ -76,9 +84,17 @@ __global__ __launch_bounds__(64 * QW * KS, DK > 192 ? 1 : 2) void latent_prefill
   const bool valid = qi < qlen;
   // positions relative to the buffer's first key
   const int qpos = p.pos[q0 + min(qi, row_hi)] - koff;
-  const int kend = min(klen, p.pos[q0 + row_hi] - koff + 1);   // positions grow along a sequence
-  const int kt0 = p.window > 0 ? max(0, p.pos[q0 + row_lo] - koff - p.window + 1) / FL_KEYS * FL_KEYS : 0;
-  const int ntiles = kend > kt0 ? (kend - kt0 + FL_KEYS - 1) / FL_KEYS : 0;
+  int kend = min(klen, p.pos[q0 + row_hi] - koff + 1);         // positions grow along a sequence
+  int kt0 = p.window > 0 ? max(0, p.pos[q0 + row_lo] - koff - p.window + 1) / FL_KEYS * FL_KEYS : 0;
+  int ntiles = kend > kt0 ? (kend - kt0 + FL_KEYS - 1) / FL_KEYS : 0, parts = 1;
+  if (p.parts > 1) {
+    parts = max(1, min(p.parts, ntiles / p.cap));
+    if (share >= parts) return;                           // uniform
+    const int len = (ntiles + parts - 1) / parts;
+    kt0 += share * len * FL_KEYS;
+    kend = min(kend, kt0 + len * FL_KEYS);
+    ntiles = max(0, min(len, ntiles - share * len));
+  }
   // what this wave's rows see at all
   const int wpos_lo = __builtin_amdgcn_readfirstlane(p.pos[q0 + min(row_lo + wq * 32, row_hi)]) - koff;
   const int wpos_hi = __builtin_amdgcn_readfirstlane(p.pos[q0 + min(row_lo + wq * 32 + 31, row_hi)]) - koff;
@@ -162,6 +178,12 @@ __global__ __launch_bounds__(64 * QW * KS, DK > 192 ? 1 : 2) void latent_prefill
   fl_sync();                                              // every wave is done with the rings
   fl_merge<NDT, QW, KS>(acc, m, l, reinterpret_cast<float*>(lds), run, wq, lane);
   if (run) return;
+  if (parts > 1) {
+    const int block = (b * p.H + head) * (int)(gridDim.x / p.parts) + bx;
+    if (!fl_join<NDT, QW>(acc, m, l, p.part + (size_t)block * p.parts * QW * fl_join_floats(NDT), p.words + (size_t)block * TICKET,
+                          parts, share, wq, lane))
+      return;
+  }
   // the sink joins the denominator only (log2 domain, like the scores)
   float f = 1.f, den = l;
   if (p.sink) {
@@ -285,6 +307,7 @@ extern "C" int loqa_latent_prefill(const void* q, long q_st, const void* k, cons
                                    const void* pos, const void* sink, float scale, int window,
                                    const void* gate, long gate_ld, int B, int H, int max_q, int DK,
                                    int DV, int Dv, const void* cs, int max_pos, int rot0, int rot_dims,
+                                   int parts, int cap, float* part, long part_floats, int* words, long tickets,
                                    hipStream_t st) {
   if (B <= 0 || H <= 0 || max_q <= 0) return 0;
   if (cs && (max_pos <= 0 || rot0 < 0 || rot0 % 8 || rot_dims <= 0 || rot_dims % 8 || rot0 + rot_dims > DK || ((size_t)cs & 15)))
@@ -296,12 +319,14 @@ extern "C" int loqa_latent_prefill(const void* q, long q_st, const void* k, cons
   p.pos = (const int*)pos; p.ctx = (const int*)ctx; p.Dv = Dv; p.window = window;
   p.sink = (const float*)sink; p.scale_log2 = scale * 1.4426950408889634f; p.H = H;
   p.gate = (const bf16_t*)gate; p.gate_ld = gate_ld;
+  p.parts = parts; p.cap = cap; p.part = part; p.words = words;
+  if (parts < 1 || parts > FL_PARTS || (parts > 1 && (cap < 1 || !part || !words || ((size_t)part & 15)))) return (int)hipErrorInvalidValue;
   p.cs = (const float*)cs; p.max_pos = max_pos; p.rot0 = rot0; p.rot_dims = rot_dims;
   p.runs = Dv % 4 == 0 && (!gate || (gate_ld % 4 == 0 && ((size_t)gate & 7) == 0));
   p.rows16 = Dv % 8 == 0 && o_ld % 8 == 0 && ((size_t)o & 15) == 0;
   // the direct-to-LDS loads take 16-byte rows, a tile's rows within 32-bit offsets
   if ((((size_t)k | (size_t)v) & 15) || (long)H * DK >= (1L << 24)) return (int)hipErrorInvalidValue;
-  // 64 rows and two runs (keys of 256 columns: one) while these workgroups are one round of the
+  // 64 rows and two runs (also where the keys are in parts; keys of 256 columns: one) while these workgroups are one round of the
   // CUs, then 128 rows and two runs (160 KB of LDS at 192 columns), or one run, whose workgroups
   // share a CU: with feeds of up to 128 rows from a second round on (us with two runs and with one,
   // 9 feeds x 32 heads: 20 rows, 192 / 128 columns: 18, 9.8; 128 rows behind 300: 41.5, 31)
@@ -312,7 +337,10 @@ extern "C" int loqa_latent_prefill(const void* q, long q_st, const void* k, cons
     constexpr int end = fl_merge_bytes(C / 32, QW, KS) + QW * fl_store_bytes(C / 32);         \
     constexpr int bytes = ring > end ? ring : end;                                            \
     static_assert(bytes <= 160 * 1024, "LDS of a CU");                                        \
-    const dim3 grid((max_q + 32 * QW - 1) / (32 * QW), H, B);                                 \
+    const long blocks = (max_q + 32 * QW - 1) / (32 * QW), all = blocks * H * B;              \
+    if (parts > 1 && (all > tickets || all * parts * QW * fl_join_floats(C / 32) > part_floats)) \
+      return (int)hipErrorInvalidValue;                                                       \
+    const dim3 grid(blocks * parts, H, B);                                                    \
     hipLaunchKernelGGL((latent_prefill_kernel<A, C, QW, KS>), grid, dim3(64 * QW * KS), bytes, st, p); \
     return (int)hipGetLastError();                                                            \
   } while (0)

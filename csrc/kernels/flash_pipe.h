@@ -24,6 +24,7 @@
 #include "common.h"
 
 #define FL_KEYS 64                     // keys of a tile
+#define FL_PARTS 4                     // parts of a row block's keys at most
 
 typedef short fl_v4s __attribute__((ext_vector_type(4)));
 typedef float fl_f2 __attribute__((ext_vector_type(2)));
@@ -374,6 +375,86 @@ __device__ __forceinline__ void fl_merge(float16v (&acc)[NDT], float& m, float& 
         for (int j = 0; j < 16; ++j) acc[d][j] = acc[d][j] * a0 + o[(d * 16 + j) * 64] * a1;
     }
   }
+}
+
+// Parts of a row block's keys in workgroups of their own (n > 1 of them): each wave of rows publishes its
+// (m, l, acc), the last part to arrive gets the joint values and returns true, whichever it is summed up in
+// the parts' order. part: n slots of the block, QW fl_join_floats each; words: the block's 2 QW <= TICKET
+// zeroed words, zero again afterwards (arrivals, and parts that can be read: the last waits for those, whose
+// owners are past everything but their own stores). Written through and read past the caches (sc1): one
+// wave a SIMD reads about 27 KB/us of them, 4 us for three parts of 64 rows of 128 columns.
+__host__ __device__ constexpr int fl_join_floats(int NDT) { return (NDT * 16 + 4) * 64; }
+
+template <int NDT, int QW>
+__device__ __forceinline__ bool fl_join(float16v (&acc)[NDT], float& m, float& l, float* part, int* words, int n, int mine, int wq,
+                                        int lane) {
+  constexpr int PER = fl_join_floats(NDT) * 4, SC1 = 16;          // bytes of a wave's slot
+  const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(part, 0, n * QW * PER, 0x00020000);
+  int* word = words + 2 * wq;
+  int old = 0;
+  if (lane == 0) old = __hip_atomic_fetch_add(word, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  old = __builtin_amdgcn_readfirstlane(old);
+  if (old != n - 1) {
+    const int at = (mine * QW + wq) * PER;
+#pragma unroll
+    for (int d = 0; d < NDT; ++d)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const fl_u4 v = {__float_as_uint(acc[d][4 * g]), __float_as_uint(acc[d][4 * g + 1]), __float_as_uint(acc[d][4 * g + 2]),
+                         __float_as_uint(acc[d][4 * g + 3])};
+        __builtin_amdgcn_raw_buffer_store_b128(v, r, at + (4 * d + g) * 1024 + lane * 16, 0, SC1);
+      }
+    const fl_u4 ml = {__float_as_uint(m), __float_as_uint(l), 0u, 0u};
+    __builtin_amdgcn_raw_buffer_store_b128(ml, r, at + 4 * NDT * 1024 + lane * 16, 0, SC1);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // written through: visible when acknowledged
+    if (lane == 0) __hip_atomic_fetch_add(word + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return false;
+  }
+  while (__hip_atomic_load(word + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != n - 1) __builtin_amdgcn_s_sleep(1);
+  asm volatile("" ::: "memory");
+  if (lane == 0) {
+    __hip_atomic_store(word, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(word + 1, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  float a[FL_PARTS], lp[FL_PARTS], top = m;
+#pragma unroll
+  for (int i = 0; i < FL_PARTS; ++i) {
+    a[i] = i == mine ? m : -1e30f;
+    lp[i] = i == mine ? l : 0.f;
+    if (i < n && i != mine) {
+      const fl_u4 v = __builtin_bit_cast(fl_u4, __builtin_amdgcn_raw_buffer_load_b128(r, (i * QW + wq) * PER + 4 * NDT * 1024 + lane * 16, 0, SC1));
+      a[i] = __uint_as_float(v[0]);
+      lp[i] = __uint_as_float(v[1]);
+    }
+    top = fmaxf(top, a[i]);
+  }
+  l = 0.f;
+#pragma unroll
+  for (int i = 0; i < FL_PARTS; ++i) {
+    a[i] = exp2f(a[i] - top);
+    l += lp[i] * a[i];
+  }
+  m = top;
+#pragma unroll
+  for (int d = 0; d < NDT; ++d) {
+    fl_u4 o[FL_PARTS][4];
+#pragma unroll
+    for (int i = 0; i < FL_PARTS; ++i)
+      if (i < n && i != mine)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          o[i][g] = __builtin_bit_cast(fl_u4, __builtin_amdgcn_raw_buffer_load_b128(r, (i * QW + wq) * PER + (4 * d + g) * 1024 + lane * 16, 0, SC1));
+    float16v sum;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) sum[j] = 0.f;
+#pragma unroll
+    for (int i = 0; i < FL_PARTS; ++i)
+      if (i < n)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) sum[j] = fmaf(i == mine ? acc[d][j] : __uint_as_float(o[i][j >> 2][j & 3]), a[i], sum[j]);
+    acc[d] = sum;
+  }
+  return true;
 }
 
 // A wave's 32 rows as bf16 to y (rows ld apart, `rows` of them exist, `cols` <= 32 NDT columns,

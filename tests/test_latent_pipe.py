@@ -62,3 +62,32 @@ def test_sizes_and_edges(DK, DV):
 @pytest.mark.parametrize("B,T,H", [(1, 700, 8), (2, 700, 24), (4, 900, 24)])
 def test_every_block_height(B, T, H):
     _check([T] * B, [7] * B, H, 192, 128, 128, 300, sink=True, seed=B)
+
+
+@pytest.mark.parametrize("feeds,pasts,H,window", [([33], [2100], 8, 0), ([1, 64, 40], [4000, 450, 700], 4, 0), ([100, 7], [1200, 1500], 16, 0),
+                                                  ([130], [3000], 8, 1030), ([64, 64], [1530, 600], 16, 0)])
+def test_parts_of_the_keys(feeds, pasts, H, window):
+    """One to four parts of a block's keys in workgroups of their own, uneven ones, blocks of other lengths in one launch."""
+    kept = sum(min(f + p, f + window - 1) if window else f + p for f, p in zip(feeds, pasts))
+    parts, rows = seqmix._latent_parts(max(feeds), H * len(feeds), kept // len(feeds))
+    assert parts > 1 and rows == 64
+    for DK, DV in ((192, 128), (256, 64), (64, 64)):
+        _check(feeds, pasts, H, DK, DV, DV - 12, window=window, sink=True, gate=True, seed=DK)
+    _check(feeds, pasts, H, 128, 128, 128, window=window, scale=-0.05, seed=5)
+
+
+def test_parts_repeat_bit_for_bit():
+    g = torch.Generator().manual_seed(9)
+    q, k, v = (torch.randn(n, 16, d, generator=g).bfloat16().to(DEV) for n, d in ((64, 192), (2064, 192), (2064, 128)))
+    i32 = lambda *x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    run = lambda: seqmix.latent_prefill(q, k, v, i32(0, 64), i32(0, 2064), i32(2064), torch.arange(2000, 2064, device=DEV).int(), None, 0.07, 64, 128)
+    first = run()
+    assert all(torch.equal(run(), first) for _ in range(10))
+    graph = torch.cuda.CUDAGraph()
+    args = (q, k, v, i32(0, 64), i32(0, 2064), i32(2064), torch.arange(2000, 2064, device=DEV).int(), None, 0.07, 64, 128)
+    with torch.cuda.graph(graph):
+        y = seqmix.latent_prefill(*args)
+    for _ in range(3):
+        y.zero_()
+        graph.replay()
+        assert torch.equal(y, first) and torch.equal(run(), first)
