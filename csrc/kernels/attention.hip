@@ -55,6 +55,8 @@ struct AttnParams {
   float* part_o;   // [num_splits, Tq, Hq, D]
   float* part_ml;  // [num_splits, Tq, Hq, 2]
   int total_q;
+  int parts;                // prompts: parts of a row block's keys at most, (fl_join)
+  float* part; int* words;
 };
 
 template <int D>
@@ -262,12 +264,13 @@ __global__ __launch_bounds__(ATT_THREADS, 1) void attn_fwd_kernel(AttnParams p) 
 template <int D, int PAGES, int QW, int KS>
 __global__ __launch_bounds__(64 * QW * KS, D == 64 && QW * KS == 4 ? 3 : 2) void attn_pipe_kernel(AttnParams p) {
   constexpr bool PAGED = PAGES > 0;
+  constexpr bool PARTS = QW == 2;      // the launch has parts of 64-row blocks only
   using L = FlashLds<D, D>;
   constexpr int NS = D / 16, NDT = D / 32, NTH = 64 * QW;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int run = wave / QW, wq = wave % QW, th = threadIdx.x - run * NTH, h = lane >> 5;
-  int bx, by, bz;
+  int bx, by, bz, share = 0;
   {
     const int gx = gridDim.x, gy = gridDim.y, heads = gy * gridDim.z, n = gx * heads;
     const int logical = xcd_remap(blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z), n);
@@ -281,6 +284,10 @@ __global__ __launch_bounds__(64 * QW * KS, D == 64 && QW * KS == 4 ? 3 : 2) void
         hd = xcd * hp + at - bx * hp;
       }
       bx = gx - 1 - bx;
+    }
+    if (PARTS && p.parts > 1) {
+      share = bx % p.parts;
+      bx /= p.parts;
     }
     by = hd % gy;
     bz = hd / gy;
@@ -304,9 +311,17 @@ __global__ __launch_bounds__(64 * QW * KS, D == 64 && QW * KS == 4 ? 3 : 2) void
   const int qpos_lo = klen - qlen + row_lo + wq * 32;       // wave's first query position
   int kend = klen;
   if (p.causal) kend = min(kend, klen - qlen + row_hi + 1);
-  const int ntiles = kend > 0 ? (kend + FL_KEYS - 1) / FL_KEYS : 0;
+  int ntiles = kend > 0 ? (kend + FL_KEYS - 1) / FL_KEYS : 0, parts = 1, t0 = 0;
+  if (PARTS && p.parts > 1) {
+    parts = max(1, min(p.parts, ntiles / FL_CAP));
+    if (share >= parts) return;                             // uniform
+    const int len = (ntiles + parts - 1) / parts;
+    t0 = share * len;
+    ntiles = max(0, min(len, ntiles - t0));
+    kend = min(kend, (t0 + len) * FL_KEYS);
+  }
   const int per = (ntiles + KS - 1) / KS;                   // tiles of a run; the last may have fewer
-  const int first = run * per;
+  const int first = t0 + run * per;
 
   bf16x8 qf[NS];
   {
@@ -328,7 +343,7 @@ __global__ __launch_bounds__(64 * QW * KS, D == 64 && QW * KS == 4 ? 3 : 2) void
   const FlFetch<D, NTH, true, false> vf(th, D, PAGED ? D : p.kv_stride);
   // Where a fetch stands: tiles come in order, one call each; past the last tile it stays there.
   // Rows past kend read the last key again (finite scores, masked to -inf, so P = 0).
-  const int kt0 = max(min(first, ntiles - 1), 0) * FL_KEYS;
+  const int kt0 = max(min(first, t0 + ntiles - 1), 0) * FL_KEYS;
   const int* btab = PAGED ? p.block_tables + (size_t)b * p.max_blocks : nullptr;
   const unsigned page_bytes = (unsigned)(p.Hkv * p.blk) * (D * 2);
   struct At {
@@ -382,6 +397,12 @@ __global__ __launch_bounds__(64 * QW * KS, D == 64 && QW * KS == 4 ? 3 : 2) void
   fl_merge<NDT, QW, KS>(acc, m, l, reinterpret_cast<float*>(lds), run, wq, lane,
                          KS == 4 && ntiles <= 1);   // (with two runs it would save less and cost long prompts up to 2 %)
   if (run) return;
+  if (PARTS && parts > 1) {
+    const int block = (b * p.Hq + head) * (int)(gridDim.x / p.parts) + bx;
+    if (!fl_join<NDT, QW>(acc, m, l, p.part + (size_t)block * p.parts * QW * fl_join_floats(NDT), p.words + (size_t)block * TICKET,
+                          parts, share, wq, lane))
+      return;
+  }
   const float inv = l > 0.f ? 1.f / l : 0.f;
 #pragma unroll
   for (int d = 0; d < NDT; ++d)
@@ -683,7 +704,7 @@ static int launch_pipe(const AttnParams& p, int B, int max_q, hipStream_t s) {
   constexpr int ring = KS * FlashLds<D, D>::RING, end = fl_merge_bytes(D / 32, QW, KS) + QW * fl_store_bytes(D / 32);
   constexpr int bytes = ring > end ? ring : end;
   static_assert(bytes <= 160 * 1024, "LDS of a CU");
-  const dim3 grid((max_q + 32 * QW - 1) / (32 * QW), p.Hq, B);
+  const dim3 grid((max_q + 32 * QW - 1) / (32 * QW) * p.parts, p.Hq, B);
   hipLaunchKernelGGL((attn_pipe_kernel<D, PAGES, QW, KS>), grid, dim3(64 * QW * KS), bytes, s, p);
   return (int)hipGetLastError();
 }
@@ -702,9 +723,10 @@ static int launch_pipe(const AttnParams& p, int B, int max_q, hipStream_t s) {
 // 29; 2048 x 20 heads 40, 50; 4096 x 12 heads 68, 94, x 20 heads 116, 121; but 4 x 700 x 16 heads
 // 18.0, 17.0, 3000 x 20 heads 76, 62, 4096 x 32 heads 121, 102.
 template <int D, int PAGES>
-static int launch_rows(const AttnParams& p, int B, int max_q, hipStream_t s) {
+static int launch_rows(AttnParams p, int B, int max_q, hipStream_t s) {
   const long n64 = (long)((max_q + 63) / 64) * p.Hq * B, n128 = (long)((max_q + 127) / 128) * p.Hq * B;
   const long two = D == 128 ? (max_q <= 128 ? 256 : 512) : !p.causal || max_q < 1024 ? 256 : max_q < 4096 ? 384 : 640;
+  if (n64 > 128) p.parts = 1;        // parts only of 64-row blocks, all of them one round
   if (n64 <= 256) return launch_pipe<D, PAGES, 2, D == 64 ? 4 : 2>(p, B, max_q, s);
   if (n128 <= two) return launch_pipe<D, PAGES, 4, 2>(p, B, max_q, s);
   return launch_pipe<D, PAGES, 4, 1>(p, B, max_q, s);
@@ -738,7 +760,8 @@ extern "C" int loqa_attention(const void* q, long long q_stride, const void* k, 
                               const int* cu_k, const int* ctx_lens, const int* block_tables,
                               int max_blocks, int blk, int B, int max_q, int Hq, int Hkv, int D,
                               float scale, int causal, int mode, int split_keys, int num_splits,
-                              float* part_o, float* part_ml, int total_q, hipStream_t s) {
+                              float* part_o, float* part_ml, int total_q, int parts, float* part,
+                              long long part_floats, int* words, long long tickets, hipStream_t s) {
   if (B <= 0) return 0;
   if (Hkv <= 0 || Hq % Hkv != 0 || (D != 64 && D != 128)) return (int)hipErrorInvalidValue;
   const bool paged = block_tables != nullptr;
@@ -758,6 +781,12 @@ extern "C" int loqa_attention(const void* q, long long q_stride, const void* k, 
   p.scale_log2 = scale * 1.4426950408889634f; p.causal = causal;
   p.split_keys = split_keys; p.num_splits = num_splits; p.part_o = part_o; p.part_ml = part_ml;
   p.total_q = total_q;
+  p.parts = parts; p.part = part; p.words = words;
+  const long long blocks = (long long)((max_q + 63) / 64) * Hq * B;
+  if (parts < 1 || parts > FL_PARTS ||
+      (parts > 1 && (mode == 1 || !part || !words || ((size_t)part & 15) || blocks > tickets ||
+                     blocks * parts * 2 * fl_join_floats(D / 32) > part_floats)))
+    return (int)hipErrorInvalidValue;
   int rc;
 #define DISPATCH(DD)                                                                    \
   if (mode == 0) rc = paged ? launch_attn<DD, true, false>(p, B, max_q, s)              \

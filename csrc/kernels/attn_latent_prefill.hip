@@ -35,7 +35,7 @@ struct LatPrefillParams {
   int H, Dv, window;
   const bf16_t* gate; long gate_ld; // [T, H * Dv] or null
   const float* cs; int max_pos, rot0, rot_dims;   // queries to be rotated: tables, first entry and width (null: done)
-  int parts, cap; float* part; int* words;        // parts of a block's keys at most, of `cap` tiles at least (fl_join)
+  int parts; float* part; int* words;             // parts of a block's keys at most (fl_join)
   int runs, rows16;                 // gate rows can be read in runs of four, output rows written in runs of eight
 };
 
@@ -47,6 +47,7 @@ struct LatPrefillParams {
 // 2048 x 8 heads 37.2, 41.8, at 128 / 128 30.6, 36.9.
 template <int DK, int DV, int QW, int KS>
 __global__ __launch_bounds__(64 * QW * KS, DK > 192 ? 1 : 2) void latent_prefill_kernel(LatPrefillParams p) {
+  constexpr bool PARTS = QW == 2;      // the launch has parts of 64-row blocks only
   using L = FlashLds<DK, DV>;
   constexpr int NS = DK / 16, NDT = DV / 32, NTH = 64 * QW;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
@@ -64,7 +65,7 @@ __global__ __launch_bounds__(64 * QW * KS, DK > 192 ? 1 : 2) void latent_prefill
       bx = in / hp;
       hd = xcd * hp + in - bx * hp;
     }
-    if (p.parts > 1) {
+    if (PARTS && p.parts > 1) {
       const int block = bx / p.parts;
       share = bx - block * p.parts;
       bx = gx / p.parts - 1 - block;
@@ -87,8 +88,8 @@ __global__ __launch_bounds__(64 * QW * KS, DK > 192 ? 1 : 2) void latent_prefill
   int kend = min(klen, p.pos[q0 + row_hi] - koff + 1);         // positions grow along a sequence
   int kt0 = p.window > 0 ? max(0, p.pos[q0 + row_lo] - koff - p.window + 1) / FL_KEYS * FL_KEYS : 0;
   int ntiles = kend > kt0 ? (kend - kt0 + FL_KEYS - 1) / FL_KEYS : 0, parts = 1;
-  if (p.parts > 1) {
-    parts = max(1, min(p.parts, ntiles / p.cap));
+  if (PARTS && p.parts > 1) {
+    parts = max(1, min(p.parts, ntiles / FL_CAP));
     if (share >= parts) return;                           // uniform
     const int len = (ntiles + parts - 1) / parts;
     kt0 += share * len * FL_KEYS;
@@ -178,7 +179,7 @@ __global__ __launch_bounds__(64 * QW * KS, DK > 192 ? 1 : 2) void latent_prefill
   fl_sync();                                              // every wave is done with the rings
   fl_merge<NDT, QW, KS>(acc, m, l, reinterpret_cast<float*>(lds), run, wq, lane);
   if (run) return;
-  if (parts > 1) {
+  if (PARTS && parts > 1) {
     const int block = (b * p.H + head) * (int)(gridDim.x / p.parts) + bx;
     if (!fl_join<NDT, QW>(acc, m, l, p.part + (size_t)block * p.parts * QW * fl_join_floats(NDT), p.words + (size_t)block * TICKET,
                           parts, share, wq, lane))
@@ -307,7 +308,7 @@ extern "C" int loqa_latent_prefill(const void* q, long q_st, const void* k, cons
                                    const void* pos, const void* sink, float scale, int window,
                                    const void* gate, long gate_ld, int B, int H, int max_q, int DK,
                                    int DV, int Dv, const void* cs, int max_pos, int rot0, int rot_dims,
-                                   int parts, int cap, float* part, long part_floats, int* words, long tickets,
+                                   int parts, float* part, long part_floats, int* words, long tickets,
                                    hipStream_t st) {
   if (B <= 0 || H <= 0 || max_q <= 0) return 0;
   if (cs && (max_pos <= 0 || rot0 < 0 || rot0 % 8 || rot_dims <= 0 || rot_dims % 8 || rot0 + rot_dims > DK || ((size_t)cs & 15)))
@@ -319,8 +320,8 @@ extern "C" int loqa_latent_prefill(const void* q, long q_st, const void* k, cons
   p.pos = (const int*)pos; p.ctx = (const int*)ctx; p.Dv = Dv; p.window = window;
   p.sink = (const float*)sink; p.scale_log2 = scale * 1.4426950408889634f; p.H = H;
   p.gate = (const bf16_t*)gate; p.gate_ld = gate_ld;
-  p.parts = parts; p.cap = cap; p.part = part; p.words = words;
-  if (parts < 1 || parts > FL_PARTS || (parts > 1 && (cap < 1 || !part || !words || ((size_t)part & 15)))) return (int)hipErrorInvalidValue;
+  p.parts = parts; p.part = part; p.words = words;
+  if (parts < 1 || parts > FL_PARTS || (parts > 1 && (!part || !words || ((size_t)part & 15)))) return (int)hipErrorInvalidValue;
   p.cs = (const float*)cs; p.max_pos = max_pos; p.rot0 = rot0; p.rot_dims = rot_dims;
   p.runs = Dv % 4 == 0 && (!gate || (gate_ld % 4 == 0 && ((size_t)gate & 7) == 0));
   p.rows16 = Dv % 8 == 0 && o_ld % 8 == 0 && ((size_t)o & 15) == 0;
@@ -338,7 +339,7 @@ extern "C" int loqa_latent_prefill(const void* q, long q_st, const void* k, cons
     constexpr int bytes = ring > end ? ring : end;                                            \
     static_assert(bytes <= 160 * 1024, "LDS of a CU");                                        \
     const long blocks = (max_q + 32 * QW - 1) / (32 * QW), all = blocks * H * B;              \
-    if (parts > 1 && (all > tickets || all * parts * QW * fl_join_floats(C / 32) > part_floats)) \
+    if (parts > 1 && (QW != 2 || all > tickets || all * parts * QW * fl_join_floats(C / 32) > part_floats)) \
       return (int)hipErrorInvalidValue;                                                       \
     const dim3 grid(blocks * parts, H, B);                                                    \
     hipLaunchKernelGGL((latent_prefill_kernel<A, C, QW, KS>), grid, dim3(64 * QW * KS), bytes, st, p); \

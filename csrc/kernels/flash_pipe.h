@@ -24,7 +24,8 @@
 #include "common.h"
 
 #define FL_KEYS 64                     // keys of a tile
-#define FL_PARTS 4                     // parts of a row block's keys at most
+#define FL_PARTS 8                     // parts of a row block's keys at most
+#define FL_CAP 8                       // tiles of one at least
 
 typedef short fl_v4s __attribute__((ext_vector_type(4)));
 typedef float fl_f2 __attribute__((ext_vector_type(2)));
@@ -381,9 +382,61 @@ __device__ __forceinline__ void fl_merge(float16v (&acc)[NDT], float& m, float& 
 // (m, l, acc), the last part to arrive gets the joint values and returns true, whichever it is summed up in
 // the parts' order. part: n slots of the block, QW fl_join_floats each; words: the block's 2 QW <= TICKET
 // zeroed words, zero again afterwards (arrivals, and parts that can be read: the last waits for those, whose
-// owners are past everything but their own stores). Written through and read past the caches (sc1): one
-// wave a SIMD reads about 27 KB/us of them, 4 us for three parts of 64 rows of 128 columns.
+// owners are past everything but their own stores). Written through and read past the caches (sc1).
+// Publishing and joining two parts takes 3 to 4 us (64 rows x 32 heads of 128 behind 1000 keys: 22.2 us whole, 16.7).
 __host__ __device__ constexpr int fl_join_floats(int NDT) { return (NDT * 16 + 4) * 64; }
+
+// The n <= N parts' values, LB 16-byte pieces of each part's slot asked for at a time.
+template <int NDT, int QW, int N, int LB>
+__device__ __forceinline__ void fl_join_sum(float16v (&acc)[NDT], float& m, float& l, const __amdgpu_buffer_rsrc_t& r, int n, int mine,
+                                            int wq, int lane) {
+  constexpr int PER = fl_join_floats(NDT) * 4, SC1 = 16, O = N == 2 ? 1 : N;   // of two parts one is the other
+  auto load = [&](int i, int piece) __attribute__((always_inline)) {
+    return __builtin_bit_cast(fl_u4, __builtin_amdgcn_raw_buffer_load_b128(r, (i * QW + wq) * PER + piece * 1024 + lane * 16, 0, SC1));
+  };
+  float a[N], lp[N], top = m;
+  fl_u4 ml[O], o[O][LB];
+  auto fetch = [&](int p0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < O; ++i)
+      if (N == 2 || (i < n && i != mine))
+#pragma unroll
+        for (int k = 0; k < LB; ++k) o[i][k] = load(N == 2 ? 1 - mine : i, p0 + k);
+  };
+#pragma unroll
+  for (int i = 0; i < O; ++i)
+    if (N == 2 || (i < n && i != mine)) ml[i] = load(N == 2 ? 1 - mine : i, 4 * NDT);
+  fetch(0);
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const bool own = i == mine, there = i < n;
+    a[i] = own ? m : there ? __uint_as_float(ml[N == 2 ? 0 : i][0]) : -1e30f;
+    lp[i] = own ? l : there ? __uint_as_float(ml[N == 2 ? 0 : i][1]) : 0.f;
+    top = fmaxf(top, a[i]);
+  }
+  l = 0.f;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    a[i] = exp2f(a[i] - top);
+    l += lp[i] * a[i];
+  }
+  m = top;
+#pragma unroll
+  for (int p0 = 0; p0 < 4 * NDT; p0 += LB) {
+    if (p0) fetch(p0);
+    float sum[LB * 4];
+#pragma unroll
+    for (int j = 0; j < LB * 4; ++j) sum[j] = 0.f;
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      if (i < n)
+#pragma unroll
+        for (int j = 0; j < LB * 4; ++j)
+          sum[j] = fmaf(i == mine ? acc[p0 / 4 + j / 16][(p0 % 4) * 4 + j % 16] : __uint_as_float(o[N == 2 ? 0 : i][j >> 2][j & 3]), a[i], sum[j]);
+#pragma unroll
+    for (int j = 0; j < LB * 4; ++j) acc[p0 / 4 + j / 16][(p0 % 4) * 4 + j % 16] = sum[j];
+  }
+}
 
 template <int NDT, int QW>
 __device__ __forceinline__ bool fl_join(float16v (&acc)[NDT], float& m, float& l, float* part, int* words, int n, int mine, int wq,
@@ -416,44 +469,10 @@ __device__ __forceinline__ bool fl_join(float16v (&acc)[NDT], float& m, float& l
     __hip_atomic_store(word, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __hip_atomic_store(word + 1, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  float a[FL_PARTS], lp[FL_PARTS], top = m;
-#pragma unroll
-  for (int i = 0; i < FL_PARTS; ++i) {
-    a[i] = i == mine ? m : -1e30f;
-    lp[i] = i == mine ? l : 0.f;
-    if (i < n && i != mine) {
-      const fl_u4 v = __builtin_bit_cast(fl_u4, __builtin_amdgcn_raw_buffer_load_b128(r, (i * QW + wq) * PER + 4 * NDT * 1024 + lane * 16, 0, SC1));
-      a[i] = __uint_as_float(v[0]);
-      lp[i] = __uint_as_float(v[1]);
-    }
-    top = fmaxf(top, a[i]);
-  }
-  l = 0.f;
-#pragma unroll
-  for (int i = 0; i < FL_PARTS; ++i) {
-    a[i] = exp2f(a[i] - top);
-    l += lp[i] * a[i];
-  }
-  m = top;
-#pragma unroll
-  for (int d = 0; d < NDT; ++d) {
-    fl_u4 o[FL_PARTS][4];
-#pragma unroll
-    for (int i = 0; i < FL_PARTS; ++i)
-      if (i < n && i != mine)
-#pragma unroll
-        for (int g = 0; g < 4; ++g)
-          o[i][g] = __builtin_bit_cast(fl_u4, __builtin_amdgcn_raw_buffer_load_b128(r, (i * QW + wq) * PER + (4 * d + g) * 1024 + lane * 16, 0, SC1));
-    float16v sum;
-#pragma unroll
-    for (int j = 0; j < 16; ++j) sum[j] = 0.f;
-#pragma unroll
-    for (int i = 0; i < FL_PARTS; ++i)
-      if (i < n)
-#pragma unroll
-        for (int j = 0; j < 16; ++j) sum[j] = fmaf(i == mine ? acc[d][j] : __uint_as_float(o[i][j >> 2][j & 3]), a[i], sum[j]);
-    acc[d] = sum;
-  }
+  // as many loads in flight as registers allow: the trip is what this costs
+  if (n == 2) fl_join_sum<NDT, QW, 2, NDT * 4>(acc, m, l, r, n, mine, wq, lane);
+  else if (n <= 4) fl_join_sum<NDT, QW, 4, 4>(acc, m, l, r, n, mine, wq, lane);
+  else fl_join_sum<NDT, QW, FL_PARTS, 2>(acc, m, l, r, n, mine, wq, lane);
   return true;
 }
 

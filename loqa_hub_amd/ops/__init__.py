@@ -185,6 +185,17 @@ ATTN8_MIN_KEYS = int(os.environ.get("LOQA_ATTN8_MIN_KEYS", "0"))
 ATTN_PF_MIN_KEYS = int(os.environ.get("LOQA_ATTN_PF_MIN_KEYS", "0"))
 
 
+def attn_parts(max_q: int, heads: int, keys: int) -> int:
+    """Parts of a row block's keys at most, for the prompt attentions over ``heads`` heads of all
+    sequences with ``keys`` keys. Few rows behind many keys are few workgroups with a long chain of tiles each:
+    parts of eight tiles or more, while all of them are one round of the 256 CUs, join in the launch (us whole and in parts, 32
+    heads of 128: 64 rows behind 1000 keys 22.2, 16.7; behind 2000 35.6, 19.9; behind 8000 121, 32; 256 behind 3000 50.4, 32.1; 8
+    heads of 64: 64 behind 1000 15.3, 12.9; behind 8000 56, 17). Past one round the CUs share what bounds them (2048 rows of
+    16 latent heads 52, the longer blocks in two parts 57), and under 1024 keys no block has 16 tiles."""
+    n64 = -(-max_q // 64) * heads
+    return min(8, 256 // n64) if keys >= 1024 and 0 < n64 <= 128 else 1
+
+
 def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu_q: torch.Tensor, *,
               n_heads: int, n_kv: int, head_dim: int, causal: bool, max_q: int,
               cu_k: torch.Tensor | None = None, ctx_lens: torch.Tensor | None = None,
@@ -260,11 +271,18 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu_q: torch.Ten
             assert workspace is not None and workspace.max_splits >= num_splits
             assert workspace.max_tokens >= Tq
             part_o, part_ml = workspace.part_o, workspace.part_ml
+    parts, ws, words, st = 1, None, None, stream_ptr(q)
+    if not grouped:
+        parts = attn_parts(max_q, n_heads * B, (max_k or 0) if paged else k.shape[0] // B)
+        if parts > 1:       # a wave's 32 rows: head_dim / 2 accumulators a lane, maximum and sum
+            blocks = -(-max_q // 64) * n_heads * B
+            ws, words = _sk_workspace(q.device, st, blocks * parts * 2 * (head_dim // 2 + 4) * 64, blocks)
     check(kernels().loqa_attention(
         ptr(q), q.stride(0), ptr(k), ptr(v), kv_stride, ptr(out), out.stride(0), ptr(cu_q),
         ptr(cu_k), ptr(ctx_lens), ptr(block_tables), max_blocks, blk, B, max_q, n_heads, n_kv,
         head_dim, scale, int(causal), int(grouped), split_keys, num_splits, ptr(part_o),
-        ptr(part_ml), Tq, stream_ptr(q)), "attention")
+        ptr(part_ml), Tq, parts, ptr(ws), ws.numel() if parts > 1 else 0, ptr(words),
+        words.numel() if parts > 1 else 0, st), "attention")
     return out
 
 

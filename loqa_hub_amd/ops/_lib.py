@@ -114,7 +114,7 @@ _KERNEL_SIGS = {
     "loqa_attention": [c_void_p, c_ll, c_void_p, c_void_p, c_ll, c_void_p, c_ll, c_void_p,
                        c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,
                        c_int, c_float, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_int,
-                       c_void_p],
+                       c_int, c_void_p, c_ll, c_void_p, c_ll, c_void_p],
     "loqa_log_mel": [c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int,
                      c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p],
     "loqa_im2col_k3": [c_void_p, c_ll, c_ll, c_ll, c_int, c_int, c_int, c_int, c_void_p,
@@ -233,7 +233,7 @@ _SEQMIX_SIGS = {
     "loqa_latent_kfill": [_vp, _vp, _i, _i, _i, _i, _i, _vp],
     "loqa_rope_pairs": [_vp, _l, _l, _i, _i, _i, _i, _vp, _vp, _i, _vp],
     "loqa_latent_prefill": [_vp, _l, _vp, _vp, _vp, _l, _vp, _vp, _vp, _vp, _vp, _f, _i, _vp, _l,
-                            _i, _i, _i, _i, _i, _i, _vp, _i, _i, _i, _i, _i, _vp, _l, _vp, _l, _vp],
+                            _i, _i, _i, _i, _i, _i, _vp, _i, _i, _i, _i, _vp, _l, _vp, _l, _vp],
     "loqa_lightning_prep": [_vp, _i, _l, _i, _i, _vp, _vp],
     "loqa_state_scan": [_vp, _l, _i, _i, _i, _i, _i, _i, _i, _vp, _i, _vp, _vp, _vp, _vp, _vp, _vp,
                         _vp, _i, _i, _i, _vp],

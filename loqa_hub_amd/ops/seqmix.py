@@ -25,7 +25,7 @@ from __future__ import annotations
 import torch
 
 from . import reference as ref
-from . import _sk_workspace
+from . import _sk_workspace, attn_parts
 from ._lib import check, kernels, ptr, stream_ptr
 
 _DT = {torch.bfloat16: 0, torch.float32: 1}
@@ -342,18 +342,6 @@ def rope_pairs_(x: torch.Tensor, off: int, dims: int, positions: torch.Tensor,
           "rope_pairs")
 
 
-def _latent_parts(max_q: int, heads: int, keys: int) -> tuple[int, int]:
-    """(parts of a row block's keys at most, rows of a block) for ``heads`` heads of all sequences of
-    ``keys`` keys on average. Few rows behind many keys are few workgroups with a long
-    chain of tiles each: parts of eight tiles or more while all of them are one round of the 256 CUs (64 rows behind
-    2000 keys x 16 heads 40.0 us, in four parts 23.8; 300 behind 1500 35.4, in three 24.3; 1000 behind 1000 x 8
-    heads 36.6, in two 27.5). Beyond that the CUs share what bounds them: the last rows of 2048 x 16
-    heads, twice the average, in parts of their own 57 us, whole 52. Under 1024 keys nothing is
-    gained (200 rows x 16 heads 13.6, in parts 13.9)."""
-    n64 = -(-max_q // 64) * heads
-    return (min(4, 256 // n64) if keys >= 1024 and n64 <= 128 else 1), 64 if n64 <= 256 else 128
-
-
 def latent_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu_q: torch.Tensor,
                    cu_k: torch.Tensor, ctx_lens: torch.Tensor, positions: torch.Tensor,
                    sink: torch.Tensor | None, scale: float, max_q: int, Dv: int, window: int = 0,
@@ -401,15 +389,15 @@ def latent_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu_q: torc
     k = k if k.data_ptr() % 16 == 0 else k.clone()
     v = v if v.data_ptr() % 16 == 0 else v.clone()
     st = stream_ptr(q)
-    parts, rows = _latent_parts(int(max_q), H * B, k.shape[0] // max(B, 1))
+    parts = attn_parts(int(max_q), H * B, k.shape[0] // max(B, 1))
     ws = words = None
     if parts > 1:           # a wave's 32 rows: DV / 2 accumulators a lane, maximum and sum
-        blocks = -(-max_q // rows) * H * B
-        ws, words = _sk_workspace(q.device, st, blocks * parts * rows // 32 * (DV // 2 + 4) * 64, blocks)
+        blocks = -(-max_q // 64) * H * B
+        ws, words = _sk_workspace(q.device, st, blocks * parts * 2 * (DV // 2 + 4) * 64, blocks)
     check(kernels().loqa_latent_prefill(
         ptr(q), q.stride(0), ptr(k), ptr(v), ptr(out), out.stride(0), ptr(cu_q), ptr(cu_k),
         ptr(ctx_lens), ptr(positions), ptr(sink), float(scale), int(window), ptr(gate),
-        gate.stride(0) if gate is not None else 0, B, H, int(max_q), DK, DV, Dv, ptr(cs), *turn, parts, 8,
+        gate.stride(0) if gate is not None else 0, B, H, int(max_q), DK, DV, Dv, ptr(cs), *turn, parts,
         ptr(ws), ws.numel() if parts > 1 else 0, ptr(words), words.numel() if parts > 1 else 0, st),
         "latent_prefill")
     return out

@@ -154,3 +154,20 @@ def test_many_short_prompts():
         return lambda: ops.attention(q, kc, kc, cu, n_heads=H, n_kv=G, head_dim=D, causal=True, max_q=n, ctx_lens=ctx, block_tables=bt,
                                      max_k=n)
     assert _us(call(9)) < 1.4 * _us(call(8))
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("qlens,klens,Hq,page", [([33], [2100], 8, 16), ([1, 64, 40], [4100, 450, 700], 4, 64), ([100, 7], [1300, 1507], 8, 8),
+                                                 ([130], [9000], 4, 1024), ([64], [1024], 8, 32), ([90, 90], [2000, 1100], 4, 0)])
+def test_parts_of_the_keys(D, qlens, klens, Hq, page):
+    """One to eight parts of a block's keys in workgroups of their own, uneven ones, short sequences beside long ones."""
+    assert ops.attn_parts(max(qlens), Hq * len(qlens), max(klens) if page else sum(klens) // len(klens)) > 1
+    _check(qlens, klens, Hq, 2, D, True, page=page, seed=7)
+    _check(qlens, klens, Hq, 2, D, False, page=page, seed=8, spread=4.0)
+    torch.cuda.synchronize()
+    assert all(int(words.abs().sum()) == 0 for _, words in ops._SK_WS.values())
+
+
+def test_when_keys_are_in_parts():
+    assert [ops.attn_parts(*x) for x in ((64, 32, 1024), (64, 32, 1023), (64, 64, 4000), (200, 32, 4000), (257, 32, 4000), (1, 1, 1024), (0, 8, 4000))] == \
+        [8, 1, 4, 2, 1, 8, 1]

@@ -8,6 +8,7 @@ import math
 import pytest
 import torch
 
+from loqa_hub_amd import ops
 from loqa_hub_amd.ops import seqmix
 
 pytestmark = pytest.mark.gpu
@@ -67,10 +68,9 @@ def test_every_block_height(B, T, H):
 @pytest.mark.parametrize("feeds,pasts,H,window", [([33], [2100], 8, 0), ([1, 64, 40], [4000, 450, 700], 4, 0), ([100, 7], [1200, 1500], 16, 0),
                                                   ([130], [3000], 8, 1030), ([64, 64], [1530, 600], 16, 0)])
 def test_parts_of_the_keys(feeds, pasts, H, window):
-    """One to four parts of a block's keys in workgroups of their own, uneven ones, blocks of other lengths in one launch."""
+    """One to eight parts of a block's keys in workgroups of their own, uneven ones, blocks of other lengths in one launch."""
     kept = sum(min(f + p, f + window - 1) if window else f + p for f, p in zip(feeds, pasts))
-    parts, rows = seqmix._latent_parts(max(feeds), H * len(feeds), kept // len(feeds))
-    assert parts > 1 and rows == 64
+    assert ops.attn_parts(max(feeds), H * len(feeds), kept // len(feeds)) > 1
     for DK, DV in ((192, 128), (256, 64), (64, 64)):
         _check(feeds, pasts, H, DK, DV, DV - 12, window=window, sink=True, gate=True, seed=DK)
     _check(feeds, pasts, H, 128, 128, 128, window=window, scale=-0.05, seed=5)
