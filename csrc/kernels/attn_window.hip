@@ -978,13 +978,14 @@ extern "C" int loqa_qk_prep_append(const void* u, int dt, long ldu, int H, int G
   return (int)hipGetLastError();
 }
 
-extern "C" int loqa_window_attention(const void* q, int dt, const void* kc, const void* vc, int blk,
+static int window_attention(const void* q, int dt, const void* kc, const void* vc, int blk,
                                      int nblocks, const void* cu_q, const void* ctx, const void* bt,
                                      int max_blocks, const void* pos, const void* gate, long gate_ld,
                                      float scale, float cap, int window, int keep_first, int B,
                                      int T, int H, int G, int D, int Dv, int max_q, int mfma,
                                      void* o, long o_ld, int ns, void* part, const void* sink,
-                                     const void* slopes, hipStream_t st) {
+                                     const void* slopes, int parts, long part_floats, int* words, long tickets,
+                                     hipStream_t st) {
   if (T <= 0) return 0;
   if (B <= 0 || H <= 0 || G <= 0 || H % G || D <= 0 || D > 512 || Dv <= 0 || Dv > 512 || blk <= 0 ||
       o_ld < (long)H * Dv)
@@ -1000,6 +1001,9 @@ extern "C" int loqa_window_attention(const void* q, int dt, const void* kc, cons
   // the matrix-core form reads the gate and writes the output in 8-byte runs
   const bool runs_ok = (!gate || (gate_ld % 4 == 0 && ((size_t)gate & 7) == 0)) && o_ld % 4 == 0 &&
                        ((size_t)o & 7) == 0;
+  p.parts = parts; p.words = words; p.part_floats = part_floats; p.tickets = tickets;
+  if (parts < 1 || (parts > 1 && (!mfma || !part || !words || ((size_t)part & 15)))) return (int)hipErrorInvalidValue;
+  if (parts > 1) p.part = (float*)part;
   if (mfma && dt == 0 && D % 8 == 0 && D <= 256 && Dv % 8 == 0 && Dv <= 512 && runs_ok)
     return window_attention_mfma(p, max_q, st);
   if (ns > 1 && part) { p.ns = ns; p.part = (float*)part; }
@@ -1054,4 +1058,32 @@ extern "C" int loqa_window_attention(const void* q, int dt, const void* kc, cons
       hipLaunchKernelGGL(window_attn_combine_kernel<float>, dim3(T, H), dim3(128), 0, st, p);
   }
   return (int)hipGetLastError();
+}
+
+extern "C" int loqa_window_attention(const void* q, int dt, const void* kc, const void* vc, int blk,
+                                     int nblocks, const void* cu_q, const void* ctx, const void* bt,
+                                     int max_blocks, const void* pos, const void* gate, long gate_ld,
+                                     float scale, float cap, int window, int keep_first, int B,
+                                     int T, int H, int G, int D, int Dv, int max_q, int mfma,
+                                     void* o, long o_ld, int ns, void* part, const void* sink,
+                                     const void* slopes, hipStream_t st) {
+  return window_attention(q, dt, kc, vc, blk, nblocks, cu_q, ctx, bt, max_blocks, pos, gate, gate_ld, scale, cap, window, keep_first,
+                          B, T, H, G, D, Dv, max_q, mfma, o, o_ld, ns, part, sink, slopes, 1, 0,
+                          nullptr, 0, st);
+}
+
+// The same with up to `parts` parts of a row block's keys in workgroups of their own, where the sizes and
+// scores take them: `part` (part_floats of them) and `words` (zeroed, `tickets` TICKETs) are theirs. An entry of its own,
+// as a token step is host work and every argument is a part of it (four more: 23.5 -> 23.8 us).
+extern "C" int loqa_window_attention_parts(const void* q, int dt, const void* kc, const void* vc, int blk,
+                                     int nblocks, const void* cu_q, const void* ctx, const void* bt,
+                                     int max_blocks, const void* pos, const void* gate, long gate_ld,
+                                     float scale, float cap, int window, int keep_first, int B,
+                                     int T, int H, int G, int D, int Dv, int max_q, int mfma,
+                                     void* o, long o_ld, int ns, void* part, const void* sink,
+                                     const void* slopes, int parts, long part_floats, int* words, long tickets,
+                                     hipStream_t st) {
+  return window_attention(q, dt, kc, vc, blk, nblocks, cu_q, ctx, bt, max_blocks, pos, gate, gate_ld, scale, cap, window, keep_first,
+                          B, T, H, G, D, Dv, max_q, mfma, o, o_ld, ns, part, sink, slopes, parts,
+                          part_floats, words, tickets, st);
 }

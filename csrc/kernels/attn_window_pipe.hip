@@ -8,7 +8,9 @@
 // and denominator are of the same rounded weights (flash_pipe.h has the errors).
 // What bounds it at 128 columns: MFMAs, LDS and L2 about alike (flash_pipe.h). 2048 rows of 16
 // heads (4 key heads) of 128, window 1024: 92 us before (256 rows a workgroup, half of the CUs;
-// tiles through registers; maximum, exponentials and products one after the other), 35 now; without a window 128, 50; 64 rows behind 2000: 99, 29.
+// tiles through registers; maximum, exponentials and products one after the other), 35 now; without a window 128, 50. Few rows
+// behind many keys: parts of a block's keys in workgroups of their own, joined in the launch (fl_join; 16 heads of 128, 64
+// rows behind 2000 42.6 -> 22.7 us, with a window of 1024 27.5 -> 21.8, 128 behind 8000 139 -> 36).
 #include "flash_pipe.h"
 #include "seqmix.h"
 
@@ -21,10 +23,11 @@ template <int DK, int DV, int QW, int KS, bool GEN>
 __global__ __launch_bounds__(64 * QW * KS, 2) void window_attn_pipe_kernel(WinAttnParams p) {
   using L = FlashLds<DK, DV>;
   constexpr int NS = DK / 16, NDT = DV / 32, NTH = 64 * QW;
+  constexpr bool PARTS = QW == 2;      // the launch has parts of 64-row blocks only
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int run = wave / QW, wq = wave % QW, th = threadIdx.x - run * NTH, h = lane >> 5;
-  int bx, head, v0, b;
+  int bx, head, v0, b, share = 0;
   {
     // row blocks with the most keys first, over all heads of an XCD where these are whole
     const int gx = gridDim.x, gy = gridDim.y, heads = gy * gridDim.z;
@@ -37,6 +40,10 @@ __global__ __launch_bounds__(64 * QW * KS, 2) void window_attn_pipe_kernel(WinAt
       hd = xcd * hp + in - bx * hp;
     }
     bx = gx - 1 - bx;
+    if (PARTS && p.parts > 1) {
+      share = bx % p.parts;
+      bx /= p.parts;
+    }
     b = hd / gy;
     head = (hd - b * gy) / p.vparts;
     v0 = ((hd - b * gy) - head * p.vparts) * DV;            // this workgroup's value columns
@@ -50,17 +57,25 @@ __global__ __launch_bounds__(64 * QW * KS, 2) void window_attn_pipe_kernel(WinAt
   const bool valid = qi < qlen;
   const int qpos = p.pos[q0 + min(qi, row_hi)];
   const int pos_lo = p.pos[q0 + row_lo];
-  const int kend = min(p.ctx[b], p.pos[q0 + row_hi] + 1);   // positions grow along a feed
+  int kend = min(p.ctx[b], p.pos[q0 + row_hi] + 1);   // positions grow along a feed
   // key tiles: those holding kept first tokens, then from the first window on
   const int wg_lo = p.window > 0 ? max(0, pos_lo - p.window + 1) : 0;
   const int lo_t = wg_lo / FL_KEYS * FL_KEYS;
   const int n1 = p.window > 0 ? min((min(p.keep_first, wg_lo) + FL_KEYS - 1) / FL_KEYS, lo_t / FL_KEYS) : 0;
-  const int ntiles = kend > 0 ? n1 + max(kend - lo_t + FL_KEYS - 1, 0) / FL_KEYS : 0;
+  int ntiles = kend > 0 ? n1 + max(kend - lo_t + FL_KEYS - 1, 0) / FL_KEYS : 0, parts = 1, t0 = 0;
   auto tile_at = [&](int i) { return i < n1 ? i * FL_KEYS : lo_t + (i - n1) * FL_KEYS; };
+  if (PARTS && p.parts > 1) {
+    parts = max(1, min(p.parts, ntiles / FL_CAP));
+    if (share >= parts) return;                             // uniform
+    const int len = (ntiles + parts - 1) / parts;
+    t0 = share * len;
+    if (t0 + len < ntiles) kend = min(kend, tile_at(t0 + len));
+    ntiles = min(t0 + len, ntiles);                         // past the part's last tile
+  }
   // what this wave's rows can see
   const int wpos_lo = __builtin_amdgcn_readfirstlane(p.pos[q0 + min(row_lo + wq * 32, row_hi)]);
   const int wpos_hi = __builtin_amdgcn_readfirstlane(p.pos[q0 + min(row_lo + wq * 32 + 31, row_hi)]);
-  const int per = (ntiles + KS - 1) / KS, first = run * per;
+  const int per = (max(ntiles - t0, 0) + KS - 1) / KS, first = t0 + run * per;
 
   bf16x8 qf[NS];
   {
@@ -146,6 +161,12 @@ __global__ __launch_bounds__(64 * QW * KS, 2) void window_attn_pipe_kernel(WinAt
   fl_sync();                                                // every wave is done with the rings
   fl_merge<NDT, QW, KS>(acc, m, l, reinterpret_cast<float*>(lds), run, wq, lane);
   if (run) return;
+  if (PARTS && parts > 1) {
+    const int block = (b * (int)gridDim.y + head * p.vparts + v0 / DV) * (int)(gridDim.x / p.parts) + bx;
+    if (!fl_join<NDT, QW>(acc, m, l, p.part + (size_t)block * p.parts * QW * fl_join_floats(NDT), p.words + (size_t)block * TICKET,
+                          parts, share, wq, lane))
+      return;
+  }
   float inv = l > 0.f ? 1.f / l : 0.f;
   if (p.sink) {
     // the running maximum and sum are in the base-2 domain
@@ -181,7 +202,11 @@ static int launch(const WinAttnParams& p, int max_q, hipStream_t st) {
   constexpr int ring = KS * FlashLds<DK, DV>::RING, end = fl_merge_bytes(DV / 32, QW, KS) + QW * fl_store_bytes(DV / 32);
   constexpr int bytes = ring > end ? ring : end;
   static_assert(bytes <= 160 * 1024, "LDS of a CU");
-  const dim3 grid((max_q + 32 * QW - 1) / (32 * QW), p.H * p.vparts, p.B);
+  const long blocks = (max_q + 32 * QW - 1) / (32 * QW), all = blocks * p.H * p.vparts * p.B;
+  if (p.parts > 1 && (QW != 2 || p.parts > FL_PARTS || all > p.tickets ||
+                      all * p.parts * QW * fl_join_floats(DV / 32) > p.part_floats))
+    return (int)hipErrorInvalidValue;
+  const dim3 grid(blocks * p.parts, p.H * p.vparts, p.B);
   hipLaunchKernelGGL((window_attn_pipe_kernel<DK, DV, QW, KS, GEN>), grid, dim3(64 * QW * KS), bytes, st, p);
   return (int)hipGetLastError();
 }
@@ -194,8 +219,9 @@ static int launch(const WinAttnParams& p, int max_q, hipStream_t st) {
 // be four more kernels to build (100 rows x 8 heads of 128: 12.4, with it 11.6; 320 behind 1000
 // x 16: 51, 47).
 template <int DK, int DV>
-static int launch_rows(const WinAttnParams& p, int max_q, hipStream_t st) {
+static int launch_rows(WinAttnParams p, int max_q, hipStream_t st) {
   const long hd = (long)p.H * p.vparts * p.B, n64 = (max_q + 63) / 64 * hd, n128 = (max_q + 127) / 128 * hd;
+  if (n64 > 128 || p.cap > 0.f || p.slopes || !(p.scale > 0.f)) p.parts = 1;   // parts only of the first form
   const bool one = n128 > (max_q <= 128 ? 256 : 512);
   if (p.cap > 0.f || p.slopes || !(p.scale > 0.f))
     return one ? launch<DK, DV, 4, 1, true>(p, max_q, st) : launch<DK, DV, 4, 2, true>(p, max_q, st);

@@ -154,6 +154,8 @@ struct WinAttnParams {
   const float* slopes;               // [H] or null: slopes[h] * (i - j) comes off head h's score
   long o_ld;                         // row stride of o (head h at column h * Dv)
   int vparts;                        // matrix-core form: workgroups that share a head's value columns
+  int parts; int* words;             // pipelined form: parts of a row block's keys at most, in part and these (fl_join)
+  long part_floats, tickets;         // how much of both there is
 };
 // Prompt portions on the pipelined tile loop; -1 where it does not take the sizes or places.
 int window_attention_pipe(const WinAttnParams& p, int max_q, hipStream_t st);

@@ -261,6 +261,9 @@ _SEQMIX_SIGS = {
     "loqa_window_attention": [_vp, _i, _vp, _vp, _i, _i, _vp, _vp, _vp, _i, _vp, _vp, _l, _f, _f,
                               _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _vp, _l, _i, _vp, _vp, _vp,
                               _vp],
+    "loqa_window_attention_parts": [_vp, _i, _vp, _vp, _i, _i, _vp, _vp, _vp, _i, _vp, _vp, _l, _f, _f,
+                                    _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _vp, _l, _i, _vp, _vp, _vp,
+                                    _i, _l, _vp, _l, _vp],
     "loqa_mamba2_prep": [_vp, _i, _l, _i, _i, _i, _i, _vp, _i, _vp, _vp, _vp, _vp, _i, _vp, _vp,
                          _vp, _i, _i, _vp, _vp, _vp],
     "loqa_residual_rms1p": [_vp, _vp, _f, _vp, _f, _vp, _f, _i, _vp, _vp, _vp, _f, _vp, _vp, _i,

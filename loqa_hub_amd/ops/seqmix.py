@@ -1003,13 +1003,22 @@ def window_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
         part = torch.empty(T * H * key_splits * (Dv + 2), dtype=torch.float32, device=q.device)
     else:
         key_splits = 1
+    call, extra, st = "loqa_window_attention", (), stream_ptr(q)
+    if mfma and D <= 128 and not softcap and slopes is None and scale > 0:
+        vparts, width = -(-Dv // 128), 64 if Dv <= 64 else 128
+        keys = int(max_ctx) if window <= 0 else min(int(max_ctx), window + 64 + keep_first)
+        parts = attn_parts(int(max_q), H * vparts * B, keys)
+        if parts > 1:       # a wave's 32 rows: width / 2 accumulators a lane, maximum and sum
+            blocks = -(-max_q // 64) * H * vparts * B
+            part, words = _sk_workspace(q.device, st, blocks * parts * 2 * (width // 2 + 4) * 64, blocks)
+            call, extra = "loqa_window_attention_parts", (parts, part.numel(), ptr(words), words.numel())
     if T:
-        check(kernels().loqa_window_attention(
+        check(getattr(kernels(), call)(
             ptr(q), _dt(q), ptr(k_cache), ptr(v_cache), k_cache.shape[1], k_cache.shape[0],
             ptr(cu_q), ptr(ctx_lens), ptr(block_tables), block_tables.shape[1], ptr(positions),
             ptr(gate), gs, float(scale), float(softcap), int(window), int(keep_first), B, T, H, G,
             D, Dv, int(max_q), int(mfma), ptr(o), o.stride(0), int(key_splits), ptr(part), ptr(sink),
-            ptr(slopes), stream_ptr(q)), "window_attention")
+            ptr(slopes), *extra, st), "window_attention")
     return o
 
 

@@ -9,6 +9,7 @@ import math
 import pytest
 import torch
 
+from loqa_hub_amd import ops
 from loqa_hub_amd.ops import seqmix
 
 pytestmark = pytest.mark.gpu
@@ -128,3 +129,15 @@ def test_many_short_feeds(cap):
         ctx, pos = torch.full((B,), n, dtype=torch.int32, device=DEV), torch.arange(n, dtype=torch.int32, device=DEV).repeat(B)
         return lambda: seqmix.window_attention(q, kc, kc, cu, ctx, bt, pos, 0.125, cap, 300, 0, None, H, 8, D, D, max_q=n, max_ctx=n)
     assert _us(call(9)) < 1.4 * _us(call(8))
+
+
+@pytest.mark.parametrize("feeds,pasts,H,window,keep", [([33], [2100], 8, 0, 0), ([1, 64, 40], [4000, 450, 700], 4, 0, 0), ([100, 7], [1200, 1500], 8, 0, 0),
+                                                       ([130], [3000], 8, 1030, 70), ([64], [1500], 16, 1100, 200)])
+def test_parts_of_the_keys(feeds, pasts, H, window, keep):
+    """One to eight parts of a block's keys in workgroups of their own; parts that end among the kept tokens' tiles."""
+    keys = min(max(f + p for f, p in zip(feeds, pasts)), window + 64 + keep if window else 1 << 30)
+    assert ops.attn_parts(max(feeds), H * len(feeds), keys) > 1
+    _check(feeds, pasts, H, 2, 128, 128, window, keep, sink=True, gate=True, seed=1)
+    _check(feeds, pasts, H, 4, 64, 64, window, keep, seed=2)
+    _check(feeds, pasts, H, 4, 96, 200, window, keep, sink=True, seed=3)
+    _check(feeds, pasts, H, 4, 64, 72, window, keep, cap=30.0, seed=4)      # transformed scores: whole
