@@ -341,7 +341,9 @@ class LlamaModel:
     def embed(self, tokens: torch.Tensor) -> torch.Tensor:
         tp = self.w.tp
         if tp.world == 1 or self.w.embed.shape[0] == self.cfg.vocab_size:   # replicated table
-            return torch.nn.functional.embedding(tokens.long(), self.w.embed)
+            # 32-bit ids as they are: a cast would be a launch of its own
+            ids = tokens if tokens.dtype in (torch.int32, torch.int64) else tokens.long()
+            return torch.nn.functional.embedding(ids, self.w.embed)
         lo = tp.rank * self.w.v
         local = tokens.long() - lo
         inr = (local >= 0) & (local < self.w.v)
@@ -643,10 +645,12 @@ class LlamaModel:
         if (hidden.is_cuda and getattr(w, "lm_head_p", None) is not None
                 and B <= ops.MPADS[-1]):
             Mpad = ops.mpad_for(B)
-            x = hidden
-            if Mpad != B:
+            x = hidden.contiguous()
+            if B == 1:          # a prompt's one row in place of padding rows (zeros and a copy: two launches)
+                x = x.expand(Mpad, -1)
+            elif Mpad != B:
                 x = torch.zeros(Mpad, hidden.shape[1], dtype=hidden.dtype, device=hidden.device)
                 x[:B] = hidden
-            return ops.skinny_gemm(x.contiguous(), w.lm_head_p, 1,
+            return ops.skinny_gemm(x, w.lm_head_p, 1,
                                    max_wgs=getattr(w, "max_wgs", ops.MAX_DECODE_WGS))[0][:B, :w.v]
         return ops.linear(hidden, w.lm_head)

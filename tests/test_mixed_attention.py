@@ -103,3 +103,17 @@ def test_mixed_split_planning_cpu():
     assert plan([0, 1], [[1], [2] * 5], ws_tokens=0)[0] is None               # workspace too small
     assert plan([0, 1], [[1], [2] * 5], on=False)[0] is None                  # LOQA_MIXED_SPLIT_ATTN=0
     assert plan([0, 1], [[1], [2] * 5], ws_counters=4)[0] is None             # counters too few
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B", [1, 2, 16])
+def test_logits_rows_do_not_depend_on_their_padding(B):
+    """One row is read sixteen times, others are padded with zeros: a row's logits are the same, and ids of every width embed."""
+    from loqa_hub_amd.models.configs import llama_config
+    from loqa_hub_amd.models.llama import LlamaModel, LlamaWeights
+    m = LlamaModel(LlamaWeights(llama_config("test-tiny"), torch.device("cuda", 0), seed=4))
+    hidden = torch.randn(16, m.cfg.d_model, device="cuda").bfloat16()
+    assert torch.equal(m.logits(hidden[:B]), m.logits(hidden)[:B])
+    assert torch.equal(m.logits(hidden.repeat(1, 2)[:B, :m.cfg.d_model]), m.logits(hidden)[:B])
+    ids = torch.tensor([5, 0, 7, 5], device="cuda")
+    assert all(torch.equal(m.embed(ids.to(t)), m.w.embed[ids]) for t in (torch.int64, torch.int32, torch.int16))
