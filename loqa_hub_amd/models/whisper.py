@@ -194,6 +194,8 @@ class WhisperModel:
         self.w = w
         self.cfg = w.cfg
         self.mel = MelConstants.create(self.cfg.n_mels)
+        # where the windows of a pass start: for up to 64 of them not a launch of every pass
+        self.starts = torch.arange(65, dtype=torch.int32, device=w.tok_embed.device) * self.cfg.n_audio_ctx
 
     # ----------------------------------------------------------------- encoder
     def encode(self, audio: torch.Tensor) -> torch.Tensor:
@@ -219,7 +221,8 @@ class WhisperModel:
             x = ops.linear(cols2, w.conv2_w)                      # [B*1500, d]
             ops.gelu_bias_(x, w.conv2_b, w.pos_enc)               # + positional embedding
         T = cfg.n_audio_ctx
-        cu = torch.arange(0, (B + 1) * T, T, dtype=torch.int32, device=audio.device)
+        cu = self.starts[:B + 1] if B <= 64 and self.starts.device == audio.device else \
+            torch.arange(0, (B + 1) * T, T, dtype=torch.int32, device=audio.device)
         H, D = cfg.n_heads, cfg.head_dim
         if tile and ENC_SK:
             return self._encode_sk(x, cu, T)
