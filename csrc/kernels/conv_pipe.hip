@@ -113,13 +113,14 @@ template <int FN, int FM, int NA, int NB> static int cp_launch(const ConvPipePar
   return (int)hipGetLastError();
 }
 
-// layout: numbers of the pipelined projections' tiles (128 x 64, 128 x 128, 256 x 128)
+// layout: numbers of the pipelined projections' tiles (64 x 64, 128 x 64, 128 x 128, 256 x 128)
 extern "C" int loqa_conv_pipe(const ConvPipeParams* p, hipStream_t st) {
   if (!p || !p->x || !p->w || !p->y || p->M <= 0 || p->cin <= 0 || p->cin % GP_BK || p->stride < 1 || p->tin < 1 ||
       p->tout != (p->tin - 1) / p->stride + 1 || p->M % p->tout || p->ldx < p->cin || p->ldx % 8 || p->ldy % 8 ||
       (p->pos && p->pos_rows < 1) || (((size_t)p->x | (size_t)p->w | (size_t)p->y | (size_t)p->pos) & 15))
     return (int)hipErrorInvalidValue;
   switch (p->layout) {
+    case 11: return cp_launch<2, 2, 5, 5>(*p, st);
     case 19: return cp_launch<4, 2, 4, 4>(*p, st);
     case 20: return cp_launch<4, 4, 5, 5>(*p, st);
     case 15: return cp_launch<8, 4, 3, 3>(*p, st);

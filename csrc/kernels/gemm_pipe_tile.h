@@ -339,6 +339,7 @@ static int gp_launch(const GemmSkCall& p, hipStream_t st) {
 // what they wait for is the first touch of cold weights
 template <bool AHEAD, bool SPLIT> static int gp_layout(const GemmSkCall& p, int layout, hipStream_t st) {
   switch (layout) {
+    case -1: return gp_launch<2, 2, 5, 5, AHEAD, SPLIT>(p, st);  // 64 x 64
     case 0: return gp_launch<8, 8, 3, 2, AHEAD, SPLIT>(p, st);   // 256 x 256
     case 1: return gp_launch<8, 6, 3, 2, AHEAD, SPLIT>(p, st);   // 256 x 192
     case 2: return gp_launch<6, 8, 3, 2, AHEAD, SPLIT>(p, st);   // 192 x 256

@@ -207,7 +207,7 @@ extern "C" int loqa_gemm_sk(const GemmSkCall* p, hipStream_t st) {
   if (p->S > 1 && (!p->ws || !p->counters)) return (int)hipErrorInvalidValue;
   if (p->ldx % 8 || p->ldy % 4) return (int)hipErrorInvalidValue;
   if ((p->epi == SK_SWIGLU && p->bias) || (p->epi != SK_BF16 && p->act)) return (int)hipErrorInvalidValue;
-  if (p->ahead_wgs && p->layout < 12) return (int)hipErrorInvalidValue;
+  if (p->ahead_wgs && p->layout < 11) return (int)hipErrorInvalidValue;
   switch (p->layout) {
     case 1: return sk_launch<2, 2, 4, 2, 2>(*p, st);
     case 7: return sk_launch<2, 2, 2, 2, 2>(*p, st);

@@ -1696,24 +1696,25 @@ def graph_capture(graph: "torch.cuda.CUDAGraph", **kw):
 # Split-K tiled GEMM with an in-launch reduction (csrc/kernels/gemm_sk.hip, gemm_pipe.hip)
 _SK_EPI = {"bf16": 0, "swiglu": 1, "resid": 2}
 # layout -> (features, rows, us a K step of 64 takes a compute unit, us around a tile's K
-# loop): 1 and 7 are the general form, 12 on the pipelined tiles, one workgroup per CU. Times
+# loop): 1 and 7 are the general form, 11 on the pipelined tiles, one workgroup per CU. Times
 # fitted to measured ones without an epilogue of weight: they are there to rank, and 0.69 to 1.26
-# of what a whole unsplit call takes (0.73 on average with GELU). Over 60 shapes (80 to 9000 rows, N 512
+# of what a whole unsplit call takes (0.73 on average with GELU). Over 75 shapes (80 to 9000 rows, N 384
 # to 28672, K 512 to 14336, cold weights, every layout and K split: profiles/gemm_plan_grid.txt)
-# the plan is the fastest in 50, 0.7 % behind the fastest on average and 8.3 % at worst (1500 x 1280 x
-# 5120 whole on 128 x 64: 29.9 us, 27.6 in three chunks of 128 x 192).
-SK_LAYOUTS = {1: (128, 64, 0.60, 4.0), 7: (64, 64, 0.55, 4.0),
+# the plan is the fastest in 59, 1.2 % behind the fastest on average and 22 % at worst (160 x 6144 x 4096 in
+# five chunks of 128 x 192: 25.9 us, 21.2 in four). Layout 18 is 1.4 us dearer with GELU than without, which counts for more.
+SK_LAYOUTS = {1: (128, 64, 0.60, 4.0), 7: (64, 64, 0.55, 4.0), 11: (64, 64, 0.19, 2.6),
               12: (256, 256, 1.20, 10.3), 13: (256, 192, 1.075, 5.5), 14: (192, 256, 1.073, 5.5),
               15: (256, 128, 0.908, 4.0), 16: (128, 256, 0.784, 6.6), 17: (128, 192, 0.667, 4.6),
-              18: (192, 192, 0.854, 4.6), 19: (128, 64, 0.309, 4.3), 20: (128, 128, 0.498, 3.6)}
-SK_PIPE = 12              # the first pipelined layout
+              18: (192, 192, 0.854, 6.0), 19: (128, 64, 0.309, 4.3), 20: (128, 128, 0.498, 3.6)}
+SK_PIPE = 11              # the first pipelined layout
 SK_WHOLE = 12             # the layout that the plan does not split along K
 # numbers of layouts that are gone (other stage counts and wave splits of the general form, 256
 # features x 64 rows) -> the pipelined tile of that size, or the next smaller one
-SK_RENAMED = {0: 20, 2: 19, 3: 15, 4: 19, 5: 20, 6: 12, 8: 19, 9: 15, 10: 20, 11: 19}
+SK_RENAMED = {0: 20, 2: 19, 3: 15, 4: 19, 5: 20, 6: 12, 8: 19, 9: 15, 10: 20}
 SK_CUS = 256
 SK_FEW = 96
-SK_WORTH = 1.03
+SK_SHARED = (700, 200)    # rows, workgroups
+SK_SMALL = 11             # the 64 x 64 tiles
 SK_GELU = 1.3e-4
 SK_PAIRED = 17            # two workgroups a compute unit, with GELU
 _SK_WS: dict = {}
@@ -1723,12 +1724,15 @@ def gemm_sk_plan(M: int, N: int, K: int, epi: str = "bf16", layouts=None, *,
                  pipe: bool = True) -> tuple[int, int]:
     """(layout, K chunks) for a shape: the fewest microseconds by SK_LAYOUTS, counting whole
     rounds of tiles over the compute units; up to SK_FEW workgroups load so little beside each other that
-    a K step takes 0.8 of its time (1500 x 512 x 2048 on 96 of them 11.0 us, in two chunks on 192 11.6).
+    a K step takes 0.8 of its time (1500 x 512 x 2048 on 96 of them 11.0 us, in two chunks on 192 11.6), and where eight or more
+    row blocks share the weights, up to SK_SHARED workgroups, 0.9 (1500 x 768 x 3072 on 144 17.1 us, 320 x 4096 x 4096
+    on 160 29). 64 x 64 tiles are for what leaves half of the units idle in 128 x 64 (1500 x 512 x 2048 11.1 -> 8.9 us, x
+    512 5.7 -> 4.7, 300 x 1280 x 1280 9.0 -> 6.6); from K = 2048 on their steps take longer.
     K chunks fill the chip where the tiles do not; each tile then pays for the trip of its f32 partials
-    through memory, 2 us and 40 us a MB, and 4 us a MB for each chunk that is read back (fitted with the
-    rest; 320 x 4096 x 4096 in four chunks of 128 x 192 22.2 us, whole 27.3 in 128 x 64). They have to be faster by SK_WORTH:
-    their partials and the weights that a launch touches for the next one (:func:`_ahead`) hold each other up (1500 x
-    1280 x 5120 in two chunks 28.3 us and whole 29.9 alone, but an encoder pass with 32 of them 4118 us and 4058). Never on 256 x 256
+    through memory, 3 us and 40 us a MB, and 4 us a MB for each chunk that is read back (fitted with the
+    rest; 320 x 4096 x 4096 in four chunks of 128 x 192 22.2 us, whole 27.3 in 128 x 64). Their partials and the weights
+    that a launch touches for the next one (:func:`_ahead`) hold each other up (1500 x 1280 x 5120 in two chunks 28.3 us and whole
+    29.9 alone, but an encoder pass with 32 of them 4118 us and 4058). Never on 256 x 256
     tiles: these fill the chip with MFMAs, where a K step takes longer than the fit has it (4096 x
     14336: 1280 rows in three chunks 160 us, the 256 x 192 tiles in two 135; 2048 rows in two 205,
     the 128 x 256 tiles whole 182; the fastest in none of the 60 shapes). ``pipe`` False:
@@ -1753,16 +1757,19 @@ def _sk_plan(M: int, N: int, K: int, pipe: bool, layouts: tuple | None = None, g
         if N % bn or (lay >= SK_PIPE) != (pipe and N % 128 == 0) or lay not in only:
             continue
         tiles = -(-M // bm) * (N // bn)
+        if lay == SK_SMALL and K > 2048:
+            step *= 1.26
         for s in (1, 2, 3, 4, 5, 6, 8):
             if s > 1 and (KT // s < 8 or lay == SK_WHOLE):
                 continue
+            few = 0.8 if tiles * s <= SK_FEW else 0.9 if M >= SK_SHARED[0] and tiles * s <= SK_SHARED[1] else 1.0
             end = around + (SK_GELU * bn * bm / s if gelu and lay >= SK_PIPE else 0.0)
-            t = -(-tiles * s // SK_CUS) * (-(-KT // s) * step * (0.8 if tiles * s <= SK_FEW else 1.0) + end)
+            t = -(-tiles * s // SK_CUS) * (-(-KT // s) * step * few + end)
             if gelu and lay == SK_PAIRED and s == 1 and tiles > SK_CUS:
                 full, rest = divmod(tiles, 2 * SK_CUS)
                 t = 2.4 + (9.0 + 1.12 * KT) * (full + (0.0 if not rest else 0.68 if rest <= SK_CUS else 1.0))
             if s > 1:
-                t = SK_WORTH * (t + 2.0 + bn * bm * 4e-6 * (40 + 4 * s))
+                t += 3.0 + bn * bm * 4e-6 * (40 + 4 * s)
             if t < best_t:
                 best, best_t = (lay, s), t
     return best
@@ -2003,7 +2010,7 @@ def gemm_ws(x: torch.Tensor, w: torch.Tensor, *, epi: str = "bf16", bias: torch.
 
 # ---------------------------------------------------------------------------
 # Conv stem of the Whisper encoder (csrc/kernels/conv_pipe.hip)
-CONV_LAYOUTS = (15, 19, 20)
+CONV_LAYOUTS = (11, 15, 19, 20)
 
 
 def conv_k3_gelu(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor, B: int, stride: int,

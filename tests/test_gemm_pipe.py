@@ -154,3 +154,11 @@ def test_the_plan_with_gelu():
     for M, N, K in ((100, 2048, 512), (1500, 2048, 512), (6000, 5120, 1280)):
         assert ops.gemm_sk_plan(M, N, K, "gelu") == ops.gemm_sk_plan(M, N, K) and ops.gemm_sk_plan(M, N, K)[0] != ops.SK_PAIRED
     assert ops.gemm_sk_plan(9000, 1088, 512, "gelu")[0] in (1, 7)
+
+
+def test_the_plan_takes_small_tiles_for_small_grids():
+    for M, N, K in ((1500, 512, 512), (1500, 512, 2048), (300, 1280, 1280), (1500, 384, 1536)):
+        assert ops.gemm_sk_plan(M, N, K) == (ops.SK_SMALL, 1)
+    for M, N, K in ((1500, 768, 3072), (1500, 1280, 1280), (9000, 512, 512), (320, 4096, 14336)):
+        assert ops.gemm_sk_plan(M, N, K)[0] != ops.SK_SMALL
+    assert not ops.gemm_sk_plan(1500, 576, 2048)[0] >= ops.SK_PIPE          # whole 128 features, as every pipelined tile
