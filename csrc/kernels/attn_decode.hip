@@ -75,7 +75,9 @@ extern "C" int loqa_attn_decode(const void* q, long long q_stride, const void* k
                       o_stride, 0, 0, g_loqa_launch_prio, 0};
   if (waves != 4 && waves != 8) return (int)hipErrorInvalidValue;
   int err = 0;
-  if (waves == 4 && !pf && attn_stream(a, B, max_q, D, s, &err)) return err;
+  const bool stream = !(pf & 2);   // 2: the form that the GEMM prologues run (gemm_skinny.hip), whatever the rows
+  pf &= 1;
+  if (stream && waves == 4 && !pf && attn_stream(a, B, max_q, D, s, &err)) return err;
   if (waves == 8) {   // 512 threads: 2 waves per SIMD, 256 registers each (no PF at D = 128)
     if (D == 128)
       hipLaunchKernelGGL((attn_decode_kernel<128, 0, 8, 1>), grid, dim3(512), 0, s, a);

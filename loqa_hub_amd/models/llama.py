@@ -554,7 +554,7 @@ class LlamaModel:
                     attn=dict(cu_q=meta.cu_q, ctx_lens=meta.ctx_lens,
                               block_tables=meta.block_tables, max_q=meta.max_q,
                               split_keys=split_keys, num_splits=num_splits, workspace=attn_ws,
-                              max_k=meta.max_ctx, out=ao))
+                              max_k=meta.max_ctx, out=ao, streamed=tp.world == 1))   # tensor parallel: as the prologues
             else:
                 ops.skinny_fused(residual, P["wqkv_f"], "rope", scratch, norm=True,
                                  eps=cfg.norm_eps,

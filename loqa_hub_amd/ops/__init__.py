@@ -202,13 +202,15 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu_q: torch.Ten
               block_tables: torch.Tensor | None = None, scale: float | None = None,
               grouped: bool = False, split_keys: int = 256, num_splits: int = 1,
               workspace: AttnWorkspace | None = None, out: torch.Tensor | None = None,
-              max_k: int | None = None) -> torch.Tensor:
+              max_k: int | None = None, streamed: bool = True) -> torch.Tensor:
     """Varlen flash attention.
 
     q: [Tq, >=H*D] (row stride may exceed H*D, e.g. a view into the fused QKV
     output). K/V: contiguous [Tk, >=Hkv*D] with ``cu_k``, or paged caches
     [n_blocks, Hkv, BLK, D] with ``ctx_lens`` + ``block_tables``.
     Query i of sequence b sits at absolute position ctx_len_b - q_len_b + i.
+    ``streamed`` False: the decode kernel that the GEMM prologues run (attn_decode.hip), bit for
+    bit, also where attn_stream.hip takes the rows.
     Returns [Tq, H*D] bf16.
     """
     scale = scale if scale is not None else 1.0 / math.sqrt(head_dim)
@@ -261,7 +263,7 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu_q: torch.Ten
             ptr(out), out.stride(0), ptr(cu_q), ptr(ctx_lens),
             ptr(block_tables) if paged else None, max_blocks, blk, B, max_q, n_heads, n_kv,
             head_dim, scale, int(causal), split_keys, num_splits, ptr(workspace.part_o),
-            ptr(workspace.part_ml), Tq, ptr(workspace.counters), waves, pf, stream_ptr(q)),
+            ptr(workspace.part_ml), Tq, ptr(workspace.counters), waves, pf if streamed else pf | 2, stream_ptr(q)),
             "attn_decode")
         return out
     if grouped:
@@ -1284,7 +1286,7 @@ def skinny_fused(x: torch.Tensor, wp, mode: str, scratch: FusedScratch, *,
                              ctx_lens=attn["ctx_lens"], block_tables=attn["block_tables"],
                              scale=attn.get("scale"), grouped=True,
                              split_keys=attn["split_keys"], num_splits=attn["num_splits"],
-                             workspace=attn["workspace"], out=attn.get("out"),
+                             workspace=attn["workspace"], out=attn.get("out"), streamed=attn.get("streamed", True),
                              max_k=attn.get("max_k"))
         return attention(qq, attn["k"], attn["v"], attn["cu_q"], n_heads=n_heads, n_kv=n_kv,
                          head_dim=head_dim, causal=False, max_q=attn["max_q"],
@@ -1396,7 +1398,7 @@ def _prologue_standalone(pro: dict, x, scratch) -> None:
               n_kv=pro["n_kv"], head_dim=pro["k_cache"].shape[3], causal=True, max_q=pro["max_q"],
               ctx_lens=pro["ctx_lens"], block_tables=pro["block_tables"], scale=pro.get("scale"),
               grouped=True, split_keys=pro["split_keys"], num_splits=pro["num_splits"],
-              workspace=pro["workspace"], out=x, max_k=pro.get("max_k"))
+              workspace=pro["workspace"], out=x, max_k=pro.get("max_k"), streamed=False)
 # tensor-parallel decode steps with the all-reduces / attention as GEMM
 # prologues (models/llama.py _decode_fused_tp_prologue; grid cap:
 # CustomAllReduce.prologue_wgs). Off by default: 328 instead of 567 launches
@@ -1873,7 +1875,7 @@ def gemm_sk(x: torch.Tensor, w: torch.Tensor, *, epi: str = "bf16", bias: torch.
             out: torch.Tensor | None = None, layout: int | None = None,
             splits: int | None = None, ahead: tuple = ()) -> torch.Tensor:
     """Y = X W^T on the split-K tiled GEMM (``csrc/kernels/gemm_sk.hip``); the
-    S K-chunks of a tile are summed in-launch by the tile's last workgroup.
+    S K-chunks of a tile are summed in-launch, by all of the tile's workgroups on the pipelined tiles.
 
     x [M, K] bf16 (row stride may exceed K), w [N, K] bf16 row-major.
     ``epi``: "bf16" -> [M, N] (+ f32 ``bias``, ``act`` "gelu"); "swiglu" -> silu(gate) * up

@@ -100,7 +100,7 @@ class TPEmulation:
                                      ctx_lens=meta.ctx_lens, block_tables=meta.block_tables,
                                      grouped=grouped, split_keys=split_keys,
                                      num_splits=num_splits if grouped else 1,
-                                     workspace=e.attn_ws, max_k=meta.max_ctx)
+                                     workspace=e.attn_ws, max_k=meta.max_ctx, streamed=False)
                 ops.skinny_fused(attn, P["wo"], "act", scratch, out=partials[r], act="f32")
             self.resid(residual, partials)
             for r, e in enumerate(self.engines):
