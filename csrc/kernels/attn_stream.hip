@@ -162,7 +162,8 @@ __global__ __launch_bounds__(NW * 64) void attn_stream_kernel(AttnDecArgs A) {
     m_run = m_new;
     // Weights as two bf16, 16 bits of mantissa, which the memory's time covers: relative error against 64 bits of
     // 1500 keys 0.00204 with one in runs of 64 keys, 0.00208 in these longer runs (fewer weights are exactly
-    // one), 0.00165 with two
+    // one), 0.00165 with two. The upper one is cut off below the weight, so that the lower one is positive as well:
+    // an infinite value stays infinite, where a lower part of zero or below makes it NaN.
     typedef __bf16 b2 __attribute__((ext_vector_type(2)));
     typedef float f2 __attribute__((ext_vector_type(2)));
     bf16x8 ph, pl;
@@ -172,9 +173,9 @@ __global__ __launch_bounds__(NW * 64) void attn_stream_kernel(AttnDecArgs A) {
 #pragma unroll
       for (int j = 0; j < 4; j += 2) {
         const f2 e = {exp2f(st[t][j] - m_new), exp2f(st[t][j + 1] - m_new)};
-        const b2 hi = __builtin_convertvector(e, b2);
-        const unsigned hb = __builtin_bit_cast(unsigned, hi);
-        const b2 lo = __builtin_convertvector((f2{e[0] - __uint_as_float(hb << 16), e[1] - __uint_as_float(hb & 0xffff0000u)}), b2);
+        const unsigned h0 = __builtin_elementwise_sub_sat(__float_as_uint(e[0]), 1u), h1 = __builtin_elementwise_sub_sat(__float_as_uint(e[1]), 1u);
+        const b2 hi = __builtin_bit_cast(b2, __builtin_amdgcn_perm(h1, h0, 0x07060302u));   // the upper halves
+        const b2 lo = __builtin_convertvector((f2{e[0] - __uint_as_float(h0 & 0xffff0000u), e[1] - __uint_as_float(h1 & 0xffff0000u)}), b2);
         ls += e[0] + e[1];
         ph[4 * t + j] = hi[0];
         ph[4 * t + j + 1] = hi[1];

@@ -111,3 +111,61 @@ def test_replays_of_a_captured_call():
         rows = [c[bt[0].long()].transpose(1, 2).reshape(-1, Hkv, D)[:n] for c in (kc, vc)]
         _close(y, _reference(q, [rows[0]], [rows[1]], [1], H, H // Hkv, D, True))
         assert torch.equal(y, run())
+
+
+def _same_kind(a, b):
+    """Infinities and NaN where ``b`` has them, the other values close."""
+    a, fine = a.double(), b.isfinite()
+    assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.isfinite(), fine)
+    assert torch.equal(a[~fine & ~b.isnan()], b[~fine & ~b.isnan()])
+    _close(a[fine], b[fine])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,G", [(64, 1), (64, 4), (128, 8)])
+@pytest.mark.parametrize("keys", [1, 40, 700])
+def test_values_that_are_not_finite(D, G, keys):
+    """An infinite value counts with every weight that is not zero, the row's largest (exactly one) among them: the
+    result is infinite, or NaN where both infinities meet, as in the form that the GEMM prologues run."""
+    Hkv, blk, g = 2, 16, torch.Generator().manual_seed(keys)
+    H, need = Hkv * G, -(-keys // 16)
+    kc, vc = (torch.randn(need, Hkv, blk, D, generator=g).bfloat16() for _ in range(2))
+    for i, x in enumerate((math.inf, -math.inf, math.nan)):
+        vc[:, 0, :, 8 * i] = x                        # all values of a column
+        vc[min(1, need - 1), 1, min(keys - 1, 15) % blk, 8 * i + 3] = x       # one of them
+    vc[0, 0, 0, 40] = math.inf
+    vc[need - 1, 0, (keys - 1) % blk, 40] = -math.inf
+    bt = torch.randperm(need, generator=g)[None].int()
+    kc, vc, bt = kc.cuda(), vc.cuda(), bt.cuda()
+    q = (3 * torch.randn(1, H * D, generator=g)).bfloat16().cuda()
+    ks, vs = ([c[bt[0].long()].transpose(1, 2).reshape(-1, Hkv, D)[:keys]] for c in (kc, vc))
+    # the sum term by term: a product over all keys at once may take 0 x inf for its padding
+    p = torch.softmax(torch.einsum("hd,lhd->hl", q.double().view(H, D), ks[0].double().repeat_interleave(G, 1)) * D ** -0.5, -1)
+    ref = (p.t()[:, :, None] * vs[0].double().repeat_interleave(G, 1)).sum(0).flatten()[None]
+    ws, ns = ops.AttnWorkspace("cuda", 16, H, D, 6), -(-keys // 128)
+    for streamed in (False, True):
+        _same_kind(ops.attention(q, kc, vc, torch.tensor([0, 1], dtype=torch.int32).cuda(), n_heads=H, n_kv=Hkv, head_dim=D, causal=True, max_q=1,
+                                 ctx_lens=torch.tensor([keys], dtype=torch.int32).cuda(), block_tables=bt, grouped=True,
+                                 split_keys=128, num_splits=ns, workspace=ws, streamed=streamed), ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [64, 128])
+def test_empty_sequences_and_feeds_of_no_tokens(D):
+    """A row without a key is zero; a feed of no tokens writes nothing and leaves the tickets of its splits zero."""
+    H, Hkv, blk, g = 8, 2, 16, torch.Generator().manual_seed(D)
+    kc, vc = (torch.randn(30, Hkv, blk, D, generator=g).bfloat16().cuda() for _ in range(2))
+    bt = torch.randperm(30, generator=g)[:30].view(1, 30).repeat(4, 1).int().cuda()
+    lens, qlens = [0, 450, 300, 33], [1, 0, 2, 1]
+    cu = torch.tensor([0, 1, 1, 3, 4], dtype=torch.int32).cuda()
+    q = torch.randn(4, H * D, generator=g).bfloat16().cuda()
+    ws = ops.AttnWorkspace("cuda", 16, H, D, 4)
+    rows = [[c[bt[0].long()].transpose(1, 2).reshape(-1, Hkv, D)[:n] for n in lens[2:]] for c in (kc, vc)]
+    ref = _reference(q[1:], *rows, qlens[2:], H, H // Hkv, D, True)
+    for streamed in (False, True):
+        out = torch.full((4, H * D), 7.0, dtype=torch.bfloat16, device="cuda")
+        ops.attention(q, kc, vc, cu, n_heads=H, n_kv=Hkv, head_dim=D, causal=True, max_q=2, ctx_lens=torch.tensor(lens, dtype=torch.int32).cuda(),
+                      block_tables=bt, grouped=True, split_keys=128, num_splits=4, workspace=ws, out=out, streamed=streamed)
+        assert (out[0] == 0).all()
+        _close(out[1:], ref)
+        assert int(ws.counters.abs().sum()) == 0
