@@ -24,8 +24,8 @@
 // K/V addresses need no per-lane dependent lookup.
 //
 // Up to 16 query rows per kv head run on attn_stream.hip; this form serves 17 to 32 rows, operands off 16
-// bytes, the 8-wave and prefetching variants where they are asked for, and the attention inside the
-// fused launches of gemm_skinny.hip.
+// bytes, more kv heads of all sequences than that form's workgroups fit on the chip, the 8-wave and prefetching
+// variants where they are asked for, and the attention inside the fused launches of gemm_skinny.hip.
 #include "attn_decode.h"
 
 thread_local int g_loqa_launch_prio = 0;

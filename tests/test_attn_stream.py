@@ -209,3 +209,15 @@ def test_merge_of_many_splits_is_one_trip():
     call = _token(64, 4, 8, 4, 2000, 128, 16)
     us, former = _us([call, lambda: call(False)])
     assert us < 1.05 * former, (us, former)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,Hkv,B,keys,split,former", [(128, 8, 33, 200, 224, True), (128, 8, 32, 200, 224, False), (128, 8, 33, 100, 128, False),
+                                                       (128, 8, 33, 200, 128, False), (64, 8, 65, 200, 224, True), (64, 8, 64, 200, 224, False),
+                                                       (64, 8, 97, 500, 512, True), (64, 8, 97, 520, 544, False), (64, 8, 96, 520, 544, True)])
+def test_many_sequences_take_the_former_kernel(D, Hkv, B, keys, split, former):
+    """Either side of each line of the rule, the forms told apart by their sums' last bits; both right."""
+    call = _token(D, Hkv, 2, B, keys, split, -(-keys // split))
+    y, z = call(), call(False)
+    assert torch.equal(y, z) == former
+    _close(y, z.double())
