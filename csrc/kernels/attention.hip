@@ -261,10 +261,9 @@ __global__ __launch_bounds__(ATT_THREADS, 1) void attn_fwd_kernel(AttnParams p) 
 // above the VALU's and MFMAs' time: the loads' share of LDS and L2 (a third at 128 columns with
 // two runs), the barrier and the maxima, each of which all waves of a workgroup meet together.
 // PAGES: 0 contiguous rows, 1 cache blocks of 64 rows or more, 2 of 8, 16 or 32.
-template <int D, int PAGES, int QW, int KS>
+template <int D, int PAGES, int QW, int KS, bool PARTS>
 __global__ __launch_bounds__(64 * QW * KS, D == 64 && QW * KS == 4 ? 3 : 2) void attn_pipe_kernel(AttnParams p) {
   constexpr bool PAGED = PAGES > 0;
-  constexpr bool PARTS = QW == 2;      // the launch has parts of 64-row blocks only
   using L = FlashLds<D, D>;
   constexpr int NS = D / 16, NDT = D / 32, NTH = 64 * QW;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
@@ -285,7 +284,7 @@ __global__ __launch_bounds__(64 * QW * KS, D == 64 && QW * KS == 4 ? 3 : 2) void
       }
       bx = gx - 1 - bx;
     }
-    if (PARTS && p.parts > 1) {
+    if constexpr (PARTS) {
       share = bx % p.parts;
       bx /= p.parts;
     }
@@ -312,7 +311,7 @@ __global__ __launch_bounds__(64 * QW * KS, D == 64 && QW * KS == 4 ? 3 : 2) void
   int kend = klen;
   if (p.causal) kend = min(kend, klen - qlen + row_hi + 1);
   int ntiles = kend > 0 ? (kend + FL_KEYS - 1) / FL_KEYS : 0, parts = 1, t0 = 0;
-  if (PARTS && p.parts > 1) {
+  if constexpr (PARTS) {
     parts = max(1, min(p.parts, ntiles / FL_CAP));
     if (share >= parts) return;                             // uniform
     const int len = (ntiles + parts - 1) / parts;
@@ -699,13 +698,13 @@ __global__ void attn_combine_kernel(const float* __restrict__ part_o,
   o[(size_t)tok * o_stride + (size_t)head * D + d] = f2bf(l > 0.f ? acc / l : 0.f);
 }
 
-template <int D, int PAGES, int QW, int KS>
+template <int D, int PAGES, int QW, int KS, bool PARTS = false>
 static int launch_pipe(const AttnParams& p, int B, int max_q, hipStream_t s) {
   constexpr int ring = KS * FlashLds<D, D>::RING, end = fl_merge_bytes(D / 32, QW, KS) + QW * fl_store_bytes(D / 32);
   constexpr int bytes = ring > end ? ring : end;
   static_assert(bytes <= 160 * 1024, "LDS of a CU");
-  const dim3 grid((max_q + 32 * QW - 1) / (32 * QW) * p.parts, p.Hq, B);
-  hipLaunchKernelGGL((attn_pipe_kernel<D, PAGES, QW, KS>), grid, dim3(64 * QW * KS), bytes, s, p);
+  const dim3 grid((max_q + 32 * QW - 1) / (32 * QW) * (PARTS ? p.parts : 1), p.Hq, B);
+  hipLaunchKernelGGL((attn_pipe_kernel<D, PAGES, QW, KS, PARTS>), grid, dim3(64 * QW * KS), bytes, s, p);
   return (int)hipGetLastError();
 }
 
@@ -723,10 +722,12 @@ static int launch_pipe(const AttnParams& p, int B, int max_q, hipStream_t s) {
 // 29; 2048 x 20 heads 40, 50; 4096 x 12 heads 68, 94, x 20 heads 116, 121; but 4 x 700 x 16 heads
 // 18.0, 17.0, 3000 x 20 heads 76, 62, 4096 x 32 heads 121, 102.
 template <int D, int PAGES>
-static int launch_rows(AttnParams p, int B, int max_q, hipStream_t s) {
+static int launch_rows(const AttnParams& p, int B, int max_q, hipStream_t s) {
   const long n64 = (long)((max_q + 63) / 64) * p.Hq * B, n128 = (long)((max_q + 127) / 128) * p.Hq * B;
   const long two = D == 128 ? (max_q <= 128 ? 256 : 512) : !p.causal || max_q < 1024 ? 256 : max_q < 4096 ? 384 : 640;
-  if (n64 > 128) p.parts = 1;        // parts only of 64-row blocks, all of them one round
+  // parts only of 64-row blocks, all of them one round, and in a kernel of their own: with both in one, launches
+  // without parts took 0.2 to 0.4 us more (17 rows x 32 heads of 128 7.8 us, 7.5 alone)
+  if (n64 <= 128 && p.parts > 1) return launch_pipe<D, PAGES, 2, D == 64 ? 4 : 2, true>(p, B, max_q, s);
   if (n64 <= 256) return launch_pipe<D, PAGES, 2, D == 64 ? 4 : 2>(p, B, max_q, s);
   if (n128 <= two) return launch_pipe<D, PAGES, 4, 2>(p, B, max_q, s);
   return launch_pipe<D, PAGES, 4, 1>(p, B, max_q, s);

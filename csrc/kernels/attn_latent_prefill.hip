@@ -45,9 +45,10 @@ struct LatPrefillParams {
 // compiler keeps MFMA results in the accumulation registers and moves them for every rescaling.
 // us with 256 registers (10 spilled at 192 / 128) and with 320 (none): 300 rows x 16 heads 13.8, 14.7;
 // 2048 x 8 heads 37.2, 41.8, at 128 / 128 30.6, 36.9.
-template <int DK, int DV, int QW, int KS>
+// PARTS: of a block's keys, a kernel of its own (in one with the others these took 0.2 to 0.6 us more, 17 rows x 16 heads of
+// 256 / 64 8.4 us, 7.8 alone).
+template <int DK, int DV, int QW, int KS, bool PARTS>
 __global__ __launch_bounds__(64 * QW * KS, DK > 192 ? 1 : 2) void latent_prefill_kernel(LatPrefillParams p) {
-  constexpr bool PARTS = QW == 2;      // the launch has parts of 64-row blocks only
   using L = FlashLds<DK, DV>;
   constexpr int NS = DK / 16, NDT = DV / 32, NTH = 64 * QW;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
@@ -65,7 +66,7 @@ __global__ __launch_bounds__(64 * QW * KS, DK > 192 ? 1 : 2) void latent_prefill
       bx = in / hp;
       hd = xcd * hp + in - bx * hp;
     }
-    if (PARTS && p.parts > 1) {
+    if constexpr (PARTS) {
       const int block = bx / p.parts;
       share = bx - block * p.parts;
       bx = gx / p.parts - 1 - block;
@@ -88,7 +89,7 @@ __global__ __launch_bounds__(64 * QW * KS, DK > 192 ? 1 : 2) void latent_prefill
   int kend = min(klen, p.pos[q0 + row_hi] - koff + 1);         // positions grow along a sequence
   int kt0 = p.window > 0 ? max(0, p.pos[q0 + row_lo] - koff - p.window + 1) / FL_KEYS * FL_KEYS : 0;
   int ntiles = kend > kt0 ? (kend - kt0 + FL_KEYS - 1) / FL_KEYS : 0, parts = 1;
-  if (PARTS && p.parts > 1) {
+  if constexpr (PARTS) {
     parts = max(1, min(p.parts, ntiles / FL_CAP));
     if (share >= parts) return;                           // uniform
     const int len = (ntiles + parts - 1) / parts;
@@ -332,25 +333,27 @@ extern "C" int loqa_latent_prefill(const void* q, long q_st, const void* k, cons
   // share a CU: with feeds of up to 128 rows from a second round on (us with two runs and with one,
   // 9 feeds x 32 heads: 20 rows, 192 / 128 columns: 18, 9.8; 128 rows behind 300: 41.5, 31)
   const long n64 = (long)((max_q + 63) / 64) * H * B, n128 = (long)((max_q + 127) / 128) * H * B;
-#define RUN(A, C, QW, KS)                                                                     \
+  if (parts > 1 && n64 > 256) return (int)hipErrorInvalidValue;
+#define RUN(A, C, QW, KS, PARTS)                                                              \
   do {                                                                                        \
     constexpr int ring = KS * FlashLds<A, C>::RING;                                           \
     constexpr int end = fl_merge_bytes(C / 32, QW, KS) + QW * fl_store_bytes(C / 32);         \
     constexpr int bytes = ring > end ? ring : end;                                            \
     static_assert(bytes <= 160 * 1024, "LDS of a CU");                                        \
     const long blocks = (max_q + 32 * QW - 1) / (32 * QW), all = blocks * H * B;              \
-    if (parts > 1 && (QW != 2 || all > tickets || all * parts * QW * fl_join_floats(C / 32) > part_floats)) \
+    if (PARTS && (all > tickets || all * parts * QW * fl_join_floats(C / 32) > part_floats))  \
       return (int)hipErrorInvalidValue;                                                       \
-    const dim3 grid(blocks * parts, H, B);                                                    \
-    hipLaunchKernelGGL((latent_prefill_kernel<A, C, QW, KS>), grid, dim3(64 * QW * KS), bytes, st, p); \
+    const dim3 grid(blocks * (PARTS ? parts : 1), H, B);                                      \
+    hipLaunchKernelGGL((latent_prefill_kernel<A, C, QW, KS, PARTS>), grid, dim3(64 * QW * KS), bytes, st, p); \
     return (int)hipGetLastError();                                                            \
   } while (0)
 #define GO(A, C)                                                                              \
   if (DK == A && DV == C) {                                                                   \
     constexpr int K2 = A > 192 ? 1 : 2;                                                       \
-    if (n64 <= 256) RUN(A, C, 2, K2);                                                         \
-    else if (n128 <= (max_q <= 128 ? 256 : 512)) RUN(A, C, 4, K2);                                                   \
-    else RUN(A, C, 4, 1);                                                                     \
+    if (parts > 1) RUN(A, C, 2, K2, true);                                                    \
+    else if (n64 <= 256) RUN(A, C, 2, K2, false);                                             \
+    else if (n128 <= (max_q <= 128 ? 256 : 512)) RUN(A, C, 4, K2, false);                     \
+    else RUN(A, C, 4, 1, false);                                                              \
   }
   GO(64, 64) GO(128, 64) GO(192, 64) GO(256, 64) GO(64, 128) GO(128, 128) GO(192, 128) GO(256, 128)
 #undef GO

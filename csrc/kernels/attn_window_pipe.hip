@@ -18,12 +18,12 @@ __device__ __forceinline__ float wp_tanh(float z) {
   return 1.f - 2.f * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(2.885390081777927f * z));
 }
 
-// GEN: a soft cap, slopes or a scale that is not positive; else scores only need masking.
-template <int DK, int DV, int QW, int KS, bool GEN>
+// GEN: a soft cap, slopes or a scale that is not positive; else scores only need masking. PARTS: of a block's keys, a kernel of
+// its own (in one with the others these took 0.2 to 0.5 us more, 300 rows x 16 heads of 128 in a window of 300 15.4 us, 14.6 alone).
+template <int DK, int DV, int QW, int KS, bool GEN, bool PARTS>
 __global__ __launch_bounds__(64 * QW * KS, 2) void window_attn_pipe_kernel(WinAttnParams p) {
   using L = FlashLds<DK, DV>;
   constexpr int NS = DK / 16, NDT = DV / 32, NTH = 64 * QW;
-  constexpr bool PARTS = QW == 2;      // the launch has parts of 64-row blocks only
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int run = wave / QW, wq = wave % QW, th = threadIdx.x - run * NTH, h = lane >> 5;
@@ -40,7 +40,7 @@ __global__ __launch_bounds__(64 * QW * KS, 2) void window_attn_pipe_kernel(WinAt
       hd = xcd * hp + in - bx * hp;
     }
     bx = gx - 1 - bx;
-    if (PARTS && p.parts > 1) {
+    if constexpr (PARTS) {
       share = bx % p.parts;
       bx /= p.parts;
     }
@@ -64,7 +64,7 @@ __global__ __launch_bounds__(64 * QW * KS, 2) void window_attn_pipe_kernel(WinAt
   const int n1 = p.window > 0 ? min((min(p.keep_first, wg_lo) + FL_KEYS - 1) / FL_KEYS, lo_t / FL_KEYS) : 0;
   int ntiles = kend > 0 ? n1 + max(kend - lo_t + FL_KEYS - 1, 0) / FL_KEYS : 0, parts = 1, t0 = 0;
   auto tile_at = [&](int i) { return i < n1 ? i * FL_KEYS : lo_t + (i - n1) * FL_KEYS; };
-  if (PARTS && p.parts > 1) {
+  if constexpr (PARTS) {
     parts = max(1, min(p.parts, ntiles / FL_CAP));
     if (share >= parts) return;                             // uniform
     const int len = (ntiles + parts - 1) / parts;
@@ -197,17 +197,16 @@ __global__ __launch_bounds__(64 * QW * KS, 2) void window_attn_pipe_kernel(WinAt
                 qlen - row_lo - wq * 32, Dv, lane);
 }
 
-template <int DK, int DV, int QW, int KS, bool GEN>
+template <int DK, int DV, int QW, int KS, bool GEN, bool PARTS = false>
 static int launch(const WinAttnParams& p, int max_q, hipStream_t st) {
   constexpr int ring = KS * FlashLds<DK, DV>::RING, end = fl_merge_bytes(DV / 32, QW, KS) + QW * fl_store_bytes(DV / 32);
   constexpr int bytes = ring > end ? ring : end;
   static_assert(bytes <= 160 * 1024, "LDS of a CU");
   const long blocks = (max_q + 32 * QW - 1) / (32 * QW), all = blocks * p.H * p.vparts * p.B;
-  if (p.parts > 1 && (QW != 2 || p.parts > FL_PARTS || all > p.tickets ||
-                      all * p.parts * QW * fl_join_floats(DV / 32) > p.part_floats))
+  if (PARTS && (p.parts > FL_PARTS || all > p.tickets || all * p.parts * QW * fl_join_floats(DV / 32) > p.part_floats))
     return (int)hipErrorInvalidValue;
-  const dim3 grid(blocks * p.parts, p.H * p.vparts, p.B);
-  hipLaunchKernelGGL((window_attn_pipe_kernel<DK, DV, QW, KS, GEN>), grid, dim3(64 * QW * KS), bytes, st, p);
+  const dim3 grid(blocks * (PARTS ? p.parts : 1), p.H * p.vparts, p.B);
+  hipLaunchKernelGGL((window_attn_pipe_kernel<DK, DV, QW, KS, GEN, PARTS>), grid, dim3(64 * QW * KS), bytes, st, p);
   return (int)hipGetLastError();
 }
 
@@ -219,12 +218,12 @@ static int launch(const WinAttnParams& p, int max_q, hipStream_t st) {
 // be four more kernels to build (100 rows x 8 heads of 128: 12.4, with it 11.6; 320 behind 1000
 // x 16: 51, 47).
 template <int DK, int DV>
-static int launch_rows(WinAttnParams p, int max_q, hipStream_t st) {
+static int launch_rows(const WinAttnParams& p, int max_q, hipStream_t st) {
   const long hd = (long)p.H * p.vparts * p.B, n64 = (max_q + 63) / 64 * hd, n128 = (max_q + 127) / 128 * hd;
-  if (n64 > 128 || p.cap > 0.f || p.slopes || !(p.scale > 0.f)) p.parts = 1;   // parts only of the first form
   const bool one = n128 > (max_q <= 128 ? 256 : 512);
   if (p.cap > 0.f || p.slopes || !(p.scale > 0.f))
     return one ? launch<DK, DV, 4, 1, true>(p, max_q, st) : launch<DK, DV, 4, 2, true>(p, max_q, st);
+  if (n64 <= 128 && p.parts > 1) return launch<DK, DV, 2, 2, false, true>(p, max_q, st);   // parts only of the first form
   if (n64 <= 256) return launch<DK, DV, 2, 2, false>(p, max_q, st);
   if (!one) return launch<DK, DV, 4, 2, false>(p, max_q, st);
   return launch<DK, DV, 4, 1, false>(p, max_q, st);
