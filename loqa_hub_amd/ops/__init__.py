@@ -1715,7 +1715,7 @@ SK_WHOLE = 12             # the layout that the plan does not split along K
 SK_RENAMED = {0: 20, 2: 19, 3: 15, 4: 19, 5: 20, 6: 12, 8: 19, 9: 15, 10: 20}
 SK_CUS = 256
 SK_FEW = 96
-SK_SHARED = (700, 200)    # rows, workgroups
+SK_SHARED = ((700, 0, 200, 8), (1600, 2048, 240, 1))   # rows and K at least, workgroups and chunks at most
 SK_SMALL = 11             # the 64 x 64 tiles
 SK_GELU = 1.3e-4
 SK_PAIRED = 17            # two workgroups a compute unit, with GELU
@@ -1726,18 +1726,21 @@ def gemm_sk_plan(M: int, N: int, K: int, epi: str = "bf16", layouts=None, *,
                  pipe: bool = True) -> tuple[int, int]:
     """(layout, K chunks) for a shape: the fewest microseconds by SK_LAYOUTS, counting whole
     rounds of tiles over the compute units; up to SK_FEW workgroups load so little beside each other that
-    a K step takes 0.8 of its time (1500 x 512 x 2048 on 96 of them 11.0 us, in two chunks on 192 11.6), and where eight or more
-    row blocks share the weights, up to SK_SHARED workgroups, 0.9 (1500 x 768 x 3072 on 144 17.1 us, 320 x 4096 x 4096
-    on 160 29). 64 x 64 tiles are for what leaves half of the units idle in 128 x 64 (1500 x 512 x 2048 11.1 -> 8.9 us, x
-    512 5.7 -> 4.7, 300 x 1280 x 1280 9.0 -> 6.6); from K = 2048 on their steps take longer.
+    a K step takes 0.8 of its time (1500 x 512 x 2048 on 96 of them 11.0 us, in two chunks on 192 11.6), and where many
+    rows share the weights, on as many workgroups as SK_SHARED says, 0.9 (1500 x 768 x 3072 on 144 17.1 us; whole tiles of 2200 x
+    4096 x 11008 on 192 171 us, in four chunks 202). 64 x 64 tiles are for what leaves half of the units idle in 128 x 64
+    (1500 x 512 x 2048 11.1 -> 8.9 us, x 512 5.7 -> 4.7, 300 x 1280 x 1280 9.0 -> 6.6); their step is charged 1.26 times from K =
+    2112 on, a step of the fit.
     K chunks fill the chip where the tiles do not; each tile then pays for the trip of its f32 partials
     through memory, 3 us and 40 us a MB, and 4 us a MB for each chunk that is read back (fitted with the
-    rest; 320 x 4096 x 4096 in four chunks of 128 x 192 22.2 us, whole 27.3 in 128 x 64). Their partials and the weights
-    that a launch touches for the next one (:func:`_ahead`) hold each other up (1500 x 1280 x 5120 in two chunks 28.3 us and whole
-    29.9 alone, but an encoder pass with 32 of them 4118 us and 4058). Never on 256 x 256
-    tiles: these fill the chip with MFMAs, where a K step takes longer than the fit has it (4096 x
+    rest; 320 x 4096 x 4096 in four chunks of 128 x 192 25.7 us, whole 29.0 in 128 x 64). Chunks of a second round are never
+    worth it: the tiles' partials then hold each other up and the first round's workgroups wait for chunks that have not
+    begun (1600 x 4096 x 14336 on 480 workgroups of five chunks 238 us, whole in 128 x 256 167; 1100 x 16384 x 3072 on 768 of two 141, whole
+    108). Their partials and the weights that a launch touches for the next one (:func:`_ahead`) hold each other up as well (1500
+    x 1280 x 5120 in two chunks 28.3 us and whole 29.9 alone, but an encoder pass with 32 of them 4118 us and 4058). Never on
+    256 x 256 tiles: these fill the chip with MFMAs, where a K step takes longer than the fit has it (4096 x
     14336: 1280 rows in three chunks 160 us, the 256 x 192 tiles in two 135; 2048 rows in two 205,
-    the 128 x 256 tiles whole 182; the fastest in none of the 60 shapes). ``pipe`` False:
+    the 128 x 256 tiles whole 182; the fastest in none of the grid's shapes). ``pipe`` False:
     the general layouts only (operands the pipelined tiles do not take). ``layouts``: among
     these only (numbers of SK_LAYOUTS or SK_RENAMED). Of the epilogues ``epi`` only "gelu" is in the
     model: SK_GELU us for a value of a tile, as nothing runs beside its arithmetic, except
@@ -1762,9 +1765,10 @@ def _sk_plan(M: int, N: int, K: int, pipe: bool, layouts: tuple | None = None, g
         if lay == SK_SMALL and K > 2048:
             step *= 1.26
         for s in (1, 2, 3, 4, 5, 6, 8):
-            if s > 1 and (KT // s < 8 or lay == SK_WHOLE):
+            if s > 1 and (KT // s < 8 or lay == SK_WHOLE or (lay >= SK_PIPE and tiles * s > SK_CUS)):
                 continue
-            few = 0.8 if tiles * s <= SK_FEW else 0.9 if M >= SK_SHARED[0] and tiles * s <= SK_SHARED[1] else 1.0
+            shared = any(M >= rows and K >= k and tiles * s <= wgs and s <= chunks for rows, k, wgs, chunks in SK_SHARED)
+            few = 0.8 if tiles * s <= SK_FEW else 0.9 if shared else 1.0
             end = around + (SK_GELU * bn * bm / s if gelu and lay >= SK_PIPE else 0.0)
             t = -(-tiles * s // SK_CUS) * (-(-KT // s) * step * few + end)
             if gelu and lay == SK_PAIRED and s == 1 and tiles > SK_CUS:

@@ -162,3 +162,16 @@ def test_the_plan_takes_small_tiles_for_small_grids():
     for M, N, K in ((1500, 768, 3072), (1500, 1280, 1280), (9000, 512, 512), (320, 4096, 14336)):
         assert ops.gemm_sk_plan(M, N, K)[0] != ops.SK_SMALL
     assert not ops.gemm_sk_plan(1500, 576, 2048)[0] >= ops.SK_PIPE          # whole 128 features, as every pipelined tile
+
+
+def test_chunks_are_one_round():
+    """Chunks beyond the compute units took 1.14 to 1.4 times the whole tiles' time, and many rows' whole tiles less than
+    their chunks (1600 x 4096 x 14336: 238 us in five chunks, 167 whole)."""
+    for M in (17, 160, 320, 640, 1100, 1600, 2200, 3300, 9000):
+        for N, K in ((1280, 5120), (2048, 8192), (3072, 8192), (4096, 11008), (4096, 14336), (5120, 3072), (16384, 3072)):
+            lay, s = ops.gemm_sk_plan(M, N, K)
+            bn, bm = ops.SK_LAYOUTS[lay][:2]
+            assert s == 1 or -(-M // bm) * (N // bn) * s <= ops.SK_CUS, (M, N, K, lay, s)
+    for shape, plan in (((1600, 4096, 14336), (16, 1)), ((3300, 5120, 3072), (17, 1)), ((2200, 4096, 11008), (13, 1)), ((1100, 16384, 3072), (17, 1)),
+                        ((1100, 4096, 11008), (13, 2)), ((2500, 2048, 8192), (17, 1)), ((320, 4096, 4096), (17, 4)), ((320, 4096, 14336), (17, 4))):
+        assert ops.gemm_sk_plan(*shape) == plan, shape
