@@ -1907,7 +1907,7 @@ def gemm_sk(x: torch.Tensor, w: torch.Tensor, *, epi: str = "bf16", bias: torch.
     if x.stride(1) != 1 or not w.is_contiguous():
         raise ValueError("gemm_sk needs K-contiguous operands")
     y = residual if epi == "resid" else out
-    if layout is None or splits is None or layout in SK_RENAMED:
+    if layout is None or splits is None or layout in SK_RENAMED or layout == SK_SMALL:
         # the pipelined tiles move whole 16-byte pieces of the rows at 32-bit offsets
         pipe = x.stride(0) >= K and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 \
             and N * K < 1 << 31 and x.stride(0) < 1 << 21 \
@@ -1915,8 +1915,11 @@ def gemm_sk(x: torch.Tensor, w: torch.Tensor, *, epi: str = "bf16", bias: torch.
         pl, ps = _sk_plan(M, N, K, pipe, None, act == "gelu")
         layout = pl if layout is None else layout
         splits = ps if splits is None else splits
-        if layout in SK_RENAMED:
-            layout = SK_RENAMED[layout] if pipe else 1
+        # (11 named the 128 x 64 tiles once, and takes and refuses what it did)
+        if layout in SK_RENAMED or layout == SK_SMALL:
+            layout = SK_RENAMED.get(layout, layout) if pipe else 1
+            if N % 128:
+                raise ValueError(f"gemm_sk layout {layout}: N {N} is no multiple of 128")
     bn, bm = SK_LAYOUTS[layout][:2]
     if N % bn or K % 64:
         raise ValueError(f"gemm_sk layout {layout}: N {N} / K {K} not tileable")

@@ -175,3 +175,16 @@ def test_chunks_are_one_round():
     for shape, plan in (((1600, 4096, 14336), (16, 1)), ((3300, 5120, 3072), (17, 1)), ((2200, 4096, 11008), (13, 1)), ((1100, 16384, 3072), (17, 1)),
                         ((1100, 4096, 11008), (13, 2)), ((2500, 2048, 8192), (17, 1)), ((320, 4096, 4096), (17, 4)), ((320, 4096, 14336), (17, 4))):
         assert ops.gemm_sk_plan(*shape) == plan, shape
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("splits", [None, 1, 2])
+def test_small_tiles_by_number_take_what_their_number_took(splits):
+    """11 named the 128 x 64 tiles before it named these: rows off 16 bytes still take the general form, and
+    features that are no multiple of 128 are still refused."""
+    g = torch.Generator().manual_seed(11)
+    x, w = torch.randn(150, 1024, generator=g).bfloat16().cuda(), (torch.randn(512, 1024, generator=g) / 32).bfloat16().cuda()
+    for out in (None, torch.zeros(150, 516, dtype=torch.bfloat16, device="cuda")[:, :512]):
+        _close(ops.gemm_sk(x, w, layout=ops.SK_SMALL, splits=splits, out=out), x.double() @ w.double().t(), 1024)
+    with pytest.raises(ValueError):
+        ops.gemm_sk(x, w[:448], layout=ops.SK_SMALL, splits=splits)
