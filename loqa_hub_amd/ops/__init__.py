@@ -1915,11 +1915,9 @@ def gemm_sk(x: torch.Tensor, w: torch.Tensor, *, epi: str = "bf16", bias: torch.
         pl, ps = _sk_plan(M, N, K, pipe, None, act == "gelu")
         layout = pl if layout is None else layout
         splits = ps if splits is None else splits
-        # (11 named the 128 x 64 tiles once, and takes and refuses what it did)
+        # (11 named the 128 x 64 tiles once, and takes what it did)
         if layout in SK_RENAMED or layout == SK_SMALL:
             layout = SK_RENAMED.get(layout, layout) if pipe else 1
-            if N % 128:
-                raise ValueError(f"gemm_sk layout {layout}: N {N} is no multiple of 128")
     bn, bm = SK_LAYOUTS[layout][:2]
     if N % bn or K % 64:
         raise ValueError(f"gemm_sk layout {layout}: N {N} / K {K} not tileable")
