@@ -1798,9 +1798,14 @@ def _sk_workspace(dev: torch.device, stream: int, floats: int, tiles: int):
         cid = ctypes.c_uint64()
         check(kernels().loqa_capture_id(stream, ctypes.byref(cid)), "capture_id")
         held, ws = _SK_WS_CAPTURE.get((dev, stream), (None, None))
-        if held != cid.value or ws[0].numel() < floats or ws[1].numel() < tiles:
-            ws = (torch.empty(floats, dtype=torch.float32, device=dev),
-                  _tickets(tiles, dev))
+        if held != cid.value:
+            ws = None
+        if ws is None or ws[0].numel() < floats or ws[1].numel() < tiles:
+            # the larger of both: launches that want much of one and little of the other, in turn, find it
+            f = max(floats, 0 if ws is None else ws[0].numel())
+            t = max(tiles, 0 if ws is None else ws[1].numel())
+            ws = (torch.empty(f, dtype=torch.float32, device=dev),
+                  _tickets(t, dev))
             _SK_WS_GRAPHS.append(ws)
             _SK_WS_CAPTURE[(dev, stream)] = (cid.value, ws)
         return ws

@@ -87,3 +87,25 @@ def test_launches_of_a_capture_share_a_workspace():
         assert all(torch.equal(y, z) for out in outs for y, z in zip(out, want))
         assert all(torch.equal(y, z) for y, z in zip(run(), want))
     assert all(int(cnt.abs().sum()) == 0 for _, cnt in ops._SK_WS_GRAPHS)
+
+
+@pytest.mark.gpu
+def test_a_captures_workspace_grows_to_the_largest_of_both():
+    """Launches that want many partials and launches that want many tickets, in turn: the first two of a capture make
+    its workspace, the others find it."""
+    g = torch.Generator().manual_seed(3)
+    x = torch.randn(64, 64 * 40, generator=g).bfloat16().cuda()
+    ws = [(torch.randn(n, x.shape[1], generator=g) / 16).bfloat16().cuda() for n in (512, 2048)]
+    # 2 tiles of 256 x 256 in five chunks; 32 tiles of 64 x 64 in two
+    run = lambda: [ops.gemm_sk(x, w, layout=lay, splits=s) for w, lay, s in 3 * ((ws[0], 12, 5), (ws[1], ops.SK_SMALL, 2))]      # noqa: E731
+    want, n = run(), len(ops._SK_WS_GRAPHS)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = run()
+    assert len(ops._SK_WS_GRAPHS) == n + 2
+    for _ in range(3):
+        for y in got:
+            y.zero_()
+        graph.replay()
+        assert all(torch.equal(y, z) for y, z in zip(got, want))
+        assert all(torch.equal(y, z) for y, z in zip(run(), want))
