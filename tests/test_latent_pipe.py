@@ -74,6 +74,9 @@ def test_parts_of_the_keys(feeds, pasts, H, window):
     for DK, DV in ((192, 128), (256, 64), (64, 64)):
         _check(feeds, pasts, H, DK, DV, DV - 12, window=window, sink=True, gate=True, seed=DK)
     _check(feeds, pasts, H, 128, 128, 128, window=window, scale=-0.05, seed=5)
+    torch.cuda.synchronize()
+    # every word of a ticket's line, as fl_join counts arrivals and published parts in four of them
+    assert all(int(words.as_strided((words.numel(), 32), (32, 1)).abs().sum()) == 0 for _, words in ops._SK_WS.values())
 
 
 def test_parts_repeat_bit_for_bit():

@@ -141,3 +141,6 @@ def test_parts_of_the_keys(feeds, pasts, H, window, keep):
     _check(feeds, pasts, H, 4, 64, 64, window, keep, seed=2)
     _check(feeds, pasts, H, 4, 96, 200, window, keep, sink=True, seed=3)
     _check(feeds, pasts, H, 4, 64, 72, window, keep, cap=30.0, seed=4)      # transformed scores: whole
+    torch.cuda.synchronize()
+    # every word of a ticket's line, as fl_join counts arrivals and published parts in four of them
+    assert all(int(words.as_strided((words.numel(), 32), (32, 1)).abs().sum()) == 0 for _, words in ops._SK_WS.values())
