@@ -33,9 +33,10 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t sk_part(const GemmSkParams& p,
   return __builtin_amdgcn_make_buffer_rsrc(p.ws + ((size_t)tile * p.S + c) * TILE, 0, TILE * 4, 0x00020000);
 }
 
-// The shares of the tile that this workgroup sums up, a bit each. late() publishes what it has kept back.
+// The shares of the tile that this workgroup sums up, a bit each. late() publishes what it has kept back. hurry: 0, or
+// SK_POLLS where a test has every workgroup but the last give its share up.
 template <typename Late>
-__device__ __forceinline__ unsigned sk_shares(int* word, int S, int s, int* flag, Late&& late) {
+__device__ __forceinline__ unsigned sk_shares(int* word, int S, int s, int hurry, int* flag, Late&& late) {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // written through: visible when acknowledged
   __syncthreads();
   if (threadIdx.x == 0) {
@@ -46,7 +47,7 @@ __device__ __forceinline__ unsigned sk_shares(int* word, int S, int s, int* flag
     } else if ((int)(old & 0xffff) == S - 1) {
       mine = 1u << s | (old >> 16 & 0xff);
     } else {
-      for (int k = 0; k < SK_POLLS && !mine; ++k)
+      for (int k = hurry; k < SK_POLLS && !mine; ++k)
         if ((__hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & 0xffff) == S) mine = 1u << s;
         else __builtin_amdgcn_s_sleep(4);
     }
@@ -158,7 +159,7 @@ __device__ __forceinline__ void sk_finish(const GemmSkParams& p, float4v (&acc)[
     __builtin_amdgcn_sched_barrier(0);
   }
   int* word = p.counters + tile * TICKET;
-  const unsigned mine = sk_shares(word, S, s, reinterpret_cast<int*>(lds + BYTES - 16), [&]() {
+  const unsigned mine = sk_shares(word, S, s, p.hurry, reinterpret_cast<int*>(lds + BYTES - 16), [&]() {
     for (int u = u0; u < u1; ++u)
 #pragma unroll
       for (int g = 0; g < G; ++g)

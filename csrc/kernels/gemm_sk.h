@@ -18,6 +18,7 @@ struct GemmSkParams {
   int* counters;                  // S > 1: [tiles] tickets, zero on entry (left zero)
   int layout;
   int ahead_wgs;                  // workgroups behind the tiles' that only touch what follows (pipelined tiles)
+  int hurry;                      // looks at a tile's word that a K chunk leaves out before it gives its share up (0, but in tests)
 };
 // A call: what the kernels without touching workgroups have no use for stands behind their arguments, as
 // a third cache line of them is another miss before the first load (0.2 us of 12 at 80 x 11264 x 2048).

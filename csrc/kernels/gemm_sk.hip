@@ -200,9 +200,9 @@ int gemm_pipe(const GemmSkCall& p, int layout, hipStream_t st);   // gemm_pipe.h
 
 // layout: 1: 128 x 64 (2 x 2 waves of 64 x 32), 7: 64 x 64 (2 x 2 waves of 32 x 32), two
 // stages each - the general forms, for feature counts that are no multiple of 128 and rows
-// that are not 16-byte aligned; 12 on: the pipelined tiles of gemm_pipe.hip
+// that are not 16-byte aligned; 11 on: the pipelined tiles of gemm_pipe.hip
 extern "C" int loqa_gemm_sk(const GemmSkCall* p, hipStream_t st) {
-  if (!p || p->M <= 0 || p->S < 1 || p->epi < 0 || p->epi > 2 || !p->x || !p->w || !p->y)
+  if (!p || p->M <= 0 || p->S < 1 || p->hurry < 0 || p->epi < 0 || p->epi > 2 || !p->x || !p->w || !p->y)
     return (int)hipErrorInvalidValue;
   if (p->S > 1 && (!p->ws || !p->counters)) return (int)hipErrorInvalidValue;
   if (p->ldx % 8 || p->ldy % 4) return (int)hipErrorInvalidValue;

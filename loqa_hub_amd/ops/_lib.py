@@ -73,7 +73,7 @@ class GemmSkParams(ctypes.Structure):
         ("epi", c_int), ("act", c_int), ("bias", c_void_p),
         ("y", c_void_p), ("ldy", c_ll),
         ("ws", c_void_p), ("counters", c_void_p), ("layout", c_int),
-        ("ahead_wgs", c_int), ("ahead", c_void_p * 2), ("ahead_bytes", c_ll * 2),
+        ("ahead_wgs", c_int), ("hurry", c_int), ("ahead", c_void_p * 2), ("ahead_bytes", c_ll * 2),
     ]
 
 

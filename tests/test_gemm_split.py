@@ -58,6 +58,39 @@ def test_a_chunk_that_starts_a_round_later():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("layout", [k for k in sorted(ops.SK_LAYOUTS) if k >= ops.SK_PIPE])
+@pytest.mark.parametrize("splits", [2, 4, 5, 8])
+def test_shares_given_up(layout, splits, monkeypatch):
+    """No looks at a tile's word: every workgroup but the last to arrive goes through publishing what it kept and giving
+    its share up, in every epilogue, with and without kept shares. Whoever sums a share up, it is the same bits."""
+    bn, bm = ops.SK_LAYOUTS[layout][:2]
+    K, N, M = 64 * 14, 4 * bn, 2 * bm + 21
+    g = torch.Generator().manual_seed(layout)
+    x = torch.randn(M, K, generator=g).bfloat16().cuda()
+    w = (torch.randn(N, K, generator=g) / 16).bfloat16().cuda()
+    b, res = torch.randn(N, generator=g).cuda(), torch.randn(M, N, generator=g).bfloat16().cuda()
+    run = lambda: [ops.gemm_sk(x, w, bias=b, layout=layout, splits=splits), ops.gemm_sk(x, w, bias=b, act="gelu", layout=layout, splits=splits),      # noqa: E731
+                   ops.gemm_sk(x, w, epi="resid", bias=b, residual=res.clone(), layout=layout, splits=splits),
+                   ops.gemm_sk(x, w, epi="swiglu", layout=layout, splits=splits)]
+    want, lib, calls = run(), ops.kernels(), []
+
+    class Hurried:
+        def __getattr__(self, name):
+            return getattr(lib, name)
+
+        def loqa_gemm_sk(self, call, stream):
+            call._obj.hurry = 1 << 20
+            calls.append(call._obj.S)
+            return lib.loqa_gemm_sk(call, stream)
+
+    monkeypatch.setattr(ops, "kernels", Hurried)
+    for _ in range(3):
+        assert all(torch.equal(y, z) for y, z in zip(run(), want))
+    assert calls == 12 * [splits]
+    _words_are_zero()
+
+
+@pytest.mark.gpu
 def test_launches_of_a_capture_share_a_workspace():
     """Two graphs, each with a launch that outgrows the first one's partials: their own memory, and every
     replay, on two streams at once, equal to the eager result."""
