@@ -187,7 +187,8 @@ ATTN_PF_MIN_KEYS = int(os.environ.get("LOQA_ATTN_PF_MIN_KEYS", "0"))
 
 def attn_parts(max_q: int, heads: int, keys: int) -> int:
     """Parts of a row block's keys at most, for the prompt attentions over ``heads`` heads of all
-    sequences with ``keys`` keys. Few rows behind many keys are few workgroups with a long chain of tiles each:
+    sequences with ``keys`` keys: the longest context where the host knows it (pages), the mean of the sequences where it only
+    knows the rows (contiguous keys; a long sequence beside many short ones then stays whole, as all did before). Few rows behind many keys are few workgroups with a long chain of tiles each:
     parts of eight tiles or more, while all of them are one round of the 256 CUs, join in the launch (us whole and in parts, 32
     heads of 128: 64 rows behind 1000 keys 22.2, 16.7; behind 2000 35.6, 19.9; behind 8000 121, 32; 256 behind 3000 50.4, 32.1; 8
     heads of 64: 64 behind 1000 15.3, 12.9; behind 8000 56, 17). Past one round the CUs share what bounds them (2048 rows of
@@ -211,6 +212,9 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu_q: torch.Ten
     Query i of sequence b sits at absolute position ctx_len_b - q_len_b + i.
     ``streamed`` False: the decode kernel that the GEMM prologues run (attn_decode.hip), bit for
     bit, also where attn_stream.hip takes the rows.
+    In which order a sequence's keys are summed up follows from the whole call (the sequences beside it, ``num_splits``, the
+    bound on the context): how many splits a workgroup of attn_stream.hip takes, and into how many parts :func:`attn_parts` divides
+    a prompt's keys. The same call repeats bit for bit, the same sequence in another batch up to the sums' rounding.
     Returns [Tq, H*D] bf16.
     """
     scale = scale if scale is not None else 1.0 / math.sqrt(head_dim)
