@@ -66,3 +66,13 @@ def test_which_kernel(case, monkeypatch):
     w, pos = make(N, 3 * cin, 4 if case.startswith("weights") else 0), make(tin, N, 4 if case.startswith("positions") else 0)
     y = ops.conv_k3_gelu(x, w, torch.zeros(N), 2, 2 if tin == 1 or ld > 1 << 20 else 1, pos=pos)
     assert (y == "gemm_tile") if case != "fits" else (len(asked) == 1 and y.shape == (80, N))
+
+
+def test_layouts_are_ranked_by_the_plans_times():
+    """As a projection of whole tiles with GELU: its cost per value, and the longer steps of the 64 x 64 tiles from K = 2112 on."""
+    assert ops._conv_layout(9000, 1024, 384, ops.CONV_LAYOUTS) == 20          # 27.5 us, 27.9 in 256 x 128
+    assert ops._conv_layout(1500, 384, 1152, ops.CONV_LAYOUTS) == ops.SK_SMALL
+    for M, N, K in ((1500, 512, 2304), (700, 768, 2304), (9000, 1280, 384), (24000, 1280, 3840)):
+        best = min((lay for lay in ops.CONV_LAYOUTS if N % ops.SK_LAYOUTS[lay][0] == 0), key=lambda lay: ops._sk_us(lay, M, N, K, 1, True))
+        assert ops._conv_layout(M, N, K, ops.CONV_LAYOUTS) == best
+        assert ops._sk_plan(M, N, K, True, ops.CONV_LAYOUTS, True)[0] == best or ops._sk_plan(M, N, K, True, ops.CONV_LAYOUTS, True)[1] > 1
