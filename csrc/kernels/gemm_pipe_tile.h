@@ -20,8 +20,8 @@ template <bool AHEAD> using GpArgs = std::conditional_t<AHEAD, GemmSkCall, GemmS
 // if one of them starts late it gives its share up to the last to arrive and leaves, so a launch always
 // drains whatever else holds the compute units. The word: arrivals in bits 0 - 15, given-up shares in
 // 16 - 23, workgroups done in 24 - 31 for up to SK_SHARE chunks; more chunks than that are summed up by
-// the last. In four chunks of 128 x 192, cold weights: 320 x 4096 x 4096 32.6 -> 23.2 us, 320 x 4096 x 14336
-// 62.2 -> 50.7.
+// the last. In four chunks of 128 x 192, cold weights: 320 x 4096 x 4096 32.6 -> 23.4 us, 320 x 4096 x 14336
+// 62.2 -> 51.1.
 #define SK_KEEP 4
 #define SK_SHARE 8
 #define SK_POLLS 48

@@ -1702,12 +1702,15 @@ def graph_capture(graph: "torch.cuda.CUDAGraph", **kw):
 # Split-K tiled GEMM with an in-launch reduction (csrc/kernels/gemm_sk.hip, gemm_pipe.hip)
 _SK_EPI = {"bf16": 0, "swiglu": 1, "resid": 2}
 # layout -> (features, rows, us a K step of 64 takes a compute unit, us around a tile's K
-# loop): 1 and 7 are the general form, 11 on the pipelined tiles, one workgroup per CU. Times
+# loop): 1 and 7 are the general form, 11 on the pipelined tiles, one workgroup per CU (two of 11 fit one, but
+# share what it loads: 4096 x 4096 in 256 tiles 17 us, in 320 33). Times
 # fitted to measured ones without an epilogue of weight: they are there to rank, and 0.69 to 1.26
-# of what a whole unsplit call takes (0.73 on average with GELU). Over 75 shapes (80 to 9000 rows, N 384
-# to 28672, K 512 to 14336, cold weights, every layout and K split: profiles/gemm_plan_grid.txt)
-# the plan is the fastest in 59, 1.2 % behind the fastest on average and 22 % at worst (160 x 6144 x 4096 in
-# five chunks of 128 x 192: 25.9 us, 21.2 in four). Layout 18 is 1.4 us dearer with GELU than without, which counts for more.
+# of what a whole unsplit call takes (0.73 on average with GELU). Over 481 shapes (17 to 12000 rows, N 384
+# to 28672, K 384 to 14336, cold weights, every layout and K split: profiles/gemm_plan_grid.txt)
+# the plan is the fastest in 404, 1.0 % behind the fastest on average, more than 5 % in 37 and 21 % at worst (320 x 3072 x
+# 8192 in two chunks of 128 x 64: 36.7 us, 30.4 in three of 128 x 128; 160 x 6144 x 4096 in five of 128 x 192 25.7, in four 21.5);
+# without five chunks it would be 1.4 %. Layout 18 stands 1.4 us above what its K steps were fitted with: at 4.6 it was taken for ten
+# shapes more, with GELU and without, each 1 to 10 % slower than what is taken now (9000 x 768 x 768 19.1 us, 17.9).
 SK_LAYOUTS = {1: (128, 64, 0.60, 4.0), 7: (64, 64, 0.55, 4.0), 11: (64, 64, 0.19, 2.6),
               12: (256, 256, 1.20, 10.3), 13: (256, 192, 1.075, 5.5), 14: (192, 256, 1.073, 5.5),
               15: (256, 128, 0.908, 4.0), 16: (128, 256, 0.784, 6.6), 17: (128, 192, 0.667, 4.6),
@@ -1734,24 +1737,24 @@ def gemm_sk_plan(M: int, N: int, K: int, epi: str = "bf16", layouts=None, *,
     rows share the weights, on as many workgroups as SK_SHARED says, 0.9 (1500 x 768 x 3072 on 144 17.1 us; whole tiles of 2200 x
     4096 x 11008 on 192 171 us, in four chunks 202). 64 x 64 tiles are for what leaves half of the units idle in 128 x 64
     (1500 x 512 x 2048 11.1 -> 8.9 us, x 512 5.7 -> 4.7, 300 x 1280 x 1280 9.0 -> 6.6); their step is charged 1.26 times from K =
-    2112 on, a step of the fit.
+    2112 on: 0.16 to 0.18 us at 2048 and 3072, 0.21 to 0.25 from 4096 on (without that the plan was 1.2 % behind on average, 36 at worst).
     K chunks fill the chip where the tiles do not; each tile then pays for the trip of its f32 partials
     through memory, 3 us and 40 us a MB, and 4 us a MB for each chunk that is read back (fitted with the
-    rest; 320 x 4096 x 4096 in four chunks of 128 x 192 25.7 us, whole 29.0 in 128 x 64). Chunks of a second round are never
+    rest; 320 x 4096 x 4096 in four chunks of 128 x 192 23.4 us, whole 29.2 in 128 x 64). Chunks of a second round are never
     worth it: the tiles' partials then hold each other up and the first round's workgroups wait for chunks that have not
     begun (1600 x 4096 x 14336 on 480 workgroups of five chunks 238 us, whole in 128 x 256 167; 1100 x 16384 x 3072 on 768 of two 141, whole
     108). Their partials and the weights that a launch touches for the next one (:func:`_ahead`) hold each other up as well (1500
     x 1280 x 5120 in two chunks 28.3 us and whole 29.9 alone, but an encoder pass with 32 of them 4118 us and 4058). Never on
     256 x 256 tiles: these fill the chip with MFMAs, where a K step takes longer than the fit has it (4096 x
     14336: 1280 rows in three chunks 160 us, the 256 x 192 tiles in two 135; 2048 rows in two 205,
-    the 128 x 256 tiles whole 182; the fastest in none of the grid's shapes). ``pipe`` False:
+    the 128 x 256 tiles whole 182; the fastest in none of 75 shapes). ``pipe`` False:
     the general layouts only (operands the pipelined tiles do not take). ``layouts``: among
     these only (numbers of SK_LAYOUTS or SK_RENAMED). Of the epilogues ``epi`` only "gelu" is in the
     model: SK_GELU us for a value of a tile, as nothing runs beside its arithmetic, except
     where the 128 x 192 tiles are more than the compute units and two share one
-    (csrc/kernels/gemm_pipe_tile.h); then a round of pairs, and 0.68 of one for up to half of it. Over 60
-    shapes of the encoders' widths (100 to 24000 rows, N = 4 K, K 384 to 1280) the plan takes 0.4 % longer than the
-    fastest tile on average, 1.8 to 9 % in nine; without GELU in the model and pairs it was 4.3 %, up to 42."""
+    (csrc/kernels/gemm_pipe_tile.h); then a round of pairs, and 0.68 of one for up to half of it. Over the
+    70 shapes with GELU among the 481 (100 to 12000 rows, N = 4 K, K 384 to 1280) the plan takes 0.2 % longer than the
+    fastest tile on average, 7 % at worst; without GELU in the model and pairs it was 4.3 %, up to 42, over 60 such."""
     return _sk_plan(M, N, K, pipe, None if layouts is None else tuple(layouts), epi == "gelu")
 
 
@@ -1766,8 +1769,6 @@ def _sk_plan(M: int, N: int, K: int, pipe: bool, layouts: tuple | None = None, g
         if N % bn or (lay >= SK_PIPE) != (pipe and N % 128 == 0) or lay not in only:
             continue
         tiles = -(-M // bm) * (N // bn)
-        if lay == SK_SMALL and K > 2048:
-            step *= 1.26
         for s in (1, 2, 3, 4, 5, 6, 8):
             if s > 1 and (KT // s < 8 or lay == SK_WHOLE or (lay >= SK_PIPE and tiles * s > SK_CUS)):
                 continue
@@ -1777,7 +1778,6 @@ def _sk_plan(M: int, N: int, K: int, pipe: bool, layouts: tuple | None = None, g
     return best
 
 
-_SK_WS_GRAPHS: list = []   # workspaces of captured graphs: they live as long as the process
 def _sk_us(lay: int, M: int, N: int, K: int, s: int, gelu: bool) -> float:
     """Microseconds of M x N x K in ``s`` K chunks of layout ``lay`` (:func:`gemm_sk_plan`)."""
     bn, bm, step, around = SK_LAYOUTS[lay]
@@ -1796,6 +1796,7 @@ def _sk_us(lay: int, M: int, N: int, K: int, s: int, gelu: bool) -> float:
     return t
 
 
+_SK_WS_GRAPHS: list = []   # workspaces of captured graphs: they live as long as the process
 _SK_WS_CAPTURE: dict = {}  # (device, stream) -> (id of its newest capture, workspace)
 
 
@@ -2039,7 +2040,6 @@ def gemm_ws(x: torch.Tensor, w: torch.Tensor, *, epi: str = "bf16", bias: torch.
 CONV_LAYOUTS = (11, 15, 19, 20)
 
 
-def conv_k3_gelu(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor, B: int, stride: int,
 @functools.lru_cache(maxsize=1024)
 def _conv_layout(M: int, N: int, K: int, layouts: tuple) -> int:
     """Whole tiles by SK_LAYOUTS, as the projections' plan with GELU. Over 70 stems (1 to 16 windows, 384 to 1280 features) 1.6 %
@@ -2047,6 +2047,7 @@ def _conv_layout(M: int, N: int, K: int, layouts: tuple) -> int:
     return min((lay for lay in layouts if N % SK_LAYOUTS[lay][0] == 0), key=lambda lay: _sk_us(lay, M, N, K, 1, True))
 
 
+def conv_k3_gelu(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor, B: int, stride: int,
                  pos: torch.Tensor | None = None) -> torch.Tensor:
     """GELU(conv1d(x)) (+ ``pos`` rows m % len(pos)), k = 3, padding 1: x time-major [B * T_in, Cin]
     bf16, w a :func:`conv_k3_weight` [N, 3 * Cin], f32 ``bias`` -> [B * T_out, N] bf16. On the
