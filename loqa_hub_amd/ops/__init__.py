@@ -1709,8 +1709,8 @@ _SK_EPI = {"bf16": 0, "swiglu": 1, "resid": 2}
 # to 28672, K 384 to 14336, cold weights, every layout and K split: profiles/gemm_plan_grid.txt)
 # the plan is the fastest in 404, 1.0 % behind the fastest on average, more than 5 % in 37 and 21 % at worst (320 x 3072 x
 # 8192 in two chunks of 128 x 64: 36.7 us, 30.4 in three of 128 x 128; 160 x 6144 x 4096 in five of 128 x 192 25.7, in four 21.5);
-# without five chunks it would be 1.4 %. Layout 18 stands 1.4 us above what its K steps were fitted with: at 4.6 it was taken for ten
-# shapes more, with GELU and without, each 1 to 10 % slower than what is taken now (9000 x 768 x 768 19.1 us, 17.9).
+# without five chunks it would be 1.4 %. Layout 18 stands 1.4 us above what its K steps were fitted with: at 4.6 it was taken for
+# seven shapes more, with GELU and without, each 3 to 10 % slower than what is taken now (9000 x 768 x 768 19.1 us, 17.9).
 SK_LAYOUTS = {1: (128, 64, 0.60, 4.0), 7: (64, 64, 0.55, 4.0), 11: (64, 64, 0.19, 2.6),
               12: (256, 256, 1.20, 10.3), 13: (256, 192, 1.075, 5.5), 14: (192, 256, 1.073, 5.5),
               15: (256, 128, 0.908, 4.0), 16: (128, 256, 0.784, 6.6), 17: (128, 192, 0.667, 4.6),
