@@ -646,7 +646,9 @@ class LlamaModel:
                 and B <= ops.MPADS[-1]):
             Mpad = ops.mpad_for(B)
             x = hidden.contiguous()
-            if B == 1:          # a prompt's one row in place of padding rows (zeros and a copy: two launches)
+            # a prompt's one row in place of padding rows (zeros and a copy: two launches), if it starts on the kernel's 16-byte
+            # pieces: a slice of one row counts as contiguous wherever it starts
+            if B == 1 and x.data_ptr() % 16 == 0:
                 x = x.expand(Mpad, -1)
             elif Mpad != B:
                 x = torch.zeros(Mpad, hidden.shape[1], dtype=hidden.dtype, device=hidden.device)

@@ -117,3 +117,16 @@ def test_logits_rows_do_not_depend_on_their_padding(B):
     assert torch.equal(m.logits(hidden.repeat(1, 2)[:B, :m.cfg.d_model]), m.logits(hidden)[:B])
     ids = torch.tensor([5, 0, 7, 5], device="cuda")
     assert all(torch.equal(m.embed(ids.to(t)), m.w.embed[ids]) for t in (torch.int64, torch.int32, torch.int16))
+
+
+@pytest.mark.gpu
+def test_one_row_that_starts_off_16_bytes_is_copied(monkeypatch):
+    from loqa_hub_amd.models.configs import llama_config
+    from loqa_hub_amd.models.llama import LlamaModel, LlamaWeights
+    m = LlamaModel(LlamaWeights(llama_config("test-tiny"), torch.device("cuda", 0), seed=4))
+    rows, seen, product = torch.randn(1, m.cfg.d_model + 8, device="cuda").bfloat16(), [], ops.skinny_gemm
+    monkeypatch.setattr(ops, "skinny_gemm", lambda x, *a, **k: (seen.append((x.data_ptr() % 16, x.stride(0))), product(x, *a, **k))[1])
+    for off in (0, 1, 8):
+        hidden = rows[:, off:off + m.cfg.d_model]
+        assert torch.equal(m.logits(hidden), m.logits(hidden.clone()))
+    assert all(at == 0 for at, _ in seen) and [st == 0 for _, st in seen] == [True, True, False, True, True, True]
