@@ -59,11 +59,11 @@ __global__ __launch_bounds__(NW * 64) void attn_stream_kernel(AttnDecArgs A) {
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int li = lane & 15, fq = lane >> 4;
   const int split = blockIdx.x, kvh = blockIdx.y, b = blockIdx.z;
-  const int G = A.Hq / A.Hkv, blk = A.blk;
+  const int G = A.Hq / A.Hkv, blk = A.blk, sh = PAGED ? __builtin_ctz(blk) : 0;   // rows of a page: a power of two
   const int kbeg = split * A.split_keys;
   // block-table entries of a tile: two pages of 16 rows, or one
   const int* bt = PAGED ? A.block_tables + (size_t)b * A.max_blocks : nullptr;
-  auto page_at = [&](int kt, int i) { return as_scalar(bt + min(kt / blk + i, A.max_blocks - 1)); };
+  auto page_at = [&](int kt, int i) { return as_scalar(bt + min((kt >> sh) + i, A.max_blocks - 1)); };
   int pages[2][2] = {{0, 0}, {0, 0}};            // of the tile asked for next and of the one behind it
   const int kt0 = kbeg + wave * DEC_TILE;
   if constexpr (PAGED) {
@@ -85,7 +85,7 @@ __global__ __launch_bounds__(NW * 64) void attn_stream_kernel(AttnDecArgs A) {
 #pragma unroll
   for (int j = 0; j < NL; ++j) {
     const int r = j * RPL + lane / LPR;
-    voff[j] = (PAGED ? lane / LPR : r) * stride + (((lane % LPR) ^ swz(r)) * 16);
+    voff[j] = (PAGED ? r % (DEC_TILE / 2) : r) * stride + (((lane % LPR) ^ swz(r)) * 16);
   }
   const unsigned ring = (unsigned)(size_t)(AS_LDS unsigned char*)lds + wave * (2 * R * TB + AS_ROWS * D * 2);
   const unsigned qrow = ring + 2 * R * TB;       // the query rows, behind the ring
@@ -102,13 +102,19 @@ __global__ __launch_bounds__(NW * 64) void attn_stream_kernel(AttnDecArgs A) {
   auto ask = [&](int kt, unsigned slot, const int (&page)[2]) {
     const int n = min(max(kend - kt, 0), DEC_TILE);
     if constexpr (PAGED) {
+      // 16 rows at a time, which a page holds whole; shifts for divisions and an address for half of a tile instead of one
+      // for each load: 1500 keys x 20 heads of 64 in one workgroup each 19.4 us with these, 16.4 without, 15.7 off contiguous rows
 #pragma unroll
-      for (int j = 0; j < NL; ++j) {
-        const int at = kt + j * RPL;
-        const size_t off = (((size_t)(at / blk == kt / blk ? page[0] : page[1]) * A.Hkv + kvh) * blk + (at & (blk - 1))) * D;
-        const unsigned bytes = min(max(n - j * RPL, 0), RPL) * (D * 2);
-        as_load_lds(as_rsrc(A.kc + off, bytes), voff[j], slot + j * 1024);
-        as_load_lds(as_rsrc(A.vc + off, bytes), voff[j], slot + TB + j * 1024);
+      for (int t = 0; t < 2; ++t) {
+        const int at = kt + t * (DEC_TILE / 2);
+        const size_t off = ((((size_t)(at >> sh == kt >> sh ? page[0] : page[1]) * A.Hkv + kvh) << sh) + (at & (blk - 1))) * D;
+        const unsigned bytes = min(max(n - t * (DEC_TILE / 2), 0), DEC_TILE / 2) * (D * 2);
+        const as_u4 rk = as_rsrc(A.kc + off, bytes), rv = as_rsrc(A.vc + off, bytes);
+#pragma unroll
+        for (int j = t * (NL / 2); j < (t + 1) * (NL / 2); ++j) {
+          as_load_lds(rk, voff[j], slot + j * 1024);
+          as_load_lds(rv, voff[j], slot + TB + j * 1024);
+        }
       }
     } else {
       const size_t off = (kv0 + kt) * (size_t)A.kv_stride + (size_t)kvh * D;

@@ -212,6 +212,19 @@ def test_merge_of_many_splits_is_one_trip():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("D", [64, 128])
+def test_pages_cost_what_rows_cost(D):
+    """1500 keys a workgroup: 1.04 of the time off contiguous rows; 1.24 with divisions by the page's rows for each load."""
+    paged, ws = _token(D, 20, 1, 1, 1500, 1536, 1), ops.AttnWorkspace("cuda", 1, 20, D, 1)
+    q, kv = torch.randn(1, 20 * D, device="cuda").bfloat16(), torch.randn(1500, 40 * D, device="cuda").bfloat16()
+    cu, st, ctx = (torch.tensor(x, dtype=torch.int32).cuda() for x in ([0, 1], [0], [1500]))
+    rows = lambda: ops.attention(q, kv[:, :20 * D], kv[:, 20 * D:], cu, n_heads=20, n_kv=20, head_dim=D, causal=True, max_q=1, cu_k=st,      # noqa: E731
+                                 ctx_lens=ctx, grouped=True, split_keys=1536, num_splits=1, workspace=ws)
+    us, other = _us([paged, rows])
+    assert us < 1.12 * other, (us, other)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("D,Hkv,B,keys,split,former", [(128, 8, 33, 200, 224, True), (128, 8, 32, 200, 224, False), (128, 8, 33, 100, 128, False),
                                                        (128, 8, 33, 200, 128, False), (64, 8, 65, 200, 224, True), (64, 8, 64, 200, 224, False),
                                                        (64, 8, 97, 500, 512, True), (64, 8, 97, 520, 544, False), (64, 8, 96, 520, 544, True)])
