@@ -328,20 +328,20 @@ static int as_launch(const AttnDecArgs& a, int B, hipStream_t st) {
 // heads of 64 in splits of 256: one sequence 8.9, 9.9 (2), 11.6 (3), 15.9 (6); four 13.2, 12.0, 13.3, 16.6;
 // eight 22.8, 18.0, 20.8, 19.1; sixteen 38.5, 31.1, 31.6, 33.6; 4000 keys x 8 heads of 128 in splits of 128, eight
 // sequences 100, 56 (2), 46 (3), 39 (4), 31 (8), 32 sequences 441, 209, 158, 136, 112 (8).
-// Left to attn_decode.hip: more kv heads of all sequences than the rings of their workgroups fit on the chip (147 KB at
-// 128 columns, one a compute unit; 74 KB at 64, two), each in one split of more than a tile a wave: its 51 KB fit
+// Left to attn_decode.hip: more workgroups than their rings fit on the chip (147 KB at 128 columns, one a compute unit; 74
+// KB at 64, two), where none takes more than one split, of more than a tile a wave: its 51 KB fit
 // three times. Measured there, us in this form and in that: 128 columns, 264 heads x 130 keys 16.8, 12.0, x 600 33.0,
 // 27.0, 512 heads x 300 27.6, 21.8, x 1500 79.6, 76.5, 1024 heads x 600 66.9, 59.2; 64 columns, 640 heads x 130 keys 12.2,
 // 10.4, x 300 18.1, 16.1. At 64 columns and more heads than three a compute unit both take rounds, and from 512 keys on
-// this form is the faster one again (1280 heads x 1500 keys 91, 101).
+// this form is the faster one again (1280 heads x 1500 keys 91, 101). Several splits: 128 columns, 160 heads x 600 keys in three
+// 19.1, 17.0, x 1500 in three 32.5, 30.2; 64 columns, 384 heads x 1000 keys in two 27.4, 24.6; of 2203 shapes with one split or
+// more seven are slower than there by more than 2 %, two by 5 to 7 (560 heads of 64 x 2500 keys 77.7, 72.3).
 bool attn_stream(AttnDecArgs a, int B, int max_q, int D, hipStream_t st, int* err) {
   // 32-bit offsets within a tile's rows and a sequence's queries, 16-byte pieces
   if (a.Hq / a.Hkv * max_q > AS_ROWS || ((size_t)a.q | (size_t)a.kc | (size_t)a.vc) & 15 || a.q_stride % 8 || a.q_stride < 0 ||
       a.q_stride >= 1 << 24 || a.kv_stride < 0 || a.kv_stride >= 1 << 25)
     return false;
-  const long long heads = (long long)B * a.Hkv;
-  if (a.num_splits == 1 && a.split_keys > 4 * DEC_TILE && heads > 256 * (128 / D) && (D == 128 || heads <= 768 || a.split_keys <= 512))
-    return false;
+  const long long heads = (long long)B * a.Hkv, all = heads * a.num_splits;
   int best = 1;
   double least = 0;
   for (int f = 1; f <= a.num_splits; ++f) {
@@ -349,6 +349,7 @@ bool attn_stream(AttnDecArgs a, int B, int max_q, int D, hipStream_t st, int* er
     const double t = n * f * (double)a.split_keys * (D * 5.6e-3 / 64) + 2.0 * (n - 1);
     if (f == 1 || t < least) { least = t; best = f; }
   }
+  if (best == 1 && a.split_keys > 4 * DEC_TILE && all > 256 * (128 / D) && (D == 128 || all <= 768 || a.split_keys <= 512)) return false;
   a.split_keys *= best;
   a.num_splits = (a.num_splits + best - 1) / best;
   *err = D == 64 ? as_launch<64, 4>(a, B, st) : as_launch<128, 4>(a, B, st);

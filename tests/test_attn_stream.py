@@ -227,7 +227,9 @@ def test_pages_cost_what_rows_cost(D):
 @pytest.mark.gpu
 @pytest.mark.parametrize("D,Hkv,B,keys,split,former", [(128, 8, 33, 200, 224, True), (128, 8, 32, 200, 224, False), (128, 8, 33, 100, 128, False),
                                                        (128, 8, 33, 200, 128, False), (64, 8, 65, 200, 224, True), (64, 8, 64, 200, 224, False),
-                                                       (64, 8, 97, 500, 512, True), (64, 8, 97, 520, 544, False), (64, 8, 96, 520, 544, True)])
+                                                       (64, 8, 97, 500, 512, True), (64, 8, 97, 520, 544, False), (64, 8, 96, 520, 544, True),
+                                                       (128, 8, 20, 600, 256, True), (128, 8, 10, 600, 256, False), (128, 8, 20, 380, 128, False),
+                                                       (64, 8, 40, 1000, 512, True), (64, 8, 32, 1000, 512, False)])
 def test_many_sequences_take_the_former_kernel(D, Hkv, B, keys, split, former):
     """Either side of each line of the rule, the forms told apart by their sums' last bits; both right."""
     call = _token(D, Hkv, 2, B, keys, split, -(-keys // split))
