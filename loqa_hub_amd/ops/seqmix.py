@@ -1006,7 +1006,7 @@ def window_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
     call, extra, st = "loqa_window_attention", (), stream_ptr(q)
     if mfma and D <= 128 and not softcap and slopes is None and scale > 0:
         vparts, width = -(-Dv // 128), 64 if Dv <= 64 else 128
-        keys = int(max_ctx) if window <= 0 else min(int(max_ctx), window + 64 + keep_first)
+        keys = int(max_ctx or 0) if window <= 0 else min(int(max_ctx or 0), window + 64 + keep_first)
         parts = attn_parts(int(max_q), H * vparts * B, keys)
         if parts > 1:       # a wave's 32 rows: width / 2 accumulators a lane, maximum and sum
             blocks = -(-max_q // 64) * H * vparts * B

@@ -144,3 +144,14 @@ def test_parts_of_the_keys(feeds, pasts, H, window, keep):
     torch.cuda.synchronize()
     # every word of a ticket's line, as fl_join counts arrivals and published parts in four of them
     assert all(int(words.as_strided((words.numel(), 32), (32, 1)).abs().sum()) == 0 for _, words in ops._SK_WS.values())
+
+
+@pytest.mark.parametrize("most", [None, 0, 2100])
+def test_prompts_of_any_context_bound(most):
+    """The bound on the context only says whether keys go in parts: prompts without one are taken, whole."""
+    g = torch.Generator().manual_seed(8)
+    q, kc, vc = (torch.randn(*s, generator=g).bfloat16().to(DEV) for s in ((33, 8 * 64), (132, 16, 2 * 64), (132, 16, 2 * 64)))
+    i32 = lambda x: torch.as_tensor(x, dtype=torch.int32, device=DEV)      # noqa: E731
+    args = (q, kc, vc, i32([0, 33]), i32([2100]), i32(torch.randperm(132, generator=g).view(1, 132)), i32(range(2067, 2100)), 0.125, 0.0, 0, 0, None, 8, 2, 64, 64)
+    y, z = (seqmix.window_attention(*args, max_q=33, max_ctx=n).double() for n in (most, 2100))
+    assert (y - z).norm() <= 4e-3 * z.norm()
