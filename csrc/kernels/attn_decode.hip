@@ -24,7 +24,7 @@
 // K/V addresses need no per-lane dependent lookup.
 //
 // Up to 16 query rows per kv head run on attn_stream.hip; this form serves 17 to 32 rows, operands off 16
-// bytes, more kv heads of all sequences than that form's workgroups fit on the chip, the 8-wave and prefetching
+// bytes, more workgroups than that form fits on the chip (attn_stream.hip has the rule), the 8-wave and prefetching
 // variants where they are asked for, and the attention inside the fused launches of gemm_skinny.hip.
 #include "attn_decode.h"
 

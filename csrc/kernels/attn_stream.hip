@@ -6,8 +6,8 @@
 // trip to memory, the merge. A wave that loads a tile of 32 keys into registers, works on it and loads the
 // next has nothing under way half of the time (2.4 us a tile). Here a wave's loads go straight to its own
 // ring of two tiles in LDS, the next tile's on their way while it works on one. 1500 keys x 20 heads of 64, eight
-// sequences (61 MB) 22.7 -> 18.1 us, one 11.7 -> 8.9; 600 keys x 8 heads of 128, eight sequences 14.0 -> 12.0;
-// 4000 keys 61 -> 32, 32 sequences of them 239 -> 99 (5.3 TB/s):
+// sequences (61 MB) 19.6 -> 16.2 us, one 10.3 -> 7.4; 600 keys x 8 heads of 128, eight sequences 12.8 -> 10.2;
+// 4000 keys in splits of 128 61 -> 25, 32 sequences of them 249 -> 92 (5.7 TB/s):
 //
 //   S^T = K Q^T    : 16 x 16 x 32 MFMAs, K rows from LDS (16-byte chunks swizzled on the source address)
 //   O^T += V^T P^T : V^T from LDS by transposing reads; P^T is the S^T accumulator as it stands: the keys of
@@ -325,9 +325,9 @@ static int as_launch(const AttnDecArgs& a, int B, hipStream_t st) {
 // Takes the call if the kernel can: true, *err says how the launch went. A workgroup takes f of the
 // caller's splits: the f with the least of a compute unit's keys, 5.6 ns each at 64 columns, and its
 // further workgroups, 2 us each (their start and their part of the merges). Measured, us by f, 1500 keys x 20
-// heads of 64 in splits of 256: one sequence 8.9, 9.9 (2), 11.6 (3), 15.9 (6); four 13.2, 12.0, 13.3, 16.6;
-// eight 22.8, 18.0, 20.8, 19.1; sixteen 38.5, 31.1, 31.6, 33.6; 4000 keys x 8 heads of 128 in splits of 128, eight
-// sequences 100, 56 (2), 46 (3), 39 (4), 31 (8), 32 sequences 441, 209, 158, 136, 112 (8).
+// heads of 64 on contiguous rows in splits of 256: one sequence 7.4, 9.1 (2), 11.0 (3), 15.7 (6); four 11.0, 10.4, 11.8, 16.2;
+// eight 19.0, 16.2, 18.5, 17.4; sixteen 34.6, 29.0, 30.1, 32.1; 4000 keys x 8 heads of 128 on pages in splits of 256, eight
+// sequences 44, 34 (2), 37 (3), 29 (4), 35 (8), 32 sequences 155, 118, 113, 103, 97 (8), 92 (16).
 // Left to attn_decode.hip: more workgroups than their rings fit on the chip (147 KB at 128 columns, one a compute unit; 74
 // KB at 64, two), where none takes more than one split, of more than a tile a wave: its 51 KB fit
 // three times. Measured there, us in this form and in that: 128 columns, 264 heads x 130 keys 16.8, 12.0, x 600 33.0,
