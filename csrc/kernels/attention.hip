@@ -322,22 +322,6 @@ __global__ __launch_bounds__(64 * QW * KS, D == 64 && QW * KS == 4 ? 3 : 2) void
   const int per = (ntiles + KS - 1) / KS;                   // tiles of a run; the last may have fewer
   const int first = t0 + run * per;
 
-  bf16x8 qf[NS];
-  {
-    const bf16_t* qrow = p.q + (size_t)(q0 + (row_valid ? qi : 0)) * p.q_stride + (size_t)head * D;
-#pragma unroll
-    for (int s = 0; s < NS; ++s) {
-      uint4 v = row_valid ? *reinterpret_cast<const uint4*>(qrow + 16 * s + 8 * h) : make_uint4(0, 0, 0, 0);
-      qf[s] = *reinterpret_cast<bf16x8*>(&v);
-    }
-  }
-  float16v acc[NDT];
-#pragma unroll
-  for (int i = 0; i < NDT; ++i)
-#pragma unroll
-    for (int j = 0; j < 16; ++j) acc[i][j] = 0.f;
-  float m = -1e30f, l = 0.f;
-
   const FlFetch<D, NTH, false, false> kf(th, D, PAGED ? D : p.kv_stride);
   const FlFetch<D, NTH, true, false> vf(th, D, PAGED ? D : p.kv_stride);
   // Where a fetch stands: tiles come in order, one call each; past the last tile it stays there.
@@ -373,10 +357,28 @@ __global__ __launch_bounds__(64 * QW * KS, D == 64 && QW * KS == 4 ? 3 : 2) void
     }
     if (last >= FL_KEYS) a.kt += FL_KEYS;
   };
-  At ka = start(p.k), va = start(p.v);
   const unsigned ring = fl_lds_at(lds) + run * L::RING;
-  fl_loop<D, D>(
-      qf, acc, m, l, ring, per, p.scale_log2, lane,
+  At ka = start(p.k), va = start(p.v);
+  if (per > 0) fetch(kf, ka, ring);
+  va.pages = ka.pages;                                      // with what it holds of the table
+
+  bf16x8 qf[NS];
+  {
+    const bf16_t* qrow = p.q + (size_t)(q0 + (row_valid ? qi : 0)) * p.q_stride + (size_t)head * D;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      uint4 v = row_valid ? *reinterpret_cast<const uint4*>(qrow + 16 * s + 8 * h) : make_uint4(0, 0, 0, 0);
+      qf[s] = *reinterpret_cast<bf16x8*>(&v);
+    }
+  }
+  float16v acc[NDT];
+#pragma unroll
+  for (int i = 0; i < NDT; ++i)
+#pragma unroll
+    for (int j = 0; j < 16; ++j) acc[i][j] = 0.f;
+  float m = -1e30f, l = 0.f;
+  fl_loop<D, D, kf.N + vf.N>(
+      qf, acc, m, l, ring, per, p.scale_log2, lane, true,
       [&](float16v(&st)[2], int i) __attribute__((always_inline)) {
         // masking only where a key can be invalid for this wave (wave-uniform test)
         const int kt = (first + i) * FL_KEYS;
@@ -393,23 +395,32 @@ __global__ __launch_bounds__(64 * QW * KS, D == 64 && QW * KS == 4 ? 3 : 2) void
       [&](int, unsigned stage) __attribute__((always_inline)) { fetch(vf, va, stage); });
 
   fl_sync();                                                // every wave is done with the rings
-  fl_merge<NDT, QW, KS>(acc, m, l, reinterpret_cast<float*>(lds), run, wq, lane,
-                         KS == 4 && ntiles <= 1);   // (with two runs it would save less and cost long prompts up to 2 %)
-  if (run) return;
-  if (PARTS && parts > 1) {
-    const int block = (b * p.Hq + head) * (int)(gridDim.x / p.parts) + bx;
-    if (!fl_join<NDT, QW>(acc, m, l, p.part + (size_t)block * p.parts * QW * fl_join_floats(NDT), p.words + (size_t)block * TICKET,
-                          parts, share, wq, lane))
-      return;
+  auto finish = [&](auto all, auto& own) __attribute__((always_inline)) {
+    constexpr bool ALL = decltype(all)::value != 0;
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+#pragma unroll
+    for (int s = 0; s < FlEnd<NDT, QW, KS, ALL>::OWN; ++s) own[s] *= inv;
+    fl_store<NDT, QW, KS, ALL>(own, lds, p.o + (size_t)(q0 + row_lo + wq * 32) * p.o_stride + (size_t)head * D, p.o_stride,
+                               qlen - row_lo - wq * 32, D, run, wq, lane);
+  };
+  if (KS == 4 && !PARTS && ntiles <= 1) {                   // only run 0 has one (64 rows and keys x 32 heads of 64: 6.6 -> 6.0 us)
+    if (run) return;
+    float4v own[4 * NDT];
+    fl_units(acc, own);
+    finish(Fl<1>{}, own);
+    return;
   }
-  const float inv = l > 0.f ? 1.f / l : 0.f;
-#pragma unroll
-  for (int d = 0; d < NDT; ++d)
-#pragma unroll
-    for (int j = 0; j < 16; ++j) acc[d][j] *= inv;
-  fl_store<NDT>(acc, lds + fl_merge_bytes(NDT, QW, KS) + wq * fl_store_bytes(NDT),
-                p.o + (size_t)(q0 + row_lo + wq * 32) * p.o_stride + (size_t)head * D, p.o_stride,
-                qlen - row_lo - wq * 32, D, lane);
+  float4v own[FlEnd<NDT, QW, KS, PARTS>::OWN];
+  fl_merge<NDT, QW, KS, PARTS>(acc, own, m, l, lds, run, wq, lane);
+  if constexpr (PARTS) {
+    if (run) return;
+    const int block = (b * p.Hq + head) * (int)(gridDim.x / p.parts) + bx;
+    if (parts > 1 && !fl_join<NDT, QW>(acc, m, l, p.part + (size_t)block * p.parts * QW * fl_join_floats(NDT),
+                                       p.words + (size_t)block * TICKET, parts, share, wq, lane))
+      return;
+    fl_units(acc, own);
+  }
+  finish(Fl<PARTS>{}, own);
 }
 
 // ---------------------------------------------------------------------------
@@ -700,7 +711,7 @@ __global__ void attn_combine_kernel(const float* __restrict__ part_o,
 
 template <int D, int PAGES, int QW, int KS, bool PARTS = false>
 static int launch_pipe(const AttnParams& p, int B, int max_q, hipStream_t s) {
-  constexpr int ring = KS * FlashLds<D, D>::RING, end = fl_merge_bytes(D / 32, QW, KS) + QW * fl_store_bytes(D / 32);
+  constexpr int ring = KS * FlashLds<D, D>::RING, end = FlEnd<D / 32, QW, KS, PARTS>::BYTES;
   constexpr int bytes = ring > end ? ring : end;
   static_assert(bytes <= 160 * 1024, "LDS of a CU");
   const dim3 grid((max_q + 32 * QW - 1) / (32 * QW) * (PARTS ? p.parts : 1), p.Hq, B);

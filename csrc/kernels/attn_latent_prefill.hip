@@ -102,6 +102,26 @@ __global__ __launch_bounds__(64 * QW * KS, DK > 192 ? 1 : 2) void latent_prefill
   const int wpos_hi = __builtin_amdgcn_readfirstlane(p.pos[q0 + min(row_lo + wq * 32 + 31, row_hi)]) - koff;
   const int per = (ntiles + KS - 1) / KS, first = run * per;
 
+  // where a fetch stands: tiles come in order; past the last one it stays there
+  const FlFetch<DK, NTH, false, false> kf(th, DK, (long long)p.H * DK);
+  const FlFetch<DV, NTH, true, false> vf(th, DV, (long long)p.H * DV);
+  struct At {
+    const bf16_t* row;
+    int kt;
+  };
+  const int at0 = kt0 + max(min(first, ntiles - 1), 0) * FL_KEYS;
+  At ka{p.k + ((size_t)(k0 + at0) * p.H + head) * DK, at0}, va{p.v + ((size_t)(k0 + at0) * p.H + head) * DV, at0};
+  auto fetch = [&](const auto& f, At& a, int cols, unsigned stage) __attribute__((always_inline)) {
+    const int last = kend - 1 - a.kt;
+    f.strided(stage, a.row, last);
+    if (last >= FL_KEYS) {
+      a.row += (size_t)FL_KEYS * p.H * cols;
+      a.kt += FL_KEYS;
+    }
+  };
+  const unsigned ring = fl_lds_at(lds) + run * L::RING;
+  if (per > 0) fetch(kf, ka, DK, ring);
+
   bf16x8 qf[NS];
   {
     const bf16_t* qrow = p.q + (size_t)(q0 + min(qi, row_hi)) * p.q_st + (size_t)head * DK;
@@ -132,26 +152,10 @@ __global__ __launch_bounds__(64 * QW * KS, DK > 192 ? 1 : 2) void latent_prefill
 #pragma unroll
     for (int j = 0; j < 16; ++j) acc[i][j] = 0.f;
   float m = -1e30f, l = 0.f;
-  // where a fetch stands: tiles come in order; past the last one it stays there
-  const FlFetch<DK, NTH, false, false> kf(th, DK, (long long)p.H * DK);
-  const FlFetch<DV, NTH, true, false> vf(th, DV, (long long)p.H * DV);
-  struct At {
-    const bf16_t* row;
-    int kt;
-  };
-  const int at0 = kt0 + max(min(first, ntiles - 1), 0) * FL_KEYS;
-  At ka{p.k + ((size_t)(k0 + at0) * p.H + head) * DK, at0}, va{p.v + ((size_t)(k0 + at0) * p.H + head) * DV, at0};
-  auto fetch = [&](const auto& f, At& a, int cols, unsigned stage) __attribute__((always_inline)) {
-    const int last = kend - 1 - a.kt;
-    f.strided(stage, a.row, last);
-    if (last >= FL_KEYS) {
-      a.row += (size_t)FL_KEYS * p.H * cols;
-      a.kt += FL_KEYS;
-    }
-  };
+  const float sink = p.sink ? p.sink[head] : 0.f;
   const bool neg = !(p.scale_log2 > 0.f);                 // the loop's maxima are of growing scores
-  fl_loop<DK, DV>(
-      qf, acc, m, l, fl_lds_at(lds) + run * L::RING, per, neg ? 1.f : p.scale_log2, lane,
+  fl_loop<DK, DV, kf.N + vf.N>(
+      qf, acc, m, l, ring, per, neg ? 1.f : p.scale_log2, lane, true,
       [&](float16v(&st)[2], int i) __attribute__((always_inline)) {
         const int kt = kt0 + (first + i) * FL_KEYS;       // tiles past the last lie behind kend
         if (neg) {
@@ -178,53 +182,62 @@ __global__ __launch_bounds__(64 * QW * KS, DK > 192 ? 1 : 2) void latent_prefill
       [&](int, unsigned stage) __attribute__((always_inline)) { fetch(vf, va, DV, stage); });
 
   fl_sync();                                              // every wave is done with the rings
-  fl_merge<NDT, QW, KS>(acc, m, l, reinterpret_cast<float*>(lds), run, wq, lane);
-  if (run) return;
-  if (PARTS && parts > 1) {
+  constexpr int OWN = FlEnd<NDT, QW, KS, PARTS>::OWN;
+  const bf16_t* grow = p.gate ? p.gate + (size_t)(q0 + min(qi, row_hi)) * p.gate_ld + (size_t)head * p.Dv : nullptr;
+  float4v own[OWN];
+  uint2 gate[OWN];
+  auto ask = [&]() __attribute__((always_inline)) {       // the gates of the run's own units
+#pragma unroll
+    for (int s = 0; s < OWN; ++s) {
+      const int d0 = fl_column<NDT, QW, KS, PARTS>(s, run, lane);
+      gate[s] = make_uint2(0, 0);
+      if (grow && p.runs) {
+        if (d0 < p.Dv) gate[s] = *reinterpret_cast<const uint2*>(grow + d0);
+      } else if (grow) {
+        unsigned e[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) e[i] = d0 + i < p.Dv ? grow[d0 + i] : 0u;
+        gate[s] = make_uint2(e[0] | e[1] << 16, e[2] | e[3] << 16);
+      }
+    }
+  };
+  if constexpr (!PARTS) ask();                            // on their way while the runs meet
+  fl_merge<NDT, QW, KS, PARTS>(acc, own, m, l, lds, run, wq, lane);
+  if constexpr (PARTS) {
+    if (run) return;
     const int block = (b * p.H + head) * (int)(gridDim.x / p.parts) + bx;
-    if (!fl_join<NDT, QW>(acc, m, l, p.part + (size_t)block * p.parts * QW * fl_join_floats(NDT), p.words + (size_t)block * TICKET,
-                          parts, share, wq, lane))
+    if (parts > 1 && !fl_join<NDT, QW>(acc, m, l, p.part + (size_t)block * p.parts * QW * fl_join_floats(NDT),
+                                       p.words + (size_t)block * TICKET, parts, share, wq, lane))
       return;
+    fl_units(acc, own);
+    ask();
   }
   // the sink joins the denominator only (log2 domain, like the scores)
   float f = 1.f, den = l;
   if (p.sink) {
-    const float sk = p.sink[head] * 1.4426950408889634f;
+    const float sk = sink * 1.4426950408889634f;
     const float M = fmaxf(m, sk);
     f = exp2f(m - M);
     den = l * f + exp2f(sk - M);
   }
   const float inv = den > 0.f ? f / den : 0.f;
-  const bf16_t* grow = p.gate ? p.gate + (size_t)(q0 + min(qi, row_hi)) * p.gate_ld + (size_t)head * p.Dv : nullptr;
 #pragma unroll
-  for (int d = 0; d < NDT; ++d)
+  for (int s = 0; s < OWN; ++s) {
+    const unsigned g[2] = {gate[s].x, gate[s].y};
 #pragma unroll
-    for (int g4 = 0; g4 < 4; ++g4) {
-      const int d0 = 32 * d + 8 * g4 + 4 * h;
-      float gv[4] = {0.f, 0.f, 0.f, 0.f};
-      if (grow && d0 < p.Dv) {
-        if (p.runs) {
-          ld_run<bf16_t, 4>(grow + d0, gv);
-        } else {
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            if (d0 + i < p.Dv) gv[i] = bf2f(grow[d0 + i]);
-        }
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) acc[d][4 * g4 + i] *= grow ? inv * sigmoid_fast(gv[i]) : inv;
-    }
+    for (int i = 0; i < 4; ++i) own[s][i] *= grow ? inv * sigmoid_fast(__uint_as_float(i % 2 ? g[i / 2] & 0xffff0000u : g[i / 2] << 16)) : inv;
+  }
   if (p.rows16) {
-    fl_store<NDT>(acc, lds + fl_merge_bytes(NDT, QW, KS) + wq * fl_store_bytes(NDT),
-                  p.o + (size_t)(q0 + row_lo + wq * 32) * p.o_ld + (size_t)head * p.Dv, p.o_ld, qlen - row_lo - wq * 32, p.Dv, lane);
+    fl_store<NDT, QW, KS, PARTS>(own, lds, p.o + (size_t)(q0 + row_lo + wq * 32) * p.o_ld + (size_t)head * p.Dv, p.o_ld,
+                                 qlen - row_lo - wq * 32, p.Dv, run, wq, lane);
   } else if (valid) {
     bf16_t* orow = p.o + (size_t)(q0 + qi) * p.o_ld + (size_t)head * p.Dv;
 #pragma unroll
-    for (int d = 0; d < NDT; ++d)
+    for (int s = 0; s < OWN; ++s)
 #pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        const int e = 32 * d + 8 * (j >> 2) + 4 * h + (j & 3);
-        if (e < p.Dv) orow[e] = f2bf(acc[d][j]);
+      for (int i = 0; i < 4; ++i) {
+        const int e = fl_column<NDT, QW, KS, PARTS>(s, run, lane) + i;
+        if (e < p.Dv) orow[e] = f2bf(own[s][i]);
       }
   }
 }
@@ -337,7 +350,7 @@ extern "C" int loqa_latent_prefill(const void* q, long q_st, const void* k, cons
 #define RUN(A, C, QW, KS, PARTS)                                                              \
   do {                                                                                        \
     constexpr int ring = KS * FlashLds<A, C>::RING;                                           \
-    constexpr int end = fl_merge_bytes(C / 32, QW, KS) + QW * fl_store_bytes(C / 32);         \
+    constexpr int end = FlEnd<C / 32, QW, KS, PARTS>::BYTES;                                  \
     constexpr int bytes = ring > end ? ring : end;                                            \
     static_assert(bytes <= 160 * 1024, "LDS of a CU");                                        \
     const long blocks = (max_q + 32 * QW - 1) / (32 * QW), all = blocks * H * B;              \

@@ -77,23 +77,9 @@ __global__ __launch_bounds__(64 * QW * KS, 2) void window_attn_pipe_kernel(WinAt
   const int wpos_hi = __builtin_amdgcn_readfirstlane(p.pos[q0 + min(row_lo + wq * 32 + 31, row_hi)]);
   const int per = (max(ntiles - t0, 0) + KS - 1) / KS, first = t0 + run * per;
 
-  bf16x8 qf[NS];
-  {
-    const bf16_t* qrow = (const bf16_t*)p.q + ((size_t)(q0 + min(qi, row_hi)) * p.H + head) * p.D;
-#pragma unroll
-    for (int s = 0; s < NS; ++s) {
-      const uint4 v = valid && 16 * s + 8 * h < p.D ? *reinterpret_cast<const uint4*>(qrow + 16 * s + 8 * h) : make_uint4(0, 0, 0, 0);
-      qf[s] = *reinterpret_cast<const bf16x8*>(&v);
-    }
-  }
-  float16v acc[NDT];
-#pragma unroll
-  for (int i = 0; i < NDT; ++i)
-#pragma unroll
-    for (int j = 0; j < 16; ++j) acc[i][j] = 0.f;
-  float m = -1e30f, l = 0.f;
   const float scale_log2 = p.scale * 1.4426950408889634f;
   const float slope_log2 = GEN && p.slopes ? p.slopes[head] * 1.4426950408889634f : 0.f;
+  const float sink = p.sink ? p.sink[head] : 0.f;
   const float cap_log2 = p.cap * 1.4426950408889634f, inv_cap = p.cap > 0.f ? p.scale / p.cap : 0.f;
 
   const unsigned ring = fl_lds_at(lds) + run * L::RING;
@@ -125,9 +111,27 @@ __global__ __launch_bounds__(64 * QW * KS, 2) void window_attn_pipe_kernel(WinAt
     });
   };
   At ka = start(p.kc, g * p.D, p.G * p.D), va = start(p.vc, g * p.Dv + v0, p.G * p.Dv);
+  if (per > 0) fetch(kf, ka, ring);
+  va.pages = ka.pages;                                      // with what it holds of the table
 
-  fl_loop<DK, DV>(
-      qf, acc, m, l, ring, per, GEN ? 1.f : scale_log2, lane,
+  bf16x8 qf[NS];
+  {
+    const bf16_t* qrow = (const bf16_t*)p.q + ((size_t)(q0 + min(qi, row_hi)) * p.H + head) * p.D;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      const uint4 v = valid && 16 * s + 8 * h < p.D ? *reinterpret_cast<const uint4*>(qrow + 16 * s + 8 * h) : make_uint4(0, 0, 0, 0);
+      qf[s] = *reinterpret_cast<const bf16x8*>(&v);
+    }
+  }
+  float16v acc[NDT];
+#pragma unroll
+  for (int i = 0; i < NDT; ++i)
+#pragma unroll
+    for (int j = 0; j < 16; ++j) acc[i][j] = 0.f;
+  float m = -1e30f, l = 0.f;
+
+  fl_loop<DK, DV, kf.N + vf.N>(
+      qf, acc, m, l, ring, per, GEN ? 1.f : scale_log2, lane, p.D == DK && Dv == DV,
       [&](float16v(&st)[2], int i) __attribute__((always_inline)) {
         const int kt = tile_at(first + i), k0 = kt + 4 * h;   // tiles past the last lie behind kend
         if constexpr (GEN) {
@@ -159,47 +163,55 @@ __global__ __launch_bounds__(64 * QW * KS, 2) void window_attn_pipe_kernel(WinAt
       [&](int, unsigned stage) __attribute__((always_inline)) { fetch(vf, va, stage); });
 
   fl_sync();                                                // every wave is done with the rings
-  fl_merge<NDT, QW, KS>(acc, m, l, reinterpret_cast<float*>(lds), run, wq, lane);
-  if (run) return;
-  if (PARTS && parts > 1) {
+  constexpr int OWN = FlEnd<NDT, QW, KS, PARTS>::OWN;
+  const bf16_t* grow = p.gate ? (const bf16_t*)p.gate + (size_t)(q0 + min(qi, row_hi)) * p.gate_ld + (size_t)head * p.Dv + v0 : nullptr;
+  float4v own[OWN];
+  uint2 gate[OWN];
+  auto ask = [&]() __attribute__((always_inline)) {         // the gates of the run's own units
+#pragma unroll
+    for (int s = 0; s < OWN; ++s) {
+      const int d0 = fl_column<NDT, QW, KS, PARTS>(s, run, lane);
+      gate[s] = grow && d0 < Dv ? *reinterpret_cast<const uint2*>(grow + d0) : make_uint2(0, 0);
+    }
+  };
+  if constexpr (!PARTS) ask();                              // on their way while the runs meet
+  fl_merge<NDT, QW, KS, PARTS>(acc, own, m, l, lds, run, wq, lane);
+  if constexpr (PARTS) {
+    if (run) return;
     const int block = (b * (int)gridDim.y + head * p.vparts + v0 / DV) * (int)(gridDim.x / p.parts) + bx;
-    if (!fl_join<NDT, QW>(acc, m, l, p.part + (size_t)block * p.parts * QW * fl_join_floats(NDT), p.words + (size_t)block * TICKET,
-                          parts, share, wq, lane))
+    if (parts > 1 && !fl_join<NDT, QW>(acc, m, l, p.part + (size_t)block * p.parts * QW * fl_join_floats(NDT),
+                                       p.words + (size_t)block * TICKET, parts, share, wq, lane))
       return;
+    fl_units(acc, own);
+    ask();
   }
   float inv = l > 0.f ? 1.f / l : 0.f;
   if (p.sink) {
     // the running maximum and sum are in the base-2 domain
-    const float sl = p.sink[head] * 1.44269504088896f;
+    const float sl = sink * 1.44269504088896f;
     const float mx2 = fmaxf(m, sl);
     const float a = __builtin_amdgcn_exp2f(m - mx2);
     inv = a / (l * a + __builtin_amdgcn_exp2f(sl - mx2));
   }
-  const bf16_t* grow = p.gate ? (const bf16_t*)p.gate + (size_t)(q0 + min(qi, row_hi)) * p.gate_ld + (size_t)head * p.Dv + v0 : nullptr;
 #pragma unroll
-  for (int d = 0; d < NDT; ++d)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int d0 = 32 * d + 8 * r + 4 * h;
-      float f[4] = {inv, inv, inv, inv};
-      if (grow && d0 < Dv) {
-        const uint2 gw = *reinterpret_cast<const uint2*>(grow + d0);
-        f[0] *= sigmoid_fast(__uint_as_float(gw.x << 16));
-        f[1] *= sigmoid_fast(__uint_as_float(gw.x & 0xffff0000u));
-        f[2] *= sigmoid_fast(__uint_as_float(gw.y << 16));
-        f[3] *= sigmoid_fast(__uint_as_float(gw.y & 0xffff0000u));
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) acc[d][4 * r + i] *= f[i];
+  for (int s = 0; s < OWN; ++s) {
+    float f[4] = {inv, inv, inv, inv};
+    if (grow) {
+      f[0] *= sigmoid_fast(__uint_as_float(gate[s].x << 16));
+      f[1] *= sigmoid_fast(__uint_as_float(gate[s].x & 0xffff0000u));
+      f[2] *= sigmoid_fast(__uint_as_float(gate[s].y << 16));
+      f[3] *= sigmoid_fast(__uint_as_float(gate[s].y & 0xffff0000u));
     }
-  fl_store<NDT>(acc, lds + fl_merge_bytes(NDT, QW, KS) + wq * fl_store_bytes(NDT),
-                (bf16_t*)p.o + (size_t)(q0 + row_lo + wq * 32) * p.o_ld + (size_t)head * p.Dv + v0, p.o_ld,
-                qlen - row_lo - wq * 32, Dv, lane);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) own[s][i] *= f[i];
+  }
+  fl_store<NDT, QW, KS, PARTS>(own, lds, (bf16_t*)p.o + (size_t)(q0 + row_lo + wq * 32) * p.o_ld + (size_t)head * p.Dv + v0, p.o_ld,
+                               qlen - row_lo - wq * 32, Dv, run, wq, lane);
 }
 
 template <int DK, int DV, int QW, int KS, bool GEN, bool PARTS = false>
 static int launch(const WinAttnParams& p, int max_q, hipStream_t st) {
-  constexpr int ring = KS * FlashLds<DK, DV>::RING, end = fl_merge_bytes(DV / 32, QW, KS) + QW * fl_store_bytes(DV / 32);
+  constexpr int ring = KS * FlashLds<DK, DV>::RING, end = FlEnd<DV / 32, QW, KS, PARTS>::BYTES;
   constexpr int bytes = ring > end ? ring : end;
   static_assert(bytes <= 160 * 1024, "LDS of a CU");
   const long blocks = (max_q + 32 * QW - 1) / (32 * QW), all = blocks * p.H * p.vparts * p.B;

@@ -38,6 +38,21 @@ __device__ __forceinline__ float16v fl_mfma(const bf16x8& a, const bf16x8& b, co
 
 template <int V> struct Fl { static constexpr int value = V; };
 
+// f(Fl<u>{}) for every u of A .. B - 1: indexes of registers that are constants from the start
+template <int A, int B, typename F> __device__ __forceinline__ void fl_each(F&& f) {
+  if constexpr (A < B) {
+    f(Fl<A>{});
+    fl_each<A + 1, B>(f);
+  }
+}
+
+// f(Fl<run>{}) for a wave-uniform run < KS: what the runs keep in registers at different places
+template <int KS, int R = 0, typename F> __device__ __forceinline__ void fl_by_run(int run, F&& f) {
+  if constexpr (R + 1 == KS) f(Fl<R>{});
+  else if (run == R) f(Fl<R>{});
+  else fl_by_run<KS, R + 1>(run, f);
+}
+
 template <int DK, int DV> struct FlashLds {
   static constexpr int K = FL_KEYS * DK * 2, V = FL_KEYS * DV * 2;   // bytes of a stage
   static constexpr int RING = 2 * (K + V);                           // K stages, then V stages
@@ -154,6 +169,21 @@ __device__ __forceinline__ void fl_sync() {
   asm volatile("" ::: "memory");
 }
 
+// the same for the first tile of K only, with N loads behind it
+template <int N> __device__ __forceinline__ void fl_sync_first() {
+  static_assert(N < 64, "vmcnt range");
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// LDS writes of all waves are visible; global loads stay in flight
+__device__ __forceinline__ void fl_meet() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
 __device__ __forceinline__ float fl_max32(float x) {   // over lane and lane ^ 32
   typedef unsigned u2 __attribute__((ext_vector_type(2)));
   const u2 r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
@@ -172,13 +202,14 @@ __device__ __forceinline__ float fl_both32(float x) {  // lane + lane ^ 32
 // lane (column, h) is key 32 t + (j & 3) + 8 (j >> 2) + 4 h; a wave whose rows see nothing of a
 // tile masks all of it (it would wait for the others anyway, and one path through the loop
 // leaves the registers where they are). load_k / load_v(i, stage) start the fetch of tile i;
-// they are called for i = 0, 1, 2, .. up to n (K) and n - 1 (V); for i = n they must fetch
-// something that exists (or nothing).
+// they are called for i = 1, 2, .. up to n (K) and i = 0 .. n - 1 (V); for i = n they must fetch
+// something that exists (or nothing). Where n > 0 the caller has started the fetch of K tile 0 into the ring, ahead of
+// its loads of Q: one trip to memory for both. counted: V 0 and K 1 are BEHIND loads of every wave exactly.
 // Before the call m = -1e30, l = 0, acc = 0; ring must not be in use. After it the waves
 // are not synchronised.
-template <int DK, int DV, typename Prep, typename LoadK, typename LoadV>
+template <int DK, int DV, int BEHIND, typename Prep, typename LoadK, typename LoadV>
 __device__ __forceinline__ void fl_loop(const bf16x8 (&qf)[DK / 16], float16v (&acc)[DV / 32], float& m, float& l,
-                                        unsigned ring, int n, float sl2, int lane, Prep&& prep,
+                                        unsigned ring, int n, float sl2, int lane, bool counted, Prep&& prep,
                                         LoadK&& load_k, LoadV&& load_v) {
   using L = FlashLds<DK, DV>;
   // The sums of a tile's P, rounded to bf16 as in the numerator, so that a row's weights add up to
@@ -210,7 +241,7 @@ __device__ __forceinline__ void fl_loop(const bf16x8 (&qf)[DK / 16], float16v (&
   for (int j = 0; j < 8; ++j) ones[j] = (__bf16)1.0f;
   const fl_b2 one2 = {(__bf16)1.0f, (__bf16)1.0f};
 
-  // Q is here before the first load whose wait the compiler does not know
+  // Q is here, and with it K 0, before the next loads whose wait the compiler does not know
   bf16x8 qr[NS];
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
@@ -262,12 +293,21 @@ __device__ __forceinline__ void fl_loop(const bf16x8 (&qf)[DK / 16], float16v (&
       }
     };
     // tile i's V and i + 1's K are here, the K of i and the V of i - 1 have been read
-    fl_sync();
+    if constexpr (SM) {
+      fl_sync();
+    } else {
+      load_v(0, ring + 2 * L::K);
+      load_k(1, ring + L::K);
+      if (counted) fl_sync_first<BEHIND>();
+      else fl_sync();
+    }
     if constexpr (QK) {
 #pragma unroll
       for (int u = 0; u < KR - 1; ++u) kread(u, 1 - S);
-      load_k(i + 2, ring + S * L::K);
-      load_v(i + 1, ring + 2 * L::K + (1 - S) * L::V);
+      if constexpr (SM) {
+        load_k(i + 2, ring + S * L::K);
+        load_v(i + 1, ring + 2 * L::K + (1 - S) * L::V);
+      }
     }
 #pragma unroll
     for (int u = 0; u < NQ; ++u) {
@@ -323,8 +363,7 @@ __device__ __forceinline__ void fl_loop(const bf16x8 (&qf)[DK / 16], float16v (&
 
   if (n <= 0) return;
   float16v sa[2], sb[2];
-  load_k(0, ring);
-  body(Fl<1>{}, Fl<0>{}, Fl<1>{}, sb, sa, -1);         // scores of tile 0; fetches K 1 and V 0
+  body(Fl<1>{}, Fl<0>{}, Fl<1>{}, sb, sa, -1);         // scores of tile 0; fetches V 0 and K 1
   int i = 0;
   for (; i + 2 < n; i += 2) {
     body(Fl<1>{}, Fl<1>{}, Fl<0>{}, sa, sb, i);
@@ -341,40 +380,121 @@ __device__ __forceinline__ void fl_loop(const bf16x8 (&qf)[DK / 16], float16v (&
   if constexpr (!ROW) l = fl_both32(l);                 // a lane has summed its half of the keys
 }
 
-// ---- the end of a pass. The KS runs of a query block meet in LDS: run 0 leaves with the
-// joint (m, l, acc) of its QW waves. Called by all waves, the rings no longer in use. one: only
-// run 0 has tiles (the same for all waves; 64 rows and keys x 32 heads of 64: 7.1 -> 6.0 us).
-__host__ __device__ constexpr int fl_merge_bytes(int NDT, int QW, int KS) { return (KS - 1) * QW * (NDT * 16 + 2) * 256; }
+// ---- the end of a pass. The KS runs of a query block meet in LDS, and each of them finishes its share of the
+// output: a unit is four columns of a lane's row (accumulators 4 g .. of block d: unit 4 d + g), a run's
+// units lie side by side. With run 0 finishing all of it, as it was, half or three quarters of the waves stood idle behind the last
+// tile (with K 0 fetched ahead of Q as well: 64 rows and keys x 16 heads of 192 / 128 9.4 -> 8.1 us, 1024 x 16 22.0 -> 20.8;
+// 1500 rows x 8 heads of 64 behind 256 keys 6.7 -> 6.2). ALL: run 0 has all units (what other workgroups join, fl_join).
+template <int NDT, int QW, int KS, bool ALL = false> struct FlEnd {
+  static constexpr int U = 4 * NDT;
+  static constexpr int first(int r) { return ALL ? (r ? U : 0) : r * U / KS; }
+  static constexpr int count(int r) { return first(r + 1) - first(r); }
+  static constexpr int OWN = ALL ? U : U / KS;
+  static_assert(ALL || OWN * KS == U, "whole units for every run");
+  static constexpr bool own(int r, int u) { return u >= first(r) && u < first(r + 1); }
+  // the place of unit u among the others' that run r leaves in LDS, a kilobyte each per wave of rows
+  static constexpr int slot(int r, int u) { return r * U - first(r) + (u < first(r) ? u : u - count(r)); }
+  static constexpr int ML = (KS - 1) * U * QW * 1024;                  // where (m, l) lie
+  static constexpr int MERGE = KS > 1 ? ML + KS * QW * 512 : 0;        // bytes
+  static constexpr int LD = NDT * 64 + 16, ROWS = 32 * LD;             // of a row and of a wave's 32 rows as bf16, behind those
+  static constexpr int BYTES = MERGE + QW * ROWS;
+};
 
-template <int NDT, int QW, int KS>
-__device__ __forceinline__ void fl_merge(float16v (&acc)[NDT], float& m, float& l, float* x, int run, int wq, int lane,
-                                         bool one = false) {
-  if constexpr (KS > 1) {
-    if (one) return;
-    constexpr int PER = (NDT * 16 + 2) * 64;
-    if (run) {
-      float* my = x + ((run - 1) * QW + wq) * PER + lane;
+template <int U, int NDT> __device__ __forceinline__ float4v fl_unit(const float16v (&acc)[NDT]) {
+  constexpr int d = U / 4, j = 4 * (U % 4);
+  return float4v{acc[d][j], acc[d][j + 1], acc[d][j + 2], acc[d][j + 3]};
+}
+
+template <int NDT, int N> __device__ __forceinline__ void fl_units(const float16v (&acc)[NDT], float4v (&own)[N]) {
+  static_assert(N == 4 * NDT, "all of them");
+  fl_each<0, N>([&](auto c) __attribute__((always_inline)) { own[decltype(c)::value] = fl_unit<decltype(c)::value>(acc); });
+}
+
+// Called by all waves, the rings no longer in use. Afterwards m and l are the joint ones and own has the run's units;
+// with ALL acc of run 0 has them, and the other runs' are of no use.
+template <int NDT, int QW, int KS, bool ALL, int N>
+__device__ __forceinline__ void fl_merge(float16v (&acc)[NDT], float4v (&own)[N], float& m, float& l,
+                                         unsigned char* lds, int run, int wq, int lane) {
+  using E = FlEnd<NDT, QW, KS, ALL>;
+  if constexpr (KS == 1) {
+    fl_units(acc, own);
+  } else {
+    unsigned char* x = lds + wq * 1024 + lane * 16;
+    fl_by_run<KS>(run, [&](auto r) __attribute__((always_inline)) {
+      constexpr int R = decltype(r)::value;
+      fl_each<0, E::U>([&](auto c) __attribute__((always_inline)) {
+        constexpr int u = decltype(c)::value;
+        if constexpr (!E::own(R, u)) *reinterpret_cast<float4v*>(x + E::slot(R, u) * QW * 1024) = fl_unit<u>(acc);
+      });
+    });
+    float2* ml = reinterpret_cast<float2*>(lds + E::ML + wq * 512 + lane * 8);
+    ml[run * QW * 64] = make_float2(m, l);
+    fl_meet();
+    if (ALL && run) return;
+    float a[KS], lr[KS];
 #pragma unroll
-      for (int d = 0; d < NDT; ++d)
-#pragma unroll
-        for (int j = 0; j < 16; ++j) my[(d * 16 + j) * 64] = acc[d][j];
-      my[NDT * 16 * 64] = m;
-      my[(NDT * 16 + 1) * 64] = l;
+    for (int r = 0; r < KS; ++r) {
+      const float2 v = ml[r * QW * 64];
+      a[r] = v.x;
+      lr[r] = v.y;
     }
-    fl_sync();
-    if (run) return;
+    m = a[0];
 #pragma unroll
-    for (int r = 1; r < KS; ++r) {
-      const float* o = x + ((r - 1) * QW + wq) * PER + lane;
-      const float m1 = o[NDT * 16 * 64], l1 = o[(NDT * 16 + 1) * 64];
-      const float top = fmaxf(m, m1), a0 = exp2f(m - top), a1 = exp2f(m1 - top);
-      m = top;
-      l = l * a0 + l1 * a1;
+    for (int r = 1; r < KS; ++r) m = fmaxf(m, a[r]);
+    l = 0.f;
 #pragma unroll
-      for (int d = 0; d < NDT; ++d)
-#pragma unroll
-        for (int j = 0; j < 16; ++j) acc[d][j] = acc[d][j] * a0 + o[(d * 16 + j) * 64] * a1;
+    for (int r = 0; r < KS; ++r) {
+      a[r] = exp2f(a[r] - m);
+      l = r ? l + lr[r] * a[r] : lr[r] * a[r];
     }
+    fl_by_run<ALL ? 1 : KS>(run, [&](auto r) __attribute__((always_inline)) {
+      constexpr int R = decltype(r)::value;
+      fl_each<E::first(R), E::first(R + 1)>([&](auto c) __attribute__((always_inline)) {
+        constexpr int u = decltype(c)::value;
+        float4v s = {0.f, 0.f, 0.f, 0.f};
+        fl_each<0, KS>([&](auto kc) __attribute__((always_inline)) {
+          constexpr int k = decltype(kc)::value;
+          float4v v;
+          if constexpr (k == R) v = fl_unit<u>(acc);
+          else v = *reinterpret_cast<const float4v*>(x + E::slot(k, u) * QW * 1024);
+          if constexpr (k == 0) s = v * a[k];
+          else s = s + v * a[k];
+        });
+        if constexpr (ALL)
+          fl_each<0, 4>([&](auto e) __attribute__((always_inline)) { acc[u / 4][4 * (u % 4) + decltype(e)::value] = s[decltype(e)::value]; });
+        else own[u - E::first(R)] = s;
+      });
+    });
+  }
+}
+
+// The first column of a run's s-th unit for a lane (the unit's own of ALL: run 0).
+template <int NDT, int QW, int KS, bool ALL> __device__ __forceinline__ int fl_column(int s, int run, int lane) {
+  return 8 * ((ALL ? 0 : run * FlEnd<NDT, QW, KS, ALL>::OWN) + s) + 4 * (lane >> 5);
+}
+
+// A run's finished units of a wave's 32 rows as bf16 to y (rows ld apart, `rows` of them exist, `cols` <= 32 NDT columns,
+// a multiple of 8), turned through LDS: a lane's units are 4 columns of its row each, and 8-byte pieces of 32 rows in one
+// store make every piece a line of its own. Each run stores its share of whole rows.
+template <int NDT, int QW, int KS, bool ALL, int OWN>
+__device__ __forceinline__ void fl_store(const float4v (&own)[OWN], unsigned char* lds, bf16_t* y, long long ld,
+                                         int rows, int cols, int run, int wq, int lane) {
+  using E = FlEnd<NDT, QW, KS, ALL>;
+  static_assert(OWN == E::OWN, "a run's units");
+  constexpr int CPR = NDT * 4, N = ALL ? 32 : 32 / KS;      // 16-byte pieces of a row, rows of a run
+  unsigned char* my = lds + E::MERGE + wq * E::ROWS;
+#pragma unroll
+  for (int s = 0; s < E::OWN; ++s)
+    *reinterpret_cast<uint2*>(my + (lane & 31) * E::LD + fl_column<NDT, QW, KS, ALL>(s, run, lane) * 2) =
+        make_uint2(pack_bf16x2(own[s][0], own[s][1]), pack_bf16x2(own[s][2], own[s][3]));
+  if constexpr (KS > 1 && !ALL) fl_meet();
+  else __builtin_amdgcn_wave_barrier();
+  const int r0 = KS > 1 && !ALL ? run * N : 0;
+#pragma unroll
+  for (int k = 0; k < N * CPR / 64; ++k) {
+    const int id = lane + 64 * k, r = r0 + id / CPR, c = id % CPR;
+    const fl_u4 v = *reinterpret_cast<const fl_u4*>(my + r * E::LD + c * 16);
+    if (r < rows && c * 8 < cols) *reinterpret_cast<fl_u4*>(y + (size_t)r * ld + c * 8) = v;
   }
 }
 
@@ -474,29 +594,4 @@ __device__ __forceinline__ bool fl_join(float16v (&acc)[NDT], float& m, float& l
   else if (n <= 4) fl_join_sum<NDT, QW, 4, 4>(acc, m, l, r, n, mine, wq, lane);
   else fl_join_sum<NDT, QW, FL_PARTS, 2>(acc, m, l, r, n, mine, wq, lane);
   return true;
-}
-
-// A wave's 32 rows as bf16 to y (rows ld apart, `rows` of them exist, `cols` <= 32 NDT columns,
-// a multiple of 8), turned through LDS: a lane's accumulators are 4 columns of its row, and 8-byte
-// pieces of 32 rows in one store make every piece a line of its own.
-__host__ __device__ constexpr int fl_store_bytes(int NDT) { return 32 * (NDT * 64 + 16); }
-
-template <int NDT>
-__device__ __forceinline__ void fl_store(const float16v (&acc)[NDT], unsigned char* my, bf16_t* y, long long ld, int rows,
-                                         int cols, int lane) {
-  constexpr int LD = NDT * 64 + 16, CPR = NDT * 4;
-  const int h = lane >> 5;
-#pragma unroll
-  for (int d = 0; d < NDT; ++d)
-#pragma unroll
-    for (int g = 0; g < 4; ++g)
-      *reinterpret_cast<uint2*>(my + (lane & 31) * LD + (32 * d + 8 * g + 4 * h) * 2) =
-          make_uint2(pack_bf16x2(acc[d][4 * g], acc[d][4 * g + 1]), pack_bf16x2(acc[d][4 * g + 2], acc[d][4 * g + 3]));
-  __builtin_amdgcn_wave_barrier();
-#pragma unroll
-  for (int k = 0; k < 32 * CPR / 64; ++k) {
-    const int id = lane + 64 * k, r = id / CPR, c = id % CPR;
-    const fl_u4 v = *reinterpret_cast<const fl_u4*>(my + r * LD + c * 16);
-    if (r < rows && c * 8 < cols) *reinterpret_cast<fl_u4*>(y + (size_t)r * ld + c * 8) = v;
-  }
 }
