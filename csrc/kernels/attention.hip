@@ -378,7 +378,7 @@ __global__ __launch_bounds__(64 * QW * KS, D == 64 && QW * KS == 4 ? 3 : 2) void
     for (int j = 0; j < 16; ++j) acc[i][j] = 0.f;
   float m = -1e30f, l = 0.f;
   fl_loop<D, D, kf.N + vf.N>(
-      qf, acc, m, l, ring, per, p.scale_log2, lane, true,
+      qf, acc, m, l, ring, per, p.scale_log2, lane, true, QW * KS == 8 ? wave >> 2 : -1,
       [&](float16v(&st)[2], int i) __attribute__((always_inline)) {
         // masking only where a key can be invalid for this wave (wave-uniform test)
         const int kt = (first + i) * FL_KEYS;

@@ -131,7 +131,7 @@ __global__ __launch_bounds__(64 * QW * KS, 2) void window_attn_pipe_kernel(WinAt
   float m = -1e30f, l = 0.f;
 
   fl_loop<DK, DV, kf.N + vf.N>(
-      qf, acc, m, l, ring, per, GEN ? 1.f : scale_log2, lane, p.D == DK && Dv == DV,
+      qf, acc, m, l, ring, per, GEN ? 1.f : scale_log2, lane, p.D == DK && Dv == DV, QW * KS == 8 ? wave >> 2 : -1,
       [&](float16v(&st)[2], int i) __attribute__((always_inline)) {
         const int kt = tile_at(first + i), k0 = kt + 4 * h;   // tiles past the last lie behind kend
         if constexpr (GEN) {

@@ -8,7 +8,7 @@
 // What bounds a tile of a wave: at 64 / 64 head columns the VALU (32 exp2 of 8 cycles, fma,
 // maximum, conversion, rescaling: ~700 cycles) as much as the MFMAs (640), at 128 / 128 the
 // MFMAs (1024). Done one after the other they add up, and two waves of a SIMD that share a barrier
-// per tile stay in step instead of filling each other's gaps. So the scores of tile i + 1 are
+// per tile stay in step instead of filling each other's gaps (fl_loop's phase has them half a tile apart). So the scores of tile i + 1 are
 // computed between the exponentials of tile i (first half of the keys), its first P V product
 // between those of the second half, and the second P V product covers the row maxima of
 // i + 1. O is rescaled in a branch, when a row of the wave has a new maximum.
@@ -177,6 +177,13 @@ template <int N> __device__ __forceinline__ void fl_sync_first() {
   asm volatile("" ::: "memory");
 }
 
+// every wave is here, whatever it waits for
+__device__ __forceinline__ void fl_step() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
 // LDS writes of all waves are visible; global loads stay in flight
 __device__ __forceinline__ void fl_meet() {
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -205,11 +212,16 @@ __device__ __forceinline__ float fl_both32(float x) {  // lane + lane ^ 32
 // they are called for i = 1, 2, .. up to n (K) and i = 0 .. n - 1 (V); for i = n they must fetch
 // something that exists (or nothing). Where n > 0 the caller has started the fetch of K tile 0 into the ring, ahead of
 // its loads of Q: one trip to memory for both. counted: V 0 and K 1 are BEHIND loads of every wave exactly.
+// phase: -1, or in workgroups of eight waves 0 for the first four and 1 for the others, which share the four SIMDs: each
+// half of a tile then begins with a barrier of all waves, and the second four run half a tile behind, their exponentials,
+// maxima and rescaling beside the scores' MFMAs of the first (in step, both waves of a SIMD want the same unit; 2048 rows of
+// 16 latent heads of 192 / 128 43.7 -> 41.6 us, of 32 58.5 -> 56.7, 1500 rows x 8 heads of 64 13.7 -> 12.9; wave priorities
+// and six or eight fragments in flight beside it: the same within 1 %).
 // Before the call m = -1e30, l = 0, acc = 0; ring must not be in use. After it the waves
 // are not synchronised.
 template <int DK, int DV, int BEHIND, typename Prep, typename LoadK, typename LoadV>
 __device__ __forceinline__ void fl_loop(const bf16x8 (&qf)[DK / 16], float16v (&acc)[DV / 32], float& m, float& l,
-                                        unsigned ring, int n, float sl2, int lane, bool counted, Prep&& prep,
+                                        unsigned ring, int n, float sl2, int lane, bool counted, int phase, Prep&& prep,
                                         LoadK&& load_k, LoadV&& load_v) {
   using L = FlashLds<DK, DV>;
   // The sums of a tile's P, rounded to bf16 as in the numerator, so that a row's weights add up to
@@ -324,6 +336,7 @@ __device__ __forceinline__ void fl_loop(const bf16x8 (&qf)[DK / 16], float16v (&
     }
     // what is used in a later block stays computed in this one
     if constexpr (SM) asm volatile("" : "+v"(pf[0][0]), "+v"(pf[0][1]));
+    if (phase >= 0) fl_step();
     if constexpr (QK) prep(nxt, i + 1);
     if constexpr (SM) {
 #pragma unroll
@@ -363,6 +376,7 @@ __device__ __forceinline__ void fl_loop(const bf16x8 (&qf)[DK / 16], float16v (&
 
   if (n <= 0) return;
   float16v sa[2], sb[2];
+  if (phase == 1) fl_step();
   body(Fl<1>{}, Fl<0>{}, Fl<1>{}, sb, sa, -1);         // scores of tile 0; fetches V 0 and K 1
   int i = 0;
   for (; i + 2 < n; i += 2) {
@@ -377,6 +391,7 @@ __device__ __forceinline__ void fl_loop(const bf16x8 (&qf)[DK / 16], float16v (&
     for (int d = 0; d < NDT; ++d) vb[d] += L::V;        // the last tile's V lies in the other stage
   }
   body(Fl<0>{}, Fl<1>{}, Fl<0>{}, sa, sb, n - 1);
+  if (phase == 0) fl_step();
   if constexpr (!ROW) l = fl_both32(l);                 // a lane has summed its half of the keys
 }
 
