@@ -1009,11 +1009,7 @@ static int window_attention(const void* q, int dt, const void* kc, const void* v
   if (ns > 1 && part) { p.ns = ns; p.part = (float*)part; }
   if (dt == 0) {
     const int rc = window_attention_token(p, st);
-    if (rc > 0) return rc;
-    if (rc == 0) {
-      if (p.ns > 1) hipLaunchKernelGGL(window_attn_combine_kernel<bf16_t>, dim3(T, H), dim3(128), 0, st, p);
-      return (int)hipGetLastError();
-    }
+    if (rc >= 0) return rc;
   }
   const int rep = H / G;
   // value layout: whole rows in 16-byte runs when Dv / (elements per run) is a

@@ -2,18 +2,19 @@
 // query rows against many keys, bound by the reads of K and V and, at the sizes of a step, by
 // the chain from the block table over the keys and their maximum to the values and the merge.
 //
-// A workgroup of 16 waves serves one token and key head (ns: or a share of its keys). A wave
-// takes 32 keys at a time: K rows go from the pages straight to the A operands of the score
+// A workgroup of 16 waves serves one token and key head, or with key splits (p.ns) one of four waves a share of
+// its keys. A wave takes 32 keys at a time: K rows go from the pages straight to the A operands of the score
 // MFMAs (16 x 16 x 32; the group's query heads, up to 16, are the columns), V rows straight to
 // its part of LDS meanwhile, whence transposed reads make them the A operands of the second
 // product, whose B operand the exponentials of the scores are as they lie. All of a wave's loads
-// are in flight together, maxima of 16 heads cost two exchanges, and 512 keys of a row are read
-// at once, so that windows of some 1000 keys need neither key splits nor a second launch.
+// are in flight together and maxima of 16 heads cost two exchanges. What one compute unit gets of K and V bounds a
+// workgroup (60 KB/us), so beyond some 400 keys a row's keys are split and the splits join in the launch.
 // The weights stay what 32 bits hold: each goes as a sum of three bf16 (24 bits), none of them
 // negative or zero, so that an infinite value stays one.
-// 8 tokens, 16 heads (4 key heads) of 128, window 1024: 20.6 + 3.9 us before (a key on one lane
-// at a time, 12 cross-lane steps a head and 64 keys, five key splits and their merge), 12.4 now,
-// two rounds of loads; up to 500 keys 17 before, 6.5 now; 64 tokens behind 2000: 168, 100.
+// 8 tokens, 16 heads (4 key heads) of 128, window 1024: 24.5 us at first (a key on one lane
+// at a time, five key splits and their merge in a second launch), 15.9 in one workgroup of 16 waves, 9.0 in eight of four;
+// 4000 keys 26.9 (splits of 16 waves and the second launch), 18.9; up to 400 keys 16 waves 6 to 8; 64 tokens
+// behind 2000: 168, 100.
 #include "flash_pipe.h"
 #include "seqmix.h"
 
@@ -32,6 +33,92 @@ __device__ __forceinline__ float wt_sum16(float x) {
 
 // place of chunk c of V row r: a half wave reads 8 rows of two chunks
 template <int DV> __device__ __forceinline__ int wt_swz(int r) { return DV == 128 ? 2 * (r & 7) : 2 * ((r >> 1) & 3); }
+
+// Of a workgroup's partial: per head and column the sum, then (maximum, sum of the weights) per head.
+__host__ __device__ __forceinline__ int wt_part_floats(int rep, int Dv) { return rep * Dv + (2 * rep + 3) / 4 * 4; }
+
+// The workgroups of a row's key splits (p.ns of them): each leaves the joint partial of its waves (mm, ll, aa in LDS, which
+// this uses up), and the last to arrive sums them up in the splits' order, whichever it is. Nobody waits for anybody.
+// Written through and read past the caches (sc1).
+template <int NW, int DV>
+__device__ __forceinline__ void wt_join(const WinAttnParams& p, float* mm, float* ll, float* aa, int t, int g, int sp, int rep) {
+  constexpr int SC1 = 16, TH = 64 * NW, BATCH = 8;
+  const int tid = threadIdx.x, Dv = p.Dv, per = wt_part_floats(rep, Dv), row = t * p.G + g, quads = rep * Dv / 4;
+  constexpr float LOG2E = 1.4426950408889634f;
+  const __amdgpu_buffer_rsrc_t part = __builtin_amdgcn_make_buffer_rsrc(p.part + (size_t)row * p.ns * per, 0, p.ns * per * 4, 0x00020000);
+  auto top = [&](int r) {
+    float M = -1e30f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) M = fmaxf(M, mm[w * 16 + r]);
+    return M;
+  };
+  for (int q = tid; q < quads; q += TH) {
+    const int r = q * 4 / Dv, e = q * 4 - r * Dv;
+    const float M = top(r);
+    float4v num = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < NW; ++w)
+      num += __builtin_amdgcn_exp2f(mm[w * 16 + r] - M) * *reinterpret_cast<const float4v*>(aa + ((size_t)w * rep + r) * DV + e);
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(fl_u4, num), part, (sp * per + q * 4) * 4, 0, SC1);
+  }
+  if (tid < rep) {
+    const float M = top(tid);
+    float den = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) den += __builtin_amdgcn_exp2f(mm[w * 16 + tid] - M) * ll[w * 16 + tid];
+    typedef unsigned u2 __attribute__((ext_vector_type(2)));
+    __builtin_amdgcn_raw_buffer_store_b64(u2{__float_as_uint(M), __float_as_uint(den)}, part, (sp * per + rep * Dv + 2 * tid) * 4, 0, SC1);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");           // written through: visible when acknowledged
+  __syncthreads();
+  int* word = p.words + (size_t)row * TICKET;
+  int* flag = reinterpret_cast<int*>(mm);                    // (mm, ll and aa have been read)
+  if (tid == 0) {
+    *flag = __hip_atomic_fetch_add(word, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == p.ns - 1;
+    if (*flag) __hip_atomic_store(word, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  if (!*flag) return;
+  // (maximum, sum) of every split and head
+  float* f = mm + 16;                                        // [rep][ns] factors, then [rep] 1 / sum
+  float* inv = f + rep * p.ns;
+  for (int i = tid; i < rep * p.ns; i += TH) {
+    const int r = i / p.ns, s = i - r * p.ns;
+    f[i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(part, (s * per + rep * Dv + 2 * r) * 4, 0, SC1));
+  }
+  __syncthreads();
+  if (tid < rep) {
+    float M = p.sink ? p.sink[g * rep + tid] * LOG2E : -1e30f;
+    for (int s = 0; s < p.ns; ++s) M = fmaxf(M, f[tid * p.ns + s]);
+    float den = p.sink ? __builtin_amdgcn_exp2f(p.sink[g * rep + tid] * LOG2E - M) : 0.f;
+    for (int s = 0; s < p.ns; ++s) {
+      const float a = __builtin_amdgcn_exp2f(f[tid * p.ns + s] - M);
+      f[tid * p.ns + s] = a;
+      den += a * __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(part, (s * per + rep * Dv + 2 * tid + 1) * 4, 0, SC1));
+    }
+    inv[tid] = den > 0.f ? 1.f / den : 0.f;
+  }
+  __syncthreads();
+  for (int q = tid; q < quads; q += TH) {
+    const int r = q * 4 / Dv, e = q * 4 - r * Dv, h = g * rep + r;
+    float4v num = {0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < p.ns; s0 += BATCH) {
+      float4v v[BATCH];
+#pragma unroll
+      for (int k = 0; k < BATCH; ++k)                        // past the last split: zeros from past the buffer, not summed up
+        v[k] = __builtin_bit_cast(float4v, __builtin_amdgcn_raw_buffer_load_b128(part, ((s0 + k) * per + q * 4) * 4, 0, SC1));
+#pragma unroll
+      for (int k = 0; k < BATCH; ++k)
+        if (s0 + k < p.ns) num += f[r * p.ns + s0 + k] * v[k];
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float out = num[i] * inv[r];
+      if (p.gate) out *= sigmoid_f(bf2f(((const bf16_t*)p.gate)[(size_t)t * p.gate_ld + (size_t)h * Dv + e + i]));
+      ((bf16_t*)p.o)[(size_t)t * p.o_ld + (size_t)h * Dv + e + i] = f2bf(out);
+    }
+  }
+}
 
 template <int DK, int DV, int WT_WAVES>
 __global__ __launch_bounds__(64 * WT_WAVES, 4) void window_attn_token_kernel(WinAttnParams p) {
@@ -172,9 +259,13 @@ __global__ __launch_bounds__(64 * WT_WAVES, 4) void window_attn_token_kernel(Win
     for (int d = 0; d < NDT; ++d)
       *reinterpret_cast<float4v*>(aa + ((size_t)wave * rep + c) * DV + 16 * d + 4 * q4) = acc[d];
   __syncthreads();
+  if (p.ns > 1) {
+    wt_join<WT_WAVES, DV>(p, mm, ll, aa, t, g, sp, rep);
+    return;
+  }
   for (int idx = threadIdx.x; idx < rep * Dv; idx += 64 * WT_WAVES) {
     const int r = idx / Dv, e = idx - r * Dv, h = g * rep + r;
-    const bool snk = p.sink && p.ns == 1;                    // with key splits the combine launch adds it
+    const bool snk = p.sink != nullptr;
     const float sk = snk ? p.sink[h] * LOG2E : -1e30f;
     float M = sk;
 #pragma unroll
@@ -186,24 +277,21 @@ __global__ __launch_bounds__(64 * WT_WAVES, 4) void window_attn_token_kernel(Win
       num += f * aa[((size_t)w * rep + r) * DV + e];
       den += f * ll[w * 16 + r];
     }
-    if (p.ns > 1) {                                          // the combine launch (natural units) finishes the row
-      float* pr = p.part + (((size_t)t * p.H + h) * p.ns + sp) * (Dv + 2);
-      if (e == 0) {
-        pr[0] = M / LOG2E;
-        pr[1] = den;
-      }
-      pr[2 + e] = num;
-      continue;
-    }
     float out = den > 0.f ? num / den : 0.f;
     if (p.gate) out *= sigmoid_f(bf2f(((const bf16_t*)p.gate)[(size_t)t * p.gate_ld + (size_t)h * Dv + e]));
     ((bf16_t*)p.o)[(size_t)t * p.o_ld + (size_t)h * Dv + e] = f2bf(out);
   }
 }
 
-// -1: not these sizes or places. The caller launches the combine for p.ns > 1.
+#define WT_SPLITS 64
+
+// -1: not these sizes or places
 int window_attention_token(const WinAttnParams& p, hipStream_t st) {
   const int rep = p.H / p.G;
+  if (p.ns > 1) {
+    if (p.ns > WT_SPLITS || !p.words || ((size_t)p.part & 15)) return -1;
+    if ((long)p.T * p.G > p.tickets || (long)p.T * p.G * p.ns * wt_part_floats(rep, p.Dv) > p.part_floats) return (int)hipErrorInvalidValue;
+  }
   if (p.D > 128 || p.Dv > 128 || p.D % 8 || p.Dv % 8 || rep > 16 || p.cache_rows > 0x7fffffffL ||
       (((size_t)p.q | (size_t)p.kc | (size_t)p.vc) & 15))
     return -1;
@@ -220,7 +308,7 @@ int window_attention_token(const WinAttnParams& p, hipStream_t st) {
   } while (0)
 #define GO(A, C)                                                                                        \
   do {                                                                                                  \
-    if (many) RUN(A, C, 4);                                                                             \
+    if (many || p.ns > 1) RUN(A, C, 4);                                                                             \
     RUN(A, C, 16);                                                                                      \
   } while (0)
   if (p.D <= 64) {

@@ -934,6 +934,23 @@ def window_token_takes(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Te
             and (q.data_ptr() | k_cache.data_ptr() | v_cache.data_ptr()) % 16 == 0)
 
 
+WT_SPLITS = 64      # splits of a row's keys that the matrix-core token form joins at most
+
+
+def window_token_splits(tiles: int, rows: int, D: int) -> int:
+    """Key splits of the matrix-core token form for ``tiles`` tiles of 32 keys at most and ``rows`` tokens times key heads. One
+    workgroup of 16 waves reads 0.5 MB for 1000 keys of 128, 8 us of what one compute unit gets; four waves a split, a tile
+    each, spread it over the chip and join in the launch for 2.5 us (us a launch whole and split, 8 tokens x 4 key heads of 128:
+    200 keys 7.9, 8.8; 400 9.9, 8.9; 1000 15.7, 8.9 in eight; 4000 26.9 by another launch, 18.9 in sixteen; 1 x 4 behind 4000
+    23.6, 11.9; 64 columns at 300 keys 6.3, 7.4). Up to 512 workgroups: 32 x 4 behind 2000 in a window of 1024 18.4, 18.1 in
+    four and 21.0 in sixteen; 32 x 8 of 64 behind 2000 31.3, 27.8 in two, 28.8 in sixteen."""
+    if tiles <= (12 if D > 64 else 16):
+        return 1
+    most = min(16, 512 // rows)
+    rounds = -(-tiles // (4 * most)) if most else 1
+    return max(1, min(most, -(-tiles // (4 * rounds))))
+
+
 def window_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
                      cu_q: torch.Tensor, ctx_lens: torch.Tensor, block_tables: torch.Tensor,
                      positions: torch.Tensor, scale: float, softcap: float, window: int,
@@ -952,8 +969,8 @@ def window_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
     keys through the block table, so prompt portions, decode tokens and mixed
     batches are one launch. Scores, softmax and accumulators are f32. A step
     with few rows over long contexts (``max_ctx``) deals each row's keys out to
-    ``key_splits`` workgroups (chosen here when None) and merges their partial
-    results in a second launch. ``sink`` f32 [H]: head h's softmax denominator
+    ``key_splits`` workgroups (chosen here when None) and joins their partial
+    results. ``sink`` f32 [H]: head h's softmax denominator
     also holds exp(sink[h]), a term that carries no value. ``slopes`` f32 [H]: a
     linear distance bias, slopes[h] * (p - j) comes off the (capped) score.
     ``out`` [T, H Dv]: where to write (may be a column slice of a wider row)."""
@@ -992,18 +1009,22 @@ def window_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
     part = None
     if key_splits is None:
         key_splits = 1
-        if not mfma and T * G < 256:
-            # 64-key windows a row can have, four (one per wave) to a workgroup; the matrix-core token
-            # form reads 512 keys a round, and up to 1152 two or three rounds cost less than splits and
-            # their merge
+        if not mfma and 0 < T * G <= 256:
             keys = max(int(max_ctx), 1) if window <= 0 else min(max(int(max_ctx), 1), window + 64 + keep_first)
-            once = 1152 if window_token_takes(q, k_cache, v_cache, H, G, D, Dv) else 256
-            key_splits = max(1, min(16, -(-keys // once), 512 // max(1, T * G)))
-    if key_splits > 1 and not mfma:
-        part = torch.empty(T * H * key_splits * (Dv + 2), dtype=torch.float32, device=q.device)
-    else:
-        key_splits = 1
+            if window_token_takes(q, k_cache, v_cache, H, G, D, Dv):
+                key_splits = window_token_splits(-(-keys // 32), T * G, D)
+            elif T * G < 256:
+                # 64-key windows a row can have, four (one per wave) to a workgroup
+                key_splits = max(1, min(16, -(-keys // 256), 512 // max(1, T * G)))
     call, extra, st = "loqa_window_attention", (), stream_ptr(q)
+    if mfma or key_splits <= 1:
+        key_splits = 1
+    elif key_splits <= WT_SPLITS and window_token_takes(q, k_cache, v_cache, H, G, D, Dv):
+        per = H // G * Dv + (2 * (H // G) + 3) // 4 * 4          # wt_part_floats
+        part, words = _sk_workspace(q.device, st, T * G * key_splits * per, T * G)
+        call, extra = "loqa_window_attention_parts", (1, part.numel(), ptr(words), words.numel())
+    else:
+        part = torch.empty(T * H * key_splits * (Dv + 2), dtype=torch.float32, device=q.device)
     if mfma and D <= 128 and not softcap and slopes is None and scale > 0:
         vparts, width = -(-Dv // 128), 64 if Dv <= 64 else 128
         keys = int(max_ctx or 0) if window <= 0 else min(int(max_ctx or 0), window + 64 + keep_first)

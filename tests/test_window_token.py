@@ -9,6 +9,7 @@ import math
 import pytest
 import torch
 
+from loqa_hub_amd import ops
 from loqa_hub_amd.ops import seqmix
 
 pytestmark = pytest.mark.gpu
@@ -144,3 +145,30 @@ def test_key_splits_of_the_other_form():
             got.append(at[0].elapsed_time(at[1]))
         return min(got)
     assert us(None) < 1.4 * us(12)
+
+
+@pytest.mark.parametrize("splits", [None, 2, 16, 64, 65])
+def test_splits_join_in_the_launch(splits):
+    # splits without keys, rows with fewer tiles than splits; more than 64 go to the other form
+    _check([1] * 4, [0, 40, 700, 2100], 8, 2, 128, 128, sink=True, gate=True, splits=splits, seed=3)
+    _check([1, 3], [2500, 90], 15, 3, 40, 120, 1000, 5, slopes=True, splits=splits, seed=4)
+    torch.cuda.synchronize()
+    assert all(int(words.as_strided((words.numel(), 32), (32, 1)).abs().sum()) == 0 for _, words in ops._SK_WS.values())
+
+
+def test_splits_repeat_bit_for_bit():
+    kc, vc = torch.randn(140, 16, 256, device=DEV).bfloat16(), torch.randn(140, 16, 256, device=DEV).bfloat16()
+    bt, cu = torch.arange(140, dtype=torch.int32, device=DEV)[None].contiguous(), torch.tensor([0, 1], dtype=torch.int32, device=DEV)
+    ctx, pos = torch.tensor([2200], dtype=torch.int32, device=DEV), torch.tensor([2199], dtype=torch.int32, device=DEV)
+    q = torch.randn(1, 1024, device=DEV).bfloat16()
+    run = lambda: seqmix.window_attention(q, kc, vc, cu, ctx, bt, pos, 0.09, 0.0, 0, 0, None, 8, 2, 128, 128, max_q=1, max_ctx=2200)
+    assert seqmix.window_token_splits(-(-2200 // 32), 2, 128) == 9
+    first = run()
+    assert all(torch.equal(run(), first) for _ in range(10))
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = run()
+    for _ in range(3):
+        y.zero_()
+        graph.replay()
+        assert torch.equal(y, first) and torch.equal(run(), first)
