@@ -1,13 +1,16 @@
 """Build the native HIP/C++ libraries in-tree for gfx950.
 
-Two shared objects are produced next to this file:
+Four shared objects are produced next to this file:
 
 * ``libloqa_kernels.so`` - every hand-written CDNA4 kernel under ``csrc/kernels``
-  (compiled with ``hipcc --offload-arch=gfx950``).
+  (compiled with ``hipcc --offload-arch=gfx950``) but the sequence mixers'.
+* ``libloqa_seqmix.so`` - the sequence-mixer kernels.
 * ``libloqa_runtime.so`` - the host runtime under ``csrc/runtime`` (pinned PCM
   staging, paged-KV block pool).
+* ``libloqa_launch.so`` - a Python module, ``csrc/launch``: entry points of token
+  steps that take tensors as they are.
 
-They are loaded with ctypes *after* ``import torch`` so the process shares
+The first three are loaded with ctypes *after* ``import torch`` so the process shares
 torch's single HIP runtime (both link ``libamdhip64.so.7``).
 
 Usage: ``python -m loqa_hub_amd._native.build [--force] [--debug]``.
@@ -17,10 +20,12 @@ from __future__ import annotations
 import argparse
 import glob
 import hashlib
+import importlib.util
 import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -95,6 +100,32 @@ SEQMIX_SOURCES = ("norm_dyt.hip", "attn_latent.hip", "attn_latent_prefill.hip", 
 NO_PACKED_F32 = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 
 
+def _build_launch(force: bool, opt: list[str]) -> str:
+    """The Python module, host code only: a plain C++ compiler against torch's headers."""
+    torch_dir = importlib.util.find_spec("torch").submodule_search_locations[0]
+    with open(os.path.join(torch_dir, "version.py")) as f:
+        version = hashlib.sha256(f.read().encode()).hexdigest()
+    src, out = os.path.join(CSRC, "launch", "launch.cpp"), os.path.join(HERE, "libloqa_launch.so")
+    flags = [*opt, "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D_GLIBCXX_USE_CXX11_ABI=1",
+             f"-I{os.path.join(torch_dir, 'include')}", f"-I{sysconfig.get_paths()['include']}"]
+    digest, stamp = _digest([src], [*flags, version]), out + ".sha256"
+    if not force and os.path.exists(out) and os.path.exists(stamp):
+        with open(stamp) as f:
+            if f.read().strip() == digest:
+                return out
+    cxx = [shutil.which("g++") or shutil.which("c++")]
+    if cxx[0] is None:
+        cxx = [_hipcc(), "-x", "c++"]
+    cmd = [*cxx, *flags, src, "-o", out + ".tmp", f"-L{os.path.join(torch_dir, 'lib')}", "-ltorch_python", "-ltorch_cpu", "-lc10"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"compile failed: {' '.join(cmd)}\n{r.stdout}\n{r.stderr}")
+    os.replace(out + ".tmp", out)
+    with open(stamp, "w") as f:
+        f.write(digest)
+    return out
+
+
 def build(force: bool = False, debug: bool = False, only=None, quiet: bool = False) -> list[str]:
     """Build the native libraries (all, or the names in ``only``) in-tree."""
     opt = ["-O0", "-g"] if debug else ["-O3"]
@@ -116,6 +147,8 @@ def build(force: bool = False, debug: bool = False, only=None, quiet: bool = Fal
     for name, src, hdr, flags in libs:
         if only is None or name in only:
             out.append(_build_lib(name, src, hdr, flags, force))
+    if only is None or "libloqa_launch.so" in only:
+        out.append(_build_launch(force, ["-O0", "-g"] if debug else ["-O2"]))
     return out
 
 

@@ -8,6 +8,8 @@ back to PyTorch.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 import threading
 
@@ -332,13 +334,44 @@ def _main_kernels() -> ctypes.CDLL:
     return _kernels
 
 
+# Entry points of token steps, which ``libloqa_launch.so`` calls without ctypes; their pointer arguments are
+# tensors, addresses or None. i32c and f32c check (tensor, name) pairs, the others the tensors of a launch.
+_LAUNCH = frozenset(("loqa_qk_prep_append", "loqa_window_attention", "loqa_window_attention_parts", "loqa_delta_prep",
+                     "loqa_delta_scan", "loqa_seq_state_save", "loqa_gated_rmsnorm", "loqa_moe_route", "i32c", "f32c",
+                     "qk_shapes", "window_shapes"))
+_launch = None
+
+
+def launch():
+    """The Python module of those entry points, with the types that this file has."""
+    global _launch
+    if _launch is None:
+        seqmix()                                  # its symbols
+        with _lock:
+            if _launch is None:
+                path = os.path.join(_NATIVE, "libloqa_launch.so")
+                if not os.path.exists(path):
+                    raise NativeLibraryMissing(f"{path} is missing: run `python -m loqa_hub_amd._native.build` (gfx950)")
+                loader = importlib.machinery.ExtensionFileLoader("libloqa_launch", path)
+                mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("libloqa_launch", loader))
+                loader.exec_module(mod)
+                code = {_vp: "p", _i: "i", _l: "l", _f: "f"}
+                for fn, sig in mod.signatures().items():
+                    if sig != "".join(code[t] for t in _SEQMIX_SIGS[fn]):
+                        raise RuntimeError(f"{fn}: libloqa_launch.so was built for other arguments")
+                _launch = mod
+    return _launch
+
+
 class _Kernels:
     """Attribute lookup over the kernel libraries: the sequence-mixer entry
     points live in ``libloqa_seqmix.so``, everything else in
     ``libloqa_kernels.so`` (loaded only when one of its kernels is called)."""
 
     def __getattr__(self, name: str):
-        if name in _SEQMIX_SIGS or name == "loqa_delta_chunks_ws":
+        if name in _LAUNCH:
+            fn = getattr(launch(), name)
+        elif name in _SEQMIX_SIGS or name == "loqa_delta_chunks_ws":
             fn = getattr(seqmix(), name)
         else:
             fn = getattr(_main_kernels(), name)
@@ -380,6 +413,7 @@ def load_all() -> None:
     """Load every native library (a missing one raises)."""
     _main_kernels()
     seqmix()
+    launch()
     runtime()
 
 

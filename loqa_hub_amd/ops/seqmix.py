@@ -510,8 +510,8 @@ def gated_rmsnorm(o: torch.Tensor, w: torch.Tensor, gate: torch.Tensor, eps: flo
     assert groups >= 1 and n % groups == 0
     y = torch.empty(T, n, dtype=out_dtype, device=o.device)
     if T:
-        check(kernels().loqa_gated_rmsnorm(ptr(o), ptr(w), ptr(gate), _dt(gate), gate.stride(0), eps,
-                                           ptr(y), _dt(y), T, n, groups,
+        check(kernels().loqa_gated_rmsnorm(o, w, gate, _dt(gate), gate.stride(0), eps,
+                                           y, _dt(y), T, n, groups,
                                            1 if silu_first else (2 if gate_act == "silu" else 0),
                                            stream_ptr(o)), "gated_rmsnorm")
     return y
@@ -566,11 +566,11 @@ def moe_route(z: torch.Tensor, correction: torch.Tensor | None, n_groups: int, k
     idx = torch.empty(T, top, dtype=torch.int32, device=z.device)
     wt = torch.empty(T, top, dtype=torch.float32, device=z.device)
     if T:
-        check(kernels().loqa_moe_route(ptr(z), ptr(correction), ptr(bias),
+        check(kernels().loqa_moe_route(z, correction, bias,
                                        1 if top_softmax else (2 if sigmoid else 0), E,
                                        max(1, n_groups), min(keep, max(1, n_groups)),
                                        max(1, group_rank), top, int(renorm), float(weight_scale),
-                                       ptr(idx), ptr(wt), T,
+                                       idx, wt, T,
                                        stream_ptr(z)), "moe_route")
     return idx, wt
 
@@ -673,9 +673,9 @@ def seq_state_save(x: torch.Tensor | None, u: torch.Tensor, prev: torch.Tensor |
         assert prev.shape == (tail.shape[0], d) and x.shape[0] == T
     B = _seq_args(state_slots, cu_q, positions, T)
     if T:
-        check(kernels().loqa_seq_state_save(ptr(x), d, ptr(u), _dt(u), u.stride(0), ptr(prev),
-                                            ptr(tail), tail.shape[0], keep, C, ptr(state_slots),
-                                            ptr(cu_q), ptr(positions), B, stream_ptr(u)),
+        check(kernels().loqa_seq_state_save(x, d, u, _dt(u), u.stride(0), prev,
+                                            tail, tail.shape[0], keep, C, state_slots,
+                                            cu_q, positions, B, stream_ptr(u)),
               "seq_state_save")
 
 
@@ -892,26 +892,17 @@ def qk_prep_append(u: torch.Tensor, H: int, G: int, D: int, Dv: int, v_off: int,
         assert vf.dtype == u.dtype
     if side is not None:
         assert side.src.shape[0] == u.shape[0] and side.src.dtype == u.dtype
-    T, W = u.shape
-    assert u.stride(1) == 1 and (H + G) * D <= W
-    assert v_off < 0 and Dv == D or v_off >= (H + G) * D and v_off + G * Dv <= W
-    assert dims % 2 == 0 and 0 <= dims <= D
-    if dims:
-        _f32c(cos_sin, "cos_sin")
-        assert cos_sin.shape[1] * 2 == dims
-    assert k_cache.is_contiguous() and v_cache.is_contiguous()
-    assert k_cache.dtype == v_cache.dtype == out_dtype == u.dtype
-    assert k_cache.shape[2] == G * D and v_cache.shape == (*k_cache.shape[:2], G * Dv)
-    _i32c(positions, "positions"); _i32c(slots, "slots")
-    assert positions.numel() >= T and slots.numel() >= T
+    lib = kernels()
+    T, ld, pages, blk, rows = lib.qk_shapes(u, k_cache, v_cache, positions, slots, cos_sin, H, G, D, Dv, v_off, dims)
+    assert out_dtype == u.dtype
     coef, every = (float(q_temp[0]), int(q_temp[1])) if q_temp is not None else (0.0, 1)
-    q = torch.empty(T, H * D, dtype=out_dtype, device=u.device)
+    q = u.new_empty((T, H * D))
     if T:
-        check(kernels().loqa_qk_prep_append(
-            ptr(u), _dt(u), u.stride(0), H, G, D, Dv, int(v_off), ptr(cos_sin) if dims else None,
-            cos_sin.shape[0] if dims else 0, dims, float(eps), coef, every, ptr(positions),
-            ptr(k_cache), ptr(v_cache), k_cache.shape[1], k_cache.shape[0], ptr(slots), ptr(q), T,
-            ptr(q_norm), ptr(k_norm), mode, ptr(vf), vf.stride(0) if vf is not None else 0,
+        check(lib.loqa_qk_prep_append(
+            u, _dt(u), ld, H, G, D, Dv, int(v_off), cos_sin if dims else None,
+            rows, dims, float(eps), coef, every, positions,
+            k_cache, v_cache, blk, pages, slots, q, T,
+            q_norm, k_norm, mode, vf, vf.stride(0) if vf is not None else 0,
             float(lam), *(side.args() if side is not None else _NO_SIDE), stream_ptr(u)),
             "qk_prep_append")
     return q
@@ -922,16 +913,6 @@ def window_mfma_sizes(D: int, Dv: int) -> bool:
     for 64 / 128 and shared out over workgroups above; multiples of 8 in between are
     padded with zeros in LDS)."""
     return D % 8 == 0 and 0 < D <= 256 and Dv % 8 == 0 and 0 < Dv <= 512
-
-
-def window_token_takes(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, H: int, G: int,
-                       D: int, Dv: int) -> bool:
-    """Whether token steps run in the matrix-core form (``csrc/kernels/attn_window_token.hip``, whose
-    rule this is): bf16, heads up to 128 in multiples of 8, up to 16 query heads a key head, rows
-    that start on 16 bytes."""
-    return (q.dtype == torch.bfloat16 and D <= 128 and Dv <= 128 and D % 8 == 0 and Dv % 8 == 0
-            and H // G <= 16 and k_cache.shape[0] * k_cache.shape[1] < 1 << 31
-            and (q.data_ptr() | k_cache.data_ptr() | v_cache.data_ptr()) % 16 == 0)
 
 
 WT_SPLITS = 64      # splits of a row's keys that the matrix-core token form joins at most
@@ -979,27 +960,20 @@ def window_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
                                  scale, softcap, window, keep_first, gate, H, G, D, Dv, q.dtype,
                                  sink, slopes)
         return o if out is None else out.copy_(o)
+    lib = kernels()
     if slopes is not None:
-        _f32c(slopes, "slopes")
+        lib.f32c(slopes, "slopes")
         assert slopes.numel() == H
     if sink is not None:
-        _f32c(sink, "sink")
+        lib.f32c(sink, "sink")
         assert sink.numel() == H
-    T = q.shape[0]
-    assert q.is_contiguous() and q.shape[1] == H * D and H % G == 0
-    assert k_cache.is_contiguous() and v_cache.is_contiguous()
-    assert k_cache.shape[2] == G * D and k_cache.dtype == v_cache.dtype == q.dtype
-    assert v_cache.shape == (*k_cache.shape[:2], G * Dv)
-    assert D <= 512 and Dv <= 512 and window >= 0 and keep_first >= 0 and softcap >= 0
-    _i32c(cu_q, "cu_q"); _i32c(ctx_lens, "ctx_lens"); _i32c(block_tables, "block_tables")
-    _i32c(positions, "positions")
-    B = ctx_lens.numel()
-    assert cu_q.numel() == B + 1 and block_tables.shape[0] == B and positions.numel() >= T
+    T, pages, blk, B, max_blocks, token = lib.window_shapes(q, k_cache, v_cache, cu_q, ctx_lens, block_tables, positions, H, G, D, Dv)
+    assert window >= 0 and keep_first >= 0 and softcap >= 0
     gs = 0
     if gate is not None:
         assert gate.shape == (T, H * Dv) and gate.stride(1) == 1 and gate.dtype == q.dtype
         gs = gate.stride(0)
-    o = torch.empty(T, H * Dv, dtype=q.dtype, device=q.device) if out is None else out
+    o = q.new_empty((T, H * Dv)) if out is None else out
     assert o.shape == (T, H * Dv) and o.stride(1) == 1 and o.dtype == q.dtype
     if matrix_cores is None:         # heads far below the built sizes would be mostly padding
         matrix_cores = max_q >= 16 and D >= 32 and Dv >= 32
@@ -1011,7 +985,7 @@ def window_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
         key_splits = 1
         if not mfma and 0 < T * G <= 256:
             keys = max(int(max_ctx), 1) if window <= 0 else min(max(int(max_ctx), 1), window + 64 + keep_first)
-            if window_token_takes(q, k_cache, v_cache, H, G, D, Dv):
+            if token:
                 key_splits = window_token_splits(-(-keys // 32), T * G, D)
             elif T * G < 256:
                 # 64-key windows a row can have, four (one per wave) to a workgroup
@@ -1019,10 +993,10 @@ def window_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
     call, extra, st = "loqa_window_attention", (), stream_ptr(q)
     if mfma or key_splits <= 1:
         key_splits = 1
-    elif key_splits <= WT_SPLITS and window_token_takes(q, k_cache, v_cache, H, G, D, Dv):
+    elif key_splits <= WT_SPLITS and token:
         per = H // G * Dv + (2 * (H // G) + 3) // 4 * 4          # wt_part_floats
         part, words = _sk_workspace(q.device, st, T * G * key_splits * per, T * G)
-        call, extra = "loqa_window_attention_parts", (1, part.numel(), ptr(words), words.numel())
+        call, extra = "loqa_window_attention_parts", (1, part.numel(), words, words.numel())
     else:
         part = torch.empty(T * H * key_splits * (Dv + 2), dtype=torch.float32, device=q.device)
     if mfma and D <= 128 and not softcap and slopes is None and scale > 0:
@@ -1032,14 +1006,13 @@ def window_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
         if parts > 1:       # a wave's 32 rows: width / 2 accumulators a lane, maximum and sum
             blocks = -(-max_q // 64) * H * vparts * B
             part, words = _sk_workspace(q.device, st, blocks * parts * 2 * (width // 2 + 4) * 64, blocks)
-            call, extra = "loqa_window_attention_parts", (parts, part.numel(), ptr(words), words.numel())
+            call, extra = "loqa_window_attention_parts", (parts, part.numel(), words, words.numel())
     if T:
-        check(getattr(kernels(), call)(
-            ptr(q), _dt(q), ptr(k_cache), ptr(v_cache), k_cache.shape[1], k_cache.shape[0],
-            ptr(cu_q), ptr(ctx_lens), ptr(block_tables), block_tables.shape[1], ptr(positions),
-            ptr(gate), gs, float(scale), float(softcap), int(window), int(keep_first), B, T, H, G,
-            D, Dv, int(max_q), int(mfma), ptr(o), o.stride(0), int(key_splits), ptr(part), ptr(sink),
-            ptr(slopes), *extra, st), "window_attention")
+        check(getattr(lib, call)(
+            q, _dt(q), k_cache, v_cache, blk, pages, cu_q, ctx_lens, block_tables, max_blocks, positions,
+            gate, gs, float(scale), float(softcap), int(window), int(keep_first), B, T, H, G,
+            D, Dv, int(max_q), int(mfma), o, o.stride(0), int(key_splits), part, sink,
+            slopes, *extra, st), "window_attention")
     return o
 
 
@@ -1279,10 +1252,10 @@ def delta_prep(u: torch.Tensor, gz: torch.Tensor, G: int, D: int, H: int, Dv: in
     tok = torch.empty(T, H, 2, dtype=torch.float32, device=u.device)
     if T:
         check(kernels().loqa_delta_prep(
-            ptr(u), _dt(u), u.stride(0), ptr(gz), ptr(za), za.stride(0) if za is not None else 0,
-            b_off, G, D, H, Dv, ptr(conv_w), taps, ptr(tail),
-            tail.shape[0], ptr(a_neg), ptr(dt_bias), ptr(state_slots), ptr(cu_q), ptr(positions), B,
-            T, ptr(act), ptr(tok), stream_ptr(u)), "delta_prep")
+            u, _dt(u), u.stride(0), gz, za, za.stride(0) if za is not None else 0,
+            b_off, G, D, H, Dv, conv_w, taps, tail,
+            tail.shape[0], a_neg, dt_bias, state_slots, cu_q, positions, B,
+            T, act, tok, stream_ptr(u)), "delta_prep")
     return act, tok
 
 
@@ -1327,10 +1300,10 @@ def delta_scan(act: torch.Tensor, H: int, D: int, Dv: int, q_off: int, k_off: in
                                   stream_ptr(act)), "delta_chunks")
         return o
     if T:
-        check(kernels().loqa_delta_scan(ptr(act), W, H, D, Dv, q_off, k_off, v_off,
-                                        -1 if g_off is None else g_off, hpg, ptr(state),
-                                        state.shape[0], ptr(state_slots), ptr(cu_q), ptr(positions),
-                                        ptr(tok), ptr(o), B, T, stream_ptr(act)), "delta_scan")
+        check(kernels().loqa_delta_scan(act, W, H, D, Dv, q_off, k_off, v_off,
+                                        -1 if g_off is None else g_off, hpg, state,
+                                        state.shape[0], state_slots, cu_q, positions,
+                                        tok, o, B, T, stream_ptr(act)), "delta_scan")
     return o
 
 
