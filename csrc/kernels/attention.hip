@@ -321,6 +321,11 @@ __global__ __launch_bounds__(64 * QW * KS, D == 64 && QW * KS == 4 ? 3 : 2) void
   }
   const int per = (ntiles + KS - 1) / KS;                   // tiles of a run; the last may have fewer
   const int first = t0 + run * per;
+  // run 0 has the only tile: the others leave before they fetch and mask a copy of it, and nothing is merged (1500 rows behind
+  // 64 keys: 8 heads of 64 5.7 -> 4.4 us, 20 heads 6.5 -> 5.0; 64 rows x 32 heads with the merge 6.6, without 6.0). A barrier
+  // waits for the waves that are left.
+  const bool alone = KS > 1 && !PARTS && ntiles <= 1;
+  if (alone && run) return;
 
   const FlFetch<D, NTH, false, false> kf(th, D, PAGED ? D : p.kv_stride);
   const FlFetch<D, NTH, true, false> vf(th, D, PAGED ? D : p.kv_stride);
@@ -378,7 +383,10 @@ __global__ __launch_bounds__(64 * QW * KS, D == 64 && QW * KS == 4 ? 3 : 2) void
     for (int j = 0; j < 16; ++j) acc[i][j] = 0.f;
   float m = -1e30f, l = 0.f;
   fl_loop<D, D, kf.N + vf.N>(
-      qf, acc, m, l, ring, per, p.scale_log2, lane, true, QW * KS == 8 ? wave >> 2 : -1,
+      qf, acc, m, l, ring, per, p.scale_log2, lane, true,
+      // half a tile apart costs 64-column heads on two runs 1 to 3 % (1500 rows x 20 heads 20.1 -> 20.5, behind 512 keys 10.0 -> 10.4),
+      // and a single tile has no other to run beside
+      QW * KS == 8 && (KS == 4 || D == 128) && per > 1 ? wave >> 2 : -1,
       [&](float16v(&st)[2], int i) __attribute__((always_inline)) {
         // masking only where a key can be invalid for this wave (wave-uniform test)
         const int kt = (first + i) * FL_KEYS;
@@ -403,8 +411,7 @@ __global__ __launch_bounds__(64 * QW * KS, D == 64 && QW * KS == 4 ? 3 : 2) void
     fl_store<NDT, QW, KS, ALL>(own, lds, p.o + (size_t)(q0 + row_lo + wq * 32) * p.o_stride + (size_t)head * D, p.o_stride,
                                qlen - row_lo - wq * 32, D, run, wq, lane);
   };
-  if (KS == 4 && !PARTS && ntiles <= 1) {                   // only run 0 has one (64 rows and keys x 32 heads of 64: 6.6 -> 6.0 us)
-    if (run) return;
+  if (alone) {
     float4v own[4 * NDT];
     fl_units(acc, own);
     finish(Fl<1>{}, own);

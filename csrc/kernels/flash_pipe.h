@@ -215,7 +215,7 @@ __device__ __forceinline__ float fl_both32(float x) {  // lane + lane ^ 32
 // phase: -1, or in workgroups of eight waves 0 for the first four and 1 for the others, which share the four SIMDs: each
 // half of a tile then begins with a barrier of all waves, and the second four run half a tile behind, their exponentials,
 // maxima and rescaling beside the scores' MFMAs of the first (in step, both waves of a SIMD want the same unit; 2048 rows of
-// 16 latent heads of 192 / 128 43.7 -> 41.6 us, of 32 58.5 -> 56.7, 1500 rows x 8 heads of 64 13.7 -> 12.9; wave priorities
+// 16 latent heads of 192 / 128 43.7 -> 41.6 us, of 32 58.5 -> 56.7, 1500 rows x 8 heads of 64 on four runs 13.7 -> 12.9; wave priorities
 // and six or eight fragments in flight beside it: the same within 1 %).
 // Before the call m = -1e30, l = 0, acc = 0; ring must not be in use. After it the waves
 // are not synchronised.

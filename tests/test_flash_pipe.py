@@ -172,3 +172,12 @@ def test_parts_of_the_keys(D, qlens, klens, Hq, page):
 def test_when_keys_are_in_parts():
     assert [ops.attn_parts(*x) for x in ((64, 32, 1024), (64, 32, 1023), (64, 64, 4000), (200, 32, 4000), (257, 32, 4000), (1, 1, 1024), (0, 8, 4000))] == \
         [8, 1, 4, 2, 1, 8, 1]
+
+
+@pytest.mark.parametrize("n,H,D", [(40, 4, 64), (200, 20, 64), (1500, 20, 64), (40, 4, 128), (1100, 32, 128)])
+def test_one_tile_on_every_block_height(n, H, D):
+    # all rows see one tile of keys: the runs without one have left (64 rows on four and two runs, 128 rows on two)
+    for m in (1, 33, 64):
+        _check([n, 1, 33], [m, 64, 1], H, H // 4, D, False, seed=m)
+        _check([m, 1], [m, 64], H, H // 4, D, True, page=16, seed=m)
+    _check([n, 70], [64, 65], H, H // 4, D, False, seed=3)          # one tile beside two
