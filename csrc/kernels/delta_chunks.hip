@@ -38,10 +38,13 @@
 
 #define DC_C 16
 
+typedef unsigned dc_u4 __attribute__((ext_vector_type(4)));
+
 struct DcParams {
   const float* act; long ld; int H, D, Dv, q_off, k_off, v_off, g_off, hpg;
   float* state; const int* slots; const int* cu_q; const int* pos; const float* tok;
   float* ws; float* o; int B;
+  bool runs;                                                // rows of q, k and decays come in 16-byte pieces
 };
 
 // Workspace of one (chunk, head), DP the padded key size: W and P q in the order of the MFMA
@@ -64,33 +67,84 @@ __device__ __forceinline__ float dc_sum16(float v) {
   return v;
 }
 
-// NT: key channels in units of 64 (DP = 64 NT)
-template <int NT, bool CHAN>
-__global__ __launch_bounds__(256) void delta_local_kernel(DcParams p) {
-  constexpr int DP = 64 * NT, LD = DP + 4;
-  __shared__ __attribute__((aligned(16))) float ks[DC_C][LD], qs[DC_C][LD], gs[DC_C][LD];
-  __shared__ __attribute__((aligned(16))) float A[DC_C][DC_C];
-  __shared__ float bs[DC_C];
-  int b, t0, n;
-  if (!seq_chunk<DC_C>(p.cu_q, p.B, blockIdx.x, b, t0, n)) return;
-  const int h = blockIdx.y, tid = threadIdx.x, D = p.D, Dv = p.Dv;
-  float* ws = p.ws + ((size_t)blockIdx.x * p.H + h) * dc_stride(DP, Dv);
+// What a workgroup that forms a chunk's block keeps in LDS (NT: key channels in units of 64, DP = 64 NT). A wave's
+// stage is 64 columns of 16 tokens, a thread's four pieces of 16 bytes at 4 l + (piece ^ l / 4 % 4), so that neither
+// the writes by columns nor the reads in order meet in a bank.
+template <int NT> struct DcLocal {
+  static constexpr int LD = 64 * NT + 4;
+  float ks[DC_C][LD];
+  union {
+    struct { float qs[DC_C][LD], gs[DC_C][LD]; };
+    float stage[4][64 * DC_C];                              // key columns: once qs is read (DP / 64 waves), values: gs as well
+  };
+  float A[DC_C][DC_C], B[DC_C][DC_C];
+  float bs[DC_C];
+};
+
+// The block of head h's chunk of tokens t0 .. t0 + n - 1, by 256 threads. All of it is written in whole 64-byte runs.
+// AUX: of the stores (16: through the caches). What bounds it is memory (2048 tokens, 16 heads of 128 x 128, a decay per
+// channel: 67 MB of rows read, 70 written; 26 us at a large copy's rate), so the waves in flight: with the triangle's
+// A in registers ahead of the substitution (166 a thread, three workgroups a CU), rows in 4-byte loads and columns stored
+// in 16-byte pieces 64 bytes apart it took 39 us, with 55 registers, five workgroups and whole runs 30.
+template <int NT, bool CHAN, int AUX>
+__device__ __forceinline__ void delta_local(const DcParams& p, DcLocal<NT>& s, float* ws, int t0, int n, int h, int tid) {
+  constexpr int DP = 64 * NT;
+  const int D = p.D, Dv = p.Dv, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const float* base = p.act + (size_t)t0 * p.ld;
+  const __amdgpu_buffer_rsrc_t block = __builtin_amdgcn_make_buffer_rsrc(ws, 0, (int)(dc_stride(DP, Dv) * 4), 0x00020000);
+  auto put = [&](int at, const float* v) {                  // four floats to entry at
+    __builtin_amdgcn_raw_buffer_store_b128(dc_u4{__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])},
+                                           block, at * 4, 0, AUX);
+  };
+  // a thread's 16 numbers of column c0 + lane, as [column][16] from entry `to` on, of `cols` columns
+  auto put_columns = [&](int to, int c0, int cols, const float (&x)[DC_C]) {
+    float* st = s.stage[wave];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) st_run<float, 4>(st + 16 * lane + 4 * (k ^ (lane >> 2 & 3)), x + 4 * k);
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int l = 16 * k + (lane >> 2);
+      float w[4];
+      ld_run<float, 4>(st + 16 * l + 4 * ((lane ^ l >> 2) & 3), w);
+      if (c0 + l < cols) put(to + (c0 + l) * DC_C + 4 * (lane & 3), w);
+    }
+    __builtin_amdgcn_wave_barrier();
+  };
   {
     const float* qr = base + p.q_off + (size_t)(h / p.hpg) * D;
     const float* kr = base + p.k_off + (size_t)(h / p.hpg) * D;
     const float* gr = CHAN ? base + p.g_off + (size_t)h * D : nullptr;
     const float* tr = p.tok + ((size_t)t0 * p.H + h) * 2;
+    if (p.runs) {                                           // whole rows of 16-byte pieces
 #pragma unroll
-    for (int j = 0; j < DC_C * DP / 256; ++j) {
-      const int i = (tid + 256 * j) / DP, d = (tid + 256 * j) % DP;
-      const bool ok = i < n && d < D;
-      const size_t row = (size_t)(i < n ? i : 0) * p.ld;
-      qs[i][d] = ok ? qr[row + d] : 0.f;
-      ks[i][d] = ok ? kr[row + d] : 0.f;
-      gs[i][d] = ok ? (CHAN ? gr[row + d] : tr[(size_t)i * p.H * 2]) : 1.f;
+      for (int j = 0; j < NT; ++j) {
+        const int i = (tid + 256 * j) / (16 * NT), d = (tid + 256 * j) % (16 * NT) * 4;
+        const size_t row = (size_t)(i < n ? i : 0) * p.ld;
+        const bool ok = i < n && d < D;
+        float q[4] = {0.f, 0.f, 0.f, 0.f}, k[4] = {0.f, 0.f, 0.f, 0.f}, g[4] = {1.f, 1.f, 1.f, 1.f};
+        if (ok) {
+          ld_run<float, 4>(qr + row + d, q);
+          ld_run<float, 4>(kr + row + d, k);
+          if constexpr (CHAN) ld_run<float, 4>(gr + row + d, g);
+          else g[0] = g[1] = g[2] = g[3] = tr[(size_t)i * p.H * 2];
+        }
+        st_run<float, 4>(&s.qs[i][d], q);
+        st_run<float, 4>(&s.ks[i][d], k);
+        st_run<float, 4>(&s.gs[i][d], g);
+      }
+    } else {
+#pragma unroll 4
+      for (int j = 0; j < DC_C * DP / 256; ++j) {
+        const int i = (tid + 256 * j) / DP, d = (tid + 256 * j) % DP;
+        const bool ok = i < n && d < D;
+        const size_t row = (size_t)(i < n ? i : 0) * p.ld;
+        s.qs[i][d] = ok ? qr[row + d] : 0.f;
+        s.ks[i][d] = ok ? kr[row + d] : 0.f;
+        s.gs[i][d] = ok ? (CHAN ? gr[row + d] : tr[(size_t)i * p.H * 2]) : 1.f;
+      }
     }
-    if (tid < DC_C) bs[tid] = tid < n ? tr[(size_t)tid * p.H * 2 + 1] : 0.f;
+    if (tid < DC_C) s.bs[tid] = tid < n ? tr[(size_t)tid * p.H * 2 + 1] : 0.f;
   }
   __syncthreads();
   // A and B: row i on 16 lanes, lane q with the channels 64 m + 4 q ..
@@ -98,10 +152,9 @@ __global__ __launch_bounds__(256) void delta_local_kernel(DcParams p) {
   float a[NT][4], c[NT][4];
 #pragma unroll
   for (int m = 0; m < NT; ++m) {
-    ld_run<float, 4>(&ks[i][64 * m + 4 * q], a[m]);
-    ld_run<float, 4>(&qs[i][64 * m + 4 * q], c[m]);
+    ld_run<float, 4>(&s.ks[i][64 * m + 4 * q], a[m]);
+    ld_run<float, 4>(&s.qs[i][64 * m + 4 * q], c[m]);
   }
-  float* Bw = ws + 49 * DP + 16 * Dv;
 #pragma unroll 4
   for (int j = DC_C - 1; j >= 0; --j) {
     float sa = 0.f, sb = 0.f;
@@ -109,8 +162,8 @@ __global__ __launch_bounds__(256) void delta_local_kernel(DcParams p) {
 #pragma unroll
       for (int m = 0; m < NT; ++m) {
         float k[4], g[4];
-        ld_run<float, 4>(&ks[j][64 * m + 4 * q], k);
-        ld_run<float, 4>(&gs[j][64 * m + 4 * q], g);
+        ld_run<float, 4>(&s.ks[j][64 * m + 4 * q], k);
+        ld_run<float, 4>(&s.gs[j][64 * m + 4 * q], g);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           sa += a[m][e] * k[e];
@@ -123,52 +176,55 @@ __global__ __launch_bounds__(256) void delta_local_kernel(DcParams p) {
     sa = dc_sum16(sa);
     sb = dc_sum16(sb);
     if (q == 0) {
-      A[i][j] = j < i ? sa : 0.f;
-      Bw[i * DC_C + j] = j <= i ? sb : 0.f;
+      s.A[i][j] = j < i ? sa : 0.f;
+      s.B[i][j] = j <= i ? sb : 0.f;
     }
   }
   // a = P(i) k_i, c = P(i) q_i now
 #pragma unroll
-  for (int m = 0; m < NT; ++m)
-    st_run<float, 4>(ws + 16 * DP + (4 * m + q / 4) * 256 + (16 * (q % 4) + i) * 4, c[m]);
+  for (int m = 0; m < NT; ++m) put(16 * DP + (4 * m + q / 4) * 256 + (16 * (q % 4) + i) * 4, c[m]);
+  __syncthreads();
   // P(16, j) k_j and P(16), a thread per channel
-  for (int d = tid; d < DP; d += 256) {
+  if (wave < NT) {
     float r = 1.f, kk[DC_C];
 #pragma unroll
     for (int j = DC_C - 1; j >= 0; --j) {
-      kk[j] = ks[j][d] * r;
-      r *= gs[j][d];
+      kk[j] = s.ks[j][tid] * r;
+      r *= s.gs[j][tid];
     }
-#pragma unroll
-    for (int j = 0; j < DC_C; j += 4) st_run<float, 4>(ws + 32 * DP + (size_t)d * DC_C + j, kk + j);
-    ws[48 * DP + d] = r;
+    put_columns(32 * DP, 64 * wave, DP, kk);
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(r), block, (48 * DP + tid) * 4, 0, AUX);
   }
   __syncthreads();
 #pragma unroll
-  for (int m = 0; m < NT; ++m) st_run<float, 4>(&ks[i][64 * m + 4 * q], a[m]);
+  for (int m = 0; m < NT; ++m) st_run<float, 4>(&s.ks[i][64 * m + 4 * q], a[m]);
+  if (wave == 3) {
+    float w[4];
+    ld_run<float, 4>(&s.B[0][0] + 4 * lane, w);
+    put(49 * DP + 16 * Dv + 4 * lane, w);
+  }
   __syncthreads();
   // forward substitution, a thread per column of [P k | v]
-  for (int col = tid; col < DP + Dv; col += 256) {
+  for (int c0 = 64 * wave; c0 < DP + Dv; c0 += 256) {
+    const int col = c0 + lane;
+    const bool key = c0 < DP;
     float x[DC_C];
-    const bool key = col < DP;
-    const float* vr = base + p.v_off + (size_t)h * Dv + (key ? 0 : col - DP);
+    const float* vr = base + p.v_off + (size_t)h * Dv + min(max(col - DP, 0), Dv - 1);
 #pragma unroll
     for (int t = 0; t < DC_C; ++t)
-      x[t] = key ? ks[t][col] : (t < n ? vr[(size_t)t * p.ld] : 0.f);
+      x[t] = key ? s.ks[t][col] : (t < n ? vr[(size_t)t * p.ld] : 0.f);
 #pragma unroll
     for (int t = 0; t < DC_C; ++t) {
-      float s = x[t];
+      float y = x[t];
 #pragma unroll
-      for (int j = 0; j < t; ++j) s -= A[t][j] * x[j];
-      x[t] = bs[t] * s;
+      for (int j = 0; j < t; ++j) y -= s.A[t][j] * x[j];
+      x[t] = s.bs[t] * y;
     }
     if (key) {
 #pragma unroll
-      for (int t = 0; t < DC_C; ++t) ks[t][col] = x[t];      // a column is its thread's own
+      for (int t = 0; t < DC_C; ++t) s.ks[t][col] = x[t];    // a column is its thread's own
     } else {
-#pragma unroll
-      for (int t = 0; t < DC_C; t += 4)
-        st_run<float, 4>(ws + 49 * DP + (size_t)(col - DP) * DC_C + t, x + t);
+      put_columns(49 * DP, c0 - DP, Dv, x);
     }
   }
   __syncthreads();
@@ -176,9 +232,17 @@ __global__ __launch_bounds__(256) void delta_local_kernel(DcParams p) {
   for (int j = 0; j < NT; ++j) {
     const int at = tid + 256 * j, l = at & 63;
     float w[4];
-    ld_run<float, 4>(&ks[l & 15][16 * (at >> 6) + 4 * (l >> 4)], w);
-    st_run<float, 4>(ws + at * 4, w);
+    ld_run<float, 4>(&s.ks[l & 15][16 * (at >> 6) + 4 * (l >> 4)], w);
+    put(at * 4, w);
   }
+}
+
+template <int NT, bool CHAN>
+__global__ __launch_bounds__(256) void delta_local_kernel(DcParams p) {
+  __shared__ __attribute__((aligned(16))) DcLocal<NT> s;
+  int b, t0, n;
+  if (!seq_chunk<DC_C>(p.cu_q, p.B, blockIdx.x, b, t0, n)) return;
+  delta_local<NT, CHAN, 0>(p, s, p.ws + ((size_t)blockIdx.x * p.H + blockIdx.y) * dc_stride(64 * NT, p.Dv), t0, n, blockIdx.y, threadIdx.x);
 }
 
 // Every wave of the workgroup is here and its LDS writes are visible; global loads stay in
@@ -387,7 +451,8 @@ extern "C" int loqa_delta_chunks(const void* act, long ld, int H, int D, int Dv,
     return (int)hipErrorInvalidValue;
   const DcParams p{(const float*)act, ld, H, D, Dv, q_off, k_off, v_off, g_off, hpg, (float*)state,
                    (const int*)state_slots, (const int*)cu_q, (const int*)positions,
-                   (const float*)tok, (float*)ws, (float*)o, B};
+                   (const float*)tok, (float*)ws, (float*)o, B,
+                   D % 4 == 0 && ld % 4 == 0 && q_off % 4 == 0 && k_off % 4 == 0 && (g_off < 0 || g_off % 4 == 0) && ((size_t)act & 15) == 0};
   const dim3 gl(T / DC_C + B, H), gp(B, H, (Dv + 15) / 16);
 #define GO(NT)                                                                                   \
   do {                                                                                           \
