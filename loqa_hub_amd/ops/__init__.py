@@ -9,7 +9,8 @@ Every op has two implementations:
   CPU inputs (the CPU test tier, the config-1 plumbing path) and as the
   numerics oracle in ``tests/test_kernels_gpu.py``.
 
-Plain GEMMs go to hipBLASLt through ``torch.nn.functional.linear``; every fused
+Plain GEMMs of a prompt's rows go to the pipelined tiles, others to hipBLASLt through
+``torch.nn.functional.linear``; every fused
 elementwise/normalisation/attention/audio op around them is ours.
 """
 from __future__ import annotations
@@ -439,8 +440,46 @@ def init_normal(rows: int, cols: int, *, seed: int, key: tuple, std: float = 0.0
     return out
 
 
+LINEAR_ROWS = 33                      # fewer are the vendor's
+LINEAR_WEIGHTS, LINEAR_MANY = 64 << 20, 1200
+
+
+def _linear_shape(M: int, N: int, K: int) -> bool:
+    """Whether the pipelined tiles take a plain product. Over 17 weights of 768 x 512 to 22016 x 4096 at 48 to 3500 rows (cold weights,
+    replayed graphs) they take 0.87 of the vendor's time on average: 2048 x 3072 x 1536 22.7 us against 23.4, 1500 rows 17.9
+    against 22.9, 320 x 4096 x 11008 42.9 against 62.6, 1024 x 2048 x 1024 8.4 against 10.9; nine of these 168 shapes are 3 to 9 % slower
+    (1024 x 2048 x 5632 40.8, 38.0). On the host a call takes 8 us against 19. Weights beyond 64 Mi entries are bound by their stream
+    up to some thousand rows, where the vendor's is 0 to 8 % faster (777 x 22016 x 4096 132 against 143; 1500 rows 290, 221)."""
+    return M >= LINEAR_ROWS and N > 0 and N % 128 == 0 and K > 0 and K % 64 == 0 and (N * K <= LINEAR_WEIGHTS or M > LINEAR_MANY)
+
+
+def _linear_own(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether a product goes to the pipelined tiles: two whole matrices of such sizes and places, whose product is no more than its
+    value, as nothing records, differentiates, maps or traces it."""
+    if type(x) is not torch.Tensor or type(w) not in (torch.Tensor, torch.nn.Parameter) or torch.compiler.is_compiling():
+        return False
+    if not (x.is_cuda and w.is_cuda) or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or x.dim() != 2 or w.dim() != 2:
+        return False
+    if not _linear_shape(x.shape[0], *w.shape) or torch.is_grad_enabled() and (x.requires_grad or w.requires_grad):
+        return False
+    if torch._C._functorch.is_functorch_wrapped_tensor(x) or torch._C._functorch.is_functorch_wrapped_tensor(w) \
+            or torch.autograd.forward_ad._current_level >= 0 or torch._C._get_tracing_state() is not None \
+            or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack() or torch.is_autocast_enabled("cuda"):
+        return False
+    return x.shape[1] == w.shape[1] and x.device == w.device and x.device.index == torch.cuda.current_device() \
+        and _linear_places(x.stride(), x.shape[1], w.is_contiguous(), x.data_ptr() | w.data_ptr())
+
+
+def _linear_places(strides: tuple, K: int, whole: bool, at: int) -> bool:
+    """The rows as gemm_sk's pipelined tiles want them: 16-byte pieces at 32-bit offsets, none over another."""
+    return strides[1] == 1 and K <= strides[0] < 1 << 21 and strides[0] % 8 == 0 and whole and at % 16 == 0
+
+
 def linear(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None) -> torch.Tensor:
-    """Plain GEMM: hipBLASLt via torch on the GPU."""
+    """Plain GEMM: bf16 matrices of more rows than a token step on the pipelined tiles (:func:`gemm_sk`), the rest by hipBLASLt
+    via torch."""
+    if b is None and type(x) is torch.Tensor and x.dim() == 2 and x.size(0) >= LINEAR_ROWS and _linear_own(x, w):
+        return gemm_sk(x, w)
     return torch.nn.functional.linear(x, w, b)
 
 
