@@ -9,7 +9,7 @@ Every op has two implementations:
   CPU inputs (the CPU test tier, the config-1 plumbing path) and as the
   numerics oracle in ``tests/test_kernels_gpu.py``.
 
-Plain GEMMs of a prompt's rows go to the pipelined tiles, others to hipBLASLt through
+Plain bf16 GEMMs go to the pipelined tiles where these are faster, others to hipBLASLt through
 ``torch.nn.functional.linear``; every fused
 elementwise/normalisation/attention/audio op around them is ours.
 """
@@ -440,8 +440,8 @@ def init_normal(rows: int, cols: int, *, seed: int, key: tuple, std: float = 0.0
     return out
 
 
-LINEAR_ROWS = 33                      # fewer are the vendor's
-LINEAR_WEIGHTS, LINEAR_MANY = 64 << 20, 1200
+LINEAR_TOKENS = 32                    # rows of a token step
+LINEAR_WEIGHTS, LINEAR_STREAM = 64 << 20, (64, 1200)
 
 
 def _linear_shape(M: int, N: int, K: int) -> bool:
@@ -449,8 +449,12 @@ def _linear_shape(M: int, N: int, K: int) -> bool:
     replayed graphs) they take 0.87 of the vendor's time on average: 2048 x 3072 x 1536 22.7 us against 23.4, 1500 rows 17.9
     against 22.9, 320 x 4096 x 11008 42.9 against 62.6, 1024 x 2048 x 1024 8.4 against 10.9; nine of these 168 shapes are 3 to 9 % slower
     (1024 x 2048 x 5632 40.8, 38.0). On the host a call takes 8 us against 19. Weights beyond 64 Mi entries are bound by their stream
-    up to some thousand rows, where the vendor's is 0 to 8 % faster (777 x 22016 x 4096 132 against 143; 1500 rows 290, 221)."""
-    return M >= LINEAR_ROWS and N > 0 and N % 128 == 0 and K > 0 and K % 64 == 0 and (N * K <= LINEAR_WEIGHTS or M > LINEAR_MANY)
+    from 65 to some thousand rows, where the vendor's is 0 to 8 % faster (777 x 22016 x 4096 132 against 143; 1500 rows 290, 221).
+    A token step's rows are taken where the plan has no K chunks: 0.90 of the vendor's time over 78 shapes (8 x 3072 x 1536 6.9,
+    7.5; 8 x 11264 x 2048 11.7, 14.6), at worst 1.03 (8 x 768 x 512 4.2, 4.1); in chunks 8 x 6144 x 4096 15.9, 14.4."""
+    if M <= 0 or N <= 0 or N % 128 or K <= 0 or K % 64 or (N * K > LINEAR_WEIGHTS and LINEAR_STREAM[0] < M <= LINEAR_STREAM[1]):
+        return False
+    return M > LINEAR_TOKENS or _sk_plan(M, N, K, True)[1] == 1
 
 
 def _linear_own(x: torch.Tensor, w: torch.Tensor) -> bool:
@@ -476,9 +480,9 @@ def _linear_places(strides: tuple, K: int, whole: bool, at: int) -> bool:
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None) -> torch.Tensor:
-    """Plain GEMM: bf16 matrices of more rows than a token step on the pipelined tiles (:func:`gemm_sk`), the rest by hipBLASLt
+    """Plain GEMM: bf16 matrices on the pipelined tiles (:func:`gemm_sk`) where these are faster, the rest by hipBLASLt
     via torch."""
-    if b is None and type(x) is torch.Tensor and x.dim() == 2 and x.size(0) >= LINEAR_ROWS and _linear_own(x, w):
+    if b is None and _linear_own(x, w):
         return gemm_sk(x, w)
     return torch.nn.functional.linear(x, w, b)
 

@@ -7,7 +7,8 @@ from loqa_hub_amd import ops
 gpu = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("M,N,K,own", [(32, 1024, 512, False), (33, 1024, 512, True), (0, 1024, 512, False), (512, 1024, 480, False),
+@pytest.mark.parametrize("M,N,K,own", [(32, 1024, 512, True), (1, 1024, 512, True), (32, 6144, 4096, False), (33, 6144, 4096, True),
+                                       (0, 1024, 512, False), (512, 1024, 480, False), (64, 16384, 4160, True), (65, 16384, 4160, False),
                                        (512, 1088, 512, False), (512, 0, 512, False), (512, 128, 0, False), (1200, 16384, 4160, False),
                                        (1201, 16384, 4160, True), (1200, 16384, 4096, True)])
 def test_shapes(M, N, K, own):
@@ -43,7 +44,7 @@ def _close(y, x, w):
 
 
 @gpu
-@pytest.mark.parametrize("M,N,K,ld", [(33, 128, 64, None), (191, 1536, 1536, None), (257, 384, 576, 584), (1201, 256, 128, 160),
+@pytest.mark.parametrize("M,N,K,ld", [(1, 256, 512, None), (33, 128, 64, None), (191, 1536, 1536, None), (257, 384, 576, 584), (1201, 256, 128, 160),
                                       (320, 1024, 5632, None)])
 def test_own_products(M, N, K, ld):
     x, w = _operands(M, N, K, ld)
