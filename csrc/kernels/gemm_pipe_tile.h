@@ -350,6 +350,8 @@ template <bool AHEAD, bool SPLIT> static int gp_layout(const GemmSkCall& p, int 
     case 6: return gp_launch<6, 6, 3, 3, AHEAD, SPLIT>(p, st);   // 192 x 192
     case 7: return gp_launch<4, 2, 4, 4, AHEAD, SPLIT>(p, st);   // 128 x 64
     case 8: return gp_launch<4, 4, 5, 5, AHEAD, SPLIT>(p, st);   // 128 x 128
+    case 9: return gp_launch<8, 5, 3, 3, AHEAD, SPLIT>(p, st);   // 256 x 160
+    case 10: return gp_launch<4, 5, 3, 3, AHEAD, SPLIT>(p, st);  // 128 x 160
     default: return (int)hipErrorInvalidValue;
   }
 }

@@ -454,7 +454,7 @@ def _linear_shape(M: int, N: int, K: int) -> bool:
     7.5; 8 x 11264 x 2048 11.7, 14.6), at worst 1.03 (8 x 768 x 512 4.2, 4.1); in chunks 8 x 6144 x 4096 15.9, 14.4."""
     if M <= 0 or N <= 0 or N % 128 or K <= 0 or K % 64 or (N * K > LINEAR_WEIGHTS and LINEAR_STREAM[0] < M <= LINEAR_STREAM[1]):
         return False
-    return M > LINEAR_TOKENS or _sk_plan(M, N, K, True)[1] == 1
+    return M > LINEAR_TOKENS or _sk_choice(M, N, K, True)[1] == 1
 
 
 def _linear_own(x: torch.Tensor, w: torch.Tensor) -> bool:
@@ -1758,6 +1758,13 @@ SK_LAYOUTS = {1: (128, 64, 0.60, 4.0), 7: (64, 64, 0.55, 4.0), 11: (64, 64, 0.19
               12: (256, 256, 1.20, 10.3), 13: (256, 192, 1.075, 5.5), 14: (192, 256, 1.073, 5.5),
               15: (256, 128, 0.908, 4.0), 16: (128, 256, 0.784, 6.6), 17: (128, 192, 0.667, 4.6),
               18: (192, 192, 0.854, 6.0), 19: (128, 64, 0.309, 4.3), 20: (128, 128, 0.498, 3.6)}
+# Tiles of 160 rows (pipelined), for row counts that pad the others: gemm_sk asks the plan's rules for these beside the plan
+# (_sk_choice). Times fitted over 256 shapes of 100 to 3000 rows, cold weights, against the plan alone: taken in 30 of them, 0.94 of the
+# time there, slower by more than 1.5 % in none; 12 more that they would win by 2 to 13 % are left to the plan. The step of 22 is fitted
+# 4 % above what it takes: it is bound by LDS, where 128 x 192 is bound by its MFMAs, and wins only by rows that it does not pad. us, the
+# plan's and these: 320 x 28672 x 4096 79.7, 73.4; 640 143, 131; 160 x 6144 x 4096 22.8, 21.1; 1280 x 4096 x 14336 135, 119; 1500 x 11264 x
+# 2048 74.5, 66.9.
+SK_ROWS160 = {21: (256, 160, 0.96, 7.0), 22: (128, 160, 0.68, 5.0)}
 SK_PIPE = 11              # the first pipelined layout
 SK_WHOLE = 12             # the layout that the plan does not split along K
 # numbers of layouts that are gone (other stage counts and wave splits of the general form, 256
@@ -1805,11 +1812,17 @@ def gemm_sk_plan(M: int, N: int, K: int, epi: str = "bf16", layouts=None, *,
 # each time, 0.1 for a shape that was asked before
 @functools.lru_cache(maxsize=4096)
 def _sk_plan(M: int, N: int, K: int, pipe: bool, layouts: tuple | None = None, gelu: bool = False) -> tuple[int, int]:
-    KT = K // 64
     only = SK_LAYOUTS if layouts is None else {SK_RENAMED.get(x, x) for x in layouts}
+    return _sk_least(M, N, K, pipe, [lay for lay in SK_LAYOUTS if lay in only], gelu)[1:]
+
+
+def _sk_least(M: int, N: int, K: int, pipe: bool, layouts, gelu: bool) -> tuple[float, int, int]:
+    """(us, layout, K chunks) of the fastest of ``layouts``."""
+    KT = K // 64
     best, best_t = (7, 1), float("inf")
-    for lay, (bn, bm, _, _) in SK_LAYOUTS.items():
-        if N % bn or (lay >= SK_PIPE) != (pipe and N % 128 == 0) or lay not in only:
+    for lay in layouts:
+        bn, bm = _sk_tile(lay)[:2]
+        if N % bn or (lay >= SK_PIPE) != (pipe and N % 128 == 0):
             continue
         tiles = -(-M // bm) * (N // bn)
         for s in (1, 2, 3, 4, 5, 6, 8):
@@ -1818,12 +1831,26 @@ def _sk_plan(M: int, N: int, K: int, pipe: bool, layouts: tuple | None = None, g
             t = _sk_us(lay, M, N, K, s, gelu)
             if t < best_t:
                 best, best_t = (lay, s), t
-    return best
+    return best_t, *best
+
+
+@functools.lru_cache(maxsize=4096)
+def _sk_choice(M: int, N: int, K: int, pipe: bool, gelu: bool = False) -> tuple[int, int]:
+    """What gemm_sk takes where it may choose: the plan's, or tiles of 160 rows where these are faster."""
+    lay, s = _sk_plan(M, N, K, pipe, None, gelu)
+    if not pipe or N % 128:
+        return lay, s
+    t, tall, ts = _sk_least(M, N, K, pipe, SK_ROWS160, gelu)
+    return (tall, ts) if t < _sk_us(lay, M, N, K, s, gelu) else (lay, s)
+
+
+def _sk_tile(lay: int) -> tuple:
+    return SK_LAYOUTS[lay] if lay in SK_LAYOUTS else SK_ROWS160[lay]
 
 
 def _sk_us(lay: int, M: int, N: int, K: int, s: int, gelu: bool) -> float:
     """Microseconds of M x N x K in ``s`` K chunks of layout ``lay`` (:func:`gemm_sk_plan`)."""
-    bn, bm, step, around = SK_LAYOUTS[lay]
+    bn, bm, step, around = _sk_tile(lay)
     tiles, KT = -(-M // bm) * (N // bn), K // 64
     if lay == SK_SMALL and K > 2048:
         step *= 1.26
@@ -1910,7 +1937,7 @@ def _ahead(p, ahead: tuple, tiles: int) -> None:
     wgs = min(SK_CUS - tiles, AHEAD_WGS[1])
     if wgs < AHEAD_WGS[0] or max(w.numel() * w.element_size() for w in ahead) < AHEAD_MIN_BYTES:
         return
-    step, around = SK_LAYOUTS[p.layout][2:]
+    step, around = _sk_tile(p.layout)[2:]
     us = p.K // 64 / p.S * step + around
     left = int(min(us * wgs * AHEAD_WG_BYTES_PER_US, us * AHEAD_BYTES_PER_US - 2.0 * p.N * p.K))
     for i, w in enumerate(ahead[:2]):
@@ -1948,7 +1975,7 @@ def gemm_sk(x: torch.Tensor, w: torch.Tensor, *, epi: str = "bf16", bias: torch.
     ``epi``: "bf16" -> [M, N] (+ f32 ``bias``, ``act`` "gelu"); "swiglu" -> silu(gate) * up
     [M, N / 2] (gate rows [0, N/2), up rows [N/2, N)); "resid" -> ``residual``
     [M, N] += X W^T (+ ``bias``) in place (one bf16 rounding), returned. ``layout``: a number of
-    SK_LAYOUTS or SK_RENAMED (None: the plan's). ``ahead``: up to two weights that later launches
+    SK_LAYOUTS, SK_ROWS160 or SK_RENAMED (None: the plan's, or SK_ROWS160's where that is faster). ``ahead``: up to two weights that later launches
     will read, touched meanwhile by workgroups on compute units that have no tile (:func:`_ahead`)."""
     N, K = w.shape
     M = x.shape[0]
@@ -1975,13 +2002,16 @@ def gemm_sk(x: torch.Tensor, w: torch.Tensor, *, epi: str = "bf16", bias: torch.
         pipe = x.stride(0) >= K and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 \
             and N * K < 1 << 31 and x.stride(0) < 1 << 21 \
             and (y is None or (y.stride(0) % 8 == 0 and y.data_ptr() % 16 == 0))
-        pl, ps = _sk_plan(M, N, K, pipe, None, act == "gelu")
+        if layout is None and splits is None:
+            pl, ps = _sk_choice(M, N, K, pipe, act == "gelu")
+        else:
+            pl, ps = _sk_plan(M, N, K, pipe, None, act == "gelu")
         layout = pl if layout is None else layout
         splits = ps if splits is None else splits
         # (11 named the 128 x 64 tiles once, and takes what it did)
         if layout in SK_RENAMED or layout == SK_SMALL:
             layout = SK_RENAMED.get(layout, layout) if pipe else 1
-    bn, bm = SK_LAYOUTS[layout][:2]
+    bn, bm = _sk_tile(layout)[:2]
     if N % bn or K % 64:
         raise ValueError(f"gemm_sk layout {layout}: N {N} / K {K} not tileable")
     p = _lib.GemmSkParams()
