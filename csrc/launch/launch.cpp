@@ -3,7 +3,8 @@
 // A step of one token a sequence is bound by the host: through ctypes an entry point of some thirty arguments
 // cost 6 to 7 us, 4 of them for turning Python's numbers and addresses into C's. Here the conversions follow from the entry
 // point's own type, and a pointer argument takes the tensor itself (its data_ptr()), a number or None. Two launches of a windowed
-// token with the checks before them: 24.5 us through ctypes, 14.4 through this.
+// token with the checks before them: 24.5 us through ctypes, 14.4 through this. Latent attention's steps, which are short prompts as
+// well, come through here too.
 //
 // The symbols are libloqa_seqmix.so's, which is loaded before this module; signatures() lets the loader compare the
 // types here with those it knows.
@@ -33,6 +34,15 @@ int loqa_delta_scan(const void*, long, int, int, int, int, int, int, int, int, v
 int loqa_seq_state_save(const void*, int, const void*, int, int, void*, void*, int, int, int, const void*, const void*, const void*, int,
                         stream_t);
 int loqa_gated_rmsnorm(const void*, const void*, const void*, int, long, float, void*, int, int, int, int, int, stream_t);
+int loqa_latent_attention(const void*, long, long, const void*, long, long, int, const void*, int, int, const void*, const void*,
+                          const void*, int, const void*, const void*, int, const void*, float, int, int, int, int, int, int, void*, int,
+                          void*, int, int, stream_t);
+int loqa_latent_kv(const void*, long, int, int, const void*, int, const void*, const void*, int, int, const void*, int, int, int, int,
+                   int, void*, void*, int, stream_t);
+int loqa_latent_prefill(const void*, long, const void*, const void*, void*, long, const void*, const void*, const void*, const void*,
+                        const void*, float, int, const void*, long, int, int, int, int, int, int, const void*, int, int, int, int,
+                        void*, long, void*, long, stream_t);
+int loqa_sigmoid_gate(const void*, long, long, int, const void*, long, void*, long, long, int, int, int, stream_t);
 int loqa_moe_route(const void*, const void*, const void*, int, int, int, int, int, int, int, float, void*, void*, int, stream_t);
 }
 
@@ -212,7 +222,8 @@ PyObject* window_shapes(PyObject*, PyObject* const* args, Py_ssize_t n) {
 
 #define ENTRIES(X)                                                                                                                \
   X(loqa_qk_prep_append) X(loqa_window_attention) X(loqa_window_attention_parts) X(loqa_delta_prep) X(loqa_delta_scan) \
-  X(loqa_seq_state_save) X(loqa_gated_rmsnorm) X(loqa_moe_route)
+  X(loqa_seq_state_save) X(loqa_gated_rmsnorm) X(loqa_moe_route) X(loqa_latent_attention) X(loqa_latent_kv) \
+  X(loqa_latent_prefill) X(loqa_sigmoid_gate)
 
 PyObject* signatures(PyObject*, PyObject*) {
   PyObject* d = PyDict_New();

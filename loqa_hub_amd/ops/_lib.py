@@ -337,8 +337,8 @@ def _main_kernels() -> ctypes.CDLL:
 # Entry points of token steps, which ``libloqa_launch.so`` calls without ctypes; their pointer arguments are
 # tensors, addresses or None. i32c and f32c check (tensor, name) pairs, the others the tensors of a launch.
 _LAUNCH = frozenset(("loqa_qk_prep_append", "loqa_window_attention", "loqa_window_attention_parts", "loqa_delta_prep",
-                     "loqa_delta_scan", "loqa_seq_state_save", "loqa_gated_rmsnorm", "loqa_moe_route", "i32c", "f32c",
-                     "qk_shapes", "window_shapes"))
+                     "loqa_delta_scan", "loqa_seq_state_save", "loqa_gated_rmsnorm", "loqa_moe_route", "loqa_latent_attention",
+                     "loqa_latent_kv", "loqa_latent_prefill", "loqa_sigmoid_gate", "i32c", "f32c", "qk_shapes", "window_shapes"))
 _launch = None
 
 

@@ -225,10 +225,11 @@ def latent_attention(qa: torch.Tensor, qr: torch.Tensor, cache: torch.Tensor, cu
     assert qa.shape[2] == R and qa.stride(2) == 1 and qr.shape == (T, H, Dr) and qr.stride(2) == 1
     assert qa.dtype == cache.dtype == qr.dtype == out.dtype and cache.is_contiguous()
     assert out.is_contiguous() and out.shape == (H, T, R)
-    _i32c(cu_q, "cu_q"); _i32c(ctx_lens, "ctx_lens"); _i32c(block_tables, "block_tables")
-    _i32c(positions, "positions"); _f32c(cos_sin, "cos_sin")
+    lib = kernels()
+    lib.i32c(cu_q, "cu_q", ctx_lens, "ctx_lens", block_tables, "block_tables", positions, "positions")
+    lib.f32c(cos_sin, "cos_sin")
     if sink is not None:
-        _f32c(sink, "sink")
+        lib.f32c(sink, "sink")
         assert sink.numel() == H
     B = ctx_lens.numel()
     assert cu_q.numel() == B + 1 and block_tables.shape[0] == B and positions.numel() >= T
@@ -239,11 +240,11 @@ def latent_attention(qa: torch.Tensor, qr: torch.Tensor, cache: torch.Tensor, cu
     ns = 1 if wgs >= 512 else max(1, min(32, -(-keys // (64 if mfma else 128)), 1024 // max(1, wgs)))
     ws = torch.empty(ns * T * H * (R + 2), dtype=torch.float32, device=qa.device) if ns > 1 else None
     if T:
-        check(kernels().loqa_latent_attention(
-            ptr(qa), qa.stride(1), qa.stride(0), ptr(qr), qr.stride(0), qr.stride(1), _dt(qa),
-            ptr(cache), cache.shape[1], cache.shape[0], ptr(cu_q), ptr(ctx_lens), ptr(block_tables),
-            block_tables.shape[1], ptr(positions), ptr(cos_sin), cos_sin.shape[0], ptr(sink),
-            float(scale), B, H, T, R, Dr, dims, ptr(out), ns, ptr(ws), int(window), int(mfma),
+        check(lib.loqa_latent_attention(
+            qa, qa.stride(1), qa.stride(0), qr, qr.stride(0), qr.stride(1), _dt(qa),
+            cache, cache.shape[1], cache.shape[0], cu_q, ctx_lens, block_tables,
+            block_tables.shape[1], positions, cos_sin, cos_sin.shape[0], sink,
+            float(scale), B, H, T, R, Dr, dims, out, ns, ws, int(window), int(mfma),
             stream_ptr(qa)),
             "latent_attention")
     return out
@@ -324,9 +325,9 @@ def latent_keys_values(cache: torch.Tensor, block_tables: torch.Tensor, cu_k: to
     def us(layout):
         bn, bm, step, around = KV_LAYOUTS[layout]
         return -(-(-(-total_k // bm) * (H * (DK + DV) // bn)) // 256) * (R // 64 * step + around)
-    check(kernels().loqa_latent_kv(ptr(cache), cache.numel() * 2, cache.shape[1], cache.shape[2], ptr(block_tables),
-                                   block_tables.shape[1], ptr(cu_k), ptr(ctx_lens), B, total_k, ptr(wkv), R, H, DK,
-                                   DV, D, ptr(k), ptr(v), min(fits, key=us), stream_ptr(cache)), "latent_kv")
+    check(kernels().loqa_latent_kv(cache, cache.numel() * 2, cache.shape[1], cache.shape[2], block_tables,
+                                   block_tables.shape[1], cu_k, ctx_lens, B, total_k, wkv, R, H, DK,
+                                   DV, D, k, v, min(fits, key=us), stream_ptr(cache)), "latent_kv")
     return k, v
 
 
@@ -395,10 +396,10 @@ def latent_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu_q: torc
         blocks = -(-max_q // 64) * H * B
         ws, words = _sk_workspace(q.device, st, blocks * parts * 2 * (DV // 2 + 4) * 64, blocks)
     check(kernels().loqa_latent_prefill(
-        ptr(q), q.stride(0), ptr(k), ptr(v), ptr(out), out.stride(0), ptr(cu_q), ptr(cu_k),
-        ptr(ctx_lens), ptr(positions), ptr(sink), float(scale), int(window), ptr(gate),
-        gate.stride(0) if gate is not None else 0, B, H, int(max_q), DK, DV, Dv, ptr(cs), *turn, parts,
-        ptr(ws), ws.numel() if parts > 1 else 0, ptr(words), words.numel() if parts > 1 else 0, st),
+        q, q.stride(0), k, v, out, out.stride(0), cu_q, cu_k,
+        ctx_lens, positions, sink, float(scale), int(window), gate,
+        gate.stride(0) if gate is not None else 0, B, H, int(max_q), DK, DV, Dv, cs, *turn, parts,
+        ws, ws.numel() if parts > 1 else 0, words, words.numel() if parts > 1 else 0, st),
         "latent_prefill")
     return out
 
@@ -1126,8 +1127,8 @@ def sigmoid_gate(o: torch.Tensor, gate: torch.Tensor, H: int, Dv: int,
     assert gate.shape == (T, H * Dv) and gate.stride(1) == 1 and gate.dtype == o.dtype
     assert out.shape == (T, H * Dv) and out.stride(1) == 1 and out.dtype == o.dtype
     if T:
-        check(kernels().loqa_sigmoid_gate(ptr(o), o.stride(0), o.stride(1), _dt(o), ptr(gate),
-                                          gate.stride(0), ptr(out), out.stride(0), Dv, T, H, Dv,
+        check(kernels().loqa_sigmoid_gate(o, o.stride(0), o.stride(1), _dt(o), gate,
+                                          gate.stride(0), out, out.stride(0), Dv, T, H, Dv,
                                           stream_ptr(o)), "sigmoid_gate")
     return out
 
