@@ -43,6 +43,7 @@ int loqa_latent_prefill(const void*, long, const void*, const void*, void*, long
                         const void*, float, int, const void*, long, int, int, int, int, int, int, const void*, int, int, int, int,
                         void*, long, void*, long, stream_t);
 int loqa_sigmoid_gate(const void*, long, long, int, const void*, long, void*, long, long, int, int, int, stream_t);
+int loqa_head_product(const void*, long, long, const void*, int, int, int, int, void*, long, long, stream_t);
 int loqa_moe_route(const void*, const void*, const void*, int, int, int, int, int, int, int, float, void*, void*, int, stream_t);
 }
 
@@ -223,7 +224,7 @@ PyObject* window_shapes(PyObject*, PyObject* const* args, Py_ssize_t n) {
 #define ENTRIES(X)                                                                                                                \
   X(loqa_qk_prep_append) X(loqa_window_attention) X(loqa_window_attention_parts) X(loqa_delta_prep) X(loqa_delta_scan) \
   X(loqa_seq_state_save) X(loqa_gated_rmsnorm) X(loqa_moe_route) X(loqa_latent_attention) X(loqa_latent_kv) \
-  X(loqa_latent_prefill) X(loqa_sigmoid_gate)
+  X(loqa_latent_prefill) X(loqa_sigmoid_gate) X(loqa_head_product)
 
 PyObject* signatures(PyObject*, PyObject*) {
   PyObject* d = PyDict_New();

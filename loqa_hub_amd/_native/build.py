@@ -94,7 +94,7 @@ SEQMIX_SOURCES = ("norm_dyt.hip", "attn_latent.hip", "attn_latent_prefill.hip", 
                   "norm_rms1p.hip", "attn_window.hip", "mamba2.hip", "matrix_memory.hip",
                   "delta_rule.hip", "norm_layer.hip", "linear_chunks.hip",
                   "delta_chunks.hip", "moe_pipe.hip", "attn_window_pipe.hip", "attn_window_token.hip",
-                  "latent_kv.hip")
+                  "latent_kv.hip", "head_product.hip")
 
 # hipcc may not form packed-f32 VALU instructions from scalar float code
 NO_PACKED_F32 = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]

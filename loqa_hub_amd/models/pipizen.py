@@ -25,7 +25,7 @@ MI355X layout, in the manner of the Llama decoder next to it:
   feed-forward are one GEMM each; the experts' weights are stacked [E, ...] for
   the grouped expert GEMMs.
 
-Plain GEMMs go to the vendor library through ``ops.linear`` / ``torch.bmm``;
+Plain GEMMs are ``ops.linear`` and ``seqmix.head_product``;
 everything around them is this repository's HIP.
 """
 from __future__ import annotations
@@ -91,11 +91,11 @@ def latent_heads(L: dict, m, q: torch.Tensor, pages: torch.Tensor, meta, prompt_
         return seqmix.latent_prefill(q, k, v, meta.cu_q, cu_k, meta.ctx_lens, meta.positions,
                                      L["sink"], m.scale, meta.max_q, Dv, window, gate, out,
                                      (D, m.rot.dims, L["cos_sin"]))
-    qa = torch.bmm(q[:, :, :D].transpose(0, 1), L["wuk"])            # [H, T, R]
+    qa = seqmix.head_product(q[:, :, :D], L["wuk"]).transpose(0, 1)  # [H, T, R]
     lat = seqmix.latent_attention(qa, q[:, :, D:D + Dr], pages, meta.cu_q, meta.ctx_lens,
                                   meta.block_tables, meta.positions, L["cos_sin"], L["sink"],
                                   m.scale, R, m.rot.dims, meta.max_ctx, window=window)
-    o = torch.bmm(lat, L["wuv_t"]).transpose(0, 1)                   # [T, H, Dv], head-major
+    o = seqmix.head_product(lat.transpose(0, 1), L["wuv_t"])         # [T, H, Dv]
     if gate is not None:
         return seqmix.sigmoid_gate(o, gate, H, Dv, out)
     if out is None:

@@ -271,6 +271,7 @@ _SEQMIX_SIGS = {
     "loqa_residual_rms1p": [_vp, _vp, _f, _vp, _f, _vp, _f, _i, _vp, _vp, _vp, _f, _vp, _vp, _i,
                             _i, _i, _vp],
     "loqa_rms_norm_cols": [_vp, _i, _l, _i, _vp, _f, _vp, _i, _i, _vp],
+    "loqa_head_product": [_vp, _l, _l, _vp, _i, _i, _i, _i, _vp, _l, _l, _vp],
     "loqa_sigmoid_gate": [_vp, _l, _l, _i, _vp, _l, _vp, _l, _l, _i, _i, _i, _vp],
     "loqa_softcap": [_vp, _l, _f, _vp],
     "loqa_exp_gate_scan": [_vp, _i, _vp, _vp, _f, _vp, _i, _vp, _vp, _vp, _i, _i, _vp, _vp, _vp],
@@ -338,7 +339,7 @@ def _main_kernels() -> ctypes.CDLL:
 # tensors, addresses or None. i32c and f32c check (tensor, name) pairs, the others the tensors of a launch.
 _LAUNCH = frozenset(("loqa_qk_prep_append", "loqa_window_attention", "loqa_window_attention_parts", "loqa_delta_prep",
                      "loqa_delta_scan", "loqa_seq_state_save", "loqa_gated_rmsnorm", "loqa_moe_route", "loqa_latent_attention",
-                     "loqa_latent_kv", "loqa_latent_prefill", "loqa_sigmoid_gate", "i32c", "f32c", "qk_shapes", "window_shapes"))
+                     "loqa_latent_kv", "loqa_latent_prefill", "loqa_sigmoid_gate", "loqa_head_product", "i32c", "f32c", "qk_shapes", "window_shapes"))
 _launch = None
 
 

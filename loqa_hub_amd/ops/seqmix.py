@@ -1112,6 +1112,25 @@ def rms_norm_cols(u: torch.Tensor, n: int, w: torch.Tensor, eps: float, out_dtyp
     return y
 
 
+HEAD_PRODUCT_ROWS = 64
+
+
+def head_product(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """y[t, h, :] = x[t, h, :] w[h] for x [T, H, K] (any strides over tokens and heads) and w [H, K, N]: a view [T, H, N]. The few
+    bf16 rows of a token step run in ``csrc/kernels/head_product.hip``, what it does not take as a batched product of the
+    vendor's."""
+    T, H, K = x.shape
+    N = w.shape[-1]
+    if not (x.is_cuda and 0 < T <= HEAD_PRODUCT_ROWS and x.dtype == w.dtype == torch.bfloat16 and w.shape == (H, K, N) and 0 < K <= 512
+            and K % 128 == 0 and N > 0 and N % 64 == 0 and x.stride(2) == 1 and (x.stride(0) | x.stride(1)) % 4 == 0
+            and w.is_contiguous() and x.data_ptr() % 8 == 0 and w.data_ptr() % 16 == 0 and w.device == x.device
+            and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))):
+        return torch.bmm(x.transpose(0, 1), w).transpose(0, 1)
+    y = x.new_empty((T, H, N))
+    check(kernels().loqa_head_product(x, x.stride(0), x.stride(1), w, T, H, K, N, y, H * N, N, stream_ptr(x)), "head_product")
+    return y
+
+
 def sigmoid_gate(o: torch.Tensor, gate: torch.Tensor, H: int, Dv: int,
                  out: torch.Tensor | None = None) -> torch.Tensor:
     """The first Dv entries of every head of o [T, H, >= Dv] (any strides over
