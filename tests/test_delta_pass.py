@@ -31,6 +31,7 @@ def test_feeds_of_few_chunks(D, Dv, off):
         assert (x - y).abs().max() < 3e-5 * max(1.0, float(y.abs().max()))
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("chan", [True, False])
 @pytest.mark.parametrize("D,Dv,hpg,shift", [(64, 64, 2, 0), (20, 1, 1, 0), (66, 37, 2, 0), (128, 200, 1, 0), (128, 128, 2, 3), (130, 70, 1, 0),
                                             (256, 300, 2, 0), (192, 64, 1, 1)])
