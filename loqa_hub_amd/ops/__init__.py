@@ -1764,7 +1764,13 @@ SK_LAYOUTS = {1: (128, 64, 0.60, 4.0), 7: (64, 64, 0.55, 4.0), 11: (64, 64, 0.19
 # 4 % above what it takes: it is bound by LDS, where 128 x 192 is bound by its MFMAs, and wins only by rows that it does not pad. us, the
 # plan's and these: 320 x 28672 x 4096 79.7, 73.4; 640 143, 131; 160 x 6144 x 4096 22.8, 21.1; 1280 x 4096 x 14336 135, 119; 1500 x 11264 x
 # 2048 74.5, 66.9.
+# In a pass of a model each K chunk costs more than it does alone, as its partials go out and back beside the next launch's cold
+# weights, and the attention behind finds less of its keys (320 rows of an 8B model: 15.2 -> 16.3 us): so at most one chunk more than
+# the plan's, none where it has none, and 128 x 160 for one tile of rows only. us a projection in the pass with the plan's tile and with
+# the one left out: 257 to 320 x 4096 x 14336 in 4 chunks of 128 x 192, + 2.3 to 6.8 in 8 of 256 x 160; x 4096 x 4096 in 4 of 128 x 192,
+# + 0.8 to 1.1 in 4 of 128 x 160; 1600 x 3072 x 8192 and 2305 to 2560 x 2048 x 8192 whole, - 0.4 to + 1.9 in 2.
 SK_ROWS160 = {21: (256, 160, 0.96, 7.0), 22: (128, 160, 0.68, 5.0)}
+SK_ONE160 = 22            # for up to 160 rows
 SK_PIPE = 11              # the first pipelined layout
 SK_WHOLE = 12             # the layout that the plan does not split along K
 # numbers of layouts that are gone (other stage counts and wave splits of the general form, 256
@@ -1816,8 +1822,8 @@ def _sk_plan(M: int, N: int, K: int, pipe: bool, layouts: tuple | None = None, g
     return _sk_least(M, N, K, pipe, [lay for lay in SK_LAYOUTS if lay in only], gelu)[1:]
 
 
-def _sk_least(M: int, N: int, K: int, pipe: bool, layouts, gelu: bool) -> tuple[float, int, int]:
-    """(us, layout, K chunks) of the fastest of ``layouts``."""
+def _sk_least(M: int, N: int, K: int, pipe: bool, layouts, gelu: bool, most: int = 8) -> tuple[float, int, int]:
+    """(us, layout, K chunks) of the fastest of ``layouts`` in up to ``most`` chunks."""
     KT = K // 64
     best, best_t = (7, 1), float("inf")
     for lay in layouts:
@@ -1826,7 +1832,7 @@ def _sk_least(M: int, N: int, K: int, pipe: bool, layouts, gelu: bool) -> tuple[
             continue
         tiles = -(-M // bm) * (N // bn)
         for s in (1, 2, 3, 4, 5, 6, 8):
-            if s > 1 and (KT // s < 8 or lay == SK_WHOLE or (lay >= SK_PIPE and tiles * s > SK_CUS)):
+            if s > 1 and (s > most or KT // s < 8 or lay == SK_WHOLE or (lay >= SK_PIPE and tiles * s > SK_CUS)):
                 continue
             t = _sk_us(lay, M, N, K, s, gelu)
             if t < best_t:
@@ -1840,7 +1846,7 @@ def _sk_choice(M: int, N: int, K: int, pipe: bool, gelu: bool = False) -> tuple[
     lay, s = _sk_plan(M, N, K, pipe, None, gelu)
     if not pipe or N % 128:
         return lay, s
-    t, tall, ts = _sk_least(M, N, K, pipe, SK_ROWS160, gelu)
+    t, tall, ts = _sk_least(M, N, K, pipe, [x for x in SK_ROWS160 if x != SK_ONE160 or M <= 160], gelu, s + (s > 1))
     return (tall, ts) if t < _sk_us(lay, M, N, K, s, gelu) else (lay, s)
 
 

@@ -31,6 +31,14 @@ def test_choice():
     assert taken and ops._sk_choice(320, 28672, 4096, True) == (21, 1)
 
 
+@pytest.mark.parametrize("M,N,K,want", [(257, 4096, 14336, (17, 4)), (320, 4096, 14336, (17, 4)), (320, 4096, 4096, (17, 4)),
+                                        (1600, 3072, 8192, (17, 1)), (2432, 2048, 8192, (17, 1)), (1599, 2048, 5632, (20, 1)),
+                                        (160, 4096, 14336, (22, 8)), (161, 4096, 14336, (17, 8)), (640, 4096, 14336, (21, 4)), (1280, 2048, 8192, (21, 4))])
+def test_chunks_that_a_pass_pays_for(M, N, K, want):
+    """At most one chunk more than the plan's and none where it has none; 128 x 160 for one tile of rows."""
+    assert ops._sk_choice(M, N, K, True) == want
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("layout", LAYOUTS)
 @pytest.mark.parametrize("stages,splits", [(1, 1), (2, 1), (7, 1), (7, 2), (14, 5), (14, 9)])
