@@ -442,19 +442,35 @@ def init_normal(rows: int, cols: int, *, seed: int, key: tuple, std: float = 0.0
 
 LINEAR_TOKENS = 32                    # rows of a token step
 LINEAR_WEIGHTS, LINEAR_STREAM = 64 << 20, (64, 1200)
+LINEAR_MOST, LINEAR_COLD = 1 << 31, 10 << 20
 
 
+@functools.lru_cache(maxsize=4096)
 def _linear_shape(M: int, N: int, K: int) -> bool:
-    """Whether the pipelined tiles take a plain product. Over 17 weights of 768 x 512 to 22016 x 4096 at 48 to 3500 rows (cold weights,
-    replayed graphs) they take 0.87 of the vendor's time on average: 2048 x 3072 x 1536 22.7 us against 23.4, 1500 rows 17.9
-    against 22.9, 320 x 4096 x 11008 42.9 against 62.6, 1024 x 2048 x 1024 8.4 against 10.9; nine of these 168 shapes are 3 to 9 % slower
-    (1024 x 2048 x 5632 40.8, 38.0). On the host a call takes 8 us against 19. Weights beyond 64 Mi entries are bound by their stream
-    from 65 to some thousand rows, where the vendor's is 0 to 8 % faster (777 x 22016 x 4096 132 against 143; 1500 rows 290, 221).
-    A token step's rows are taken where the plan has no K chunks: 0.90 of the vendor's time over 78 shapes (8 x 3072 x 1536 6.9,
-    7.5; 8 x 11264 x 2048 11.7, 14.6), at worst 1.03 (8 x 768 x 512 4.2, 4.1); in chunks 8 x 6144 x 4096 15.9, 14.4."""
-    if M <= 0 or N <= 0 or N % 128 or K <= 0 or K % 64 or (N * K > LINEAR_WEIGHTS and LINEAR_STREAM[0] < M <= LINEAR_STREAM[1]):
+    """Whether the pipelined tiles take a plain product. Both were timed at 1014 shapes of 1 to 3500 rows and 52 weights (cold weights,
+    replayed graphs: profiles/linear_products.txt): 887 are taken, at 0.86 of the vendor's time on average, 35 of them 3 to 12 % slower
+    (512 x 5120 x 3072 32.6 us, 29.2; 256 x 256 tiles with more than 64 Mi weights 4 to 7 %, 0.68 to 0.78 elsewhere).
+    On the host a call takes 8 us against 19. The vendor's are, by what the two take there (own, vendor's):
+    * the 64 x 64 tiles in K chunks up to K = 4096 (48 x 2048 x 4096 11.0 us, 9.7; 64 x 8192 x 4096 21.2, 18.5) and
+      a token step's rows in any chunks (8 x 6144 x 4096 15.9, 14.4);
+    * more than 192 rows on 128 x 64 tiles in one or two chunks with more than 10 Mi weights, which each row of tiles reads again
+      (320 x 5120 x 3072 25.6, 22.8; 1024 x 2048 x 5632 40.5, 38.1);
+    * 256 x 256 tiles (3500 x 4096 x 4096 94.5, 86.9), but for more than 64 Mi weights (2048 x 22016 x 4096 271, 400);
+    * more than 64 Mi weights from 65 to 1200 rows, bound by their stream (512 x 22016 x 4096 90.2, 82.7);
+    * weights of 2^31 entries and more, to which the pipelined tiles' offsets do not reach."""
+    if M <= 0 or N <= 0 or N % 128 or K <= 0 or K % 64 or N * K >= LINEAR_MOST:
         return False
-    return M > LINEAR_TOKENS or _sk_choice(M, N, K, True)[1] == 1
+    many = N * K > LINEAR_WEIGHTS
+    if many and LINEAR_STREAM[0] < M <= LINEAR_STREAM[1]:
+        return False
+    lay, s = _sk_choice(M, N, K, True)
+    if M <= LINEAR_TOKENS and s > 1:
+        return False
+    if lay == SK_SMALL:
+        return s == 1 or K > 4096
+    if lay == 19:                       # 128 x 64
+        return s > 2 or M <= 192 or N * K <= LINEAR_COLD
+    return lay != SK_WHOLE or many
 
 
 def _linear_own(x: torch.Tensor, w: torch.Tensor) -> bool:

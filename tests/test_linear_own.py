@@ -15,6 +15,15 @@ def test_shapes(M, N, K, own):
     assert ops._linear_shape(M, N, K) is own
 
 
+@pytest.mark.parametrize("M,N,K,own", [(64, 8192, 4096, False), (64, 4096, 8192, True), (96, 2048, 4096, False), (400, 2048, 4096, True),  # 64 x 64 in chunks, and whole
+                                       (320, 5120, 3072, False), (192, 5632, 2048, True), (193, 5632, 2048, False), (257, 4096, 2048, True),
+                                       (257, 3072, 8192, False), (160, 3072, 8192, True), (1024, 2048, 5632, False),                       # 128 x 64
+                                       (3500, 4096, 4096, False), (2048, 22016, 4096, True),                                               # 256 x 256
+                                       (2048, 131072, 16384, False), (2048, 131072, 16320, True)])                                         # 2^31 entries
+def test_what_the_vendor_keeps(M, N, K, own):
+    assert ops._linear_shape(M, N, K) is own
+
+
 @pytest.mark.parametrize("strides,whole,at,own", [((64, 1), True, 32, True), ((72, 1), True, 0, True), ((64, 2), True, 0, False),
                                                   ((56, 1), True, 0, False), ((0, 1), True, 0, False), ((68, 1), True, 0, False),
                                                   ((64, 1), False, 0, False), ((64, 1), True, 8, False), ((1 << 21, 1), True, 0, False)])
