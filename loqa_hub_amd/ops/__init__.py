@@ -480,6 +480,8 @@ def _linear_own(x: torch.Tensor, w: torch.Tensor) -> bool:
         return False
     if not (x.is_cuda and w.is_cuda) or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or x.dim() != 2 or w.dim() != 2:
         return False
+    if x.layout is not torch.strided or w.layout is not torch.strided or x.is_neg() or w.is_neg():
+        return False
     if not _linear_shape(x.shape[0], *w.shape) or torch.is_grad_enabled() and (x.requires_grad or w.requires_grad):
         return False
     if torch._C._functorch.is_functorch_wrapped_tensor(x) or torch._C._functorch.is_functorch_wrapped_tensor(w) \

@@ -69,6 +69,8 @@ def test_what_stays_with_torch():
     for a, b in ((off, w), (wide, w), (x[None], w), (x, w.t().contiguous().t()), (x.float(), w.float()), (x[:1].expand(96, 128), w)):
         assert not ops._linear_own(a, b)
         assert torch.equal(ops.linear(a, b), torch.nn.functional.linear(a, b))
+    assert not ops._linear_own(x.to_sparse(), w) and not ops._linear_own(x, w.to_sparse())
+    assert not ops._linear_own(torch._neg_view(x), w) and torch.equal(ops.linear(torch._neg_view(x), w), torch.nn.functional.linear(-x, w))
     leaf = w.clone().requires_grad_()
     ops.linear(x, leaf).float().sum().backward()
     assert leaf.grad is not None
