@@ -919,17 +919,27 @@ def window_mfma_sizes(D: int, Dv: int) -> bool:
 WT_SPLITS = 64      # splits of a row's keys that the matrix-core token form joins at most
 
 
+def window_token_tiles(ctx: int, window: int, keep_first: int) -> int:
+    """Tiles of 32 keys that a row of the matrix-core token form has at most: from the window's first key on, and the kept
+    first keys before it."""
+    if window <= 0:
+        return -(-ctx // 32)
+    return -(-min(ctx, window) // 32) + -(-min(keep_first, max(ctx - window, 0)) // 32)
+
+
 def window_token_splits(tiles: int, rows: int, D: int) -> int:
     """Key splits of the matrix-core token form for ``tiles`` tiles of 32 keys at most and ``rows`` tokens times key heads. One
     workgroup of 16 waves reads 0.5 MB for 1000 keys of 128, 8 us of what one compute unit gets; four waves a split, a tile
     each, spread it over the chip and join in the launch for 2.5 us (us a launch whole and split, 8 tokens x 4 key heads of 128:
     200 keys 7.9, 8.8; 400 9.9, 8.9; 1000 15.7, 8.9 in eight; 4000 26.9 by another launch, 18.9 in sixteen; 1 x 4 behind 4000
     23.6, 11.9; 64 columns at 300 keys 6.3, 7.4). Up to 512 workgroups: 32 x 4 behind 2000 in a window of 1024 18.4, 18.1 in
-    four and 21.0 in sixteen; 32 x 8 of 64 behind 2000 31.3, 27.8 in two, 28.8 in sixteen."""
+    four and 21.0 in sixteen; 32 x 8 of 64 behind 2000 31.3, 27.8 in two, 28.8 in sixteen. The tiles are counted exactly: with two more, as
+    a window that starts within a tile would have, 16 x 4 behind 2000 in 1024 took five splits, 14.0, for 13.1 in eight, 32 x 4 three, 19.7
+    for 19.2, and a window of 512 with 64 columns five, 7.8, for 7.0 whole."""
     if tiles <= (12 if D > 64 else 16):
         return 1
     most = min(16, 512 // rows)
-    rounds = -(-tiles // (4 * most)) if most else 1
+    rounds = -(-tiles // (4 * most))
     return max(1, min(most, -(-tiles // (4 * rounds))))
 
 
@@ -985,11 +995,12 @@ def window_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
     if key_splits is None:
         key_splits = 1
         if not mfma and 0 < T * G <= 256:
-            keys = max(int(max_ctx), 1) if window <= 0 else min(max(int(max_ctx), 1), window + 64 + keep_first)
+            ctx = max(int(max_ctx), 1)
             if token:
-                key_splits = window_token_splits(-(-keys // 32), T * G, D)
+                key_splits = window_token_splits(window_token_tiles(ctx, window, keep_first), T * G, D)
             elif T * G < 256:
                 # 64-key windows a row can have, four (one per wave) to a workgroup
+                keys = ctx if window <= 0 else min(ctx, window + 64 + keep_first)
                 key_splits = max(1, min(16, -(-keys // 256), 512 // max(1, T * G)))
     call, extra, st = "loqa_window_attention", (), stream_ptr(q)
     if mfma or key_splits <= 1:
