@@ -1890,8 +1890,14 @@ def _sk_us(lay: int, M: int, N: int, K: int, s: int, gelu: bool) -> float:
     return t
 
 
-_SK_WS_GRAPHS: list = []   # workspaces of captured graphs: they live as long as the process
+_SK_WS_GRAPHS: list = []   # workspaces of captures, until the next eager launch that wants one
 _SK_WS_CAPTURE: dict = {}  # (device, stream) -> (id of its newest capture, workspace)
+_SK_WS_KEPT = 16           # ... or until there are as many
+
+
+def _sk_let_go() -> None:
+    _SK_WS_GRAPHS.clear()
+    _SK_WS_CAPTURE.clear()
 
 
 def _sk_workspace(dev: torch.device, stream: int, floats: int, tiles: int):
@@ -1900,15 +1906,18 @@ def _sk_workspace(dev: torch.device, stream: int, floats: int, tiles: int):
     (stream order serialises them). So do the launches that one capture records on
     one stream: the graph then clears the tickets once, not before each launch
     (2.5 us each: 32 of them are 2 % of a pass of Whisper's large encoder). No
-    two captures share one: it could be regrown by a later capture, freeing memory
-    an earlier graph still replays into, and two graphs replayed on different
-    streams would race on it."""
+    two captures share one: two graphs replayed on different streams would race on it. A capture's lies in its graph's
+    own pool, as all that the capture allocates: once this lets go of it, it stays mapped as long as the graph lives and
+    goes back with it, and only a capture into the same pool, whose graphs do not run beside each other, may
+    get it meanwhile. In a capture that still runs, the launches behind find a new one."""
     if dev.type == "cuda" and torch.cuda.is_current_stream_capturing():
         cid = ctypes.c_uint64()
         check(kernels().loqa_capture_id(stream, ctypes.byref(cid)), "capture_id")
         held, ws = _SK_WS_CAPTURE.get((dev, stream), (None, None))
         if held != cid.value:
             ws = None
+            if len(_SK_WS_GRAPHS) >= _SK_WS_KEPT:
+                _sk_let_go()
         if ws is None or ws[0].numel() < floats or ws[1].numel() < tiles:
             # the larger of both: launches that want much of one and little of the other, in turn, find it
             f = max(floats, 0 if ws is None else ws[0].numel())
@@ -1918,6 +1927,8 @@ def _sk_workspace(dev: torch.device, stream: int, floats: int, tiles: int):
             _SK_WS_GRAPHS.append(ws)
             _SK_WS_CAPTURE[(dev, stream)] = (cid.value, ws)
         return ws
+    if _SK_WS_GRAPHS and _CAPTURES[0] == 0:
+        _sk_let_go()
     key = (dev, stream)
     ws = _SK_WS.get(key)
     if ws is None or ws[0].numel() < floats or ws[1].numel() < tiles:

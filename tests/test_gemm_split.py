@@ -142,3 +142,58 @@ def test_a_captures_workspace_grows_to_the_largest_of_both():
         graph.replay()
         assert all(torch.equal(y, z) for y, z in zip(got, want))
         assert all(torch.equal(y, z) for y, z in zip(run(), want))
+
+
+@pytest.mark.gpu
+def test_captures_give_their_workspaces_back():
+    """Graphs captured and dropped again and again: what is held for them does not grow, the memory is that of before, and a
+    graph that lives replays right beside eager launches and later captures."""
+    g = torch.Generator().manual_seed(4)
+    x = torch.randn(300, 64 * 24, generator=g).bfloat16().cuda()
+    w = (torch.randn(256, x.shape[1], generator=g) / 16).bfloat16().cuda()
+    run = lambda: ops.gemm_sk(x, w, layout=15, splits=3)      # noqa: E731
+
+    def capture():
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            y = run()
+        return graph, y
+    want, (kept, out) = run(), capture()
+    before = torch.cuda.memory_allocated()
+    for _ in range(ops._SK_WS_KEPT + 3):
+        graph, y = capture()
+        y.zero_()
+        graph.replay()
+        assert torch.equal(y, want)
+        del graph, y
+        assert 0 < len(ops._SK_WS_GRAPHS) <= ops._SK_WS_KEPT
+    assert torch.equal(run(), want)
+    assert not ops._SK_WS_GRAPHS and not ops._SK_WS_CAPTURE and torch.cuda.memory_allocated() <= before
+    for _ in range(3):
+        junk = [torch.full((1 << 20,), 7.0, device="cuda") for _ in range(4)]
+        out.zero_()
+        kept.replay()
+        assert torch.equal(out, want) and torch.equal(run(), want) and all((j == 7).all() for j in junk)
+    _words_are_zero()
+
+
+@pytest.mark.gpu
+def test_launches_of_a_capture_whose_workspace_is_let_go():
+    """The workspace of a running capture goes (another thread's eager launch may do that): the launches behind
+    clear their own."""
+    g = torch.Generator().manual_seed(5)
+    x = torch.randn(300, 64 * 24, generator=g).bfloat16().cuda()
+    ws = [(torch.randn(n, x.shape[1], generator=g) / 16).bfloat16().cuda() for n in (256, 1024, 512)]
+    run = lambda w: ops.gemm_sk(x, w, layout=15, splits=3)      # noqa: E731
+    want = [run(w) for w in ws]
+    graph, got = torch.cuda.CUDAGraph(), []
+    with torch.cuda.graph(graph):
+        for w in ws:
+            got.append(run(w))
+            ops._sk_let_go()
+    for _ in range(3):
+        for y in got:
+            y.zero_()
+        graph.replay()
+        assert all(torch.equal(y, z) for y, z in zip(got, want))
+        assert all(torch.equal(run(w), z) for w, z in zip(ws, want))
