@@ -204,6 +204,11 @@ def latent_mfma_sizes(R: int, Dr: int) -> bool:
     return R % 16 == 0 and 0 < R <= 512 and (R + Dr) % 8 == 0 and R + Dr <= 640
 
 
+def _window(window: int, keep_first: int = 0) -> int:
+    """The window as a kernel's int: one that leaves out no key of a position below 2^31 is none."""
+    return window if window + keep_first < 1 << 31 else 0
+
+
 def latent_attention(qa: torch.Tensor, qr: torch.Tensor, cache: torch.Tensor, cu_q: torch.Tensor,
                      ctx_lens: torch.Tensor, block_tables: torch.Tensor, positions: torch.Tensor,
                      cos_sin: torch.Tensor, sink: torch.Tensor | None, scale: float, R: int,
@@ -221,7 +226,7 @@ def latent_attention(qa: torch.Tensor, qr: torch.Tensor, cache: torch.Tensor, cu
     if not qa.is_cuda:
         return ref.latent_attention(qa, qr, cache, cu_q, ctx_lens, block_tables, positions,
                                     cos_sin, sink, scale, R, dims, out, window)
-    Dr = cache.shape[2] - R
+    Dr, window = cache.shape[2] - R, _window(window)
     assert qa.shape[2] == R and qa.stride(2) == 1 and qr.shape == (T, H, Dr) and qr.stride(2) == 1
     assert qa.dtype == cache.dtype == qr.dtype == out.dtype and cache.is_contiguous()
     assert out.is_contiguous() and out.shape == (H, T, R)
@@ -363,6 +368,7 @@ def latent_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu_q: torc
     assert q.stride(2) == 1 and q.stride(1) == DK and k.is_contiguous() and v.is_contiguous()
     assert k.shape[1:] == (H, DK) and v.shape[:2] == k.shape[:2]
     assert DK in PREFILL_DK and DV in PREFILL_DV and 0 < Dv <= DV and window >= 0
+    window = _window(window)
     _i32c(cu_q, "cu_q"); _i32c(cu_k, "cu_k"); _i32c(positions, "positions")
     _i32c(ctx_lens, "ctx_lens")
     B = cu_q.numel() - 1
@@ -980,6 +986,8 @@ def window_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
         assert sink.numel() == H
     T, pages, blk, B, max_blocks, token = lib.window_shapes(q, k_cache, v_cache, cu_q, ctx_lens, block_tables, positions, H, G, D, Dv)
     assert window >= 0 and keep_first >= 0 and softcap >= 0
+    window = _window(window, keep_first)
+    keep_first = keep_first if window else 0
     gs = 0
     if gate is not None:
         assert gate.shape == (T, H * Dv) and gate.stride(1) == 1 and gate.dtype == q.dtype

@@ -94,3 +94,16 @@ def test_parts_repeat_bit_for_bit():
         y.zero_()
         graph.replay()
         assert torch.equal(y, first) and torch.equal(run(), first)
+
+
+@pytest.mark.parametrize("window", [(1 << 31) - 1, 1 << 31, (1 << 32) + 5])
+def test_windows_beyond_all_positions(window):
+    _check([33, 5], [100, 0], 2, 128, 128, 128, window=window, sink=True)
+    g = torch.Generator().manual_seed(1)
+    T, H, R, dims = 3, 4, 128, 64
+    qa, qr, cache = (torch.randn(*s, generator=g).bfloat16().to(DEV) for s in ((H, T, R), (T, H, dims), (9, 16, R + dims)))
+    ints = lambda *x: torch.tensor(x, dtype=torch.int32, device=DEV)      # noqa: E731
+    cs = torch.randn(256, dims // 2, 2, generator=g).to(DEV)
+    run = lambda w: seqmix.latent_attention(qa, qr, cache, ints(0, 1, 3), ints(130, 2), torch.arange(9, dtype=torch.int32, device=DEV)[None].repeat(2, 1),      # noqa: E731
+                                            ints(129, 0, 1), cs, None, 0.1, R, dims, 130, window=w)
+    assert torch.equal(run(window), run(0))

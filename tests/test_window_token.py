@@ -172,3 +172,9 @@ def test_splits_repeat_bit_for_bit():
         y.zero_()
         graph.replay()
         assert torch.equal(y, first) and torch.equal(run(), first)
+
+
+@pytest.mark.parametrize("window,keep", [((1 << 31) - 1, 0), (1 << 31, 0), ((1 << 32) + 5, 3), (1 << 62, 1 << 62), (40, 1 << 31), (40, (1 << 31) - 1), ((1 << 31) - 1, (1 << 31) - 1)])
+def test_windows_and_kept_keys_beyond_all_positions(window, keep):
+    _check([1, 1, 2], [0, 700, 90], 8, 2, 128, 128, window, keep, sink=True)
+    _check([1, 40], [300, 64], 8, 2, 72, 72, window, keep)
