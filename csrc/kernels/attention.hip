@@ -364,8 +364,12 @@ __global__ __launch_bounds__(64 * QW * KS, D == 64 && QW * KS == 4 ? 3 : 2) void
   };
   const unsigned ring = fl_lds_at(lds) + run * L::RING;
   At ka = start(p.k), va = start(p.v);
-  if (per > 0) fetch(kf, ka, ring);
-  va.pages = ka.pages;                                      // with what it holds of the table
+  constexpr bool AHEAD = D == 128 && PAGED && QW == 2;      // K 0 before Q (fl_loop)
+  auto fetch_first = [&]() __attribute__((always_inline)) {
+    if (per > 0) fetch(kf, ka, ring);
+    va.pages = ka.pages;                                    // with what it holds of the table
+  };
+  if constexpr (AHEAD) fetch_first();
 
   bf16x8 qf[NS];
   {
@@ -382,11 +386,11 @@ __global__ __launch_bounds__(64 * QW * KS, D == 64 && QW * KS == 4 ? 3 : 2) void
 #pragma unroll
     for (int j = 0; j < 16; ++j) acc[i][j] = 0.f;
   float m = -1e30f, l = 0.f;
-  fl_loop<D, D, kf.N + vf.N>(
+  if constexpr (!AHEAD) fetch_first();
+  fl_loop<D, D, vf.N + (AHEAD ? kf.N : 0), AHEAD>(
       qf, acc, m, l, ring, per, p.scale_log2, lane, true,
-      // half a tile apart costs 64-column heads on two runs 1 to 3 % (1500 rows x 20 heads 20.1 -> 20.5, behind 512 keys 10.0 -> 10.4),
-      // and a single tile has no other to run beside
-      QW * KS == 8 && (KS == 4 || D == 128) && per > 1 ? wave >> 2 : -1,
+      // half a tile apart costs 64-column heads on two runs off contiguous keys up to 4 % (1500 rows x 20 heads 20.1 -> 20.5)
+      QW * KS == 8 && (PAGED || KS == 4 || D == 128) && per >= FL_APART ? wave >> 2 : -1,
       [&](float16v(&st)[2], int i) __attribute__((always_inline)) {
         // masking only where a key can be invalid for this wave (wave-uniform test)
         const int kt = (first + i) * FL_KEYS;

@@ -111,7 +111,6 @@ __global__ __launch_bounds__(64 * QW * KS, 2) void window_attn_pipe_kernel(WinAt
     });
   };
   At ka = start(p.kc, g * p.D, p.G * p.D), va = start(p.vc, g * p.Dv + v0, p.G * p.Dv);
-  if (!GEN && per > 0) fetch(kf, ka, ring);
 
   bf16x8 qf[NS];
   {
@@ -128,16 +127,14 @@ __global__ __launch_bounds__(64 * QW * KS, 2) void window_attn_pipe_kernel(WinAt
 #pragma unroll
     for (int j = 0; j < 16; ++j) acc[i][j] = 0.f;
   float m = -1e30f, l = 0.f;
-  if (GEN && per > 0) fetch(kf, ka, ring);
+  if (per > 0) fetch(kf, ka, ring);
   va.pages = ka.pages;                                      // with what it holds of the table
 
   // Waves half a tile apart only where a tile's halves weigh alike: transformed scores add a tanh or a bias a score to the
-  // second half, and every half then waits for the longer one. Their run 0 finishes alone and their queries come before the first
-  // keys: with few registers left the other way round was 1 to 5 % slower (us a call, apart, in step, and like this: 2716 rows
-  // x 8 heads of 96, window 1024, bias 57.9, 52.6, 49.7; 951 x 16 of 128, cap 30 and bias 49.7, 49.4, 47.7; 230 x 4 of 96 in two feeds 29.4,
-  // 26.5, 25.9; only 3493 x 8 of 64, window 512, bias 35.2, 31.0, 31.4).
-  fl_loop<DK, DV, kf.N + vf.N>(
-      qf, acc, m, l, ring, per, GEN ? 1.f : scale_log2, lane, p.D == DK && Dv == DV, !GEN && QW * KS == 8 ? wave >> 2 : -1,
+  // second half, and every half then waits for the longer one (us a call, apart, in step: 2716 rows x 8 heads of 96, window
+  // 1024, bias 57.9, 52.6; 951 x 16 of 128, cap 30 and bias 49.7, 49.4; 3493 x 8 of 64, window 512, bias 35.2, 31.0).
+  fl_loop<DK, DV, vf.N, false>(
+      qf, acc, m, l, ring, per, GEN ? 1.f : scale_log2, lane, p.D == DK && Dv == DV, !GEN && QW * KS == 8 && per >= FL_APART ? wave >> 2 : -1,
       [&](float16v(&st)[2], int i) __attribute__((always_inline)) {
         const int kt = tile_at(first + i), k0 = kt + 4 * h;   // tiles past the last lie behind kend
         if constexpr (GEN) {
@@ -169,30 +166,25 @@ __global__ __launch_bounds__(64 * QW * KS, 2) void window_attn_pipe_kernel(WinAt
       [&](int, unsigned stage) __attribute__((always_inline)) { fetch(vf, va, stage); });
 
   fl_sync();                                                // every wave is done with the rings
-  constexpr bool ALL = PARTS || GEN;                        // run 0 finishes alone
-  constexpr int OWN = FlEnd<NDT, QW, KS, ALL>::OWN;
+  constexpr int OWN = FlEnd<NDT, QW, KS, PARTS>::OWN;
   const bf16_t* grow = p.gate ? (const bf16_t*)p.gate + (size_t)(q0 + min(qi, row_hi)) * p.gate_ld + (size_t)head * p.Dv + v0 : nullptr;
   float4v own[OWN];
   uint2 gate[OWN];
   auto ask = [&]() __attribute__((always_inline)) {         // the gates of the run's own units
 #pragma unroll
     for (int s = 0; s < OWN; ++s) {
-      const int d0 = fl_column<NDT, QW, KS, ALL>(s, run, lane);
+      const int d0 = fl_column<NDT, QW, KS, PARTS>(s, run, lane);
       gate[s] = grow && d0 < Dv ? *reinterpret_cast<const uint2*>(grow + d0) : make_uint2(0, 0);
     }
   };
-  if constexpr (!ALL) ask();                                // on their way while the runs meet
-  fl_merge<NDT, QW, KS, ALL>(acc, own, m, l, lds, run, wq, lane);
-  if constexpr (ALL) {
-    if (KS > 1 && run) return;
-  }
+  if constexpr (!PARTS) ask();                              // on their way while the runs meet
+  fl_merge<NDT, QW, KS, PARTS>(acc, own, m, l, lds, run, wq, lane);
   if constexpr (PARTS) {
+    if (run) return;
     const int block = (b * (int)gridDim.y + head * p.vparts + v0 / DV) * (int)(gridDim.x / p.parts) + bx;
     if (parts > 1 && !fl_join<NDT, QW>(acc, m, l, p.part + (size_t)block * p.parts * QW * fl_join_floats(NDT),
                                        p.words + (size_t)block * TICKET, parts, share, wq, lane))
       return;
-  }
-  if constexpr (ALL) {
     fl_units(acc, own);
     ask();
   }
@@ -216,13 +208,13 @@ __global__ __launch_bounds__(64 * QW * KS, 2) void window_attn_pipe_kernel(WinAt
 #pragma unroll
     for (int i = 0; i < 4; ++i) own[s][i] *= f[i];
   }
-  fl_store<NDT, QW, KS, ALL>(own, lds, (bf16_t*)p.o + (size_t)(q0 + row_lo + wq * 32) * p.o_ld + (size_t)head * p.Dv + v0, p.o_ld,
+  fl_store<NDT, QW, KS, PARTS>(own, lds, (bf16_t*)p.o + (size_t)(q0 + row_lo + wq * 32) * p.o_ld + (size_t)head * p.Dv + v0, p.o_ld,
                                qlen - row_lo - wq * 32, Dv, run, wq, lane);
 }
 
 template <int DK, int DV, int QW, int KS, bool GEN, bool PARTS = false>
 static int launch(const WinAttnParams& p, int max_q, hipStream_t st) {
-  constexpr int ring = KS * FlashLds<DK, DV>::RING, end = FlEnd<DV / 32, QW, KS, PARTS || GEN>::BYTES;
+  constexpr int ring = KS * FlashLds<DK, DV>::RING, end = FlEnd<DV / 32, QW, KS, PARTS>::BYTES;
   constexpr int bytes = ring > end ? ring : end;
   static_assert(bytes <= 160 * 1024, "LDS of a CU");
   const long blocks = (max_q + 32 * QW - 1) / (32 * QW), all = blocks * p.H * p.vparts * p.B;

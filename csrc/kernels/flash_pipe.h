@@ -211,15 +211,23 @@ __device__ __forceinline__ float fl_both32(float x) {  // lane + lane ^ 32
 // leaves the registers where they are). load_k / load_v(i, stage) start the fetch of tile i;
 // they are called for i = 1, 2, .. up to n (K) and i = 0 .. n - 1 (V); for i = n they must fetch
 // something that exists (or nothing). Where n > 0 the caller has started the fetch of K tile 0 into the ring, ahead of
-// its loads of Q: one trip to memory for both. counted: V 0 and K 1 are BEHIND loads of every wave exactly.
+// its loads of Q or behind them: one trip to memory for both. V 0 is asked for before the first wait, which is for K 0, and K 1 behind
+// it, or with BOTH before it as well; counted: those are BEHIND loads of every wave exactly.
+// (What a form takes is what it measured: with K 0 behind Q and K 1 behind the wait, windowed prompts of 64-column heads in 512
+// keys 17.0 -> 16.3 us, causal ones of 1300 rows x 32 such heads 24.7 -> 23.9; 64-row blocks of 128-column heads off pages go with K 0 ahead
+// of Q and BOTH, as the other order leaves registers to scratch there, and so do latent prompts, which it cost 1 %.)
 // phase: -1, or in workgroups of eight waves 0 for the first four and 1 for the others, which share the four SIMDs: each
 // half of a tile then begins with a barrier of all waves, and the second four run half a tile behind, their exponentials,
 // maxima and rescaling beside the scores' MFMAs of the first (in step, both waves of a SIMD want the same unit; 2048 rows of
 // 16 latent heads of 192 / 128 43.7 -> 41.6 us, of 32 58.5 -> 56.7, 1500 rows x 8 heads of 64 on four runs 13.7 -> 12.9; wave priorities
-// and six or eight fragments in flight beside it: the same within 1 %).
+// and six or eight fragments in flight beside it: the same within 1 %). The half tile more is too much for runs of few tiles
+// (windows of 300 keys, four tiles a run: 2048 rows x 16 heads of 64 14.5 us in step, 15.3 apart; of 128 19.3, 19.7), so a workgroup
+// takes it from FL_APART tiles a run on.
 // Before the call m = -1e30, l = 0, acc = 0; ring must not be in use. After it the waves
 // are not synchronised.
-template <int DK, int DV, int BEHIND, typename Prep, typename LoadK, typename LoadV>
+#define FL_APART 6
+
+template <int DK, int DV, int BEHIND, bool BOTH, typename Prep, typename LoadK, typename LoadV>
 __device__ __forceinline__ void fl_loop(const bf16x8 (&qf)[DK / 16], float16v (&acc)[DV / 32], float& m, float& l,
                                         unsigned ring, int n, float sl2, int lane, bool counted, int phase, Prep&& prep,
                                         LoadK&& load_k, LoadV&& load_v) {
@@ -253,7 +261,7 @@ __device__ __forceinline__ void fl_loop(const bf16x8 (&qf)[DK / 16], float16v (&
   for (int j = 0; j < 8; ++j) ones[j] = (__bf16)1.0f;
   const fl_b2 one2 = {(__bf16)1.0f, (__bf16)1.0f};
 
-  // Q is here, and with it K 0, before the next loads whose wait the compiler does not know
+  // Q is here, and a K 0 asked for ahead of it, before the next loads whose wait the compiler does not know
   bf16x8 qr[NS];
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
@@ -309,7 +317,7 @@ __device__ __forceinline__ void fl_loop(const bf16x8 (&qf)[DK / 16], float16v (&
       fl_sync();
     } else {
       load_v(0, ring + 2 * L::K);
-      load_k(1, ring + L::K);
+      if constexpr (BOTH) load_k(1, ring + L::K);
       if (counted) fl_sync_first<BEHIND>();
       else fl_sync();
     }
@@ -319,6 +327,8 @@ __device__ __forceinline__ void fl_loop(const bf16x8 (&qf)[DK / 16], float16v (&
       if constexpr (SM) {
         load_k(i + 2, ring + S * L::K);
         load_v(i + 1, ring + 2 * L::K + (1 - S) * L::V);
+      } else if constexpr (!BOTH) {
+        load_k(1, ring + L::K);
       }
     }
 #pragma unroll

@@ -181,3 +181,14 @@ def test_one_tile_on_every_block_height(n, H, D):
         _check([n, 1, 33], [m, 64, 1], H, H // 4, D, False, seed=m)
         _check([m, 1], [m, 64], H, H // 4, D, True, page=16, seed=m)
     _check([n, 70], [64, 65], H, H // 4, D, False, seed=3)          # one tile beside two
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_runs_of_few_tiles_and_many(D):
+    # five and six tiles a run, around which the waves of a SIMD go half a tile apart: two runs of 128 rows, four (two) of 64
+    for n in (640, 641):
+        _check([700], [n], 20, 20, D, False, seed=n)
+    _check([850], [1400], 32, 8, D, True, page=16, seed=1)
+    _check([850], [1400], 32, 8, D, True, page=64, seed=2)
+    _check([64, 40], [1280, 1281], 8, 8, D, False, seed=3)
+    _check([64, 40], [640, 641], 8, 8, D, False, seed=4)

@@ -155,3 +155,12 @@ def test_prompts_of_any_context_bound(most):
     args = (q, kc, vc, i32([0, 33]), i32([2100]), i32(torch.randperm(132, generator=g).view(1, 132)), i32(range(2067, 2100)), 0.125, 0.0, 0, 0, None, 8, 2, 64, 64)
     y, z = (seqmix.window_attention(*args, max_q=33, max_ctx=n).double() for n in (most, 2100))
     assert (y - z).norm() <= 4e-3 * z.norm()
+
+
+@pytest.mark.parametrize("D,Dv", [(64, 64), (128, 128), (64, 128), (96, 96)])
+@pytest.mark.parametrize("window", [300, 513, 600, 0])
+def test_runs_of_few_tiles_and_many(D, Dv, window):
+    # four to six tiles a run and more, around which the waves of a SIMD go half a tile apart; transformed scores in step
+    _check([900], [60], 32, 8, D, Dv, window, 5, sink=True, gate=True, seed=1)
+    _check([900], [60], 32, 8, D, Dv, window, 5, cap=30.0, gate=True, seed=2)
+    _check([900], [60], 32, 8, D, Dv, window, 0, slopes=True, sink=True, seed=3)
