@@ -364,7 +364,7 @@ __global__ __launch_bounds__(64 * QW * KS, D == 64 && QW * KS == 4 ? 3 : 2) void
   };
   const unsigned ring = fl_lds_at(lds) + run * L::RING;
   At ka = start(p.k), va = start(p.v);
-  constexpr bool AHEAD = D == 128 && PAGED && QW == 2;      // K 0 before Q (fl_loop)
+  constexpr bool AHEAD = PAGED ? D == 128 && QW == 2 : KS == 1;   // K 0 before Q (fl_loop)
   auto fetch_first = [&]() __attribute__((always_inline)) {
     if (per > 0) fetch(kf, ka, ring);
     va.pages = ka.pages;                                    // with what it holds of the table

@@ -215,7 +215,8 @@ __device__ __forceinline__ float fl_both32(float x) {  // lane + lane ^ 32
 // it, or with BOTH before it as well; counted: those are BEHIND loads of every wave exactly.
 // (What a form takes is what it measured: with K 0 behind Q and K 1 behind the wait, windowed prompts of 64-column heads in 512
 // keys 17.0 -> 16.3 us, causal ones of 1300 rows x 32 such heads 24.7 -> 23.9; 64-row blocks of 128-column heads off pages go with K 0 ahead
-// of Q and BOTH, as the other order leaves registers to scratch there, and so do latent prompts, which it cost 1 %.)
+// of Q and BOTH, as the other order leaves registers to scratch there, and so do latent prompts and runs of four waves off
+// contiguous keys, which it cost 1 % and 0.5: 8 x 1500 rows x 8 heads of 64 52.9 us, 52.4.)
 // phase: -1, or in workgroups of eight waves 0 for the first four and 1 for the others, which share the four SIMDs: each
 // half of a tile then begins with a barrier of all waves, and the second four run half a tile behind, their exponentials,
 // maxima and rescaling beside the scores' MFMAs of the first (in step, both waves of a SIMD want the same unit; 2048 rows of
