@@ -82,11 +82,10 @@ template <int NT> struct DcLocal {
 };
 
 // The block of head h's chunk of tokens t0 .. t0 + n - 1, by 256 threads. All of it is written in whole 64-byte runs.
-// AUX: of the stores (16: through the caches). What bounds it is memory (2048 tokens, 16 heads of 128 x 128, a decay per
-// channel: 67 MB of rows read, 70 written; 26 us at a large copy's rate), so the waves in flight: with the triangle's
+// What bounds it is memory (2048 tokens, 16 heads of 128 x 128, a decay per channel: 67 MB of rows read, 70 written; 26 us at a large copy's rate), so the waves in flight: with the triangle's
 // A in registers ahead of the substitution (166 a thread, three workgroups a CU), rows in 4-byte loads and columns stored
 // in 16-byte pieces 64 bytes apart it took 39 us, with 55 registers, five workgroups and whole runs 30.
-template <int NT, bool CHAN, int AUX>
+template <int NT, bool CHAN>
 __device__ __forceinline__ void delta_local(const DcParams& p, DcLocal<NT>& s, float* ws, int t0, int n, int h, int tid) {
   constexpr int DP = 64 * NT;
   const int D = p.D, Dv = p.Dv, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -94,7 +93,7 @@ __device__ __forceinline__ void delta_local(const DcParams& p, DcLocal<NT>& s, f
   const __amdgpu_buffer_rsrc_t block = __builtin_amdgcn_make_buffer_rsrc(ws, 0, (int)(dc_stride(DP, Dv) * 4), 0x00020000);
   auto put = [&](int at, const float* v) {                  // four floats to entry at
     __builtin_amdgcn_raw_buffer_store_b128(dc_u4{__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])},
-                                           block, at * 4, 0, AUX);
+                                           block, at * 4, 0, 0);
   };
   // a thread's 16 numbers of column c0 + lane, as [column][16] from entry `to` on, of `cols` columns
   auto put_columns = [&](int to, int c0, int cols, const float (&x)[DC_C]) {
@@ -193,7 +192,7 @@ __device__ __forceinline__ void delta_local(const DcParams& p, DcLocal<NT>& s, f
       r *= s.gs[j][tid];
     }
     put_columns(32 * DP, 64 * wave, DP, kk);
-    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(r), block, (48 * DP + tid) * 4, 0, AUX);
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(r), block, (48 * DP + tid) * 4, 0, 0);
   }
   __syncthreads();
 #pragma unroll
@@ -242,7 +241,7 @@ __global__ __launch_bounds__(256) void delta_local_kernel(DcParams p) {
   __shared__ __attribute__((aligned(16))) DcLocal<NT> s;
   int b, t0, n;
   if (!seq_chunk<DC_C>(p.cu_q, p.B, blockIdx.x, b, t0, n)) return;
-  delta_local<NT, CHAN, 0>(p, s, p.ws + ((size_t)blockIdx.x * p.H + blockIdx.y) * dc_stride(64 * NT, p.Dv), t0, n, blockIdx.y, threadIdx.x);
+  delta_local<NT, CHAN>(p, s, p.ws + ((size_t)blockIdx.x * p.H + blockIdx.y) * dc_stride(64 * NT, p.Dv), t0, n, blockIdx.y, threadIdx.x);
 }
 
 // Every wave of the workgroup is here and its LDS writes are visible; global loads stay in
