@@ -100,14 +100,18 @@ SEQMIX_SOURCES = ("norm_dyt.hip", "attn_latent.hip", "attn_latent_prefill.hip", 
 NO_PACKED_F32 = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 
 
-def _build_launch(force: bool, opt: list[str]) -> str:
-    """The Python module, host code only: a plain C++ compiler against torch's headers."""
-    torch_dir = importlib.util.find_spec("torch").submodule_search_locations[0]
+def _build_launch(force: bool, opt: list[str]) -> str | None:
+    """The Python module, host code only: a plain C++ compiler against torch's headers, in the ABI that torch was built in. None where
+    there is no torch, which no kernel of the others needs to be built."""
+    spec = importlib.util.find_spec("torch")
+    if spec is None:
+        return None
+    torch_dir = spec.submodule_search_locations[0]
     with open(os.path.join(torch_dir, "version.py")) as f:
         version = hashlib.sha256(f.read().encode()).hexdigest()
     src, out = os.path.join(CSRC, "launch", "launch.cpp"), os.path.join(HERE, "libloqa_launch.so")
-    flags = [*opt, "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D_GLIBCXX_USE_CXX11_ABI=1",
-             f"-I{os.path.join(torch_dir, 'include')}", f"-I{sysconfig.get_paths()['include']}"]
+    flags = [*opt, "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", f"-I{os.path.join(torch_dir, 'include')}",
+             f"-I{sysconfig.get_paths()['include']}"]
     digest, stamp = _digest([src], [*flags, version]), out + ".sha256"
     if not force and os.path.exists(out) and os.path.exists(stamp):
         with open(stamp) as f:
@@ -116,6 +120,8 @@ def _build_launch(force: bool, opt: list[str]) -> str:
     cxx = [shutil.which("g++") or shutil.which("c++")]
     if cxx[0] is None:
         cxx = [_hipcc(), "-x", "c++"]
+    import torch
+    flags.append(f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}")
     cmd = [*cxx, *flags, src, "-o", out + ".tmp", f"-L{os.path.join(torch_dir, 'lib')}", "-ltorch_python", "-ltorch_cpu", "-lc10"]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
@@ -148,7 +154,8 @@ def build(force: bool = False, debug: bool = False, only=None, quiet: bool = Fal
         if only is None or name in only:
             out.append(_build_lib(name, src, hdr, flags, force))
     if only is None or "libloqa_launch.so" in only:
-        out.append(_build_launch(force, ["-O0", "-g"] if debug else ["-O2"]))
+        made = _build_launch(force, ["-O0", "-g"] if debug else ["-O2"])
+        out += [made] if made else []
     return out
 
 
