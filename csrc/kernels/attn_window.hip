@@ -1069,8 +1069,9 @@ extern "C" int loqa_window_attention(const void* q, int dt, const void* kc, cons
 }
 
 // The same with up to `parts` parts of a row block's keys in workgroups of their own, where the sizes and
-// scores take them: `part` (part_floats of them) and `words` (zeroed, `tickets` TICKETs) are theirs. An entry of its own,
-// as a token step is host work and every argument is a part of it (four more: 23.5 -> 23.8 us).
+// scores take them, or with a token step's key splits (ns) joined in the launch: `part` (part_floats of them) and `words`
+// (zeroed, `tickets` TICKETs) are theirs. An entry of its own, as launches without them are host work and every
+// argument is a part of it (four more: 23.5 -> 23.8 us).
 extern "C" int loqa_window_attention_parts(const void* q, int dt, const void* kc, const void* vc, int blk,
                                      int nblocks, const void* cu_q, const void* ctx, const void* bt,
                                      int max_blocks, const void* pos, const void* gate, long gate_ld,

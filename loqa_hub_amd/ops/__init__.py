@@ -1805,7 +1805,8 @@ _SK_WS: dict = {}
 
 def gemm_sk_plan(M: int, N: int, K: int, epi: str = "bf16", layouts=None, *,
                  pipe: bool = True) -> tuple[int, int]:
-    """(layout, K chunks) for a shape: the fewest microseconds by SK_LAYOUTS, counting whole
+    """(layout, K chunks) for a shape among SK_LAYOUTS (what :func:`gemm_sk` takes but where a tile of SK_ROWS160 is
+    faster: :func:`_sk_choice`): the fewest microseconds, counting whole
     rounds of tiles over the compute units; up to SK_FEW workgroups load so little beside each other that
     a K step takes 0.8 of its time (1500 x 512 x 2048 on 96 of them 11.0 us, in two chunks on 192 11.6), and where many
     rows share the weights, on as many workgroups as SK_SHARED says, 0.9 (1500 x 768 x 3072 on 144 17.1 us; whole tiles of 2200 x

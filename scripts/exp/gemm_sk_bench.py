@@ -1,7 +1,7 @@
 """Split-K tiled GEMM (ops.gemm_sk) vs hipBLASLt (torch.matmul) on the prefill
 and Whisper-encoder projection shapes, cold weights (a ring of weight copies
 larger than the 256 MiB Infinity Cache), CUDA-event timing; prints one JSON
-line per (shape, variant) and the planner's pick.
+line per (shape, variant) and what gemm_sk takes by itself.
 
     python scripts/exp/gemm_sk_bench.py [--ms 300,600,1200] [--grid]
 """
@@ -59,7 +59,7 @@ def main():
         res = torch.randn(M, N, device=dev).bfloat16()
         flops = 2.0 * M * N * K
         t_blas = timeit(lambda i: torch.matmul(x, ws[i].t()), n_w)
-        lay, s = ops.gemm_sk_plan(M, N, K, epi)
+        lay, s = ops._sk_choice(M, N, K, True)
 
         def run(i, lay=lay, s=s):
             if epi == "resid":
@@ -82,8 +82,8 @@ def main():
         if a.grid:
             best = None
             grid = {}
-            for l2 in sorted(ops.SK_LAYOUTS):
-                bn, bm = ops.SK_LAYOUTS[l2][:2]
+            for l2 in sorted({**ops.SK_LAYOUTS, **ops.SK_ROWS160}):
+                bn, bm = ops._sk_tile(l2)[:2]
                 if N % bn:
                     continue
                 for s2 in (1, 2, 3, 4, 6, 8):
