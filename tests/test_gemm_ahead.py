@@ -45,7 +45,7 @@ def test_only_tensors_of_the_same_device(device):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("layout", [k for k in sorted(ops.SK_LAYOUTS) if k >= ops.SK_PIPE])
+@pytest.mark.parametrize("layout", [k for k in sorted({**ops.SK_LAYOUTS, **ops.SK_ROWS160}) if k >= ops.SK_PIPE])
 def test_product_is_the_same(layout, monkeypatch):
     g = torch.Generator().manual_seed(layout)
     x = torch.randn(300, 1024, generator=g).bfloat16().cuda()

@@ -18,11 +18,11 @@ def _words_are_zero():
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("layout", [k for k in sorted(ops.SK_LAYOUTS) if k >= ops.SK_PIPE])
+@pytest.mark.parametrize("layout", [k for k in sorted({**ops.SK_LAYOUTS, **ops.SK_ROWS160}) if k >= ops.SK_PIPE])
 @pytest.mark.parametrize("splits", [2, 3, 4, 5, 8, 9, 14])
 def test_shares_of_a_tile(layout, splits):
     """More chunks than units of 16 x 16 in a share divide evenly, more than SK_SHARE, ragged rows, every epilogue."""
-    bn, bm = ops.SK_LAYOUTS[layout][:2]
+    bn, bm = ops._sk_tile(layout)[:2]
     K, N, M = 64 * 14, 2 * bn, bm + 21
     g = torch.Generator().manual_seed(layout)
     x = torch.randn(M, K, generator=g).bfloat16().cuda()
@@ -58,12 +58,12 @@ def test_a_chunk_that_starts_a_round_later():
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("layout", [k for k in sorted(ops.SK_LAYOUTS) if k >= ops.SK_PIPE])
+@pytest.mark.parametrize("layout", [k for k in sorted({**ops.SK_LAYOUTS, **ops.SK_ROWS160}) if k >= ops.SK_PIPE])
 @pytest.mark.parametrize("splits", [2, 4, 5, 8])
 def test_shares_given_up(layout, splits, monkeypatch):
     """No looks at a tile's word: every workgroup but the last to arrive goes through publishing what it kept and giving
     its share up, in every epilogue, with and without kept shares. Whoever sums a share up, it is the same bits."""
-    bn, bm = ops.SK_LAYOUTS[layout][:2]
+    bn, bm = ops._sk_tile(layout)[:2]
     K, N, M = 64 * 14, 4 * bn, 2 * bm + 21
     g = torch.Generator().manual_seed(layout)
     x = torch.randn(M, K, generator=g).bfloat16().cuda()
