@@ -31,8 +31,8 @@
 // 64 x 64 tiles keep the chip busy where 128 x 64 leave half of it idle: 80 KB of rings, a K step of 16 KB (0.18 us, 128 x
 // 64 0.27). 1500 x 512 x 2048 11.1 -> 8.9 us, x 512 5.7 -> 4.7, 300 x 1280 x 1280 9.0 -> 6.6, 200 x 3072 x 2048 11.9 -> 9.0.
 //
-// Tiles of 160 rows are for what pads the others: 320 rows are five sixths of two tiles of 192. 320 x 28672 x 4096 79.7 -> 73.4 us,
-// 640 143 -> 131, 1280 x 4096 x 14336 135 -> 119 in two chunks. Four stages instead of three of 128 x 160: 2 % slower.
+// Tiles of 160 rows are for what pads the others: 320 rows are five sixths of two tiles of 192. 320 x 28672 x 4096 76.1 -> 73.0 us,
+// 640 138 -> 127, 1280 x 4096 x 14336 127 -> 118 in two chunks. Four stages instead of three of 128 x 160: 2 % slower.
 //
 // Workgroups behind the tiles' (AHEAD: a variant, as the others start 0.15 us sooner without the
 // question) bring the weights of later launches into the Infinity Cache.

@@ -1777,11 +1777,11 @@ SK_LAYOUTS = {1: (128, 64, 0.60, 4.0), 7: (64, 64, 0.55, 4.0), 11: (64, 64, 0.19
               15: (256, 128, 0.908, 4.0), 16: (128, 256, 0.784, 6.6), 17: (128, 192, 0.667, 4.6),
               18: (192, 192, 0.854, 6.0), 19: (128, 64, 0.309, 4.3), 20: (128, 128, 0.498, 3.6)}
 # Tiles of 160 rows (pipelined), for row counts that pad the others: gemm_sk asks the plan's rules for these beside the plan
-# (_sk_choice). Times fitted over 256 shapes of 100 to 3000 rows, cold weights, against the plan alone: taken in 30 of them, 0.94 of the
-# time there, slower by more than 1.5 % in none; 12 more that they would win by 2 to 13 % are left to the plan. The step of 22 is fitted
-# 4 % above what it takes: it is bound by LDS, where 128 x 192 is bound by its MFMAs, and wins only by rows that it does not pad. us, the
-# plan's and these: 320 x 28672 x 4096 79.7, 73.4; 640 143, 131; 160 x 6144 x 4096 22.8, 21.1; 1280 x 4096 x 14336 135, 119; 1500 x 11264 x
-# 2048 74.5, 66.9.
+# (_sk_choice). Times fitted over 256 shapes of 100 to 3000 rows, cold weights, against the plan alone (profiles/rows160.txt): taken in
+# 25 of them, 0.94 of the time there, 1.003 at worst; 40 that they would win alone by 2 to 19 % are left to the plan. The step of 22 is
+# fitted 4 % above what it takes: it is bound by LDS, where 128 x 192 is bound by its MFMAs, and wins only by rows that it does not pad.
+# us, the plan's and these: 320 x 28672 x 4096 76.1, 73.0; 640 138, 127; 160 x 6144 x 4096 23.3, 21.6; 1280 x 4096 x 14336 127, 118; 1500 x
+# 11264 x 2048 74.1, 65.4.
 # In a pass of a model each K chunk costs more than it does alone, as its partials go out and back beside the next launch's cold
 # weights, and the attention behind finds less of its keys (320 rows of an 8B model: 15.2 -> 16.3 us): so at most one chunk more than
 # the plan's, none where it has none, and 128 x 160 for one tile of rows only. us a projection in the pass with the plan's tile and with
