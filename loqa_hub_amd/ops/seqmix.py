@@ -22,6 +22,8 @@ norm statistics are f32 in both.
 """
 from __future__ import annotations
 
+import functools
+
 import torch
 
 from . import reference as ref
@@ -204,9 +206,9 @@ def latent_mfma_sizes(R: int, Dr: int) -> bool:
     return R % 16 == 0 and 0 < R <= 512 and (R + Dr) % 8 == 0 and R + Dr <= 640
 
 
-def _window(window: int, keep_first: int = 0) -> int:
+def _window(window: int) -> int:
     """The window as a kernel's int: one that leaves out no key of a position below 2^31 is none."""
-    return window if window + keep_first < 1 << 31 else 0
+    return window if window < 1 << 31 else 0
 
 
 def latent_attention(qa: torch.Tensor, qr: torch.Tensor, cache: torch.Tensor, cu_q: torch.Tensor,
@@ -949,6 +951,12 @@ def window_token_splits(tiles: int, rows: int, D: int) -> int:
     return max(1, min(most, -(-tiles // (4 * rounds))))
 
 
+@functools.lru_cache(maxsize=4096)
+def _window_token_plan(ctx: int, window: int, keep_first: int, rows: int, D: int) -> int:
+    """:func:`window_token_splits` by a step's plain values, which all layers of a model share: 0.8 us on the host, 0.15 asked again."""
+    return window_token_splits(window_token_tiles(ctx, window, keep_first), rows, D)
+
+
 def window_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
                      cu_q: torch.Tensor, ctx_lens: torch.Tensor, block_tables: torch.Tensor,
                      positions: torch.Tensor, scale: float, softcap: float, window: int,
@@ -986,8 +994,8 @@ def window_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
         assert sink.numel() == H
     T, pages, blk, B, max_blocks, token = lib.window_shapes(q, k_cache, v_cache, cu_q, ctx_lens, block_tables, positions, H, G, D, Dv)
     assert window >= 0 and keep_first >= 0 and softcap >= 0
-    window = _window(window, keep_first)
-    keep_first = keep_first if window else 0
+    if window == 0 or window + keep_first >= 1 << 31:       # as _window()
+        window = keep_first = 0
     gs = 0
     if gate is not None:
         assert gate.shape == (T, H * Dv) and gate.stride(1) == 1 and gate.dtype == q.dtype
@@ -1005,7 +1013,7 @@ def window_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
         if not mfma and 0 < T * G <= 256:
             ctx = max(int(max_ctx), 1)
             if token:
-                key_splits = window_token_splits(window_token_tiles(ctx, window, keep_first), T * G, D)
+                key_splits = _window_token_plan(ctx, window, keep_first, T * G, D)
             elif T * G < 256:
                 # 64-key windows a row can have, four (one per wave) to a workgroup
                 keys = ctx if window <= 0 else min(ctx, window + 64 + keep_first)

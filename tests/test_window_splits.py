@@ -19,4 +19,4 @@ def test_tiles_are_those_of_the_kernel(ctx, window, keep, tiles):
 @pytest.mark.parametrize("window,rows,D,splits", [(1024, 32, 128, 8), (1024, 64, 128, 8), (1024, 128, 128, 4), (512, 32, 128, 4), (512, 128, 128, 4),
                                                   (512, 32, 64, 1), (1024, 32, 64, 8), (300, 32, 128, 1), (1024, 256, 128, 2)])
 def test_splits_of_whole_windows(window, rows, D, splits):
-    assert seqmix.window_token_splits(seqmix.window_token_tiles(2048, window, 0), rows, D) == splits
+    assert seqmix.window_token_splits(seqmix.window_token_tiles(2048, window, 0), rows, D) == seqmix._window_token_plan(2048, window, 0, rows, D) == splits
