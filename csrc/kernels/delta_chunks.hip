@@ -82,9 +82,10 @@ template <int NT> struct DcLocal {
 };
 
 // The block of head h's chunk of tokens t0 .. t0 + n - 1, by 256 threads. All of it is written in whole 64-byte runs.
-// What bounds it is memory (2048 tokens, 16 heads of 128 x 128, a decay per channel: 67 MB of rows read, 70 written; 26 us at a large copy's rate), so the waves in flight: with the triangle's
-// A in registers ahead of the substitution (166 a thread, three workgroups a CU), rows in 4-byte loads and columns stored
-// in 16-byte pieces 64 bytes apart it took 39 us, with 55 registers, five workgroups and whole runs 30.
+// What bounds it is memory (2048 tokens, 16 heads of 128 x 128, a decay per channel: 67 MB of rows read, 70 written; 26 us
+// at a large copy's rate), so the waves in flight: with the triangle's A in registers ahead of the substitution (166 a
+// thread, three workgroups a CU), rows in 4-byte loads and columns stored in 16-byte pieces 64 bytes apart it took 39 us,
+// with 55 registers, five workgroups and whole runs 30.
 template <int NT, bool CHAN>
 __device__ __forceinline__ void delta_local(const DcParams& p, DcLocal<NT>& s, float* ws, int t0, int n, int h, int tid) {
   constexpr int DP = 64 * NT;
